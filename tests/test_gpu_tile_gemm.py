@@ -1,0 +1,39 @@
+"""Prompt-sized products on the shared matrix-core tiles (csrc/tile_gemm.h) at the edges of their tiles, stages and shape choices."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import torch
+    import vllm_rust_amd as vmx
+    assert torch.cuda.is_available()
+    vmx.init(0)
+    return vmx, torch
+
+
+# rows and columns one below, at and one above the 64- and 128-wide tiles; one, two, three and many 64-deep stages; the last three take
+# the 128 x 128 tiles (a workgroup for every compute unit), 40 x 20000 the 64 x 64 tiles in two stages
+@pytest.mark.parametrize("M,N,K", [(17, 1, 64), (63, 64, 128), (64, 65, 192), (65, 63, 64), (127, 129, 256), (129, 200, 2048), (40, 20000, 128),
+                                   (129, 16385, 64), (300, 12289, 192), (257, 16384, 320)])
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+def test_bf16_linear_tiles(gpu, M, N, K, out):
+    """Against float64 on the same bf16 operands: an f32 sum of K exact products is off by at most (K + 8) 2^-24 sum |x w| (the matrix
+    core adds in f32, in blocks), a bf16 result by half an ulp more."""
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    g = torch.Generator(device="cuda").manual_seed(M * 131 + N + K)
+    x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
+    w = torch.randn((N, K), device="cuda", generator=g).to(torch.bfloat16)
+    guard = torch.full((M + 2, N), 7.0, device="cuda", dtype=torch.float32 if out == "f32" else torch.bfloat16)
+    y = guard[1:M + 1]
+    check(lib.vmx_linear_bf16w(y.data_ptr(), 0 if out == "f32" else 1, x.data_ptr(), 1, w.data_ptr(), M, N, K, 0, None))
+    torch.cuda.synchronize()
+    ref = x.double() @ w.double().T
+    bound = (K + 8) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    if out == "bf16":
+        bound = bound + 2.0 ** -8 * ref.abs()
+    assert bool(((y.double() - ref).abs() <= bound).all())
+    assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all())

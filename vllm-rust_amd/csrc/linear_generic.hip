@@ -8,13 +8,13 @@
 //   * an optional bf16 bias per output column, then an epilogue: plain store, squared ReLU, tanh-form GELU, accumulate into an
 //     f32 residual stream, multiply by sigmoid(gate), or both of the last two (a gated residual update); a range of output columns
 //     may go through SiLU, so that one product serves readers that want it and readers that do not.
-// Kernels: `linear_mfma_kernel` (64-row tiles for prompts and 64-row expert blocks; a staged 16-row form for shapes the streaming
-// kernel does not take) and `linear_skinny_kernel` (up to 16 rows: decode steps and 16-row expert blocks, weights streamed once)
-// round the activations to bf16 and run v_mfma_f32_16x16x32_bf16; `linear_fma_kernel` multiplies in true f32 on the vector ALU
-// (the 32-bit mode of a model), `linear_fewcols_f32_kernel` does the same for a few output columns (router logits) with one
-// kernel for every row count.  A row's result never depends on the other rows of the call: within a kernel a row is summed in
+// Kernels: `linear_tile_kernel` (prompts and 64-row expert blocks with bf16 rows in whole 64-deep stages), `linear_mfma_kernel` (the same
+// for f32 or unaligned rows; a staged 16-row form for shapes the streaming kernel does not take) and `linear_skinny_kernel` (up to 16
+// rows: decode steps and 16-row expert blocks, weights streamed once) round the activations to bf16 and multiply on the matrix cores;
+// `linear_fma_kernel` multiplies in true f32 on the vector ALU (the 32-bit mode of a model), `linear_fewcols_f32_kernel` does the
+// same for a few output columns (router logits) with one kernel for every row count.  A row's result never depends on the other rows of the call: within a kernel a row is summed in
 // the same order whatever M is; between the streaming and the tiled kernels the order differs (rounding-level differences).
-#include "vmx_kernels.h"
+#include "tile_gemm.h"
 
 namespace {
 
@@ -234,6 +234,65 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const VmxLinear p) {
         }
 }
 
+// Prompt-sized bf16 products on the core of tile_gemm.h: plain, batched, gathered rows and 64-row expert blocks alike.  EP: the
+// finished sums are stored as they are, with a bias and a SiLU range, or through linear_store (whose run-time choices per element cost a
+// 1500 x 12288 output as much as half of its product: 159 against 101 us).
+enum { TILE_PLAIN, TILE_BIAS_SILU, TILE_ANY };
+template <class S, int EP>
+__global__ __launch_bounds__(S::THREADS) void linear_tile_kernel(const VmxLinear p, int row_tiles, int tiles) {
+    extern __shared__ __align__(16) uint16_t tg_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tile = tg_tile(blockIdx.x, tiles), z = blockIdx.y;
+    if (tile < 0) return;
+    const int m0 = tile % row_tiles * S::BM, n0 = tile / row_tiles * S::BN;
+    if (p.total_rows && m0 >= *p.total_rows) return;
+    const uint16_t *W = p.W + z * p.w_bs;
+    if (p.block_expert) W += (int64_t)p.block_expert[m0 / p.block_rows] * p.expert_stride;
+    // rows and columns past the end (and padding rows) fetch a row that exists; what they give is not stored
+    uint32_t a_src[S::AQ], b_src[S::BQ];
+#pragma unroll
+    for (int q = 0; q < S::AQ; q++) {
+        const int64_t r = linear_src_row(p, m0 + tg_src_row<S::AQ>(wave, lane, q));
+        a_src[q] = (uint32_t)((r < 0 ? 0 : r) * p.lda * 2) + tg_src_byte(lane);
+    }
+#pragma unroll
+    for (int q = 0; q < S::BQ; q++)
+        b_src[q] = (uint32_t)((int64_t)min(n0 + tg_src_row<S::BQ>(wave, lane, q), p.N - 1) * p.w_sn * 2) + tg_src_byte(lane);
+    tg_f32x16 acc[S::MI][S::NJ];
+#pragma unroll
+    for (int i = 0; i < S::MI; i++)
+#pragma unroll
+        for (int j = 0; j < S::NJ; j++) acc[i][j] = tg_f32x16{};
+    tg_product<false, S>((const char *)((const uint16_t *)p.A + z * p.a_bs), a_src, (const char *)W, b_src, p.K, tg_lds, wave, lane, acc, [](int) {});
+    const int wm = m0 + wave / S::WN * (S::MI * 32), wn = n0 + wave % S::WN * (S::NJ * 32) + (lane & 31);
+#pragma unroll
+    for (int j = 0; j < S::NJ; j++) {
+        const int n = wn + 32 * j;
+        if (n >= p.N) continue;
+        const float bias = EP == TILE_BIAS_SILU && p.bias ? vmx_bf16_to_f32(p.bias[n + z * p.bias_bs]) : 0.f;
+        const bool silu = n >= p.silu_begin && n < p.silu_end;
+#pragma unroll
+        for (int i = 0; i < S::MI; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int m = wm + 32 * i + tg_acc_row(lane, r);
+                if (m >= p.M || (p.row_ids && linear_src_row(p, m) < 0)) continue;
+                float v = acc[i][j][r];
+                if constexpr (EP == TILE_ANY) {
+                    linear_store(p, z, m, n, v);
+                    continue;
+                }
+                if constexpr (EP == TILE_BIAS_SILU) {
+                    v += bias;
+                    if (silu) v /= 1.0f + expf(-v);
+                }
+                const int64_t o = (int64_t)m * p.ldc + n + z * p.c_bs;
+                if (p.c_f32) ((float *)p.C)[o] = v;
+                else ((uint16_t *)p.C)[o] = vmx_f32_to_bf16(v);
+            }
+    }
+}
+
 // Up to 16 rows (decode steps, 16-row expert blocks): the product is a stream over the weights.  A workgroup owns 16 output
 // columns; its four waves split K in 128-deep blocks (wave w takes blocks w, w + 4, ...), lane (n, g) reads the 64 contiguous
 // bytes W[n][128 b + 32 g ..] of a block straight from memory, two blocks ahead of the one being multiplied, and the activation
@@ -342,6 +401,40 @@ __global__ __launch_bounds__(256) void linear_fewcols_f32_kernel(const VmxLinear
     if (tid < 16 && n0 + tid < p.N) linear_store(p, 0, m, n0 + tid, (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]));
 }
 
+// What linear_tile_kernel takes: bf16 rows in 16-byte chunks, whole 64-deep stages, operands (one batch) inside 32-bit byte offsets.
+bool tile_ok(const VmxLinear &p, bool direct) {
+    const int64_t a_rows = p.row_ids ? (p.row_limit + p.row_div - 1) / p.row_div : p.M;
+    return direct && !p.a_f32 && p.K % TG_BK == 0 && a_rows * p.lda * 2 < (int64_t)1 << 32 && (int64_t)p.N * p.w_sn * 2 < (int64_t)1 << 32 &&
+           p.lda >= 0 && p.w_sn >= 0;
+}
+
+template <class S, int EP>
+int launch_tile_as(const VmxLinear &p, hipStream_t st) {
+    const int row_tiles = (p.M + S::BM - 1) / S::BM, tiles = row_tiles * ((p.N + S::BN - 1) / S::BN);
+    static_assert(S::LDS <= 64 * 1024, "no attribute needed");
+    hipLaunchKernelGGL((linear_tile_kernel<S, EP>), dim3(tg_grid(tiles), p.batch), dim3(S::THREADS), S::LDS, st, p, row_tiles, tiles);
+    return VMX_OK;
+}
+
+template <class S>
+int launch_tile_shape(const VmxLinear &p, hipStream_t st) {
+    if (p.epilogue != VMX_EP_STORE || p.out_scale != 1.0f) return launch_tile_as<S, TILE_ANY>(p, st);
+    if (p.bias || p.silu_end > p.silu_begin) return launch_tile_as<S, TILE_BIAS_SILU>(p, st);
+    return launch_tile_as<S, TILE_PLAIN>(p, st);
+}
+
+// 128 x 128 tiles, two stages (two workgroups a compute unit) where there is one for every compute unit; else 64 x 64 tiles, with a
+// third stage where two or fewer of them share a unit and latency is all that counts.  us on 256 units, 128 x 128 / 64 x 64 in two / in
+// three stages:  1500 x 12288 x 2048 101 / 132 / 142;  1500 x 3664 x 2048 (348 tiles of 128) 35 / 45 / 45;  1500 x 2048 x 2048 (192)
+// 29 / 24 / 26;  100 x 12288 x 2048 (96) 27 / 19 / 17;  65 x 2048 x 2048 25 / 13 / 13.  Every shape adds an element's k in the same order.
+int launch_tile(const VmxLinear &p, hipStream_t st) {
+    const int64_t cus = vmx_num_cus();
+    const int64_t t128 = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch, t64 = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
+    if (!p.block_expert && t128 >= cus) return launch_tile_shape<TgShape<2, 2, 2, 2, 2>>(p, st);
+    if (t64 > 2 * cus) return launch_tile_shape<TgShape<2, 2, 1, 1, 2>>(p, st);
+    return launch_tile_shape<TgShape<2, 2, 1, 1, 3>>(p, st);
+}
+
 }  // namespace
 
 int vmx_linear_launch(const VmxLinear &p, hipStream_t st) {
@@ -367,7 +460,9 @@ int vmx_linear_launch(const VmxLinear &p, hipStream_t st) {
         // 16-byte loads straight from the operands: whole 8-element chunks, aligned rows
         const bool direct = p.w_sk == 1 && p.K % 8 == 0 && p.w_sn % 8 == 0 && p.lda % 8 == 0 && p.a_bs % 8 == 0 && p.w_bs % 8 == 0 &&
                             p.expert_stride % 8 == 0 && ((uintptr_t)p.W & 15) == 0 && ((uintptr_t)p.A & 31) == 0;
-        if (bm == 16 && direct) {
+        if (bm == 64 && tile_ok(p, direct)) {
+            if (int rc = launch_tile(p, st)) return rc;
+        } else if (bm == 16 && direct) {
             grid.x = (p.N + 15) / 16;
             hipLaunchKernelGGL(linear_skinny_kernel, grid, dim3(256), 0, st, p);
         } else if (bm == 16) hipLaunchKernelGGL(linear_mfma_kernel<16>, grid, dim3(256), 0, st, p);

@@ -1,0 +1,123 @@
+// Matrix-core GEMM core for prompt-sized products of 16-bit operands, C[m, n] = sum_k A[m, k] * B[n, k], both K-contiguous, f32
+// accumulation.  Shared by the bf16 linears (linear_generic.hip) and the integer form of the I-quant linears (split_gemm.hip).
+//
+// A workgroup owns a tile of C, a wave a part of it in 32 x 32 accumulators of v_mfma_f32_32x32x16 (TgShape).  What bounds such a kernel on gfx950 is everything beside the matrix cores, so:
+//   * both operand tiles (64 deep) go from global memory straight into LDS (global_load_lds, 16 bytes per lane: no registers, no
+//     vector-ALU work).  A staged row is 128 bytes, unpadded; the 16-byte chunk c of row r sits at position c ^ (r & 7), so the eight
+//     rows that a group of eight lanes reads lie in eight different bank groups;
+//   * two or three stages; the requests are issued by an instruction the compiler does not track (tg_request_1k), because behind one that it does it
+//     makes every LDS read wait for all requests under way, the other stage's included.  The waits are written out instead;
+//   * one barrier per stage, a later stage's requests right behind it;
+//   * tiles are numbered row-fastest and dealt to the eight XCDs in contiguous runs (workgroup i runs on XCD i % 8), so the rows of a
+//     column block are multiplied out of one XCD's L2.
+#pragma once
+#include "vmx_kernels.h"
+
+typedef float tg_f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 tg_f16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int TG_BK = 64;
+
+template <bool F16>
+__device__ __forceinline__ tg_f32x16 tg_mfma(uint4 a, uint4 b, tg_f32x16 c) {
+    if constexpr (F16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(tg_f16x8, a), __builtin_bit_cast(tg_f16x8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(vmx_bf16x8, a), __builtin_bit_cast(vmx_bf16x8, b), c, 0, 0, 0);
+}
+
+// Tile of workgroup `id` in a grid of tg_grid(tiles) workgroups, or -1.
+__device__ __forceinline__ int tg_tile(int id, int tiles) {
+    const int run = (tiles + 7) >> 3, t = (id & 7) * run + (id >> 3);
+    return t < tiles ? t : -1;
+}
+inline unsigned tg_grid(int tiles) { return (unsigned)((tiles + 7) / 8 * 8); }
+
+// Row of element r (0 .. 15) of a 32 x 32 accumulator in lane `lane` (its column is lane & 31).
+__device__ __forceinline__ int tg_acc_row(int lane, int r) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
+
+// 64 lanes x 16 bytes from base + off (per lane) to 1 KiB of LDS at `lds` (wave-uniform), in flight until vmcnt says otherwise.
+__device__ __forceinline__ void tg_request_1k(const void *lds, const char *base, uint32_t off) {
+    const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)lds);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(at), "v"(off), "s"(base) : "m0", "memory");
+}
+
+// Shape of a workgroup: WM x WN waves, each MI x NJ accumulators; STAGES tiles of both operands in LDS.
+template <int WM_, int WN_, int MI_, int NJ_, int STAGES_>
+struct TgShape {
+    static constexpr int WM = WM_, WN = WN_, MI = MI_, NJ = NJ_, STAGES = STAGES_;
+    static constexpr int BM = WM * MI * 32, BN = WN * NJ * 32, WAVES = WM * WN, THREADS = 64 * WAVES;
+    static constexpr int AQ = BM / (8 * WAVES), BQ = BN / (8 * WAVES);            // requests of eight rows a wave makes per operand and stage
+    static constexpr int STAGE = (BM + BN) * TG_BK, LDS = STAGES * STAGE * 2;     // elements, bytes
+    static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0 && STAGES >= 2, "whole requests per wave");
+};
+
+// Row of a tile that the lane fetches for request q of its wave (Q requests a wave), and the byte its chunk starts at in that row.
+template <int Q>
+__device__ __forceinline__ int tg_src_row(int wave, int lane, int q) { return (wave * Q + q) * 8 + (lane >> 3); }
+__device__ __forceinline__ uint32_t tg_src_byte(int lane) { return (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4); }
+
+template <int N>
+__device__ __forceinline__ void tg_wait_requests() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
+
+// The product over k in [0, K), K a positive multiple of 64.  a_src / b_src: byte offsets of the lane's chunks (tg_src_row, tg_src_byte)
+// from the uniform pointers A and B.  after(t): called when 64 deep step t has been multiplied.
+template <bool F16, class S, class After>
+__device__ __forceinline__ void tg_product(const char *A, const uint32_t (&a_src)[S::AQ], const char *B, const uint32_t (&b_src)[S::BQ], int K,
+                                           uint16_t *lds, int wave, int lane, tg_f32x16 (&acc)[S::MI][S::NJ], After &&after) {
+    constexpr int MI = S::MI, NJ = S::NJ, REQ = S::AQ + S::BQ, AHEAD = S::STAGES - 1;
+    const int fr = lane & 31, fh = lane >> 5, steps = K / TG_BK;
+    const int arow = ((wave / S::WN) * (MI * 32) + fr) * TG_BK, brow = S::BM * TG_BK + ((wave % S::WN) * (NJ * 32) + fr) * TG_BK;
+    auto request = [&](int t, uint16_t *stage) {
+#pragma unroll
+        for (int q = 0; q < S::AQ; q++) tg_request_1k(stage + (wave * S::AQ + q) * 8 * TG_BK, A + (int64_t)t * (2 * TG_BK), a_src[q]);
+#pragma unroll
+        for (int q = 0; q < S::BQ; q++) tg_request_1k(stage + (S::BM + (wave * S::BQ + q) * 8) * TG_BK, B + (int64_t)t * (2 * TG_BK), b_src[q]);
+    };
+    auto multiply = [&](const uint16_t *stage) {
+        uint4 af[2][MI], bf[2][NJ];   // fragments of the 16 deep step in use and of the next one
+        auto read = [&](int s) {
+            const int c = ((2 * s + fh) ^ (fr & 7)) << 3;
+#pragma unroll
+            for (int i = 0; i < MI; i++) af[s & 1][i] = *reinterpret_cast<const uint4 *>(stage + arow + i * 32 * TG_BK + c);
+#pragma unroll
+            for (int j = 0; j < NJ; j++) bf[s & 1][j] = *reinterpret_cast<const uint4 *>(stage + brow + j * 32 * TG_BK + c);
+        };
+        read(0);
+#pragma unroll
+        for (int s = 0; s < TG_BK / 16; s++) {
+            if (s + 1 < TG_BK / 16) read(s + 1);
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) acc[i][j] = tg_mfma<F16>(af[s & 1][i], bf[s & 1][j], acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);   // the reads stay ahead of the products they run under
+        }
+    };
+    // a step's stage is complete when this wave's share has landed and everybody has said so; behind that barrier nobody reads the
+    // previous step's stage any more, and the step AHEAD further on is requested into it
+    auto barrier = [&] {
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+#pragma unroll
+    for (int t = 0; t < AHEAD; t++)
+        if (t < steps) request(t, lds + t * S::STAGE);
+    int cur = 0, t = 0;
+    for (; t + AHEAD < steps; t++) {
+        tg_wait_requests<REQ *(AHEAD - 1)>();
+        barrier();
+        const int last = cur == 0 ? AHEAD : cur - 1;
+        request(t + AHEAD, lds + last * S::STAGE);
+        multiply(lds + cur * S::STAGE);
+        after(t);
+        cur = cur == AHEAD ? 0 : cur + 1;
+    }
+    for (; t < steps; t++) {
+        tg_wait_requests<0>();
+        barrier();
+        multiply(lds + cur * S::STAGE);
+        after(t);
+        cur = cur == AHEAD ? 0 : cur + 1;
+    }
+}
