@@ -37,3 +37,24 @@ def test_bf16_linear_tiles(gpu, M, N, K, out):
         bound = bound + 2.0 ** -8 * ref.abs()
     assert bool(((y.double() - ref).abs() <= bound).all())
     assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all())
+
+
+# rows around the 64- and 128-row tiles; columns around the 128-wide ones; K of one super-block, an odd number of them, and enough with
+# few tiles that the sums are cut into slices ((2048, 8192) gives the workspace room for them, (64, 256) does not)
+@pytest.mark.parametrize("M", [17, 64, 65, 129, 300])
+@pytest.mark.parametrize("ggml_type,N,K", [(18, 64, 256), (22, 129, 768), (21, 2048, 8192), (17, 2052, 7936)])
+def test_iq_prompt_linear_tiles(gpu, M, ggml_type, N, K):
+    """Against float64 on the dequantised weight: products of an fp16 activation and an integer are exact, 256 of them are added in
+    f32 (error (256 + 8) 2^-24 of the sum of magnitudes), scaled and added up in f32 again."""
+    vmx, torch = gpu
+    from tests.helpers import random_iq_blocks
+    ts = vmx.iq_type_size(ggml_type)
+    raw = torch.from_numpy(np.ascontiguousarray(random_iq_blocks(np.random.default_rng(N + K), ts, N * K // 256))).reshape(-1).cuda()
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
+    y = vmx.iq_gemm(ggml_type, raw, x, N)
+    torch.cuda.synchronize()
+    w = vmx.iq_dequantize(ggml_type, raw, N * K // 256).reshape(N, K).double()
+    ref = x.double() @ w.T
+    bound = (264 + K // 256 + 8) * 2.0 ** -24 * (x.double().abs() @ w.abs().T)
+    assert bool(((y.double() - ref).abs() <= bound).all())

@@ -399,6 +399,7 @@ struct vmx_gemma4 {
     int vocab_local() const { return cfg.tp_size > 1 ? cfg.vocab_size / cfg.tp_size : cfg.vocab_size; }
     float kv_headroom = 1.5f;   // DEFAULT_KV_HEADROOM_FACTOR (kv_cache/quantization.rs:108)
     Buf gemm_ws;                // dequantised weight of one projection (f32 + bf16 halves) for passes of more than 16 rows
+    Buf gemm_part;              // slice sums of a prompt-sized product with few tiles
     Buf a16;                    // fp16 copy of the rows a prompt-sized linear multiplies (the one-pass integer form)
     Buf kv_stage;               // bf16 K | V rows of one pass, used by an FP8 cache's first (calibrating) write
     int mmvq_mask = 15;         // measurement: which projections vmx_gemma4_mmvq_only launches (1 q|k|v, 2 o, 4 gate|up, 8 down)
@@ -460,24 +461,51 @@ bool g_split_always = false;   // measurement: prompt-sized linears always throu
 
 // A linear on `rows` token rows: the q8_1 MMVQ up to IQ_GEMV_MAX_M = 16 rows (activations already quantised in m->q8), beyond that
 // the reference's large-M form (gguf/mod.rs:358-365): dequantise the weight once, multiply the unquantised bf16 rows `a`.
+// a_is_f16: the rows are fp16 already (what g4_gateup_prompt leaves)
+bool int_form_ok(const IqLin &l, int rows) {
+    return vmx_iq_int_form_ok(l.ggml_type) && !g_split_always && vmx_int_gemm_ok(rows, l.out_features, l.in_features);
+}
+
+// m->gemm_ws = the integer form of the projections' weights, one behind the other
+int int_weights(vmx_gemma4 *m, const IqLin *const *lins, int n, int total, int K, hipStream_t st) {
+    for (int i = 0, row = 0; i < n; row += lins[i]->out_features, i++)
+        if (int rc = vmx_iq_dequant_int(lins[i]->ggml_type, lins[i]->raw.p, m->gemm_ws.p, row, lins[i]->out_features, total, K, st)) return rc;
+    return VMX_OK;
+}
+
 int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, const uint16_t *a, float *y, int ldy, int rows,
-               hipStream_t st) {
+               hipStream_t st, bool a_is_f16 = false) {
     if (rows <= 16) {
         if (n == 1 && offs[0] == 0) return mmvq(m, *lins[0], y, ldy, rows, st);
         return mmvq_group(m, lins, offs, n, y, ldy, rows, st);
     }
     // types whose dequantised weight is (f32 scale per super-block) x (integer that fp16 holds exactly) take one matrix-core pass
     // over fp16 activations; the others (IQ4_XS) the exact two-term bf16 split
-    bool a16_ready = false;
+    const int K = lins[0]->in_features;
+    int total = 0;
+    bool merge = true;
+    for (int i = 0; i < n; i++) {
+        merge = merge && int_form_ok(*lins[i], rows) && offs[i] == total;
+        total += lins[i]->out_features;
+    }
+    if (merge && vmx_int_gemm_ok(rows, total, K)) {   // one product over the projections' rows, one behind the other
+        if (int rc = int_weights(m, lins, n, total, K, st)) return rc;
+        const uint16_t *a16 = a;
+        if (!a_is_f16) {
+            if (int rc = vmx_bf16_rows_to_f16(a, (uint16_t *)m->a16.p, (int64_t)rows * K, st)) return rc;
+            a16 = (const uint16_t *)m->a16.p;
+        }
+        return vmx_int_gemm_f32(a16, m->gemm_ws.p, y, rows, total, K, ldy, (float *)m->gemm_part.p, st);
+    }
+    VMX_REQUIRE(!a_is_f16, "gemma4: fp16 rows for a projection without an integer form");
     for (int i = 0; i < n; i++) {
         const IqLin &l = *lins[i];
-        if (vmx_iq_int_form_ok(l.ggml_type) && !g_split_always) {
-            if (!a16_ready) {
-                if (int rc = vmx_bf16_rows_to_f16(a, (uint16_t *)m->a16.p, (int64_t)rows * l.in_features, st)) return rc;
-                a16_ready = true;
-            }
-            if (int rc = vmx_iq_dequant_int(l.ggml_type, l.raw.p, m->gemm_ws.p, l.out_features, l.in_features, st)) return rc;
-            if (int rc = vmx_int_gemm_f32((const uint16_t *)m->a16.p, m->gemm_ws.p, y + offs[i], rows, l.out_features, l.in_features, ldy, st))
+        if (int_form_ok(l, rows)) {
+            const IqLin *one[1] = {&l};
+            if (int rc = vmx_bf16_rows_to_f16(a, (uint16_t *)m->a16.p, (int64_t)rows * K, st)) return rc;
+            if (int rc = int_weights(m, one, 1, l.out_features, K, st)) return rc;
+            if (int rc = vmx_int_gemm_f32((const uint16_t *)m->a16.p, m->gemm_ws.p, y + offs[i], rows, l.out_features, K, ldy,
+                                          (float *)m->gemm_part.p, st))
                 return rc;
             continue;
         }
@@ -487,10 +515,26 @@ int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, 
     return VMX_OK;
 }
 
-int g4_linear(vmx_gemma4 *m, const IqLin &l, const uint16_t *a, float *y, int ldy, int rows, hipStream_t st) {
+int g4_linear(vmx_gemma4 *m, const IqLin &l, const uint16_t *a, float *y, int ldy, int rows, hipStream_t st, bool a_is_f16 = false) {
     const IqLin *one[1] = {&l};
     const int off[1] = {0};
-    return g4_linears(m, one, off, 1, a, y, ldy, rows, st);
+    return g4_linears(m, one, off, 1, a, y, ldy, rows, st, a_is_f16);
+}
+
+// Prompt-sized gate|up with the GeGLU in its epilogue: possible where gate, up and the down projection that reads the result (fp16 rows,
+// left in `act`) all have the integer form.
+bool gateup_prompt_ok(const G4Layer &L, int rows) {
+    const IqLin &g = L.lin[VMX_L_GATE], &u = L.lin[VMX_L_UP];
+    return rows > 16 && int_form_ok(g, rows) && int_form_ok(u, rows) && int_form_ok(L.lin[VMX_L_DOWN], rows) &&
+           vmx_int_gemm_ok(rows, g.out_features + u.out_features, g.in_features);
+}
+
+int g4_gateup_prompt(vmx_gemma4 *m, const G4Layer &L, const uint16_t *x, uint16_t *act, int rows, hipStream_t st) {
+    const IqLin *gu[2] = {&L.lin[VMX_L_GATE], &L.lin[VMX_L_UP]};
+    const int K = gu[0]->in_features, inter = gu[0]->out_features;
+    if (int rc = int_weights(m, gu, 2, 2 * inter, K, st)) return rc;
+    if (int rc = vmx_bf16_rows_to_f16(x, (uint16_t *)m->a16.p, (int64_t)rows * K, st)) return rc;
+    return vmx_int_gemm_geglu((const uint16_t *)m->a16.p, m->gemm_ws.p, act, rows, inter, K, st);
 }
 
 // Row-parallel linear under tensor parallelism: each rank's f32 output is rounded to bf16 (the reference's local matmul result),
@@ -679,7 +723,19 @@ extern "C" int vmx_gemma4_create(const vmx_gemma4_config *cfg, const int *layer_
             const size_t w = vmx_iq_gemm_workspace(LP, H);
             wmax = w > wmax ? w : wmax;
         }
+        // or of the integer forms of the projections that share a product
+        auto fits = [&](int n, int k) {
+            const size_t w = vmx_iq_gemm_int_weight_bytes(n, k);
+            wmax = w > wmax ? w : wmax;
+        };
+        for (const G4Layer &L : m->layers) {
+            fits(c.num_heads * L.hd + 2 * L.kvh * L.hd, H);
+            fits(2 * L.inter, H);
+            fits(H, c.num_heads * L.hd);
+            fits(H, L.inter);
+        }
         TRY(m->gemm_ws.alloc(wmax));
+        TRY(m->gemm_part.alloc(vmx_int_gemm_part_bytes()));
         int kmax = H;
         for (const G4Layer &L : m->layers)
             for (const IqLin &l : L.lin) kmax = l.in_features > kmax ? l.in_features : kmax;
@@ -735,7 +791,7 @@ extern "C" void vmx_gemma4_destroy(vmx_gemma4 *m) {
     }
     m->ple_model_proj.raw.release();
     m->ple_model_proj.packed.release();
-    for (Buf *b : {&m->ple_embed, &m->ple_proj_norm, &m->ple_e, &m->ple_p, &m->pli, &m->kv_stage, &m->red_bf16, &m->keys, &m->gemm_ws, &m->a16}) b->release();
+    for (Buf *b : {&m->ple_embed, &m->ple_proj_norm, &m->ple_e, &m->ple_p, &m->pli, &m->kv_stage, &m->red_bf16, &m->keys, &m->gemm_ws, &m->gemm_part, &m->a16}) b->release();
     for (Buf *b : {&m->embed, &m->final_norm, &m->cos_sin_s, &m->cos_sin_f, &m->positions, &m->h, &m->x, &m->q, &m->attn, &m->act, &m->proj, &m->out,
                    &m->logits, &m->logits_f32, &m->x_f32, &m->attn_ws, &m->argmax_ws, &m->q8, &m->q8b, &m->h2})
         b->release();
@@ -1002,6 +1058,8 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
                 m->q8_alt = nullptr;
                 return rc_glu;
             }
+        } else if (gateup_prompt_ok(L, B)) {
+            if (int rc = g4_gateup_prompt(m, L, x, act, B, st)) return rc;
         } else {
             const IqLin *gu[2] = {&L.lin[VMX_L_GATE], &L.lin[VMX_L_UP]};
             const int offs[2] = {0, I};
@@ -1010,7 +1068,7 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
             hipLaunchKernelGGL(g4_geglu_kernel, dim3((unsigned)(blocks > 1024 ? 1024 : blocks)), dim3(256), 0, st, proj, B, act, I, aq_of(m),
                                ad_of(m, B, I));
         }
-        const int rc_down = g4_linear(m, L.lin[VMX_L_DOWN], act, out, H, B, st);
+        const int rc_down = g4_linear(m, L.lin[VMX_L_DOWN], act, out, H, B, st, gateup_prompt_ok(L, B));
         m->q8_alt = nullptr;
         if (rc_down) return rc_down;
         if (tp)

@@ -129,11 +129,11 @@ __global__ __launch_bounds__(256) void iq_dequant_split_kernel(const uint8_t *__
 // Dequantise into the EXACT integer form of the prompt-sized GEMM.  A dequantised I-quant weight is d * c * I with d the f16
 // super-block scale, c a power of two and I = (2 ls + 1) * (signed codebook byte) an integer of at most 11 bits (IQ3_XXS: 31 * 62),
 // so I is exact in fp16 and the f32 product the reference forms (iq_dequant.cu: db * grid byte, no rounding: 11 + 5 + 6 bits)
-// equals (d * c) * I.  Q [rows][K] fp16 = I, Dt [K / 256][rows] f32 = d * c (transposed: a wave reads the scales of 16
+// equals (d * c) * I.  Q [rows][K] fp16 = I, Dt [K / 256][dt_ld] f32 = d * c (transposed: a wave reads the scales of 16
 // neighbouring columns in one line).  Same LDS staging of the stores as the split kernel.  Not for IQ4_XS (its integers need 13 bits).
 template <int T>
 __global__ __launch_bounds__(256) void iq_dequant_int_kernel(const uint8_t *__restrict__ blocks, uint16_t *__restrict__ Q,
-                                                              float *__restrict__ Dt, int64_t n_blocks, int rows, int nsb) {
+                                                              float *__restrict__ Dt, int64_t n_blocks, int dt_ld, int nsb) {
     __shared__ uint32_t cb[IqTraits<T>::LDS_WORDS];
     __shared__ uint2 sg[SignLut<T>::N];
     __shared__ __align__(16) uint16_t stage[256 * 32];
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void iq_dequant_int_kernel(const uint8_t *__re
             if (ib == 0) {
                 const float d = vmx_f16_to_f32((uint16_t)ld16(b));
                 const float c = (T == 17 || T == 22) ? 0.125f : (T == 18 ? 0.25f : 1.0f);
-                Dt[(blk % nsb) * rows + blk / nsb] = d * c;
+                Dt[(blk % nsb) * dt_ld + blk / nsb] = d * c;
             }
         }
         __syncthreads();
@@ -654,11 +654,11 @@ int vmx_iq_dequantize_split_bf16(int ggml_type, const void *blocks, uint16_t *hi
 
 bool vmx_iq_int_form_ok(int ggml_type) { return ggml_type == 17 || ggml_type == 18 || ggml_type == 21 || ggml_type == 22; }
 
-int vmx_iq_dequantize_int_f16(int ggml_type, const void *blocks, uint16_t *Q, float *Dt, int rows, int nsb, hipStream_t st) {
+int vmx_iq_dequantize_int_f16(int ggml_type, const void *blocks, uint16_t *Q, float *Dt, int rows, int dt_ld, int nsb, hipStream_t st) {
     const int64_t n_blocks = (int64_t)rows * nsb;
     if (n_blocks <= 0) return VMX_OK;
     const int grid = grid_for(n_blocks * 8, 256, 16384);
-#define CALL(T) hipLaunchKernelGGL((iq_dequant_int_kernel<T>), dim3(grid), dim3(256), 0, st, (const uint8_t *)blocks, Q, Dt, n_blocks, rows, nsb)
+#define CALL(T) hipLaunchKernelGGL((iq_dequant_int_kernel<T>), dim3(grid), dim3(256), 0, st, (const uint8_t *)blocks, Q, Dt, n_blocks, dt_ld, nsb)
     switch (ggml_type) {
         case 17: CALL(17); break;
         case 18: CALL(18); break;

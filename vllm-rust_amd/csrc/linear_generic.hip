@@ -263,7 +263,8 @@ __global__ __launch_bounds__(S::THREADS) void linear_tile_kernel(const VmxLinear
     for (int i = 0; i < S::MI; i++)
 #pragma unroll
         for (int j = 0; j < S::NJ; j++) acc[i][j] = tg_f32x16{};
-    tg_product<false, S>((const char *)((const uint16_t *)p.A + z * p.a_bs), a_src, (const char *)W, b_src, p.K, tg_lds, wave, lane, acc, [](int) {});
+    const TgCore<false, S> core{(const char *)((const uint16_t *)p.A + z * p.a_bs), (const char *)W, a_src, b_src, tg_lds, wave, lane};
+    tg_product(core, p.K, acc);
     const int wm = m0 + wave / S::WN * (S::MI * 32), wn = n0 + wave % S::WN * (S::NJ * 32) + (lane & 31);
 #pragma unroll
     for (int j = 0; j < S::NJ; j++) {

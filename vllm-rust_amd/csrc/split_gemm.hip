@@ -6,7 +6,7 @@
 // 2^-17 relative -- below the f32 summation noise of a dot over thousands of terms.
 #include <algorithm>
 #include "vmx_internal.h"
-#include "vmx_kernels.h"
+#include "tile_gemm.h"
 
 namespace {
 
@@ -99,107 +99,100 @@ __global__ __launch_bounds__(256) void split_gemm_kernel(const uint16_t *__restr
         }
 }
 
+// bf16 -> fp16, saturating at the largest finite half (a bf16 value inside fp16's normal range converts exactly; smaller ones
+// lose bits that are below 2^-24 in absolute terms)
+__device__ __forceinline__ uint16_t bf16_value_to_f16(uint16_t v) {
+    return __builtin_bit_cast(uint16_t, (_Float16)fminf(fmaxf(vmx_bf16_to_f32(v), -65504.0f), 65504.0f));
+}
+
 // The one-pass form for weights that are (f32 scale per super-block) x (small integer), see iq_dequant_int_kernel:
 // C[m, n] = sum_sb Dt[sb][n] * ( sum_{k in sb} A16[m, k] * Q[n, k] ), A16 = the activations as fp16 (bf16 values convert exactly
 // inside fp16's range), Q fp16 integers: every product is exact, the 256 products of a super-block are added in f32 by the matrix
 // core, and the scale is applied once per super-block to the finished sum -- the reference's f32 GEMM on the dequantised
-// weight up to summation order, at half the matrix instructions of the hi / lo split.  Same tiling as split_gemm_kernel;
-// KSPLIT: the four waves of a workgroup share one 64 x 64 tile and take the super-block ranges [nsb w / 4, nsb (w + 1) / 4).
-template <bool KSPLIT>
-__global__ __launch_bounds__(256) void int_gemm_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ Q,
-                                                        const float *__restrict__ Dt, float *__restrict__ C, int M, int N, int K, int ldc) {
-    typedef _Float16 sg_f16x8 __attribute__((ext_vector_type(8)));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int i = lane & 15, g = lane >> 4;
-    const int m0 = blockIdx.y * 64, n0 = KSPLIT ? blockIdx.x * 64 : blockIdx.x * 256 + wave * 64;
-    if (!KSPLIT && n0 >= N) return;
-    const int nsb = K >> 8;
-    const int sb_begin = KSPLIT ? (nsb * wave) / 4 : 0, sb_end = KSPLIT ? (nsb * (wave + 1)) / 4 : nsb;
-    int64_t arow[4], brow[4];
-    int dcol[4];
+// weight up to summation order.  On the tiles of tile_gemm.h; blockIdx.y = slice of super-blocks (few tiles: down_proj, o_proj, short
+// prompts), whose sums go to slices [M][N] of their own and are added in slice order by int_slices_kernel.
+// GEGLU: Q holds `inter` gate rows, then `inter` up rows; a tile takes 64 of each, side by side in every wave, and stores
+// act[m][i] = bf16(bf16(gelu_erf(bf16(gate))) * bf16(up)) as the fp16 operand of the next product (one slice).
+// Against one 16-byte operand load per lane straight from global memory (no LDS), 256 rows x 30720 x 3840 (gate|up): 222 -> 107 us (566 TFLOP/s).
+template <class S, bool GEGLU>
+__global__ __launch_bounds__(S::THREADS) void int_tile_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ Q,
+                                                               const float *__restrict__ Dt, float *__restrict__ C, uint16_t *__restrict__ act,
+                                                               int M, int N, int K, int64_t ldc, int row_tiles, int tiles, int per_slice) {
+    extern __shared__ __align__(16) uint16_t tg_lds[];
+    static_assert(!GEGLU || (S::WN == 2 && S::NJ == 2), "a wave holds 32 gate columns and the same 32 up columns");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tile = tg_tile(blockIdx.x, tiles);
+    if (tile < 0) return;
+    const int m0 = tile % row_tiles * S::BM, ct = tile / row_tiles, nsb = K >> 8, inter = N >> 1;
+    const int sb0 = blockIdx.y * per_slice, groups = min(per_slice, nsb - sb0);
+    // tile column -> row of Q
+    auto q_row = [&](int c) {
+        if constexpr (GEGLU) return (c & 32 ? inter : 0) + min(ct * 64 + (c >> 6) * 32 + (c & 31), inter - 1);
+        else return min(ct * S::BN + c, N - 1);
+    };
+    uint32_t a_src[S::AQ], b_src[S::BQ];
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-        arow[b] = (int64_t)min(m0 + b * 16 + i, M - 1) * K + 8 * g;
-        brow[b] = (int64_t)min(n0 + b * 16 + i, N - 1) * K + 8 * g;
-        dcol[b] = min(n0 + b * 16 + i, N - 1);
-    }
-    sg_f32x4 acc[4][4];
+    for (int q = 0; q < S::AQ; q++) a_src[q] = (uint32_t)((int64_t)min(m0 + tg_src_row<S::AQ>(wave, lane, q), M - 1) * K * 2) + tg_src_byte(lane);
 #pragma unroll
-    for (int rb = 0; rb < 4; rb++)
+    for (int q = 0; q < S::BQ; q++) b_src[q] = (uint32_t)((int64_t)q_row(tg_src_row<S::BQ>(wave, lane, q)) * K * 2) + tg_src_byte(lane);
+    const int wc = wave % S::WN * (S::NJ * 32) + (lane & 31);   // this lane's column of the tile (and 32 j further on)
+    int dcol[S::NJ];
 #pragma unroll
-        for (int cb = 0; cb < 4; cb++) acc[rb][cb] = sg_f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int sb = sb_begin; sb < sb_end; sb++) {
-        float dsc[4];
+    for (int j = 0; j < S::NJ; j++) dcol[j] = q_row(wc + 32 * j);
+    tg_f32x16 acc[S::MI][S::NJ];
 #pragma unroll
-        for (int cb = 0; cb < 4; cb++) dsc[cb] = Dt[(int64_t)sb * N + dcol[cb]];
-        sg_f32x4 tmp[4][4];
+    for (int i = 0; i < S::MI; i++)
 #pragma unroll
-        for (int rb = 0; rb < 4; rb++)
+        for (int j = 0; j < S::NJ; j++) acc[i][j] = tg_f32x16{};
+    const TgCore<true, S> core{(const char *)(A + sb0 * 256), (const char *)(Q + sb0 * 256), a_src, b_src, tg_lds, wave, lane};
+    tg_product_scaled(core, groups, acc, [&](int g, float (&d)[S::NJ]) {
 #pragma unroll
-            for (int cb = 0; cb < 4; cb++) tmp[rb][cb] = sg_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-        for (int k0 = sb * 256; k0 < sb * 256 + 256; k0 += 32) {
-            uint4 a[4], q[4];
+        for (int j = 0; j < S::NJ; j++) d[j] = Dt[(int64_t)(sb0 + g) * N + dcol[j]];
+    });
+    const int wm = m0 + wave / S::WN * (S::MI * 32);
+    if constexpr (GEGLU) {
+        const int col = ct * 64 + wave % S::WN * 32 + (lane & 31);
+        if (col >= inter) return;
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                a[b] = *reinterpret_cast<const uint4 *>(A + arow[b] + k0);
-                q[b] = *reinterpret_cast<const uint4 *>(Q + brow[b] + k0);
+        for (int i = 0; i < S::MI; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int m = wm + 32 * i + tg_acc_row(lane, r);
+                if (m >= M) continue;
+                const float g = vmx_bf16_to_f32(vmx_f32_to_bf16(acc[i][0][r])), u = vmx_bf16_to_f32(vmx_f32_to_bf16(acc[i][1][r]));
+                const float ge = vmx_bf16_to_f32(vmx_f32_to_bf16(0.5f * g * (1.0f + erff(g * 0.70710678118654752f))));
+                act[(int64_t)m * inter + col] = bf16_value_to_f16(vmx_f32_to_bf16(ge * u));
             }
+    } else {
+        float *out = C + (int64_t)blockIdx.y * M * ldc;
 #pragma unroll
-            for (int cb = 0; cb < 4; cb++)
+        for (int j = 0; j < S::NJ; j++) {
+            const int n = ct * S::BN + wc + 32 * j;
+            if (n >= N) continue;
 #pragma unroll
-                for (int rb = 0; rb < 4; rb++)
-                    tmp[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(sg_f16x8, a[rb]), __builtin_bit_cast(sg_f16x8, q[cb]),
-                                                                         tmp[rb][cb], 0, 0, 0);
+            for (int i = 0; i < S::MI; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int m = wm + 32 * i + tg_acc_row(lane, r);
+                    if (m < M) out[(int64_t)m * ldc + n] = acc[i][j][r];
+                }
         }
-#pragma unroll
-        for (int rb = 0; rb < 4; rb++)
-#pragma unroll
-            for (int cb = 0; cb < 4; cb++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[rb][cb][j] = fmaf(dsc[cb], tmp[rb][cb][j], acc[rb][cb][j]);
     }
-    if constexpr (KSPLIT) {
-        __shared__ sg_f32x4 red[4][4][4][64];   // [source wave][row block][column block][lane]: 64 KiB
-#pragma unroll
-        for (int rb = 0; rb < 4; rb++)
-#pragma unroll
-            for (int cb = 0; cb < 4; cb++) red[wave][rb][cb][lane] = acc[rb][cb];
-        __syncthreads();
-#pragma unroll
-        for (int cb = 0; cb < 4; cb++) {
-            sg_f32x4 t = red[0][wave][cb][lane];
-#pragma unroll
-            for (int w = 1; w < 4; w++) {
-                const sg_f32x4 o = red[w][wave][cb][lane];
-                t[0] += o[0]; t[1] += o[1]; t[2] += o[2]; t[3] += o[3];
-            }
-            const int col = n0 + cb * 16 + i;
-            if (col >= N) continue;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int row = m0 + wave * 16 + 4 * g + j;
-                if (row < M) C[(int64_t)row * ldc + col] = t[j];
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int rb = 0; rb < 4; rb++)
-#pragma unroll
-        for (int cb = 0; cb < 4; cb++) {
-            const int col = n0 + cb * 16 + i;
-            if (col >= N) continue;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int row = m0 + rb * 16 + 4 * g + j;
-                if (row < M) C[(int64_t)row * ldc + col] = acc[rb][cb][j];
-            }
-        }
 }
 
-// bf16 -> fp16, saturating at the largest finite half (a bf16 value inside fp16's normal range converts exactly; smaller ones
-// lose bits that are below 2^-24 in absolute terms)
+// y[m][n] (rows ldy apart) = the slices [slices][M][N] added in slice order; N % 4 == 0
+__global__ __launch_bounds__(256) void int_slices_kernel(const float *__restrict__ part, float *__restrict__ y, int slices, int M, int N, int64_t ldy) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, quads = (int64_t)M * N / 4;
+    if (i >= quads) return;
+    float4 v = reinterpret_cast<const float4 *>(part)[i];
+    for (int s = 1; s < slices; s++) {
+        const float4 o = reinterpret_cast<const float4 *>(part)[i + s * quads];
+        v.x += o.x, v.y += o.y, v.z += o.z, v.w += o.w;
+    }
+    const int64_t m = 4 * i / N, n = 4 * i - m * N;
+    *reinterpret_cast<float4 *>(y + m * ldy + n) = v;
+}
+
 __global__ __launch_bounds__(256) void bf16_to_f16_kernel(uint16_t *__restrict__ out, const uint16_t *__restrict__ in, int64_t n8) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += (int64_t)gridDim.x * 256) {
         const uint4 v = reinterpret_cast<const uint4 *>(in)[i];
@@ -207,9 +200,7 @@ __global__ __launch_bounds__(256) void bf16_to_f16_kernel(uint16_t *__restrict__
         uint32_t o[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const float a = fminf(fmaxf(__uint_as_float(w[j] << 16), -65504.0f), 65504.0f);
-            const float b = fminf(fmaxf(__uint_as_float(w[j] & 0xFFFF0000u), -65504.0f), 65504.0f);
-            o[j] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)b) << 16);
+            o[j] = (uint32_t)bf16_value_to_f16((uint16_t)w[j]) | ((uint32_t)bf16_value_to_f16((uint16_t)(w[j] >> 16)) << 16);
         }
         reinterpret_cast<uint4 *>(out)[i] = make_uint4(o[0], o[1], o[2], o[3]);
     }
@@ -295,14 +286,14 @@ int vmx_split_gemm_f32(const uint16_t *A, const void *workspace, float *C, int M
 }
 
 // ---- the integer form: workspace = Q fp16 [N*K] | Dt f32 [K/256][N] | A16 fp16 [M*K]
-size_t vmx_iq_gemm_int_workspace(int M, int N, int K) {
-    return (size_t)N * K * 2 + (((size_t)N * (K / 256) * 4 + 255) & ~(size_t)255) + (size_t)M * K * 2;
-}
+size_t vmx_iq_gemm_int_weight_bytes(int N, int K) { return (size_t)N * K * 2 + (((size_t)N * (K / 256) * 4 + 255) & ~(size_t)255); }
+size_t vmx_iq_gemm_int_workspace(int M, int N, int K) { return vmx_iq_gemm_int_weight_bytes(N, K) + (size_t)M * K * 2; }
 
-int vmx_iq_dequant_int(int ggml_type, const void *blocks, void *workspace, int N, int K, hipStream_t st) {
+// rows [row0, row0 + rows) of the integer form of N rows
+int vmx_iq_dequant_int(int ggml_type, const void *blocks, void *workspace, int row0, int rows, int N, int K, hipStream_t st) {
     uint16_t *Q = (uint16_t *)workspace;
     float *Dt = (float *)(Q + (int64_t)N * K);
-    return vmx_iq_dequantize_int_f16(ggml_type, blocks, Q, Dt, N, K / 256, st);
+    return vmx_iq_dequantize_int_f16(ggml_type, blocks, Q + (int64_t)row0 * K, Dt + row0, rows, N, K / 256, st);
 }
 
 // a16: fp16 copy of the activations (vmx_bf16_rows_to_f16), shared by the linears that read the same rows
@@ -314,15 +305,59 @@ int vmx_bf16_rows_to_f16(const uint16_t *A, uint16_t *a16, int64_t n, hipStream_
     return VMX_OK;
 }
 
-int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, hipStream_t st) {
+namespace {
+typedef TgShape<2, 2, 2, 2, 2> IntWide;     // 128 x 128
+typedef TgShape<2, 2, 1, 2, 2> IntMid;      // 64 x 128
+typedef TgShape<2, 2, 1, 1, 2> IntSmall;    // 64 x 64
+
+template <class S, bool GEGLU>
+void launch_int_tile(const uint16_t *a16, const uint16_t *Q, const float *Dt, float *C, uint16_t *act, int M, int N, int K, int64_t ldc, int slices,
+                     hipStream_t st) {
+    const int row_tiles = (M + S::BM - 1) / S::BM, tiles = row_tiles * (GEGLU ? (N / 2 + 63) / 64 : (N + S::BN - 1) / S::BN);
+    const int nsb = K / 256, per_slice = (nsb + slices - 1) / slices;
+    hipLaunchKernelGGL((int_tile_kernel<S, GEGLU>), dim3(tg_grid(tiles), (nsb + per_slice - 1) / per_slice), dim3(S::THREADS), S::LDS, st, a16, Q, Dt, C,
+                       act, M, N, K, ldc, row_tiles, tiles, per_slice);
+}
+
+// tiles of the plain form and the slices of super-blocks that give every compute unit about two workgroups
+int int_rows(int M) { return M > 64 ? 128 : 64; }
+int int_slices(int M, int N, int K) {
+    const int64_t tiles = (int64_t)((M + int_rows(M) - 1) / int_rows(M)) * ((N + 127) / 128), want = 2 * (int64_t)vmx_num_cus() / tiles;
+    const int nsb = K / 256;
+    if (want <= 1 || N % 4) return 1;
+    const int per = (int)((nsb + want - 1) / want);
+    return (nsb + per - 1) / per;
+}
+}  // namespace
+
+// most bytes of slice sums any call can want: two tiles of 128 x 128 a compute unit, and the tiles' overhang
+size_t vmx_int_gemm_part_bytes() { return (size_t)2 * vmx_num_cus() * 128 * 128 * 4; }
+
+bool vmx_int_gemm_ok(int M, int N, int K) { return (int64_t)M * K * 2 < (int64_t)1 << 32 && (int64_t)N * K * 2 < (int64_t)1 << 32; }
+
+// part: vmx_int_gemm_part_bytes() of scratch, or NULL (no slices).  ldy % 4 == 0 for slices.
+int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, float *part, hipStream_t st) {
     const uint16_t *Q = (const uint16_t *)workspace;
     const float *Dt = (const float *)(Q + (int64_t)N * K);
-    const int wide_wgs = ((N + 255) / 256) * ((M + 63) / 64);
-    if (wide_wgs < 2 * vmx_num_cus() && K >= 1024)
-        hipLaunchKernelGGL((int_gemm_kernel<true>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, st, a16, Q, Dt, C, M, N, K, ldc);
-    else
-        hipLaunchKernelGGL((int_gemm_kernel<false>), dim3((N + 255) / 256, (M + 63) / 64), dim3(256), 0, st, a16, Q, Dt, C, M, N, K, ldc);
+    const int slices = part && ldc % 4 == 0 ? int_slices(M, N, K) : 1;
+    float *to = slices > 1 ? part : C;
+    const int64_t ld = slices > 1 ? N : ldc;
+    if (int_rows(M) == 128) launch_int_tile<IntWide, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
+    else launch_int_tile<IntMid, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
+    if (slices > 1)
+        hipLaunchKernelGGL(int_slices_kernel, dim3((unsigned)(((int64_t)M * N / 4 + 255) / 256)), dim3(256), 0, st, part, C, slices, M, N, (int64_t)ldc);
     VMX_CHECK_LAUNCH("int_gemm");
+    return VMX_OK;
+}
+
+// act16 [M][inter] (fp16) of the gate rows and up rows that `workspace` holds one behind the other (N = 2 inter)
+int vmx_int_gemm_geglu(const uint16_t *a16, const void *workspace, uint16_t *act, int M, int inter, int K, hipStream_t st) {
+    const int N = 2 * inter;
+    const uint16_t *Q = (const uint16_t *)workspace;
+    const float *Dt = (const float *)(Q + (int64_t)N * K);
+    if (int_rows(M) == 128) launch_int_tile<IntWide, true>(a16, Q, Dt, nullptr, act, M, N, K, 0, 1, st);
+    else launch_int_tile<IntMid, true>(a16, Q, Dt, nullptr, act, M, N, K, 0, 1, st);
+    VMX_CHECK_LAUNCH("int_gemm(geglu)");
     return VMX_OK;
 }
 
@@ -339,12 +374,14 @@ extern "C" int vmx_iq_gemm_f32(int ggml_type, const void *blocks, const uint16_t
                 vmx_iq_gemm_workspace(n_out, n_in));
     if (m == 0) return VMX_OK;
     hipStream_t st = vmx_stream(stream);
-    if (vmx_iq_int_form_ok(ggml_type) && workspace_bytes >= vmx_iq_gemm_int_workspace(m, n_out, n_in)) {
-        // exact one-pass form: integer weights in fp16, one f32 scale per super-block
+    if (vmx_iq_int_form_ok(ggml_type) && workspace_bytes >= vmx_iq_gemm_int_workspace(m, n_out, n_in) && vmx_int_gemm_ok(m, n_out, n_in)) {
+        // exact one-pass form: integer weights in fp16, one f32 scale per super-block; slice sums where the workspace has room for them
         uint16_t *a16 = (uint16_t *)((char *)workspace + vmx_iq_gemm_int_workspace(0, n_out, n_in));
-        if (int rc = vmx_iq_dequant_int(ggml_type, blocks, workspace, n_out, n_in, st)) return rc;
+        const size_t used = (vmx_iq_gemm_int_workspace(m, n_out, n_in) + 255) & ~(size_t)255;
+        float *part = workspace_bytes >= used + vmx_int_gemm_part_bytes() ? (float *)((char *)workspace + used) : nullptr;
+        if (int rc = vmx_iq_dequant_int(ggml_type, blocks, workspace, 0, n_out, n_out, n_in, st)) return rc;
         if (int rc = vmx_bf16_rows_to_f16(x, a16, (int64_t)m * n_in, st)) return rc;
-        return vmx_int_gemm_f32(a16, workspace, y, m, n_out, n_in, n_out, st);
+        return vmx_int_gemm_f32(a16, workspace, y, m, n_out, n_in, n_out, part, st);
     }
     if (int rc = vmx_iq_dequant_split(ggml_type, blocks, workspace, n_out, n_in, st)) return rc;
     return vmx_split_gemm_f32(x, workspace, y, m, n_out, n_in, n_out, st);

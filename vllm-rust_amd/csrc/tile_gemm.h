@@ -57,67 +57,105 @@ template <int Q>
 __device__ __forceinline__ int tg_src_row(int wave, int lane, int q) { return (wave * Q + q) * 8 + (lane >> 3); }
 __device__ __forceinline__ uint32_t tg_src_byte(int lane) { return (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4); }
 
-template <int N>
-__device__ __forceinline__ void tg_wait_requests() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
+// What the two products below share: where a lane's fragments lie, the requests of one 64 deep step, the products of one stage.
+template <bool F16, class S>
+struct TgCore {
+    const char *A, *B;                       // uniform; the lane's chunks at a_src / b_src bytes from them (tg_src_row, tg_src_byte)
+    const uint32_t (&a_src)[S::AQ];
+    const uint32_t (&b_src)[S::BQ];
+    uint16_t *lds;
+    int wave, lane;
 
-// The product over k in [0, K), K a positive multiple of 64.  a_src / b_src: byte offsets of the lane's chunks (tg_src_row, tg_src_byte)
-// from the uniform pointers A and B.  after(t): called when 64 deep step t has been multiplied.
-template <bool F16, class S, class After>
-__device__ __forceinline__ void tg_product(const char *A, const uint32_t (&a_src)[S::AQ], const char *B, const uint32_t (&b_src)[S::BQ], int K,
-                                           uint16_t *lds, int wave, int lane, tg_f32x16 (&acc)[S::MI][S::NJ], After &&after) {
-    constexpr int MI = S::MI, NJ = S::NJ, REQ = S::AQ + S::BQ, AHEAD = S::STAGES - 1;
-    const int fr = lane & 31, fh = lane >> 5, steps = K / TG_BK;
-    const int arow = ((wave / S::WN) * (MI * 32) + fr) * TG_BK, brow = S::BM * TG_BK + ((wave % S::WN) * (NJ * 32) + fr) * TG_BK;
-    auto request = [&](int t, uint16_t *stage) {
+    __device__ __forceinline__ void request(int t, int stage) const {
+        uint16_t *to = lds + stage * S::STAGE;
 #pragma unroll
-        for (int q = 0; q < S::AQ; q++) tg_request_1k(stage + (wave * S::AQ + q) * 8 * TG_BK, A + (int64_t)t * (2 * TG_BK), a_src[q]);
+        for (int q = 0; q < S::AQ; q++) tg_request_1k(to + (wave * S::AQ + q) * 8 * TG_BK, A + (int64_t)t * (2 * TG_BK), a_src[q]);
 #pragma unroll
-        for (int q = 0; q < S::BQ; q++) tg_request_1k(stage + (S::BM + (wave * S::BQ + q) * 8) * TG_BK, B + (int64_t)t * (2 * TG_BK), b_src[q]);
-    };
-    auto multiply = [&](const uint16_t *stage) {
-        uint4 af[2][MI], bf[2][NJ];   // fragments of the 16 deep step in use and of the next one
+        for (int q = 0; q < S::BQ; q++) tg_request_1k(to + (S::BM + (wave * S::BQ + q) * 8) * TG_BK, B + (int64_t)t * (2 * TG_BK), b_src[q]);
+    }
+    // acc += the 64 deep products of a stage; FRESH: acc = them
+    template <bool FRESH = false>
+    __device__ __forceinline__ void multiply(int stage, tg_f32x16 (&acc)[S::MI][S::NJ]) const {
+        const uint16_t *from = lds + stage * S::STAGE;
+        const int fr = lane & 31, fh = lane >> 5;
+        const int arow = ((wave / S::WN) * (S::MI * 32) + fr) * TG_BK, brow = S::BM * TG_BK + ((wave % S::WN) * (S::NJ * 32) + fr) * TG_BK;
+        uint4 af[2][S::MI], bf[2][S::NJ];   // fragments of the 16 deep step in use and of the next one
         auto read = [&](int s) {
             const int c = ((2 * s + fh) ^ (fr & 7)) << 3;
 #pragma unroll
-            for (int i = 0; i < MI; i++) af[s & 1][i] = *reinterpret_cast<const uint4 *>(stage + arow + i * 32 * TG_BK + c);
+            for (int i = 0; i < S::MI; i++) af[s & 1][i] = *reinterpret_cast<const uint4 *>(from + arow + i * 32 * TG_BK + c);
 #pragma unroll
-            for (int j = 0; j < NJ; j++) bf[s & 1][j] = *reinterpret_cast<const uint4 *>(stage + brow + j * 32 * TG_BK + c);
+            for (int j = 0; j < S::NJ; j++) bf[s & 1][j] = *reinterpret_cast<const uint4 *>(from + brow + j * 32 * TG_BK + c);
         };
         read(0);
 #pragma unroll
         for (int s = 0; s < TG_BK / 16; s++) {
             if (s + 1 < TG_BK / 16) read(s + 1);
 #pragma unroll
-            for (int i = 0; i < MI; i++)
+            for (int i = 0; i < S::MI; i++)
 #pragma unroll
-                for (int j = 0; j < NJ; j++) acc[i][j] = tg_mfma<F16>(af[s & 1][i], bf[s & 1][j], acc[i][j]);
+                for (int j = 0; j < S::NJ; j++) acc[i][j] = tg_mfma<F16>(af[s & 1][i], bf[s & 1][j], FRESH && s == 0 ? tg_f32x16{} : acc[i][j]);
             __builtin_amdgcn_sched_barrier(0);   // the reads stay ahead of the products they run under
         }
-    };
-    // a step's stage is complete when this wave's share has landed and everybody has said so; behind that barrier nobody reads the
-    // previous step's stage any more, and the step AHEAD further on is requested into it
-    auto barrier = [&] {
+    }
+    // all but N of this wave's requests have landed, and everybody's of that step; nobody reads the step before it any more
+    template <int N>
+    __device__ __forceinline__ void arrive() const {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-    };
+    }
+};
+
+// acc += sum over k in [0, K), K a positive multiple of 64.
+template <bool F16, class S>
+__device__ __forceinline__ void tg_product(const TgCore<F16, S> &core, int K, tg_f32x16 (&acc)[S::MI][S::NJ]) {
+    constexpr int AHEAD = S::STAGES - 1;
+    const int steps = K / TG_BK;
 #pragma unroll
     for (int t = 0; t < AHEAD; t++)
-        if (t < steps) request(t, lds + t * S::STAGE);
+        if (t < steps) core.request(t, t);
     int cur = 0, t = 0;
     for (; t + AHEAD < steps; t++) {
-        tg_wait_requests<REQ *(AHEAD - 1)>();
-        barrier();
-        const int last = cur == 0 ? AHEAD : cur - 1;
-        request(t + AHEAD, lds + last * S::STAGE);
-        multiply(lds + cur * S::STAGE);
-        after(t);
+        core.template arrive<(S::AQ + S::BQ) * (AHEAD - 1)>();
+        core.request(t + AHEAD, cur == 0 ? AHEAD : cur - 1);
+        core.multiply(cur, acc);
         cur = cur == AHEAD ? 0 : cur + 1;
     }
     for (; t < steps; t++) {
-        tg_wait_requests<0>();
-        barrier();
-        multiply(lds + cur * S::STAGE);
-        after(t);
+        core.template arrive<0>();
+        core.multiply(cur, acc);
         cur = cur == AHEAD ? 0 : cur + 1;
+    }
+}
+
+// acc[m][n] += sum over groups of 256 k of scale(group, n) * (sum over the group's k), groups of them; two stages.
+// load(g, d): the lane's NJ scales of group g.
+template <bool F16, class S, class Load>
+__device__ __forceinline__ void tg_product_scaled(const TgCore<F16, S> &core, int groups, tg_f32x16 (&acc)[S::MI][S::NJ], Load &&load) {
+    static_assert(S::STAGES == 2, "the scales of a group are requested between two waits for everything");
+    const int steps = groups * 4;
+    if (steps > 0) core.request(0, 0);
+    for (int g = 0; g < groups; g++) {
+        tg_f32x16 part[S::MI][S::NJ];
+        float d[S::NJ];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            core.template arrive<0>();
+            if (u == 0) load(g, d);
+            if (u == 1) {   // a use right behind that wait: the compiler's own wait for the scales falls here, where it costs nothing
+#pragma unroll
+                for (int j = 0; j < S::NJ; j++) asm volatile("" : "+v"(d[j]));
+            }
+            if (4 * g + u + 1 < steps) core.request(4 * g + u + 1, (u + 1) & 1);
+            if (u == 0) core.template multiply<true>(0, part);
+            else core.multiply(u & 1, part);
+        }
+#pragma unroll
+        for (int i = 0; i < S::MI; i++)
+#pragma unroll
+            for (int j = 0; j < S::NJ; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[i][j][r] = fmaf(d[j], part[i][j][r], acc[i][j][r]);
     }
 }

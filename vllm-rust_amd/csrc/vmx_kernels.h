@@ -159,11 +159,16 @@ int vmx_iq_dequant_split(int ggml_type, const void *blocks, void *workspace, int
 int vmx_split_gemm_f32(const uint16_t *A, const void *workspace, float *C, int M, int N, int K, int ldc, hipStream_t st);
 // the exact one-pass form (weights = f32 super-block scale x fp16 integer; IQ2_XS, IQ2_S, IQ3_XXS, IQ3_S)
 bool vmx_iq_int_form_ok(int ggml_type);
-int vmx_iq_dequantize_int_f16(int ggml_type, const void *blocks, uint16_t *Q, float *Dt, int rows, int nsb, hipStream_t st);
+// Q [rows][nsb * 256], Dt [nsb][dt_ld]
+int vmx_iq_dequantize_int_f16(int ggml_type, const void *blocks, uint16_t *Q, float *Dt, int rows, int dt_ld, int nsb, hipStream_t st);
 size_t vmx_iq_gemm_int_workspace(int M, int N, int K);
-int vmx_iq_dequant_int(int ggml_type, const void *blocks, void *workspace, int N, int K, hipStream_t st);
+size_t vmx_iq_gemm_int_weight_bytes(int N, int K);
+int vmx_iq_dequant_int(int ggml_type, const void *blocks, void *workspace, int row0, int rows, int N, int K, hipStream_t st);
 int vmx_bf16_rows_to_f16(const uint16_t *A, uint16_t *a16, int64_t n, hipStream_t st);
-int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, hipStream_t st);
+bool vmx_int_gemm_ok(int M, int N, int K);
+size_t vmx_int_gemm_part_bytes();
+int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, float *part, hipStream_t st);
+int vmx_int_gemm_geglu(const uint16_t *a16, const void *workspace, uint16_t *act16, int M, int inter, int K, hipStream_t st);
 int vmx_dense_gemv_launch(uint16_t *y, const uint16_t *x, const uint16_t *W, const uint16_t *bias, int M, int N, int K, hipStream_t st,
                           int f16 = 0);   // f16: x, W, bias and y hold fp16 (same f32 accumulation, fp16 matrix / dot instructions)
 // bf16 matrix-core GEMM y = bf16(bf16(x @ W^T) + bias), W [N, K] bf16 (fp8_kernels.hip)
