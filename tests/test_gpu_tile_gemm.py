@@ -58,3 +58,28 @@ def test_iq_prompt_linear_tiles(gpu, M, ggml_type, N, K):
     ref = x.double() @ w.T
     bound = (264 + K // 256 + 8) * 2.0 ** -24 * (x.double().abs() @ w.abs().T)
     assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+# 256-column blocks; one k-block, odd numbers of them (17: a second step of the zero-point term; 33 in slices) and groups wider than a
+# k-block; rows around the 64-row tiles and past a strip of eight of them
+@pytest.mark.parametrize("M", [49, 64, 65, 200, 577])
+@pytest.mark.parametrize("N,K,group", [(256, 128, 128), (512, 2176, 128), (2304, 4224, 128), (256, 1536, 512), (256, 16384, 128)])
+def test_int4_prompt_tiles(gpu, M, N, K, group):
+    """Against float64 on (nibble - zero point) * scale.  The kernel adds x * (128 + nibble) and x * (128 + zero point) apart, in f32, so
+    their rounding is bounded by (k-block + k-blocks + 32) 2^-24 of sum |x| s (143 + 143); half a bf16 ulp for the result on top."""
+    vmx, torch = gpu
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
+    words = lambda *s: torch.randint(-2 ** 31, 2 ** 31 - 1, s, dtype=torch.int32, device="cuda", generator=g)   # noqa: E731
+    qw, qz = words(K // 8, N), words(K // group, N // 8)
+    sc = ((torch.rand((K // group, N), device="cuda", generator=g) + 0.5) * 0.01).to(torch.bfloat16)
+    bias = torch.randn(N, device="cuda", generator=g).to(torch.bfloat16)
+    y = vmx.int4_gemm(x, vmx.int4_pack(qw, sc, qz, K, N, group), bias, N, K, group)
+    torch.cuda.synchronize()
+    sh = torch.arange(0, 32, 4, dtype=torch.int32, device="cuda")
+    nib = ((qw.unsqueeze(-1) >> sh) & 15).permute(0, 2, 1).reshape(K, N)
+    zp = ((qz.unsqueeze(-1) >> sh) & 15).reshape(K // group, N).repeat_interleave(group, 0)
+    s = sc.double().repeat_interleave(group, 0)
+    ref = x.double() @ ((nib - zp).double() * s) + bias.double()
+    bound = 2.0 ** -8 * ref.abs() + (128 + K // 128 + 32) * 2.0 ** -24 * 286 * (x.double().abs() @ s)
+    assert bool(((y.double() - ref).abs() <= bound).all())

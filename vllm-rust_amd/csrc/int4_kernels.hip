@@ -18,7 +18,7 @@
 //   SZ [N/16][G][16] u32 : low half = bf16 scale bits, high half = bf16 bits of 128 + zp.
 // One wave-load is therefore 1 KiB contiguous = 16 columns x one 128-deep group slice,
 // and feeds four v_mfma_f32_16x16x32_bf16 (A = activations, rows = m).
-#include "vmx_kernels.h"
+#include "tile_gemm.h"
 #include <stdlib.h>
 
 namespace {
@@ -1249,17 +1249,22 @@ __global__ __launch_bounds__(256) void int4_gemm_tiled_kernel(const uint4 *__res
             }
 }
 
-// The same product with a 64-row x 256-column workgroup tile, built around what bounds the 64 x 128 form on gfx950 (its vector
-// ALU: staging, row sums and the per-k-block epilogue cost twice the cycles of its matrix instructions):
-//   * a wave owns FOUR column tiles (64 x 64 outputs): one A-fragment read from LDS feeds four matrix instructions;
-//   * the activation tile goes from global memory straight into LDS (global_load_lds, no registers, no vector-ALU work).
-//     Rows are 256 bytes unpadded; lane l of a 1 KiB request fills slot (row l / 16, position l % 16) with the row's 16-byte
-//     chunk  position ^ (row & 15), so the 16 rows a fragment read touches lie in 16 different bank groups;
-//   * the row sums of the zero-point term come from the matrix cores: wave w multiplies row tile w by a matrix of ones
-//     (4 extra instructions per k-block), leaves the 16 sums in LDS, and every wave applies  -(s (128 + zp)) * sum  one
-//     k-block later, after the barrier it needs anyway; the epilogue per k-block is two fused multiply-adds per element.
-// 1-D grid, ordered so that the row tiles of one column block are neighbours in time AND run on the same XCD (workgroup i
-// runs on XCD i % 8): the block's weights come from HBM once and from that XCD's L2 for the other row tiles.  N % 256 == 0.
+// The same product with a 64-row x 256-column workgroup tile: a wave owns 64 x 64 outputs in 2 x 2 accumulators of
+// v_mfma_f32_32x32x16_bf16, two workgroups share a compute unit.  The vector ALU (unpacking, group scales) and the matrix cores both
+// need most of the time a k-block takes, so what counts is that neither waits:
+//   * the activation tile goes from global memory straight into LDS, one k-block ahead (tg_request_1k: with a request the compiler tracks,
+//     it puts a wait for the NEXT tile in front of every LDS read of this one).  Rows are 256 bytes unpadded; chunk c of row r sits at
+//     position c ^ (r & 15), so the rows that eight lanes read lie in different bank groups;
+//   * weights go straight to registers, one k-block ahead.  A lane of the instruction's B operand is column l & 31: tile (l >> 4) & 1 of a
+//     pair, and of that tile's unit the words of the k chunks 2 t + (l >> 5) -- every byte of the unit is still used by one wave once;
+//   * fragments of the next 16 deep step are read and unpacked under the products of the current one;
+//   * the zero-point term -(s (128 + zp)) * (row sum of the k-block) costs no vector-ALU work per output: the row sums (a 16 x 16 matrix
+//     product with ones, wave w for rows 16 w ..) are kept in LDS for all k-blocks and multiplied with the factors at the end, 16 k-blocks
+//     per matrix step, both sides cut into bf16 parts that together hold all their bits (row sums three parts, factors two);
+//   * the scales of a finished pair of column tiles are applied under the other pair's products.
+// us against the form it replaces (64 x 64 per wave in 16 x 16 accumulators, every LDS read behind the next tile's arrival), rows x columns x
+// depth: 2048 x 24576 x 4096 545 -> 481 (857 TFLOP/s, matrix cores 56 % busy, 1.8 GHz), 333 x 24576 x 4096 124 -> 104, 100 x 24576 x 4096
+// 58 -> 42, 2048 x 4096 x 12288 267 -> 249.  N % 256 == 0.
 // (w & 0x000F000F) | base in one instruction (the compiler emits v_and + v_or: VOP3 takes no second literal)
 __device__ __forceinline__ uint32_t nib_pair(uint32_t w, uint32_t base) {
     uint32_t r;
@@ -1267,25 +1272,43 @@ __device__ __forceinline__ uint32_t nib_pair(uint32_t w, uint32_t base) {
     return r;
 }
 
+// v cut into bf16 parts: parts[0] + parts[1] + .. = v to the last bit that they hold
+template <int P>
+__device__ __forceinline__ void bf16_parts(float v, uint16_t (&part)[P]) {
+#pragma unroll
+    for (int i = 0; i < P; i++) {
+        part[i] = vmx_f32_to_bf16(v);
+        v -= vmx_bf16_to_f32(part[i]);
+    }
+}
+
 template <bool GLU, bool GROUPED = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void int4_gemm_tiled4_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void int4_gemm_prompt_kernel(
     const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ, const uint16_t *__restrict__ x, float *__restrict__ partial,
     uint16_t *__restrict__ act, int M, int N, int K, int group, int kb_per_split, int slice_rows, Int4GroupedArgs ga, int row_tiles,
-    uint16_t *__restrict__ ybf, const uint16_t *__restrict__ bias) {
+    int splits, uint16_t *__restrict__ ybf, const uint16_t *__restrict__ bias) {
     // ybf (one split only): the finished bf16 output y = bf16(sum + bias) instead of f32 slices
-    __shared__ __align__(16) uint16_t xs[2][PF_BM * KB];
-    __shared__ __align__(16) float sumx[2][PF_BM];
+    __shared__ __align__(256) uint16_t xs[2][PF_BM * KB];
     __shared__ int32_t prow_s[PF_BM];
+    extern __shared__ __align__(16) float row_sums[];   // [k-blocks of the slice, rounded up to 16][PF_BM]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nl = lane & 15, h = lane >> 4;
+    const int nl = lane & 15, ct = (lane >> 4) & 1, kh = lane >> 5;
     const int kblocks = K / KB, G = K / group;
-    const int col_blocks = N >> 8, cbg = (col_blocks + 7) >> 3;
-    // id -> (split, group of 8 column blocks, row tile, column block inside the group)
-    const int per_split = cbg * 8 * row_tiles;
-    const int ks = (int)blockIdx.x / per_split, rid = (int)blockIdx.x % per_split;
-    const int g8 = rid / (8 * row_tiles), rem = rid % (8 * row_tiles);
-    const int rt = rem >> 3, cb = g8 * 8 + (rem & 7);
-    if (cb >= col_blocks) return;
+    const int col_blocks = N >> 8;
+    int ks, rt, cb;
+    if constexpr (GROUPED) {
+        // an expert's row blocks share nothing with their neighbours but the columns: all of a column block's on one XCD
+        const int cbg = (col_blocks + 7) >> 3, per_split = cbg * 8 * row_tiles, rid = (int)blockIdx.x % per_split, rem = rid % (8 * row_tiles);
+        ks = (int)blockIdx.x / per_split, rt = rem >> 3, cb = rid / (8 * row_tiles) * 8 + (rem & 7);
+        if (cb >= col_blocks) return;
+    } else {
+        // strips of eight row tiles, column by column, dealt to the XCDs in contiguous runs: the 64 workgroups of an XCD are eight row
+        // tiles by eight column blocks, whose operands it fetches once into its L2
+        const int per_split = row_tiles * col_blocks, t = tg_tile(blockIdx.x, per_split * splits);
+        if (t < 0) return;
+        const int in_split = t % per_split, strip = in_split / (8 * col_blocks), rem = in_split - strip * 8 * col_blocks, height = min(8, row_tiles - strip * 8);
+        ks = t / per_split, cb = rem / height, rt = strip * 8 + rem % height;
+    }
     const int row0 = rt * PF_BM;
     const int nt0 = cb * 16 + wave * 4;   // this wave's four column tiles
     const int kb_begin = ks * kb_per_split, kb_end = min(kblocks, kb_begin + kb_per_split);
@@ -1305,7 +1328,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     // The four 1 KiB pieces of the activation tile this wave requests per k-block: piece q = rows 16 wave + 4 q .. + 3.  A row
     // past the end (or a padding pair) reads row 0: its outputs are never stored.
-    const uint16_t *xsrc[4];
+    uint32_t xsrc[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const int r = wave * 16 + q * 4 + (lane >> 4);
@@ -1316,141 +1339,206 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         } else {
             grow = row0 + r < M ? row0 + r : 0;
         }
-        xsrc[q] = x + grow * K + (((lane & 15) ^ (r & 15)) << 3);
+        xsrc[q] = (uint32_t)(grow * K * 2) + (uint32_t)(((lane & 15) ^ (r & 15)) << 4);
     }
+    const uint32_t w_at = (uint32_t)(ct * kblocks * 64 + kh * 16 + nl);   // of unit (nt0 + 2 j, kb); chunk pair t is 32 further on
+    const uint32_t sz_at = (uint32_t)(ct * G * 16 + nl);
 
-    vmx_f32x4 fin[4][4];
+    tg_f32x16 fin[2][2];
 #pragma unroll
-    for (int mt = 0; mt < 4; mt++)
+    for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int c = 0; c < 4; c++) fin[mt][c] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
-
-    uint4 wr[4];
-    uint32_t szr[4];
-    auto fetch = [&](int kb, int b) {
+        for (int j = 0; j < 2; j++) fin[i][j] = tg_f32x16{};
+    tg_u32x4 w[2][2];        // [column pair j][chunk pair t]
+    uint32_t sz[2];
+    const int gkb = group / KB;   // k-blocks that share a scale
+    const uint32_t xs_at = tg_lds_at(xs);   // a multiple of 256
+    auto fetch_x = [&](int kb, int stage) {
 #pragma unroll
         for (int q = 0; q < 4; q++)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(xsrc[q] + kb * KB),
-                                             (__attribute__((address_space(3))) void *)(&xs[b][(wave * 16 + q * 4) * KB]), 16, 0, 0);
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            wr[c] = W[((int64_t)(nt0 + c) * kblocks + kb) * 64 + lane];
-            szr[c] = SZ[((int64_t)(nt0 + c) * G + (kb * KB) / group) * 16 + nl];
-        }
+            tg_request_1k(xs_at + (stage * PF_BM + wave * 16 + q * 4) * (KB * 2), reinterpret_cast<const char *>(x) + (int64_t)kb * (KB * 2), xsrc[q]);
     };
-    if (kb_begin < kb_end) fetch(kb_begin, 0);
-    int buf = 0;
-    float nsz_prev[4] = {0.f, 0.f, 0.f, 0.f};   // -(s (128 + zp)) of the previous k-block
+    auto fetch_w = [&](int kb, int j) {   // three requests
+        const tg_u32x4 *unit = reinterpret_cast<const tg_u32x4 *>(W) + ((int64_t)(nt0 + 2 * j) * kblocks + kb) * 64;
+        w[j][0] = unit[w_at];
+        w[j][1] = unit[w_at + 32];
+        sz[j] = (SZ + ((int64_t)(nt0 + 2 * j) * G + (gkb == 1 ? kb : kb / gkb)) * 16)[sz_at];
+    };
+    // (w & nibbles) | base in one v_and_or_b32: one operand from a scalar, one from a vector register (an instruction takes no two literals)
+    uint32_t base = 0x43004300u, nibbles = 0x000F000Fu;
+    asm volatile("" : "+v"(base), "+s"(nibbles));
     const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
-    uint32_t base = 0x43004300u;
-    asm volatile("" : "+v"(base));   // kept in a vector register: the third operand of v_and_or_b32
-    // byte offset of this lane's A fragments inside a tile: row (mt * 16 + nl), chunk (4 i + h) at position chunk ^ nl
-    for (int kb = kb_begin; kb < kb_end; kb++) {
-        const uint4 wc[4] = {wr[0], wr[1], wr[2], wr[3]};
-        float sc[4], nsz[4];
+    const uint32_t a_first = xs_at + (lane & 31) * (KB * 2) + ((kh ^ nl) << 4);              // row l & 31 (and 32 further on), chunk kh
+    const uint32_t r_first = xs_at + (wave * 16 + nl) * (KB * 2) + (((lane >> 4) ^ nl) << 4);   // row 16 wave + nl, chunk l / 16
+    const int nkb = kb_end - kb_begin;
+    if (nkb > 0) {
+        fetch_x(kb_begin, 0);
+        fetch_w(kb_begin, 0);
+        fetch_w(kb_begin, 1);
+        // Requests run half a k-block ahead: the next tile and the next weights of pair 0 leave when pair 0 has been unpacked, the next
+        // weights of pair 1 when pair 1 has.  At the top everything but the latter (three requests) must have arrived.
+        tg_f32x16 acc0[2], acc1[2] = {tg_f32x16{}, tg_f32x16{}};   // a pair's sums of one k-block; pair 1's are scaled in the next block
+        float sc1 = 0.f;
+        for (int kb = kb_begin; kb < kb_end; kb++) {
+            const int stage = (kb - kb_begin) & 1, next = min(kb + 1, kb_end - 1);   // the last block requests itself again: the same counts everywhere
+            asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)" ::: "memory");
+            asm volatile("" : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(sz[0]));   // the compiler's own wait for pair 0 falls here, where it costs nothing
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            // chunk c of a row sits at position c ^ (row & 15), so the byte address of step s is that of step 0 with 32 s (64 s) flipped in
+            const uint32_t a_at = a_first + stage * (PF_BM * KB * 2), r_at = r_first + stage * (PF_BM * KB * 2);
+            tg_u32x4 au[2][2], bu[2];
+            auto read_a = [&](int s, tg_u32x4 (&d)[2]) {   // step s = 2 word + t: chunk 2 s + kh
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            sc[c] = __uint_as_float(szr[c] << 16);
-            nsz[c] = -sc[c] * __uint_as_float(szr[c] & 0xFFFF0000u);
+                for (int i = 0; i < 2; i++) d[i] = tg_lds_read((a_at ^ (32 * s)) + i * (32 * KB * 2));
+            };
+            auto unpack = [&](int j, int s) {
+                const uint32_t v = w[j][s & 1][s / 2];
+                return tg_u32x4{(v & nibbles) | base, ((v >> 4) & nibbles) | base, ((v >> 8) & nibbles) | base, ((v >> 12) & nibbles) | base};
+            };
+            // elements [32 e / n, 32 (e + 1) / n) of pair j's finished sums of a k-block, times its scale, into the result
+            auto scale_part = [&](int j, float sc, const tg_f32x16 (&acc)[2], int e, int n) {
+#pragma unroll
+                for (int r = 32 * e / n; r < 32 * (e + 1) / n; r++) fin[r >> 4][j][r & 15] = fmaf(sc, acc[r >> 4][r & 15], fin[r >> 4][j][r & 15]);
+                asm volatile("" : "+v"(fin[0][j]), "+v"(fin[1][j]));   // in this step, not in one heap at the end
+            };
+            read_a(0, au[0]);
+            bu[0] = unpack(0, 0);
+            vmx_f32x4 rs = {0.f, 0.f, 0.f, 0.f};   // sums of rows 16 wave ..
+            float sc0 = 0.f;
+            // One pair of column tiles after the other, 16 steps of two matrix products.  Every step also unpacks the next step's weights and
+            // scales a part of the pair before it (pair 1's of the previous k-block under pair 0, pair 0's under pair 1): about seven
+            // vector instructions behind each product, which is what fits under it.
+#pragma unroll
+            for (int u = 0; u < 16; u++) {
+                const int j = u >> 3, s = u & 7, at = u & 1;
+                // nothing moves over a step's start: pair 1 reads its fragments again instead of keeping sixteen of them in registers, and no
+                // unpacked weight waits longer than a step
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+                if (u == 7) asm volatile("" : "+v"(w[1][0]), "+v"(w[1][1]), "+v"(sz[1]));   // pair 1 is waited for here: nothing else is under way
+                if (u < 15) {
+                    read_a((s + 1) & 7, au[at ^ 1]);
+                    bu[at ^ 1] = unpack((u + 1) >> 3, (s + 1) & 7);
+                }
+                if (j == 0 && (s & 1)) {   // chunks 4 (s / 2) + lane / 16: 32 of the block's k
+                    const tg_u32x4 aw = tg_lds_read(r_at ^ (64 * (s / 2)));
+                    rs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, aw), __builtin_bit_cast(vmx_bf16x8, ones), rs, 0, 0, 0);
+                }
+                if (u == 7) {
+                    sc0 = __uint_as_float(sz[0] << 16);
+                    fetch_x(next, stage ^ 1);
+                    fetch_w(next, 0);
+                }
+                tg_f32x16(&acc)[2] = j ? acc1 : acc0;
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(vmx_bf16x8, au[at][i]), __builtin_bit_cast(vmx_bf16x8, bu[at]),
+                                                                     s == 0 ? tg_f32x16{} : acc[i], 0, 0, 0);
+                if (j == 0) scale_part(1, sc1, acc1, s, 8);
+                else if (s > 0) scale_part(0, sc0, acc0, s - 1, 7);
+                if (u == 15) {
+                    sc1 = __uint_as_float(sz[1] << 16);
+                    fetch_w(next, 1);
+                }
+            }
+            if (nl == 0) *reinterpret_cast<float4 *>(&row_sums[(kb - kb_begin) * PF_BM + wave * 16 + 4 * (lane >> 4)]) = make_float4(rs[0], rs[1], rs[2], rs[3]);
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the tile requested one iteration ago has landed in LDS
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) fin[i][1][r] = fmaf(sc1, acc1[i][r], fin[i][1][r]);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (kb + 1 < kb_end) fetch(kb + 1, buf ^ 1);   // next block's loads fly under this block's matrix work
-        const uint16_t *xb = xs[buf];
-
-        // zero-point term of the previous k-block (its row sums became visible with the barrier above)
-        if (kb > kb_begin) {
+        // zero-point term, 16 k-blocks a step: lane (row or column l & 31) holds k-blocks 16 t + 8 kh .. + 7
+        for (int t = 0; t < nkb; t += 16) {
+            uint4 bp[2][2];   // [column pair][part]
 #pragma unroll
-            for (int mt = 0; mt < 4; mt++) {
-                const float4 sx = *reinterpret_cast<const float4 *>(&sumx[buf ^ 1][mt * 16 + 4 * h]);
+            for (int j = 0; j < 2; j++) {
+                uint16_t q[8][2];
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    fin[mt][c][0] = fmaf(nsz_prev[c], sx.x, fin[mt][c][0]);
-                    fin[mt][c][1] = fmaf(nsz_prev[c], sx.y, fin[mt][c][1]);
-                    fin[mt][c][2] = fmaf(nsz_prev[c], sx.z, fin[mt][c][2]);
-                    fin[mt][c][3] = fmaf(nsz_prev[c], sx.w, fin[mt][c][3]);
+                for (int e = 0; e < 8; e++) {
+                    const int b = t + 8 * kh + e;
+                    const uint32_t z = b < nkb ? (SZ + ((int64_t)(nt0 + 2 * j) * G + (kb_begin + b) / gkb) * 16)[sz_at] : 0u;
+                    bf16_parts<2>(-__uint_as_float(z << 16) * __uint_as_float(z & 0xFFFF0000u), q[e]);
                 }
-            }
-        }
-        vmx_f32x4 acc[4][4];
 #pragma unroll
-        for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-            for (int c = 0; c < 4; c++) acc[mt][c] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
-        vmx_f32x4 rs = {0.f, 0.f, 0.f, 0.f};   // row sums of row tile `wave`
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            uint4 bu[4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const uint32_t w = i == 0 ? wc[c].x : (i == 1 ? wc[c].y : (i == 2 ? wc[c].z : wc[c].w));
-                bu[c].x = nib_pair(w, base);
-                bu[c].y = nib_pair(w >> 4, base);
-                bu[c].z = nib_pair(w >> 8, base);
-                bu[c].w = nib_pair(w >> 12, base);
-            }
-            {
-                const uint4 aw = *reinterpret_cast<const uint4 *>(xb + (wave * 16 + nl) * KB + (((4 * i + h) ^ nl) << 3));
-                rs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, aw), __builtin_bit_cast(vmx_bf16x8, ones), rs, 0, 0, 0);
+                for (int p = 0; p < 2; p++)
+                    bp[j][p] = make_uint4(q[0][p] | ((uint32_t)q[1][p] << 16), q[2][p] | ((uint32_t)q[3][p] << 16), q[4][p] | ((uint32_t)q[5][p] << 16),
+                                          q[6][p] | ((uint32_t)q[7][p] << 16));
             }
 #pragma unroll
-            for (int mt = 0; mt < 4; mt++) {
-                const uint4 au = *reinterpret_cast<const uint4 *>(xb + (mt * 16 + nl) * KB + (((4 * i + h) ^ nl) << 3));
+            for (int i = 0; i < 2; i++) {
+                uint16_t q[8][3];
 #pragma unroll
-                for (int c = 0; c < 4; c++)
-                    acc[mt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, au), __builtin_bit_cast(vmx_bf16x8, bu[c]),
-                                                                         acc[mt][c], 0, 0, 0);
-            }
-        }
-        if (nl == 0) *reinterpret_cast<float4 *>(&sumx[buf][wave * 16 + 4 * h]) = make_float4(rs[0], rs[1], rs[2], rs[3]);
+                for (int e = 0; e < 8; e++) {
+                    const int b = t + 8 * kh + e;
+                    bf16_parts<3>(b < nkb ? row_sums[b * PF_BM + i * 32 + (lane & 31)] : 0.f, q[e]);
+                }
 #pragma unroll
-        for (int mt = 0; mt < 4; mt++)
+                for (int p = 0; p < 3; p++) {
+                    const uint4 ap = make_uint4(q[0][p] | ((uint32_t)q[1][p] << 16), q[2][p] | ((uint32_t)q[3][p] << 16),
+                                                q[4][p] | ((uint32_t)q[5][p] << 16), q[6][p] | ((uint32_t)q[7][p] << 16));
 #pragma unroll
-            for (int c = 0; c < 4; c++)
+                    for (int j = 0; j < 2; j++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) fin[mt][c][r] = fmaf(sc[c], acc[mt][c][r], fin[mt][c][r]);
-#pragma unroll
-        for (int c = 0; c < 4; c++) nsz_prev[c] = nsz[c];
-        buf ^= 1;
-    }
-    if (kb_begin < kb_end) {   // zero-point term of the last k-block
-        __syncthreads();
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++) {
-            const float4 sx = *reinterpret_cast<const float4 *>(&sumx[buf ^ 1][mt * 16 + 4 * h]);
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                fin[mt][c][0] = fmaf(nsz_prev[c], sx.x, fin[mt][c][0]);
-                fin[mt][c][1] = fmaf(nsz_prev[c], sx.y, fin[mt][c][1]);
-                fin[mt][c][2] = fmaf(nsz_prev[c], sx.z, fin[mt][c][2]);
-                fin[mt][c][3] = fmaf(nsz_prev[c], sx.w, fin[mt][c][3]);
+                        for (int o = 0; o < 2; o++)
+                            fin[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(vmx_bf16x8, ap), __builtin_bit_cast(vmx_bf16x8, bp[j][o]),
+                                                                                fin[i][j], 0, 0, 0);
+                }
             }
         }
     }
+    // Outputs lie at a uniform row's start plus the lane's 32-bit offset (row 4 kh of an eight-row group, its column): no address
+    // arithmetic per element.  Row of element (i, r): 32 i + 8 (r / 4) + 4 kh + r % 4.
+    const bool whole = !GROUPED && row0 + PF_BM <= M;
+    auto row_ok = [&](int i, int r) {   // GROUPED: the pair the row belongs to (-1: padding), else 0 or -1
+        const int lr = i * 32 + tg_acc_row(lane, r);
+        if constexpr (GROUPED) return prow_s[lr];
+        else return whole || row0 + lr < M ? 0 : -1;
+    };
+    if constexpr (GLU) {
+        // Lanes 0 .. 7 of a row of 16 hold gate columns, lanes 8 .. 15 the up columns: of two neighbouring rows the former finish the
+        // first and the latter the second
+        const int half = N >> 1, odd = nl >> 3, col = nt0 * 8 + ct * 8 + (nl & 7);
+        const uint32_t off = (uint32_t)(((4 * kh + odd) * (int64_t)(GROUPED ? 0 : half) + col) * 2);
 #pragma unroll
-    for (int mt = 0; mt < 4; mt++)
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int c = 0; c < 4; c++)
+            for (int r = 0; r < 16; r += 2) {
+                const int p = odd ? row_ok(i, r + 1) : row_ok(i, r);
+                char *at = GROUPED ? reinterpret_cast<char *>(act) + (int64_t)max(p, 0) * half * 2
+                                   : reinterpret_cast<char *>(act) + (int64_t)(row0 + 32 * i + 8 * (r >> 2) + (r & 3)) * half * 2;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                int row = row0 + mt * 16 + 4 * h + r;
-                if constexpr (GROUPED) {
-                    const int p = prow_s[mt * 16 + 4 * h + r];
-                    row = p < 0 ? M : p;   // padding rows fail the bound check below (M = numel)
-                }
-                if constexpr (GLU) {
-                    const float up = vmx_lane_xor<8>(fin[mt][c][r]);
-                    if (row < M && nl < 8) {
-                        const float gg = vmx_bf16_to_f32(vmx_f32_to_bf16(fin[mt][c][r]));
-                        const float uu = vmx_bf16_to_f32(vmx_f32_to_bf16(up));
-                        act[(int64_t)row * (N >> 1) + (nt0 + c) * 8 + nl] = vmx_f32_to_bf16((gg / (1.0f + expf(-gg))) * uu);
-                    }
-                } else if (row < M) {
-                    const int n = (nt0 + c) * 16 + nl;
-                    if (ybf) ybf[(int64_t)row * N + n] = vmx_f32_to_bf16(bias ? fin[mt][c][r] + vmx_bf16_to_f32(bias[n]) : fin[mt][c][r]);
-                    else partial[((int64_t)ks * slice_rows + row) * N + n] = fin[mt][c][r];
+                for (int j = 0; j < 2; j++) {
+                    const float v0 = fin[i][j][r], v1 = fin[i][j][r + 1], other = vmx_lane_xor<8>(odd ? v0 : v1);
+                    const float gg = vmx_bf16_to_f32(vmx_f32_to_bf16(odd ? other : v0)), uu = vmx_bf16_to_f32(vmx_f32_to_bf16(odd ? v1 : other));
+                    const uint16_t y = vmx_f32_to_bf16((gg / (1.0f + expf(-gg))) * uu);
+                    if (p >= 0) *reinterpret_cast<uint16_t *>(at + off + j * 32) = y;
                 }
             }
+    } else {
+        const int col = (nt0 + ct) * 16 + nl;
+        const uint32_t off = (uint32_t)((GROUPED ? 0 : 4 * kh * (int64_t)N) + col);
+        const float b0 = ybf && bias ? vmx_bf16_to_f32(bias[col]) : 0.f, b1 = ybf && bias ? vmx_bf16_to_f32(bias[col + 32]) : 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int p = row_ok(i, r);
+                if (p < 0) continue;
+                const int64_t row = GROUPED ? p : row0 + 32 * i + 8 * (r >> 2) + (r & 3);
+                if (ybf) {
+                    char *at = reinterpret_cast<char *>(ybf + row * N);
+                    *reinterpret_cast<uint16_t *>(at + off * 2) = vmx_f32_to_bf16(fin[i][0][r] + b0);
+                    *reinterpret_cast<uint16_t *>(at + off * 2 + 64) = vmx_f32_to_bf16(fin[i][1][r] + b1);
+                } else {
+                    char *at = reinterpret_cast<char *>(partial + ((int64_t)ks * slice_rows + row) * N);
+                    *reinterpret_cast<float *>(at + off * 4) = fin[i][0][r];
+                    *reinterpret_cast<float *>(at + off * 4 + 128) = fin[i][1][r];
+                }
+            }
+    }
 }
 
 // Token-grouped form for a handful of rows per expert (decode batches): row block blockIdx.y = 16 sorted (token, slot) pairs
@@ -1765,20 +1853,22 @@ static bool tiled_ok(int M, int N, int K) {
     return !off && M >= min_m && N % 128 == 0;
 }
 
-// Launch of the prompt-shaped kernel: 64 x 256 workgroup tiles where N allows (VMX_INT4_TILED_WIDE=0 keeps 64 x 128 for A/B runs)
-static bool tiled_wide_ok(int N) {
+// Launch of the prompt-shaped kernel: 64 x 256 workgroup tiles where N allows, the row sums of a slice's kbs k-blocks fit beside the two
+// tiles in 64 KiB of LDS, and a row starts inside a 32-bit byte offset (VMX_INT4_TILED_WIDE=0 keeps 64 x 128 for A/B runs)
+static bool tiled_wide_ok(int M, int N, int K, int kbs) {
     static const bool wide = vmx_tune("VMX_INT4_TILED_WIDE", 1) != 0;
-    return wide && N % 256 == 0;
+    return wide && N % 256 == 0 && kbs <= 127 && (int64_t)M * K * 2 < (int64_t)1 << 32;
 }
 
 template <bool GLU, bool GROUPED>
 static void launch_tiled(const uint4 *W, const uint32_t *SZ, const uint16_t *x, float *partial, uint16_t *act, int M, int N, int K, int group,
                          int kbs, int slice_rows, const Int4GroupedArgs &ga, int row_tiles, int splits, hipStream_t st,
                          uint16_t *ybf = nullptr, const uint16_t *bias = nullptr) {
-    if (tiled_wide_ok(N)) {
-        const int cbg = ((N >> 8) + 7) >> 3;
-        hipLaunchKernelGGL((int4_gemm_tiled4_kernel<GLU, GROUPED>), dim3(cbg * 8 * row_tiles * splits), dim3(256), 0, st, W, SZ, x, partial, act, M, N,
-                           K, group, kbs, slice_rows, ga, row_tiles, ybf, bias);
+    if (tiled_wide_ok(M, N, K, kbs)) {
+        const unsigned grid = GROUPED ? (unsigned)(((N >> 8) + 7) / 8 * 8 * row_tiles * splits) : tg_grid((N >> 8) * row_tiles * splits);
+        const size_t sums = (size_t)kbs * PF_BM * 4;
+        hipLaunchKernelGGL((int4_gemm_prompt_kernel<GLU, GROUPED>), dim3(grid), dim3(256), sums, st, W, SZ, x, partial, act, M, N,
+                           K, group, kbs, slice_rows, ga, row_tiles, splits, ybf, bias);
     } else {
         hipLaunchKernelGGL((int4_gemm_tiled_kernel<GLU, GROUPED>), dim3(N / 128, row_tiles, splits), dim3(256), 0, st, W, SZ, x, partial, act, M, N,
                            K, group, kbs, slice_rows, ga);
@@ -2210,12 +2300,12 @@ extern "C" int vmx_int4_gemm_bf16(uint16_t *y, const uint16_t *x, const void *pa
         const int kblocks = K / KB, row_tiles = (M + PF_BM - 1) / PF_BM;
         // split-K only while the tiles alone leave compute units idle (the plan's slice count is sized for one row tile)
         int splits = p.splits;
-        if (tiled_wide_ok(N)) {
+        if (tiled_wide_ok(M, N, K, 1)) {
             const int tiles = (N >> 8) * row_tiles, want = (2 * vmx_num_cus() + tiles - 1) / tiles;
             splits = want < splits ? (want < 1 ? 1 : want) : splits;
         }
         const int kbs = (kblocks + splits - 1) / splits;
-        if (splits == 1 && tiled_wide_ok(N)) {   // one slice: the kernel writes the bf16 output itself
+        if (splits == 1 && tiled_wide_ok(M, N, K, kbs)) {   // one slice: the kernel writes the bf16 output itself
             launch_tiled<false, false>(W, SZ, x, nullptr, nullptr, M, N, K, group, kbs, M, Int4GroupedArgs{}, row_tiles, 1, st, y, bias);
             VMX_CHECK_LAUNCH("int4_gemm(tiled)");
             return VMX_OK;

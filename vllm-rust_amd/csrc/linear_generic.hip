@@ -240,7 +240,7 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const VmxLinear p) {
 enum { TILE_PLAIN, TILE_BIAS_SILU, TILE_ANY };
 template <class S, int EP>
 __global__ __launch_bounds__(S::THREADS) void linear_tile_kernel(const VmxLinear p, int row_tiles, int tiles) {
-    extern __shared__ __align__(16) uint16_t tg_lds[];
+    extern __shared__ __align__(1024) uint16_t tg_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tile = tg_tile(blockIdx.x, tiles), z = blockIdx.y;
     if (tile < 0) return;
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(S::THREADS) void linear_tile_kernel(const VmxLinear
     for (int i = 0; i < S::MI; i++)
 #pragma unroll
         for (int j = 0; j < S::NJ; j++) acc[i][j] = tg_f32x16{};
-    const TgCore<false, S> core{(const char *)((const uint16_t *)p.A + z * p.a_bs), (const char *)W, a_src, b_src, tg_lds, wave, lane};
+    const TgCore<false, S> core{(const char *)((const uint16_t *)p.A + z * p.a_bs), (const char *)W, a_src, b_src, tg_lds_at(tg_lds), wave, lane};
     tg_product(core, p.K, acc);
     const int wm = m0 + wave / S::WN * (S::MI * 32), wn = n0 + wave % S::WN * (S::NJ * 32) + (lane & 31);
 #pragma unroll

@@ -118,7 +118,7 @@ template <class S, bool GEGLU>
 __global__ __launch_bounds__(S::THREADS) void int_tile_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ Q,
                                                                const float *__restrict__ Dt, float *__restrict__ C, uint16_t *__restrict__ act,
                                                                int M, int N, int K, int64_t ldc, int row_tiles, int tiles, int per_slice) {
-    extern __shared__ __align__(16) uint16_t tg_lds[];
+    extern __shared__ __align__(1024) uint16_t tg_lds[];
     static_assert(!GEGLU || (S::WN == 2 && S::NJ == 2), "a wave holds 32 gate columns and the same 32 up columns");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tile = tg_tile(blockIdx.x, tiles);
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(S::THREADS) void int_tile_kernel(const uint16_t *__
     for (int i = 0; i < S::MI; i++)
 #pragma unroll
         for (int j = 0; j < S::NJ; j++) acc[i][j] = tg_f32x16{};
-    const TgCore<true, S> core{(const char *)(A + sb0 * 256), (const char *)(Q + sb0 * 256), a_src, b_src, tg_lds, wave, lane};
+    const TgCore<true, S> core{(const char *)(A + sb0 * 256), (const char *)(Q + sb0 * 256), a_src, b_src, tg_lds_at(tg_lds), wave, lane};
     tg_product_scaled(core, groups, acc, [&](int g, float (&d)[S::NJ]) {
 #pragma unroll
         for (int j = 0; j < S::NJ; j++) d[j] = Dt[(int64_t)(sb0 + g) * N + dcol[j]];

@@ -15,11 +15,12 @@
 
 typedef float tg_f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 tg_f16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t tg_u32x4 __attribute__((ext_vector_type(4)));   // a native vector: HIP's uint4 in arrays ends in scratch or in 4-byte LDS reads
 
 constexpr int TG_BK = 64;
 
 template <bool F16>
-__device__ __forceinline__ tg_f32x16 tg_mfma(uint4 a, uint4 b, tg_f32x16 c) {
+__device__ __forceinline__ tg_f32x16 tg_mfma(tg_u32x4 a, tg_u32x4 b, tg_f32x16 c) {
     if constexpr (F16)
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(tg_f16x8, a), __builtin_bit_cast(tg_f16x8, b), c, 0, 0, 0);
     else
@@ -36,9 +37,14 @@ inline unsigned tg_grid(int tiles) { return (unsigned)((tiles + 7) / 8 * 8); }
 // Row of element r (0 .. 15) of a 32 x 32 accumulator in lane `lane` (its column is lane & 31).
 __device__ __forceinline__ int tg_acc_row(int lane, int r) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
-// 64 lanes x 16 bytes from base + off (per lane) to 1 KiB of LDS at `lds` (wave-uniform), in flight until vmcnt says otherwise.
-__device__ __forceinline__ void tg_request_1k(const void *lds, const char *base, uint32_t off) {
-    const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)lds);
+// LDS byte address of a __shared__ array (taken once: the cast of a pointer computed from it costs a null check each time)
+__device__ __forceinline__ uint32_t tg_lds_at(const void *array) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)array; }
+// 16 bytes of LDS at a byte address
+__device__ __forceinline__ tg_u32x4 tg_lds_read(uint32_t at) { return *(const __attribute__((address_space(3))) tg_u32x4 *)(uintptr_t)at; }
+
+// 64 lanes x 16 bytes from base + off (per lane) to the 1 KiB of LDS from byte `at` on (wave-uniform), in flight until vmcnt says otherwise.
+__device__ __forceinline__ void tg_request_1k(uint32_t at, const char *base, uint32_t off) {
+    at = __builtin_amdgcn_readfirstlane(at);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(at), "v"(off), "s"(base) : "m0", "memory");
 }
 
@@ -63,29 +69,30 @@ struct TgCore {
     const char *A, *B;                       // uniform; the lane's chunks at a_src / b_src bytes from them (tg_src_row, tg_src_byte)
     const uint32_t (&a_src)[S::AQ];
     const uint32_t (&b_src)[S::BQ];
-    uint16_t *lds;
+    uint32_t lds;                            // byte address of the stages (tg_lds_at)
     int wave, lane;
 
     __device__ __forceinline__ void request(int t, int stage) const {
-        uint16_t *to = lds + stage * S::STAGE;
+        const uint32_t to = lds + stage * (S::STAGE * 2);
 #pragma unroll
-        for (int q = 0; q < S::AQ; q++) tg_request_1k(to + (wave * S::AQ + q) * 8 * TG_BK, A + (int64_t)t * (2 * TG_BK), a_src[q]);
+        for (int q = 0; q < S::AQ; q++) tg_request_1k(to + (wave * S::AQ + q) * (8 * TG_BK * 2), A + (int64_t)t * (2 * TG_BK), a_src[q]);
 #pragma unroll
-        for (int q = 0; q < S::BQ; q++) tg_request_1k(to + (S::BM + (wave * S::BQ + q) * 8) * TG_BK, B + (int64_t)t * (2 * TG_BK), b_src[q]);
+        for (int q = 0; q < S::BQ; q++) tg_request_1k(to + (S::BM + (wave * S::BQ + q) * 8) * (TG_BK * 2), B + (int64_t)t * (2 * TG_BK), b_src[q]);
     }
     // acc += the 64 deep products of a stage; FRESH: acc = them
     template <bool FRESH = false>
     __device__ __forceinline__ void multiply(int stage, tg_f32x16 (&acc)[S::MI][S::NJ]) const {
-        const uint16_t *from = lds + stage * S::STAGE;
-        const int fr = lane & 31, fh = lane >> 5;
-        const int arow = ((wave / S::WN) * (S::MI * 32) + fr) * TG_BK, brow = S::BM * TG_BK + ((wave % S::WN) * (S::NJ * 32) + fr) * TG_BK;
-        uint4 af[2][S::MI], bf[2][S::NJ];   // fragments of the 16 deep step in use and of the next one
+        // byte addresses of step 0; chunk c lies at c ^ (row & 7), so step s is step 0 with 32 s flipped in
+        const int fr = lane & 31, first = (((lane >> 5) ^ (fr & 7)) << 4);
+        const uint32_t from = lds + stage * (S::STAGE * 2);
+        const uint32_t arow = from + ((wave / S::WN) * (S::MI * 32) + fr) * (TG_BK * 2) + first;
+        const uint32_t brow = from + (S::BM + (wave % S::WN) * (S::NJ * 32) + fr) * (TG_BK * 2) + first;
+        tg_u32x4 af[2][S::MI], bf[2][S::NJ];   // fragments of the 16 deep step in use and of the next one
         auto read = [&](int s) {
-            const int c = ((2 * s + fh) ^ (fr & 7)) << 3;
 #pragma unroll
-            for (int i = 0; i < S::MI; i++) af[s & 1][i] = *reinterpret_cast<const uint4 *>(from + arow + i * 32 * TG_BK + c);
+            for (int i = 0; i < S::MI; i++) af[s & 1][i] = tg_lds_read((arow ^ (32 * s)) + i * (32 * TG_BK * 2));
 #pragma unroll
-            for (int j = 0; j < S::NJ; j++) bf[s & 1][j] = *reinterpret_cast<const uint4 *>(from + brow + j * 32 * TG_BK + c);
+            for (int j = 0; j < S::NJ; j++) bf[s & 1][j] = tg_lds_read((brow ^ (32 * s)) + j * (32 * TG_BK * 2));
         };
         read(0);
 #pragma unroll
