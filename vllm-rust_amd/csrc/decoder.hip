@@ -635,7 +635,6 @@ struct vmx_qwen3 {
     bool lm_head_tied = false;
     DevBuf h, x, q, attn, act, partial, partial_b, logits, attn_ws, argmax_ws, red_bf16, keys, q8, positions, ssq;
     DevBuf router_logits, topk_w, topk_ids, moe_ws, moe_out;   // MoE models only
-    DevBuf dense_tmp;                                          // unquantized layers only: bf16 [16][widest projection], grown by the loader
     DevBuf exl3_ws;                                            // EXL3 models only: grown by the loader
     vmx_comm *comm = nullptr;  // tensor-parallel group (not owned); NULL = single GPU
     int lin_mask = 15;  // measurement aid: which linears vmx_qwen3_linears_only launches (1 q|k|v, 2 o, 4 gate|up, 8 down)
@@ -704,24 +703,14 @@ int exl3_forward_group(vmx_qwen3 *m, const Layer &L, std::initializer_list<int> 
                                       m->exl3_ws.p, m->exl3_ws.bytes, st, partial_out, splits_out, norm_w, blk_ssq, eps, attn_parts);
 }
 
-__global__ __launch_bounds__(256) void bf16_rows_to_f32_kernel(const uint16_t *__restrict__ in, float *__restrict__ out, int rows, int cols,
-                                                                 int ldo) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < (int64_t)rows * cols) out[(i / cols) * ldo + (i % cols)] = vmx_bf16_to_f32(in[i]);
-}
-
-// Unquantized Linear (no bias) on decode / prompt rows: y = bf16(x W^T), 16 rows per launch, widened to the f32 form the
-// vector kernels take with one slice (they round to bf16 again, which changes nothing).
-int dense_forward(vmx_qwen3 *m, const void *W, const uint16_t *x, float *y, int ldy, int N, int K, int tokens, hipStream_t st) {
-    uint16_t *tmp = (uint16_t *)m->dense_tmp.p;
-    for (int r0 = 0; r0 < tokens; r0 += 16) {
-        const int mr = tokens - r0 < 16 ? tokens - r0 : 16;
-        if (int rc = vmx_dense_gemv_launch(tmp, x + (size_t)r0 * K, (const uint16_t *)W, nullptr, mr, N, K, st)) return rc;
-        const int64_t n = (int64_t)mr * N;
-        hipLaunchKernelGGL(bf16_rows_to_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, tmp, y + (size_t)r0 * ldy, mr, N, ldy);
-    }
-    VMX_CHECK_LAUNCH("dense_forward");
-    return VMX_OK;
+// Unquantized Linear (no bias): y = x W^T as one f32 slice, which its consumers round to bf16.  Up to 16 rows: the decode kernel, one
+// launch (the GEMV with bf16 results and a kernel that widened them took 12 + 5 us for q|k|v of Qwen3-0.6B at one row); prompts: the
+// tiled linears, which read the weights once per 128 rows and not once per 16.
+int dense_forward(const void *W, const uint16_t *x, float *y, int N, int K, int tokens, hipStream_t st) {
+    if (vmx_dense_decode_ok(tokens, N, K)) return vmx_dense_decode_f32(y, x, (const uint16_t *)W, tokens, N, K, st);
+    VmxLinear p;
+    p.A = x, p.lda = K, p.W = (const uint16_t *)W, p.w_sn = K, p.w_sk = 1, p.C = y, p.c_f32 = 1, p.ldc = N, p.M = tokens, p.N = N, p.K = K;
+    return vmx_linear_launch(p, st);
 }
 
 // Row-parallel epilogue: red_bf16 = all_reduce_sum(bf16(sum of this rank's split-K slices)) — what composing the
@@ -911,7 +900,7 @@ extern "C" int vmx_qwen3_create(const vmx_qwen3_config *cfg, vmx_qwen3 **out) {
     TRY(m->act.alloc((size_t)B * I * 2));
     TRY(m->logits.alloc((size_t)c.max_batch * VL * 2));
     TRY(m->positions.alloc((size_t)B * 4));
-    TRY(m->ssq.alloc((size_t)4 * (H / 16 + 4) * 4));   // per-tile sums of squares of up to four decode rows
+    TRY(m->ssq.alloc((size_t)16 * (H / 16 + 4) * 4));   // per-tile sums of squares of up to sixteen decode rows
     TRY(m->red_bf16.alloc((size_t)B * H * 2));
     {   // q8_1 staging for I-quant linears: int8 [B][Kmax] + f32 [B][Kmax/32]
         const size_t kmax = (size_t)(H > I ? (H > NO ? H : NO) : (I > NO ? I : NO));
@@ -963,7 +952,7 @@ extern "C" void vmx_qwen3_destroy(vmx_qwen3 *m) {
     }
     for (DevBuf *b : {&m->embed, &m->lm_head, &m->final_norm, &m->cos_sin, &m->h, &m->x, &m->q, &m->attn, &m->act, &m->partial, &m->partial_b,
                       &m->logits, &m->attn_ws, &m->argmax_ws, &m->red_bf16, &m->keys, &m->q8, &m->positions, &m->router_logits, &m->topk_w, &m->topk_ids,
-                      &m->moe_ws, &m->moe_out, &m->exl3_ws, &m->ssq, &m->dense_tmp})
+                      &m->moe_ws, &m->moe_out, &m->exl3_ws, &m->ssq})
         b->release();
     delete m;
 }
@@ -1167,12 +1156,6 @@ extern "C" int vmx_qwen3_load_dense_linear(vmx_qwen3 *m, int layer, int slot, co
     if (!b.p)
         if (int rc = b.alloc((size_t)rows_of[buf_of[slot]] * K * 2)) return rc;
     VMX_CHECK_HIP(hipMemcpyAsync((char *)b.p + (size_t)row0[slot] * K * 2, weight_bf16, need, hipMemcpyDefault, vmx_stream(stream)));
-    const size_t tmp_need = (size_t)16 * (2 * I > NQ + 2 * NKV ? 2 * I : NQ + 2 * NKV) * 2;
-    if (m->dense_tmp.bytes < tmp_need) {
-        VMX_CHECK_HIP(hipStreamSynchronize(vmx_stream(stream)));
-        m->dense_tmp.release();
-        if (int rc = m->dense_tmp.alloc(tmp_need)) return rc;
-    }
     L.dn_filled |= 1 << slot;
     return VMX_OK;
 }
@@ -1297,7 +1280,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
     uint16_t *attn = (uint16_t *)m->attn.p, *act = (uint16_t *)m->act.p;
     const int NQ = Hq * hd, NKV = Hkv * hd;
     float *ssq = (float *)m->ssq.p;
-    bool have_ssq = false;   // ssq holds the tile sums of squares of the current h (left by a residual-epilogue linear)
+    int ssq_tiles = 0;   // > 0: ssq holds that many tile sums of squares per row of the current h (left by a residual-epilogue linear)
     for (const Layer &L : m->layers) {
         const bool moe = c.num_experts > 0;  // int4 attention projections + mixture-of-experts MLP
         const bool ex = !moe && !L.int4_ready() && L.exl3_ready();   // EXL3 layer: every projection an Exl3Linear
@@ -1321,7 +1304,11 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
         const bool mfold = moe && folded_layers_enabled() && !tp && !pending && prefill_offset < 0 && !m->rows_share_cache &&
                            L.int4_attn_ready() && H % 256 == 0 && NQ <= 4 * 16 * 128 && vmx_int4_norm_splits(B, NQKV_, H, 0) > 0 &&
                            vmx_int4_resid_fusable(B, H, NQ) && vmx_split_decode_attention_parts(hd, Hq / Hkv, hd, max_seq_len, 0) > 0;
-        const bool fold_in = (fold || mfold) && have_ssq;   // the first layer's h comes from the embedding: no tile sums yet
+        // Unquantised layer on decode rows: the same five launches (norms in the prologues, residual adds in the epilogues)
+        const bool dfold = dn && !f16 && folded_layers_enabled() && !tp && !pending && prefill_offset < 0 && vmx_dense_decode_ok(B, NQKV_, H) &&
+                           vmx_dense_decode_ok(B, H, NQ) && vmx_dense_decode_ok(B, 2 * I, H) && vmx_dense_decode_ok(B, H, I);
+        // the first layer's h comes from the embedding: no tile sums yet
+        const bool fold_in = ((fold || mfold) && ssq_tiles == H / 16) || (dfold && ssq_tiles > 0 && ssq_tiles % 4 == 0);
         // EXL3 decode rows: the residual kernel leaves block sums of squares and q|k|v normalises its rows itself
         const bool ex_norm_in = ex && B <= 4 && L.ex_svh_qkv.p && pending_svh && exl3_resid_stats_ok(B, pending_splits, H);
         const uint16_t *ex_in = ex_norm_in ? h : x, *ex_in_w = ex_norm_in ? (const uint16_t *)L.input_ln.p : nullptr;
@@ -1336,12 +1323,18 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
                               embed_pending ? (const uint16_t *)m->embed.p : nullptr, input_ids, c.vocab_size, f16);
         embed_pending = false;
         pending_svh = nullptr;
-        have_ssq = false;
-        if (fold_in) s_qkv = vmx_int4_norm_splits(B, NQKV_, H, 0);   // the wide kernel has its own k slicing
+        const int tiles_in = ssq_tiles;
+        ssq_tiles = 0;
+        if (fold_in && !dfold) s_qkv = vmx_int4_norm_splits(B, NQKV_, H, 0);   // the wide kernel has its own k slicing
         const float *qkv_src = PA;
         const uint16_t *qkv_svh = nullptr;
         bool ex_split = false;
-        if (fold_in) {
+        if (dfold) {
+            const uint16_t *W = (const uint16_t *)L.dn[0].p;
+            if (int rc = fold_in ? vmx_dense_decode_norm_f32(PA, h, (const uint16_t *)L.input_ln.p, c.rms_norm_eps, ssq, tiles_in, W, B, NQKV_, H, st)
+                                 : vmx_dense_decode_f32(PA, x, W, B, NQKV_, H, st))
+                return rc;
+        } else if (fold_in) {
             if (int rc = vmx_int4_gemm_partial_norm(L.qkv.packed.p, h, (const uint16_t *)L.input_ln.p, c.rms_norm_eps, ssq, PA, B, NQKV_, H,
                                                     L.qkv.group, st))
                 return rc;
@@ -1367,7 +1360,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
             if (int rc = exl3_forward(m, L.ex[VMX_L_K], x, PA + NQ, NQKV_, B, st)) return rc;
             if (int rc = exl3_forward(m, L.ex[VMX_L_V], x, PA + NQ + NKV, NQKV_, B, st)) return rc;
         } else if (dn) {
-            if (int rc = dense_forward(m, L.dn[0].p, x, PA, NQKV_, NQKV_, H, B, st)) return rc;
+            if (int rc = dense_forward(L.dn[0].p, x, PA, NQKV_, H, B, st)) return rc;
         } else if (iq) {
             if (int rc = iq_forward(m, L.iq[VMX_L_Q], PA, NQKV_, B, st)) return rc;
             if (int rc = iq_forward(m, L.iq[VMX_L_K], PA + NQ, NQKV_, B, st)) return rc;
@@ -1375,8 +1368,9 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
         } else if (int rc = run_linear(m, L.qkv, x, PA, B, st)) return rc;
         const float *ks = (const float *)L.kv_scales.p;
         // five-launch layers: attention spread over several workgroups per KV head, merged by o_proj while it stages its activations
-        const bool split_attn = ex_split || ((fold || mfold) && prefill_offset < 0 && !m->rows_share_cache && NQ <= 4 * 16 * 128 &&
-                                             vmx_split_decode_attention_parts(hd, Hq / Hkv, hd, max_seq_len, 0) > 0);
+        const int split_p = vmx_split_decode_attention_parts(hd, Hq / Hkv, hd, max_seq_len, 0);
+        const bool split_attn = ex_split || ((fold || mfold || (dfold && vmx_dense_decode_merge_ok(B, NQ, hd, split_p))) && prefill_offset < 0 &&
+                                             !m->rows_share_cache && NQ <= 4 * 16 * 128 && split_p > 0);
         VmxAttnParts sparts{};
         // long contexts: the same kernel with many partitions and the separate merge instead of the three-launch path
         int long_p = !split_attn && prefill_offset < 0 && !m->rows_share_cache
@@ -1439,6 +1433,16 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
                                                    iq ? q8_ad(m, B, NQ) : nullptr, f16 ? 1 : 0))
                 return rc;
         }
+        if (dfold) {   // h += o_proj(attn);  act = glu(gate|up(rms_norm(h)));  h += down(act)
+            if (int rc = vmx_dense_decode_resid(h, ssq, attn, split_attn ? &sparts : nullptr, hd, (const uint16_t *)L.dn[1].p, B, H, NQ, st)) return rc;
+            ssq_tiles = vmx_dense_decode_tiles(B, H);
+            if (int rc = vmx_dense_decode_norm_glu(act, h, (const uint16_t *)L.post_ln.p, c.rms_norm_eps, ssq, ssq_tiles, (const uint16_t *)L.dn[2].p, B,
+                                                   2 * I, H, st))
+                return rc;
+            if (int rc = vmx_dense_decode_resid(h, ssq, act, nullptr, hd, (const uint16_t *)L.dn[3].p, B, H, I, st)) return rc;
+            pending = nullptr;
+            continue;
+        }
         if (fold) {   // h += o_proj(attn);  act = glu(gate|up(rms_norm(h)));  h += down(act)
             if (split_attn) {
                 if (int rc = vmx_int4_gemm_resid_attn(L.o.packed.p, &sparts, hd, h, ssq, B, H, NQ, L.o.group, st)) return rc;
@@ -1448,7 +1452,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
                 return rc;
             if (int rc = vmx_int4_gemm_resid(L.down.packed.p, act, h, ssq, B, H, I, L.down.group, st)) return rc;
             pending = nullptr;
-            have_ssq = true;
+            ssq_tiles = H / 16;
             continue;
         }
         if (mfold) {   // h += o_proj(attn);  x = rms_norm(h);  h += experts(x)
@@ -1479,7 +1483,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
                                                   vmx_int4_glu_fusable(2 * I, H) ? 1 : 0, st, h, ssq))
                 return rc;
             pending = nullptr;
-            have_ssq = true;
+            ssq_tiles = H / 16;
             continue;
         }
         const float *o_src = PB;
@@ -1493,7 +1497,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
         } else if (ex) {
             if (int rc = exl3_forward(m, L.ex[VMX_L_O], attn, PB, H, B, st)) return rc;
         } else if (dn) {
-            if (int rc = dense_forward(m, L.dn[1].p, attn, PB, H, H, NQ, B, st)) return rc;
+            if (int rc = dense_forward(L.dn[1].p, attn, PB, H, NQ, B, st)) return rc;
         } else if (iq) {
             if (int rc = iq_forward(m, L.iq[VMX_L_O], PB, H, B, st)) return rc;
         } else if (int rc = run_linear(m, L.o, attn, PB, B, st)) return rc;
@@ -1546,7 +1550,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
             if (int rc = exl3_forward(m, L.ex[VMX_L_GATE], x, PA, 2 * I, B, st)) return rc;
             if (int rc = exl3_forward(m, L.ex[VMX_L_UP], x, PA + I, 2 * I, B, st)) return rc;
         } else if (dn) {
-            if (int rc = dense_forward(m, L.dn[2].p, x, PA, 2 * I, 2 * I, H, B, st)) return rc;
+            if (int rc = dense_forward(L.dn[2].p, x, PA, 2 * I, H, B, st)) return rc;
         } else if (iq) {
             if (int rc = iq_forward(m, L.iq[VMX_L_GATE], PA, 2 * I, B, st)) return rc;
             if (int rc = iq_forward(m, L.iq[VMX_L_UP], PA + I, 2 * I, B, st)) return rc;
@@ -1573,7 +1577,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
         } else if (ex) {
             if (int rc = exl3_forward(m, L.ex[VMX_L_DOWN], act, PB, H, B, st)) return rc;
         } else if (dn) {
-            if (int rc = dense_forward(m, L.dn[3].p, act, PB, H, H, I, B, st)) return rc;
+            if (int rc = dense_forward(L.dn[3].p, act, PB, H, I, B, st)) return rc;
         } else if (iq) {
             if (int rc = iq_forward(m, L.iq[VMX_L_DOWN], PB, H, B, st)) return rc;
         } else if (int rc = run_linear(m, L.down, act, PB, B, st)) return rc;

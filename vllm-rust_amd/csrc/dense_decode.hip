@@ -1,0 +1,302 @@
+// Decode steps (up to 16 rows) of a layer whose projections are plain bf16 matrices W [N][K]: every projection is ONE launch that owns
+// both sides of what would be kernel boundaries -- the RMSNorm of the residual stream or the merge of the attention partitions while
+// its rows become matrix operands, and behind the sum the residual addition, the gated activation, or the f32 rows the attention reads.
+// Such a step is a chain of short launches over weights that are read once (Qwen3-0.6B: 4 .. 13 MB each), so what bounds it is the
+// latency of each link: the weights of a workgroup are requested before anything they wait for is computed, and no result is converted
+// by a launch of its own.  Qwen3-0.6B at one row, 128 tokens: 12 launches and 43 us a layer as norm, GEMV, widening, activation kernels;
+// 5 launches and 28 us now (q|k|v 4.9 us, attention 7.6, o 4.7, gate|up 6.4 = 2.0 TB/s, down 4.5); the whole step 1269 -> 819 us.
+#include "vmx_kernels.h"
+
+namespace {
+
+typedef uint32_t dd_u32x4 __attribute__((ext_vector_type(4)));
+
+enum { DD_ROWS = 0, DD_NORM = 1, DD_MERGE = 2, DD_NORM_REG = 3 };   // where the rows come from (DD_NORM_REG: DD_NORM of rows too long for LDS)
+enum { DD_F32 = 0, DD_RESID = 1, DD_GLU = 2 };          // what becomes of the sums
+
+struct DenseDecode {
+    const uint16_t *W, *x;          // x: bf16 rows [M][K] (DD_ROWS), the residual stream (DD_NORM)
+    const uint16_t *norm_w;         // DD_NORM
+    const float *ssq;               // DD_NORM: sums of squares of the stream's tiles, [M][tiles]
+    float eps;
+    int tiles;
+    const float *part, *part_max, *part_sum;   // DD_MERGE: [M][K / head][P][head], [M][K / head][P] twice
+    int P, head;
+    float *y;                       // DD_F32: [M][N]
+    uint16_t *h;                    // DD_RESID: stream [M][N], and the tiles' new sums of squares [M][N / CW]
+    float *ssq_out;
+    uint16_t *act;                  // DD_GLU: [M][N / 2]; rows [0, N / 2) of W are the gate, the others the up projection
+    int M, N, K;
+};
+
+__device__ __forceinline__ dd_u32x4 dd_pack(const float (&f)[8]) {
+    dd_u32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = (uint32_t)vmx_f32_to_bf16(f[2 * e]) | ((uint32_t)vmx_f32_to_bf16(f[2 * e + 1]) << 16);
+    return v;
+}
+__device__ __forceinline__ void dd_unpack(dd_u32x4 v, float (&f)[8]) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        f[2 * e] = __uint_as_float(v[e] << 16);
+        f[2 * e + 1] = __uint_as_float(v[e] & 0xFFFF0000u);
+    }
+}
+
+constexpr int DD_STAGE = 16 * 1032;   // values that the norm and the merge stage in LDS at most: rows of K + 8
+
+// A workgroup owns CW columns: 16, or for up to four rows of a narrow product 4 (DD_GLU: half gate and the same up columns).  Lane
+// (c = l & 15, g = l / 16) of v_mfma_f32_16x16x32_bf16 stands for column and row c % CW and for part c / CW of a block's k, so with
+// four columns the tile's diagonal 4 x 4 squares are the partial sums of four parts of k and the others are not used: the matrix core
+// idles anyway and the product has four times the workgroups (down of Qwen3-0.6B, [1024, 3072] at one row: 8.9 us in 64 workgroups
+// of 16 columns, 4.8 in 256 of 4).  A wave takes the blocks w, w + NW, .. of 128 values a part; eight values feed one of four
+// products; the four lanes g of a column read 64 consecutive bytes (as 16 bytes of four places 64 apart: gate|up 8.1 us, now 6.4).
+// Rows that have to be normed or merged are worked out once per workgroup, spread over its threads, and staged in LDS: computed by
+// each lane for its own operands, one live row of sixteen kept four lanes of a wave busy (q|k|v 6.7 -> 5.0 us, gate|up 9.1 -> 8.1).
+// Their inputs come from the caches and are requested ahead of the weights of the first DEPTH blocks, because loads return in order.
+template <int NW, int CW, int DEPTH, int SRC, int DST>
+__global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const DenseDecode p) {
+    constexpr int PARTS = 16 / CW, DEEP = 128 * PARTS;
+    constexpr bool STAGED = SRC == DD_NORM || SRC == DD_MERGE, NORM = SRC == DD_NORM || SRC == DD_NORM_REG;
+    __shared__ float red[NW][64][4];
+    __shared__ __align__(16) uint16_t rows_lds[STAGED ? DD_STAGE : 8];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & (CW - 1), part = (lane & 15) / CW, g = lane >> 4, nt = blockIdx.x;
+    const int K = p.K, nblk = (K + DEEP - 1) / DEEP, row = min(c, p.M - 1);
+    const bool live = c < p.M;
+    const uint16_t *wrow = p.W + (int64_t)(DST == DD_GLU ? (c < CW / 2 ? 0 : p.N / 2) + nt * (CW / 2) + (c & (CW / 2 - 1)) : nt * CW + c) * K;
+    const int k0 = 128 * part + 8 * g;
+    dd_u32x4 w[DEPTH][4], xr[DEPTH][4], nr[DEPTH][SRC == DD_NORM_REG ? 4 : 1];
+    auto load_w = [&](int b, dd_u32x4 (&d)[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int k = DEEP * b + k0 + 32 * j;
+            d[j] = k < K ? __builtin_nontemporal_load(reinterpret_cast<const dd_u32x4 *>(wrow + k)) : dd_u32x4{0, 0, 0, 0};
+        }
+    };
+    auto load_rows = [&](int b, dd_u32x4 (&x)[4], dd_u32x4 (&n)[SRC == DD_NORM_REG ? 4 : 1]) {
+        if constexpr (!STAGED) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int k = DEEP * b + k0 + 32 * j;
+                x[j] = live && k < K ? *reinterpret_cast<const dd_u32x4 *>(p.x + (int64_t)row * K + k) : dd_u32x4{0, 0, 0, 0};
+                if constexpr (SRC == DD_NORM_REG) n[j] = k < K ? *reinterpret_cast<const dd_u32x4 *>(p.norm_w + k) : dd_u32x4{0, 0, 0, 0};
+            }
+        }
+    };
+    // staged rows: a thread works out eight consecutive values of a row at a time
+    const int chunks = STAGED ? p.M * (K / 8) : 0, chunk0 = min(tid, chunks - 1);
+    float4 lo[4], hi[4];
+    float most[4], total[4];
+    auto load_parts = [&](int i) {
+        const int m = i / (K / 8), k = (i - m * (K / 8)) * 8;
+        const int64_t at = ((int64_t)m * (K / p.head) + k / p.head) * p.P;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {   // partitions past P read the last one again; their weight is zero below
+            const int64_t from = at + min(q, p.P - 1);
+            const float4 *src = reinterpret_cast<const float4 *>(p.part + from * p.head + k % p.head);
+            lo[q] = src[0], hi[q] = src[1], most[q] = p.part_max[from], total[q] = p.part_sum[from];
+        }
+    };
+    auto merge_parts = [&](int i) {
+        float top = -3.402823466e+38f, sum = 0.f, f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 4; q++) top = fmaxf(top, q < p.P ? most[q] : -3.402823466e+38f);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float wt = q < p.P ? total[q] * __expf(most[q] - top) : 0.f;
+            sum += wt;
+            f[0] += lo[q].x * wt, f[1] += lo[q].y * wt, f[2] += lo[q].z * wt, f[3] += lo[q].w * wt;
+            f[4] += hi[q].x * wt, f[5] += hi[q].y * wt, f[6] += hi[q].z * wt, f[7] += hi[q].w * wt;
+        }
+        const float scale = 1.0f / (sum + 1e-6f);
+#pragma unroll
+        for (int e = 0; e < 8; e++) f[e] *= scale;
+        const int m = i / (K / 8);
+        *reinterpret_cast<dd_u32x4 *>(&rows_lds[m * (K + 8) + (i - m * (K / 8)) * 8]) = dd_pack(f);
+    };
+
+    // DD_NORM: the wave's lanes share the tiles' sums of its rows out (lane % rows is the row, as it is for c)
+    const int rows = p.M <= 1 ? 1 : p.M <= 2 ? 2 : p.M <= 4 ? 4 : p.M <= 8 ? 8 : 16, quads = NORM ? p.tiles / 4 : 1;
+    const float4 *tile = NORM ? reinterpret_cast<const float4 *>(p.ssq + (int64_t)min(lane & (rows - 1), p.M - 1) * p.tiles) : nullptr;
+    float4 t0;
+    dd_u32x4 x0, n0;
+    if constexpr (NORM) t0 = tile[min(lane / rows, quads - 1)];
+    if constexpr (SRC == DD_NORM) {
+        x0 = *reinterpret_cast<const dd_u32x4 *>(p.x + (int64_t)chunk0 * 8);
+        n0 = *reinterpret_cast<const dd_u32x4 *>(p.norm_w + chunk0 % (K / 8) * 8);
+    }
+    if constexpr (SRC == DD_MERGE) load_parts(chunk0);
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++)
+        if (wave + d * NW < nblk) load_rows(wave + d * NW, xr[d], nr[d]);
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) load_w(wave + d * NW, w[d]);   // past the end of K: no request
+    float inv = 0.f;
+    if constexpr (NORM) {
+        float sq = lane / rows < quads ? (t0.x + t0.y) + (t0.z + t0.w) : 0.f;
+        for (int i = lane / rows + 64 / rows; i < quads; i += 64 / rows) {
+            const float4 v = tile[i];
+            sq += (v.x + v.y) + (v.z + v.w);
+        }
+        if (rows <= 1) sq += vmx_lane_xor<1>(sq);
+        if (rows <= 2) sq += vmx_lane_xor<2>(sq);
+        if (rows <= 4) sq += vmx_lane_xor<4>(sq);
+        if (rows <= 8) sq += vmx_lane_xor<8>(sq);
+        sq += vmx_lane_xor<16>(sq);
+        sq += vmx_lane_xor<32>(sq);
+        inv = rsqrtf(sq / (float)K + p.eps);
+    }
+    auto norm8 = [&](dd_u32x4 x, dd_u32x4 n, float by) {
+        float f[8], gain[8];
+        dd_unpack(x, f);
+        dd_unpack(n, gain);
+#pragma unroll
+        for (int e = 0; e < 8; e++) f[e] = f[e] * by * gain[e];
+        return dd_pack(f);
+    };
+    if constexpr (SRC == DD_NORM) {
+        for (int i = tid; i - lane < chunks; i += 64 * NW) {   // whole waves: the statistic of a row is held by the lane of its number
+            const int at = min(i, chunks - 1), m = at / (K / 8), k = (at - m * (K / 8)) * 8;
+            const float by = __shfl(inv, m);
+            if (i != tid) {
+                x0 = *reinterpret_cast<const dd_u32x4 *>(p.x + (int64_t)at * 8);
+                n0 = *reinterpret_cast<const dd_u32x4 *>(p.norm_w + k);
+            }
+            if (i < chunks) *reinterpret_cast<dd_u32x4 *>(&rows_lds[m * (K + 8) + k]) = norm8(x0, n0, by);
+        }
+    }
+    if constexpr (SRC == DD_MERGE) {
+        if (tid < chunks) merge_parts(tid);
+        for (int i = tid + 64 * NW; i < chunks; i += 64 * NW) {
+            load_parts(i);
+            merge_parts(i);
+        }
+    }
+    if constexpr (STAGED) __syncthreads();
+    vmx_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto step = [&](int b, dd_u32x4 (&d)[4], dd_u32x4 (&x)[4], dd_u32x4 (&n)[SRC == DD_NORM_REG ? 4 : 1]) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            dd_u32x4 a = x[j];
+            if constexpr (SRC == DD_NORM_REG) a = norm8(a, n[j], inv);
+            else if constexpr (STAGED) {
+                const int k = DEEP * b + k0 + 32 * j;
+                a = live && k < K ? *reinterpret_cast<const dd_u32x4 *>(&rows_lds[row * (K + 8) + k]) : dd_u32x4{0, 0, 0, 0};
+            }
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, a), __builtin_bit_cast(vmx_bf16x8, d[j]), acc, 0, 0, 0);
+        }
+        if (DEPTH > 1 && b + DEPTH * NW < nblk) {
+            load_w(b + DEPTH * NW, d);
+            load_rows(b + DEPTH * NW, x, n);
+        }
+    };
+    if constexpr (DEPTH == 1) {   // one block a wave
+        if (wave < nblk) step(wave, w[0], xr[0], nr[0]);
+    } else {
+        for (int b = wave; b < nblk; b += 2 * NW) {
+            step(b, w[0], xr[0], nr[0]);
+            if (b + NW < nblk) step(b + NW, w[1], xr[1], nr[1]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) red[wave][lane][r] = acc[r];
+    __syncthreads();
+    if (tid >= (CW == 4 ? 64 : 256)) return;
+    // CW 16: thread -> row tid / 16, column tid % 16 (element (4 g + r, c) of a tile sits with lane 16 g + c); CW 4: thread -> part
+    // tid / 16, row tid / 4 % 4, column tid % 4, the square of part i at rows and columns 4 i ..
+    const int m = CW == 16 ? tid >> 4 : (tid >> 2) & 3, n = tid & (CW - 1);
+    const int from = CW == 16 ? (m >> 2) * 16 + n : (tid >> 4) * 20 + n, r = m & 3;
+    float v = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; i++) v += red[i][from][r];
+    if constexpr (CW == 4) {
+        v += vmx_lane_xor<16>(v);
+        v += vmx_lane_xor<32>(v);
+    }
+    const bool keep = m < p.M && (CW == 16 || tid < 16);
+    if constexpr (DST == DD_F32) {
+        if (keep) p.y[(int64_t)m * p.N + nt * CW + n] = v;
+    } else if constexpr (DST == DD_GLU) {
+        const float up = vmx_lane_xor<CW / 2>(v);
+        if (keep && n < CW / 2) {
+            const float gg = vmx_bf16_to_f32(vmx_f32_to_bf16(v)), uu = vmx_bf16_to_f32(vmx_f32_to_bf16(up));
+            p.act[(int64_t)m * (p.N / 2) + nt * (CW / 2) + n] = vmx_f32_to_bf16((gg / (1.0f + expf(-gg))) * uu);
+        }
+    } else {
+        const int64_t at = (int64_t)min(m, p.M - 1) * p.N + nt * CW + n;
+        const uint16_t hn = vmx_f32_to_bf16(vmx_bf16_to_f32(p.h[at]) + vmx_bf16_to_f32(vmx_f32_to_bf16(v)));
+        const float f = vmx_bf16_to_f32(hn);
+        float s = f * f;
+        s += vmx_lane_xor<1>(s);
+        s += vmx_lane_xor<2>(s);
+        if constexpr (CW == 16) {
+            s += vmx_lane_xor<4>(s);
+            s += vmx_lane_xor<8>(s);
+        }
+        if (keep) {
+            p.h[at] = hn;
+            if (n == 0) p.ssq_out[m * (p.N / CW) + nt] = s;
+        }
+    }
+}
+
+template <int CW, int SRC, int DST>
+int dd_launch(const DenseDecode &p, hipStream_t st) {
+    const int nblk = (p.K + 128 * (16 / CW) - 1) / (128 * (16 / CW));
+    const dim3 grid((unsigned)(p.N / CW));
+    if (nblk <= 4) hipLaunchKernelGGL((dense_decode_kernel<4, CW, 1, SRC, DST>), grid, dim3(256), 0, st, p);
+    else if (nblk <= 8) hipLaunchKernelGGL((dense_decode_kernel<8, CW, 1, SRC, DST>), grid, dim3(512), 0, st, p);
+    else if (nblk <= 16 || SRC == DD_NORM_REG) hipLaunchKernelGGL((dense_decode_kernel<8, CW, 2, SRC, DST>), grid, dim3(512), 0, st, p);
+    else hipLaunchKernelGGL((dense_decode_kernel<SRC == DD_NORM_REG ? 8 : 16, CW, 2, SRC, DST>), grid, dim3(1024), 0, st, p);
+    VMX_CHECK_LAUNCH("dense_decode");
+    return VMX_OK;
+}
+
+// Four columns a workgroup where sixteen would leave compute units without one (figures: see the kernel)
+bool dd_narrow(int M, int N) { return M <= 4 && N / 16 < vmx_num_cus(); }
+
+}  // namespace
+
+// A product of N columns over K: whole 16-column tiles, 16-byte rows
+bool vmx_dense_decode_ok(int M, int N, int K) { return M >= 1 && M <= 16 && N % 16 == 0 && K % 16 == 0; }
+
+// Sums of squares per row that vmx_dense_decode_resid leaves
+int vmx_dense_decode_tiles(int M, int N) { return N / (dd_narrow(M, N) ? 4 : 16); }
+
+int vmx_dense_decode_f32(float *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, hipStream_t st) {
+    DenseDecode p{};
+    p.W = W, p.x = x, p.y = y, p.M = M, p.N = N, p.K = K;
+    return dd_launch<16, DD_ROWS, DD_F32>(p, st);
+}
+
+// y = rms_norm(h) W^T; ssq: what vmx_dense_decode_resid left for h
+int vmx_dense_decode_norm_f32(float *y, const uint16_t *h, const uint16_t *norm_w, float eps, const float *ssq, int tiles, const uint16_t *W, int M,
+                              int N, int K, hipStream_t st) {
+    DenseDecode p{};
+    p.W = W, p.x = h, p.norm_w = norm_w, p.eps = eps, p.ssq = ssq, p.tiles = tiles, p.y = y, p.M = M, p.N = N, p.K = K;
+    return M * (K + 8) <= DD_STAGE ? dd_launch<16, DD_NORM, DD_F32>(p, st) : dd_launch<16, DD_NORM_REG, DD_F32>(p, st);
+}
+
+// act [M][N / 2] = silu(gate) * up of rms_norm(h) W^T
+int vmx_dense_decode_norm_glu(uint16_t *act, const uint16_t *h, const uint16_t *norm_w, float eps, const float *ssq, int tiles, const uint16_t *W, int M,
+                              int N, int K, hipStream_t st) {
+    DenseDecode p{};
+    p.W = W, p.x = h, p.norm_w = norm_w, p.eps = eps, p.ssq = ssq, p.tiles = tiles, p.act = act, p.M = M, p.N = N, p.K = K;
+    return M * (K + 8) <= DD_STAGE ? dd_launch<16, DD_NORM, DD_GLU>(p, st) : dd_launch<16, DD_NORM_REG, DD_GLU>(p, st);
+}
+
+bool vmx_dense_decode_merge_ok(int M, int K, int head_dim, int parts) {
+    return M <= 4 && M * (K + 8) <= DD_STAGE && parts >= 1 && parts <= 4 && head_dim % 8 == 0 && K % head_dim == 0;
+}
+
+// h += x W^T (x the merged attention partitions if `parts`), ssq [M][vmx_dense_decode_tiles] = sums of squares of the new h's tiles
+int vmx_dense_decode_resid(uint16_t *h, float *ssq, const uint16_t *x, const VmxAttnParts *parts, int head_dim, const uint16_t *W, int M, int N, int K,
+                           hipStream_t st) {
+    DenseDecode p{};
+    p.W = W, p.x = x, p.h = h, p.ssq_out = ssq, p.M = M, p.N = N, p.K = K;
+    const bool narrow = dd_narrow(M, N);
+    if (!parts) return narrow ? dd_launch<4, DD_ROWS, DD_RESID>(p, st) : dd_launch<16, DD_ROWS, DD_RESID>(p, st);
+    VMX_REQUIRE(vmx_dense_decode_merge_ok(M, K, head_dim, parts->max_parts), "dense_decode: partitions not covered");
+    p.part = parts->tmp_out, p.part_max = parts->max_logits, p.part_sum = parts->exp_sums, p.P = parts->max_parts, p.head = head_dim;
+    return narrow ? dd_launch<4, DD_MERGE, DD_RESID>(p, st) : dd_launch<16, DD_MERGE, DD_RESID>(p, st);
+}

@@ -58,6 +58,19 @@ int vmx_fused_decode_attention(uint16_t *out, const float *qkv_partial, int spli
                                const float *v_scale, int8_t *aq, float *ad, int v_norm, hipStream_t st,   // v_norm: weightless RMSNorm on v
                                const uint16_t *had_svh = nullptr);   // EXL3: qkv_partial is the trellis GEMM before its output transform
 
+// dense_decode.hip: the projections of an unquantised bf16 layer on decode rows (see there)
+struct VmxAttnParts;
+bool vmx_dense_decode_ok(int M, int N, int K);
+bool vmx_dense_decode_merge_ok(int M, int K, int head_dim, int parts);
+int vmx_dense_decode_f32(float *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, hipStream_t st);
+int vmx_dense_decode_tiles(int M, int N);
+int vmx_dense_decode_norm_f32(float *y, const uint16_t *h, const uint16_t *norm_w, float eps, const float *ssq, int tiles, const uint16_t *W, int M,
+                              int N, int K, hipStream_t st);
+int vmx_dense_decode_norm_glu(uint16_t *act, const uint16_t *h, const uint16_t *norm_w, float eps, const float *ssq, int tiles, const uint16_t *W, int M,
+                              int N, int K, hipStream_t st);
+int vmx_dense_decode_resid(uint16_t *h, float *ssq, const uint16_t *x, const VmxAttnParts *parts, int head_dim, const uint16_t *W, int M, int N, int K,
+                           hipStream_t st);
+
 // exl3_kernels.hip: Exl3Linear::forward for the whole-token executor; workspace = vmx_exl3_gemm_workspace_bytes(M, K, N)
 int vmx_exl3_forward_f32(const uint16_t *x, int x_bf16, const void *trellis, const uint16_t *suh, const uint16_t *svh, float *y32,
                          int ld, int M, int K, int N, int bits, int codebook, void *workspace, size_t workspace_bytes, hipStream_t st);
