@@ -1,4 +1,5 @@
-"""Prompt-sized products on the shared matrix-core tiles (csrc/tile_gemm.h) at the edges of their tiles, stages and shape choices."""
+"""Prompt-sized products on the shared matrix-core tiles (csrc/tile_gemm.h) at the edges of their tiles, stages and shape choices,
+and the decode-row linears at the edges of theirs."""
 import numpy as np
 import pytest
 
@@ -83,3 +84,22 @@ def test_int4_prompt_tiles(gpu, M, N, K, group):
     ref = x.double() @ ((nib - zp).double() * s) + bias.double()
     bound = 2.0 ** -8 * ref.abs() + (128 + K // 128 + 32) * 2.0 ** -24 * 286 * (x.double().abs() @ s)
     assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+# decode rows: column groups below one per compute unit (halved k; 4 and 8 waves, a second round), between one and two, and above
+@pytest.mark.parametrize("M,N,K", [(1, 40, 72), (16, 2048, 2040), (5, 1000, 2312), (3, 4100, 520), (16, 4096, 1032), (7, 6000, 2056), (16, 9000, 136)])
+@pytest.mark.parametrize("x_f32", [False, True])
+def test_bf16_linear_decode_rows(gpu, M, N, K, x_f32):
+    """f32 sums of bf16 products in at most K terms: |error| <= K 2^-24 sum |x w|, doubled for the order of the partial sums."""
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    g = torch.Generator(device="cuda").manual_seed(M * 7 + N + K)
+    x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
+    w = torch.randn((N, K), device="cuda", generator=g).to(torch.bfloat16)
+    xin = x.float() if x_f32 else x
+    y = torch.full((M, N), float("nan"), device="cuda")
+    check(lib.vmx_linear_bf16w(y.data_ptr(), 0, xin.data_ptr(), 0 if x_f32 else 1, w.data_ptr(), M, N, K, 0, None))
+    torch.cuda.synchronize()
+    exact = x.double() @ w.double().T
+    bound = K * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((y.double() - exact).abs() <= bound).all())

@@ -294,86 +294,123 @@ __global__ __launch_bounds__(S::THREADS) void linear_tile_kernel(const VmxLinear
     }
 }
 
-// Up to 16 rows (decode steps, 16-row expert blocks): the product is a stream over the weights.  A workgroup owns 16 output
-// columns; its four waves split K in 128-deep blocks (wave w takes blocks w, w + 4, ...), lane (n, g) reads the 64 contiguous
-// bytes W[n][128 b + 32 g ..] of a block straight from memory, two blocks ahead of the one being multiplied, and the activation
-// fragment at the same k from the (cache-resident) rows; chunk j of both feeds MFMA step j -- the instruction only needs A and B
-// to agree on which k sits where.  The four partial tiles are added in wave order through LDS.
-__global__ __launch_bounds__(256) void linear_skinny_kernel(const VmxLinear p) {
-    __shared__ float red[3][64][4];
-    __shared__ int64_t rows[16];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fl = lane & 15, fg = lane >> 4;
-    const int m0 = blockIdx.y * 16, n0 = blockIdx.x * 16, z = blockIdx.z;
+// Up to 16 rows (decode steps, 16-row expert blocks): the product is a stream over the weights.  A workgroup owns 16 output columns, or
+// with PARTS = 2 eight columns whose k is halved over the two halves of a tile's columns: each weight fragment then meets two
+// activation fragments, and of either product the half that belongs to its part is kept.  Its NW waves take the blocks w, w + NW, ..
+// of 128 values a part.  Lane (c, g) reads 16 of the 64 consecutive bytes that the four lanes g share of a column, straight from memory
+// and DEPTH blocks ahead, and the activation fragment at the same k from the (cache-resident) rows.  The waves' tiles are added in
+// wave order through LDS.
+template <int NW, int PARTS, int DEPTH>
+__global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const VmxLinear p) {
+    constexpr int CW = 16 / PARTS, DEEP = 128 * PARTS;
+    __shared__ float red[NW][64][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fl = lane & 15, c = fl & (CW - 1), part = fl / CW, fg = lane >> 4;
+    const int m0 = blockIdx.y * 16, n0 = blockIdx.x * CW, z = blockIdx.z;
     if (p.total_rows && m0 >= *p.total_rows) return;
     const uint16_t *W = p.W + z * p.w_bs;
     if (p.block_expert) W += (int64_t)p.block_expert[m0 / p.block_rows] * p.expert_stride;
-    if (tid < 16) rows[tid] = linear_src_row(p, m0 + tid);
-    __syncthreads();
-    const int64_t ar = rows[fl];
-    const int n = min(n0 + fl, p.N - 1);
-    const uint16_t *wrow = W + (int64_t)n * p.w_sn;
-    const int64_t a_at = z * p.a_bs + (ar < 0 ? 0 : ar) * p.lda;
-    const int nblk = (p.K + 127) >> 7;
-    auto load_w = [&](int b, uint4 (&w)[4]) {
+    const uint16_t *wrow = W + (int64_t)min(n0 + c, p.N - 1) * p.w_sn;
+    const int64_t ar = linear_src_row(p, m0 + fl), a_at = z * p.a_bs + (ar < 0 ? 0 : ar) * p.lda;
+    const int nblk = (p.K + DEEP - 1) / DEEP;
+    tg_u32x4 w[DEPTH][4], a[DEPTH][PARTS][4];
+    auto load_w = [&](int b, tg_u32x4 (&d)[4]) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int k = 128 * b + 32 * fg + 8 * j;
-            w[j] = k < p.K ? *reinterpret_cast<const uint4 *>(wrow + k) : make_uint4(0, 0, 0, 0);
+            const int k = DEEP * b + 128 * part + 32 * j + 8 * fg;
+            d[j] = k < p.K ? *reinterpret_cast<const tg_u32x4 *>(wrow + k) : tg_u32x4{0, 0, 0, 0};
         }
     };
-    auto load_a = [&](int b, uint4 (&a)[4]) {
+    auto load_a = [&](int b, tg_u32x4 (&d)[PARTS][4]) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int k = 128 * b + 32 * fg + 8 * j;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (ar >= 0 && k < p.K) {
-                if (p.a_f32) {
-                    const float *src = (const float *)p.A + a_at + k;
-                    const float4 f0 = *reinterpret_cast<const float4 *>(src), f1 = *reinterpret_cast<const float4 *>(src + 4);
-                    const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
-                    v = vmx_pack16x8<false>(f);
-                } else {
-                    v = *reinterpret_cast<const uint4 *>((const uint16_t *)p.A + a_at + k);
+        for (int q = 0; q < PARTS; q++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int k = DEEP * b + 128 * q + 32 * j + 8 * fg;
+                tg_u32x4 v = {0, 0, 0, 0};
+                if (ar >= 0 && k < p.K) {
+                    if (p.a_f32) {
+                        const float *src = (const float *)p.A + a_at + k;
+                        const float4 f0 = *reinterpret_cast<const float4 *>(src), f1 = *reinterpret_cast<const float4 *>(src + 4);
+                        const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+                        v = __builtin_bit_cast(tg_u32x4, vmx_pack16x8<false>(f));
+                    } else {
+                        v = *reinterpret_cast<const tg_u32x4 *>((const uint16_t *)p.A + a_at + k);
+                    }
                 }
+                d[q][j] = v;
             }
-            a[j] = v;
-        }
     };
-    vmx_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    uint4 w0[4], w1[4], a0[4], a1[4];
-    int b = wave;
-    if (b < nblk) { load_w(b, w0); load_a(b, a0); }
-    if (b + 4 < nblk) { load_w(b + 4, w1); load_a(b + 4, a1); }
-    for (; b < nblk; b += 8) {
-        uint4 wc[4], ac[4];
+    vmx_f32x4 acc[PARTS];
 #pragma unroll
-        for (int j = 0; j < 4; j++) wc[j] = w0[j], ac[j] = a0[j];
-        if (b + 8 < nblk) { load_w(b + 8, w0); load_a(b + 8, a0); }
+    for (int q = 0; q < PARTS; q++) acc[q] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto step = [&](int b, tg_u32x4 (&wv)[4], tg_u32x4 (&av)[PARTS][4]) {
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, ac[j]), __builtin_bit_cast(vmx_bf16x8, wc[j]), acc, 0, 0, 0);
-        if (b + 4 < nblk) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) wc[j] = w1[j], ac[j] = a1[j];
-            if (b + 12 < nblk) { load_w(b + 12, w1); load_a(b + 12, a1); }
+            for (int q = 0; q < PARTS; q++)
+                acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, av[q][j]), __builtin_bit_cast(vmx_bf16x8, wv[j]),
+                                                                 acc[q], 0, 0, 0);
+        if (DEPTH > 1 && b + DEPTH * NW < nblk) {
+            load_w(b + DEPTH * NW, wv);
+            load_a(b + DEPTH * NW, av);
+        }
+    };
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, ac[j]), __builtin_bit_cast(vmx_bf16x8, wc[j]), acc, 0, 0, 0);
+    for (int d = 0; d < DEPTH; d++)
+        if (wave + d * NW < nblk) {
+            load_w(wave + d * NW, w[d]);
+            load_a(wave + d * NW, a[d]);
+        }
+    if constexpr (DEPTH == 1) {   // one block a wave
+        if (wave < nblk) step(wave, w[0], a[0]);
+    } else {
+        for (int b = wave; b < nblk; b += 2 * NW) {
+            step(b, w[0], a[0]);
+            if (b + NW < nblk) step(b + NW, w[1], a[1]);
         }
     }
-    if (wave > 0) {
+    // the product of a column's own part
+    vmx_f32x4 own = acc[0];
+    if constexpr (PARTS == 2) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) red[wave - 1][lane][r] = acc[r];
+        for (int r = 0; r < 4; r++) own[r] = part ? acc[1][r] : acc[0][r];
     }
+#pragma unroll
+    for (int r = 0; r < 4; r++) red[wave][lane][r] = own[r];
     __syncthreads();
-    if (wave == 0) {
+    if (tid >= 16 * CW) return;
+    const int ml = tid / CW, nl = tid & (CW - 1), m = m0 + ml;   // element (4 g + r, c) of a tile sits with lane 16 g + c
+    float v = 0.f;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float v = ((acc[r] + red[0][lane][r]) + red[1][lane][r]) + red[2][lane][r];
-            const int ml = 4 * fg + r, m = m0 + ml;
-            if (m < p.M && !(p.row_ids && rows[ml] < 0) && n0 + fl < p.N) linear_store(p, z, m, n0 + fl, v);
-        }
+    for (int q = 0; q < PARTS; q++)
+#pragma unroll
+        for (int i = 0; i < NW; i++) v += red[i][(ml >> 2) * 16 + CW * q + nl][ml & 3];
+    if (m < p.M && n0 + nl < p.N && !(p.row_ids && linear_src_row(p, m) < 0)) linear_store(p, z, m, n0 + nl, v);
+}
+
+template <int NW, int PARTS, int DEPTH>
+void launch_skinny_as(const VmxLinear &p, hipStream_t st) {
+    constexpr int CW = 16 / PARTS;
+    hipLaunchKernelGGL((linear_skinny_kernel<NW, PARTS, DEPTH>), dim3((p.N + CW - 1) / CW, (p.M + 15) / 16, p.batch), dim3(64 * NW), 0, st, p);
+}
+
+// What bounds these is the number of requests under way, so the split follows the number of 16-column groups (and K, never M: a row's
+// sums do not depend on its neighbours).  16 rows, before (one form: 4 waves, 16 columns, a lane's 64 bytes in a row) and now:
+//   [12288, 2048], two groups a compute unit or more: 21.3 -> 16.6 us (the 64 bytes across lanes; 8 waves: 16.8); [32000, 2048]: 46.6 -> 36.7
+//   [11264, 2048]: 21.2 -> 16.4;  [3664, 2048], fewer groups than compute units: 10.4 -> 8.4
+//   [2048, 2048] and [2048, 6144], 128 groups: 12.4 on average -> 6.4 and 12.7
+// Expert blocks bring row blocks of their own and keep four waves.
+void launch_skinny(const VmxLinear &p, hipStream_t st) {
+    const int cols = (p.N + 15) / 16 * p.batch, cus = vmx_num_cus();
+    if (p.block_expert || cols >= 2 * cus) return launch_skinny_as<4, 1, 2>(p, st);
+    if (cols >= cus) {
+        const int nblk = (p.K + 127) / 128;
+        return nblk <= 4 ? launch_skinny_as<4, 1, 1>(p, st) : nblk <= 8 ? launch_skinny_as<8, 1, 1>(p, st) : launch_skinny_as<8, 1, 2>(p, st);
     }
+    const int nblk = (p.K + 255) / 256;
+    if (nblk <= 4) return launch_skinny_as<4, 2, 1>(p, st);
+    if (nblk <= 8) return launch_skinny_as<8, 2, 1>(p, st);
+    launch_skinny_as<8, 2, 2>(p, st);
 }
 
 // A few output columns in true f32 (router logits): one workgroup per row and group of 16 columns; a thread walks its k with
@@ -464,8 +501,7 @@ int vmx_linear_launch(const VmxLinear &p, hipStream_t st) {
         if (bm == 64 && tile_ok(p, direct)) {
             if (int rc = launch_tile(p, st)) return rc;
         } else if (bm == 16 && direct) {
-            grid.x = (p.N + 15) / 16;
-            hipLaunchKernelGGL(linear_skinny_kernel, grid, dim3(256), 0, st, p);
+            launch_skinny(p, st);
         } else if (bm == 16) hipLaunchKernelGGL(linear_mfma_kernel<16>, grid, dim3(256), 0, st, p);
         else hipLaunchKernelGGL(linear_mfma_kernel<64>, grid, dim3(256), 0, st, p);
     }
