@@ -70,3 +70,24 @@ def test_dense_prompt_rows(gpu, tokens):
         assert np.linalg.norm(got - exp) <= 2e-2 * np.linalg.norm(exp)
     finally:
         model.close()
+
+
+# KV heads times rows of 6, 128, 256 and 512 on 256 compute units: 42, 4, 2 and 1 partitions a KV head, block tables of more than 64 entries
+@pytest.mark.parametrize("heads,kv_heads,head_dim,rows", [(4, 2, 64, 3), (8, 8, 128, 16), (16, 16, 64, 16), (32, 32, 64, 16)])
+def test_long_contexts_partitions(gpu, heads, kv_heads, head_dim, rows):
+    from tests.test_gpu_true_geometry import _decode_and_compare, _fill_kv
+    from tests.model_oracle import OracleQwen3
+    from vllm_rust_amd.qwen3 import QuantizedQwen3ForCausalLM, Qwen3Spec, rope_cos_sin_cache
+    vmx, torch = gpu
+    contexts = [1100, 3, 1030, 0, 15, 16, 17, 511, 512, 700, 1023, 1024, 255, 64, 900, 1][:rows]
+    spec = Qwen3Spec(256, 2, heads, kv_heads, head_dim, 256, 512, tie_word_embeddings=True, max_position=2048, num_blocks=72 * rows, max_batch=rows,
+                     max_seq_len=1200, max_prefill_tokens=16)
+    model = QuantizedQwen3ForCausalLM(spec)
+    try:
+        ck = model.load_synthetic_bf16(seed=21, keep_host_copy=True)
+        ref = OracleQwen3(spec, ck, rope_cos_sin_cache(spec.head_dim, spec.max_position, spec.rope_theta))
+        shape = (spec.num_blocks, spec.block_size, spec.num_kv_heads, spec.head_dim)
+        _fill_kv(torch, model, ref, spec.num_layers, [shape] * spec.num_layers, spec.kv_cache_dtype, seed=3)
+        _decode_and_compare(torch, model, ref, spec, contexts, 1, [17 + 5 * b for b in range(rows)])
+    finally:
+        model.close()

@@ -130,18 +130,18 @@ template <int HD, int FP8> struct AttnTile {
 // Request tile [t0, min(t0 + 16, p1)): lane (token tl, dim group dg) takes 16-byte pieces of its token's K row, and every
 // V row of the tile is one coalesced wave access (row base broadcast from the lane that owns the token).  Lanes past the
 // end re-read the last valid row; their logits are masked later.
-// BTREG: lane l of bt_reg holds the sequence's block-table entry l (read once at kernel start) and the lookup is a lane
-// exchange instead of a dependent global load.
+// BTREG: lane l of bt_reg holds the sequence's block-table entry bt_base + l (read once) and the lookup is a lane exchange
+// instead of a dependent global load -- which, loads returning in order, would also wait for the tile requested before.
 template <int HD, int FP8, bool BTREG = false>
 __device__ __forceinline__ void attn_tile_load(AttnTile<HD, FP8> &t, const void *__restrict__ k_cache, const void *__restrict__ v_cache,
                                                const int32_t *__restrict__ bt_row, int t0, int p1, int block_size, int64_t tok_stride,
-                                               int kvh, int lane, int bt_reg = 0) {
+                                               int kvh, int lane, int bt_reg = 0, int bt_base = 0) {
     constexpr int KSTEPS = HD / 32, NP = HD >= 128 ? HD / 128 : 1;
     const int tl = lane & 15, dg = lane >> 4;
     const bool lane_live = (HD >= 128) || (lane < 32);
     const int ntok = min(16, p1 - t0);
     const int tok = t0 + min(tl, ntok - 1);
-    const int blk = BTREG ? __shfl(bt_reg, tok / block_size, 64) : bt_row[tok / block_size];
+    const int blk = BTREG ? __shfl(bt_reg, tok / block_size - bt_base, 64) : bt_row[tok / block_size];
     const int64_t base = ((int64_t)blk * block_size + tok % block_size) * tok_stride + (int64_t)kvh * HD;
 #pragma unroll
     for (int i = 0; i < KSTEPS; i++) t.kraw[i] = load8_raw<FP8>(k_cache, base + 32 * i + 8 * dg);
@@ -231,7 +231,7 @@ __device__ __forceinline__ void attn_walk(const uint4 (&qa)[HD / 32], const void
                                           const int32_t *__restrict__ bt_row, int p0, int p1, int block_size, int64_t tok_stride,
                                           int kvh, float lscale, float vsc, int lane, float (&m_run)[4], float (&s_run)[4],
                                           float (&o)[QPK][HD >= 128 ? HD / 128 : 1][2], AttnTile<HD, FP8> &first, bool first_loaded,
-                                          int bt_reg = 0) {
+                                          int bt_reg = 0, int bt_base = 0) {
     constexpr int NP = HD >= 128 ? HD / 128 : 1;
 #pragma unroll
     for (int r = 0; r < 4; r++) { m_run[r] = -FLT_MAX; s_run[r] = 0.f; }
@@ -239,11 +239,11 @@ __device__ __forceinline__ void attn_walk(const uint4 (&qa)[HD / 32], const void
     for (int h = 0; h < QPK; h++)
 #pragma unroll
         for (int p = 0; p < NP; p++) o[h][p][0] = o[h][p][1] = 0.f;
-    if (!first_loaded) attn_tile_load<HD, FP8, BTREG>(first, k_cache, v_cache, bt_row, p0, p1, block_size, tok_stride, kvh, lane, bt_reg);
+    if (!first_loaded) attn_tile_load<HD, FP8, BTREG>(first, k_cache, v_cache, bt_row, p0, p1, block_size, tok_stride, kvh, lane, bt_reg, bt_base);
     for (int t0 = p0; t0 < p1; t0 += 16) {   // the next tile is requested before the current one is folded
         AttnTile<HD, FP8> next;
         const bool more = t0 + 16 < p1;
-        if (more) attn_tile_load<HD, FP8, BTREG>(next, k_cache, v_cache, bt_row, t0 + 16, p1, block_size, tok_stride, kvh, lane, bt_reg);
+        if (more) attn_tile_load<HD, FP8, BTREG>(next, k_cache, v_cache, bt_row, t0 + 16, p1, block_size, tok_stride, kvh, lane, bt_reg, bt_base);
         attn_tile_fold<HD, QPK, FP8>(first, min(16, p1 - t0), qa, lscale, vsc, lane, m_run, s_run, o);
         if (more) first = next;
     }
@@ -824,7 +824,7 @@ __global__ __launch_bounds__(64 * NW) void split_decode_attn_kernel(
     const int pos = positions[seq];
     const int slot = slots[seq];
     const int32_t *bt_row = block_tables + (int64_t)seq * max_blocks_per_seq;
-    const int bt_reg = bt_row[min(lane, max_blocks_per_seq - 1)];
+    int bt_reg = bt_row[min(lane, max_blocks_per_seq - 1)], bt_base = 0;
     const float ksc = (FP8 && k_scale_ptr) ? *k_scale_ptr : 1.0f;
     const float vsc = (FP8 && v_scale_ptr) ? *v_scale_ptr : 1.0f;
 
@@ -874,12 +874,17 @@ __global__ __launch_bounds__(64 * NW) void split_decode_attn_kernel(
     const int w0 = ng >= NW ? g0 + wave * ng / NW : g0 + min(wave, ng), w1 = ng >= NW ? g0 + (wave + 1) * ng / NW : g0 + min(wave + 1, ng);
     const bool active = seq_len > 0 && w0 < w1;
     const int p0 = start + 16 * w0, p1 = min(start + 16 * w1, seq_len);
-    // block-table entries in a register: every token of the walk lies in the first 64 blocks
-    const bool bt_regs = (seq_len + block_size - 1) / block_size <= 64;
+    // block-table entries in a register: every token of the walk lies in the first 64 blocks, or else in 64 of the wave's own
+    bool bt_regs = (seq_len + block_size - 1) / block_size <= 64;
+    if (!bt_regs && active && (p1 - 1) / block_size - p0 / block_size < 64) {
+        bt_base = p0 / block_size;
+        bt_reg = bt_row[min(bt_base + lane, max_blocks_per_seq - 1)];
+        bt_regs = true;
+    }
     AttnTile<HD, FP8> tile;
     const bool pre = active && p0 + 16 < seq_len;
     if (pre) {
-        if (bt_regs) attn_tile_load<HD, FP8, true>(tile, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, lane, bt_reg);
+        if (bt_regs) attn_tile_load<HD, FP8, true>(tile, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, lane, bt_reg, bt_base);
         else attn_tile_load<HD, FP8, false>(tile, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, lane);
     }
 
@@ -955,7 +960,7 @@ __global__ __launch_bounds__(64 * NW) void split_decode_attn_kernel(
         }
         if (bt_regs)
             attn_walk<HD, QPK, FP8, true>(qa, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, scale * ksc, vsc, lane,
-                                          m_run, s_run, o, tile, pre, bt_reg);
+                                          m_run, s_run, o, tile, pre, bt_reg, bt_base);
         else
             attn_walk<HD, QPK, FP8, false>(qa, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, scale * ksc, vsc, lane,
                                            m_run, s_run, o, tile, pre);
@@ -1489,8 +1494,8 @@ size_t vmx_split_decode_attention_workspace_bytes(int num_seqs, int num_heads, i
     return (size_t)num_seqs * num_heads * 8 * ((size_t)head_dim + 2) * 4;
 }
 
-// Contexts beyond the reach of the few-partition form (from 512 tokens on): the same kernel with 8 ... 64 workgroups of 8 waves per KV head (as many
-// as give every compute unit one workgroup) and the separate merge (vmx_paged_attention_merge) behind it, in place of
+// Contexts beyond the reach of the few-partition form (from 512 tokens on): the same kernel with 1 ... 64 workgroups of 8 waves per KV head (as many
+// as give every compute unit one workgroup, or two where they would be fewer than four) and the separate merge (vmx_paged_attention_merge) behind it, in place of
 // "q/k/v post-processing + one wave per partition + merge": at 8192 tokens the one-wave partitions put 464 waves on the
 // chip for 24 us per layer (Qwen3-8B, one row).  Returns the partition count, 0 = not covered.  VMX_NO_SPLIT_ATTN_LONG=1
 // switches the form off.
@@ -1502,12 +1507,15 @@ int vmx_split_decode_attention_long_parts(int head_dim, int qpk, int rot_dim, in
     const int ctx = window > 0 && window < max_seq_len ? window : max_seq_len;
     if (ctx <= split_long_min_ctx()) return 0;
     static const int p_env = vmx_tune("VMX_SPLIT_LONG_P", 0);   // measurement: force the count
-    if (p_env >= 8 && p_env <= 64) return p_env;
+    if (p_env >= 1 && p_env <= 64) return p_env;
     // one workgroup per compute unit: measured on Qwen3-8B (8 KV heads, one row) at 1024 ... 32768 tokens, 32 partitions beat
     // 12 / 16 / 24 / 64 at every length (8192 tokens: 420 / 440 / 475 / 441 against 478 tok/s; 33 partitions = 264 workgroups
     // on 256 compute units cost 6 %)
-    const int per = vmx_num_cus() / (num_kv_heads * num_seqs > 0 ? num_kv_heads * num_seqs : 1);
-    return per < 8 ? 8 : (per > 64 ? 64 : per);
+    // Many rows: a compute unit holds two workgroups, and more than that many only repeat the prologue of q heads (16 rows of 1500 /
+    // 700 tokens: 8 partitions 31.8 / 21.8 us, 4 partitions 26.1 / 17.9, 2 partitions 28.3 / 18.0; 12 rows of 2000: 2 / 4 / 6 = 31.9 /
+    // 29.3 / 30.8; 8 rows of 500: 8 partitions 10.3, 4 9.9; 4 rows of 1500: 8 / 16 = 13.7 / 13.2; 1 row of 1500: 32 / 64 = 9.0 / 10.2)
+    const int pairs = num_kv_heads * num_seqs > 0 ? num_kv_heads * num_seqs : 1, per = vmx_num_cus() / pairs, two = 2 * vmx_num_cus() / pairs;
+    return per >= 4 ? (per > 64 ? 64 : per) : two < 1 ? 1 : two > 4 ? 4 : two;
 }
 size_t vmx_split_decode_attention_long_workspace_bytes(int num_seqs, int num_heads, int head_dim, int parts) {
     return (size_t)num_seqs * num_heads * parts * ((size_t)head_dim + 2) * 4;
