@@ -45,15 +45,17 @@ def test_dense_decode_rows(gpu, geometry, contexts):
         model.close()
 
 
+# every head width (heads, KV heads, head_dim, FP8 cache): the q/k/v kernel's lanes a head, the attention's tiles before, at and past 16 tokens
+@pytest.mark.parametrize("heads,kv_heads,head_dim,fp8", [(3, 1, 64, 0), (2, 1, 128, 1), (2, 1, 256, 0), (3, 1, 256, 1), (2, 2, 512, 0), (4, 1, 512, 1)])
 @pytest.mark.parametrize("tokens", [2, 17, 40])
-def test_dense_prompt_rows(gpu, tokens):
+def test_dense_prompt_rows(gpu, tokens, heads, kv_heads, head_dim, fp8):
     """The last hidden row of a prompt pass against the oracle fed the same tokens one at a time."""
     from tests.model_oracle import OracleQwen3
     from vllm_rust_amd.qwen3 import QuantizedQwen3ForCausalLM, Qwen3Spec, rope_cos_sin_cache
     from oracle import oracle as orc
     vmx, torch = gpu
-    spec = Qwen3Spec(640, 3, 3, 1, 64, 1152, 512, tie_word_embeddings=True, max_position=256, num_blocks=8, max_batch=1, max_seq_len=64,
-                     max_prefill_tokens=48)
+    spec = Qwen3Spec(640, 3, heads, kv_heads, head_dim, 1152, 512, tie_word_embeddings=True, max_position=256, num_blocks=8, max_batch=1,
+                     max_seq_len=64, max_prefill_tokens=48, kv_cache_dtype=fp8)
     model = QuantizedQwen3ForCausalLM(spec)
     try:
         ck = model.load_synthetic_bf16(seed=5, keep_host_copy=True)
