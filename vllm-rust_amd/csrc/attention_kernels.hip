@@ -1100,7 +1100,9 @@ static int parts_for_impl(int max_seq_len) {
 // paged cache holds for the sequence up to and including themselves (the caller wrote the new K/V rows first, as the
 // reference's naive backend does: write, read back, softmax(QK^T * scale + mask) V; layers/attention/naive.rs:38-83).
 // Flash-style on the matrix cores.  A workgroup = 4 waves = up to 4 query heads of one KV head x 16-token query tiles;
-// KV tiles of 16 tokens are staged through LDS once per workgroup (K row-major, V transposed), then per wave
+// KV tiles of 16 tokens are staged through LDS once per workgroup (K row-major, V transposed; the next tile's rows are under way while a
+// tile is multiplied: 256 tokens of Gemma-4-12B, a chain of up to 16 tiles in 64 workgroups that its latency bounds, 48.7 -> 28.6 us
+// with 256-wide and 74 -> 46 us with 512-wide heads), then per wave
 //   S^T = K Q^T      v_mfma_f32_16x16x32_bf16: A = K rows (row = token), B = the wave's q rows (column = query token);
 //                    the accumulator then holds, per lane, 4 consecutive tokens of ONE query row, which is
 //   O^T += V^T P^T   exactly the B fragment of v_mfma_f32_16x16x16_bf16 (k = token); A = V^T from LDS (row = head dim).
@@ -1120,8 +1122,8 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(uint16_t *__restrict_
     constexpr int KSTEPS = HD / 32, DT = HD / 16;
     constexpr int KROW = HD + 8;             // bf16 per K row in LDS (16 B pad)
     constexpr int VROW = 20;                 // bf16 per V^T row: 16 tokens + pad (rows stay 8-byte aligned)
-    __shared__ __align__(16) uint16_t Ks[16 * KROW];
-    __shared__ __align__(16) uint16_t Vt[HD * VROW];
+    constexpr int BUF = 16 * KROW + HD * VROW, CHUNKS = HD / 128;   // 16 x HD / 8 pieces of eight elements, CHUNKS a thread
+    extern __shared__ __align__(16) uint16_t pf_lds[];              // two tiles, written and read in turn
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, n = lane & 15;
     const int hh = wave % HPW, tt = wave / HPW;
@@ -1155,32 +1157,53 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(uint16_t *__restrict_
 #pragma unroll
     for (int d = 0; d < DT; d++) acc[d] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
 
-    for (int t0 = lo; t0 < hi; t0 += 16) {
-        __syncthreads();   // the previous tile is no longer read
-        for (int c = tid; c < 2 * HD; c += 256) {   // 16 tokens x HD / 8 chunks of 8 elements
-            const int tok = c / (HD / 8), dc = c % (HD / 8);
-            const int t = min(t0 + tok, hi - 1);    // rows past the end repeat the last valid row (their weights are 0)
-            const int blk = block_table[t / block_size];
-            const int64_t base = ((int64_t)blk * block_size + t % block_size) * tok_stride + (int64_t)kvh * HD + dc * 8;
-            if constexpr (FP8 == 3) {   // fp16 cache, fp16 matrix instructions: the bits go to LDS as they are
-                const uint4 kr = load8_raw<FP8>(k_cache, base), vr = load8_raw<FP8>(v_cache, base);
-                *reinterpret_cast<uint4 *>(&Ks[tok * KROW + dc * 8]) = kr;
-                const uint32_t vw[4] = {vr.x, vr.y, vr.z, vr.w};
+    // A tile's rows are requested while the one before it is multiplied, their block-table entry one tile earlier still.  Thread -> token
+    // tid % 16, so that the sixteen lanes of a V^T row's store share its banks out; rows past the end repeat the last valid row (weight 0).
+    const int tok = tid & 15, dc0 = tid >> 4;
+    auto entry = [&](int t0) { return block_table[min(t0 + tok, hi - 1) / block_size]; };
+    typename Raw8<FP8>::T kr[CHUNKS > 0 ? CHUNKS : 1], vr[CHUNKS > 0 ? CHUNKS : 1];
+    auto request = [&](int t0, int blk) {
+        const int64_t base = ((int64_t)blk * block_size + min(t0 + tok, hi - 1) % block_size) * tok_stride + (int64_t)kvh * HD;
+#pragma unroll
+        for (int i = 0; i < (CHUNKS > 0 ? CHUNKS : 1); i++)
+            if (CHUNKS > 0 || tid < 2 * HD) {
+                kr[i] = load8_raw<FP8>(k_cache, base + (dc0 + 16 * i) * 8);
+                vr[i] = load8_raw<FP8>(v_cache, base + (dc0 + 16 * i) * 8);
+            }
+    };
+    int blk_next = 0, turn = 0;
+    if (lo < hi) {
+        request(lo, entry(lo));
+        blk_next = entry(lo + 16);
+    }
+    for (int t0 = lo; t0 < hi; t0 += 16, turn ^= 1) {
+        uint16_t *Ks = pf_lds + turn * BUF, *Vt = Ks + 16 * KROW;
+#pragma unroll
+        for (int i = 0; i < (CHUNKS > 0 ? CHUNKS : 1); i++) {
+            const int dc = dc0 + 16 * i;
+            if (CHUNKS == 0 && tid >= 2 * HD) continue;
+            if constexpr (kv16<FP8>()) {   // bf16 or fp16 rows: the bits go to LDS as they are
+                *reinterpret_cast<uint4 *>(&Ks[tok * KROW + dc * 8]) = kr[i];
+                const uint32_t vw[4] = {vr[i].x, vr[i].y, vr[i].z, vr[i].w};
 #pragma unroll
                 for (int e = 0; e < 8; e++) Vt[(dc * 8 + e) * VROW + tok] = (uint16_t)(e & 1 ? vw[e >> 1] >> 16 : vw[e >> 1] & 0xFFFFu);
             } else {
-            float kf[8], vf[8];
-            cvt8<FP8>(load8_raw<FP8>(k_cache, base), 1.0f, kf);
-            cvt8<FP8>(load8_raw<FP8>(v_cache, base), 1.0f, vf);
-            uint32_t kw[4];
+                float kf[8], vf[8];
+                cvt8<FP8>(kr[i], 1.0f, kf);
+                cvt8<FP8>(vr[i], 1.0f, vf);
+                uint32_t kw[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) kw[j] = (__float_as_uint(kf[2 * j]) >> 16) | (__float_as_uint(kf[2 * j + 1]) & 0xFFFF0000u);
-            *reinterpret_cast<uint4 *>(&Ks[tok * KROW + dc * 8]) = make_uint4(kw[0], kw[1], kw[2], kw[3]);
+                for (int j = 0; j < 4; j++) kw[j] = (__float_as_uint(kf[2 * j]) >> 16) | (__float_as_uint(kf[2 * j + 1]) & 0xFFFF0000u);
+                *reinterpret_cast<uint4 *>(&Ks[tok * KROW + dc * 8]) = make_uint4(kw[0], kw[1], kw[2], kw[3]);
 #pragma unroll
-            for (int e = 0; e < 8; e++) Vt[(dc * 8 + e) * VROW + tok] = (uint16_t)(__float_as_uint(vf[e]) >> 16);
+                for (int e = 0; e < 8; e++) Vt[(dc * 8 + e) * VROW + tok] = (uint16_t)(__float_as_uint(vf[e]) >> 16);
             }
         }
-        __syncthreads();
+        if (t0 + 16 < hi) {
+            request(t0 + 16, blk_next);
+            blk_next = entry(t0 + 32);
+        }
+        __syncthreads();   // one a tile: a wave that is a tile ahead writes the other buffer
         // wave-uniform: does this KV tile intersect the wave's causal / window range at all
         const bool need = wave_live && t0 <= wave_last_pos && (window <= 0 || t0 + 15 > wave_first_pos - window);
         if (need) {
@@ -1247,7 +1270,10 @@ int launch_prefill(hipStream_t st, uint16_t *out, const uint16_t *q, const void 
                    float scale, int H, int KVH, int bs, int window, const float *ks, const float *vs) {
     constexpr int HPW = QPK < 4 ? QPK : 4, TT = 4 / HPW;
     const dim3 grid((q_len + 16 * TT - 1) / (16 * TT), KVH * (QPK / HPW));
-    hipLaunchKernelGGL((prefill_attn_kernel<HD, QPK, FP8>), grid, dim3(256), 0, st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window,
+    constexpr size_t lds = 2 * (16 * (HD + 8) + HD * 20) * 2;
+    if (lds > 64 * 1024)
+        VMX_CHECK_HIP(hipFuncSetAttribute((const void *)prefill_attn_kernel<HD, QPK, FP8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((prefill_attn_kernel<HD, QPK, FP8>), grid, dim3(256), lds, st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window,
                        ks, vs);
     VMX_CHECK_LAUNCH("prefill_attention");
     return VMX_OK;
