@@ -1,0 +1,56 @@
+"""Latent attention over rows of 512 + 64 values (the form with constant sizes and rows requested a tile ahead) at the edges of its
+64-key tiles: prompts with more row tiles than compute units (not partitioned) and decode steps (partitioned)."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import torch
+    import vllm_rust_amd as vmx
+    vmx.init(0)
+    return vmx, torch
+
+
+# (contexts per sequence, new tokens per sequence, heads, window)
+@pytest.mark.parametrize("contexts,new,heads,window", [
+    ([300], 300, 16, 0), ([321], 257, 16, 70), ([64, 63, 65, 1], 1, 16, 0), ([128, 129, 700], 1, 20, 0), ([200, 513], 3, 3, 64),
+    ([530, 90], 600, 8, 0),
+])
+def test_whole_rows(gpu, contexts, new, heads, window):
+    """Against float64 on the operands the kernel multiplies (bf16 rows, queries rounded to bf16).  A score is an f32 sum of 576 products
+    (off by at most d = 576 2^-24 scale sum |q k|), a weight is then off by a factor exp(2 d), its two bf16 halves by 2^-16, and the sums
+    of up to 1024 weighted rows by 1024 2^-24 of sum p |c| <= max |c|."""
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    R, RD, bs, scale = 512, 64, 16, 0.06
+    g = torch.Generator(device="cuda").manual_seed(sum(contexts) + heads)
+    n = len(contexts)
+    mb = (max(contexts) + bs - 1) // bs
+    bt = torch.randperm(n * mb, device="cuda", generator=g).to(torch.int32).view(n, mb)
+    cache = torch.randn((n * mb * bs, R + RD), device="cuda", generator=g).to(torch.bfloat16)
+    sid, pos = [], []
+    for b, c in enumerate(contexts):
+        k = min(new, c)
+        sid += [b] * k
+        pos += list(range(c - k, c))
+    T = len(pos)
+    qa = torch.randn((T, heads, R), device="cuda", generator=g).to(torch.bfloat16).float()
+    qr = torch.randn((T, heads, RD), device="cuda", generator=g).to(torch.bfloat16).float()
+    ts, tp = (torch.tensor(v, device="cuda", dtype=torch.int32) for v in (sid, pos))
+    out = torch.full((T, heads, R), float("nan"), device="cuda")
+    need = lib.vmx_latent_attention_workspace_bytes(T, heads, R, window, mb, bs)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    check(lib.vmx_latent_attention(out.data_ptr(), qa.data_ptr(), qr.data_ptr(), cache.data_ptr(), 1, bt.data_ptr(), mb, ts.data_ptr(), tp.data_ptr(),
+                                   None, scale, window, T, heads, R, RD, bs, ws.data_ptr(), ws.numel(), None))
+    torch.cuda.synchronize()
+    for t in range(T):
+        lo = max(0, pos[t] - window + 1) if window else 0
+        j = torch.arange(lo, pos[t] + 1, device="cuda")
+        rows = cache[bt[sid[t]].long()[j // bs] * bs + j % bs].double()
+        q = torch.cat([qa[t], qr[t]], 1).double()
+        d = 576 * 2.0 ** -24 * scale * (q.abs() @ rows.abs().T).max()
+        exact = torch.softmax(q @ rows.T * scale, 1) @ rows[:, :R]
+        bound = (torch.expm1(4 * d) + 2.0 ** -15 + 1024 * 2.0 ** -24) * rows[:, :R].abs().max()
+        assert bool(((out[t].double() - exact).abs() <= bound).all()), (t, float((out[t].double() - exact).abs().max()), float(bound))

@@ -234,25 +234,31 @@ struct LatentAttnArgs {
 
 constexpr int LA_KT = 64, LA_LD = LA_KT + 8;   // keys per tile; row stride of the P tiles
 constexpr int LA_PAD = 32;                    // the row-major latent tile pads its rows by 64 bytes: four consecutive rows, four bank groups
+typedef uint32_t la_u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) uint16_t la_lds;
 typedef short la_s16x4 __attribute__((ext_vector_type(4)));
 typedef short la_s16x8 __attribute__((ext_vector_type(8)));
 
-template <int KSMAX, int DTW>
-__global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const LatentAttnArgs a) {
+// WHOLE > 0: rows of exactly 32 KSMAX values with 64 DTW latents (512 + 64).  Every size is then a constant, which leaves the registers for
+// requesting a tile's rows while the one before it is worked on, and with WHOLE = 2 for two workgroups per compute unit: 1500 tokens
+// of 16 heads 270 -> 178 us.  A partitioned launch (decode steps: one workgroup per compute unit, a tile or two each) has WHOLE = 1,
+// which keeps the setup out of scratch memory: 16 rows of 1000 tokens 22.3 -> 17.9 us
+// (WHOLE = 2: 29.7).  Other sizes (0) request a tile's rows when its turn comes.
+template <int KSMAX, int DTW, int WHOLE>
+__global__ __launch_bounds__(256, WHOLE == 2 ? 2 : 1) void latent_attn_mfma_kernel(const LatentAttnArgs a) {
     extern __shared__ __align__(16) unsigned char la_smem[];
-    const int R = a.R, RW = a.R + a.rd;
-    const int ROWE = R + LA_PAD;
-    uint16_t *KT = reinterpret_cast<uint16_t *>(la_smem);            // [LA_KT][R + LA_PAD]: the tile's latents, row-major
+    const int R = WHOLE ? 64 * DTW : a.R, RW = WHOLE ? 32 * KSMAX : a.R + a.rd;
+    constexpr int ROWE = 64 * DTW + LA_PAD;   // of the largest latent this form takes, so that offsets are constants
+    uint16_t *KT = reinterpret_cast<uint16_t *>(la_smem);            // [LA_KT][ROWE]: the tile's latents, row-major
     uint16_t *Phi = KT + (size_t)LA_KT * ROWE;                        // [16][LA_LD]
     uint16_t *Plo = Phi + 16 * LA_LD;                                 // [16][LA_LD]
     float *red_max = reinterpret_cast<float *>(Plo + 16 * LA_LD);     // [4][16]
     float *red_sum = red_max + 64;                                    // [4][16]
-    int32_t *sl = reinterpret_cast<int32_t *>(red_sum + 64);          // [64]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fl = lane & 15, fg = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fl = lane & 15, fg = lane >> 4;
     const int tb = blockIdx.x / a.NHG, hg = blockIdx.x % a.NHG, part = blockIdx.y;
     const int t0 = tb * a.TPT, t_end = min(t0 + a.TPT, a.T);
-    const int ksteps = (RW + 31) >> 5;
-    const int dtiles = (R + 15) >> 4, dt_per_wave = (dtiles + 3) >> 2, dt0 = wave * dt_per_wave;
+    const int ksteps = WHOLE ? KSMAX : (RW + 31) >> 5;
+    const int dtiles = WHOLE ? 4 * DTW : (R + 15) >> 4, dt_per_wave = WHOLE ? DTW : (dtiles + 3) >> 2, dt0 = wave * dt_per_wave;
     for (int first = t0; first < t_end;) {
         const int seq = a.seq_ids[first];
         int last = first;
@@ -263,19 +269,19 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const LatentAttnA
         const int ntiles = (hi - lo) / LA_KT + 1, tpp = (ntiles + a.NP - 1) / a.NP;
         const int kt_begin = part * tpp, kt_end = min(ntiles, kt_begin + tpp);
         // A operand of S: the query of row fl
-        uint4 qf[KSMAX];
+        la_u32x4 qf[KSMAX];
         {
             const int tq = t0 + fl / a.HPT, hq = hg * a.HPT + fl % a.HPT;
             const bool act = fl < a.TPT * a.HPT && tq >= first && tq <= last && hq < a.H;
 #pragma unroll
             for (int s = 0; s < KSMAX; s++) {
                 const int k = 32 * s + 8 * fg;
-                uint4 v = make_uint4(0, 0, 0, 0);
+                la_u32x4 v = {0, 0, 0, 0};
                 if (s < ksteps && act && k < RW) {
                     const float *src = k < R ? a.q_abs + ((int64_t)tq * a.H + hq) * R + k : a.q_rot + ((int64_t)tq * a.H + hq) * a.rd + (k - R);
                     const float4 f0 = *reinterpret_cast<const float4 *>(src), f1 = *reinterpret_cast<const float4 *>(src + 4);
                     const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
-                    v = vmx_pack16x8<false>(f);
+                    v = __builtin_bit_cast(la_u32x4, vmx_pack16x8<false>(f));
                 }
                 qf[s] = v;
             }
@@ -295,44 +301,53 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const LatentAttnA
             m_r[r] = -FLT_MAX;
             l_r[r] = 0.f;
         }
+        la_lds *const kt_read = (la_lds *)KT + (8 * fg + (fl >> 2)) * ROWE + 16 * dt0 + 4 * (fl & 3);
         vmx_f32x4 acc[DTW];
 #pragma unroll
         for (int d = 0; d < DTW; d++) acc[d] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
-        // cache rows of a tile's keys: looked up one tile ahead, so the block table's latency is not on the tile's critical path
-        auto key_slot = [&](int kt) {
-            const int j = lo + LA_KT * kt + tid;
-            return (tid < LA_KT && kt < kt_end && j <= hi) ? bt[j / a.block_size] * a.block_size + j % a.block_size : -1;
+        // this wave's 16 keys of a tile: lane (n, g) reads the 16-byte chunks 32 s + 8 g of key n's cache row.  They are the B operand of
+        // the score product and, for the latent part of the row, the tile of the value product: each chunk is also written to
+        // KT[key][latent dim], so the cache is read once per tile.  WHOLE: the rows are requested one tile ahead, as soon as the score
+        // product has let go of the registers, and their block-table entry two.  Keys past `hi` repeat its row; their weights are 0.
+        auto key_row = [&](int kt) {
+            const int j = min(lo + LA_KT * kt + 16 * wave + fl, hi);
+            return bt[j / a.block_size] * a.block_size + j % a.block_size;
         };
-        int next_slot = key_slot(kt_begin);
+        la_u32x4 kf[KSMAX];
+        auto request = [&](int row) {
+            const uint16_t *at = a.cache + (int64_t)row * RW + 8 * fg;
+#pragma unroll
+            for (int s = 0; s < KSMAX; s++) {
+                if (!WHOLE) kf[s] = la_u32x4{0, 0, 0, 0};
+                if (WHOLE || (s < ksteps && 32 * s + 8 * fg < RW)) kf[s] = *reinterpret_cast<const la_u32x4 *>(at + 32 * s);
+            }
+        };
+        int next_row = 0;
+        if (kt_begin < kt_end) {
+            if (WHOLE) request(key_row(kt_begin));
+            next_row = key_row(kt_begin + (WHOLE ? 1 : 0));
+        }
         for (int kt = kt_begin; kt < kt_end; kt++) {
             const int kbase = lo + LA_KT * kt;
-            __syncthreads();   // the previous tile's latents / P / slots have been read
-            if (tid < LA_KT) sl[tid] = next_slot;
-            __syncthreads();
-            next_slot = key_slot(kt + 1);
-            // this wave's 16 keys: lane (n, g) reads the 16-byte chunks 32 s + 8 g of key n's cache row.  They are the B operand of
-            // the score product and, for the latent part of the row, the tile of the value product: each chunk is also written to
-            // KT[key][latent dim], so the cache is read once per tile.
+            if (!WHOLE) {
+                request(next_row);
+                next_row = key_row(kt + 1);
+            }
+            __syncthreads();   // the previous tile's latents and P have been read
             vmx_f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
-            {
-                const int slot = sl[16 * wave + fl];
-                uint4 kf[KSMAX];
 #pragma unroll
-                for (int s = 0; s < KSMAX; s++) {
-                    const int k = 32 * s + 8 * fg;
-                    kf[s] = make_uint4(0, 0, 0, 0);
-                    if (s < ksteps && slot >= 0 && k < RW) kf[s] = *reinterpret_cast<const uint4 *>(a.cache + (int64_t)slot * RW + k);
-                }
+            for (int s = 0; s < KSMAX; s++) {
+                const int k = 32 * s + 8 * fg;
+                if (s < ksteps && k < R) *reinterpret_cast<la_u32x4 *>(KT + (16 * wave + fl) * ROWE + k) = kf[s];
+            }
 #pragma unroll
-                for (int s = 0; s < KSMAX; s++) {
-                    const int k = 32 * s + 8 * fg;
-                    if (s < ksteps && k < R) *reinterpret_cast<uint4 *>(KT + (16 * wave + fl) * ROWE + k) = kf[s];
-                }
-#pragma unroll
-                for (int s = 0; s < KSMAX; s++)
-                    if (s < ksteps)
-                        sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, qf[s]), __builtin_bit_cast(vmx_bf16x8, kf[s]), sacc,
-                                                                       0, 0, 0);
+            for (int s = 0; s < KSMAX; s++)
+                if (s < ksteps)
+                    sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, qf[s]), __builtin_bit_cast(vmx_bf16x8, kf[s]), sacc, 0, 0,
+                                                                   0);
+            if (WHOLE && kt + 1 < kt_end) {
+                request(next_row);
+                next_row = key_row(kt + 2);
             }
             const int j = kbase + 16 * wave + fl;
             bool ok[4];
@@ -372,14 +387,14 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const LatentAttnA
                 for (int r = 0; r < 4; r++) acc[d][r] *= alpha[r];
 #pragma unroll
             for (int ks = 0; ks < LA_KT / 32; ks++) {
-                const uint4 ah = *reinterpret_cast<const uint4 *>(Phi + fl * LA_LD + 32 * ks + 8 * fg);
-                const uint4 al = *reinterpret_cast<const uint4 *>(Plo + fl * LA_LD + 32 * ks + 8 * fg);
+                const la_u32x4 ah = *reinterpret_cast<const la_u32x4 *>(Phi + fl * LA_LD + 32 * ks + 8 * fg);
+                const la_u32x4 al = *reinterpret_cast<const la_u32x4 *>(Plo + fl * LA_LD + 32 * ks + 8 * fg);
 #pragma unroll
                 for (int d = 0; d < DTW; d++) {
-                    if (d < dt_per_wave && dt0 + d < dtiles) {
+                    if (WHOLE || (d < dt_per_wave && dt0 + d < dtiles)) {
                         // B operand = C^T: the transposing LDS read hands lane n the values of column 16 dt + n for the four rows
                         // (keys) its 16-lane group addressed; two reads give the eight keys 32 ks + 8 g .. + 7 of this lane's k slots
-                        const uint16_t *src = KT + (32 * ks + 8 * fg + (fl >> 2)) * ROWE + 16 * (dt0 + d) + 4 * (fl & 3);
+                        la_lds *const src = kt_read + 32 * ks * ROWE + 16 * d;
                         const la_s16x4 c0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((la_s16x4 __attribute__((address_space(3))) *)src);
                         const la_s16x4 c1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((la_s16x4 __attribute__((address_space(3))) *)(src + 4 * ROWE));
                         const la_s16x8 cf = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
@@ -534,13 +549,19 @@ extern "C" int vmx_latent_attention(float *out_latent, const float *q_abs, const
         a.part_m = (float *)workspace;
         a.part_l = a.part_m + (size_t)tokens * heads * a.NP;
         a.part_o = a.part_l + (size_t)tokens * heads * a.NP;
-        const size_t lds = ((size_t)LA_KT * (kv_rank + LA_PAD) + 2 * 16 * LA_LD) * 2 + (64 + 64) * 4 + 64 * 4;
         dim3 grid((unsigned)(((tokens + a.TPT - 1) / a.TPT) * a.NHG), a.NP);
         const bool small = RW <= 160 && kv_rank <= 128;
-        const void *fn = small ? (const void *)latent_attn_mfma_kernel<5, 2> : (const void *)latent_attn_mfma_kernel<18, 8>;
+        const size_t lds = ((size_t)LA_KT * ((small ? 128 : 512) + LA_PAD) + 2 * 16 * LA_LD) * 2 + (64 + 64) * 4;
+        const bool whole = kv_rank == 512 && rot_dim == 64;
+        const void *fn = small              ? (const void *)latent_attn_mfma_kernel<5, 2, 0>
+                         : !whole           ? (const void *)latent_attn_mfma_kernel<18, 8, 0>
+                         : a.NP > 1         ? (const void *)latent_attn_mfma_kernel<18, 8, 1>
+                                            : (const void *)latent_attn_mfma_kernel<18, 8, 2>;
         if (lds > 64 * 1024) VMX_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        if (small) hipLaunchKernelGGL((latent_attn_mfma_kernel<5, 2>), grid, dim3(256), lds, st, a);
-        else hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8>), grid, dim3(256), lds, st, a);
+        if (small) hipLaunchKernelGGL((latent_attn_mfma_kernel<5, 2, 0>), grid, dim3(256), lds, st, a);
+        else if (!whole) hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8, 0>), grid, dim3(256), lds, st, a);
+        else if (a.NP > 1) hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8, 1>), grid, dim3(256), lds, st, a);
+        else hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8, 2>), grid, dim3(256), lds, st, a);
         VMX_CHECK_LAUNCH("latent_attention (matrix cores)");
         if (a.NP > 1) {
             hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(tokens * heads), dim3(256), 0, st, out_latent, a.part_m, a.part_l, a.part_o, sink_bf16,
