@@ -603,7 +603,8 @@ struct Int4Linear {
     DevBuf packed;
     bool loaded = false;
     bool glu = false;  // merged gate|up packed for the fused activation epilogue (forward_glu instead of forward_partial)
-    int splits() const { return vmx_int4_splits(out_features, in_features); }
+    int splits() const { return vmx_int4_splits(out_features, in_features); }   // the most
+    int splits(int M) const { return vmx_int4_splits_rows(M, out_features, in_features); }
     int forward_partial(const uint16_t *x, float *partial, int M, hipStream_t st) const {
         return vmx_int4_gemm_partial(packed.p, x, partial, M, out_features, in_features, group, st);
     }
@@ -1319,9 +1320,8 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
         const bool dn = !moe && !L.int4_ready() && !ex && !L.iq_ready() && L.dense_ready();   // unquantized layer: bf16 matrices
         const bool iq = !moe && !L.int4_ready() && !ex && !dn;       // GGUF I-quant layer: every projection is an IqLinear
         const bool one = iq || ex || dn;                             // linear outputs arrive as one f32 slice
-        int s_qkv = one ? 1 : L.qkv.splits();
-        const int s_o = one ? 1 : L.o.splits(), s_gu = one ? 1 : L.gate_up.splits(),
-                  s_down = one ? 1 : L.down.splits();
+        int s_qkv = one ? 1 : L.qkv.splits(B);
+        const int s_o = one ? 1 : L.o.splits(B), s_gu = one ? 1 : L.gate_up.splits(B), s_down = one ? 1 : L.down.splits(B);
         // h += pending; x = rms_norm(h);  q|k|v = linear(x)
         // EXL3 decode rows: the consumers of o, gate|up and down apply the output transform themselves (one launch less each)
         const bool ex_fold = ex && B <= 4 && !tp && H % 128 == 0 && I % 128 == 0 && L.ex_svh_gu.p;

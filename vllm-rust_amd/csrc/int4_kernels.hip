@@ -1878,14 +1878,33 @@ static void launch_tiled(const uint4 *W, const uint32_t *SZ, const uint16_t *x, 
 // ---- internal (C++) entry points used by the decoder ---------------------------------------
 int vmx_int4_splits(int N, int K) { return plan_gemm(N, K).splits; }
 
-// partial[splits][M][N] f32, also when splits == 1.  Arguments must already satisfy check_int4_shape.
+// Slices that vmx_int4_gemm_partial writes for M rows, at most vmx_int4_splits.  A prompt's tiles may fill the chip by themselves; every
+// further slice is then f32 rows written and read again.  Taken is the count whose last round of workgroups (two fit a compute unit)
+// ends first, the smallest of equals.  2048 tokens of Qwen3-8B: o 4 slices -> 1, down 3 -> 1, q|k|v (768 tiles) 2 as before: the three
+// products together 421 -> 405 us a layer, the norm kernel that adds the slices 26 -> 15.5.
+int vmx_int4_splits_rows(int M, int N, int K) {
+    const int plan = plan_gemm(N, K).splits, kblocks = K / KB;
+    if (plan == 1 || !tiled_ok(M, N, K)) return plan;
+    const int64_t tiles = (int64_t)(N >> 8) * ((M + PF_BM - 1) / PF_BM), slots = 2 * (int64_t)vmx_num_cus();
+    int best = plan;
+    int64_t least = INT64_MAX;
+    for (int s = 1; s <= plan; s++) {
+        const int kbs = (kblocks + s - 1) / s;
+        if (!tiled_wide_ok(M, N, K, kbs) || (s < plan && (s - 1) * kbs >= kblocks)) continue;
+        const int64_t cost = (tiles * s + slots - 1) / slots * kbs;
+        if (cost < least) least = cost, best = s;
+    }
+    return best;
+}
+
+// partial[vmx_int4_splits_rows][M][N] f32, also with one slice.  Arguments must already satisfy check_int4_shape.
 int vmx_int4_gemm_partial(const void *packed, const uint16_t *x, float *partial, int M, int N, int K, int group, hipStream_t st) {
     const GemmPlan p = plan_gemm(N, K);
     const uint4 *W = (const uint4 *)packed;
     const uint32_t *SZ = (const uint32_t *)((const char *)packed + sz_offset_bytes(K, N));
-    if (tiled_ok(M, N, K)) {   // prompt chunk: 64 x 128 output tiles, the same split-K slices as the small-M plan
-        const int kblocks = K / KB, kbs = (kblocks + p.splits - 1) / p.splits;
-        launch_tiled<false, false>(W, SZ, x, partial, nullptr, M, N, K, group, kbs, M, Int4GroupedArgs{}, (M + PF_BM - 1) / PF_BM, p.splits, st);
+    if (tiled_ok(M, N, K)) {   // prompt chunk
+        const int splits = vmx_int4_splits_rows(M, N, K), kblocks = K / KB, kbs = (kblocks + splits - 1) / splits;
+        launch_tiled<false, false>(W, SZ, x, partial, nullptr, M, N, K, group, kbs, M, Int4GroupedArgs{}, (M + PF_BM - 1) / PF_BM, splits, st);
         VMX_CHECK_LAUNCH("int4_gemm(tiled)");
         return VMX_OK;
     }

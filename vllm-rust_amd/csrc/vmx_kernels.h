@@ -4,6 +4,7 @@
 
 // int4_kernels.hip
 int vmx_int4_splits(int N, int K);
+int vmx_int4_splits_rows(int M, int N, int K);   // of M rows: what vmx_int4_gemm_partial writes
 int vmx_int4_gemm_grouped(const void *const *packed_table, const int32_t *expert_ids, int num_experts, const uint16_t *x,
                           int x_row_div, float *partial, int pairs, int N, int K, int group, hipStream_t st);
 int vmx_int4_gemm_partial(const void *packed, const uint16_t *x, float *partial, int M, int N, int K, int group, hipStream_t st);
