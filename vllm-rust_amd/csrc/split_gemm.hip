@@ -308,7 +308,6 @@ int vmx_bf16_rows_to_f16(const uint16_t *A, uint16_t *a16, int64_t n, hipStream_
 namespace {
 typedef TgShape<2, 2, 2, 2, 2> IntWide;     // 128 x 128
 typedef TgShape<2, 2, 1, 2, 2> IntMid;      // 64 x 128
-typedef TgShape<2, 2, 1, 1, 2> IntSmall;    // 64 x 64
 
 template <class S, bool GEGLU>
 void launch_int_tile(const uint16_t *a16, const uint16_t *Q, const float *Dt, float *C, uint16_t *act, int M, int N, int K, int64_t ldc, int slices,
