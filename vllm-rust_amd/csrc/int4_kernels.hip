@@ -1265,13 +1265,6 @@ __global__ __launch_bounds__(256) void int4_gemm_tiled_kernel(const uint4 *__res
 // us against the form it replaces (64 x 64 per wave in 16 x 16 accumulators, every LDS read behind the next tile's arrival), rows x columns x
 // depth: 2048 x 24576 x 4096 545 -> 481 (857 TFLOP/s, matrix cores 56 % busy, 1.8 GHz), 333 x 24576 x 4096 124 -> 104, 100 x 24576 x 4096
 // 58 -> 42, 2048 x 4096 x 12288 267 -> 249.  N % 256 == 0.
-// (w & 0x000F000F) | base in one instruction (the compiler emits v_and + v_or: VOP3 takes no second literal)
-__device__ __forceinline__ uint32_t nib_pair(uint32_t w, uint32_t base) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(w), "s"(0x000F000Fu), "v"(base));
-    return r;
-}
-
 // v cut into bf16 parts: parts[0] + parts[1] + .. = v to the last bit that they hold
 template <int P>
 __device__ __forceinline__ void bf16_parts(float v, uint16_t (&part)[P]) {
