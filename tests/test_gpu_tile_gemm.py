@@ -86,6 +86,31 @@ def test_int4_prompt_tiles(gpu, M, N, K, group):
     assert bool(((y.double() - ref).abs() <= bound).all())
 
 
+# weights equal to their zero points: the product is exactly zero and the output is the rounding of the f32 sums itself
+@pytest.mark.parametrize("M,N,K", [(2048, 4096, 12288), (333, 1024, 16512)])
+@pytest.mark.parametrize("mean", [0, 1, 5])
+def test_int4_prompt_f32_sums(gpu, M, N, K, mean):
+    """The zero-point term comes off with every k-block, so no partial sum outgrows a k-block's offset (16 + zero point) s sum x.  A k-block
+    rounds eight chained products (sizes 1/8 .. 1: 3.2 in squares), four of its row sum (1.9), its scaling and its zero-point term; eight
+    roundings of at most 2^-24 of the largest prefix, of independent sign, bound the rms.  (Taken off once at the end, the sums grow with
+    the number of k-blocks: up to fifty times this bound.)"""
+    vmx, torch = gpu
+    g = torch.Generator(device="cuda").manual_seed(M + N + K + mean)
+    x = (torch.randn((M, K), device="cuda", generator=g) + mean).to(torch.bfloat16)
+    qz = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 128, N // 8), dtype=torch.int32, device="cuda", generator=g)
+    sc = ((torch.rand((K // 128, N), device="cuda", generator=g) + 0.5) * 0.01).to(torch.bfloat16)
+    zp = ((qz.unsqueeze(-1) >> torch.arange(0, 32, 4, dtype=torch.int32, device="cuda")) & 15).reshape(K // 128, N)
+    eight = torch.zeros_like(zp)
+    for i in range(8):
+        eight |= zp << (4 * i)
+    qw = eight.repeat_interleave(16, 0).contiguous()   # [K / 8, N]: eight nibbles of one column in a word
+    y = vmx.int4_gemm(x, vmx.int4_pack(qw, sc, qz, K, N, 128), None, N, K, 128).double()
+    torch.cuda.synchronize()
+    prefix = x.double().reshape(M, K // 128, 128).cumsum(2).abs().amax(2)
+    size = (prefix ** 2).mean().sqrt() * ((sc.double() * (16 + zp)) ** 2).mean().sqrt()
+    assert float((y ** 2).mean().sqrt()) <= float(2.0 ** -24 * (8 * K // 128) ** 0.5 * size)
+
+
 # decode rows: column groups below one per compute unit (halved k; 4 and 8 waves, a second round), between one and two, and above
 @pytest.mark.parametrize("M,N,K", [(1, 40, 72), (16, 2048, 2040), (5, 1000, 2312), (3, 4100, 520), (16, 4096, 1032), (7, 6000, 2056), (16, 9000, 136)])
 @pytest.mark.parametrize("x_f32", [False, True])

@@ -23,6 +23,8 @@
 
 namespace {
 
+typedef short i4_s16x4 __attribute__((ext_vector_type(4)));   // operand of the K = 8 bf16 matrix instruction
+
 constexpr int KB = 128;     // k-values per unit
 constexpr int NT = 16;      // columns per unit
 
@@ -1258,23 +1260,19 @@ __global__ __launch_bounds__(256) void int4_gemm_tiled_kernel(const uint4 *__res
 //   * weights go straight to registers, one k-block ahead.  A lane of the instruction's B operand is column l & 31: tile (l >> 4) & 1 of a
 //     pair, and of that tile's unit the words of the k chunks 2 t + (l >> 5) -- every byte of the unit is still used by one wave once;
 //   * fragments of the next 16 deep step are read and unpacked under the products of the current one;
-//   * the zero-point term -(s (128 + zp)) * (row sum of the k-block) costs no vector-ALU work per output: the row sums (a 16 x 16 matrix
-//     product with ones, wave w for rows 16 w ..) are kept in LDS for all k-blocks and multiplied with the factors at the end, 16 k-blocks
-//     per matrix step, both sides cut into bf16 parts that together hold all their bits (row sums three parts, factors two);
+//   * weights are unpacked to 16 + nibble (the nibble in the upper mantissa bits of 16.0), not 128 + nibble: one shift more a step, and every
+//     f32 sum runs at a sixth of the size;
+//   * the zero-point term -(s (16 + zp)) * (row sum of the k-block) costs no vector-ALU work per output: wave w leaves the sums of rows 16 w ..
+//     (a 16 x 16 matrix product with ones) in LDS, and one k-block later one v_mfma_f32_32x32x8_bf16 per accumulator adds the term, both
+//     sides cut into bf16 parts that together hold all their bits (row sums three parts, factors two).  The parts are rounded to nearest, so
+//     the lower ones have either sign: the instruction cuts small products off towards zero beside a large accumulator, which with
+//     parts of one sign adds up (rms error of 12288-deep sums x 5).  rms error against float64 where the product is zero, 2048 x 4096 x
+//     12288, rows of mean 0 / 1 / 5 and deviation 1: 1.0e-6 / 1.4e-5 / 4.4e-5; with 128 + nibble 7.6e-6 / 1.0e-4 / 2.7e-4 (16 x 16
+//     accumulators and vector-ALU terms: 7.0e-6 / 9.6e-5 / 2.4e-4); all terms at the end of the slice 3.4e-5 / 2.6e-3 / 1.4e-2;
 //   * the scales of a finished pair of column tiles are applied under the other pair's products.
-// us against the form it replaces (64 x 64 per wave in 16 x 16 accumulators, every LDS read behind the next tile's arrival), rows x columns x
-// depth: 2048 x 24576 x 4096 545 -> 481 (857 TFLOP/s, matrix cores 56 % busy, 1.8 GHz), 333 x 24576 x 4096 124 -> 104, 100 x 24576 x 4096
-// 58 -> 42, 2048 x 4096 x 12288 267 -> 249.  N % 256 == 0.
-// v cut into bf16 parts: parts[0] + parts[1] + .. = v to the last bit that they hold
-template <int P>
-__device__ __forceinline__ void bf16_parts(float v, uint16_t (&part)[P]) {
-#pragma unroll
-    for (int i = 0; i < P; i++) {
-        part[i] = vmx_f32_to_bf16(v);
-        v -= vmx_bf16_to_f32(part[i]);
-    }
-}
-
+// us against the form it replaced (64 x 64 per wave in 16 x 16 accumulators, every LDS read behind the next tile's arrival), rows x columns x
+// depth, packed weights in bf16 out: 2048 x 24576 x 4096 461 -> 424 (970 TFLOP/s), 333 x 24576 x 4096 121 -> 105, 100 x 24576 x 4096 58 -> 41,
+// 2048 x 4096 x 12288 224 -> 212.  N % 256 == 0.
 template <bool GLU, bool GROUPED = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void int4_gemm_prompt_kernel(
     const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ, const uint16_t *__restrict__ x, float *__restrict__ partial,
@@ -1283,7 +1281,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // ybf (one split only): the finished bf16 output y = bf16(sum + bias) instead of f32 slices
     __shared__ __align__(256) uint16_t xs[2][PF_BM * KB];
     __shared__ int32_t prow_s[PF_BM];
-    extern __shared__ __align__(16) float row_sums[];   // [k-blocks of the slice, rounded up to 16][PF_BM]
+    __shared__ __align__(16) uint2 row_parts[2][PF_BM];   // row sums of a k-block as three bf16 parts (and a zero), by turns
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nl = lane & 15, ct = (lane >> 4) & 1, kh = lane >> 5;
     const int kblocks = K / KB, G = K / group;
@@ -1358,13 +1356,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         sz[j] = (SZ + ((int64_t)(nt0 + 2 * j) * G + (gkb == 1 ? kb : kb / gkb)) * 16)[sz_at];
     };
     // (w & nibbles) | base in one v_and_or_b32: one operand from a scalar, one from a vector register (an instruction takes no two literals)
-    uint32_t base = 0x43004300u, nibbles = 0x000F000Fu;
+    uint32_t base = 0x41804180u, nibbles = 0x00780078u;
     asm volatile("" : "+v"(base), "+s"(nibbles));
     const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
     const uint32_t a_first = xs_at + (lane & 31) * (KB * 2) + ((kh ^ nl) << 4);              // row l & 31 (and 32 further on), chunk kh
     const uint32_t r_first = xs_at + (wave * 16 + nl) * (KB * 2) + (((lane >> 4) ^ nl) << 4);   // row 16 wave + nl, chunk l / 16
-    const int nkb = kb_end - kb_begin;
-    if (nkb > 0) {
+    // The zero-point term of pair j for the k-block whose row sums lie in row_parts[turn].  A lane of the instruction (K = 8) holds four k:
+    // three parts of its row's sum and a zero; of its column's factor the lanes of k 0 .. 3 the upper part and those of k 4 .. 7 the lower.
+    uint32_t zf[2] = {0u, 0u};   // the lane's part of the factor of pair j, in both halves
+    auto zero_factor = [&](int j) {
+        const float f = __uint_as_float(sz[j] << 16) * (112.f - __uint_as_float(sz[j] & 0xFFFF0000u));   // 8 bits x 5 bits
+        const uint32_t part = vmx_f32_to_bf16(kh ? f - vmx_rnd16<false>(f) : f);
+        zf[j] = part | (part << 16);
+    };
+    auto zero_term = [&](int j, int turn) {
+        const uint2 f = make_uint2(zf[j], zf[j] & 0xFFFFu);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            fin[i][j] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(i4_s16x4, row_parts[turn][i * 32 + (lane & 31)]),
+                                                                 __builtin_bit_cast(i4_s16x4, f), fin[i][j], 0, 0, 0);
+    };
+    const bool odd_row = nl & 1, high_row = nl & 2;
+    auto keep_row_sums = [&](const vmx_f32x4 &rs, int turn) {   // lane's row: 16 wave + 4 (lane / 16) + nl % 4; four lanes store the same
+        const float v = high_row ? (odd_row ? rs[3] : rs[2]) : (odd_row ? rs[1] : rs[0]);
+        const uint32_t p0 = vmx_f32_to_bf16(v);
+        const float v1 = v - __uint_as_float(p0 << 16);
+        const uint32_t p1 = vmx_f32_to_bf16(v1);
+        row_parts[turn][wave * 16 + 4 * (lane >> 4) + (nl & 3)] = make_uint2(p0 | (p1 << 16), vmx_f32_to_bf16(v1 - __uint_as_float(p1 << 16)));
+    };
+    if (kb_begin < kb_end) {
+        if (tid < PF_BM) row_parts[1][tid] = make_uint2(0u, 0u);   // the first k-block finds nothing before it
         fetch_x(kb_begin, 0);
         fetch_w(kb_begin, 0);
         fetch_w(kb_begin, 1);
@@ -1387,7 +1408,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             };
             auto unpack = [&](int j, int s) {
                 const uint32_t v = w[j][s & 1][s / 2];
-                return tg_u32x4{(v & nibbles) | base, ((v >> 4) & nibbles) | base, ((v >> 8) & nibbles) | base, ((v >> 12) & nibbles) | base};
+                return tg_u32x4{((v << 3) & nibbles) | base, ((v >> 1) & nibbles) | base, ((v >> 5) & nibbles) | base, ((v >> 9) & nibbles) | base};
             };
             // elements [32 e / n, 32 (e + 1) / n) of pair j's finished sums of a k-block, times its scale, into the result
             auto scale_part = [&](int j, float sc, const tg_f32x16 (&acc)[2], int e, int n) {
@@ -1418,8 +1439,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     const tg_u32x4 aw = tg_lds_read(r_at ^ (64 * (s / 2)));
                     rs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, aw), __builtin_bit_cast(vmx_bf16x8, ones), rs, 0, 0, 0);
                 }
+                if (u == 2) zero_term(0, stage ^ 1);    // of the k-block before this one; nobody else writes these results now
+                if (u == 10) zero_term(1, stage ^ 1);
+                if (u == 9) keep_row_sums(rs, stage);
                 if (u == 7) {
                     sc0 = __uint_as_float(sz[0] << 16);
+                    zero_factor(0);
                     fetch_x(next, stage ^ 1);
                     fetch_w(next, 0);
                 }
@@ -1432,10 +1457,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 else if (s > 0) scale_part(0, sc0, acc0, s - 1, 7);
                 if (u == 15) {
                     sc1 = __uint_as_float(sz[1] << 16);
+                    zero_factor(1);
                     fetch_w(next, 1);
                 }
             }
-            if (nl == 0) *reinterpret_cast<float4 *>(&row_sums[(kb - kb_begin) * PF_BM + wave * 16 + 4 * (lane >> 4)]) = make_float4(rs[0], rs[1], rs[2], rs[3]);
         }
 #pragma unroll
         for (int i = 0; i < 2; i++)
@@ -1443,44 +1468,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             for (int r = 0; r < 16; r++) fin[i][1][r] = fmaf(sc1, acc1[i][r], fin[i][1][r]);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        // zero-point term, 16 k-blocks a step: lane (row or column l & 31) holds k-blocks 16 t + 8 kh .. + 7
-        for (int t = 0; t < nkb; t += 16) {
-            uint4 bp[2][2];   // [column pair][part]
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                uint16_t q[8][2];
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int b = t + 8 * kh + e;
-                    const uint32_t z = b < nkb ? (SZ + ((int64_t)(nt0 + 2 * j) * G + (kb_begin + b) / gkb) * 16)[sz_at] : 0u;
-                    bf16_parts<2>(-__uint_as_float(z << 16) * __uint_as_float(z & 0xFFFF0000u), q[e]);
-                }
-#pragma unroll
-                for (int p = 0; p < 2; p++)
-                    bp[j][p] = make_uint4(q[0][p] | ((uint32_t)q[1][p] << 16), q[2][p] | ((uint32_t)q[3][p] << 16), q[4][p] | ((uint32_t)q[5][p] << 16),
-                                          q[6][p] | ((uint32_t)q[7][p] << 16));
-            }
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                uint16_t q[8][3];
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int b = t + 8 * kh + e;
-                    bf16_parts<3>(b < nkb ? row_sums[b * PF_BM + i * 32 + (lane & 31)] : 0.f, q[e]);
-                }
-#pragma unroll
-                for (int p = 0; p < 3; p++) {
-                    const uint4 ap = make_uint4(q[0][p] | ((uint32_t)q[1][p] << 16), q[2][p] | ((uint32_t)q[3][p] << 16),
-                                                q[4][p] | ((uint32_t)q[5][p] << 16), q[6][p] | ((uint32_t)q[7][p] << 16));
-#pragma unroll
-                    for (int j = 0; j < 2; j++)
-#pragma unroll
-                        for (int o = 0; o < 2; o++)
-                            fin[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(vmx_bf16x8, ap), __builtin_bit_cast(vmx_bf16x8, bp[j][o]),
-                                                                                fin[i][j], 0, 0, 0);
-                }
-            }
-        }
+        zero_term(0, (kb_end - 1 - kb_begin) & 1);
+        zero_term(1, (kb_end - 1 - kb_begin) & 1);
     }
     // Outputs lie at a uniform row's start plus the lane's 32-bit offset (row 4 kh of an eight-row group, its column): no address
     // arithmetic per element.  Row of element (i, r): 32 i + 8 (r / 4) + 4 kh + r % 4.
@@ -1846,21 +1835,20 @@ static bool tiled_ok(int M, int N, int K) {
     return !off && M >= min_m && N % 128 == 0;
 }
 
-// Launch of the prompt-shaped kernel: 64 x 256 workgroup tiles where N allows, the row sums of a slice's kbs k-blocks fit beside the two
-// tiles in 64 KiB of LDS, and a row starts inside a 32-bit byte offset (VMX_INT4_TILED_WIDE=0 keeps 64 x 128 for A/B runs)
-static bool tiled_wide_ok(int M, int N, int K, int kbs) {
+// Launch of the prompt-shaped kernel: 64 x 256 workgroup tiles where N allows and a row starts inside a 32-bit byte offset
+// (VMX_INT4_TILED_WIDE=0 keeps 64 x 128 for A/B runs)
+static bool tiled_wide_ok(int M, int N, int K) {
     static const bool wide = vmx_tune("VMX_INT4_TILED_WIDE", 1) != 0;
-    return wide && N % 256 == 0 && kbs <= 127 && (int64_t)M * K * 2 < (int64_t)1 << 32;
+    return wide && N % 256 == 0 && (int64_t)M * K * 2 < (int64_t)1 << 32;
 }
 
 template <bool GLU, bool GROUPED>
 static void launch_tiled(const uint4 *W, const uint32_t *SZ, const uint16_t *x, float *partial, uint16_t *act, int M, int N, int K, int group,
                          int kbs, int slice_rows, const Int4GroupedArgs &ga, int row_tiles, int splits, hipStream_t st,
                          uint16_t *ybf = nullptr, const uint16_t *bias = nullptr) {
-    if (tiled_wide_ok(M, N, K, kbs)) {
+    if (tiled_wide_ok(M, N, K)) {
         const unsigned grid = GROUPED ? (unsigned)(((N >> 8) + 7) / 8 * 8 * row_tiles * splits) : tg_grid((N >> 8) * row_tiles * splits);
-        const size_t sums = (size_t)kbs * PF_BM * 4;
-        hipLaunchKernelGGL((int4_gemm_prompt_kernel<GLU, GROUPED>), dim3(grid), dim3(256), sums, st, W, SZ, x, partial, act, M, N,
+        hipLaunchKernelGGL((int4_gemm_prompt_kernel<GLU, GROUPED>), dim3(grid), dim3(256), 0, st, W, SZ, x, partial, act, M, N,
                            K, group, kbs, slice_rows, ga, row_tiles, splits, ybf, bias);
     } else {
         hipLaunchKernelGGL((int4_gemm_tiled_kernel<GLU, GROUPED>), dim3(N / 128, row_tiles, splits), dim3(256), 0, st, W, SZ, x, partial, act, M, N,
@@ -1883,7 +1871,7 @@ int vmx_int4_splits_rows(int M, int N, int K) {
     int64_t least = INT64_MAX;
     for (int s = 1; s <= plan; s++) {
         const int kbs = (kblocks + s - 1) / s;
-        if (!tiled_wide_ok(M, N, K, kbs) || (s < plan && (s - 1) * kbs >= kblocks)) continue;
+        if (!tiled_wide_ok(M, N, K) || (s < plan && (s - 1) * kbs >= kblocks)) continue;
         const int64_t cost = (tiles * s + slots - 1) / slots * kbs;
         if (cost < least) least = cost, best = s;
     }
@@ -2312,12 +2300,12 @@ extern "C" int vmx_int4_gemm_bf16(uint16_t *y, const uint16_t *x, const void *pa
         const int kblocks = K / KB, row_tiles = (M + PF_BM - 1) / PF_BM;
         // split-K only while the tiles alone leave compute units idle (the plan's slice count is sized for one row tile)
         int splits = p.splits;
-        if (tiled_wide_ok(M, N, K, 1)) {
+        if (tiled_wide_ok(M, N, K)) {
             const int tiles = (N >> 8) * row_tiles, want = (2 * vmx_num_cus() + tiles - 1) / tiles;
             splits = want < splits ? (want < 1 ? 1 : want) : splits;
         }
         const int kbs = (kblocks + splits - 1) / splits;
-        if (splits == 1 && tiled_wide_ok(M, N, K, kbs)) {   // one slice: the kernel writes the bf16 output itself
+        if (splits == 1 && tiled_wide_ok(M, N, K)) {   // one slice: the kernel writes the bf16 output itself
             launch_tiled<false, false>(W, SZ, x, nullptr, nullptr, M, N, K, group, kbs, M, Int4GroupedArgs{}, row_tiles, 1, st, y, bias);
             VMX_CHECK_LAUNCH("int4_gemm(tiled)");
             return VMX_OK;
