@@ -54,3 +54,38 @@ def test_whole_rows(gpu, contexts, new, heads, window):
         exact = torch.softmax(q @ rows.T * scale, 1) @ rows[:, :R]
         bound = (torch.expm1(4 * d) + 2.0 ** -15 + 1024 * 2.0 ** -24) * rows[:, :R].abs().max()
         assert bool(((out[t].double() - exact).abs() <= bound).all()), (t, float((out[t].double() - exact).abs().max()), float(bound))
+
+
+# rows of 512 + 64 values, 256 + 32 and 96 + 32: the three forms; 16 heads (a tile is one token) and 3 (five tokens of several sequences)
+@pytest.mark.parametrize("R,RD", [(512, 64), (256, 32), (96, 32)])
+@pytest.mark.parametrize("heads", [16, 3])
+@pytest.mark.parametrize("parts", [True, False])
+def test_position_without_keys(gpu, R, RD, heads, parts):
+    """A token at position -1 has no keys: its output is zero whatever the cache and the memory before it hold (NaN here), and its neighbours
+    are what they are without it."""
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    bs, mb = 16, 10
+    g = torch.Generator(device="cuda").manual_seed(R + heads)
+    held = torch.full(((4 * mb + 1) * bs, R + RD), float("nan"), device="cuda", dtype=torch.bfloat16)
+    cache = held[bs:]
+    cache.copy_(torch.randn((4 * mb * bs, R + RD), device="cuda", generator=g))
+    bt = torch.arange(4 * mb, dtype=torch.int32, device="cuda").view(4, mb)
+    pos = torch.tensor([-1, 130, -1, 3], dtype=torch.int32, device="cuda")
+    sid = torch.arange(4, dtype=torch.int32, device="cuda")
+    qa = torch.randn((4, heads, R), device="cuda", generator=g)
+    qr = torch.randn((4, heads, RD), device="cuda", generator=g)
+    ws = torch.empty(lib.vmx_latent_attention_workspace_bytes(4, heads, R, 0, mb, bs) if parts else 16, dtype=torch.uint8, device="cuda")
+
+    def run(pick):
+        o = torch.full((len(pick), heads, R), float("nan"), device="cuda")
+        a, r, t, p = (v[pick].contiguous() for v in (qa, qr, sid, pos))
+        check(lib.vmx_latent_attention(o.data_ptr(), a.data_ptr(), r.data_ptr(), cache.data_ptr(), 1, bt.data_ptr(), mb, t.data_ptr(), p.data_ptr(), None,
+                                       0.05, 0, len(pick), heads, R, RD, bs, ws.data_ptr(), ws.numel(), None))
+        torch.cuda.synchronize()
+        return o
+
+    out, alone = run([0, 1, 2, 3]), run([1, 3])
+    assert bool((out[[0, 2]] == 0).all())
+    # the keys may be cut into other partitions: a weight's two bf16 halves are off by 2^-16, on either side
+    assert float((out[[1, 3]] - alone).abs().max()) <= 2.0 ** -15 * float(cache.abs().max())

@@ -266,7 +266,8 @@ __global__ __launch_bounds__(256, WHOLE == 2 ? 2 : 1) void latent_attn_mfma_kern
         const int32_t *bt = a.block_tables + (int64_t)seq * a.max_blocks;
         const int hi = a.positions[last];
         const int lo = a.window > 0 ? max(0, a.positions[first] - a.window + 1) : 0;
-        const int ntiles = (hi - lo) / LA_KT + 1, tpp = (ntiles + a.NP - 1) / a.NP;
+        // no keys (a padding token's position -1): no tile, so no row is ever asked for below
+        const int ntiles = hi < lo ? 0 : (hi - lo) / LA_KT + 1, tpp = (ntiles + a.NP - 1) / a.NP;
         const int kt_begin = part * tpp, kt_end = min(ntiles, kt_begin + tpp);
         // A operand of S: the query of row fl
         la_u32x4 qf[KSMAX];
