@@ -444,8 +444,8 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(const WinAttn p) 
     __shared__ __align__(16) uint16_t Vt[16 * VS * LDV];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fl = lane & 15, fg = lane >> 4;
     const int qpk = p.heads / p.kv_heads, hq = min(qpk, 4), nt = 4 / hq, RT = 16 * nt;
-    const int share = blockIdx.x % p.parts;
-    int tile = blockIdx.x / p.parts, r0 = 0, nrows = 0;
+    const int zq = (qpk + 3) / 4, share = blockIdx.z / zq;   // a run's shares lie furthest apart: those without keys are launched last
+    int tile = blockIdx.x, r0 = 0, nrows = 0;
     for (int s = 0; s < p.num_seqs; s++) {
         const int a = p.seq_starts[s], len = p.seq_starts[s + 1] - a, n = (len + RT - 1) / RT;
         if (tile < n) {
@@ -456,7 +456,7 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(const WinAttn p) 
         tile -= n;
     }
     if (nrows <= 0) return;   // the same for the whole workgroup
-    const int kvh = blockIdx.y, sub = wave / hq, hh = blockIdx.z * 4 + wave % hq;
+    const int kvh = blockIdx.y, sub = wave / hq, hh = (blockIdx.z - share * zq) * 4 + wave % hq;
     const bool active = sub < nt && hh < qpk && 16 * sub < nrows;
     const int head = kvh * qpk + (hh < qpk ? hh : 0);
     const int D = p.dim, V = p.vdim;
@@ -468,6 +468,14 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(const WinAttn p) 
     const uint16_t *kc = (const uint16_t *)p.kc, *vc = (const uint16_t *)p.vc;
     const int qrow = 16 * sub + fl, qi = i0 + qrow, qlo = p.first_key(qi);
     const bool qlive = active && qrow < nrows;
+    // this workgroup's share of the run's key tiles
+    const int ntile = (nk + KT - 1) / KT, per = (ntile + p.parts - 1) / p.parts;
+    const int kb0 = share * per * KT, kb1 = min(nk, (share + 1) * per * KT);
+    if (p.parts > 1 && kb0 >= kb1) {   // more shares than tiles: this one says that it has no keys, and the merge reads no sums of it
+        float *w = p.ws + (((int64_t)(r0 + qrow) * p.heads + head) * p.parts + share) * (V + 2);
+        if (qlive && fg == 0) w[V] = -FLT_MAX, w[V + 1] = 0.f;
+        return;
+    }
     uint4 qf[DS];
 #pragma unroll
     for (int s = 0; s < DS; s++) {
@@ -485,9 +493,6 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(const WinAttn p) 
     const float smul = p.scale * (p.temp ? vmx_bf16_to_f32(p.temp[head]) : 1.0f);
     const float inv_cap = p.softcap > 0.f ? 1.0f / p.softcap : 0.f;
     const float dr1 = p.r1 ? vmx_bf16_to_f32(p.r1[head]) : 0.f, dr2 = p.r1 ? vmx_bf16_to_f32(p.r2[head]) : 0.f;
-    // this workgroup's share of the run's key tiles
-    const int ntile = (nk + KT - 1) / KT, per = (ntile + p.parts - 1) / p.parts;
-    const int kb0 = share * per * KT, kb1 = min(nk, (share + 1) * per * KT);
     uint4 kr[KCH], vr[VCH];
     int krow[KCH], vrow[VCH];    // cache rows of the tile to fetch next: looked up one tile earlier, so that a fetch is one trip to memory
     auto cache_row = [&](int idx) -> int {
@@ -975,6 +980,7 @@ __global__ __launch_bounds__(64) void window_attn_merge_kernel(const WinAttn p) 
     const float sink = p.sink ? vmx_bf16_to_f32(p.sink[h]) : -FLT_MAX;
     const float M = fmaxf(vmx_wave_max(mq), sink);
     const float eq = mine ? expf(mq - M) : 0.f;            // a share without keys: e^(-huge) = 0
+    const uint64_t held = __ballot(mine && dq != 0.f);     // the others may have left their sums unwritten
     float g = 1.0f / (vmx_wave_sum(eq * dq) + (p.sink ? expf(sink - M) : 0.f));
     if (p.gate && !p.gate_elem) g *= sigmoid_f32(p.gate[(int64_t)t * p.ldgate + h]);
     for (int c0 = 0; c0 < V; c0 += 64) {
@@ -983,7 +989,7 @@ __global__ __launch_bounds__(64) void window_attn_merge_kernel(const WinAttn p) 
         for (int q0 = 0; q0 < p.parts; q0 += 16) {         // sixteen shares' values first: independent loads, one wait
             float x[16];
 #pragma unroll
-            for (int q = 0; q < 16; q++) x[q] = q0 + q < p.parts ? w[(q0 + q) * (V + 2) + cc] : 0.f;
+            for (int q = 0; q < 16; q++) x[q] = held >> (q0 + q) & 1 ? w[(q0 + q) * (V + 2) + cc] : 0.f;
 #pragma unroll
             for (int q = 0; q < 16; q++) acc = fmaf(__shfl(eq, q0 + q, 64), x[q], acc);
         }
@@ -1171,16 +1177,18 @@ extern "C" int vmx_window_attention_ex(void *out, int out_dtype, const float *q,
         const int qpk = heads / kv_heads, hq = qpk < 4 ? qpk : 4, rt = 16 * (4 / hq);
         const int runs = tokens / rt + num_seqs;                              // at most one partly filled run per sequence
         const int base = runs * kv_heads * ((qpk + 3) / 4);
-        // few workgroups: deal each run's key tiles to several, up to the two workgroups that a compute unit holds (decode of a model with 16
-        // heads over 4, up to one -> up to two: 16 rows of 1000 tokens 38.5 -> 27.8 us, 12 of 700 23.0 -> 21.1, 8 of 1500 23.6 -> 22.3,
-        // 16 of 100, where a share is less than a tile, 13.2 -> 14.1)
+        // few workgroups: deal each run's key tiles to several, up to the two workgroups that a compute unit holds.  Decode of a model with 16
+        // heads over 4, rows x tokens, attention and merge, up to one -> up to two workgroups: 16 x 1000 40.0 -> 29.8 us, 16 x 300 19.5 -> 16.8,
+        // 12 x 700 24.0 -> 19.4, 8 x 1500 25.0 -> 23.6, 16 x 100 14.7 -> 14.6.  Tables say how long a sequence can be, not how long it is: shares beyond
+        // its tiles leave at once and are launched last (16 x 100 in tables of 4096: 14.7; as whole shares among the others 15.9)
         if (workspace && base < 128) {
             int parts = 512 / base < 16 ? 512 / base : 16;
             if (span > 0) parts = std::min(parts, (span + keep_first + rt + 63) / 64);
+            parts = (int)std::min<int64_t>(parts, ((int64_t)max_blocks_per_seq * block_size + 63) / 64);   // no sequence is longer than its table
             parts = std::min<size_t>(parts, workspace_bytes / ((size_t)tokens * heads * (vdim + 2) * 4));
             if (parts > 1) p.parts = parts;
         }
-        const dim3 mgrid(runs * p.parts, kv_heads, (qpk + 3) / 4);
+        const dim3 mgrid(runs, kv_heads, (qpk + 3) / 4 * p.parts);
         const int ds = dim <= 64 ? 2 : (dim <= 128 ? 4 : 8), vs = vdim <= 32 ? 2 : (vdim <= 64 ? 4 : 8);
 #define WM_LAUNCH(A, B) hipLaunchKernelGGL((window_attn_mfma_kernel<A, B>), mgrid, dim3(256), 0, st, p)
         if (ds == 2) {
