@@ -74,16 +74,19 @@ def test_dense_prompt_rows(gpu, tokens, heads, kv_heads, head_dim, fp8):
         model.close()
 
 
-# KV heads times rows of 6, 128, 256 and 512 on 256 compute units: 42, 4, 2 and 1 partitions a KV head, block tables of more than 64 entries
-@pytest.mark.parametrize("heads,kv_heads,head_dim,rows", [(4, 2, 64, 3), (8, 8, 128, 16), (16, 16, 64, 16), (32, 32, 64, 16)])
-def test_long_contexts_partitions(gpu, heads, kv_heads, head_dim, rows):
+# KV heads times rows of 6, 128, 256 and 512 on 256 compute units: 42 and 4 partitions a KV head up to 2048 tokens, block tables of more than 64
+# entries; of 128, 256 and 512 up to 1024 tokens: 4, 2 and 1; beyond 2048 tokens never fewer than 8
+@pytest.mark.parametrize("heads,kv_heads,head_dim,rows,longest", [
+    (4, 2, 64, 3, 1100), (8, 8, 128, 16, 1100), (16, 16, 64, 16, 1100), (32, 32, 64, 16, 1100), (8, 8, 128, 16, 900), (16, 16, 64, 16, 900),
+    (32, 32, 64, 16, 900), (32, 32, 64, 9, 2100)])
+def test_long_contexts_partitions(gpu, heads, kv_heads, head_dim, rows, longest):
     from tests.test_gpu_true_geometry import _decode_and_compare, _fill_kv
     from tests.model_oracle import OracleQwen3
     from vllm_rust_amd.qwen3 import QuantizedQwen3ForCausalLM, Qwen3Spec, rope_cos_sin_cache
     vmx, torch = gpu
-    contexts = [1100, 3, 1030, 0, 15, 16, 17, 511, 512, 700, 1023, 1024, 255, 64, 900, 1][:rows]
-    spec = Qwen3Spec(256, 2, heads, kv_heads, head_dim, 256, 512, tie_word_embeddings=True, max_position=2048, num_blocks=72 * rows, max_batch=rows,
-                     max_seq_len=1200, max_prefill_tokens=16)
+    contexts = [min(c, longest) for c in [longest, 3, 1030, 0, 15, 16, 17, 511, 512, 700, 1023, 1024, 255, 64, 900, 1][:rows]]
+    spec = Qwen3Spec(256, 2, heads, kv_heads, head_dim, 256, 512, tie_word_embeddings=True, max_position=4096, num_blocks=(longest // 16 + 4) * rows,
+                     max_batch=rows, max_seq_len=longest + 100, max_prefill_tokens=16)
     model = QuantizedQwen3ForCausalLM(spec)
     try:
         ck = model.load_synthetic_bf16(seed=21, keep_host_copy=True)

@@ -1521,7 +1521,7 @@ size_t vmx_split_decode_attention_workspace_bytes(int num_seqs, int num_heads, i
 }
 
 // Contexts beyond the reach of the few-partition form (from 512 tokens on): the same kernel with 1 ... 64 workgroups of 8 waves per KV head (as many
-// as give every compute unit one workgroup, or two where they would be fewer than four) and the separate merge (vmx_paged_attention_merge) behind it, in place of
+// as give every compute unit one workgroup, but no fewer than the context bound asks for) and the separate merge (vmx_paged_attention_merge) behind it, in place of
 // "q/k/v post-processing + one wave per partition + merge": at 8192 tokens the one-wave partitions put 464 waves on the
 // chip for 24 us per layer (Qwen3-8B, one row).  Returns the partition count, 0 = not covered.  VMX_NO_SPLIT_ATTN_LONG=1
 // switches the form off.
@@ -1537,11 +1537,18 @@ int vmx_split_decode_attention_long_parts(int head_dim, int qpk, int rot_dim, in
     // one workgroup per compute unit: measured on Qwen3-8B (8 KV heads, one row) at 1024 ... 32768 tokens, 32 partitions beat
     // 12 / 16 / 24 / 64 at every length (8192 tokens: 420 / 440 / 475 / 441 against 478 tok/s; 33 partitions = 264 workgroups
     // on 256 compute units cost 6 %)
-    // Many rows: a compute unit holds two workgroups, and more than that many only repeat the prologue of q heads (16 rows of 1500 /
-    // 700 tokens: 8 partitions 31.8 / 21.8 us, 4 partitions 26.1 / 17.9, 2 partitions 28.3 / 18.0; 12 rows of 2000: 2 / 4 / 6 = 31.9 /
-    // 29.3 / 30.8; 8 rows of 500: 8 partitions 10.3, 4 9.9; 4 rows of 1500: 8 / 16 = 13.7 / 13.2; 1 row of 1500: 32 / 64 = 9.0 / 10.2)
+    // Many rows: a compute unit holds two workgroups, and more than that many only repeat the prologue of q heads (8 KV heads, 16 rows of
+    // 1500 / 700 tokens: 8 partitions 31.8 / 21.8 us, 4 partitions 26.1 / 17.9, 2 partitions 28.3 / 18.0; 12 rows of 2000: 2 / 4 / 6 = 31.9 /
+    // 29.3 / 30.8; 8 rows of 500: 8 partitions 10.3, 4 9.9; 4 rows of 1500: 8 / 16 = 13.7 / 13.2; 1 row of 1500: 32 / 64 = 9.0 / 10.2).
+    // The rows of a batch may be of any length up to the bound, and the longest is walked by its own partitions alone, so the least count
+    // grows with the bound.  A layer's time (attention and 25 us of the rest), partitions 1 / 2 / 4 / 8, one row among 15 of 100 or 200 tokens:
+    //    8 KV heads: 2000 tokens 79 / 61 / 56 / 56, 4000 118 / 80 / 71 / 63, 8000 198 / 125 / 103 / 80, 32000 785 / 415 / 286 / 173
+    //   32 KV heads: 1000 tokens 58 / 54 / 59 / 71, 2000 76 / 64 / 64 / 78, 4000 110 / 82 / 76 / 85, 8000 176 / 118 / 111 / 104, 32000 688 / 378 / 281 / 212
+    // and of 16 equal rows, 8 KV heads: 1500 tokens 74 / 61 / 59 / 67, 3000 106 / 78 / 78 / 82, 8000 211 / 134 / 141 / 137;
+    //   32 KV heads: 700 tokens 75 / 76 / 80 / 93, 1500 114 / 111 / 111 / 131, 3000 185 / 179 / 176 / 181, 8000 420 / 408 / 400 / 402.
     const int pairs = num_kv_heads * num_seqs > 0 ? num_kv_heads * num_seqs : 1, per = vmx_num_cus() / pairs, two = 2 * vmx_num_cus() / pairs;
-    return per >= 4 ? (per > 64 ? 64 : per) : two < 1 ? 1 : two > 4 ? 4 : two;
+    const int least = ctx > 2048 ? 8 : ctx > 1024 || two > 4 ? 4 : two < 1 ? 1 : two;
+    return per < least ? least : per > 64 ? 64 : per;
 }
 size_t vmx_split_decode_attention_long_workspace_bytes(int num_seqs, int num_heads, int head_dim, int parts) {
     return (size_t)num_seqs * num_heads * parts * ((size_t)head_dim + 2) * 4;
