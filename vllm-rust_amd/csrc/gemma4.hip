@@ -459,9 +459,7 @@ bool mma_geglu_ok(vmx_gemma4 *m, const G4Layer &L, int H, int tokens) {
 
 bool g_split_always = false;   // measurement: prompt-sized linears always through the two-term bf16 split (vmx_debug_gemma4_split_always)
 
-// A linear on `rows` token rows: the q8_1 MMVQ up to IQ_GEMV_MAX_M = 16 rows (activations already quantised in m->q8), beyond that
-// the reference's large-M form (gguf/mod.rs:358-365): dequantise the weight once, multiply the unquantised bf16 rows `a`.
-// a_is_f16: the rows are fp16 already (what g4_gateup_prompt leaves)
+// A prompt-sized linear in the exact integer form (iq_dequant_int_kernel)
 bool int_form_ok(const IqLin &l, int rows) {
     return vmx_iq_int_form_ok(l.ggml_type) && !g_split_always && vmx_int_gemm_ok(rows, l.out_features, l.in_features);
 }
@@ -473,6 +471,9 @@ int int_weights(vmx_gemma4 *m, const IqLin *const *lins, int n, int total, int K
     return VMX_OK;
 }
 
+// n linears on the same `rows` token rows: the q8_1 MMVQ up to IQ_GEMV_MAX_M = 16 rows (activations already quantised in m->q8), beyond that
+// the reference's large-M form (gguf/mod.rs:358-365): dequantise the weight once, multiply the unquantised bf16 rows `a`.
+// a_is_f16: the rows are fp16 already (what g4_gateup_prompt leaves)
 int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, const uint16_t *a, float *y, int ldy, int rows,
                hipStream_t st, bool a_is_f16 = false) {
     if (rows <= 16) {
@@ -498,11 +499,14 @@ int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, 
         return vmx_int_gemm_f32(a16, m->gemm_ws.p, y, rows, total, K, ldy, (float *)m->gemm_part.p, st);
     }
     VMX_REQUIRE(!a_is_f16, "gemma4: fp16 rows for a projection without an integer form");
+    bool a16_ready = false;
     for (int i = 0; i < n; i++) {
         const IqLin &l = *lins[i];
         if (int_form_ok(l, rows)) {
             const IqLin *one[1] = {&l};
-            if (int rc = vmx_bf16_rows_to_f16(a, (uint16_t *)m->a16.p, (int64_t)rows * K, st)) return rc;
+            if (!a16_ready)
+                if (int rc = vmx_bf16_rows_to_f16(a, (uint16_t *)m->a16.p, (int64_t)rows * K, st)) return rc;
+            a16_ready = true;
             if (int rc = int_weights(m, one, 1, l.out_features, K, st)) return rc;
             if (int rc = vmx_int_gemm_f32((const uint16_t *)m->a16.p, m->gemm_ws.p, y + offs[i], rows, l.out_features, K, ldy,
                                           (float *)m->gemm_part.p, st))
