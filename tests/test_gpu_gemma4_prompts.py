@@ -2,6 +2,7 @@
 groups whose projections do not all have the integer form."""
 import ctypes as C
 
+import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -13,6 +14,37 @@ def gpu():
     import vllm_rust_amd as vmx
     vmx.init(0)
     return vmx, torch
+
+
+# rows below, at and past a tile of 64 and past one of 128 (64 x 128 and 128 x 128 tiles); one, two and five scale groups; gate columns below, at and past the
+# 64 that a tile takes
+@pytest.mark.parametrize("M", [17, 64, 65, 129])
+@pytest.mark.parametrize("inter,K", [(40, 256), (64, 512), (200, 1280)])
+def test_geglu_tiles(gpu, M, inter, K):
+    """act = bf16(bf16(gelu(gate)) * up) with gate and up rounded to bf16, against float64 on the same integers, scales and fp16 rows.  The
+    f32 sums may fall on the other side of a bf16 rounding: one step (2^-8 relative) of gate and of up, and one of each product behind."""
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    g = torch.Generator(device="cuda").manual_seed(M + inter + K)
+    N = 2 * inter
+    q = torch.randint(-1922, 1923, (N, K), device="cuda", generator=g).to(torch.float16)
+    dt = (torch.rand((K // 256, N), device="cuda", generator=g) + 0.5) * (1.0 / (1100 * K ** 0.5))
+    x = torch.randn((M, K), device="cuda", generator=g).to(torch.float16)
+    ws = torch.cat([q.reshape(-1).view(torch.uint8), dt.reshape(-1).view(torch.uint8)])
+    guard = torch.full((M + 2, inter), 7.0, dtype=torch.float16, device="cuda")
+    act = guard[1:M + 1]
+    check(lib._Z18vmx_int_gemm_gegluPKtPKvPtiiiP12ihipStream_t(C.c_void_p(x.data_ptr()), C.c_void_p(ws.data_ptr()), C.c_void_p(act.data_ptr()), M, inter,
+                                                              K, None))
+    torch.cuda.synchronize()
+    w = q.double() * dt.double().T.repeat_interleave(256, 1)
+    s = x.double() @ w.T
+    gate, up = s[:, :inter].to(torch.bfloat16).double(), s[:, inter:].to(torch.bfloat16).double()
+    cdf = 0.5 * (1 + torch.erf(gate / 2 ** 0.5))
+    slope = cdf + gate * torch.exp(-gate * gate / 2) / (2 * np.pi) ** 0.5
+    ref = gate * cdf * up
+    bound = 2.0 ** -8 * ((slope * gate * up).abs() + 3 * ref.abs()) + 2.0 ** -20
+    assert bool(((act.double() - ref).abs() <= bound).all())
+    assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all())
 
 
 def _model(spec, types, seed=5):
@@ -28,6 +60,35 @@ def _model(spec, types, seed=5):
             model.load_tensor(which, li, w)
             ck[f"{li}.{name}"] = w.cpu()
     return model, ck
+
+
+# hidden 768: three scale groups, whose sums q|k|v, o and down take in slices; 128-row tiles from 65 rows on.  IQ4_XS (23) has no integer form: v, then
+# gate (no GEGLU epilogue), then down (the epilogue's fp16 rows would have no reader)
+@pytest.mark.parametrize("rows,types", [(65, {}), (130, {}), (300, {}), (130, {2: 23}), (65, {4: 23}), (65, {6: 23}), (33, {0: 17, 1: 21, 2: 22, 3: 17, 6: 22})])
+def test_prompt_rows(gpu, rows, types):
+    """Every row of the residual stream after one pass against the CPU oracle, which takes the same rows as one batch: 2e-2 relative L2 a row,
+    as for the whole model."""
+    vmx, torch = gpu
+    from oracle import oracle as orc
+    from tests.model_oracle import OracleGemma4
+    from vllm_rust_amd.gemma4 import GEMMA4_12B_IQ3_MIX, Gemma4Spec
+    spec = Gemma4Spec(768, 2, 4, 1280, 512, head_dim_sliding=64, head_dim_full=128, kv_heads_sliding=2, kv_heads_full=1, sliding_window=24,
+                      full_every=2, max_position=512, kv_cache_dtype=0, num_blocks=24, max_batch=1, max_seq_len=320, max_prefill_tokens=300)
+    model, ck = _model(spec, {**GEMMA4_12B_IQ3_MIX, **types})
+    try:
+        ref = OracleGemma4(spec, ck, model.cos_sin_sliding, model.cos_sin_full)
+        bs = spec.block_size
+        bt = np.random.default_rng(2).permutation(spec.num_blocks)[:20].astype(np.int32)[None]
+        prompt = np.random.default_rng(1).integers(0, spec.vocab_size, rows).astype(np.int32)
+        model.prefill(torch.from_numpy(prompt).cuda(), 0, torch.from_numpy(bt).cuda()[0])
+        torch.cuda.synchronize()
+        got = model.debug_read(0, (rows, spec.hidden_size)).double().cpu().numpy()
+        pos = np.arange(rows, dtype=np.int32)
+        _, h, _ = ref.decode(prompt, pos, (bt[0, pos // bs] * bs + pos % bs).astype(np.int32), np.repeat(bt, rows, axis=0), pos + 1)
+        exp = orc.bf16_to_f32(h).astype(np.float64)
+        assert (np.linalg.norm(got - exp, axis=1) <= 2e-2 * np.linalg.norm(exp, axis=1)).all()
+    finally:
+        model.close()
 
 
 def _launches(torch, types):
