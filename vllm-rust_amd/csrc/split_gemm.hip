@@ -180,7 +180,9 @@ __global__ __launch_bounds__(S::THREADS) void int_tile_kernel(const uint16_t *__
     }
 }
 
-// y[m][n] (rows ldy apart) = the slices [slices][M][N] added in slice order; N % 4 == 0
+// y[m][n] (rows ldy apart) = the slices [slices][M][N] added in slice order; N % 4 == 0.  WIDE: y and its rows lie on 16 bytes (a caller's
+// output may be a view that starts anywhere).
+template <bool WIDE>
 __global__ __launch_bounds__(256) void int_slices_kernel(const float *__restrict__ part, float *__restrict__ y, int slices, int M, int N, int64_t ldy) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, quads = (int64_t)M * N / 4;
     if (i >= quads) return;
@@ -190,7 +192,9 @@ __global__ __launch_bounds__(256) void int_slices_kernel(const float *__restrict
         v.x += o.x, v.y += o.y, v.z += o.z, v.w += o.w;
     }
     const int64_t m = 4 * i / N, n = 4 * i - m * N;
-    *reinterpret_cast<float4 *>(y + m * ldy + n) = v;
+    float *to = y + m * ldy + n;
+    if constexpr (WIDE) *reinterpret_cast<float4 *>(to) = v;
+    else to[0] = v.x, to[1] = v.y, to[2] = v.z, to[3] = v.w;
 }
 
 __global__ __launch_bounds__(256) void bf16_to_f16_kernel(uint16_t *__restrict__ out, const uint16_t *__restrict__ in, int64_t n8) {
@@ -329,22 +333,25 @@ int int_slices(int M, int N, int K) {
 }
 }  // namespace
 
-// most bytes of slice sums any call can want: two tiles of 128 x 128 a compute unit, and the tiles' overhang
+// most bytes of slice sums any call can want: int_slices gives at most two tiles a compute unit, of at most 128 x 128 sums
 size_t vmx_int_gemm_part_bytes() { return (size_t)2 * vmx_num_cus() * 128 * 128 * 4; }
 
 bool vmx_int_gemm_ok(int M, int N, int K) { return (int64_t)M * K * 2 < (int64_t)1 << 32 && (int64_t)N * K * 2 < (int64_t)1 << 32; }
 
-// part: vmx_int_gemm_part_bytes() of scratch, or NULL (no slices).  ldy % 4 == 0 for slices.
+// part: vmx_int_gemm_part_bytes() of scratch, or NULL (no slices)
 int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, float *part, hipStream_t st) {
     const uint16_t *Q = (const uint16_t *)workspace;
     const float *Dt = (const float *)(Q + (int64_t)N * K);
-    const int slices = part && ldc % 4 == 0 ? int_slices(M, N, K) : 1;
+    const int slices = part ? int_slices(M, N, K) : 1;
     float *to = slices > 1 ? part : C;
     const int64_t ld = slices > 1 ? N : ldc;
     if (int_rows(M) == 128) launch_int_tile<IntWide, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
     else launch_int_tile<IntMid, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
-    if (slices > 1)
-        hipLaunchKernelGGL(int_slices_kernel, dim3((unsigned)(((int64_t)M * N / 4 + 255) / 256)), dim3(256), 0, st, part, C, slices, M, N, (int64_t)ldc);
+    if (slices > 1) {
+        const dim3 grid((unsigned)(((int64_t)M * N / 4 + 255) / 256));
+        if (ldc % 4 == 0 && ((uintptr_t)C & 15) == 0) hipLaunchKernelGGL(int_slices_kernel<true>, grid, dim3(256), 0, st, part, C, slices, M, N, (int64_t)ldc);
+        else hipLaunchKernelGGL(int_slices_kernel<false>, grid, dim3(256), 0, st, part, C, slices, M, N, (int64_t)ldc);
+    }
     VMX_CHECK_LAUNCH("int_gemm");
     return VMX_OK;
 }
