@@ -171,3 +171,33 @@ def test_int4_prompt_slices(gpu):
         assert float((last[0] - last[1]).norm() / last[0].norm()) <= 2e-2
     finally:
         model.close()
+
+
+# every count of slices (K = 33 k-blocks: slices of unequal length), a chip that is less than, just and more than filled, a remainder of rows
+@pytest.mark.parametrize("M,N,K", [(49, 1024, 4224), (65, 4096, 4224), (200, 4096, 4096), (300, 4096, 4096), (333, 4096, 4224), (640, 2048, 4096), (1024, 4096, 4096)])
+def test_int4_partial_slices(gpu, M, N, K):
+    """The f32 slices that the executor's consumers add, against float64.  A path through the sums has at most four roundings in each of a k-block's
+    eight instructions and two more a k-block, and no term is larger than |x| s (16 + nibble + 16 + zero point) <= 62 |x| s.  Nothing is
+    written behind the last slice."""
+    import ctypes as C
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
+    words = lambda *s: torch.randint(-2 ** 31, 2 ** 31 - 1, s, dtype=torch.int32, device="cuda", generator=g)   # noqa: E731
+    qw, qz = words(K // 8, N), words(K // 128, N // 8)
+    sc = ((torch.rand((K // 128, N), device="cuda", generator=g) + 0.5) * 0.01).to(torch.bfloat16)
+    packed = vmx.int4_pack(qw, sc, qz, K, N, 128)
+    n = lib._Z20vmx_int4_splits_rowsiii(M, N, K)
+    part = torch.full((n * M * N + 64,), float("nan"), device="cuda")
+    check(lib._Z21vmx_int4_gemm_partialPKvPKtPfiiiiP12ihipStream_t(C.c_void_p(packed.data_ptr()), C.c_void_p(x.data_ptr()), C.c_void_p(part.data_ptr()), M, N, K,
+                                                                128, None))
+    torch.cuda.synchronize()
+    sh = torch.arange(0, 32, 4, dtype=torch.int32, device="cuda")
+    nib = ((qw.unsqueeze(-1) >> sh) & 15).permute(0, 2, 1).reshape(K, N)
+    zp = ((qz.unsqueeze(-1) >> sh) & 15).reshape(K // 128, N).repeat_interleave(128, 0)
+    s = sc.double().repeat_interleave(128, 0)
+    y = part[:n * M * N].view(n, M, N).double().sum(0)
+    bound = (32 + 2 * K // 128 + 8) * 2.0 ** -24 * 62 * (x.double().abs() @ s)
+    assert bool(((y - x.double() @ ((nib - zp).double() * s)).abs() <= bound).all())
+    assert bool(part[n * M * N:].isnan().all())

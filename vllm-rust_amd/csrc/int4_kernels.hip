@@ -1859,24 +1859,31 @@ static void launch_tiled(const uint4 *W, const uint32_t *SZ, const uint16_t *x, 
 // ---- internal (C++) entry points used by the decoder ---------------------------------------
 int vmx_int4_splits(int N, int K) { return plan_gemm(N, K).splits; }
 
-// Slices that vmx_int4_gemm_partial writes for M rows, at most vmx_int4_splits.  A prompt's tiles may fill the chip by themselves; every
-// further slice is then f32 rows written and read again.  Taken is the count whose last round of workgroups (two fit a compute unit)
-// ends first, the smallest of equals.  2048 tokens of Qwen3-8B: o 4 slices -> 1, down 3 -> 1, q|k|v (768 tiles) 2 as before: the three
-// products together 421 -> 405 us a layer, the norm kernel that adds the slices 26 -> 15.5.
-int vmx_int4_splits_rows(int M, int N, int K) {
-    const int plan = plan_gemm(N, K).splits, kblocks = K / KB;
-    if (plan == 1 || !tiled_ok(M, N, K)) return plan;
-    const int64_t tiles = (int64_t)(N >> 8) * ((M + PF_BM - 1) / PF_BM), slots = 2 * (int64_t)vmx_num_cus();
+// Slices of k for a product of M rows on the prompt-shaped kernel, at most the plan's: the count with the least estimated time.
+//   * a k-block takes a compute unit that holds one workgroup 1.15 us and one that holds two 1.95, so w workgroups a unit cost what 1.7 (w / 2) + w % 2
+//     cost alone;
+//   * a slice is M N f32 written and read again, at 4.5 TB/s.  `own_pass`: the slices are added in a pass of their own (3 us), and one
+//     slice is stored as bf16 by the product itself; else the reader of the rows adds them, one slice as well.
+// Whole call in us with 1 / 2 / 3 / 4 slices, the taken one last:  4096 x 4096, 200 rows 39 / 29 / 25 / 24: 4; 333 rows 40 / 33 / 35 / 34: 2; 512 rows
+// 42 / 34 / 35 / 38: 2; 1024 rows 44 / 51 / 56 / 59: 1;  4096 x 12288, 333 rows 112 / 66 / 68: 2; 640 rows 112 / 98 / 79: 3; 800 rows 113 / 105 / 113: 2; 2048 rows
+// 203 / 225 / 232: 1;  2048 x 4096, 640 rows 42 / 32 / 29 / 33: 3;  6144 x 4096, 256 rows 40 / 33: 2; 640 rows 43 / 50: 1; 2048 rows 108 / 137: 1.
+static int prompt_slices(int M, int N, int K, bool own_pass) {
+    const int plan = plan_gemm(N, K).splits, kblocks = K / KB, cus = vmx_num_cus();
+    if (plan == 1 || !tiled_ok(M, N, K) || !tiled_wide_ok(M, N, K)) return plan;
+    const int64_t tiles = (int64_t)(N >> 8) * ((M + PF_BM - 1) / PF_BM), slice_ns = (int64_t)M * N * 8 / 4500;
     int best = plan;
     int64_t least = INT64_MAX;
     for (int s = 1; s <= plan; s++) {
         const int kbs = (kblocks + s - 1) / s;
-        if (!tiled_wide_ok(M, N, K) || (s < plan && (s - 1) * kbs >= kblocks)) continue;
-        const int64_t cost = (tiles * s + slots - 1) / slots * kbs;
-        if (cost < least) least = cost, best = s;
+        if ((s - 1) * kbs >= kblocks) continue;   // the last slice would be empty
+        const int64_t w = (tiles * s + cus - 1) / cus, ns = kbs * (1955 * (w / 2) + 1150 * (w % 2)) + (own_pass ? (s > 1) * (3000 + s * slice_ns) : s * slice_ns);
+        if (ns < least) least = ns, best = s;
     }
     return best;
 }
+
+// Slices that vmx_int4_gemm_partial writes for M rows, at most vmx_int4_splits
+int vmx_int4_splits_rows(int M, int N, int K) { return prompt_slices(M, N, K, false); }
 
 // partial[vmx_int4_splits_rows][M][N] f32, also with one slice.  Arguments must already satisfy check_int4_shape.
 int vmx_int4_gemm_partial(const void *packed, const uint16_t *x, float *partial, int M, int N, int K, int group, hipStream_t st) {
@@ -2296,14 +2303,8 @@ extern "C" int vmx_int4_gemm_bf16(uint16_t *y, const uint16_t *x, const void *pa
     hipStream_t st = vmx_stream(stream);
     float *partial = (float *)workspace;
     (void)mc;
-    if (tiled_ok(M, N, K)) {   // prompt chunk: 64 x 128 output tiles, then the slices are summed (+ bias) into bf16
-        const int kblocks = K / KB, row_tiles = (M + PF_BM - 1) / PF_BM;
-        // split-K only while the tiles alone leave compute units idle (the plan's slice count is sized for one row tile)
-        int splits = p.splits;
-        if (tiled_wide_ok(M, N, K)) {
-            const int tiles = (N >> 8) * row_tiles, want = (2 * vmx_num_cus() + tiles - 1) / tiles;
-            splits = want < splits ? (want < 1 ? 1 : want) : splits;
-        }
+    if (tiled_ok(M, N, K)) {   // prompt chunk: output tiles, then the slices are summed (+ bias) into bf16
+        const int kblocks = K / KB, row_tiles = (M + PF_BM - 1) / PF_BM, splits = prompt_slices(M, N, K, true);
         const int kbs = (kblocks + splits - 1) / splits;
         if (splits == 1 && tiled_wide_ok(M, N, K)) {   // one slice: the kernel writes the bf16 output itself
             launch_tiled<false, false>(W, SZ, x, nullptr, nullptr, M, N, K, group, kbs, M, Int4GroupedArgs{}, row_tiles, 1, st, y, bias);
