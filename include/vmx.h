@@ -68,8 +68,9 @@ int vmx_iq_dequantize_f32(int ggml_type, const void *blocks, float *out, int64_t
 
 /* IqLinear::forward for more than IQ_GEMV_MAX_M = 16 rows (crates/core/src/quantization/gguf/mod.rs:358-365): the weight is
  * dequantised to dense f32 once and multiplied with the UNQUANTISED activations, y[m, n] = sum_k x[m,k] * w[n,k] in f32.
- * x bf16 [m, n_in], y f32 [m, n_out]; workspace of vmx_iq_gemm_workspace_bytes(n_out, n_in) bytes.  The f32 weight runs on the bf16
- * matrix cores as an exact two-term split (w = hi + lo), so the result differs from an f32 GEMM only by summation order. */
+ * x bf16 [m, n_in], y f32 [m, n_out]; workspace of vmx_iq_gemm_workspace_bytes(n_out, n_in) bytes (4 n_out n_in are enough; the rest lets
+ * a product of few rows and columns sum slices of k).  The f32 weight runs on the matrix cores exactly -- as integers with a scale per
+ * super-block, or as a two-term bf16 split (w = hi + lo) -- so the result differs from an f32 GEMM only by summation order. */
 size_t vmx_iq_gemm_workspace_bytes(int n_out, int n_in);
 int vmx_iq_gemm_f32(int ggml_type, const void *blocks, const uint16_t *x, float *y, int m, int n_out, int n_in, void *workspace,
                     size_t workspace_bytes, void *stream);

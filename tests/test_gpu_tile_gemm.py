@@ -61,17 +61,21 @@ def test_iq_prompt_linear_tiles(gpu, M, ggml_type, N, K):
     assert bool(((y.double() - ref).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("offset", [0, 1, 2, 3])
-def test_iq_prompt_linear_output_anywhere(gpu, offset):
-    """The output of a product whose sums come in slices may start at any f32 of a larger tensor: the same values, nothing written beside it."""
+# columns that are no multiple of four; a workspace that holds every slice, or the 4 N K bytes that the product must have and what slices fit them
+@pytest.mark.parametrize("offset,M,N,room", [(0, 33, 512, 64 << 20), (1, 33, 512, 64 << 20), (2, 33, 512, 64 << 20), (3, 33, 512, 64 << 20), (0, 65, 131, 64 << 20),
+                                             (1, 300, 130, 64 << 20), (0, 200, 512, 0), (0, 700, 131, 0), (3, 4000, 132, 0)])
+def test_iq_prompt_linear_slices(gpu, offset, M, N, room):
+    """The output of a product whose sums come in slices may start at any f32 of a larger tensor: the same values, nothing written beside it or
+    behind the workspace."""
     vmx, torch = gpu
     from tests.helpers import random_iq_blocks
     from vllm_rust_amd._lib import check, lib
-    M, N, K, t = 33, 512, 8192, 18
+    K, t = 8192, 18
     raw = torch.from_numpy(np.ascontiguousarray(random_iq_blocks(np.random.default_rng(1), vmx.iq_type_size(t), N * K // 256))).reshape(-1).cuda()
     x = torch.randn((M, K), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)).to(torch.bfloat16)
-    need = lib.vmx_iq_gemm_workspace_bytes(N, K) + (64 << 20)   # room for the slices
-    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    need = 4 * N * K + room
+    assert lib.vmx_iq_gemm_workspace_bytes(N, K) >= 4 * N * K
+    ws = torch.full((need + 64,), 7, dtype=torch.uint8, device="cuda")
     held = torch.full((M * N + 8,), 7.0, device="cuda")
     y = held[offset:offset + M * N]
     check(lib.vmx_iq_gemm_f32(t, raw.data_ptr(), x.data_ptr(), y.data_ptr(), M, N, K, ws.data_ptr(), need, None))
@@ -79,7 +83,7 @@ def test_iq_prompt_linear_output_anywhere(gpu, offset):
     w = vmx.iq_dequantize(t, raw, N * K // 256).reshape(N, K).double()
     bound = (264 + K // 256 + 8) * 2.0 ** -24 * (x.double().abs() @ w.abs().T)
     assert bool(((y.view(M, N).double() - x.double() @ w.T).abs() <= bound).all())
-    assert bool((held[:offset] == 7.0).all()) and bool((held[offset + M * N:] == 7.0).all())
+    assert bool((held[:offset] == 7.0).all()) and bool((held[offset + M * N:] == 7.0).all()) and bool((ws[need:] == 7).all())
 
 
 # 256-column blocks; one k-block, odd numbers of them (17: a second step of the zero-point term; 33 in slices) and groups wider than a

@@ -496,7 +496,7 @@ int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, 
             if (int rc = vmx_bf16_rows_to_f16(a, (uint16_t *)m->a16.p, (int64_t)rows * K, st)) return rc;
             a16 = (const uint16_t *)m->a16.p;
         }
-        return vmx_int_gemm_f32(a16, m->gemm_ws.p, y, rows, total, K, ldy, (float *)m->gemm_part.p, st);
+        return vmx_int_gemm_f32(a16, m->gemm_ws.p, y, rows, total, K, ldy, (float *)m->gemm_part.p, m->gemm_part.bytes, st);
     }
     VMX_REQUIRE(!a_is_f16, "gemma4: fp16 rows for a projection without an integer form");
     bool a16_ready = false;
@@ -509,7 +509,7 @@ int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, 
             a16_ready = true;
             if (int rc = int_weights(m, one, 1, l.out_features, K, st)) return rc;
             if (int rc = vmx_int_gemm_f32((const uint16_t *)m->a16.p, m->gemm_ws.p, y + offs[i], rows, l.out_features, K, ldy,
-                                          (float *)m->gemm_part.p, st))
+                                          (float *)m->gemm_part.p, m->gemm_part.bytes, st))
                 return rc;
             continue;
         }

@@ -180,21 +180,17 @@ __global__ __launch_bounds__(S::THREADS) void int_tile_kernel(const uint16_t *__
     }
 }
 
-// y[m][n] (rows ldy apart) = the slices [slices][M][N] added in slice order; N % 4 == 0.  WIDE: y and its rows lie on 16 bytes (a caller's
-// output may be a view that starts anywhere).
-template <bool WIDE>
+// y[m][n] (rows ldy apart) = the slices [slices][M][N] added in slice order, V elements a thread.  V = 4: N % 4 == 0, y and its rows on 16 bytes
+// (a caller's output may be a view that starts anywhere).
+template <int V>
 __global__ __launch_bounds__(256) void int_slices_kernel(const float *__restrict__ part, float *__restrict__ y, int slices, int M, int N, int64_t ldy) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, quads = (int64_t)M * N / 4;
-    if (i >= quads) return;
-    float4 v = reinterpret_cast<const float4 *>(part)[i];
-    for (int s = 1; s < slices; s++) {
-        const float4 o = reinterpret_cast<const float4 *>(part)[i + s * quads];
-        v.x += o.x, v.y += o.y, v.z += o.z, v.w += o.w;
-    }
-    const int64_t m = 4 * i / N, n = 4 * i - m * N;
-    float *to = y + m * ldy + n;
-    if constexpr (WIDE) *reinterpret_cast<float4 *>(to) = v;
-    else to[0] = v.x, to[1] = v.y, to[2] = v.z, to[3] = v.w;
+    typedef float Vec __attribute__((ext_vector_type(V)));
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, n_vec = (int64_t)M * N / V;
+    if (i >= n_vec) return;
+    Vec v = reinterpret_cast<const Vec *>(part)[i];
+    for (int s = 1; s < slices; s++) v += reinterpret_cast<const Vec *>(part)[i + s * n_vec];
+    const int64_t m = V * i / N, n = V * i - m * N;
+    *reinterpret_cast<Vec *>(y + m * ldy + n) = v;
 }
 
 __global__ __launch_bounds__(256) void bf16_to_f16_kernel(uint16_t *__restrict__ out, const uint16_t *__restrict__ in, int64_t n8) {
@@ -322,12 +318,18 @@ void launch_int_tile(const uint16_t *a16, const uint16_t *Q, const float *Dt, fl
                        act, M, N, K, ldc, row_tiles, tiles, per_slice);
 }
 
-// tiles of the plain form and the slices of super-blocks that give every compute unit about two workgroups
-int int_rows(int M) { return M > 64 ? 128 : 64; }
-int int_slices(int M, int N, int K) {
-    const int64_t tiles = (int64_t)((M + int_rows(M) - 1) / int_rows(M)) * ((N + 127) / 128), want = 2 * (int64_t)vmx_num_cus() / tiles;
-    const int nsb = K / 256;
-    if (want <= 1 || N % 4) return 1;
+// Rows of a tile: 128 where there are more than 32 such tiles.  Whole call in us, 128 / 64 rows (slices as below): 4096 columns x 2048, 100 rows
+// 33.2 / 32.0, 200 rows 26.8 / 31.0;  2048 x 3840, 65 rows 33.6 / 31.8, 400 rows 30.5 / 31.7;  512 x 1024, 65 rows 19.6 / 16.7, 256 rows 20.0 / 17.0;
+// 3840 x 15360, 128 rows 62.6 / 59.7, 256 rows 73.3 / 75.5, 400 rows 102 / 109.
+int int_rows(int M, int N) { return M > 64 && (int64_t)((M + 127) / 128) * ((N + 127) / 128) > 32 ? 128 : 64; }
+
+// Slices of super-blocks, at most `most`, that give every compute unit about two workgroups.  Without them a product with few tiles walks its K
+// alone (one / all slices: 3840 x 3840, 100 rows 56 / 30 us, 2048 x 3840 50 / 32, 512 x 2048 25 / 15); four super-blocks take little longer than
+// the launch that adds the slices.
+int int_slices(int M, int N, int K, int64_t most) {
+    const int rows = int_rows(M, N), nsb = K / 256;
+    const int64_t tiles = (int64_t)((M + rows - 1) / rows) * ((N + 127) / 128), want = std::min(2 * (int64_t)vmx_num_cus() / tiles, most);
+    if (want <= 1 || nsb <= 4) return 1;
     const int per = (int)((nsb + want - 1) / want);
     return (nsb + per - 1) / per;
 }
@@ -338,19 +340,20 @@ size_t vmx_int_gemm_part_bytes() { return (size_t)2 * vmx_num_cus() * 128 * 128 
 
 bool vmx_int_gemm_ok(int M, int N, int K) { return (int64_t)M * K * 2 < (int64_t)1 << 32 && (int64_t)N * K * 2 < (int64_t)1 << 32; }
 
-// part: vmx_int_gemm_part_bytes() of scratch, or NULL (no slices)
-int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, float *part, hipStream_t st) {
+// part: scratch for slices, as many as fit part_bytes; vmx_int_gemm_part_bytes() hold all that are wanted
+int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, float *part, size_t part_bytes, hipStream_t st) {
     const uint16_t *Q = (const uint16_t *)workspace;
     const float *Dt = (const float *)(Q + (int64_t)N * K);
-    const int slices = part ? int_slices(M, N, K) : 1;
+    const int slices = int_slices(M, N, K, (int64_t)(part_bytes / ((size_t)M * N * 4)));
     float *to = slices > 1 ? part : C;
     const int64_t ld = slices > 1 ? N : ldc;
-    if (int_rows(M) == 128) launch_int_tile<IntWide, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
+    if (int_rows(M, N) == 128) launch_int_tile<IntWide, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
     else launch_int_tile<IntMid, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
     if (slices > 1) {
-        const dim3 grid((unsigned)(((int64_t)M * N / 4 + 255) / 256));
-        if (ldc % 4 == 0 && ((uintptr_t)C & 15) == 0) hipLaunchKernelGGL(int_slices_kernel<true>, grid, dim3(256), 0, st, part, C, slices, M, N, (int64_t)ldc);
-        else hipLaunchKernelGGL(int_slices_kernel<false>, grid, dim3(256), 0, st, part, C, slices, M, N, (int64_t)ldc);
+        const bool wide = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0;
+        const dim3 grid((unsigned)(((int64_t)M * N / (wide ? 4 : 1) + 255) / 256));
+        if (wide) hipLaunchKernelGGL(int_slices_kernel<4>, grid, dim3(256), 0, st, part, C, slices, M, N, (int64_t)ldc);
+        else hipLaunchKernelGGL(int_slices_kernel<1>, grid, dim3(256), 0, st, part, C, slices, M, N, (int64_t)ldc);
     }
     VMX_CHECK_LAUNCH("int_gemm");
     return VMX_OK;
@@ -361,14 +364,17 @@ int vmx_int_gemm_geglu(const uint16_t *a16, const void *workspace, uint16_t *act
     const int N = 2 * inter;
     const uint16_t *Q = (const uint16_t *)workspace;
     const float *Dt = (const float *)(Q + (int64_t)N * K);
-    if (int_rows(M) == 128) launch_int_tile<IntWide, true>(a16, Q, Dt, nullptr, act, M, N, K, 0, 1, st);
+    if (int_rows(M, N) == 128) launch_int_tile<IntWide, true>(a16, Q, Dt, nullptr, act, M, N, K, 0, 1, st);
     else launch_int_tile<IntMid, true>(a16, Q, Dt, nullptr, act, M, N, K, 0, 1, st);
     VMX_CHECK_LAUNCH("int_gemm(geglu)");
     return VMX_OK;
 }
 
 extern "C" size_t vmx_iq_gemm_workspace_bytes(int n_out, int n_in) {
-    return n_out > 0 && n_in > 0 ? vmx_iq_gemm_workspace(n_out, n_in) : 0;
+    if (n_out <= 0 || n_in <= 0) return 0;
+    // what the product must have, and room for the slices of one with few tiles
+    const size_t least = vmx_iq_gemm_workspace(n_out, n_in);
+    return least + std::min(least, vmx_int_gemm_part_bytes());
 }
 
 extern "C" int vmx_iq_gemm_f32(int ggml_type, const void *blocks, const uint16_t *x, float *y, int m, int n_out, int n_in, void *workspace,
@@ -384,10 +390,10 @@ extern "C" int vmx_iq_gemm_f32(int ggml_type, const void *blocks, const uint16_t
         // exact one-pass form: integer weights in fp16, one f32 scale per super-block; slice sums where the workspace has room for them
         uint16_t *a16 = (uint16_t *)((char *)workspace + vmx_iq_gemm_int_workspace(0, n_out, n_in));
         const size_t used = (vmx_iq_gemm_int_workspace(m, n_out, n_in) + 255) & ~(size_t)255;
-        float *part = workspace_bytes >= used + vmx_int_gemm_part_bytes() ? (float *)((char *)workspace + used) : nullptr;
+        const size_t room = workspace_bytes > used ? workspace_bytes - used : 0;
         if (int rc = vmx_iq_dequant_int(ggml_type, blocks, workspace, 0, n_out, n_out, n_in, st)) return rc;
         if (int rc = vmx_bf16_rows_to_f16(x, a16, (int64_t)m * n_in, st)) return rc;
-        return vmx_int_gemm_f32(a16, workspace, y, m, n_out, n_in, n_out, part, st);
+        return vmx_int_gemm_f32(a16, workspace, y, m, n_out, n_in, n_out, (float *)((char *)workspace + used), room, st);
     }
     if (int rc = vmx_iq_dequant_split(ggml_type, blocks, workspace, n_out, n_in, st)) return rc;
     return vmx_split_gemm_f32(x, workspace, y, m, n_out, n_in, n_out, st);

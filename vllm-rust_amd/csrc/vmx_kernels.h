@@ -181,7 +181,7 @@ int vmx_iq_dequant_int(int ggml_type, const void *blocks, void *workspace, int r
 int vmx_bf16_rows_to_f16(const uint16_t *A, uint16_t *a16, int64_t n, hipStream_t st);
 bool vmx_int_gemm_ok(int M, int N, int K);
 size_t vmx_int_gemm_part_bytes();
-int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, float *part, hipStream_t st);
+int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, float *part, size_t part_bytes, hipStream_t st);
 int vmx_int_gemm_geglu(const uint16_t *a16, const void *workspace, uint16_t *act16, int M, int inter, int K, hipStream_t st);
 int vmx_dense_gemv_launch(uint16_t *y, const uint16_t *x, const uint16_t *W, const uint16_t *bias, int M, int N, int K, hipStream_t st,
                           int f16 = 0);   // f16: x, W, bias and y hold fp16 (same f32 accumulation, fp16 matrix / dot instructions)
