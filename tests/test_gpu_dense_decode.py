@@ -23,6 +23,7 @@ def gpu():
     ((2176, 16, 8, 128, 640), [600]),
     ((640, 5, 5, 64, 2176), [9, 2, 33, 70, 0]),
     ((1664, 18, 6, 128, 640), list(range(1, 17))),
+    ((640, 3, 1, 64, 8960), [40, 7]),
 ])
 def test_dense_decode_rows(gpu, geometry, contexts):
     """bf16 rounding points are the oracle's and only the order of the f32 sums differs: 2e-2 relative L2, as for the whole models."""

@@ -45,7 +45,7 @@ __device__ __forceinline__ void dd_unpack(dd_u32x4 v, float (&f)[8]) {
 
 constexpr int DD_STAGE = 16 * 1032;   // values that the norm and the merge stage in LDS at most: rows of K + 8
 
-// A workgroup owns CW columns: 16, or for up to four rows of a narrow product 4 (DD_GLU: half gate and the same up columns).  Lane
+// A workgroup owns CW columns: 16, or for up to four rows of a narrow product 4 (dd_narrow; DD_GLU: half gate and the same up columns).  Lane
 // (c = l & 15, g = l / 16) of v_mfma_f32_16x16x32_bf16 stands for column and row c % CW and for part c / CW of a block's k, so with
 // four columns the tile's diagonal 4 x 4 squares are the partial sums of four parts of k and the others are not used: the matrix core
 // idles anyway and the product has four times the workgroups (down of Qwen3-0.6B, [1024, 3072] at one row: 8.9 us in 64 workgroups
@@ -252,8 +252,15 @@ int dd_launch(const DenseDecode &p, hipStream_t st) {
     return VMX_OK;
 }
 
-// Four columns a workgroup where sixteen would leave compute units without one (figures: see the kernel)
-bool dd_narrow(int M, int N) { return M <= 4 && N / 16 < vmx_num_cus(); }
+// Four columns a workgroup where sixteen would leave half of the compute units or more without one: each workgroup norms or merges all rows for
+// itself, so rows times workgroups is bounded too.  us a layer (300 tokens, 100 for one row), sixteen / four columns for o and down:  hidden size 896, four
+// rows 38.1 / 35.7;  1024, one row 31.0 / 27.2, four 37.0 / 35.2;  1536, two 55.1 / 50.7, four 59.8 / 61.2;  2048, one 48.6 / 44.6, two 49.9 / 46.4, four
+// 55.1 / 55.7;  2560, one 76.6 / 77.2, two 77.9 / 83.4, four 87.0 / 112.5 (104.7 as twelve launches);  3072, one 73.3 / 77.0, four 82.6 / 106.5;  3584, two
+// 115.7 / 135.4, four 128.8 / 180.8.
+bool dd_narrow(int M, int N) {
+    const int cus = vmx_num_cus(), wide = N / 16;
+    return M <= 4 && wide <= cus / 2 && M * wide <= cus;
+}
 
 }  // namespace
 
