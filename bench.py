@@ -161,11 +161,11 @@ def prefill_block(tokens, seconds, spec):
            "frac_of_mfma_peak": round(flop / seconds / 1e12 / 2500.0, 4),
            "note": "one vmx_qwen3_prefill call (64x256-tile MFMA int4 GEMM, 32x32-tile MFMA prompt attention); untimed part of the job"}
     try:
-        j = json.loads((ROOT / "profiles" / "r03_pmc_prefill_mfma.json").read_text())
+        j = json.loads((ROOT / "profiles" / "qwen3_prompt_mfma.json").read_text())
         blk["mfma_busy_frac"] = {f"{tag}: {name.split(' (')[0]}": v["mfma_busy_frac"] for tag in ("prompt_256", "prompt_2048")
                                  for name, v in j[tag].items()}
-        blk["mfma_busy_source"] = ("profiles/r03_pmc_prefill_mfma.json (committed rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES pass over the same "
-                                   "kernels at 256- and 2048-token prompts; not measured in this run)")
+        blk["mfma_busy_source"] = ("profiles/qwen3_prompt_mfma.json (committed rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES / GRBM_GUI_ACTIVE pass over the "
+                                   "same kernels at 256- and 2048-token prompts; not measured in this run)")
     except Exception:
         pass
     return blk

@@ -10,5 +10,5 @@ timeout -s KILL 120 rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES SQ_W
 python3 tools/pmc_csv_summary.py $(find /tmp/pmc_pf$P -name "*counter_collection.csv" | head -1) > gpurun_out/pmc_prefill_$P.txt
 timeout -k 10 200 rocprofv3 --kernel-trace --stats -d /tmp/prof_pf$P -o pf -- python3 tools/prefill_long.py $P > gpurun_out/prof_pf${P}_run.log 2>&1
 python3 tools/rocpd_summary.py $(find /tmp/prof_pf$P -name "*_results.db" | head -1) > gpurun_out/prof_pf${P}_kernels.txt 2>&1 || true
-grep -A6 "prefill_attn\|int4_gemm_tiled" gpurun_out/pmc_prefill_$P.txt | head -60
-grep "prefill_attn\|int4_gemm_tiled" gpurun_out/prof_pf${P}_kernels.txt
+grep -A6 "prefill_attn\|int4_gemm_prompt" gpurun_out/pmc_prefill_$P.txt | head -60
+grep "prefill_attn\|int4_gemm_prompt" gpurun_out/prof_pf${P}_kernels.txt

@@ -241,9 +241,10 @@ typedef short la_s16x8 __attribute__((ext_vector_type(8)));
 
 // WHOLE > 0: rows of exactly 32 KSMAX values with 64 DTW latents (512 + 64).  Every size is then a constant, which leaves the registers for
 // requesting a tile's rows while the one before it is worked on, and with WHOLE = 2 for two workgroups per compute unit: 1500 tokens
-// of 16 heads 270 -> 178 us.  A partitioned launch (decode steps: one workgroup per compute unit, a tile or two each) has WHOLE = 1,
-// which keeps the setup out of scratch memory: 16 rows of 1000 tokens 22.3 -> 17.9 us
-// (WHOLE = 2: 29.7).  Other sizes (0) request a tile's rows when its turn comes.
+// of 16 heads 270 -> 178 us.  Two workgroups cap the registers at 256, and 52 more (212 bytes a lane of scratch memory) are spilled while the
+// queries and rows are set up and read back there and behind the loop; the loop over key tiles itself touches no scratch.  A partitioned
+// launch (decode steps: one workgroup per compute unit, a tile or two each) is mostly setup, so it has WHOLE = 1 without the cap and without
+// spills: 16 rows of 1000 tokens 22.3 -> 17.9 us (WHOLE = 2: 29.7).  Other sizes (0) request a tile's rows when its turn comes.
 template <int KSMAX, int DTW, int WHOLE>
 __global__ __launch_bounds__(256, WHOLE == 2 ? 2 : 1) void latent_attn_mfma_kernel(const LatentAttnArgs a) {
     extern __shared__ __align__(16) unsigned char la_smem[];
