@@ -86,13 +86,14 @@ def test_iq_prompt_linear_slices(gpu, offset, M, N, room):
     assert bool((held[:offset] == 7.0).all()) and bool((held[offset + M * N:] == 7.0).all()) and bool((ws[need:] == 7).all())
 
 
-# 256-column blocks; one k-block, odd numbers of them (17: a second step of the zero-point term; 33 in slices) and groups wider than a
+# 256-column blocks; one k-block, odd numbers of them (17; 33 in slices) and groups wider than a
 # k-block; rows around the 64-row tiles and past a strip of eight of them
 @pytest.mark.parametrize("M", [49, 64, 65, 200, 577])
 @pytest.mark.parametrize("N,K,group", [(256, 128, 128), (512, 2176, 128), (2304, 4224, 128), (256, 1536, 512), (256, 16384, 128)])
 def test_int4_prompt_tiles(gpu, M, N, K, group):
-    """Against float64 on (nibble - zero point) * scale.  The kernel adds x * (128 + nibble) and x * (128 + zero point) apart, in f32, so
-    their rounding is bounded by (k-block + k-blocks + 32) 2^-24 of sum |x| s (143 + 143); half a bf16 ulp for the result on top."""
+    """Against float64 on (nibble - zero point) * scale.  The kernel adds x * (16 + nibble) and x * (16 + zero point) apart, in f32: a path through
+    the sums has at most four roundings in each of a k-block's eight instructions and two more a k-block, and no term is larger than
+    |x| s (31 + 31); half a bf16 ulp for the result on top."""
     vmx, torch = gpu
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
@@ -107,7 +108,7 @@ def test_int4_prompt_tiles(gpu, M, N, K, group):
     zp = ((qz.unsqueeze(-1) >> sh) & 15).reshape(K // group, N).repeat_interleave(group, 0)
     s = sc.double().repeat_interleave(group, 0)
     ref = x.double() @ ((nib - zp).double() * s) + bias.double()
-    bound = 2.0 ** -8 * ref.abs() + (128 + K // 128 + 32) * 2.0 ** -24 * 286 * (x.double().abs() @ s)
+    bound = 2.0 ** -8 * ref.abs() + (32 + 2 * K // 128 + 8) * 2.0 ** -24 * 62 * (x.double().abs() @ s)
     assert bool(((y.double() - ref).abs() <= bound).all())
 
 
