@@ -86,6 +86,40 @@ def test_iq_prompt_linear_slices(gpu, offset, M, N, room):
     assert bool((held[:offset] == 7.0).all()) and bool((held[offset + M * N:] == 7.0).all()) and bool((ws[need:] == 7).all())
 
 
+# fewer than eight super-blocks: 64 x 64 tiles around whose edges rows and columns lie, in no slices, in as many as there are super-blocks, in slices of unequal
+# length (seven super-blocks in four), and one super-block more and a tile row more than that form takes (1100 x 3900: 1116 tiles)
+@pytest.mark.parametrize("M,N,K,sliced", [(17, 512, 1024, True), (65, 130, 512, False), (63, 65, 768, True), (129, 4100, 1024, False), (300, 1000, 1792, True),
+                                          (64, 2048, 1024, True), (65, 4096, 1792, True), (1200, 512, 1024, False), (1100, 3900, 512, False), (65, 512, 2048, True)])
+def test_iq_prompt_linear_short(gpu, M, N, K, sliced):
+    """Against float64 as above.  A short product is a chain of stages, and where its output is small the chain is cut although it is short: the
+    launch that adds the slices is one kernel more (weights, rows, product, sum), counted in a captured graph."""
+    import ctypes as C
+    vmx, torch = gpu
+    from tests.helpers import random_iq_blocks
+    from vllm_rust_amd._lib import check, lib
+    t = 22
+    raw = torch.from_numpy(np.ascontiguousarray(random_iq_blocks(np.random.default_rng(N + K), vmx.iq_type_size(t), N * K // 256))).reshape(-1).cuda()
+    x = torch.randn((M, K), device="cuda", generator=torch.Generator(device="cuda").manual_seed(M + N)).to(torch.bfloat16)
+    need = 4 * N * K + (32 << 20)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    held = torch.full((M + 2, N), 7.0, device="cuda")
+    y = held[1:M + 1]
+    run = lambda: check(lib.vmx_iq_gemm_f32(t, raw.data_ptr(), x.data_ptr(), y.data_ptr(), M, N, K, ws.data_ptr(), need,   # noqa: E731
+                                            torch.cuda.current_stream().cuda_stream))
+    run()
+    torch.cuda.synchronize()
+    w = vmx.iq_dequantize(t, raw, N * K // 256).reshape(N, K).double()
+    bound = (264 + K // 256 + 8) * 2.0 ** -24 * (x.double().abs() @ w.abs().T)
+    assert bool(((y.double() - x.double() @ w.T).abs() <= bound).all())
+    assert bool((held[0] == 7.0).all()) and bool((held[M + 1] == 7.0).all())
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        run()
+    n = C.c_size_t(0)
+    assert C.CDLL("libamdhip64.so").hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None, C.byref(n)) == 0
+    assert n.value == (4 if sliced else 3)
+
+
 # 256-column blocks; one k-block, odd numbers of them (17; 33 in slices) and groups wider than a
 # k-block; rows around the 64-row tiles and past a strip of eight of them
 @pytest.mark.parametrize("M", [49, 64, 65, 200, 577])

@@ -308,6 +308,7 @@ int vmx_bf16_rows_to_f16(const uint16_t *A, uint16_t *a16, int64_t n, hipStream_
 namespace {
 typedef TgShape<2, 2, 2, 2, 2> IntWide;     // 128 x 128
 typedef TgShape<2, 2, 1, 2, 2> IntMid;      // 64 x 128
+typedef TgShape<2, 2, 1, 1, 2> IntSmall;    // 64 x 64
 
 template <class S, bool GEGLU>
 void launch_int_tile(const uint16_t *a16, const uint16_t *Q, const float *Dt, float *C, uint16_t *act, int M, int N, int K, int64_t ldc, int slices,
@@ -319,19 +320,39 @@ void launch_int_tile(const uint16_t *a16, const uint16_t *Q, const float *Dt, fl
 }
 
 // Rows of a tile: 128 where there are more than 32 such tiles.  Whole call in us, 128 / 64 rows (slices as below): 4096 columns x 2048, 100 rows
-// 33.2 / 32.0, 200 rows 26.8 / 31.0;  2048 x 3840, 65 rows 33.6 / 31.8, 400 rows 30.5 / 31.7;  512 x 1024, 65 rows 19.6 / 16.7, 256 rows 20.0 / 17.0;
-// 3840 x 15360, 128 rows 62.6 / 59.7, 256 rows 73.3 / 75.5, 400 rows 102 / 109.
+// 33.2 / 32.0, 200 rows 26.8 / 31.0;  2048 x 3840, 65 rows 33.6 / 31.8, 400 rows 30.5 / 31.7;  3840 x 15360, 128 rows 62.6 / 59.7, 256 rows
+// 73.3 / 75.5, 400 rows 102 / 109.
 int int_rows(int M, int N) { return M > 64 && (int64_t)((M + 127) / 128) * ((N + 127) / 128) > 32 ? 128 : 64; }
 
 // Slices of super-blocks, at most `most`, that give every compute unit about two workgroups.  Without them a product with few tiles walks its K
-// alone (one / all slices: 3840 x 3840, 100 rows 56 / 30 us, 2048 x 3840 50 / 32, 512 x 2048 25 / 15); four super-blocks take little longer than
-// the launch that adds the slices.
+// alone (one / all slices: 3840 x 3840, 100 rows 56 / 30 us, 2048 x 3840 50 / 32, 512 x 2048 25 / 15).
 int int_slices(int M, int N, int K, int64_t most) {
     const int rows = int_rows(M, N), nsb = K / 256;
     const int64_t tiles = (int64_t)((M + rows - 1) / rows) * ((N + 127) / 128), want = std::min(2 * (int64_t)vmx_num_cus() / tiles, most);
-    if (want <= 1 || nsb <= 4) return 1;
+    if (want <= 1) return 1;
     const int per = (int)((nsb + want - 1) / want);
     return (nsb + per - 1) / per;
+}
+
+// A short K is a chain of few stages whose latency the tile's size decides: below eight super-blocks tiles are 64 x 64, up to four a compute unit.
+// us, 128- or 64-row tiles as above uncut / 64 x 64 tiles with the slices below: 17 x 512 x 1024 17.9 / 13.3, 65 x 8192 x 1024 31.3 / 26.7, 200 x 4096 x
+// 1024 25.2 / 20.7, 600 x 4096 x 1024 26.9 / 23.3, 400 x 2048 x 1280 29.8 / 21.2, 1000 x 2048 x 512 18.7 / 15.9; six tiles a unit no longer, 1200 x 8192 x
+// 1024 45.8 / 47.2.  From eight super-blocks on slices hide the latency: 200 x 4096 x 2048 28.5 / 30.9, 400 x 4096 x 4096 41.9 / 43.6.
+bool int_short(int M, int N, int K) { return K < 8 * 256 && (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 4 * vmx_num_cus(); }
+
+// Its slices: the count with the least estimated time of 1.6 us a super-block (1.9 with two workgroups a unit) and, for more than one, of a
+// launch and the f32 sums written and read.  1024 deep, one / two / four slices in us: 17 x 512 16.0 / 14.5 / 13.3, 200 x 1024 17.1 / 16.0 / 15.5,
+// 65 x 4096 20.1 / 19.6 / 19.8, 400 x 2048 18.8 / 20.7 / 24.1; 512 deep, 17 x 2048 12.9 / 13.2.
+int int_short_slices(int M, int N, int K, int64_t most) {
+    const int nsb = K / 256, tiles = ((M + 63) / 64) * ((N + 63) / 64), cus = vmx_num_cus();
+    int best = 1;
+    int64_t least = nsb * (tiles > cus ? 1900 : 1600);
+    for (int s = 2; s <= nsb && s <= most && tiles * s <= 2 * cus; s++) {
+        const int per = (nsb + s - 1) / s;
+        const int64_t ns = per * (tiles * s > cus ? 1900 : 1600) + 1700 + (int64_t)s * M * N * 8 / 5000;
+        if ((nsb + per - 1) / per == s && ns < least) least = ns, best = s;
+    }
+    return best;
 }
 }  // namespace
 
@@ -344,10 +365,13 @@ bool vmx_int_gemm_ok(int M, int N, int K) { return (int64_t)M * K * 2 < (int64_t
 int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, float *part, size_t part_bytes, hipStream_t st) {
     const uint16_t *Q = (const uint16_t *)workspace;
     const float *Dt = (const float *)(Q + (int64_t)N * K);
-    const int slices = int_slices(M, N, K, (int64_t)(part_bytes / ((size_t)M * N * 4)));
+    const int64_t fit = (int64_t)(part_bytes / ((size_t)M * N * 4));
+    const bool brief = int_short(M, N, K);
+    const int slices = brief ? int_short_slices(M, N, K, fit) : int_slices(M, N, K, fit);
     float *to = slices > 1 ? part : C;
     const int64_t ld = slices > 1 ? N : ldc;
-    if (int_rows(M, N) == 128) launch_int_tile<IntWide, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
+    if (brief) launch_int_tile<IntSmall, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
+    else if (int_rows(M, N) == 128) launch_int_tile<IntWide, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
     else launch_int_tile<IntMid, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
     if (slices > 1) {
         const bool wide = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0;
