@@ -171,8 +171,8 @@ def test_int4_prompt_f32_sums(gpu, M, N, K, mean):
     assert float((y ** 2).mean().sqrt()) <= float(2.0 ** -24 * (8 * K // 128) ** 0.5 * size)
 
 
-# decode rows: column groups below one per compute unit (halved k; 4 and 8 waves, a second round), between one and two, and above
-@pytest.mark.parametrize("M,N,K", [(1, 40, 72), (16, 2048, 2040), (5, 1000, 2312), (3, 4100, 520), (16, 4096, 1032), (7, 6000, 2056), (16, 9000, 136)])
+# decode rows: column groups below one per compute unit (up to 512 deep, beyond with halved k; 4 and 8 waves, a second round), between one and two, and above
+@pytest.mark.parametrize("M,N,K", [(1, 40, 72), (16, 30, 384), (9, 2100, 512), (4, 200, 520), (16, 2048, 2040), (5, 1000, 2312), (3, 4100, 520), (16, 4096, 1032), (7, 6000, 2056), (16, 9000, 136)])
 @pytest.mark.parametrize("x_f32", [False, True])
 def test_bf16_linear_decode_rows(gpu, M, N, K, x_f32):
     """f32 sums of bf16 products in at most K terms: |error| <= K 2^-24 sum |x w|, doubled for the order of the partial sums."""

@@ -399,11 +399,13 @@ void launch_skinny_as(const VmxLinear &p, hipStream_t st) {
 //   [12288, 2048], two groups a compute unit or more: 21.3 -> 16.6 us (the 64 bytes across lanes; 8 waves: 16.8); [32000, 2048]: 46.6 -> 36.7
 //   [11264, 2048]: 21.2 -> 16.4;  [3664, 2048], fewer groups than compute units: 10.4 -> 8.4
 //   [2048, 2048] and [2048, 6144], 128 groups: 12.4 on average -> 6.4 and 12.7
+// Up to 512 deep a wave has one block of 16 columns: with eight columns and k halved it loads twice the rows for the same chain, which one f32 row paid
+// for.  1 / 16 f32 rows, before / eight columns / now: [256, 256] 3.7 / 3.9 / 3.2 and 4.6 / 4.3 / 3.3, [4000, 512] 4.1 / 4.5 / 3.5 and 5.3 / 4.8 / 3.8
 // Expert blocks bring row blocks of their own and keep four waves.
 void launch_skinny(const VmxLinear &p, hipStream_t st) {
     const int cols = (p.N + 15) / 16 * p.batch, cus = vmx_num_cus();
     if (p.block_expert || cols >= 2 * cus) return launch_skinny_as<4, 1, 2>(p, st);
-    if (cols >= cus) {
+    if (cols >= cus || p.K <= 512) {
         const int nblk = (p.K + 127) / 128;
         return nblk <= 4 ? launch_skinny_as<4, 1, 1>(p, st) : nblk <= 8 ? launch_skinny_as<8, 1, 1>(p, st) : launch_skinny_as<8, 1, 2>(p, st);
     }
