@@ -40,6 +40,16 @@ def test_bf16_linear_tiles(gpu, M, N, K, out):
     assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all())
 
 
+# on 256 compute units, in this order: 64 x 128 tiles, 128 x 128 two a unit, 128 x 128 one a unit, 192 x 128 (rows and columns past the last whole
+# tile; whole tiles, whose bf16 results go out in pairs), 256 x 128 (the same two)
+@pytest.mark.parametrize("M,N,K", [(129, 12801, 128), (513, 11001, 320), (1023, 2049, 2048), (383, 12281, 1024), (384, 12288, 1024), (511, 12281, 2048),
+                                   (512, 12288, 2048)])
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+def test_bf16_linear_tile_shapes(gpu, M, N, K, out):
+    """As test_bf16_linear_tiles, the same bounds."""
+    test_bf16_linear_tiles(gpu, M, N, K, out)
+
+
 # rows around the 64- and 128-row tiles; columns around the 128-wide ones; K of one super-block, an odd number of them, and enough with
 # few tiles that the sums are cut into slices ((2048, 8192) gives the workspace room for them, (64, 256) does not)
 @pytest.mark.parametrize("M", [17, 64, 65, 129, 300])

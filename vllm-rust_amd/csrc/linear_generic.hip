@@ -14,6 +14,7 @@
 // `linear_fma_kernel` multiplies in true f32 on the vector ALU (the 32-bit mode of a model), `linear_fewcols_f32_kernel` does the
 // same for a few output columns (router logits) with one kernel for every row count.  A row's result never depends on the other rows of the call: within a kernel a row is summed in
 // the same order whatever M is; between the streaming and the tiled kernels the order differs (rounding-level differences).
+#include <algorithm>
 #include "tile_gemm.h"
 
 namespace {
@@ -234,12 +235,64 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const VmxLinear p) {
         }
 }
 
+// The accumulators to rows wm .., columns wn .. of C.  A tile inside C goes out without a look at each row: the choices and 64-bit
+// addresses of the general form cost a 192 x 128 tile 6 us, a fifth of its products 2048 deep (1500 x 12288 x 2048: 105 -> 86 us).  bf16 columns go out in
+// pairs: lane c even takes columns c, c + 1 of one row, its neighbour the same of the next row.
+template <class S, typename T>
+__device__ __forceinline__ void linear_tile_store(const VmxLinear &p, int z, int wm, int wn, int lane, tg_f32x16 (&acc)[S::MI][S::NJ]) {
+    const int col = lane & 31;
+    T *C = (T *)p.C + z * p.c_bs;
+    if (!p.row_ids && wm + 32 * S::MI <= p.M && wn + 32 * S::NJ <= p.N) {
+        constexpr bool PAIRS = sizeof(T) == 2;
+        const bool odd = lane & 1, pairs = PAIRS && (((uintptr_t)C | (2 * p.ldc) | (2 * wn)) & 3) == 0;
+        T *at = C + (int64_t)wm * p.ldc + wn;                                               // uniform
+        const uint32_t off = (uint32_t)(4 * (lane >> 5)) * (uint32_t)p.ldc;                 // elements
+#pragma unroll
+        for (int i = 0; i < S::MI; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                T *row = at + (int64_t)(32 * i + 8 * (r >> 2) + (r & 3)) * p.ldc;
+#pragma unroll
+                for (int j = 0; j < S::NJ; j++) {
+                    const float a = acc[i][j][r], b = acc[i][j][r + 1];
+                    if constexpr (!PAIRS) {
+                        row[32 * j + off + col] = a;
+                        row[32 * j + p.ldc + off + col] = b;
+                    } else if (pairs) {
+                        const float got = vmx_dpp<VMX_DPP_XOR1>(odd ? a : b);
+                        const uint32_t two = odd ? (uint32_t)vmx_f32_to_bf16(got) | (uint32_t)vmx_f32_to_bf16(b) << 16
+                                                 : (uint32_t)vmx_f32_to_bf16(a) | (uint32_t)vmx_f32_to_bf16(got) << 16;
+                        *reinterpret_cast<uint32_t *>(row + 32 * j + (off + (odd ? (uint32_t)p.ldc : 0u) + (col & 30))) = two;
+                    } else {
+                        row[32 * j + off + col] = vmx_f32_to_bf16(a);
+                        row[32 * j + p.ldc + off + col] = vmx_f32_to_bf16(b);
+                    }
+                }
+            }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < S::MI; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int m = wm + 32 * i + tg_acc_row(lane, r);
+            if (m >= p.M || (p.row_ids && linear_src_row(p, m) < 0)) continue;
+            T *row = C + (int64_t)m * p.ldc + wn + col;
+#pragma unroll
+            for (int j = 0; j < S::NJ; j++) {
+                if (wn + 32 * j + col >= p.N) continue;
+                if constexpr (sizeof(T) == 4) row[32 * j] = acc[i][j][r];
+                else row[32 * j] = vmx_f32_to_bf16(acc[i][j][r]);
+            }
+        }
+}
+
 // Prompt-sized bf16 products on the core of tile_gemm.h: plain, batched, gathered rows and 64-row expert blocks alike.  EP: the
 // finished sums are stored as they are, with a bias and a SiLU range, or through linear_store (whose run-time choices per element cost a
 // 1500 x 12288 output as much as half of its product: 159 against 101 us).
 enum { TILE_PLAIN, TILE_BIAS_SILU, TILE_ANY };
 template <class S, int EP>
-__global__ __launch_bounds__(S::THREADS) void linear_tile_kernel(const VmxLinear p, int row_tiles, int tiles) {
+__global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(const VmxLinear p, int row_tiles, int tiles) {
     extern __shared__ __align__(1024) uint16_t tg_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tile = tg_tile(blockIdx.x, tiles), z = blockIdx.y;
@@ -265,33 +318,38 @@ __global__ __launch_bounds__(S::THREADS) void linear_tile_kernel(const VmxLinear
         for (int j = 0; j < S::NJ; j++) acc[i][j] = tg_f32x16{};
     const TgCore<false, S> core{(const char *)((const uint16_t *)p.A + z * p.a_bs), (const char *)W, a_src, b_src, tg_lds_at(tg_lds), wave, lane};
     tg_product(core, p.K, acc);
-    const int wm = m0 + wave / S::WN * (S::MI * 32), wn = n0 + wave % S::WN * (S::NJ * 32) + (lane & 31);
-#pragma unroll
-    for (int j = 0; j < S::NJ; j++) {
-        const int n = wn + 32 * j;
-        if (n >= p.N) continue;
-        const float bias = EP == TILE_BIAS_SILU && p.bias ? vmx_bf16_to_f32(p.bias[n + z * p.bias_bs]) : 0.f;
-        const bool silu = n >= p.silu_begin && n < p.silu_end;
+    const int wm = m0 + wave / S::WN * (S::MI * 32), wn = n0 + wave % S::WN * (S::NJ * 32), col = lane & 31;
+    if constexpr (EP == TILE_ANY) {
 #pragma unroll
         for (int i = 0; i < S::MI; i++)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int m = wm + 32 * i + tg_acc_row(lane, r);
                 if (m >= p.M || (p.row_ids && linear_src_row(p, m) < 0)) continue;
-                float v = acc[i][j][r];
-                if constexpr (EP == TILE_ANY) {
-                    linear_store(p, z, m, n, v);
-                    continue;
-                }
-                if constexpr (EP == TILE_BIAS_SILU) {
-                    v += bias;
-                    if (silu) v /= 1.0f + expf(-v);
-                }
-                const int64_t o = (int64_t)m * p.ldc + n + z * p.c_bs;
-                if (p.c_f32) ((float *)p.C)[o] = v;
-                else ((uint16_t *)p.C)[o] = vmx_f32_to_bf16(v);
+#pragma unroll
+                for (int j = 0; j < S::NJ; j++)
+                    if (wn + 32 * j + col < p.N) linear_store(p, z, m, wn + 32 * j + col, acc[i][j][r]);
             }
+        return;
     }
+    if constexpr (EP == TILE_BIAS_SILU) {
+#pragma unroll
+        for (int j = 0; j < S::NJ; j++) {
+            const int n = wn + 32 * j + col;
+            const float bias = p.bias && n < p.N ? vmx_bf16_to_f32(p.bias[n + z * p.bias_bs]) : 0.f;
+            const bool silu = n >= p.silu_begin && n < p.silu_end;
+#pragma unroll
+            for (int i = 0; i < S::MI; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    float v = acc[i][j][r] + bias;
+                    if (silu) v /= 1.0f + expf(-v);
+                    acc[i][j][r] = v;
+                }
+        }
+    }
+    if (p.c_f32) linear_tile_store<S, float>(p, z, wm, wn, lane, acc);
+    else linear_tile_store<S, uint16_t>(p, z, wm, wn, lane, acc);
 }
 
 // Up to 16 rows (decode steps, 16-row expert blocks): the product is a stream over the weights.  A workgroup owns 16 output columns, or
@@ -451,7 +509,7 @@ bool tile_ok(const VmxLinear &p, bool direct) {
 template <class S, int EP>
 int launch_tile_as(const VmxLinear &p, hipStream_t st) {
     const int row_tiles = (p.M + S::BM - 1) / S::BM, tiles = row_tiles * ((p.N + S::BN - 1) / S::BN);
-    static_assert(S::LDS <= 64 * 1024, "no attribute needed");
+    VMX_CHECK_HIP(hipFuncSetAttribute((const void *)linear_tile_kernel<S, EP>, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS));
     hipLaunchKernelGGL((linear_tile_kernel<S, EP>), dim3(tg_grid(tiles), p.batch), dim3(S::THREADS), S::LDS, st, p, row_tiles, tiles);
     return VMX_OK;
 }
@@ -463,16 +521,45 @@ int launch_tile_shape(const VmxLinear &p, hipStream_t st) {
     return launch_tile_as<S, TILE_PLAIN>(p, st);
 }
 
-// 128 x 128 tiles, two stages (two workgroups a compute unit) where there is one for every compute unit; else 64 x 64 tiles, with a
-// third stage where two or fewer of them share a unit and latency is all that counts.  us on 256 units, 128 x 128 / 64 x 64 in two / in
-// three stages:  1500 x 12288 x 2048 101 / 132 / 142;  1500 x 3664 x 2048 (348 tiles of 128) 35 / 45 / 45;  1500 x 2048 x 2048 (192)
-// 29 / 24 / 26;  100 x 12288 x 2048 (96) 27 / 19 / 17;  65 x 2048 x 2048 25 / 13 / 13.  Every shape adds an element's k in the same order.
+// Every shape adds an element's k in the same order.
+typedef TgShape<2, 2, 1, 1, 5> Tile64;       // 64 x 64, two workgroups a compute unit
+typedef TgShape<2, 2, 1, 2, 3> Tile64w;      // 64 x 128, two
+typedef TgShape<2, 2, 2, 2, 2> Tile128two;   // 128 x 128, two
+typedef TgShape<2, 4, 2, 1, 4> Tile128;      // 128 x 128, one
+typedef TgShape<2, 2, 3, 2, 3> Tile192;      // 192 x 128, one
+typedef TgShape<4, 2, 2, 2, 3> Tile256;      // 256 x 128, one
+
+// Estimated ns of a launch.  It runs in rounds of one tile for every place; a 64-deep step of a full round takes `full`, one with at most a
+// workgroup for every second place `few` (shapes with two places a unit), and a last round is shorter, the emptier it is (least so where it is the
+// only one of a shape with two places).  The results leave at 9.2 TB/s (into the L2), half of that time under the products of the unit's other
+// workgroup where it has one.
+template <class S>
+int64_t tile_ns(const VmxLinear &p, int full, int few) {
+    const int64_t tiles = (int64_t)((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN) * p.batch, places = (int64_t)vmx_num_cus() * S::PER_UNIT;
+    const int64_t rounds = tiles / places, rest = tiles % places, out = (int64_t)p.M * p.N * p.batch * (p.c_f32 ? 4 : 2) / (S::PER_UNIT > 1 ? 18400 : 9200);
+    if (S::PER_UNIT > 1 && tiles <= places / 2) return p.K / TG_BK * (int64_t)few + out;
+    const int64_t last = rest == 0 ? 0 : S::PER_UNIT == 1 ? full * (3 * places + rest) / (4 * places)
+                                       : rounds == 0 ? full * (4 * places + rest) / (5 * places) : full * (2 * places + 3 * rest) / (5 * places);
+    return p.K / TG_BK * (rounds * full + last) + out;
+}
+
+// The shape with the least estimate.  Fitted to bf16 products of 17 .. 2000 rows on 256 units, weights out of HBM.  us, 64 x 64 / 64 x 128 / 128 x 128
+// two / one a unit / 192 / 256 x 128 (rows x columns x depth, bf16 results):  100 x 12288 x 2048 19 / 19 / 31 / 21 / 25 / 25;  200 24 / 25 / 33 / 21 /
+// 26 / 29;  500 49 / 42 / 38 / 42 / 51 / 32;  700 67 / 59 / 64 / 57 / 53 / 59;  1000 94 / 77 / 68 / 64 / 75 / 62;  1500 139 / 107 / 99 / 99 / 83 / 90;
+// 1500 x 11264 x 2048 129 / 99 / 89 / 92 / 83 / 81;  1500 x 3664 x 2048 47 / 38 / 33 / 41 / 28 / 30;  1000 x 2048 x 6144 48 / 47 / 79 / 53 / 57 / 73;
+// 1500 x 2048 x 6144 74 / 61 / 81 / 53 / 65 / 73.  The call before (128 x 128 two a unit, or 64 x 64 in two or three stages, requests at the head of a
+// stage, results element by element) and now:  1500 x 12288 x 2048 107 -> 85, 1500 x 3664 x 2048 36 -> 28, 1500 x 2048 x 6144 72 -> 53, 500 x 12288 x
+// 2048 42 -> 33, 333 x 2048 x 6144 35 -> 25, 100 x 3664 x 2048 14.6 -> 11.2.  Expert blocks bring 64 rows each.
 int launch_tile(const VmxLinear &p, hipStream_t st) {
-    const int64_t cus = vmx_num_cus();
-    const int64_t t128 = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch, t64 = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
-    if (!p.block_expert && t128 >= cus) return launch_tile_shape<TgShape<2, 2, 2, 2, 2>>(p, st);
-    if (t64 > 2 * cus) return launch_tile_shape<TgShape<2, 2, 1, 1, 2>>(p, st);
-    return launch_tile_shape<TgShape<2, 2, 1, 1, 3>>(p, st);
+    const int64_t t64 = tile_ns<Tile64>(p, 490, 280), t64w = tile_ns<Tile64w>(p, 700, 450);
+    if (p.block_expert) return t64 <= t64w ? launch_tile_shape<Tile64>(p, st) : launch_tile_shape<Tile64w>(p, st);
+    const int64_t two = tile_ns<Tile128two>(p, 1130, 800), t128 = tile_ns<Tile128>(p, 640, 0), t192 = tile_ns<Tile192>(p, 850, 0),
+                  t256 = tile_ns<Tile256>(p, 1000, 0), least = std::min({t64, t64w, two, t128, t192, t256});
+    if (least == t64) return launch_tile_shape<Tile64>(p, st);
+    if (least == t64w) return launch_tile_shape<Tile64w>(p, st);
+    if (least == t128) return launch_tile_shape<Tile128>(p, st);
+    if (least == t192) return launch_tile_shape<Tile192>(p, st);
+    return least == t256 ? launch_tile_shape<Tile256>(p, st) : launch_tile_shape<Tile128two>(p, st);
 }
 
 }  // namespace

@@ -5,12 +5,17 @@
 //   * both operand tiles (64 deep) go from global memory straight into LDS (global_load_lds, 16 bytes per lane: no registers, no
 //     vector-ALU work).  A staged row is 128 bytes, unpadded; the 16-byte chunk c of row r sits at position c ^ (r & 7), so the eight
 //     rows that a group of eight lanes reads lie in eight different bank groups;
-//   * two or three stages; the requests are issued by an instruction the compiler does not track (tg_request_1k), because behind one that it does it
+//   * the requests are issued by an instruction the compiler does not track (tg_request_1k), because behind one that it does it
 //     makes every LDS read wait for all requests under way, the other stage's included.  The waits are written out instead;
-//   * one barrier per stage, a later stage's requests right behind it;
+//   * a request occupies the address path of the compute unit for 16 clocks and a wave that issues several in a row stands still while the
+//     path is busy, its products included.  tg_product therefore spreads the requests of the stage two ahead between the products of the
+//     stage in use (three stages in LDS), and reads a stage's first fragments under the last products of the one before it.  Against all requests at the
+//     head of a stage, bf16, rows x columns x depth: 128 x 128 tiles 1500 x 2048 x 6144 51 -> 43 us (727 -> 889 TFLOP/s), 256 x 128 tiles 2048 x 24576 x
+//     4096 404 -> 369 us (1116 TFLOP/s; products alone, no memory: 1550 on random numbers, where the clock falls to 1.6 GHz);
 //   * tiles are numbered row-fastest and dealt to the eight XCDs in contiguous runs (workgroup i runs on XCD i % 8), so the rows of a
 //     column block are multiplied out of one XCD's L2.
 #pragma once
+#include <type_traits>
 #include "vmx_kernels.h"
 
 typedef float tg_f32x16 __attribute__((ext_vector_type(16)));
@@ -55,6 +60,7 @@ struct TgShape {
     static constexpr int BM = WM * MI * 32, BN = WN * NJ * 32, WAVES = WM * WN, THREADS = 64 * WAVES;
     static constexpr int AQ = BM / (8 * WAVES), BQ = BN / (8 * WAVES);            // requests of eight rows a wave makes per operand and stage
     static constexpr int STAGE = (BM + BN) * TG_BK, LDS = STAGES * STAGE * 2;     // elements, bytes
+    static constexpr int PER_UNIT = 160 * 1024 / LDS, PER_SIMD = PER_UNIT * WAVES > 4 ? PER_UNIT * WAVES / 4 : 1;   // workgroups a compute unit, waves a SIMD
     static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0 && STAGES >= 2, "whole requests per wave");
 };
 
@@ -72,32 +78,35 @@ struct TgCore {
     uint32_t lds;                            // byte address of the stages (tg_lds_at)
     int wave, lane;
 
-    __device__ __forceinline__ void request(int t, int stage) const {
+    // request q (of AQ + BQ) of this wave for step t
+    __device__ __forceinline__ void request_one(int t, int stage, int q) const {
         const uint32_t to = lds + stage * (S::STAGE * 2);
-#pragma unroll
-        for (int q = 0; q < S::AQ; q++) tg_request_1k(to + (wave * S::AQ + q) * (8 * TG_BK * 2), A + (int64_t)t * (2 * TG_BK), a_src[q]);
-#pragma unroll
-        for (int q = 0; q < S::BQ; q++) tg_request_1k(to + (S::BM + (wave * S::BQ + q) * 8) * (TG_BK * 2), B + (int64_t)t * (2 * TG_BK), b_src[q]);
+        if (q < S::AQ) tg_request_1k(to + (wave * S::AQ + q) * (8 * TG_BK * 2), A + (int64_t)t * (2 * TG_BK), a_src[q < S::AQ ? q : 0]);
+        else tg_request_1k(to + (S::BM + (wave * S::BQ + q - S::AQ) * 8) * (TG_BK * 2), B + (int64_t)t * (2 * TG_BK), b_src[q < S::AQ ? 0 : q - S::AQ]);
     }
-    // acc += the 64 deep products of a stage; FRESH: acc = them
-    template <bool FRESH = false>
-    __device__ __forceinline__ void multiply(int stage, tg_f32x16 (&acc)[S::MI][S::NJ]) const {
-        // byte addresses of step 0; chunk c lies at c ^ (row & 7), so step s is step 0 with 32 s flipped in
+    __device__ __forceinline__ void request(int t, int stage) const {
+#pragma unroll
+        for (int q = 0; q < S::AQ + S::BQ; q++) request_one(t, stage, q);
+    }
+    // the wave's fragments of the 16 deep step s of a stage.  Chunk c lies at c ^ (row & 7), so step s is step 0 with 32 s flipped in.
+    __device__ __forceinline__ void read(int stage, int s, tg_u32x4 (&af)[S::MI], tg_u32x4 (&bf)[S::NJ]) const {
         const int fr = lane & 31, first = (((lane >> 5) ^ (fr & 7)) << 4);
         const uint32_t from = lds + stage * (S::STAGE * 2);
         const uint32_t arow = from + ((wave / S::WN) * (S::MI * 32) + fr) * (TG_BK * 2) + first;
         const uint32_t brow = from + (S::BM + (wave % S::WN) * (S::NJ * 32) + fr) * (TG_BK * 2) + first;
+#pragma unroll
+        for (int i = 0; i < S::MI; i++) af[i] = tg_lds_read((arow ^ (32 * s)) + i * (32 * TG_BK * 2));
+#pragma unroll
+        for (int j = 0; j < S::NJ; j++) bf[j] = tg_lds_read((brow ^ (32 * s)) + j * (32 * TG_BK * 2));
+    }
+    // acc += the 64 deep products of a stage; FRESH: acc = them
+    template <bool FRESH = false>
+    __device__ __forceinline__ void multiply(int stage, tg_f32x16 (&acc)[S::MI][S::NJ]) const {
         tg_u32x4 af[2][S::MI], bf[2][S::NJ];   // fragments of the 16 deep step in use and of the next one
-        auto read = [&](int s) {
-#pragma unroll
-            for (int i = 0; i < S::MI; i++) af[s & 1][i] = tg_lds_read((arow ^ (32 * s)) + i * (32 * TG_BK * 2));
-#pragma unroll
-            for (int j = 0; j < S::NJ; j++) bf[s & 1][j] = tg_lds_read((brow ^ (32 * s)) + j * (32 * TG_BK * 2));
-        };
-        read(0);
+        read(stage, 0, af[0], bf[0]);
 #pragma unroll
         for (int s = 0; s < TG_BK / 16; s++) {
-            if (s + 1 < TG_BK / 16) read(s + 1);
+            if (s + 1 < TG_BK / 16) read(stage, s + 1, af[(s + 1) & 1], bf[(s + 1) & 1]);
 #pragma unroll
             for (int i = 0; i < S::MI; i++)
 #pragma unroll
@@ -117,23 +126,69 @@ struct TgCore {
 // acc += sum over k in [0, K), K a positive multiple of 64.
 template <bool F16, class S>
 __device__ __forceinline__ void tg_product(const TgCore<F16, S> &core, int K, tg_f32x16 (&acc)[S::MI][S::NJ]) {
-    constexpr int AHEAD = S::STAGES - 1;
+    if constexpr (S::STAGES == 2) {   // a whole stage's requests at its head; the other workgroup of the compute unit multiplies meanwhile
+        const int steps = K / TG_BK;
+        core.request(0, 0);
+        for (int t = 0; t < steps; t++) {
+            core.template arrive<0>();
+            if (t + 1 < steps) core.request(t + 1, (t + 1) & 1);
+            core.multiply(t & 1, acc);
+        }
+        return;
+    }
+    constexpr int AHEAD = S::STAGES - 1, R = S::AQ + S::BQ, SUB = TG_BK / 16, P = S::MI * S::NJ;
     const int steps = K / TG_BK;
+    tg_u32x4 af[2][S::MI], bf[2][S::NJ];   // fragments of the 16 deep step in use and of the next one
+    // the products of stage `cur` (its first fragments are in af[0], bf[0]); REQUEST: with the requests of step t + AHEAD between them, which go to
+    // the stage that was read before this one; MORE: the next stage's first fragments are read
+    auto stage = [&](auto request, auto more, int t, int cur) {
+        constexpr bool REQUEST = decltype(request)::value, MORE = decltype(more)::value;
+        const int next = cur == AHEAD ? 0 : cur + 1, free = cur == 0 ? AHEAD : cur - 1;
+#pragma unroll
+        for (int s = 0; s < SUB; s++) {
+            if (s + 1 < SUB) {
+                core.read(cur, s + 1, af[(s + 1) & 1], bf[(s + 1) & 1]);
+            } else if (MORE) {
+                core.template arrive<REQUEST ? R * (AHEAD - 1) : 0>();
+                core.read(next, 0, af[0], bf[0]);
+            }
+#pragma unroll
+            for (int i = 0; i < S::MI; i++)
+#pragma unroll
+                for (int j = 0; j < S::NJ; j++) {
+                    acc[i][j] = tg_mfma<F16>(af[s & 1][i], bf[s & 1][j], acc[i][j]);
+                    // behind product n of the first SUB - 1 sub-steps: requests up to R (n + 1) / all of those products
+                    const int n = s * P + i * S::NJ + j;
+                    if (REQUEST && s + 1 < SUB) {
+#pragma unroll
+                        for (int q = 0; q < R; q++)
+                            if (q >= (n * R + (SUB - 1) * P - 1) / ((SUB - 1) * P) && q < ((n + 1) * R + (SUB - 1) * P - 1) / ((SUB - 1) * P)) {
+                                __builtin_amdgcn_sched_barrier(0);
+                                core.request_one(t + AHEAD, free, q);
+                            }
+                    }
+                }
+            __builtin_amdgcn_sched_barrier(0);   // the reads stay ahead of the products they run under
+        }
+    };
+    const std::true_type yes;
+    const std::false_type no;
 #pragma unroll
     for (int t = 0; t < AHEAD; t++)
         if (t < steps) core.request(t, t);
+    if (steps >= AHEAD) core.template arrive<R * (AHEAD - 1)>();
+    else core.template arrive<0>();
+    core.read(0, 0, af[0], bf[0]);
     int cur = 0, t = 0;
     for (; t + AHEAD < steps; t++) {
-        core.template arrive<(S::AQ + S::BQ) * (AHEAD - 1)>();
-        core.request(t + AHEAD, cur == 0 ? AHEAD : cur - 1);
-        core.multiply(cur, acc);
+        stage(yes, yes, t, cur);
         cur = cur == AHEAD ? 0 : cur + 1;
     }
-    for (; t < steps; t++) {
-        core.template arrive<0>();
-        core.multiply(cur, acc);
+    for (; t + 1 < steps; t++) {
+        stage(no, yes, t, cur);
         cur = cur == AHEAD ? 0 : cur + 1;
     }
+    stage(no, no, t, cur);
 }
 
 // acc[m][n] += sum over groups of 256 k of scale(group, n) * (sum over the group's k), groups of them; two stages.
