@@ -1,5 +1,7 @@
 """Prompt-sized products on the shared matrix-core tiles (csrc/tile_gemm.h) at the edges of their tiles, stages and shape choices,
 and the decode-row linears at the edges of theirs."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -128,6 +130,90 @@ def test_iq_prompt_linear_short(gpu, M, N, K, sliced):
     n = C.c_size_t(0)
     assert C.CDLL("libamdhip64.so").hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None, C.byref(n)) == 0
     assert n.value == (4 if sliced else 3)
+
+
+# raw blocks decoded inside the product: rows at and past every tile height; an odd number of super-blocks (block starts alternate between
+# the halves of a dword along a row and from row to row) and an even one; columns past a tile; a weight that starts in the middle of a dword; room for
+# slices of k and none
+@pytest.mark.parametrize("M", [17, 64, 65, 129, 192, 256, 333])
+@pytest.mark.parametrize("ggml_type,N,K,start,room", [(18, 2052, 4352, 2, 64 << 20), (21, 2177, 4096, 0, 64 << 20), (22, 1100, 7936, 2, 0), (17, 8193, 1024, 0, 64 << 20)])
+def test_iq_prompt_decoded(gpu, M, ggml_type, N, K, start, room):
+    """Against float64 on the dequantised weight, bounds as above; nothing written beside the result or behind the workspace."""
+    vmx, torch = gpu
+    from tests.helpers import random_iq_blocks
+    from vllm_rust_amd._lib import check, lib
+    ts = vmx.iq_type_size(ggml_type)
+    raw = torch.from_numpy(np.ascontiguousarray(random_iq_blocks(np.random.default_rng(N + K), ts, N * K // 256))).reshape(-1)
+    held = torch.zeros(start + raw.numel(), dtype=torch.uint8, device="cuda")
+    held[start:] = raw.cuda()
+    x = torch.randn((M, K), device="cuda", generator=torch.Generator(device="cuda").manual_seed(M + N)).to(torch.bfloat16)
+    need = 4 * N * K + room
+    ws = torch.full((need + 64,), 7, dtype=torch.uint8, device="cuda")
+    guard = torch.full((M + 2, N), 7.0, device="cuda")
+    y = guard[1:M + 1]
+    check(lib.vmx_iq_gemm_f32(ggml_type, held.data_ptr() + start, x.data_ptr(), y.data_ptr(), M, N, K, ws.data_ptr(), need, None))
+    torch.cuda.synchronize()
+    w = vmx.iq_dequantize(ggml_type, raw.cuda(), N * K // 256).reshape(N, K).double()
+    bound = (264 + K // 256 + 8) * 2.0 ** -24 * (x.double().abs() @ w.abs().T)
+    assert bool(((y.double() - x.double() @ w.T).abs() <= bound).all())
+    assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all()) and bool((ws[need:] == 7).all())
+
+
+class _Seg(C.Structure):
+    _fields_ = [("w", C.c_void_p), ("ggml_type", C.c_int), ("n_out", C.c_int), ("y_off", C.c_int)]
+
+
+# three projections of three types as one product, none of whose widths is whole tiles; rows in one tile height and in two, in slices and in none
+@pytest.mark.parametrize("M", [33, 130, 300])
+@pytest.mark.parametrize("K,room", [(1280, 0), (4096, 64 << 20)])
+def test_iq_prompt_projections(gpu, M, K, room):
+    """Against float64 as above; the columns beside the projections' stay as they were."""
+    vmx, torch = gpu
+    from tests.helpers import random_iq_blocks
+    from vllm_rust_amd._lib import check, lib
+    types, widths = (18, 22, 21), (300, 129, 64)
+    raws = [torch.from_numpy(np.ascontiguousarray(random_iq_blocks(np.random.default_rng(t + K), vmx.iq_type_size(t), n * K // 256))).reshape(-1).cuda()
+            for t, n in zip(types, widths)]
+    x = torch.randn((M, K), device="cuda", generator=torch.Generator(device="cuda").manual_seed(M + K)).to(torch.float16)
+    N, off = sum(widths), [0, widths[0], widths[0] + widths[1]]
+    segs = (_Seg * 3)(*[_Seg(r.data_ptr(), t, n, o) for r, t, n, o in zip(raws, types, widths, off)])
+    y = torch.full((M, N + 3), 7.0, device="cuda")
+    part = torch.empty(max(room, 1), dtype=torch.uint8, device="cuda")
+    check(lib._Z17vmx_iq_prompt_f32PK10VmxMmvqSegiPKtPfiilS4_mP12ihipStream_t(segs, 3, C.c_void_p(x.data_ptr()), C.c_void_p(y.data_ptr()), M, K, C.c_int64(N + 3),
+                                                                              C.c_void_p(part.data_ptr()), C.c_size_t(room), None))
+    torch.cuda.synchronize()
+    w = torch.cat([vmx.iq_dequantize(t, r, n * K // 256).reshape(n, K).double() for r, t, n in zip(raws, types, widths)])
+    bound = (264 + K // 256 + 8) * 2.0 ** -24 * (x.double().abs() @ w.abs().T)
+    assert bool(((y[:, :N].double() - x.double() @ w.T).abs() <= bound).all())
+    assert bool((y[:, N:] == 7.0).all())
+
+
+# gate columns below, at and past the 64 that a tile takes; rows in every tile height
+@pytest.mark.parametrize("M", [17, 65, 129, 192, 256])
+@pytest.mark.parametrize("ggml_type,inter,K", [(18, 40, 256), (21, 64, 512), (22, 200, 1280), (17, 130, 768)])
+def test_iq_prompt_geglu(gpu, M, ggml_type, inter, K):
+    """act = bf16(bf16(gelu(gate)) * up), gate and up rounded to bf16, against float64 on the dequantised weights.  The f32 sums may fall on the
+    other side of a bf16 rounding: one step (2^-8 relative) of gate and of up, and one of each product behind."""
+    vmx, torch = gpu
+    from tests.helpers import random_iq_blocks
+    from vllm_rust_amd._lib import check, lib
+    raw = [torch.from_numpy(np.ascontiguousarray(random_iq_blocks(np.random.default_rng(s + K), vmx.iq_type_size(ggml_type), inter * K // 256))).reshape(-1).cuda()
+           for s in (1, 2)]
+    w = [vmx.iq_dequantize(ggml_type, r, inter * K // 256).reshape(inter, K).double() for r in raw]
+    scale = 1.0 / float((w[0] ** 2).mean().sqrt() * K ** 0.5)           # sums of order 1
+    x = (torch.randn((M, K), device="cuda", generator=torch.Generator(device="cuda").manual_seed(M + K)) * scale).to(torch.float16)
+    guard = torch.full((M + 2, inter), 7.0, dtype=torch.float16, device="cuda")
+    act = guard[1:M + 1]
+    gate, up = [_Seg(r.data_ptr(), ggml_type, inter, 0) for r in raw]
+    check(lib._Z19vmx_iq_prompt_gegluRK10VmxMmvqSegS1_PKtPtiiP12ihipStream_t(C.byref(gate), C.byref(up), C.c_void_p(x.data_ptr()), C.c_void_p(act.data_ptr()), M, K, None))
+    torch.cuda.synchronize()
+    gate, up = [(x.double() @ m.T).to(torch.bfloat16).double() for m in w]
+    cdf = 0.5 * (1 + torch.erf(gate / 2 ** 0.5))
+    slope = cdf + gate * torch.exp(-gate * gate / 2) / (2 * np.pi) ** 0.5
+    ref = gate * cdf * up
+    bound = 2.0 ** -8 * ((slope * gate * up).abs() + 3 * ref.abs()) + 2.0 ** -20
+    assert bool(((act.double() - ref).abs() <= bound).all())
+    assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all())
 
 
 # 256-column blocks; one k-block, odd numbers of them (17; 33 in slices) and groups wider than a

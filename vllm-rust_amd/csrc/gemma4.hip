@@ -464,7 +464,7 @@ bool int_form_ok(const IqLin &l, int rows) {
     return vmx_iq_int_form_ok(l.ggml_type) && !g_split_always && vmx_int_gemm_ok(rows, l.out_features, l.in_features);
 }
 
-// m->gemm_ws = the integer form of the projections' weights, one behind the other
+// m->gemm_ws = the integer form of the projections' weights, one behind the other (products too small for vmx_iq_prompt_ok, gate and up of two types)
 int int_weights(vmx_gemma4 *m, const IqLin *const *lins, int n, int total, int K, hipStream_t st) {
     for (int i = 0, row = 0; i < n; row += lins[i]->out_features, i++)
         if (int rc = vmx_iq_dequant_int(lins[i]->ggml_type, lins[i]->raw.p, m->gemm_ws.p, row, lins[i]->out_features, total, K, st)) return rc;
@@ -490,12 +490,15 @@ int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, 
         total += lins[i]->out_features;
     }
     if (merge && vmx_int_gemm_ok(rows, total, K)) {   // one product over the projections' rows, one behind the other
-        if (int rc = int_weights(m, lins, n, total, K, st)) return rc;
         const uint16_t *a16 = a;
         if (!a_is_f16) {
             if (int rc = vmx_bf16_rows_to_f16(a, (uint16_t *)m->a16.p, (int64_t)rows * K, st)) return rc;
             a16 = (const uint16_t *)m->a16.p;
         }
+        VmxMmvqSeg segs[3];
+        for (int i = 0; i < n; i++) segs[i] = VmxMmvqSeg{lins[i]->raw.p, lins[i]->ggml_type, lins[i]->out_features, offs[i]};
+        if (vmx_iq_prompt_ok(segs, n, rows, K)) return vmx_iq_prompt_f32(segs, n, a16, y, rows, K, ldy, (float *)m->gemm_part.p, m->gemm_part.bytes, st);
+        if (int rc = int_weights(m, lins, n, total, K, st)) return rc;
         return vmx_int_gemm_f32(a16, m->gemm_ws.p, y, rows, total, K, ldy, (float *)m->gemm_part.p, m->gemm_part.bytes, st);
     }
     VMX_REQUIRE(!a_is_f16, "gemma4: fp16 rows for a projection without an integer form");
@@ -536,8 +539,11 @@ bool gateup_prompt_ok(const G4Layer &L, int rows) {
 int g4_gateup_prompt(vmx_gemma4 *m, const G4Layer &L, const uint16_t *x, uint16_t *act, int rows, hipStream_t st) {
     const IqLin *gu[2] = {&L.lin[VMX_L_GATE], &L.lin[VMX_L_UP]};
     const int K = gu[0]->in_features, inter = gu[0]->out_features;
-    if (int rc = int_weights(m, gu, 2, 2 * inter, K, st)) return rc;
     if (int rc = vmx_bf16_rows_to_f16(x, (uint16_t *)m->a16.p, (int64_t)rows * K, st)) return rc;
+    const VmxMmvqSeg segs[2] = {{gu[0]->raw.p, gu[0]->ggml_type, inter, 0}, {gu[1]->raw.p, gu[1]->ggml_type, inter, inter}};
+    if (segs[0].ggml_type == segs[1].ggml_type && vmx_iq_prompt_ok(segs, 2, rows, K))
+        return vmx_iq_prompt_geglu(segs[0], segs[1], (const uint16_t *)m->a16.p, act, rows, K, st);
+    if (int rc = int_weights(m, gu, 2, 2 * inter, K, st)) return rc;
     return vmx_int_gemm_geglu((const uint16_t *)m->a16.p, m->gemm_ws.p, act, rows, inter, K, st);
 }
 

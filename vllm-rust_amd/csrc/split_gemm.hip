@@ -99,12 +99,6 @@ __global__ __launch_bounds__(256) void split_gemm_kernel(const uint16_t *__restr
         }
 }
 
-// bf16 -> fp16, saturating at the largest finite half (a bf16 value inside fp16's normal range converts exactly; smaller ones
-// lose bits that are below 2^-24 in absolute terms)
-__device__ __forceinline__ uint16_t bf16_value_to_f16(uint16_t v) {
-    return __builtin_bit_cast(uint16_t, (_Float16)fminf(fmaxf(vmx_bf16_to_f32(v), -65504.0f), 65504.0f));
-}
-
 // The one-pass form for weights that are (f32 scale per super-block) x (small integer), see iq_dequant_int_kernel:
 // C[m, n] = sum_sb Dt[sb][n] * ( sum_{k in sb} A16[m, k] * Q[n, k] ), A16 = the activations as fp16 (bf16 values convert exactly
 // inside fp16's range), Q fp16 integers: every product is exact, the 256 products of a super-block are added in f32 by the matrix
@@ -361,6 +355,15 @@ size_t vmx_int_gemm_part_bytes() { return (size_t)2 * vmx_num_cus() * 128 * 128 
 
 bool vmx_int_gemm_ok(int M, int N, int K) { return (int64_t)M * K * 2 < (int64_t)1 << 32 && (int64_t)N * K * 2 < (int64_t)1 << 32; }
 
+int vmx_int_slices(const float *part, float *y, int slices, int M, int N, int64_t ldy, hipStream_t st) {
+    const bool wide = N % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & 15) == 0;
+    const dim3 grid((unsigned)(((int64_t)M * N / (wide ? 4 : 1) + 255) / 256));
+    if (wide) hipLaunchKernelGGL(int_slices_kernel<4>, grid, dim3(256), 0, st, part, y, slices, M, N, ldy);
+    else hipLaunchKernelGGL(int_slices_kernel<1>, grid, dim3(256), 0, st, part, y, slices, M, N, ldy);
+    VMX_CHECK_LAUNCH("int_slices");
+    return VMX_OK;
+}
+
 // part: scratch for slices, as many as fit part_bytes; vmx_int_gemm_part_bytes() hold all that are wanted
 int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, float *part, size_t part_bytes, hipStream_t st) {
     const uint16_t *Q = (const uint16_t *)workspace;
@@ -373,12 +376,8 @@ int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M
     if (brief) launch_int_tile<IntSmall, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
     else if (int_rows(M, N) == 128) launch_int_tile<IntWide, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
     else launch_int_tile<IntMid, false>(a16, Q, Dt, to, nullptr, M, N, K, ld, slices, st);
-    if (slices > 1) {
-        const bool wide = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0;
-        const dim3 grid((unsigned)(((int64_t)M * N / (wide ? 4 : 1) + 255) / 256));
-        if (wide) hipLaunchKernelGGL(int_slices_kernel<4>, grid, dim3(256), 0, st, part, C, slices, M, N, (int64_t)ldc);
-        else hipLaunchKernelGGL(int_slices_kernel<1>, grid, dim3(256), 0, st, part, C, slices, M, N, (int64_t)ldc);
-    }
+    if (slices > 1)
+        if (int rc = vmx_int_slices(part, C, slices, M, N, ldc, st)) return rc;
     VMX_CHECK_LAUNCH("int_gemm");
     return VMX_OK;
 }
@@ -410,6 +409,12 @@ extern "C" int vmx_iq_gemm_f32(int ggml_type, const void *blocks, const uint16_t
                 vmx_iq_gemm_workspace(n_out, n_in));
     if (m == 0) return VMX_OK;
     hipStream_t st = vmx_stream(stream);
+    const VmxMmvqSeg seg = {blocks, ggml_type, n_out, 0};
+    const size_t rows = ((size_t)m * n_in * 2 + 255) & ~(size_t)255;
+    if (vmx_iq_prompt_ok(&seg, 1, m, n_in) && workspace_bytes >= rows) {   // decoded inside the product: the workspace holds the rows, then slice sums
+        if (int rc = vmx_bf16_rows_to_f16(x, (uint16_t *)workspace, (int64_t)m * n_in, st)) return rc;
+        return vmx_iq_prompt_f32(&seg, 1, (const uint16_t *)workspace, y, m, n_in, n_out, (float *)((char *)workspace + rows), workspace_bytes - rows, st);
+    }
     if (vmx_iq_int_form_ok(ggml_type) && workspace_bytes >= vmx_iq_gemm_int_workspace(m, n_out, n_in) && vmx_int_gemm_ok(m, n_out, n_in)) {
         // exact one-pass form: integer weights in fp16, one f32 scale per super-block; slice sums where the workspace has room for them
         uint16_t *a16 = (uint16_t *)((char *)workspace + vmx_iq_gemm_int_workspace(0, n_out, n_in));

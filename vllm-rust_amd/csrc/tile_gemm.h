@@ -24,6 +24,12 @@ typedef uint32_t tg_u32x4 __attribute__((ext_vector_type(4)));   // a native vec
 
 constexpr int TG_BK = 64;
 
+// bf16 -> fp16, saturating at the largest finite half (a bf16 value inside fp16's normal range converts exactly; smaller ones
+// lose bits that are below 2^-24 in absolute terms)
+__device__ __forceinline__ uint16_t bf16_value_to_f16(uint16_t v) {
+    return __builtin_bit_cast(uint16_t, (_Float16)fminf(fmaxf(vmx_bf16_to_f32(v), -65504.0f), 65504.0f));
+}
+
 template <bool F16>
 __device__ __forceinline__ tg_f32x16 tg_mfma(tg_u32x4 a, tg_u32x4 b, tg_f32x16 c) {
     if constexpr (F16)
