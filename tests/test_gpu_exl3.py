@@ -60,7 +60,9 @@ def test_zero_trellis_constant_and_hadamard(gpu):
 
 
 @pytest.mark.parametrize("M,K,N,bits,cb", [(2, 512, 128, 4, 0), (1, 4096, 1024, 4, 0), (16, 1024, 256, 3, 1), (5, 512, 384, 2, 2),
-                                           (1, 2048, 512, 6, 0), (20, 256, 128, 8, 1)])
+                                           (1, 2048, 512, 6, 0), (20, 256, 128, 8, 1),
+                                           # last slice of k with one chunk of four (16 and 32 k-tiles a slice), every codebook, a width that is not 4 bits
+                                           (1, 384, 192 * 2, 4, 0), (3, 640, 16384, 4, 0), (2, 640, 16384, 4, 1), (4, 384, 256, 4, 2), (2, 640, 16384, 3, 0)])
 def test_gemm_matches_oracle(gpu, M, K, N, bits, cb):
     from oracle import oracle as orc
     from vllm_rust_amd._lib import lib, check

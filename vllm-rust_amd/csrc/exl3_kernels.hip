@@ -141,40 +141,42 @@ __global__ __launch_bounds__(64) void exl3_out_had_kernel(const float *__restric
 // the <= 24-bit window pair of weights (t, t+1) is always inside the two consecutive slots {s, s+1} = stream words
 // {i, i-1 (cyclic)}: one two-dword LDS read and one funnel shift per pair, with per-lane slot/shift constants computed
 // once.  (The first version moved words between lanes with 16 wave permutes per k-step.)
-template <int CB> __device__ __forceinline__ uint32_t exl3_hash(uint32_t w) {  // w < 2^16
-    // 32-bit products are quarter rate on CDNA: w * C (mod 2^32) comes from two full-rate 24-bit multiplies,
-    // w * (C & 0xFFFFFF) [+ ADD] + ((w * (C >> 24)) << 24).  Written as instructions because the optimiser folds the
-    // expression back into one v_mul_lo_u32.
-    constexpr uint32_t C = CB == 0 ? 89226354u : (CB == 1 ? 0xCBAC1FEDu : 0x83DCD12Du);
-    constexpr uint32_t ADD = CB == 0 ? 64248484u : 0u;
-    uint32_t lo, hi, x;
-    if constexpr (ADD != 0) asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(lo) : "v"(w), "s"(C & 0xFFFFFFu), "v"(ADD));
-    else asm("v_mul_u32_u24 %0, %1, %2" : "=v"(lo) : "s"(C & 0xFFFFFFu), "v"(w));
-    asm("v_mul_u32_u24 %0, %1, %2" : "=v"(hi) : "s"(C >> 24), "v"(w));
-    asm("v_lshl_add_u32 %0, %1, 24, %2" : "=v"(x) : "v"(hi), "v"(lo));
-    return x;
-}
-
-// decoded weights of the windows w0, w1 as a packed fp16 pair (w0 low)
-template <int CB> __device__ __forceinline__ uint32_t exl3_decode_pair(uint32_t w0, uint32_t w1) {
+// Decoded weights of four windows, each the low 16 bits of w[i] (whatever lies above them is not looked at), as two packed fp16 pairs (even window low).
+// A 32-bit product is quarter rate on CDNA, so w * C + ADD mod 2^32 is w * (C & 0xFFFF) + ADD in 32 bits and then w * (C >> 16) added to the upper
+// half alone: two full-rate instructions that read half registers, so that a window needs no mask either (two 24-bit products took three and a mask).
+// half(lo16) + half(hi16) picks its operands by sub-dword addressing (SDWA); the second add of a pair writes the high half and keeps the low one.
+// Four instructions a weight.  One block, because an instruction that writes part of a register must not be followed at once by one that reads
+// it: four chains in turn keep them apart, where the compiler would put an idle instruction behind each.
+template <int CB> __device__ __forceinline__ uint2 exl3_decode4(const uint32_t (&w)[4]) {
     if constexpr (CB == 0 || CB == 1) {
-#ifdef VMX_EXL3_PERM_ADD
-        typedef __attribute__((ext_vector_type(2))) _Float16 h2;
-#endif
-        const uint32_t x0 = (exl3_hash<CB>(w0) & 0x8fff8fffu) ^ 0x3b603b60u, x1 = (exl3_hash<CB>(w1) & 0x8fff8fffu) ^ 0x3b603b60u;
-#ifdef VMX_EXL3_PERM_ADD
-        const uint32_t lo = __builtin_amdgcn_perm(x1, x0, 0x05040100u), hi = __builtin_amdgcn_perm(x1, x0, 0x07060302u);
-        return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, lo) + __builtin_bit_cast(h2, hi));
-#else
-        // half(lo16) + half(hi16) of each word with the operand halves picked by sub-dword addressing (SDWA): two instructions for the pair instead of
-        // two byte permutes and a packed add.  The second add writes the high half of d and keeps the low one.
-        uint32_t d;
-        asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1" : "=v"(d) : "v"(x0));
-        asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1" : "+v"(d) : "v"(x1));
+        constexpr uint32_t C = CB == 0 ? 89226354u : 0xCBAC1FEDu, ADD = CB == 0 ? 64248484u : 0u;
+        uint32_t x0, x1, x2, x3;
+        uint2 d;
+        asm("v_mad_u32_u16 %[x0], %[w0], %[cl], %[add]\n\t"
+            "v_mad_u32_u16 %[x1], %[w1], %[cl], %[add]\n\t"
+            "v_mad_u32_u16 %[x2], %[w2], %[cl], %[add]\n\t"
+            "v_mad_u32_u16 %[x3], %[w3], %[cl], %[add]\n\t"
+            "v_mad_u16 %[x0], %[w0], %[ch], %[x0] op_sel:[0,0,1,1]\n\t"
+            "v_mad_u16 %[x1], %[w1], %[ch], %[x1] op_sel:[0,0,1,1]\n\t"
+            "v_mad_u16 %[x2], %[w2], %[ch], %[x2] op_sel:[0,0,1,1]\n\t"
+            "v_mad_u16 %[x3], %[w3], %[ch], %[x3] op_sel:[0,0,1,1]\n\t"
+            "v_bitop3_b32 %[x0], %[x0], %[flip], %[keep] bitop3:0x6c\n\t"   // (x & keep) ^ flip
+            "v_bitop3_b32 %[x1], %[x1], %[flip], %[keep] bitop3:0x6c\n\t"
+            "v_bitop3_b32 %[x2], %[x2], %[flip], %[keep] bitop3:0x6c\n\t"
+            "v_bitop3_b32 %[x3], %[x3], %[flip], %[keep] bitop3:0x6c\n\t"
+            "v_add_f16_sdwa %[d0], %[x0], %[x0] dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+            "v_add_f16_sdwa %[d1], %[x2], %[x2] dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+            "v_add_f16_sdwa %[d0], %[x1], %[x1] dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+            "v_add_f16_sdwa %[d1], %[x3], %[x3] dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
+            : [x0] "=&v"(x0), [x1] "=&v"(x1), [x2] "=&v"(x2), [x3] "=&v"(x3), [d0] "=&v"(d.x), [d1] "=&v"(d.y)
+            : [w0] "v"(w[0]), [w1] "v"(w[1]), [w2] "v"(w[2]), [w3] "v"(w[3]), [cl] "s"(C & 0xFFFFu), [ch] "s"(C >> 16), [add] "v"(ADD),
+              [flip] "s"(0x3b603b60u), [keep] "v"(0x8fff8fffu));
         return d;
-#endif
     } else {
-        return (uint32_t)half_to_bits(exl3_decode<2>(w0)) | ((uint32_t)half_to_bits(exl3_decode<2>(w1)) << 16);
+        uint32_t h[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) h[i] = half_to_bits(exl3_decode<CB>(w[i] & 0xffffu));
+        return make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
     }
 }
 
@@ -362,6 +364,27 @@ __global__ __launch_bounds__(256) void exl3_gemm_kernel(Exl3Segs segs, const uin
     }
     const uint16_t *xrow = xs + min(n, M - 1) * XROW + 8 * g;
     vmx_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    // kt: first k-tile of the step inside the slice.  At 4 bits the four windows of a lane end in adjacent words, the last of them at a slot that is a multiple of
+    // 4: five words by one 16-byte and one 4-byte read at the same shift, every step at a constant distance from the lane's one address.
+    const uint32_t *lane_tile = tb + ((g >> 1) * CT + wave) * TS;
+    const uint32_t *lane_words = lane_tile + (W - 4 - 4 * (n & 7));
+    auto step = [&](int kt) {
+        uint32_t v[4];
+        if constexpr (BITS == 4) {
+            const uint4 e = *reinterpret_cast<const uint4 *>(lane_words + kt * (CT * TS));
+            const uint32_t words[5] = {lane_words[kt * (CT * TS) + 4], e.w, e.z, e.y, e.x};
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[q] = __builtin_amdgcn_alignbit(words[q], words[q + 1], sh[0]);
+        } else {
+            const uint32_t *tile = lane_tile + kt * (CT * TS);
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[q] = __builtin_amdgcn_alignbit(tile[slot[q] + 1], tile[slot[q]], sh[q]);
+        }
+        const uint2 lo = exl3_decode4<CB>({v[0] >> BITS, v[0], v[1] >> BITS, v[1]}), hi = exl3_decode4<CB>({v[2] >> BITS, v[2], v[3] >> BITS, v[3]});
+        const uint4 bw = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        const uint4 au = *reinterpret_cast<const uint4 *>(xrow + kt * 16);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, au), __builtin_bit_cast(f16x8_t, bw), acc, 0, 0, 0);
+    };
 #pragma unroll
     for (int c = 0; c < NCH; c++) {
 #pragma unroll
@@ -375,21 +398,9 @@ __global__ __launch_bounds__(256) void exl3_gemm_kernel(Exl3Segs segs, const uin
             }
         }
         __syncthreads();
-        for (int s = 0; s < KTC / 2; s++) {
-            const int kt = c * KTC + 2 * s;   // first k-tile of the step inside the slice
-            if (kt0 + kt < ktiles) {          // wave-uniform; K % 32 == 0, so a step is all in or all out
-                const uint32_t *tile = tb + ((kt + (g >> 1)) * CT + wave) * TS;
-                uint4 bw;
-                uint32_t *bwp = reinterpret_cast<uint32_t *>(&bw);
+        if (kt0 + c * KTC < ktiles) {   // wave-uniform; K % 128 == 0 and KTC <= 8: a chunk is all in or all out
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const uint32_t lo = tile[slot[q]], hi = tile[slot[q] + 1];
-                    const uint32_t v = __builtin_amdgcn_alignbit(hi, lo, sh[q]);
-                    bwp[q] = exl3_decode_pair<CB>((v >> BITS) & 0xffffu, v & 0xffffu);
-                }
-                const uint4 au = *reinterpret_cast<const uint4 *>(xrow + kt * 16);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, au), __builtin_bit_cast(f16x8_t, bw), acc, 0, 0, 0);
-            }
+            for (int s = 0; s < KTC / 2; s++) step(c * KTC + 2 * s);
         }
     }
 #pragma unroll
