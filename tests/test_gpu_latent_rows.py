@@ -89,3 +89,52 @@ def test_position_without_keys(gpu, R, RD, heads, parts):
     assert bool((out[[0, 2]] == 0).all())
     # the keys may be cut into other partitions: a weight's two bf16 halves are off by 2^-16, on either side
     assert float((out[[1, 3]] - alone).abs().max()) <= 2.0 ** -15 * float(cache.abs().max())
+
+
+# row tiles of a workgroup that share their keys (one sequence), that do not (decode steps, ends of prompts), with two head groups, few heads, a
+# window's lower edge inside a tile, tokens out of order, a padding token among them
+@pytest.mark.parametrize("contexts,new,heads,window,shuffled", [
+    ([270], 270, 20, 0, False), ([97, 66, 110], 110, 16, 33, True), ([33] * 259, 1, 16, 0, False), ([700], 600, 5, 100, True), ([257], 257, 16, 0, True),
+])
+def test_shared_keys(gpu, contexts, new, heads, window, shuffled):
+    """Launches of more row tiles than compute units, with a sink, against float64; the bound is the one above."""
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    R, RD, bs, scale = 512, 64, 16, 0.06
+    g = torch.Generator(device="cuda").manual_seed(sum(contexts) + heads)
+    n = len(contexts)
+    mb = (max(contexts) + bs - 1) // bs
+    bt = torch.randperm(n * mb, device="cuda", generator=g).to(torch.int32).view(n, mb)
+    cache = torch.randn((n * mb * bs, R + RD), device="cuda", generator=g).to(torch.bfloat16)
+    sid, pos = [], []
+    for b, c in enumerate(contexts):
+        k = min(new, c)
+        p = list(range(c - k, c))
+        if shuffled:
+            p = p[::-1]
+            p[1] = -1
+        sid += [b] * k
+        pos += p
+    T = len(pos)
+    qa = torch.randn((T, heads, R), device="cuda", generator=g).to(torch.bfloat16).float()
+    qr = torch.randn((T, heads, RD), device="cuda", generator=g).to(torch.bfloat16).float()
+    sink = torch.randn(heads, device="cuda", generator=g).to(torch.bfloat16)
+    ts, tp = (torch.tensor(v, device="cuda", dtype=torch.int32) for v in (sid, pos))
+    out = torch.full((T, heads, R), float("nan"), device="cuda")
+    assert lib.vmx_latent_attention_workspace_bytes(T, heads, R, window, mb, bs) == 0
+    check(lib.vmx_latent_attention(out.data_ptr(), qa.data_ptr(), qr.data_ptr(), cache.data_ptr(), 1, bt.data_ptr(), mb, ts.data_ptr(), tp.data_ptr(),
+                                   sink.data_ptr(), scale, window, T, heads, R, RD, bs, None, 0, None))
+    torch.cuda.synchronize()
+    for t in range(T):
+        lo = max(0, pos[t] - window + 1) if window else 0
+        j = torch.arange(lo, pos[t] + 1, device="cuda")
+        if not len(j):
+            assert bool((out[t] == 0).all())
+            continue
+        rows = cache[bt[sid[t]].long()[j // bs] * bs + j % bs].double()
+        q = torch.cat([qa[t], qr[t]], 1).double()
+        d = 576 * 2.0 ** -24 * scale * (q.abs() @ rows.abs().T).max()
+        logits = torch.cat([q @ rows.T * scale, sink.double()[:, None]], 1)
+        exact = torch.softmax(logits, 1)[:, :-1] @ rows[:, :R]
+        bound = (torch.expm1(4 * d) + 2.0 ** -15 + 1024 * 2.0 ** -24) * rows[:, :R].abs().max()
+        assert bool(((out[t].double() - exact).abs() <= bound).all()), (t, float((out[t].double() - exact).abs().max()), float(bound))

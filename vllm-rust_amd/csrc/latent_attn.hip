@@ -14,8 +14,10 @@
 // Scores, softmax, the weighted sum, norms and angles are f32.  Queries are packed: token t belongs to sequence seq_ids[t] at
 // position positions[t], so prompts of different lengths, prompt portions and single decode tokens are the same launch, and a
 // token's result depends only on its own query and the cache rows of its window.
+#include "tile_gemm.h"
 #include "vmx_kernels.h"
 #include <float.h>
+#include <limits.h>
 
 namespace {
 
@@ -240,14 +242,14 @@ typedef short la_s16x4 __attribute__((ext_vector_type(4)));
 typedef short la_s16x8 __attribute__((ext_vector_type(8)));
 
 // WHOLE > 0: rows of exactly 32 KSMAX values with 64 DTW latents (512 + 64).  Every size is then a constant, which leaves the registers for
-// requesting a tile's rows while the one before it is worked on, and with WHOLE = 2 for two workgroups per compute unit: 1500 tokens
-// of 16 heads 270 -> 178 us.  Two workgroups cap the registers at 256, and 52 more (212 bytes a lane of scratch memory) are spilled while the
+// requesting a tile's rows while the one before it is worked on, and with WHOLE = 2 (inside latent_attn_shared_kernel) for two workgroups per compute unit: 1500
+// tokens of 16 heads 270 -> 178 us.  Two workgroups cap the registers at 256, and 52 more (212 bytes a lane of scratch memory) are spilled while the
 // queries and rows are set up and read back there and behind the loop; the loop over key tiles itself touches no scratch.  A partitioned
 // launch (decode steps: one workgroup per compute unit, a tile or two each) is mostly setup, so it has WHOLE = 1 without the cap and without
 // spills: 16 rows of 1000 tokens 22.3 -> 17.9 us (WHOLE = 2: 29.7).  Other sizes (0) request a tile's rows when its turn comes.
 template <int KSMAX, int DTW, int WHOLE>
-__global__ __launch_bounds__(256, WHOLE == 2 ? 2 : 1) void latent_attn_mfma_kernel(const LatentAttnArgs a) {
-    extern __shared__ __align__(16) unsigned char la_smem[];
+__device__ __forceinline__ void latent_row_tile(const LatentAttnArgs &a, int tb, int hg, int part) {
+    extern __shared__ __align__(256) unsigned char la_smem[];
     const int R = WHOLE ? 64 * DTW : a.R, RW = WHOLE ? 32 * KSMAX : a.R + a.rd;
     constexpr int ROWE = 64 * DTW + LA_PAD;   // of the largest latent this form takes, so that offsets are constants
     uint16_t *KT = reinterpret_cast<uint16_t *>(la_smem);            // [LA_KT][ROWE]: the tile's latents, row-major
@@ -256,7 +258,6 @@ __global__ __launch_bounds__(256, WHOLE == 2 ? 2 : 1) void latent_attn_mfma_kern
     float *red_max = reinterpret_cast<float *>(Plo + 16 * LA_LD);     // [4][16]
     float *red_sum = red_max + 64;                                    // [4][16]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fl = lane & 15, fg = lane >> 4;
-    const int tb = blockIdx.x / a.NHG, hg = blockIdx.x % a.NHG, part = blockIdx.y;
     const int t0 = tb * a.TPT, t_end = min(t0 + a.TPT, a.T);
     const int ksteps = WHOLE ? KSMAX : (RW + 31) >> 5;
     const int dtiles = WHOLE ? 4 * DTW : (R + 15) >> 4, dt_per_wave = WHOLE ? DTW : (dtiles + 3) >> 2, dt0 = wave * dt_per_wave;
@@ -440,6 +441,186 @@ __global__ __launch_bounds__(256, WHOLE == 2 ? 2 : 1) void latent_attn_mfma_kern
     }
 }
 
+template <int KSMAX, int DTW, int WHOLE>
+__global__ __launch_bounds__(256, 1) void latent_attn_mfma_kernel(const LatentAttnArgs a) {
+    latent_row_tile<KSMAX, DTW, WHOLE>(a, blockIdx.x / a.NHG, blockIdx.x % a.NHG, blockIdx.y);
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------
+// Prompts, rows of 512 + 64: FOUR row tiles a workgroup, one a wave, over the same keys.  With one row tile a workgroup the trips of its cache rows to the L2
+// are what the time goes into (74 KB a 64-key tile for 16 rows of products); here a tile is fetched once for 64 rows:
+//   * 32 keys at a time lie whole (latent | rotated part) in LDS, two tiles deep, filled by LDS-DMA one tile ahead: no registers, one barrier a tile.  Rows are
+//     1152 bytes unpadded; 16-byte chunk c of row r sits at c ^ la_swizzle(r), so that neither the 16 rows that a score fragment reads at one chunk nor
+//     the eight that a transposing read takes 32 bytes of share a bank group;
+//   * S^T = K Q^T leaves a lane the scores of ONE row (fl) against keys 4 fg + r of both 16-key halves: maximum, weights and sum need no LDS, and
+//     the weights go straight into the second product O^T = C^T P^T, whose k slots are assigned to the keys a lane already holds;
+//   * the 128 accumulators are rescaled only on tiles where a row's maximum grew.  (Leaving it behind by up to 8 saves little and costs precision: the largest
+//     weight is then no longer 1, which its two bf16 halves hold exactly.)
+// us, 16 heads, one row tile a workgroup -> this: 600 + 500 + 400 tokens packed 177 -> 68, 1000 tokens 175 -> 86, 4000 tokens 1667 -> 499, 130 tokens 27 -> 19;
+// 32 heads, 500 + 400 tokens 185 -> 62; 3 heads, 700 + 300 tokens 68 -> 58; decode steps of 300 sequences 117 -> 110.  Error against 64 bits as before (1.2e-6).
+// The queries (72 registers) and the accumulators (128) leave two waves a SIMD.  Blocks are numbered from the last token backwards: later tokens have
+// more keys.  A group of row tiles over several sequences (a large decode step) has no keys to share: its tiles go the way above, one a workgroup,
+// the first by the group's own workgroup and the others by those behind the groups.
+__device__ __forceinline__ int la_swizzle(int r) { return ((((r >> 2) ^ (r >> 3)) & 1) << 2) | (r & 2) | ((r >> 3) & 1); }
+
+__device__ __forceinline__ void la_request_1k(uint32_t at, const char *from) {   // 64 lanes x 16 bytes to the 1 KiB of LDS from byte `at` on
+    at = __builtin_amdgcn_readfirstlane(at);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(at), "v"(from) : "m0", "memory");
+}
+
+constexpr int LS_KT = 32, LS_ROW = 1152, LS_TILE = LS_KT * LS_ROW, LS_REQ = LS_TILE / 4096;   // keys a tile; bytes of a row and a tile; requests a wave
+
+__global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const LatentAttnArgs a) {
+    extern __shared__ __align__(256) unsigned char la_smem[];
+    constexpr int R = 512, RD = 64, KS = (R + RD) / 32, DT = R / 16;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fl = lane & 15, fg = lane >> 4;
+    const int row_tiles = (a.T + a.TPT - 1) / a.TPT, groups = (row_tiles + 3) / 4, leaders = groups * a.NHG;
+    const bool leader = (int)blockIdx.x < leaders;
+    const int id = leader ? leaders - 1 - (int)blockIdx.x : (int)blockIdx.x - leaders;
+    const int hg = id % a.NHG, gi = id / a.NHG, group = leader ? gi : gi / 3, which = leader ? 0 : 1 + gi % 3;
+    const int t0 = group * 4 * a.TPT, n = min(4 * a.TPT, a.T - t0);   // at most 64 tokens
+    const int seq = a.seq_ids[t0];
+    if (!__all(a.seq_ids[t0 + min(lane, n - 1)] == seq)) {
+        if (4 * group + which < row_tiles) latent_row_tile<KS, R / 64, 2>(a, 4 * group + which, hg, 0);
+        return;
+    }
+    if (!leader) return;
+    const int32_t *bt = a.block_tables + (int64_t)seq * a.max_blocks;
+    int hi = a.positions[t0 + min(lane, n - 1)], lo = hi < 0 ? INT_MAX : a.window > 0 ? max(0, hi - a.window + 1) : 0;
+    for (int m = 1; m < 64; m <<= 1) hi = max(hi, __shfl_xor(hi, m)), lo = min(lo, __shfl_xor(lo, m));
+    hi = __builtin_amdgcn_readfirstlane(hi), lo = __builtin_amdgcn_readfirstlane(lo);
+    const int ntiles = hi < lo ? 0 : (hi - lo) / LS_KT + 1;
+    // the lane's row
+    const int tq = t0 + wave * a.TPT + fl / a.HPT, hq = hg * a.HPT + fl % a.HPT;
+    const bool act = fl < a.TPT * a.HPT && tq < a.T && hq < a.H;
+    const int rpos = act ? a.positions[tq] : -1, rlo = a.window > 0 ? max(0, rpos - a.window + 1) : 0;
+    const int64_t th = act ? (int64_t)tq * a.H + hq : 0;
+    tg_u32x4 qf[KS];
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+        const float *src = s < R / 32 ? a.q_abs + th * R + 32 * s + 8 * fg : a.q_rot + th * RD + 32 * s - R + 8 * fg;
+        const float4 f0 = *reinterpret_cast<const float4 *>(src), f1 = *reinterpret_cast<const float4 *>(src + 4);
+        const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+        qf[s] = __builtin_bit_cast(tg_u32x4, vmx_pack16x8<false>(f));
+    }
+    // this wave fetches keys 8 wave .. + 7 of a tile: piece q's lane takes the chunk that belongs at byte 16 (64 q + lane) of those eight rows
+    uint32_t piece[LS_REQ];   // byte in the source row | 4 x row << 16
+#pragma unroll
+    for (int q = 0; q < LS_REQ; q++) {
+        const int c = 64 * q + lane, r = c / (LS_ROW / 16), at = c % (LS_ROW / 16);
+        piece[q] = (uint32_t)((at ^ la_swizzle(8 * wave + r)) * 16) | (uint32_t)(4 * r) << 16;
+    }
+    // Key 8 wave + lane % 8 of a tile (keys past `hi` repeat its row, and their weights are 0) and its block's table entry, which is not looked at
+    // before the next tile's turn: a wait for it would be one for the rows requested before it
+    auto key_of = [&](int kt) { return min(lo + LS_KT * kt + 8 * wave + (lane & 7), hi); };
+    auto entry_of = [&](int kt) { return bt[key_of(kt) / a.block_size]; };
+    const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)la_smem;
+    auto request = [&](int kt, int entry, int stage) {
+        const int row = entry * a.block_size + key_of(kt) % a.block_size;
+#pragma unroll
+        for (int q = 0; q < LS_REQ; q++) {
+            uint32_t p = piece[q];
+            asm volatile("" : "+v"(p));   // or nine 64-bit sums are kept in scratch memory, and each read of one waits for all requests under way
+            const int from = __builtin_amdgcn_ds_bpermute((int)(p >> 16), row);
+            la_request_1k(lds + stage * LS_TILE + (wave * LS_REQ + q) * 1024, reinterpret_cast<const char *>(a.cache) + (uint64_t)(uint32_t)from * LS_ROW + (p & 0xFFFFu));
+        }
+    };
+    vmx_f32x4 acc[DT];
+#pragma unroll
+    for (int d = 0; d < DT; d++) acc[d] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_r = -FLT_MAX, l_r = 0.f;   // l_r: the lane's own keys
+    const uint32_t k_at = lds + fl * LS_ROW + ((fg ^ la_swizzle(fl)) << 4);
+    const int vr = 4 * fg + (fl >> 2);
+    const uint32_t v_at = lds + vr * LS_ROW + ((((fl >> 1) & 1) ^ la_swizzle(vr)) << 4) + 8 * (fl & 1);
+    int next_entry = 0;
+    if (ntiles > 0) {
+        request(0, entry_of(0), 0);
+        next_entry = entry_of(1);
+    }
+    for (int kt = 0; kt < ntiles; kt++) {
+        const int stage = kt & 1, kbase = lo + LS_KT * kt;
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(next_entry) : : "memory");
+        __builtin_amdgcn_s_barrier();   // this tile is whole, and nobody reads the one before it any more
+        asm volatile("" ::: "memory");
+        if (kt + 1 < ntiles) {
+            request(kt + 1, next_entry, stage ^ 1);
+            next_entry = entry_of(kt + 2);
+        }
+        const uint32_t k_even = k_at + stage * LS_TILE, k_odd = k_even ^ 64;
+        vmx_f32x4 sacc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        // fragments are read AHEAD products before their use; the compiler alone reads each where it is needed and waits for it
+        constexpr int AHEAD_K = 4, AHEAD_V = 3;
+        tg_u32x4 kf[AHEAD_K];
+        auto read_k = [&](int i) { return tg_lds_read((i & 2 ? k_odd : k_even) + (i >> 2) * 128 + (i & 1) * 16 * LS_ROW); };   // step i / 2, keys 16 (i % 2) ..
+#pragma unroll
+        for (int i = 0; i < AHEAD_K; i++) kf[i] = read_k(i);
+#pragma unroll
+        for (int i = 0; i < 2 * KS; i++) {
+            sacc[i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, kf[i % AHEAD_K]), __builtin_bit_cast(vmx_bf16x8, qf[i >> 1]), sacc[i & 1], 0, 0, 0);
+            if (i + AHEAD_K < 2 * KS) kf[i % AHEAD_K] = read_k(i + AHEAD_K);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        float p[8], top = -FLT_MAX;
+        bool ok[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int j = kbase + 16 * (e >> 2) + 4 * fg + (e & 3);
+            ok[e] = j <= rpos && j >= rlo;
+            p[e] = ok[e] ? sacc[e >> 2][e & 3] * a.scale : -FLT_MAX;
+            top = fmaxf(top, p[e]);
+        }
+        top = fmaxf(top, vmx_lane_xor_m(top, 16));
+        top = fmaxf(top, vmx_lane_xor_m(top, 32));
+        const bool moves = top > m_r;
+        if (__any(moves)) {
+            const float alpha = moves ? expf(m_r - top) : 1.f;
+            if (moves) m_r = top;
+            l_r *= alpha;
+#pragma unroll
+            for (int d = 0; d < DT; d++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[d][r] *= alpha;
+        }
+        float lo8[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            p[e] = ok[e] ? expf(p[e] - m_r) : 0.f;
+            l_r += p[e];
+        }
+        const vmx_bf16x8 ph = __builtin_bit_cast(vmx_bf16x8, vmx_pack16x8<false>(p));
+#pragma unroll
+        for (int e = 0; e < 8; e++) lo8[e] = p[e] - vmx_bf16_to_f32(vmx_f32_to_bf16(p[e]));
+        const vmx_bf16x8 pl = __builtin_bit_cast(vmx_bf16x8, vmx_pack16x8<false>(lo8));
+        const uint32_t v_stage = v_at + stage * LS_TILE;
+        typedef la_s16x4 __attribute__((address_space(3))) *lds_s16x4;
+        auto read_v = [&](int d, int half) {   // four keys of latent dimensions 16 d ..
+            return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(uintptr_t)((v_stage ^ (32 * (d & 3))) + (d >> 2) * 128 + half * 16 * LS_ROW));
+        };
+        la_s16x4 vf[AHEAD_V][2];
+#pragma unroll
+        for (int d = 0; d < AHEAD_V; d++) vf[d][0] = read_v(d, 0), vf[d][1] = read_v(d, 1);
+#pragma unroll
+        for (int d = 0; d < DT; d++) {
+            const la_s16x4 c0 = vf[d % AHEAD_V][0], c1 = vf[d % AHEAD_V][1];
+            const la_s16x8 cf = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
+            acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, cf), ph, acc[d], 0, 0, 0);
+            acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, cf), pl, acc[d], 0, 0, 0);
+            if (d + AHEAD_V < DT) vf[d % AHEAD_V][0] = read_v(d + AHEAD_V, 0), vf[d % AHEAD_V][1] = read_v(d + AHEAD_V, 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    l_r += vmx_lane_xor_m(l_r, 16);
+    l_r += vmx_lane_xor_m(l_r, 32);
+    if (!act) return;
+    const float sk = a.sink ? vmx_bf16_to_f32(a.sink[hq]) : -FLT_MAX;
+    const float M = fmaxf(m_r, sk), w = expf(m_r - M);
+    const float den = l_r * w + (a.sink ? expf(sk - M) : 0.f);
+    const float f = den > 0.f ? w / den : 0.f;
+#pragma unroll
+    for (int d = 0; d < DT; d++)   // latent dimensions 16 d + 4 fg ..
+        *reinterpret_cast<float4 *>(a.out + th * R + 16 * d + 4 * fg) = make_float4(acc[d][0] * f, acc[d][1] * f, acc[d][2] * f, acc[d][3] * f);
+}
+
 // out[t, h] = sum_p e^(m_p - M) O_p / (sum_p e^(m_p - M) l_p + e^(sink - M)), M = max(sink, max_p m_p); NP <= 64.
 // Wave 0 turns the partitions' (m, l) into one weight each (one round trip to memory), then every thread sums its dimensions.
 __global__ __launch_bounds__(256) void latent_attn_merge_kernel(float *__restrict__ out, const float *__restrict__ part_m,
@@ -558,12 +739,12 @@ extern "C" int vmx_latent_attention(float *out_latent, const float *q_abs, const
         const void *fn = small              ? (const void *)latent_attn_mfma_kernel<5, 2, 0>
                          : !whole           ? (const void *)latent_attn_mfma_kernel<18, 8, 0>
                          : a.NP > 1         ? (const void *)latent_attn_mfma_kernel<18, 8, 1>
-                                            : (const void *)latent_attn_mfma_kernel<18, 8, 2>;
+                                            : (const void *)latent_attn_shared_kernel;
         if (lds > 64 * 1024) VMX_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         if (small) hipLaunchKernelGGL((latent_attn_mfma_kernel<5, 2, 0>), grid, dim3(256), lds, st, a);
         else if (!whole) hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8, 0>), grid, dim3(256), lds, st, a);
         else if (a.NP > 1) hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8, 1>), grid, dim3(256), lds, st, a);
-        else hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8, 2>), grid, dim3(256), lds, st, a);
+        else hipLaunchKernelGGL(latent_attn_shared_kernel, dim3((unsigned)(((tokens + a.TPT - 1) / a.TPT + 3) / 4 * 4 * a.NHG)), dim3(256), lds, st, a);
         VMX_CHECK_LAUNCH("latent_attention (matrix cores)");
         if (a.NP > 1) {
             hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(tokens * heads), dim3(256), 0, st, out_latent, a.part_m, a.part_l, a.part_o, sink_bf16,
