@@ -52,6 +52,29 @@ def test_bf16_linear_tile_shapes(gpu, M, N, K, out):
     test_bf16_linear_tiles(gpu, M, N, K, out)
 
 
+# f32 rows (64 x 128 tiles in two stages): rows and columns one below, at and one above a tile, one to many stages
+@pytest.mark.parametrize("M,N,K", [(17, 1, 64), (63, 127, 128), (64, 128, 192), (65, 129, 64), (129, 130, 2048), (300, 1000, 320)])
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+def test_f32_row_linear_tiles(gpu, M, N, K, out):
+    """As test_bf16_linear_tiles, on the rows rounded to bf16 (which the kernel does): the same bounds."""
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    g = torch.Generator(device="cuda").manual_seed(M * 131 + N + K)
+    x = torch.randn((M, K), device="cuda", generator=g)
+    w = torch.randn((N, K), device="cuda", generator=g).to(torch.bfloat16)
+    guard = torch.full((M + 2, N), 7.0, device="cuda", dtype=torch.float32 if out == "f32" else torch.bfloat16)
+    y = guard[1:M + 1]
+    check(lib.vmx_linear_bf16w(y.data_ptr(), 0 if out == "f32" else 1, x.data_ptr(), 0, w.data_ptr(), M, N, K, 0, None))
+    torch.cuda.synchronize()
+    xr = x.to(torch.bfloat16).double()
+    ref = xr @ w.double().T
+    bound = (K + 8) * 2.0 ** -24 * (xr.abs() @ w.double().abs().T)
+    if out == "bf16":
+        bound = bound + 2.0 ** -8 * ref.abs()
+    assert bool(((y.double() - ref).abs() <= bound).all())
+    assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all())
+
+
 # rows around the 64- and 128-row tiles; columns around the 128-wide ones; K of one super-block, an odd number of them, and enough with
 # few tiles that the sums are cut into slices ((2048, 8192) gives the workspace room for them, (64, 256) does not)
 @pytest.mark.parametrize("M", [17, 64, 65, 129, 300])

@@ -362,21 +362,23 @@ int latent_attention(vmx_fofinex *m, Layer &L, const Step &s) {
         pq.kv_rank = R, pq.rot_dim = RD, pq.inv_freq = L.rot_steps.as<float>(), pq.rot_dims = lc.rot.dims, pq.rot_halves = 1, pq.rot_mul = L.rot_mul;
         if (int rc = vmx_latent_prepare_rows(&pq, s.positions, nullptr, nullptr, cdt, nullptr, T, s.st)) return rc;
     }
+    // The attention rounds its queries to bf16 and the product behind it its rows: where the attention takes them, both are stored as bf16
+    const int f32_lat = vmx_latent_attention_takes_bf16(cdt, R, RD) ? 0 : 1;
     if (D > 0) {    // qa_h = U_h^T q_h: per head, [T, D] x [D, R]
         VmxLinear a;
         a.A = m->q.p, a.a_f32 = 1, a.lda = NQ, a.a_bs = D + RD;
         a.W = L.uk_t.as<uint16_t>(), a.w_sn = D, a.w_sk = 1, a.w_bs = (int64_t)D * R;
-        a.C = m->qabs.p, a.c_f32 = 1, a.ldc = (int64_t)H * R, a.c_bs = R;
+        a.C = m->qabs.p, a.c_f32 = f32_lat, a.ldc = (int64_t)H * R, a.c_bs = R;
         a.M = T, a.N = R, a.K = D, a.batch = H, a.exact = f32;
         if (int rc = vmx_linear_launch(a, s.st)) return rc;
     } else {
         if (int rc = vmx_zero_f32(m->qabs.as<float>(), (int64_t)T * H * R, s.st)) return rc;
     }
-    if (int rc = vmx_latent_attention(m->olat.as<float>(), m->qabs.as<float>(), m->qrot.as<float>(), cache.p, cdt, s.block_tables, s.max_blocks, s.seq_ids,
+    if (int rc = vmx_latent_attention_launch(m->olat.p, m->qabs.p, !f32_lat, m->qrot.as<float>(), cache.p, cdt, s.block_tables, s.max_blocks, s.seq_ids,
                                       s.positions, nullptr, lc.scale, 0, T, H, R, RD, m->cfg.block_size, m->attn_ws.p, m->attn_ws.bytes, s.st))
         return rc;
     VmxLinear v;    // v_h = V_h o_h: per head, [T, R] x [V, R]^T
-    v.A = m->olat.p, v.a_f32 = 1, v.lda = (int64_t)H * R, v.a_bs = R;
+    v.A = m->olat.p, v.a_f32 = f32_lat, v.lda = (int64_t)H * R, v.a_bs = R;
     v.W = L.uv.as<uint16_t>(), v.w_sn = R, v.w_sk = 1, v.w_bs = (int64_t)V * R;
     v.C = m->attn.p, v.c_f32 = f32, v.ldc = (int64_t)H * V, v.c_bs = V;
     v.M = T, v.N = V, v.K = R, v.batch = H, v.exact = f32;

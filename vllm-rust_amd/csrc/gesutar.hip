@@ -316,23 +316,25 @@ extern "C" int vmx_gesutar_forward(vmx_gesutar *m, const int32_t *tokens, const 
                                            L.inv_freq.as<float>(), lc.rot_dims, positions, slots, L.cache.p, cdt, m->qrot.as<float>(), T, H, dim,
                                            rd, R, st))
             return rc;
+        // The attention rounds its queries to bf16 and the product behind it its rows: where the attention takes them, both are stored as bf16
+        const int f32_lat = vmx_latent_attention_takes_bf16(cdt, R, rd) ? 0 : 1;
         if (dim > 0) {   // qa_h = U_h^T q_h: per head, [T, dim] x [dim, R]
             VmxLinear a;
             a.A = m->fused.as<float>() + L.q_off, a.a_f32 = 1, a.lda = L.nf, a.a_bs = dim + rd;
             a.W = L.uk_t.as<uint16_t>(), a.w_sn = dim, a.w_sk = 1, a.w_bs = (int64_t)dim * R;
-            a.C = m->qabs.p, a.c_f32 = 1, a.ldc = (int64_t)H * R, a.c_bs = R;
+            a.C = m->qabs.p, a.c_f32 = f32_lat, a.ldc = (int64_t)H * R, a.c_bs = R;
             a.M = T, a.N = R, a.K = dim, a.batch = H, a.exact = f32;
             if (int rc = vmx_linear_launch(a, st)) return rc;
         } else {
             if (int rc = vmx_zero_f32(m->qabs.as<float>(), (int64_t)T * H * R, st)) return rc;
         }
-        if (int rc = vmx_latent_attention(m->olat.as<float>(), m->qabs.as<float>(), m->qrot.as<float>(), L.cache.p, cdt, block_tables,
+        if (int rc = vmx_latent_attention_launch(m->olat.p, m->qabs.p, !f32_lat, m->qrot.as<float>(), L.cache.p, cdt, block_tables,
                                           max_blocks_per_seq, seq_ids, positions, L.sink.as<uint16_t>(), lc.scale, lc.window, T, H, R, rd,
                                           c.block_size, m->attn_ws.p, m->attn_ws.bytes, st))
             return rc;
         {   // v_h = V_h o_h, times sigmoid(gate): per head, [T, R] x [vd, R]^T
             VmxLinear v;
-            v.A = m->olat.p, v.a_f32 = 1, v.lda = (int64_t)H * R, v.a_bs = R;
+            v.A = m->olat.p, v.a_f32 = f32_lat, v.lda = (int64_t)H * R, v.a_bs = R;
             v.W = L.uv.as<uint16_t>(), v.w_sn = R, v.w_sk = 1, v.w_bs = (int64_t)vd * R;
             v.C = m->attn.p, v.c_f32 = f32, v.ldc = (int64_t)H * vd, v.c_bs = vd;
             v.M = T, v.N = vd, v.K = R, v.batch = H, v.exact = f32;

@@ -342,21 +342,23 @@ int latent_attention(vmx_larolorn *m, Layer &L, const Layer &w, const Step &s) {
     if (RD > 0) p.q = fused + w.q_off, p.ldq = nf, p.heads = H, p.dim = D, p.q_rot = m->q.as<float>();
     p.kv_rank = R, p.rot_dim = RD, p.inv_freq = w.rot_steps.as<float>(), p.rot_dims = lc.rot.dims, p.rot_mul = w.rot_mul;
     if (int rc = vmx_latent_prepare_rows(&p, s.positions, s.slots, L.cache.p, cdt, nullptr, T, s.st)) return rc;
+    // The attention rounds its queries to bf16 and the product behind it its rows: where the attention takes them, both are stored as bf16
+    const int f32_lat = vmx_latent_attention_takes_bf16(cdt, R, RD) ? 0 : 1;
     if (D > 0) {    // qa_h = U_h^T q_h: per head, [T, D] x [D, R]
         VmxLinear a;
         a.A = fused + w.q_off, a.a_f32 = 1, a.lda = nf, a.a_bs = D + RD;
         a.W = w.uk_t.as<uint16_t>(), a.w_sn = D, a.w_sk = 1, a.w_bs = (int64_t)D * R;
-        a.C = m->qabs.p, a.c_f32 = 1, a.ldc = (int64_t)H * R, a.c_bs = R;
+        a.C = m->qabs.p, a.c_f32 = f32_lat, a.ldc = (int64_t)H * R, a.c_bs = R;
         a.M = T, a.N = R, a.K = D, a.batch = H, a.exact = f32;
         if (int rc = vmx_linear_launch(a, s.st)) return rc;
     } else {
         if (int rc = vmx_zero_f32(m->qabs.as<float>(), (int64_t)T * H * R, s.st)) return rc;
     }
-    if (int rc = vmx_latent_attention(m->olat.as<float>(), m->qabs.as<float>(), m->q.as<float>(), L.cache.p, cdt, s.block_tables, s.max_blocks, s.seq_ids,
-                                      s.positions, nullptr, lc.scale, lc.mask, T, H, R, RD, m->cfg.block_size, m->attn_ws.p, m->attn_ws.bytes, s.st))
+    if (int rc = vmx_latent_attention_launch(m->olat.p, m->qabs.p, !f32_lat, m->q.as<float>(), L.cache.p, cdt, s.block_tables, s.max_blocks, s.seq_ids, s.positions,
+                                             nullptr, lc.scale, lc.mask, T, H, R, RD, m->cfg.block_size, m->attn_ws.p, m->attn_ws.bytes, s.st))
         return rc;
     VmxLinear v;    // V_h o_h times the head's sigmoid: per head, [T, R] x [V, R]^T
-    v.A = m->olat.p, v.a_f32 = 1, v.lda = (int64_t)H * R, v.a_bs = R;
+    v.A = m->olat.p, v.a_f32 = f32_lat, v.lda = (int64_t)H * R, v.a_bs = R;
     v.W = w.uv.as<uint16_t>(), v.w_sn = R, v.w_sk = 1, v.w_bs = (int64_t)V * R;
     v.C = m->attn.p, v.c_f32 = f32, v.ldc = (int64_t)H * V, v.c_bs = V;
     v.M = T, v.N = V, v.K = R, v.batch = H, v.exact = f32;

@@ -224,15 +224,33 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(float *__restrict__ ou
 // sequence with the other rows masked.  blockIdx.y splits the key range into partitions for launches with few row tiles; their
 // (max, sum, O) triples are merged, with the sink, by latent_attn_merge_kernel.
 struct LatentAttnArgs {
-    float *out;
-    const float *q_abs, *q_rot;
+    void *out;
+    const void *q_abs;   // f32, or (io16) bf16 like out
+    const float *q_rot;
     const uint16_t *cache;
     const int32_t *block_tables, *seq_ids, *positions;
     const uint16_t *sink;
     float *part_m, *part_l, *part_o;   // [T][H][NP], [T][H][NP], [T][H][NP][R]
     float scale;
-    int max_blocks, window, T, H, R, rd, block_size, HPT, TPT, NHG, NP;
+    int max_blocks, window, T, H, R, rd, block_size, HPT, TPT, NHG, NP, io16;
 };
+
+// the eight query values from element `at` of the latent-space query on, rounded to bf16
+__device__ __forceinline__ uint4 la_query8(const LatentAttnArgs &a, int64_t at) {
+    if (a.io16) return *reinterpret_cast<const uint4 *>((const uint16_t *)a.q_abs + at);
+    const float4 f0 = *reinterpret_cast<const float4 *>((const float *)a.q_abs + at), f1 = *reinterpret_cast<const float4 *>((const float *)a.q_abs + at + 4);
+    const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+    return vmx_pack16x8<false>(f);
+}
+__device__ __forceinline__ uint4 la_query8(const float *rot) {
+    const float4 f0 = *reinterpret_cast<const float4 *>(rot), f1 = *reinterpret_cast<const float4 *>(rot + 4);
+    const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+    return vmx_pack16x8<false>(f);
+}
+__device__ __forceinline__ void la_store(void *out, int io16, int64_t at, float v) {
+    if (io16) ((uint16_t *)out)[at] = vmx_f32_to_bf16(v);
+    else ((float *)out)[at] = v;
+}
 
 constexpr int LA_KT = 64, LA_LD = LA_KT + 8;   // keys per tile; row stride of the P tiles
 constexpr int LA_PAD = 32;                    // the row-major latent tile pads its rows by 64 bytes: four consecutive rows, four bank groups
@@ -281,10 +299,8 @@ __device__ __forceinline__ void latent_row_tile(const LatentAttnArgs &a, int tb,
                 const int k = 32 * s + 8 * fg;
                 la_u32x4 v = {0, 0, 0, 0};
                 if (s < ksteps && act && k < RW) {
-                    const float *src = k < R ? a.q_abs + ((int64_t)tq * a.H + hq) * R + k : a.q_rot + ((int64_t)tq * a.H + hq) * a.rd + (k - R);
-                    const float4 f0 = *reinterpret_cast<const float4 *>(src), f1 = *reinterpret_cast<const float4 *>(src + 4);
-                    const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
-                    v = __builtin_bit_cast(la_u32x4, vmx_pack16x8<false>(f));
+                    const int64_t row = (int64_t)tq * a.H + hq;
+                    v = __builtin_bit_cast(la_u32x4, k < R ? la_query8(a, row * R + k) : la_query8(a.q_rot + row * a.rd + (k - R)));
                 }
                 qf[s] = v;
             }
@@ -422,7 +438,7 @@ __device__ __forceinline__ void latent_row_tile(const LatentAttnArgs &a, int tb,
 #pragma unroll
                 for (int d = 0; d < DTW; d++) {
                     const int dim = 16 * (dt0 + d) + fl;
-                    if (d < dt_per_wave && dim < R) a.out[th * R + dim] = acc[d][r] * f;
+                    if (d < dt_per_wave && dim < R) la_store(a.out, a.io16, th * R + dim, acc[d][r] * f);
                 }
             } else {
                 const int64_t tp = th * a.NP + part;
@@ -498,10 +514,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const Latent
     tg_u32x4 qf[KS];
 #pragma unroll
     for (int s = 0; s < KS; s++) {
-        const float *src = s < R / 32 ? a.q_abs + th * R + 32 * s + 8 * fg : a.q_rot + th * RD + 32 * s - R + 8 * fg;
-        const float4 f0 = *reinterpret_cast<const float4 *>(src), f1 = *reinterpret_cast<const float4 *>(src + 4);
-        const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
-        qf[s] = __builtin_bit_cast(tg_u32x4, vmx_pack16x8<false>(f));
+        qf[s] = __builtin_bit_cast(tg_u32x4, s < R / 32 ? la_query8(a, th * R + 32 * s + 8 * fg) : la_query8(a.q_rot + th * RD + 32 * s - R + 8 * fg));
     }
     // this wave fetches keys 8 wave .. + 7 of a tile: piece q's lane takes the chunk that belongs at byte 16 (64 q + lane) of those eight rows
     uint32_t piece[LS_REQ];   // byte in the source row | 4 x row << 16
@@ -617,13 +630,18 @@ __global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const Latent
     const float den = l_r * w + (a.sink ? expf(sk - M) : 0.f);
     const float f = den > 0.f ? w / den : 0.f;
 #pragma unroll
-    for (int d = 0; d < DT; d++)   // latent dimensions 16 d + 4 fg ..
-        *reinterpret_cast<float4 *>(a.out + th * R + 16 * d + 4 * fg) = make_float4(acc[d][0] * f, acc[d][1] * f, acc[d][2] * f, acc[d][3] * f);
+    for (int d = 0; d < DT; d++) {   // latent dimensions 16 d + 4 fg ..
+        const int64_t at = th * R + 16 * d + 4 * fg;
+        const float4 v = make_float4(acc[d][0] * f, acc[d][1] * f, acc[d][2] * f, acc[d][3] * f);
+        if (a.io16)
+            *reinterpret_cast<uint2 *>((uint16_t *)a.out + at) = make_uint2(vmx_f32_to_bf16(v.x) | (uint32_t)vmx_f32_to_bf16(v.y) << 16, vmx_f32_to_bf16(v.z) | (uint32_t)vmx_f32_to_bf16(v.w) << 16);
+        else *reinterpret_cast<float4 *>((float *)a.out + at) = v;
+    }
 }
 
 // out[t, h] = sum_p e^(m_p - M) O_p / (sum_p e^(m_p - M) l_p + e^(sink - M)), M = max(sink, max_p m_p); NP <= 64.
 // Wave 0 turns the partitions' (m, l) into one weight each (one round trip to memory), then every thread sums its dimensions.
-__global__ __launch_bounds__(256) void latent_attn_merge_kernel(float *__restrict__ out, const float *__restrict__ part_m,
+__global__ __launch_bounds__(256) void latent_attn_merge_kernel(void *__restrict__ out, int io16, const float *__restrict__ part_m,
                                                                  const float *__restrict__ part_l, const float *__restrict__ part_o,
                                                                  const uint16_t *__restrict__ sink, int H, int R, int NP) {
     __shared__ float wgt[64];
@@ -641,7 +659,7 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(float *__restric
     for (int d = threadIdx.x; d < R; d += 256) {
         float v = 0.f;
         for (int p = 0; p < NP; p++) v = fmaf(wgt[p], part_o[(th * NP + p) * R + d], v);
-        out[th * R + d] = v;
+        la_store(out, io16, th * R + d, v);
     }
 }
 
@@ -707,21 +725,27 @@ extern "C" size_t vmx_latent_attention_workspace_bytes(int tokens, int heads, in
     return np == 1 ? 0 : (size_t)tokens * heads * np * (kv_rank + 2) * sizeof(float);
 }
 
-extern "C" int vmx_latent_attention(float *out_latent, const float *q_abs, const float *q_rot, const void *cache, int cache_dtype,
-                                    const int32_t *block_tables, int max_blocks_per_seq, const int32_t *seq_ids, const int32_t *positions,
-                                    const uint16_t *sink_bf16, float scale, int window, int tokens, int heads, int kv_rank, int rot_dim,
-                                    int block_size, void *workspace, size_t workspace_bytes, void *stream) {
+// The matrix-core form: 16-byte chunks of a cache row must not straddle the latent / rotated boundary
+static bool latent_on_matrix_cores(int cache_dtype, int kv_rank, int rot_dim) {
+    return cache_dtype == VMX_BF16 && kv_rank % 8 == 0 && rot_dim % 8 == 0 && kv_rank + rot_dim <= 576;
+}
+
+bool vmx_latent_attention_takes_bf16(int cache_dtype, int kv_rank, int rot_dim) { return latent_on_matrix_cores(cache_dtype, kv_rank, rot_dim); }
+
+int vmx_latent_attention_launch(void *out_latent, const void *q_abs, int io_bf16, const float *q_rot, const void *cache, int cache_dtype,
+                                const int32_t *block_tables, int max_blocks_per_seq, const int32_t *seq_ids, const int32_t *positions,
+                                const uint16_t *sink_bf16, float scale, int window, int tokens, int heads, int kv_rank, int rot_dim, int block_size,
+                                void *workspace, size_t workspace_bytes, hipStream_t st) {
     VMX_REQUIRE(out_latent && q_abs && q_rot && cache && block_tables && seq_ids && positions, "latent_attention: null pointer");
     VMX_REQUIRE(cache_dtype == VMX_F32 || cache_dtype == VMX_BF16, "latent_attention: the cache holds f32 or bf16");
     VMX_REQUIRE(kv_rank >= 1 && kv_rank <= 512, "latent_attention: kv_rank (%d) must be in 1..512", kv_rank);
     VMX_REQUIRE(heads >= 1 && rot_dim >= 0 && block_size >= 1 && max_blocks_per_seq >= 1 && window >= 0, "latent_attention: bad sizes");
+    VMX_REQUIRE(!io_bf16 || latent_on_matrix_cores(cache_dtype, kv_rank, rot_dim), "latent_attention: bf16 queries need the matrix-core form");
     if (tokens <= 0) return VMX_OK;
-    hipStream_t st = vmx_stream(stream);
     const int RW = kv_rank + rot_dim;
-    // matrix-core form: bf16 cache, 16-byte chunks of a row must not straddle the latent / rotated boundary
-    if (cache_dtype == VMX_BF16 && kv_rank % 8 == 0 && rot_dim % 8 == 0 && RW <= 576) {
+    if (latent_on_matrix_cores(cache_dtype, kv_rank, rot_dim)) {
         LatentAttnArgs a;
-        a.out = out_latent, a.q_abs = q_abs, a.q_rot = q_rot, a.cache = (const uint16_t *)cache;
+        a.out = out_latent, a.q_abs = q_abs, a.io16 = io_bf16, a.q_rot = q_rot, a.cache = (const uint16_t *)cache;
         a.block_tables = block_tables, a.seq_ids = seq_ids, a.positions = positions, a.sink = sink_bf16;
         a.scale = scale, a.max_blocks = max_blocks_per_seq, a.window = window, a.T = tokens, a.H = heads, a.R = kv_rank, a.rd = rot_dim;
         a.block_size = block_size;
@@ -747,7 +771,7 @@ extern "C" int vmx_latent_attention(float *out_latent, const float *q_abs, const
         else hipLaunchKernelGGL(latent_attn_shared_kernel, dim3((unsigned)(((tokens + a.TPT - 1) / a.TPT + 3) / 4 * 4 * a.NHG)), dim3(256), lds, st, a);
         VMX_CHECK_LAUNCH("latent_attention (matrix cores)");
         if (a.NP > 1) {
-            hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(tokens * heads), dim3(256), 0, st, out_latent, a.part_m, a.part_l, a.part_o, sink_bf16,
+            hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(tokens * heads), dim3(256), 0, st, out_latent, io_bf16, a.part_m, a.part_l, a.part_o, sink_bf16,
                                heads, kv_rank, a.NP);
             VMX_CHECK_LAUNCH("latent_attention (merge)");
         }
@@ -756,11 +780,19 @@ extern "C" int vmx_latent_attention(float *out_latent, const float *q_abs, const
     const size_t lds = (size_t)(kv_rank + rot_dim + 256 + 256 + 8 + 4 * kv_rank) * 4;
     dim3 grid(heads, tokens);
     if (cache_dtype == VMX_F32)
-        hipLaunchKernelGGL(latent_attn_kernel<true>, grid, dim3(256), lds, st, out_latent, q_abs, q_rot, cache, block_tables,
+        hipLaunchKernelGGL(latent_attn_kernel<true>, grid, dim3(256), lds, st, (float *)out_latent, (const float *)q_abs, q_rot, cache, block_tables,
                            max_blocks_per_seq, seq_ids, positions, sink_bf16, scale, window, heads, kv_rank, rot_dim, block_size);
     else
-        hipLaunchKernelGGL(latent_attn_kernel<false>, grid, dim3(256), lds, st, out_latent, q_abs, q_rot, cache, block_tables,
+        hipLaunchKernelGGL(latent_attn_kernel<false>, grid, dim3(256), lds, st, (float *)out_latent, (const float *)q_abs, q_rot, cache, block_tables,
                            max_blocks_per_seq, seq_ids, positions, sink_bf16, scale, window, heads, kv_rank, rot_dim, block_size);
     VMX_CHECK_LAUNCH("latent_attention");
     return VMX_OK;
+}
+
+extern "C" int vmx_latent_attention(float *out_latent, const float *q_abs, const float *q_rot, const void *cache, int cache_dtype,
+                                    const int32_t *block_tables, int max_blocks_per_seq, const int32_t *seq_ids, const int32_t *positions,
+                                    const uint16_t *sink_bf16, float scale, int window, int tokens, int heads, int kv_rank, int rot_dim,
+                                    int block_size, void *workspace, size_t workspace_bytes, void *stream) {
+    return vmx_latent_attention_launch(out_latent, q_abs, 0, q_rot, cache, cache_dtype, block_tables, max_blocks_per_seq, seq_ids, positions, sink_bf16, scale,
+                                       window, tokens, heads, kv_rank, rot_dim, block_size, workspace, workspace_bytes, vmx_stream(stream));
 }

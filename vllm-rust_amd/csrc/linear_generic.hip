@@ -8,8 +8,8 @@
 //   * an optional bf16 bias per output column, then an epilogue: plain store, squared ReLU, tanh-form GELU, accumulate into an
 //     f32 residual stream, multiply by sigmoid(gate), or both of the last two (a gated residual update); a range of output columns
 //     may go through SiLU, so that one product serves readers that want it and readers that do not.
-// Kernels: `linear_tile_kernel` (prompts and 64-row expert blocks with bf16 rows in whole 64-deep stages), `linear_mfma_kernel` (the same
-// for f32 or unaligned rows; a staged 16-row form for shapes the streaming kernel does not take) and `linear_skinny_kernel` (up to 16
+// Kernels: `linear_tile_kernel` (prompts and 64-row expert blocks in whole 64-deep stages), `linear_mfma_kernel` (the same
+// for unaligned rows and other depths; a staged 16-row form for shapes the streaming kernel does not take) and `linear_skinny_kernel` (up to 16
 // rows: decode steps and 16-row expert blocks, weights streamed once) round the activations to bf16 and multiply on the matrix cores;
 // `linear_fma_kernel` multiplies in true f32 on the vector ALU (the 32-bit mode of a model), `linear_fewcols_f32_kernel` does the
 // same for a few output columns (router logits) with one kernel for every row count.  A row's result never depends on the other rows of the call: within a kernel a row is summed in
@@ -288,9 +288,10 @@ __device__ __forceinline__ void linear_tile_store(const VmxLinear &p, int z, int
 }
 
 // Prompt-sized bf16 products on the core of tile_gemm.h: plain, batched, gathered rows and 64-row expert blocks alike.  EP: the
-// finished sums are stored as they are, with a bias and a SiLU range, or through linear_store (whose run-time choices per element cost a
-// 1500 x 12288 output as much as half of its product: 159 against 101 us).
-enum { TILE_PLAIN, TILE_BIAS_SILU, TILE_ANY };
+// finished sums are stored as they are, with a bias and a SiLU range, times the sigmoids of a gate, or through linear_store (whose run-time choices per
+// element cost a 1500 x 12288 output as much as half of its product: 159 against 101 us; gates read there wait for the store before them, each in
+// turn: 16 products of 1500 x 128 x 512 33 -> 27 us).
+enum { TILE_PLAIN, TILE_BIAS_SILU, TILE_GATE, TILE_ANY };
 template <class S, int EP>
 __global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(const VmxLinear p, int row_tiles, int tiles) {
     extern __shared__ __align__(1024) uint16_t tg_lds[];
@@ -305,8 +306,9 @@ __global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(co
     uint32_t a_src[S::AQ], b_src[S::BQ];
 #pragma unroll
     for (int q = 0; q < S::AQ; q++) {
-        const int64_t r = linear_src_row(p, m0 + tg_src_row<S::AQ>(wave, lane, q));
-        a_src[q] = (uint32_t)((r < 0 ? 0 : r) * p.lda * 2) + tg_src_byte(lane);
+        const int row = S::A32 ? tg_src_row32<S::AQ>(wave, lane, q) : tg_src_row<S::AQ>(wave, lane, q);
+        const int64_t r = linear_src_row(p, m0 + row);
+        a_src[q] = (uint32_t)((r < 0 ? 0 : r) * p.lda * (S::A32 ? 4 : 2)) + (S::A32 ? tg_src_byte32(lane, row) : tg_src_byte(lane));
     }
 #pragma unroll
     for (int q = 0; q < S::BQ; q++)
@@ -316,7 +318,7 @@ __global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(co
     for (int i = 0; i < S::MI; i++)
 #pragma unroll
         for (int j = 0; j < S::NJ; j++) acc[i][j] = tg_f32x16{};
-    const TgCore<false, S> core{(const char *)((const uint16_t *)p.A + z * p.a_bs), (const char *)W, a_src, b_src, tg_lds_at(tg_lds), wave, lane};
+    const TgCore<false, S> core{(const char *)p.A + z * p.a_bs * (S::A32 ? 4 : 2), (const char *)W, a_src, b_src, tg_lds_at(tg_lds), wave, lane};
     tg_product(core, p.K, acc);
     const int wm = m0 + wave / S::WN * (S::MI * 32), wn = n0 + wave % S::WN * (S::NJ * 32), col = lane & 31;
     if constexpr (EP == TILE_ANY) {
@@ -347,6 +349,16 @@ __global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(co
                     acc[i][j][r] = v;
                 }
         }
+    }
+    if constexpr (EP == TILE_GATE) {
+#pragma unroll
+        for (int i = 0; i < S::MI; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float *gate = p.aux + (int64_t)min(wm + 32 * i + tg_acc_row(lane, r), p.M - 1) * p.ldaux + z * p.aux_bs;
+#pragma unroll
+                for (int j = 0; j < S::NJ; j++) acc[i][j][r] *= 1.0f / (1.0f + expf(-gate[(int64_t)min(wn + 32 * j + col, p.N - 1) * p.aux_sn]));
+            }
     }
     if (p.c_f32) linear_tile_store<S, float>(p, z, wm, wn, lane, acc);
     else linear_tile_store<S, uint16_t>(p, z, wm, wn, lane, acc);
@@ -499,10 +511,10 @@ __global__ __launch_bounds__(256) void linear_fewcols_f32_kernel(const VmxLinear
     if (tid < 16 && n0 + tid < p.N) linear_store(p, 0, m, n0 + tid, (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]));
 }
 
-// What linear_tile_kernel takes: bf16 rows in 16-byte chunks, whole 64-deep stages, operands (one batch) inside 32-bit byte offsets.
+// What linear_tile_kernel takes: rows in 16-byte chunks, whole 64-deep stages, operands (one batch) inside 32-bit byte offsets.
 bool tile_ok(const VmxLinear &p, bool direct) {
     const int64_t a_rows = p.row_ids ? (p.row_limit + p.row_div - 1) / p.row_div : p.M;
-    return direct && !p.a_f32 && p.K % TG_BK == 0 && a_rows * p.lda * 2 < (int64_t)1 << 32 && (int64_t)p.N * p.w_sn * 2 < (int64_t)1 << 32 &&
+    return direct && p.K % TG_BK == 0 && a_rows * p.lda * (p.a_f32 ? 4 : 2) < (int64_t)1 << 32 && (int64_t)p.N * p.w_sn * 2 < (int64_t)1 << 32 &&
            p.lda >= 0 && p.w_sn >= 0;
 }
 
@@ -516,8 +528,10 @@ int launch_tile_as(const VmxLinear &p, hipStream_t st) {
 
 template <class S>
 int launch_tile_shape(const VmxLinear &p, hipStream_t st) {
+    const bool plain = !p.bias && p.silu_end <= p.silu_begin;
+    if (p.epilogue == VMX_EP_MUL_SIGMOID && plain && p.out_scale == 1.0f) return launch_tile_as<S, TILE_GATE>(p, st);
     if (p.epilogue != VMX_EP_STORE || p.out_scale != 1.0f) return launch_tile_as<S, TILE_ANY>(p, st);
-    if (p.bias || p.silu_end > p.silu_begin) return launch_tile_as<S, TILE_BIAS_SILU>(p, st);
+    if (!plain) return launch_tile_as<S, TILE_BIAS_SILU>(p, st);
     return launch_tile_as<S, TILE_PLAIN>(p, st);
 }
 
@@ -528,6 +542,9 @@ typedef TgShape<2, 2, 2, 2, 2> Tile128two;   // 128 x 128, two
 typedef TgShape<2, 4, 2, 1, 4> Tile128;      // 128 x 128, one
 typedef TgShape<2, 2, 3, 2, 3> Tile192;      // 192 x 128, one
 typedef TgShape<4, 2, 2, 2, 3> Tile256;      // 256 x 128, one
+// f32 rows: 64 x 128, two a unit (64 x 64, 128 x 64, 128 x 128 one a unit: 16 products of 1500 x 512 x 128 in 30 / 31 / 27 us against 22).  us, linear_mfma_kernel
+// -> this: those products 53 -> 22; 17 x 64 x 512 12 -> 8, 64 x 256 x 2048 42 -> 21, 500 x 8192 x 128 19 -> 8, 1500 x 12288 x 2048 337 -> 160, 2000 x 2048 x 6144 304 -> 95.
+typedef TgShape<2, 2, 1, 2, 2, true> Tile64f;
 
 // Estimated ns of a launch.  It runs in rounds of one tile for every place; a 64-deep step of a full round takes `full`, one with at most a
 // workgroup for every second place `few` (shapes with two places a unit), and a last round is shorter, the emptier it is (least so where it is the
@@ -551,6 +568,7 @@ int64_t tile_ns(const VmxLinear &p, int full, int few) {
 // stage, results element by element) and now:  1500 x 12288 x 2048 107 -> 85, 1500 x 3664 x 2048 36 -> 28, 1500 x 2048 x 6144 72 -> 53, 500 x 12288 x
 // 2048 42 -> 33, 333 x 2048 x 6144 35 -> 25, 100 x 3664 x 2048 14.6 -> 11.2.  Expert blocks bring 64 rows each.
 int launch_tile(const VmxLinear &p, hipStream_t st) {
+    if (p.a_f32) return launch_tile_shape<Tile64f>(p, st);
     const int64_t t64 = tile_ns<Tile64>(p, 490, 280), t64w = tile_ns<Tile64w>(p, 700, 450);
     if (p.block_expert) return t64 <= t64w ? launch_tile_shape<Tile64>(p, st) : launch_tile_shape<Tile64w>(p, st);
     const int64_t two = tile_ns<Tile128two>(p, 1130, 800), t128 = tile_ns<Tile128>(p, 640, 0), t192 = tile_ns<Tile192>(p, 850, 0),

@@ -59,13 +59,16 @@ __device__ __forceinline__ void tg_request_1k(uint32_t at, const char *base, uin
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(at), "v"(off), "s"(base) : "m0", "memory");
 }
 
-// Shape of a workgroup: WM x WN waves, each MI x NJ accumulators; STAGES tiles of both operands in LDS.
-template <int WM_, int WN_, int MI_, int NJ_, int STAGES_>
+// Shape of a workgroup: WM x WN waves, each MI x NJ accumulators; STAGES tiles of both operands in LDS.  A32: the rows of A are f32, staged as they
+// are (256 bytes a row: the chunk c of row r at c ^ 2 (r & 7)) and rounded to bf16 as fragments.
+template <int WM_, int WN_, int MI_, int NJ_, int STAGES_, bool A32_ = false>
 struct TgShape {
     static constexpr int WM = WM_, WN = WN_, MI = MI_, NJ = NJ_, STAGES = STAGES_;
+    static constexpr bool A32 = A32_;
     static constexpr int BM = WM * MI * 32, BN = WN * NJ * 32, WAVES = WM * WN, THREADS = 64 * WAVES;
-    static constexpr int AQ = BM / (8 * WAVES), BQ = BN / (8 * WAVES);            // requests of eight rows a wave makes per operand and stage
-    static constexpr int STAGE = (BM + BN) * TG_BK, LDS = STAGES * STAGE * 2;     // elements, bytes
+    static constexpr int AR = A32 ? 2 * BM : BM;                                  // 128-byte pieces of A a stage
+    static constexpr int AQ = AR / (8 * WAVES), BQ = BN / (8 * WAVES);            // requests of eight pieces a wave makes per operand and stage
+    static constexpr int STAGE = (AR + BN) * TG_BK, LDS = STAGES * STAGE * 2;     // 16-bit elements, bytes
     static constexpr int PER_UNIT = 160 * 1024 / LDS, PER_SIMD = PER_UNIT * WAVES > 4 ? PER_UNIT * WAVES / 4 : 1;   // workgroups a compute unit, waves a SIMD
     static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0 && STAGES >= 2, "whole requests per wave");
 };
@@ -74,6 +77,10 @@ struct TgShape {
 template <int Q>
 __device__ __forceinline__ int tg_src_row(int wave, int lane, int q) { return (wave * Q + q) * 8 + (lane >> 3); }
 __device__ __forceinline__ uint32_t tg_src_byte(int lane) { return (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4); }
+// ... and of an f32 operand (four rows a request)
+template <int Q>
+__device__ __forceinline__ int tg_src_row32(int wave, int lane, int q) { return (wave * Q + q) * 4 + (lane >> 4); }
+__device__ __forceinline__ uint32_t tg_src_byte32(int lane, int row) { return (uint32_t)(((lane & 15) ^ (2 * (row & 7))) << 4); }
 
 // What the two products below share: where a lane's fragments lie, the requests of one 64 deep step, the products of one stage.
 template <bool F16, class S>
@@ -87,8 +94,8 @@ struct TgCore {
     // request q (of AQ + BQ) of this wave for step t
     __device__ __forceinline__ void request_one(int t, int stage, int q) const {
         const uint32_t to = lds + stage * (S::STAGE * 2);
-        if (q < S::AQ) tg_request_1k(to + (wave * S::AQ + q) * (8 * TG_BK * 2), A + (int64_t)t * (2 * TG_BK), a_src[q < S::AQ ? q : 0]);
-        else tg_request_1k(to + (S::BM + (wave * S::BQ + q - S::AQ) * 8) * (TG_BK * 2), B + (int64_t)t * (2 * TG_BK), b_src[q < S::AQ ? 0 : q - S::AQ]);
+        if (q < S::AQ) tg_request_1k(to + (wave * S::AQ + q) * (8 * TG_BK * 2), A + (int64_t)t * ((S::A32 ? 4 : 2) * TG_BK), a_src[q < S::AQ ? q : 0]);
+        else tg_request_1k(to + (S::AR + (wave * S::BQ + q - S::AQ) * 8) * (TG_BK * 2), B + (int64_t)t * (2 * TG_BK), b_src[q < S::AQ ? 0 : q - S::AQ]);
     }
     __device__ __forceinline__ void request(int t, int stage) const {
 #pragma unroll
@@ -99,9 +106,21 @@ struct TgCore {
         const int fr = lane & 31, first = (((lane >> 5) ^ (fr & 7)) << 4);
         const uint32_t from = lds + stage * (S::STAGE * 2);
         const uint32_t arow = from + ((wave / S::WN) * (S::MI * 32) + fr) * (TG_BK * 2) + first;
-        const uint32_t brow = from + (S::BM + (wave % S::WN) * (S::NJ * 32) + fr) * (TG_BK * 2) + first;
+        const uint32_t brow = from + (S::AR + (wave % S::WN) * (S::NJ * 32) + fr) * (TG_BK * 2) + first;
+        if constexpr (S::A32) {   // chunks 4 s + 2 (lane / 32) and the one behind it
+            const uint32_t at = from + ((wave / S::WN) * (S::MI * 32) + fr) * (TG_BK * 4) + (((lane >> 5) ^ (fr & 7)) << 5);
 #pragma unroll
-        for (int i = 0; i < S::MI; i++) af[i] = tg_lds_read((arow ^ (32 * s)) + i * (32 * TG_BK * 2));
+            for (int i = 0; i < S::MI; i++) {
+                const uint32_t chunk = (at ^ (64 * s)) + i * (32 * TG_BK * 4);
+                const tg_u32x4 lo = tg_lds_read(chunk), hi = tg_lds_read(chunk + 16);
+                const float f[8] = {__uint_as_float(lo[0]), __uint_as_float(lo[1]), __uint_as_float(lo[2]), __uint_as_float(lo[3]),
+                                    __uint_as_float(hi[0]), __uint_as_float(hi[1]), __uint_as_float(hi[2]), __uint_as_float(hi[3])};
+                af[i] = __builtin_bit_cast(tg_u32x4, vmx_pack16x8<false>(f));
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < S::MI; i++) af[i] = tg_lds_read((arow ^ (32 * s)) + i * (32 * TG_BK * 2));
+        }
 #pragma unroll
         for (int j = 0; j < S::NJ; j++) bf[j] = tg_lds_read((brow ^ (32 * s)) + j * (32 * TG_BK * 2));
     }

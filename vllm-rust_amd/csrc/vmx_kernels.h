@@ -232,6 +232,13 @@ int vmx_linear_launch(const VmxLinear &p, hipStream_t st);
 
 // latent_attn.hip: out[h][r][d] = in[h][d][r], the key up-projection turned for q_abs = U_h^T q_h
 int vmx_latent_transpose_heads(uint16_t *out, const uint16_t *in, int heads, int dim, int kv_rank, hipStream_t st);
+// vmx_latent_attention with latent-space queries and results both f32 or (io_bf16, where vmx_latent_attention_takes_bf16) both bf16: the kernel rounds its
+// queries to bf16 anyway, so a caller whose next product rounds its rows as well gets the same bits with half the traffic.
+bool vmx_latent_attention_takes_bf16(int cache_dtype, int kv_rank, int rot_dim);
+int vmx_latent_attention_launch(void *out_latent, const void *q_abs, int io_bf16, const float *q_rot, const void *cache, int cache_dtype,
+                                const int32_t *block_tables, int max_blocks_per_seq, const int32_t *seq_ids, const int32_t *positions,
+                                const uint16_t *sink_bf16, float scale, int window, int tokens, int heads, int kv_rank, int rot_dim, int block_size,
+                                void *workspace, size_t workspace_bytes, hipStream_t st);
 
 // packed_ops.hip: what the packed-step executors share
 // A device allocation owned by an executor (host-side handle).
