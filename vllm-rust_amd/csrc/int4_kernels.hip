@@ -1259,29 +1259,31 @@ __global__ __launch_bounds__(256) void int4_gemm_tiled_kernel(const uint4 *__res
 //     position c ^ (r & 15), so the rows that eight lanes read lie in different bank groups;
 //   * weights go straight to registers, one k-block ahead.  A lane of the instruction's B operand is column l & 31: tile (l >> 4) & 1 of a
 //     pair, and of that tile's unit the words of the k chunks 2 t + (l >> 5) -- every byte of the unit is still used by one wave once;
-//   * fragments of the next 16 deep step are read and unpacked under the products of the current one;
+//   * fragments of the next 16 deep step are read and unpacked under the products of the current one, all four of which share them;
 //   * weights are unpacked to 16 + nibble (the nibble in the upper mantissa bits of 16.0), not 128 + nibble: one shift more a step, and every
 //     f32 sum runs at a sixth of the size;
-//   * the zero-point term -(s (16 + zp)) * (row sum of the k-block) costs no vector-ALU work per output: wave w leaves the sums of rows 16 w ..
-//     (a 16 x 16 matrix product with ones) in LDS, and one k-block later one v_mfma_f32_32x32x8_bf16 per accumulator adds the term, both
-//     sides cut into bf16 parts that together hold all their bits (row sums three parts, factors two).  The parts are rounded to nearest, so
-//     the lower ones have either sign: the instruction cuts small products off towards zero beside a large accumulator, which with
-//     parts of one sign adds up (rms error of 12288-deep sums x 5).  rms error against float64 where the product is zero, 2048 x 4096 x
-//     12288, rows of mean 0 / 1 / 5 and deviation 1: 1.0e-6 / 1.4e-5 / 4.4e-5; with 128 + nibble 7.6e-6 / 1.0e-4 / 2.7e-4 (16 x 16
-//     accumulators and vector-ALU terms: 7.0e-6 / 9.6e-5 / 2.4e-4); all terms at the end of the slice 3.4e-5 / 2.6e-3 / 1.4e-2;
-//   * the scales of a finished pair of column tiles are applied under the other pair's products.
-// us against the form it replaced (64 x 64 per wave in 16 x 16 accumulators, every LDS read behind the next tile's arrival), rows x columns x
-// depth, packed weights in bf16 out: 2048 x 24576 x 4096 461 -> 424 (970 TFLOP/s), 333 x 24576 x 4096 121 -> 105, 100 x 24576 x 4096 58 -> 41,
-// 2048 x 4096 x 12288 224 -> 212.  N % 256 == 0.
-template <bool GLU, bool GROUPED = false>
+//   * the zero-point term -(16 + zp) * (row sum of the k-block) costs no vector-ALU work per output: wave w leaves the sums of rows 16 w ..
+//     (a 16 x 16 matrix product with ones) in LDS as three bf16 parts that together hold all their bits, and under the block's last products one
+//     v_mfma_f32_32x32x8_bf16 per accumulator adds the term to the block's unscaled sums.  The parts are rounded to nearest, so the lower ones have
+//     either sign: the instruction cuts small products off towards zero beside a large accumulator, which with parts of one sign adds up.  bf16 results that differ from the rounded exact ones: 0.8e-4 .. 2.3e-4 of all
+//     (4096 and 12288 deep, rows of mean 0, 1 and 5), 2.0e-4 .. 3.4e-4 with the term of two-part factors on the scaled result a block later;
+//   * the scales of a finished k-block are applied between the first products of the next one.
+// What is left: matrix cores busy 0.59 of the time at 1.94 GHz and the vector ALU (unpacking 128, scales 64 of 250 instructions a k-block) about as long; the two
+// waves of a SIMD hardly overlap them.  One wave a SIMD with 96 rows of accumulators 570 us where this takes 385 (an instruction every 4.5 clocks is
+// what one wave issues); clusters of four products behind the unpacking, with or without a raised priority, 1 % slower than one by one.
+// us against the form before (one pair of column tiles after the other, so that every fragment of x was read twice; everything waited for at
+// the block's head), rows x columns x depth, weights in HBM: 2048 x 24576 x 4096 419 -> 385 (1070 TFLOP/s), 2048 x 6144 x 4096 109 -> 102, 333 x 24576 x 4096 106 -> 100,
+// 8 experts of 64 rows x 28672 x 4096 230 -> 211, x 4096 x 14336 125 -> 106.  N % 256 == 0.
+template <bool GLU, bool GROUPED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void int4_gemm_prompt_kernel(
     const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ, const uint16_t *__restrict__ x, float *__restrict__ partial,
     uint16_t *__restrict__ act, int M, int N, int K, int group, int kb_per_split, int slice_rows, Int4GroupedArgs ga, int row_tiles,
     int splits, uint16_t *__restrict__ ybf, const uint16_t *__restrict__ bias) {
     // ybf (one split only): the finished bf16 output y = bf16(sum + bias) instead of f32 slices
-    __shared__ __align__(256) uint16_t xs[2][PF_BM * KB];
-    __shared__ int32_t prow_s[PF_BM];
-    __shared__ __align__(16) uint2 row_parts[2][PF_BM];   // row sums of a k-block as three bf16 parts (and a zero), by turns
+    constexpr int BM = PF_BM, STRIP = 8;
+    __shared__ __align__(256) uint16_t xs[2][BM * KB];
+    __shared__ int32_t prow_s[BM];
+    __shared__ __align__(16) uint2 row_parts[2][BM];   // row sums of a k-block as three bf16 parts (and a zero), by turns
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nl = lane & 15, ct = (lane >> 4) & 1, kh = lane >> 5;
     const int kblocks = K / KB, G = K / group;
@@ -1293,14 +1295,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         ks = (int)blockIdx.x / per_split, rt = rem >> 3, cb = rid / (8 * row_tiles) * 8 + (rem & 7);
         if (cb >= col_blocks) return;
     } else {
-        // strips of eight row tiles, column by column, dealt to the XCDs in contiguous runs: the 64 workgroups of an XCD are eight row
+        // strips of STRIP row tiles, column by column, dealt to the XCDs in contiguous runs: the workgroups of an XCD at a time are eight row
         // tiles by eight column blocks, whose operands it fetches once into its L2
         const int per_split = row_tiles * col_blocks, t = tg_tile(blockIdx.x, per_split * splits);
         if (t < 0) return;
-        const int in_split = t % per_split, strip = in_split / (8 * col_blocks), rem = in_split - strip * 8 * col_blocks, height = min(8, row_tiles - strip * 8);
-        ks = t / per_split, cb = rem / height, rt = strip * 8 + rem % height;
+        const int in_split = t % per_split, strip = in_split / (STRIP * col_blocks), rem = in_split - strip * STRIP * col_blocks, height = min(STRIP, row_tiles - strip * STRIP);
+        ks = t / per_split, cb = rem / height, rt = strip * STRIP + rem % height;
     }
-    const int row0 = rt * PF_BM;
+    const int row0 = rt * BM;
     const int nt0 = cb * 16 + wave * 4;   // this wave's four column tiles
     const int kb_begin = ks * kb_per_split, kb_end = min(kblocks, kb_begin + kb_per_split);
     if constexpr (GROUPED) {
@@ -1311,7 +1313,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (!packed) return;
         W = reinterpret_cast<const uint4 *>(packed);
         SZ = reinterpret_cast<const uint32_t *>(packed + sz_offset_bytes(K, N));
-        if (tid < PF_BM) {
+        if (tid < BM) {
             const int p = ga.sorted[row0 + tid];
             prow_s[tid] = p >= 0 && p < ga.numel ? p : -1;
         }
@@ -1335,25 +1337,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint32_t w_at = (uint32_t)(ct * kblocks * 64 + kh * 16 + nl);   // of unit (nt0 + 2 j, kb); chunk pair t is 32 further on
     const uint32_t sz_at = (uint32_t)(ct * G * 16 + nl);
 
-    tg_f32x16 fin[2][2];
+    tg_f32x16 fin[2][2], sum[2][2];   // the result; a k-block's sums, scaled into it under the next block's first products
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) fin[i][j] = tg_f32x16{};
-    tg_u32x4 w[2][2];        // [column pair j][chunk pair t]
-    uint32_t sz[2];
+        for (int j = 0; j < 2; j++) fin[i][j] = sum[i][j] = tg_f32x16{};
     const int gkb = group / KB;   // k-blocks that share a scale
     const uint32_t xs_at = tg_lds_at(xs);   // a multiple of 256
-    auto fetch_x = [&](int kb, int stage) {
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            tg_request_1k(xs_at + (stage * PF_BM + wave * 16 + q * 4) * (KB * 2), reinterpret_cast<const char *>(x) + (int64_t)kb * (KB * 2), xsrc[q]);
+    struct Weights {             // of one k-block
+        tg_u32x4 w[2][2];        // [column pair j][chunk pair t]
+        uint32_t sz[2];
     };
-    auto fetch_w = [&](int kb, int j) {   // three requests
+    auto fetch_x = [&](int kb, int stage, int q) {
+        tg_request_1k(xs_at + (stage * BM + wave * 16 + q * 4) * (KB * 2), reinterpret_cast<const char *>(x) + (int64_t)kb * (KB * 2), xsrc[q]);
+    };
+    auto fetch_w = [&](int kb, int j, Weights &d) {   // three requests
         const tg_u32x4 *unit = reinterpret_cast<const tg_u32x4 *>(W) + ((int64_t)(nt0 + 2 * j) * kblocks + kb) * 64;
-        w[j][0] = unit[w_at];
-        w[j][1] = unit[w_at + 32];
-        sz[j] = (SZ + ((int64_t)(nt0 + 2 * j) * G + (gkb == 1 ? kb : kb / gkb)) * 16)[sz_at];
+        d.w[j][0] = unit[w_at];
+        d.w[j][1] = unit[w_at + 32];
+        d.sz[j] = (SZ + ((int64_t)(nt0 + 2 * j) * G + kb / gkb) * 16)[sz_at];
     };
     // (w & nibbles) | base in one v_and_or_b32: one operand from a scalar, one from a vector register (an instruction takes no two literals)
     uint32_t base = 0x41804180u, nibbles = 0x00780078u;
@@ -1361,20 +1363,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
     const uint32_t a_first = xs_at + (lane & 31) * (KB * 2) + ((kh ^ nl) << 4);              // row l & 31 (and 32 further on), chunk kh
     const uint32_t r_first = xs_at + (wave * 16 + nl) * (KB * 2) + (((lane >> 4) ^ nl) << 4);   // row 16 wave + nl, chunk l / 16
-    // The zero-point term of pair j for the k-block whose row sums lie in row_parts[turn].  A lane of the instruction (K = 8) holds four k:
-    // three parts of its row's sum and a zero; of its column's factor the lanes of k 0 .. 3 the upper part and those of k 4 .. 7 the lower.
-    uint32_t zf[2] = {0u, 0u};   // the lane's part of the factor of pair j, in both halves
-    auto zero_factor = [&](int j) {
-        const float f = __uint_as_float(sz[j] << 16) * (112.f - __uint_as_float(sz[j] & 0xFFFF0000u));   // 8 bits x 5 bits
-        const uint32_t part = vmx_f32_to_bf16(kh ? f - vmx_rnd16<false>(f) : f);
-        zf[j] = part | (part << 16);
-    };
-    auto zero_term = [&](int j, int turn) {
-        const uint2 f = make_uint2(zf[j], zf[j] & 0xFFFFu);
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-            fin[i][j] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(i4_s16x4, row_parts[turn][i * 32 + (lane & 31)]),
-                                                                 __builtin_bit_cast(i4_s16x4, f), fin[i][j], 0, 0, 0);
+    // The zero-point term of a k-block, -(16 + zp) times the row sums in row_parts[turn], under its last products.  A lane of the instruction (K = 8) holds four k: those
+    // of k 0 .. 3 three parts of their row's sum (and a zero) and the factor of their column, 5 bits; the others' factors are zero.
+    float sc[2] = {0.f, 0.f};
+    auto zero_term = [&](int i, int j, uint32_t z, const uint2 &parts) {
+        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(i4_s16x4, parts), __builtin_bit_cast(i4_s16x4, make_uint2(z, z & 0xFFFFu)), sum[i][j], 0, 0, 0);
     };
     const bool odd_row = nl & 1, high_row = nl & 2;
     auto keep_row_sums = [&](const vmx_f32x4 &rs, int turn) {   // lane's row: 16 wave + 4 (lane / 16) + nl % 4; four lanes store the same
@@ -1384,96 +1377,108 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const uint32_t p1 = vmx_f32_to_bf16(v1);
         row_parts[turn][wave * 16 + 4 * (lane >> 4) + (nl & 3)] = make_uint2(p0 | (p1 << 16), vmx_f32_to_bf16(v1 - __uint_as_float(p1 << 16)));
     };
-    if (kb_begin < kb_end) {
-        if (tid < PF_BM) row_parts[1][tid] = make_uint2(0u, 0u);   // the first k-block finds nothing before it
-        fetch_x(kb_begin, 0);
-        fetch_w(kb_begin, 0);
-        fetch_w(kb_begin, 1);
-        // Requests run half a k-block ahead: the next tile and the next weights of pair 0 leave when pair 0 has been unpacked, the next
-        // weights of pair 1 when pair 1 has.  At the top everything but the latter (three requests) must have arrived.
-        tg_f32x16 acc0[2], acc1[2] = {tg_f32x16{}, tg_f32x16{}};   // a pair's sums of one k-block; pair 1's are scaled in the next block
-        float sc1 = 0.f;
-        for (int kb = kb_begin; kb < kb_end; kb++) {
-            const int stage = (kb - kb_begin) & 1, next = min(kb + 1, kb_end - 1);   // the last block requests itself again: the same counts everywhere
-            asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)" ::: "memory");
-            asm volatile("" : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(sz[0]));   // the compiler's own wait for pair 0 falls here, where it costs nothing
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            // chunk c of a row sits at position c ^ (row & 15), so the byte address of step s is that of step 0 with 32 s (64 s) flipped in
-            const uint32_t a_at = a_first + stage * (PF_BM * KB * 2), r_at = r_first + stage * (PF_BM * KB * 2);
-            tg_u32x4 au[2][2], bu[2];
-            auto read_a = [&](int s, tg_u32x4 (&d)[2]) {   // step s = 2 word + t: chunk 2 s + kh
+    auto scale = [&](int i, int j) {
 #pragma unroll
-                for (int i = 0; i < 2; i++) d[i] = tg_lds_read((a_at ^ (32 * s)) + i * (32 * KB * 2));
-            };
-            auto unpack = [&](int j, int s) {
-                const uint32_t v = w[j][s & 1][s / 2];
-                return tg_u32x4{((v << 3) & nibbles) | base, ((v >> 1) & nibbles) | base, ((v >> 5) & nibbles) | base, ((v >> 9) & nibbles) | base};
-            };
-            // elements [32 e / n, 32 (e + 1) / n) of pair j's finished sums of a k-block, times its scale, into the result
-            auto scale_part = [&](int j, float sc, const tg_f32x16 (&acc)[2], int e, int n) {
+        for (int r = 0; r < 16; r++) fin[i][j][r] = fmaf(sc[j], sum[i][j][r], fin[i][j][r]);
+        asm volatile("" : "+v"(fin[i][j]));   // here, not in one heap at the end
+    };
+    tg_u32x4 au[2], bu[2][2];   // fragments of x (read again as soon as the step is done with one) and of unpacked weights (of this step and the next)
+    auto read_a = [&](int stage, int s, int i) {   // step s = 2 word + t: chunk 2 s + kh, which lies at its position ^ (row & 15): 32 s flipped in
+        au[i] = tg_lds_read(((a_first + stage * (BM * KB * 2)) ^ (32 * s)) + i * (32 * KB * 2));
+    };
+    auto unpack = [&](const Weights &d, int j, int s) {
+        const uint32_t v = d.w[j][s & 1][s / 2];
+        return tg_u32x4{((v << 3) & nibbles) | base, ((v >> 1) & nibbles) | base, ((v >> 5) & nibbles) | base, ((v >> 9) & nibbles) | base};
+    };
+    // One k-block: eight steps, 16 deep, of four products (two row tiles x two pairs of column tiles), so that a fragment of x is read once for both pairs.
+    // Each step reads and unpacks what the next one multiplies, the last one for the next block: behind step 6 nobody reads this block's rows
+    // any more and the next block's rows and weights are waited for, and under step 7 the requests of the block after that go out, into the
+    // places of this one.
+    auto block = [&](int kb, int stage, Weights &now, Weights &after) {
+        const int next = min(kb + 2, kb_end - 1);   // the last blocks request the last one again
+        const uint32_t r_at = r_first + stage * (BM * KB * 2);
+        vmx_f32x4 rs = {0.f, 0.f, 0.f, 0.f};   // sums of rows 16 wave ..
+        float nsc[2];
+        uint32_t z[2];
+        uint2 parts[2];
 #pragma unroll
-                for (int r = 32 * e / n; r < 32 * (e + 1) / n; r++) fin[r >> 4][j][r & 15] = fmaf(sc, acc[r >> 4][r & 15], fin[r >> 4][j][r & 15]);
-                asm volatile("" : "+v"(fin[0][j]), "+v"(fin[1][j]));   // in this step, not in one heap at the end
-            };
-            read_a(0, au[0]);
-            bu[0] = unpack(0, 0);
-            vmx_f32x4 rs = {0.f, 0.f, 0.f, 0.f};   // sums of rows 16 wave ..
-            float sc0 = 0.f;
-            // One pair of column tiles after the other, 16 steps of two matrix products.  Every step also unpacks the next step's weights and
-            // scales a part of the pair before it (pair 1's of the previous k-block under pair 0, pair 0's under pair 1): about seven
-            // vector instructions behind each product, which is what fits under it.
+        for (int s = 0; s < 8; s++) {
+            const int at = s & 1;
 #pragma unroll
-            for (int u = 0; u < 16; u++) {
-                const int j = u >> 3, s = u & 7, at = u & 1;
-                // nothing moves over a step's start: pair 1 reads its fragments again instead of keeping sixteen of them in registers, and no
-                // unpacked weight waits longer than a step
-                asm volatile("" ::: "memory");
+            for (int p = 0; p < 4; p++) {
+                const int i = p >> 1, j = p & 1;
                 __builtin_amdgcn_sched_barrier(0);
-                if (u == 7) asm volatile("" : "+v"(w[1][0]), "+v"(w[1][1]), "+v"(sz[1]));   // pair 1 is waited for here: nothing else is under way
-                if (u < 15) {
-                    read_a((s + 1) & 7, au[at ^ 1]);
-                    bu[at ^ 1] = unpack((u + 1) >> 3, (s + 1) & 7);
+                if (s == 0) scale(i, j);   // of the block before this one
+                sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(vmx_bf16x8, au[i]), __builtin_bit_cast(vmx_bf16x8, bu[at][j]),
+                                                                    s == 0 ? tg_f32x16{} : sum[i][j], 0, 0, 0);
+                if (j == 1) {
+                    if (s < 7) read_a(stage, s + 1, i);
+                    else read_a(stage ^ 1, 0, i);
+                } else {
+                    bu[at ^ 1][i] = s < 7 ? unpack(now, i, s + 1) : unpack(after, i, 0);
                 }
-                if (j == 0 && (s & 1)) {   // chunks 4 (s / 2) + lane / 16: 32 of the block's k
-                    const tg_u32x4 aw = tg_lds_read(r_at ^ (64 * (s / 2)));
+                if (p == 1 && s < 4) {   // chunks 4 s + lane / 16: 32 of the block's k
+                    const tg_u32x4 aw = tg_lds_read(r_at ^ (64 * s));
                     rs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, aw), __builtin_bit_cast(vmx_bf16x8, ones), rs, 0, 0, 0);
                 }
-                if (u == 2) zero_term(0, stage ^ 1);    // of the k-block before this one; nobody else writes these results now
-                if (u == 10) zero_term(1, stage ^ 1);
-                if (u == 9) keep_row_sums(rs, stage);
-                if (u == 7) {
-                    sc0 = __uint_as_float(sz[0] << 16);
-                    zero_factor(0);
-                    fetch_x(next, stage ^ 1);
-                    fetch_w(next, 0);
+                if (s == 5 && p == 2) keep_row_sums(rs, stage);
+                if (s == 6 && p < 2) {
+                    nsc[j] = __uint_as_float(now.sz[j] << 16);
+                    const uint32_t f = vmx_f32_to_bf16(kh ? 0.f : 112.f - __uint_as_float(now.sz[j] & 0xFFFF0000u));
+                    z[j] = f | (f << 16);
                 }
-                tg_f32x16(&acc)[2] = j ? acc1 : acc0;
-#pragma unroll
-                for (int i = 0; i < 2; i++)
-                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(vmx_bf16x8, au[at][i]), __builtin_bit_cast(vmx_bf16x8, bu[at]),
-                                                                     s == 0 ? tg_f32x16{} : acc[i], 0, 0, 0);
-                if (j == 0) scale_part(1, sc1, acc1, s, 8);
-                else if (s > 0) scale_part(0, sc0, acc0, s - 1, 7);
-                if (u == 15) {
-                    sc1 = __uint_as_float(sz[1] << 16);
-                    zero_factor(1);
-                    fetch_w(next, 1);
+                if (s == 7) {
+                    if (p == 0) parts[0] = row_parts[stage][lane & 31], parts[1] = row_parts[stage][32 + (lane & 31)];
+                    if (p > 1) zero_term(0, p - 2, z[p - 2], parts[0]);
+                    fetch_x(next, stage, p);
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);
+            if (s == 6) {   // the fragments of step 7 are in registers
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                asm volatile("" : "+v"(after.w[0][0]), "+v"(after.w[0][1]), "+v"(after.w[1][0]), "+v"(after.w[1][1]), "+v"(after.sz[0]), "+v"(after.sz[1]));
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+            }
         }
+        zero_term(1, 0, z[0], parts[1]);
+        zero_term(1, 1, z[1], parts[1]);
+        fetch_w(next, 0, now);
+        fetch_w(next, 1, now);
+        sc[0] = nsc[0], sc[1] = nsc[1];
+    };
+    if (kb_begin < kb_end) {
+        Weights even, odd;
+        const int second = min(kb_begin + 1, kb_end - 1);
+#pragma unroll
+        for (int q = 0; q < 4; q++) fetch_x(kb_begin, 0, q), fetch_x(second, 1, q);
+        fetch_w(kb_begin, 0, even);
+        fetch_w(kb_begin, 1, even);
+        fetch_w(second, 0, odd);
+        fetch_w(second, 1, odd);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        asm volatile("" : "+v"(even.w[0][0]), "+v"(even.w[0][1]), "+v"(even.w[1][0]), "+v"(even.w[1][1]), "+v"(even.sz[0]), "+v"(even.sz[1]));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read_a(0, 0, 0);
+        read_a(0, 0, 1);
+        bu[0][0] = unpack(even, 0, 0);
+        bu[0][1] = unpack(even, 1, 0);
+        int kb = kb_begin;
+        for (; kb + 1 < kb_end; kb += 2) {
+            block(kb, 0, even, odd);
+            block(kb + 1, 1, odd, even);
+        }
+        if (kb < kb_end) block(kb, 0, even, odd);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) fin[i][1][r] = fmaf(sc1, acc1[i][r], fin[i][1][r]);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        zero_term(0, (kb_end - 1 - kb_begin) & 1);
-        zero_term(1, (kb_end - 1 - kb_begin) & 1);
+            for (int j = 0; j < 2; j++) scale(i, j);
     }
     // Outputs lie at a uniform row's start plus the lane's 32-bit offset (row 4 kh of an eight-row group, its column): no address
     // arithmetic per element.  Row of element (i, r): 32 i + 8 (r / 4) + 4 kh + r % 4.
-    const bool whole = !GROUPED && row0 + PF_BM <= M;
+    const bool whole = !GROUPED && row0 + BM <= M;
     auto row_ok = [&](int i, int r) {   // GROUPED: the pair the row belongs to (-1: padding), else 0 or -1
         const int lr = i * 32 + tg_acc_row(lane, r);
         if constexpr (GROUPED) return prow_s[lr];
