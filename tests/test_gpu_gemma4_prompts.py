@@ -91,6 +91,34 @@ def test_prompt_rows(gpu, rows, types):
         model.close()
 
 
+# 256- and 512-wide heads (attention results as fp16 rows) and projections of more than 8 M weights, whose slices of q|k|v, o and down the launches behind them
+# add; IQ4_XS o (fp16 rows would have no reader) and k (no merged q|k|v) among them
+@pytest.mark.parametrize("rows,types", [(65, {}), (200, {}), (65, {3: 23}), (65, {1: 23})])
+def test_prompt_rows_wide_heads(gpu, rows, types):
+    """As test_prompt_rows, the same bound."""
+    vmx, torch = gpu
+    from oracle import oracle as orc
+    from tests.model_oracle import OracleGemma4
+    from vllm_rust_amd.gemma4 import GEMMA4_12B_IQ3_MIX, Gemma4Spec
+    spec = Gemma4Spec(2048, 2, 16, 4096, 512, head_dim_sliding=256, head_dim_full=512, kv_heads_sliding=2, kv_heads_full=1, sliding_window=24,
+                      full_every=2, max_position=512, kv_cache_dtype=0, num_blocks=24, max_batch=1, max_seq_len=320, max_prefill_tokens=300)
+    model, ck = _model(spec, {**GEMMA4_12B_IQ3_MIX, **types})
+    try:
+        ref = OracleGemma4(spec, ck, model.cos_sin_sliding, model.cos_sin_full)
+        bs = spec.block_size
+        bt = np.random.default_rng(2).permutation(spec.num_blocks)[:20].astype(np.int32)[None]
+        prompt = np.random.default_rng(1).integers(0, spec.vocab_size, rows).astype(np.int32)
+        model.prefill(torch.from_numpy(prompt).cuda(), 0, torch.from_numpy(bt).cuda()[0])
+        torch.cuda.synchronize()
+        got = model.debug_read(0, (rows, spec.hidden_size)).double().cpu().numpy()
+        pos = np.arange(rows, dtype=np.int32)
+        _, h, _ = ref.decode(prompt, pos, (bt[0, pos // bs] * bs + pos % bs).astype(np.int32), np.repeat(bt, rows, axis=0), pos + 1)
+        exp = orc.bf16_to_f32(h).astype(np.float64)
+        assert (np.linalg.norm(got - exp, axis=1) <= 2e-2 * np.linalg.norm(exp, axis=1)).all()
+    finally:
+        model.close()
+
+
 def _launches(torch, types):
     """Kernels of one prompt pass, counted in a captured graph."""
     from vllm_rust_amd._lib import check, lib

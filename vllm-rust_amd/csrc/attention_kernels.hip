@@ -11,6 +11,7 @@
 // on the matrix cores over 16-token tiles, PV on the vector ALU with one V row per wave access
 // (details at the kernel).  At most 64 partitions per sequence; a second kernel (or the consumer)
 // merges them.
+#include "tile_gemm.h"
 #include "vmx_kernels.h"
 #include <float.h>
 #include <mutex>
@@ -1116,7 +1117,8 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(uint16_t *__restrict_
                                                             const void *__restrict__ k_cache, const void *__restrict__ v_cache,
                                                             const int32_t *__restrict__ block_table, int q_len, int offset, float scale,
                                                             int num_heads, int num_kv_heads, int block_size, int window,
-                                                            const float *__restrict__ k_scale_ptr, const float *__restrict__ v_scale_ptr) {
+                                                            const float *__restrict__ k_scale_ptr, const float *__restrict__ v_scale_ptr,
+                                                            int out_f16) {   // out_f16: results rounded to bf16 go out as fp16
     constexpr int HPW = QPK < 4 ? QPK : 4;   // query heads per workgroup
     constexpr int TT = 4 / HPW;              // 16-token query tiles per workgroup
     constexpr int KSTEPS = HD / 32, DT = HD / 16;
@@ -1258,23 +1260,27 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(uint16_t *__restrict_
         uint16_t *o = out + ((int64_t)qi * num_heads + head) * HD;
 #pragma unroll
         for (int d = 0; d < DT; d++) {   // acc[d][i] = O[query row n][dim 16 d + 4 g + i]
-            const uint32_t w0 = (uint32_t)vmx_st16<FP8 == 3>(acc[d][0] * inv) | ((uint32_t)vmx_st16<FP8 == 3>(acc[d][1] * inv) << 16);
-            const uint32_t w1 = (uint32_t)vmx_st16<FP8 == 3>(acc[d][2] * inv) | ((uint32_t)vmx_st16<FP8 == 3>(acc[d][3] * inv) << 16);
-            *reinterpret_cast<uint2 *>(o + 16 * d + 4 * g) = make_uint2(w0, w1);
+            uint16_t v[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                v[i] = vmx_st16<FP8 == 3>(acc[d][i] * inv);
+                if (FP8 != 3 && out_f16) v[i] = bf16_value_to_f16(v[i]);
+            }
+            *reinterpret_cast<uint2 *>(o + 16 * d + 4 * g) = make_uint2((uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16));
         }
     }
 }
 
 template <int HD, int QPK, int FP8>
 int launch_prefill(hipStream_t st, uint16_t *out, const uint16_t *q, const void *kc, const void *vc, const int32_t *bt, int q_len, int offset,
-                   float scale, int H, int KVH, int bs, int window, const float *ks, const float *vs) {
+                   float scale, int H, int KVH, int bs, int window, const float *ks, const float *vs, int out_f16) {
     constexpr int HPW = QPK < 4 ? QPK : 4, TT = 4 / HPW;
     const dim3 grid((q_len + 16 * TT - 1) / (16 * TT), KVH * (QPK / HPW));
     constexpr size_t lds = 2 * (16 * (HD + 8) + HD * 20) * 2;
     if (lds > 64 * 1024)
         VMX_CHECK_HIP(hipFuncSetAttribute((const void *)prefill_attn_kernel<HD, QPK, FP8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL((prefill_attn_kernel<HD, QPK, FP8>), grid, dim3(256), lds, st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window,
-                       ks, vs);
+                       ks, vs, out_f16);
     VMX_CHECK_LAUNCH("prefill_attention");
     return VMX_OK;
 }
@@ -1283,7 +1289,7 @@ int launch_prefill(hipStream_t st, uint16_t *out, const uint16_t *q, const void 
 static int prefill_attention_impl(uint16_t *out, const uint16_t *q, const void *k_cache, const void *v_cache,
                                   const int32_t *block_table, int q_len, int seqlen_offset, float scale, int num_heads,
                                   int num_kv_heads, int head_dim, int block_size, int window, int kv_dtype, const float *k_scale,
-                                  const float *v_scale, void *stream, bool f16) {
+                                  const float *v_scale, void *stream, bool f16, int out_f16 = 0) {
     VMX_REQUIRE(out && q && k_cache && v_cache && block_table, "prefill_attention: null pointer");
     VMX_REQUIRE(q_len >= 0 && seqlen_offset >= 0, "prefill_attention: q_len %d / seqlen_offset %d", q_len, seqlen_offset);
     VMX_REQUIRE(num_heads > 0 && num_kv_heads > 0 && num_heads % num_kv_heads == 0,
@@ -1297,7 +1303,7 @@ static int prefill_attention_impl(uint16_t *out, const uint16_t *q, const void *
     int rc = vmx_prefill_attention_tiled(out, q, k_cache, v_cache, block_table, q_len, seqlen_offset, scale, num_heads, num_kv_heads, head_dim,
                                          block_size, window, f16 ? 3 : (fp8 ? 1 : 0), k_scale, v_scale, st);   // 64- / 128-wide heads
     if (rc != VMX_EUNSUPPORTED) return rc;
-#define ARGS st, out, q, k_cache, v_cache, block_table, q_len, seqlen_offset, scale, num_heads, num_kv_heads, block_size, window, k_scale, v_scale
+#define ARGS st, out, q, k_cache, v_cache, block_table, q_len, seqlen_offset, scale, num_heads, num_kv_heads, block_size, window, k_scale, v_scale, out_f16
 #define PF_ONE(HD, Q) rc = f16 ? launch_prefill<HD, Q, 3>(ARGS) : fp8 ? launch_prefill<HD, Q, 1>(ARGS) : launch_prefill<HD, Q, 0>(ARGS)
 #define BY_QPK(HD)                                                                                                          \
     switch (qpk) {                                                                                                          \
@@ -1329,6 +1335,17 @@ extern "C" int vmx_prefill_attention_bf16(uint16_t *out, const uint16_t *q, cons
                                           const float *v_scale, void *stream) {
     return prefill_attention_impl(out, q, k_cache, v_cache, block_table, q_len, seqlen_offset, scale, num_heads, num_kv_heads, head_dim,
                                   block_size, window, kv_dtype, k_scale, v_scale, stream, false);
+}
+
+// vmx_prefill_attention_bf16 with results that go out as fp16 (of the bf16 value) where out_f16 (head sizes vmx_prefill_attention_gives_f16 names): what a
+// product over fp16 rows reads next
+bool vmx_prefill_attention_gives_f16(int head_dim) { return head_dim > 128; }
+int vmx_prefill_attention_rows(uint16_t *out, const uint16_t *q, const void *k_cache, const void *v_cache, const int32_t *block_table, int q_len, int seqlen_offset,
+                               float scale, int num_heads, int num_kv_heads, int head_dim, int block_size, int window, int kv_dtype, const float *k_scale,
+                               const float *v_scale, bool out_f16, hipStream_t st) {
+    VMX_REQUIRE(!out_f16 || vmx_prefill_attention_gives_f16(head_dim), "prefill_attention: no fp16 results for head_dim %d", head_dim);
+    return prefill_attention_impl(out, q, k_cache, v_cache, block_table, q_len, seqlen_offset, scale, num_heads, num_kv_heads, head_dim, block_size, window, kv_dtype,
+                                  k_scale, v_scale, st, false, out_f16);
 }
 
 // The same over fp16 queries and an fp16 cache, fp16 out (models that run in fp16): the fp16 forms of the matrix instructions,

@@ -9,6 +9,7 @@
 // "bf16(linear out) -> post-norm -> + residual -> * layer_scalar -> next pre-norm -> q8_1" (the sandwich norms of
 // two consecutive sub-blocks), one kernel does per-head q/k/v norms + RoPE + KV write, one does GeGLU + q8_1.
 // A layer is 10 launches (4 MMVQ: q|k|v and gate|up each go out as one multi-tensor launch); the step is a fixed launch sequence (hipGraph-capturable).
+#include "tile_gemm.h"
 #include "vmx_kernels.h"
 
 #include <math.h>
@@ -52,16 +53,27 @@ __global__ __launch_bounds__(256) void g4_embed_kernel(uint16_t *__restrict__ ou
     }
 }
 
+__device__ __forceinline__ uint4 bf16_rows_as_f16(const uint4 v) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) o[j] = (uint32_t)bf16_value_to_f16((uint16_t)w[j]) | ((uint32_t)bf16_value_to_f16((uint16_t)(w[j] >> 16)) << 16);
+    return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
 // One workgroup per token; thread t owns the 8-element chunks t, t+256, ... (CH of them) in registers.
+// PROMPT: o may lie in slices [slices][tokens][hidden], whose sum it is; x16 != nullptr: x as fp16 as well, what the products behind it read.  (Decode steps
+// have a form without either: their 5.2 us, four a step, were 6.2 with the choices in it.)  A 256-token prompt of Gemma-4-12B, where sums and conversions were
+// launches of their own: 3204 -> 2925 us for 12 layers.
 //   o given:  o_r = bf16(o);  n = bf16(o_r * rsqrt(mean(o_r^2) + eps) * w_post);  h = bf16(n + h_in);
 //             scalar given: h = bf16(h * scalar)                       (post-norm, residual add, layer_scalar)
 //   always:   x = bf16(h * rsqrt(mean(h^2) + eps) * w_next)  (+ its q8_1 form)   (the next sub-block's pre-norm);
 //             w_next == nullptr: x = h (the per-layer-input gate projects the residual stream itself)
-template <int CH>
+template <int CH, bool PROMPT>
 __global__ __launch_bounds__(256) void g4_norm_kernel(uint16_t *__restrict__ h, const uint16_t *__restrict__ h_in, uint16_t *__restrict__ x, const float *__restrict__ o,
                                                        const uint16_t *__restrict__ w_post, const uint16_t *__restrict__ scalar,
                                                        const uint16_t *__restrict__ w_next, float eps, int hidden,
-                                                       int8_t *__restrict__ aq, float *__restrict__ ad) {
+                                                       int8_t *__restrict__ aq, float *__restrict__ ad, int slices, uint16_t *__restrict__ x16) {
     __shared__ float red[4];
     const int64_t row = (int64_t)blockIdx.x * hidden;
     const int nchunk = hidden >> 3;
@@ -81,6 +93,18 @@ __global__ __launch_bounds__(256) void g4_norm_kernel(uint16_t *__restrict__ h, 
     }
     const float sc = scalar ? vmx_bf16_to_f32(scalar[0]) : 1.0f;
     float hv[CH][8];
+    if constexpr (PROMPT) {
+#pragma unroll 4
+        for (int s = 1; s < slices; s++) {   // in slice order
+#pragma unroll
+            for (int c = 0; c < CH; c++) {
+                const float *at = o + (int64_t)s * gridDim.x * hidden + row + 8 * min((int)threadIdx.x + 256 * c, nchunk - 1);
+                const float4 a4 = *reinterpret_cast<const float4 *>(at), b4 = *reinterpret_cast<const float4 *>(at + 4);
+                oa[c] = make_float4(oa[c].x + a4.x, oa[c].y + a4.y, oa[c].z + a4.z, oa[c].w + a4.w);
+                ob[c] = make_float4(ob[c].x + b4.x, ob[c].y + b4.y, ob[c].z + b4.z, ob[c].w + b4.w);
+            }
+        }
+    }
     if (o) {
         float ov[CH][8];
         float v1 = 0.f;
@@ -134,6 +158,7 @@ __global__ __launch_bounds__(256) void g4_norm_kernel(uint16_t *__restrict__ h, 
             for (int j = 0; j < 8; j++) out[j] = w_next ? hv[c][j] * inv2 * wv[j] : hv[c][j];
             const uint4 packed = pack8(out);
             *reinterpret_cast<uint4 *>(x + row + 8 * ci) = packed;
+            if (PROMPT && x16) *reinterpret_cast<uint4 *>(x16 + row + 8 * ci) = bf16_rows_as_f16(packed);
             if (aq) {
                 float xr[8];
                 unpack8(packed, xr);
@@ -145,8 +170,9 @@ __global__ __launch_bounds__(256) void g4_norm_kernel(uint16_t *__restrict__ h, 
 
 // grid (Hq + 2*Hkv, tokens), block 64.  proj: f32 [tokens][ntot] = q | k | (v) projections.  Per head: bf16 round,
 // per-head RMSNorm (q, k weighted; v unweighted), NeoX RoPE on the first rot_dim dims of q and k, bf16 rounds after
-// each; q -> q_out, k and v -> the layer's paged cache (bf16 or FP8 e4m3).  v_from_k: V is the K projection
+// each (proj may lie in slices [slices][tokens][ntot], whose sum it is); q -> q_out, k and v -> the layer's paged cache (bf16 or FP8 e4m3).  v_from_k: V is the K projection
 // (before K's norm and rotation) put through the unweighted norm.  stage != nullptr: K and V go to that bf16 buffer instead of the cache.
+template <bool SLICED>
 __global__ __launch_bounds__(64) void g4_qkv_post_kernel(const float *__restrict__ proj, int ntot, uint16_t *__restrict__ q_out,
                                                           void *__restrict__ k_cache, void *__restrict__ v_cache,
                                                           const uint16_t *__restrict__ q_norm_w, const uint16_t *__restrict__ k_norm_w,
@@ -154,7 +180,7 @@ __global__ __launch_bounds__(64) void g4_qkv_post_kernel(const float *__restrict
                                                           const int32_t *__restrict__ positions, const int32_t *__restrict__ slots, int Hq,
                                                           int Hkv, int hd, int rot_dim, int v_from_k, int fp8,
                                                           const float *__restrict__ k_scale, const float *__restrict__ v_scale,
-                                                          uint16_t *__restrict__ stage) {
+                                                          uint16_t *__restrict__ stage, int slices) {
     __shared__ float vals[512];
     const int head = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
     const bool is_q = head < Hq, is_k = !is_q && head < Hq + Hkv;
@@ -173,6 +199,12 @@ __global__ __launch_bounds__(64) void g4_qkv_post_kernel(const float *__restrict
         const int i = min(lane + 64 * j, hd - 1);
         pv[j] = proj[base + i];
         nwv[j] = nw ? vmx_bf16_to_f32(nw[i]) : 1.0f;
+    }
+    if constexpr (SLICED) {
+#pragma unroll 2
+        for (int s = 1; s < slices; s++)   // in slice order
+#pragma unroll
+            for (int j = 0; j < 8; j++) pv[j] += proj[(int64_t)s * gridDim.y * ntot + base + min(lane + 64 * j, hd - 1)];
     }
     const int half = rot_dim >> 1;
     const bool rot = (is_q || is_k) && half > 0;
@@ -473,9 +505,10 @@ int int_weights(vmx_gemma4 *m, const IqLin *const *lins, int n, int total, int K
 
 // n linears on the same `rows` token rows: the q8_1 MMVQ up to IQ_GEMV_MAX_M = 16 rows (activations already quantised in m->q8), beyond that
 // the reference's large-M form (gguf/mod.rs:358-365): dequantise the weight once, multiply the unquantised bf16 rows `a`.
-// a_is_f16: the rows are fp16 already (what g4_gateup_prompt leaves)
+// a_is_f16: the rows are fp16 already.  left: as in vmx_iq_prompt_f32, the slices in m->gemm_part
 int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, const uint16_t *a, float *y, int ldy, int rows,
-               hipStream_t st, bool a_is_f16 = false) {
+               hipStream_t st, bool a_is_f16 = false, int *left = nullptr) {
+    if (left) *left = 1;
     if (rows <= 16) {
         if (n == 1 && offs[0] == 0) return mmvq(m, *lins[0], y, ldy, rows, st);
         return mmvq_group(m, lins, offs, n, y, ldy, rows, st);
@@ -497,7 +530,8 @@ int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, 
         }
         VmxMmvqSeg segs[3];
         for (int i = 0; i < n; i++) segs[i] = VmxMmvqSeg{lins[i]->raw.p, lins[i]->ggml_type, lins[i]->out_features, offs[i]};
-        if (vmx_iq_prompt_ok(segs, n, rows, K)) return vmx_iq_prompt_f32(segs, n, a16, y, rows, K, ldy, (float *)m->gemm_part.p, m->gemm_part.bytes, st);
+        if (vmx_iq_prompt_ok(segs, n, rows, K)) return vmx_iq_prompt_f32(segs, n, a16, y, rows, K, ldy, (float *)m->gemm_part.p, m->gemm_part.bytes, st,
+                                                                        left);
         if (int rc = int_weights(m, lins, n, total, K, st)) return rc;
         return vmx_int_gemm_f32(a16, m->gemm_ws.p, y, rows, total, K, ldy, (float *)m->gemm_part.p, m->gemm_part.bytes, st);
     }
@@ -522,10 +556,20 @@ int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, 
     return VMX_OK;
 }
 
-int g4_linear(vmx_gemma4 *m, const IqLin &l, const uint16_t *a, float *y, int ldy, int rows, hipStream_t st, bool a_is_f16 = false) {
+int g4_linear(vmx_gemma4 *m, const IqLin &l, const uint16_t *a, float *y, int ldy, int rows, hipStream_t st, bool a_is_f16 = false, int *left = nullptr) {
     const IqLin *one[1] = {&l};
     const int off[1] = {0};
-    return g4_linears(m, one, off, 1, a, y, ldy, rows, st, a_is_f16);
+    return g4_linears(m, one, off, 1, a, y, ldy, rows, st, a_is_f16, left);
+}
+
+// Prompt rows on which all of these projections run as ONE product over fp16 rows
+bool f16_rows_ok(const IqLin *const *lins, int n, int rows) {
+    int total = 0;
+    for (int i = 0; i < n; i++) {
+        if (!int_form_ok(*lins[i], rows)) return false;
+        total += lins[i]->out_features;
+    }
+    return rows > 16 && vmx_int_gemm_ok(rows, total, lins[0]->in_features);
 }
 
 // Prompt-sized gate|up with the GeGLU in its epilogue: possible where gate, up and the down projection that reads the result (fp16 rows,
@@ -536,10 +580,10 @@ bool gateup_prompt_ok(const G4Layer &L, int rows) {
            vmx_int_gemm_ok(rows, g.out_features + u.out_features, g.in_features);
 }
 
-int g4_gateup_prompt(vmx_gemma4 *m, const G4Layer &L, const uint16_t *x, uint16_t *act, int rows, hipStream_t st) {
+// the rows are in m->a16 as fp16
+int g4_gateup_prompt(vmx_gemma4 *m, const G4Layer &L, uint16_t *act, int rows, hipStream_t st) {
     const IqLin *gu[2] = {&L.lin[VMX_L_GATE], &L.lin[VMX_L_UP]};
     const int K = gu[0]->in_features, inter = gu[0]->out_features;
-    if (int rc = vmx_bf16_rows_to_f16(x, (uint16_t *)m->a16.p, (int64_t)rows * K, st)) return rc;
     const VmxMmvqSeg segs[2] = {{gu[0]->raw.p, gu[0]->ggml_type, inter, 0}, {gu[1]->raw.p, gu[1]->ggml_type, inter, inter}};
     if (segs[0].ggml_type == segs[1].ggml_type && vmx_iq_prompt_ok(segs, 2, rows, K))
         return vmx_iq_prompt_geglu(segs[0], segs[1], (const uint16_t *)m->a16.p, act, rows, K, st);
@@ -558,12 +602,20 @@ int g4_tp_reduce(vmx_gemma4 *m, float *out, int tokens, int hidden, hipStream_t 
 }
 
 void launch_norm(hipStream_t st, int tokens, uint16_t *h, uint16_t *x, const float *o, const uint16_t *w_post, const uint16_t *scalar,
-                 const uint16_t *w_next, float eps, int hidden, int8_t *aq, float *ad, const uint16_t *h_in = nullptr) {
+                 const uint16_t *w_next, float eps, int hidden, int8_t *aq, float *ad, const uint16_t *h_in = nullptr, int slices = 1, uint16_t *x16 = nullptr) {
     if (!h_in) h_in = h;
-    if (hidden <= 2048) hipLaunchKernelGGL(g4_norm_kernel<1>, dim3(tokens), dim3(256), 0, st, h, h_in, x, o, w_post, scalar, w_next, eps, hidden, aq, ad);
-    else if (hidden <= 4096) hipLaunchKernelGGL(g4_norm_kernel<2>, dim3(tokens), dim3(256), 0, st, h, h_in, x, o, w_post, scalar, w_next, eps, hidden, aq, ad);
-    else if (hidden <= 8192) hipLaunchKernelGGL(g4_norm_kernel<4>, dim3(tokens), dim3(256), 0, st, h, h_in, x, o, w_post, scalar, w_next, eps, hidden, aq, ad);
-    else hipLaunchKernelGGL(g4_norm_kernel<8>, dim3(tokens), dim3(256), 0, st, h, h_in, x, o, w_post, scalar, w_next, eps, hidden, aq, ad);
+#define G4_NORM(CH)                                                                                                                                \
+    do {                                                                                                                                           \
+        if (slices > 1 || x16) hipLaunchKernelGGL((g4_norm_kernel<CH, true>), dim3(tokens), dim3(256), 0, st, h, h_in, x, o, w_post, scalar, w_next, eps, \
+                                           hidden, aq, ad, slices, x16);                                                                           \
+        else hipLaunchKernelGGL((g4_norm_kernel<CH, false>), dim3(tokens), dim3(256), 0, st, h, h_in, x, o, w_post, scalar, w_next, eps, hidden,   \
+                                aq, ad, 1, nullptr);                                                                                                   \
+    } while (0)
+    if (hidden <= 2048) G4_NORM(1);
+    else if (hidden <= 4096) G4_NORM(2);
+    else if (hidden <= 8192) G4_NORM(4);
+    else G4_NORM(8);
+#undef G4_NORM
 }
 }  // namespace
 
@@ -929,6 +981,9 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
     // pending: the previous layer's last linear output still to be post-normed, added, scaled
     const float *pending = nullptr;
     const uint16_t *pending_w = nullptr, *pending_scalar = nullptr;
+    int pending_left = 1;              // its slices (in m->gemm_part, where the reader adds them)
+    // q8_1 rows are for the products of up to 16 rows
+    int8_t *const aq8 = B <= 16 ? aq_of(m) : nullptr;
     const uint16_t *h_src = nullptr;   // non-null: the stream was left in m->h2 by a norm-fused gate|up launch; the next norm moves it back to h
     int li = -1;
     for (const G4Layer &L : m->layers) {
@@ -955,13 +1010,17 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
                 h_src = nullptr;
             }
         }
+        int qkv_left = 1;
         if (!norm_in_qkv) {
-            launch_norm(st, B, h, x, pending, pending_w, pending_scalar, (const uint16_t *)L.input_ln.p, c.rms_norm_eps, H, aq_of(m),
-                        ad_of(m, B, H), h_src);
-            h_src = nullptr;
             const IqLin *qkv[3] = {&L.lin[VMX_L_Q], &L.lin[VMX_L_K], &L.lin[VMX_L_V]};
             const int offs[3] = {0, NQ, NQ + NKV};
-            if (int rc = g4_linears(m, qkv, offs, nseg, x, proj, ntot, B, st)) return rc;
+            const bool rows16 = f16_rows_ok(qkv, nseg, B);
+            launch_norm(st, B, h, x, pending, pending_w, pending_scalar, (const uint16_t *)L.input_ln.p, c.rms_norm_eps, H, aq8, ad_of(m, B, H), h_src,
+                        pending_left, rows16 ? (uint16_t *)m->a16.p : nullptr);
+            h_src = nullptr;
+            // a prompt's slices stay where they are for the launch behind the product
+            if (int rc = g4_linears(m, qkv, offs, nseg, rows16 ? (const uint16_t *)m->a16.p : x, proj, ntot, B, st, rows16, prefill_offset >= 0 ? &qkv_left : nullptr))
+                return rc;
         }
         const float *ks = (const float *)KV.kv_scales.p;
         // short contexts: per-head norms + RoPE + KV write + attention + merge in one launch (not for K == V or KV-shared layers)
@@ -974,6 +1033,8 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
         // then the merge that also emits q8_1 for o_proj: two launches instead of three
         const bool split_attn = !fused_attn && prefill_offset < 0 && !L.k_eq_v && !L.kv_shared && !first_write && hd == 256 &&
                                 vmx_split_decode_attention_parts_wide(hd, Hq / Hkv, L.rot, max_seq_len, L.window) > 0;
+        const IqLin *const o_lin[1] = {&L.lin[VMX_L_O]};
+        const bool attn16 = prefill_offset >= 0 && vmx_prefill_attention_gives_f16(hd) && f16_rows_ok(o_lin, 1, B);
         if (split_attn) {
             VmxAttnParts ap;
             // workgroups per (sequence, KV head): 8 for a few rows; with many rows every compute unit has work at fewer, and each
@@ -996,10 +1057,11 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
                 return rc;
         } else {
             // a KV-shared layer launches the query heads only: its K/V for these tokens were written by the target layer
-            hipLaunchKernelGGL(g4_qkv_post_kernel, dim3(L.kv_shared ? Hq : Hq + 2 * Hkv, B), dim3(64), 0, st, proj, ntot, q, KV.k_cache.p,
+            const auto post = qkv_left > 1 ? g4_qkv_post_kernel<true> : g4_qkv_post_kernel<false>;
+            hipLaunchKernelGGL(post, dim3(L.kv_shared ? Hq : Hq + 2 * Hkv, B), dim3(64), 0, st, qkv_left > 1 ? (const float *)m->gemm_part.p : proj, ntot, q, KV.k_cache.p,
                                KV.v_cache.p, (const uint16_t *)L.q_norm.p, (const uint16_t *)L.k_norm.p, c.rms_norm_eps,
                                (const float *)(L.sliding ? m->cos_sin_s.p : m->cos_sin_f.p), positions, slot_mapping, Hq, Hkv, hd, L.rot,
-                               L.k_eq_v ? 1 : 0, fp8, ks, ks + 1, first_write ? stage : nullptr);
+                               L.k_eq_v ? 1 : 0, fp8, ks, ks + 1, first_write ? stage : nullptr, qkv_left);
             if (first_write) {
                 const int64_t n = (int64_t)B * NKV;
                 if (int rc = vmx_kv_scales_calibrate_if_needed(L.kv_scales.p, stage, n, stage + n, n, m->kv_headroom, st)) return rc;
@@ -1007,11 +1069,12 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
                                                    c.kv_cache_dtype, ks, ks + 1, st))
                     return rc;
             }
-            if (prefill_offset >= 0) {   // the rows' K/V are in the cache: causal (windowed) attention over it, then q8_1 for o_proj
-                if (int rc = vmx_prefill_attention_bf16(attn, q, KV.k_cache.p, KV.v_cache.p, block_tables, B, prefill_offset, 1.0f, Hq, Hkv,
-                                                        hd, c.block_size, L.window, c.kv_cache_dtype, ks, ks + 1, st))
+            if (prefill_offset >= 0) {   // the rows' K/V are in the cache: causal (windowed) attention over it, then q8_1 for o_proj (fp16 rows: attn16)
+                if (int rc = vmx_prefill_attention_rows(attn, q, KV.k_cache.p, KV.v_cache.p, block_tables, B, prefill_offset, 1.0f, Hq, Hkv, hd, c.block_size,
+                                                        L.window, c.kv_cache_dtype, ks, ks + 1, attn16, st))
                     return rc;
-                if (int rc = vmx_quantize_q8_1_bf16(attn, aq_of(m), ad_of(m, B, NQ), (int64_t)B * (NQ / 32), st)) return rc;
+                if (B <= 16)
+                    if (int rc = vmx_quantize_q8_1_bf16(attn, aq_of(m), ad_of(m, B, NQ), (int64_t)B * (NQ / 32), st)) return rc;
             } else {
                 VmxAttnParts ap;
                 if (int rc = vmx_paged_attention_parts(q, KV.k_cache.p, KV.v_cache.p, block_tables, seq_lens, 1.0f, B, Hq, Hkv,
@@ -1021,7 +1084,8 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
                 if (int rc = vmx_paged_attention_merge(attn, &ap, seq_lens, B, Hq, hd, L.window, st, aq_of(m), ad_of(m, B, NQ))) return rc;
             }
         }
-        if (int rc = g4_linear(m, L.lin[VMX_L_O], attn, out, H, B, st)) return rc;
+        int o_left = 1;
+        if (int rc = g4_linear(m, L.lin[VMX_L_O], attn, out, H, B, st, attn16, prefill_offset >= 0 && !tp ? &o_left : nullptr)) return rc;
         if (tp)
             if (int rc = g4_tp_reduce(m, out, B, H, st)) return rc;
         const VmxMmvqSeg gate_pk = {L.lin[VMX_L_GATE].packed.p, L.lin[VMX_L_GATE].ggml_type, L.lin[VMX_L_GATE].out_features, 0};
@@ -1040,8 +1104,8 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
             h_src = (const uint16_t *)m->h2.p;
         } else {
         // post_attention_layernorm + residual, pre_feedforward_layernorm -> x, q8_1(x)
-        launch_norm(st, B, h, x, out, (const uint16_t *)L.post_attn_ln.p, nullptr, (const uint16_t *)L.pre_ffn_ln.p, c.rms_norm_eps, H,
-                    aq_of(m), ad_of(m, B, H));
+        launch_norm(st, B, h, x, o_left > 1 ? (const float *)m->gemm_part.p : out, (const uint16_t *)L.post_attn_ln.p, nullptr, (const uint16_t *)L.pre_ffn_ln.p,
+                    c.rms_norm_eps, H, aq8, ad_of(m, B, H), nullptr, o_left, gateup_prompt_ok(L, B) ? (uint16_t *)m->a16.p : nullptr);
         }
         if (norm_in_mlp) {
         } else if (B == 1 && vmx_iq_packed_geglu_ok(&gate_pk, &up_pk, H, B)) {
@@ -1069,7 +1133,7 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
                 return rc_glu;
             }
         } else if (gateup_prompt_ok(L, B)) {
-            if (int rc = g4_gateup_prompt(m, L, x, act, B, st)) return rc;
+            if (int rc = g4_gateup_prompt(m, L, act, B, st)) return rc;
         } else {
             const IqLin *gu[2] = {&L.lin[VMX_L_GATE], &L.lin[VMX_L_UP]};
             const int offs[2] = {0, I};
@@ -1078,25 +1142,26 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
             hipLaunchKernelGGL(g4_geglu_kernel, dim3((unsigned)(blocks > 1024 ? 1024 : blocks)), dim3(256), 0, st, proj, B, act, I, aq_of(m),
                                ad_of(m, B, I));
         }
-        const int rc_down = g4_linear(m, L.lin[VMX_L_DOWN], act, out, H, B, st, gateup_prompt_ok(L, B));
+        const int rc_down = g4_linear(m, L.lin[VMX_L_DOWN], act, out, H, B, st, gateup_prompt_ok(L, B), prefill_offset >= 0 && !tp ? &pending_left : nullptr);
         m->q8_alt = nullptr;
         if (rc_down) return rc_down;
         if (tp)
             if (int rc = g4_tp_reduce(m, out, B, H, st)) return rc;
-        pending = out;
+        pending = pending_left > 1 ? (const float *)m->gemm_part.p : out;
         pending_w = (const uint16_t *)L.post_ffn_ln.p;
         pending_scalar = (const uint16_t *)L.scalar.p;
         if (L.ple) {   // apply_ple (:1663-1683): h += norm(per_layer_projection(gelu_tanh(gate(h)) * pli[layer])), before the scalar
-            launch_norm(st, B, h, x, pending, pending_w, nullptr, nullptr, c.rms_norm_eps, H, aq_of(m), ad_of(m, B, H), h_src);
+            launch_norm(st, B, h, x, pending, pending_w, nullptr, nullptr, c.rms_norm_eps, H, aq8, ad_of(m, B, H), h_src, pending_left);
             h_src = nullptr;
             if (int rc = g4_linear(m, L.lin[VMX_L_PLE_GATE], x, proj, P, B, st)) return rc;
             hipLaunchKernelGGL(g4_ple_gate_kernel, dim3((unsigned)(((int64_t)B * P / 8 + 255) / 256)), dim3(256), 0, st, proj,
                                (const uint16_t *)m->pli.p + (size_t)li * P, (int64_t)LP, B, P, act, aq_of(m), ad_of(m, B, P));
             if (int rc = g4_linear(m, L.lin[VMX_L_PLE_PROJ], act, out, H, B, st)) return rc;
+            pending = out, pending_left = 1;
             pending_w = (const uint16_t *)L.post_ple_norm.p;
         }
     }
-    launch_norm(st, B, h, x, pending, pending_w, pending_scalar, (const uint16_t *)m->final_norm.p, c.rms_norm_eps, H, nullptr, nullptr, h_src);
+    launch_norm(st, B, h, x, pending, pending_w, pending_scalar, (const uint16_t *)m->final_norm.p, c.rms_norm_eps, H, nullptr, nullptr, h_src, pending_left);
     VMX_CHECK_LAUNCH("gemma4 layers");
     for (G4Layer &L : m->layers) L.kv_calibrated = true;   // every cache has had its first write
     return VMX_OK;

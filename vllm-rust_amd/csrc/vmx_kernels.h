@@ -179,6 +179,10 @@ size_t vmx_iq_gemm_int_workspace(int M, int N, int K);
 size_t vmx_iq_gemm_int_weight_bytes(int N, int K);
 int vmx_iq_dequant_int(int ggml_type, const void *blocks, void *workspace, int row0, int rows, int N, int K, hipStream_t st);
 int vmx_bf16_rows_to_f16(const uint16_t *A, uint16_t *a16, int64_t n, hipStream_t st);
+bool vmx_prefill_attention_gives_f16(int head_dim);
+int vmx_prefill_attention_rows(uint16_t *out, const uint16_t *q, const void *k_cache, const void *v_cache, const int32_t *block_table, int q_len, int seqlen_offset,
+                               float scale, int num_heads, int num_kv_heads, int head_dim, int block_size, int window, int kv_dtype, const float *k_scale,
+                               const float *v_scale, bool out_f16, hipStream_t st);
 bool vmx_int_gemm_ok(int M, int N, int K);
 size_t vmx_int_gemm_part_bytes();
 int vmx_int_gemm_f32(const uint16_t *a16, const void *workspace, float *C, int M, int N, int K, int ldc, float *part, size_t part_bytes, hipStream_t st);
@@ -186,7 +190,8 @@ int vmx_int_gemm_geglu(const uint16_t *a16, const void *workspace, uint16_t *act
 int vmx_int_slices(const float *part, float *y, int slices, int M, int N, int64_t ldy, hipStream_t st);   // y = part [slices][M][N] in slice order
 // iq_prompt.hip: the same product with the raw blocks decoded inside it (a segment's `w` = its raw blocks)
 bool vmx_iq_prompt_ok(const VmxMmvqSeg *segs, int nseg, int M, int K);
-int vmx_iq_prompt_f32(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st);
+int vmx_iq_prompt_f32(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st,
+                      int *left = nullptr);
 int vmx_iq_prompt_geglu(const VmxMmvqSeg &gate, const VmxMmvqSeg &up, const uint16_t *a16, uint16_t *act16, int M, int K, hipStream_t st);
 int vmx_dense_gemv_launch(uint16_t *y, const uint16_t *x, const uint16_t *W, const uint16_t *bias, int M, int N, int K, hipStream_t st,
                           int f16 = 0);   // f16: x, W, bias and y hold fp16 (same f32 accumulation, fp16 matrix / dot instructions)
