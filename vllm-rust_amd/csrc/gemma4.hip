@@ -505,7 +505,7 @@ int int_weights(vmx_gemma4 *m, const IqLin *const *lins, int n, int total, int K
 
 // n linears on the same `rows` token rows: the q8_1 MMVQ up to IQ_GEMV_MAX_M = 16 rows (activations already quantised in m->q8), beyond that
 // the reference's large-M form (gguf/mod.rs:358-365): dequantise the weight once, multiply the unquantised bf16 rows `a`.
-// a_is_f16: the rows are fp16 already.  left: as in vmx_iq_prompt_f32, the slices in m->gemm_part
+// a_is_f16: the rows are fp16 already.  left: as in vmx_iq_prompt_slices, the slices in m->gemm_part
 int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, const uint16_t *a, float *y, int ldy, int rows,
                hipStream_t st, bool a_is_f16 = false, int *left = nullptr) {
     if (left) *left = 1;
@@ -530,8 +530,7 @@ int g4_linears(vmx_gemma4 *m, const IqLin *const *lins, const int *offs, int n, 
         }
         VmxMmvqSeg segs[3];
         for (int i = 0; i < n; i++) segs[i] = VmxMmvqSeg{lins[i]->raw.p, lins[i]->ggml_type, lins[i]->out_features, offs[i]};
-        if (vmx_iq_prompt_ok(segs, n, rows, K)) return vmx_iq_prompt_f32(segs, n, a16, y, rows, K, ldy, (float *)m->gemm_part.p, m->gemm_part.bytes, st,
-                                                                        left);
+        if (vmx_iq_prompt_ok(segs, n, rows, K)) return vmx_iq_prompt_slices(segs, n, a16, y, rows, K, ldy, (float *)m->gemm_part.p, m->gemm_part.bytes, st, left);
         if (int rc = int_weights(m, lins, n, total, K, st)) return rc;
         return vmx_int_gemm_f32(a16, m->gemm_ws.p, y, rows, total, K, ldy, (float *)m->gemm_part.p, m->gemm_part.bytes, st);
     }

@@ -479,8 +479,8 @@ bool vmx_iq_prompt_ok(const VmxMmvqSeg *segs, int nseg, int M, int K) {
 // y[:, y_off of a segment ..] (f32, rows ldy apart) = a16 [M][K] times the segments' raw blocks, one product.  The segments' columns lie one behind the
 // other from column 0 on.  part: scratch for slices, as many as fit part_bytes.  left: a reader that adds slices itself; *left = their count where they stay in part
 // ([*left][M][ldy], rows without gaps), else 1 and the result is in y.
-int vmx_iq_prompt_f32(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st,
-                      int *left) {
+int vmx_iq_prompt_slices(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st,
+                         int *left) {
     IqpArgs p = {};
     int tiles = 0, N = 0;
     for (int i = 0; i < nseg; i++) {
@@ -497,6 +497,10 @@ int vmx_iq_prompt_f32(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, flo
         if (*left > 1) return VMX_OK;
     }
     return plan.slices > 1 ? vmx_int_slices(part, y, plan.slices, M, N, ldy, st) : VMX_OK;
+}
+
+int vmx_iq_prompt_f32(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st) {
+    return vmx_iq_prompt_slices(segs, nseg, a16, y, M, K, ldy, part, part_bytes, st, nullptr);
 }
 
 // act16 [M][inter] (fp16) = GeGLU of gate and up, both of one type

@@ -190,8 +190,9 @@ int vmx_int_gemm_geglu(const uint16_t *a16, const void *workspace, uint16_t *act
 int vmx_int_slices(const float *part, float *y, int slices, int M, int N, int64_t ldy, hipStream_t st);   // y = part [slices][M][N] in slice order
 // iq_prompt.hip: the same product with the raw blocks decoded inside it (a segment's `w` = its raw blocks)
 bool vmx_iq_prompt_ok(const VmxMmvqSeg *segs, int nseg, int M, int K);
-int vmx_iq_prompt_f32(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st,
-                      int *left = nullptr);
+int vmx_iq_prompt_f32(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st);
+int vmx_iq_prompt_slices(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st,
+                         int *left);
 int vmx_iq_prompt_geglu(const VmxMmvqSeg &gate, const VmxMmvqSeg &up, const uint16_t *a16, uint16_t *act16, int M, int K, hipStream_t st);
 int vmx_dense_gemv_launch(uint16_t *y, const uint16_t *x, const uint16_t *W, const uint16_t *bias, int M, int N, int K, hipStream_t st,
                           int f16 = 0);   // f16: x, W, bias and y hold fp16 (same f32 accumulation, fp16 matrix / dot instructions)
