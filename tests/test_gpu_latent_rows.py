@@ -138,3 +138,43 @@ def test_shared_keys(gpu, contexts, new, heads, window, shuffled):
         exact = torch.softmax(logits, 1)[:, :-1] @ rows[:, :R]
         bound = (torch.expm1(4 * d) + 2.0 ** -15 + 1024 * 2.0 ** -24) * rows[:, :R].abs().max()
         assert bool(((out[t].double() - exact).abs() <= bound).all()), (t, float((out[t].double() - exact).abs().max()), float(bound))
+
+
+# one token a row tile, with one and two head groups, and two tokens a row tile; a whole prompt and a window
+@pytest.mark.parametrize("heads,window", [(16, 0), (16, 40), (20, 0), (8, 0), (8, 40)])
+def test_rows_that_are_not_finite(gpu, heads, window):
+    """An infinity or a NaN in a token's cache row reaches the tokens that have it among their keys (at least one result of each is not finite) and
+    of the others at most those of its own row tile, before it: row tiles that share their keys with that token keep every bit."""
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    R, RD, bs, scale, T = 512, 64, 16, 0.06, 532
+    g = torch.Generator(device="cuda").manual_seed(heads + window)
+    mb = (T + bs - 1) // bs
+    bt = torch.randperm(mb, device="cuda", generator=g).to(torch.int32).view(1, mb)
+    cache = torch.randn((mb * bs, R + RD), device="cuda", generator=g).to(torch.bfloat16)
+    qa = torch.randn((T, heads, R), device="cuda", generator=g).to(torch.bfloat16).float()
+    qr = torch.randn((T, heads, RD), device="cuda", generator=g).to(torch.bfloat16).float()
+    pos = torch.arange(T, dtype=torch.int32, device="cuda")
+    sid = torch.zeros(T, dtype=torch.int32, device="cuda")
+    assert lib.vmx_latent_attention_workspace_bytes(T, heads, R, window, mb, bs) == 0
+
+    def run():
+        out = torch.full((T, heads, R), 7.0, device="cuda")
+        check(lib.vmx_latent_attention(out.data_ptr(), qa.data_ptr(), qr.data_ptr(), cache.data_ptr(), 1, bt.data_ptr(), mb, sid.data_ptr(), pos.data_ptr(),
+                                       None, scale, window, T, heads, R, RD, bs, None, 0, None))
+        torch.cuda.synchronize()
+        return out
+
+    clean = run()
+    tile = 16 // min(heads, 16)   # tokens a row tile
+    for at, value in ((3, float("inf")), (98, float("nan")), (255, float("-inf")), (T - 1, float("nan"))):   # last of four tiles, in the middle, of a 32-key tile, of all
+        row = int(bt[0, at // bs]) * bs + at % bs
+        held = cache[row].clone()
+        cache[row, 5:R:64] = value
+        out = run()
+        cache[row] = held
+        last = min(T, at + window) if window else T      # tokens at .. last - 1 have the key
+        assert bool((~torch.isfinite(out[at:last])).flatten(1).any(1).all())
+        assert torch.equal(out[:at // tile * tile], clean[:at // tile * tile])
+        first = (last + tile - 1) // tile * tile
+        assert torch.equal(out[first:], clean[first:])

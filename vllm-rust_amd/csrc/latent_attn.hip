@@ -485,6 +485,7 @@ __device__ __forceinline__ void la_request_1k(uint32_t at, const char *from) {  
 }
 
 constexpr int LS_KT = 32, LS_ROW = 1152, LS_TILE = LS_KT * LS_ROW, LS_REQ = LS_TILE / 4096;   // keys a tile; bytes of a row and a tile; requests a wave
+constexpr int LS_ZEROS = 1024;                                                                // bytes of zeros: a latent's
 
 __global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const LatentAttnArgs a) {
     extern __shared__ __align__(256) unsigned char la_smem[];
@@ -511,6 +512,10 @@ __global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const Latent
     const bool act = fl < a.TPT * a.HPT && tq < a.T && hq < a.H;
     const int rpos = act ? a.positions[tq] : -1, rlo = a.window > 0 ? max(0, rpos - a.window + 1) : 0;
     const int64_t th = act ? (int64_t)tq * a.H + hq : 0;
+    // the keys of this wave's own tokens
+    int own_hi = rpos, own_lo = rpos < 0 ? INT_MAX : rlo;
+    for (int m = 1; m < 64; m <<= 1) own_hi = max(own_hi, __shfl_xor(own_hi, m)), own_lo = min(own_lo, __shfl_xor(own_lo, m));
+    own_hi = __builtin_amdgcn_readfirstlane(own_hi), own_lo = __builtin_amdgcn_readfirstlane(own_lo);
     tg_u32x4 qf[KS];
 #pragma unroll
     for (int s = 0; s < KS; s++) {
@@ -543,8 +548,13 @@ __global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const Latent
     for (int d = 0; d < DT; d++) acc[d] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
     float m_r = -FLT_MAX, l_r = 0.f;   // l_r: the lane's own keys
     const uint32_t k_at = lds + fl * LS_ROW + ((fg ^ la_swizzle(fl)) << 4);
-    const int vr = 4 * fg + (fl >> 2);
+    const int vr = 4 * fg + (fl >> 2);   // key of the first half of a tile whose values this lane asks for
     const uint32_t v_at = lds + vr * LS_ROW + ((((fl >> 1) & 1) ^ la_swizzle(vr)) << 4) + 8 * (fl & 1);
+    // A wave's second product takes zeros for the keys that none of its own tokens has: their weights are 0, but 0 times an infinity or a NaN in another token's
+    // cache row is a NaN.  Its reads of such a key go to a kilobyte of zeros behind the tiles.
+    const uint32_t zeros = lds + 2 * LS_TILE;
+    if (tid < LS_ZEROS / 16) *(__attribute__((address_space(3))) tg_u32x4 *)(uintptr_t)(zeros + 16 * tid) = tg_u32x4{};
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     int next_entry = 0;
     if (ntiles > 0) {
         request(0, entry_of(0), 0);
@@ -604,10 +614,14 @@ __global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const Latent
 #pragma unroll
         for (int e = 0; e < 8; e++) lo8[e] = p[e] - vmx_bf16_to_f32(vmx_f32_to_bf16(p[e]));
         const vmx_bf16x8 pl = __builtin_bit_cast(vmx_bf16x8, vmx_pack16x8<false>(lo8));
-        const uint32_t v_stage = v_at + stage * LS_TILE;
+        auto v_from = [&](int half) {
+            const int j = kbase + 16 * half + vr;
+            return j >= own_lo && j <= own_hi ? v_at + stage * LS_TILE + half * 16 * LS_ROW : zeros;
+        };
+        const uint32_t v_half[2] = {v_from(0), v_from(1)};
         typedef la_s16x4 __attribute__((address_space(3))) *lds_s16x4;
         auto read_v = [&](int d, int half) {   // four keys of latent dimensions 16 d ..
-            return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(uintptr_t)((v_stage ^ (32 * (d & 3))) + (d >> 2) * 128 + half * 16 * LS_ROW));
+            return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(uintptr_t)((v_half[half] ^ (32 * (d & 3))) + (d >> 2) * 128));
         };
         la_s16x4 vf[AHEAD_V][2];
 #pragma unroll
@@ -759,6 +773,7 @@ int vmx_latent_attention_launch(void *out_latent, const void *q_abs, int io_bf16
         dim3 grid((unsigned)(((tokens + a.TPT - 1) / a.TPT) * a.NHG), a.NP);
         const bool small = RW <= 160 && kv_rank <= 128;
         const size_t lds = ((size_t)LA_KT * ((small ? 128 : 512) + LA_PAD) + 2 * 16 * LA_LD) * 2 + (64 + 64) * 4;
+        static_assert(2 * LS_TILE + LS_ZEROS <= (LA_KT * (512 + LA_PAD) + 2 * 16 * LA_LD) * 2 + (64 + 64) * 4, "the shared form fits the row tiles' memory");
         const bool whole = kv_rank == 512 && rot_dim == 64;
         const void *fn = small              ? (const void *)latent_attn_mfma_kernel<5, 2, 0>
                          : !whole           ? (const void *)latent_attn_mfma_kernel<18, 8, 0>
