@@ -178,3 +178,40 @@ def test_rows_that_are_not_finite(gpu, heads, window):
         assert torch.equal(out[:at // tile * tile], clean[:at // tile * tile])
         first = (last + tile - 1) // tile * tile
         assert torch.equal(out[first:], clean[first:])
+
+
+# the prompt alone, behind a whole group of row tiles of another one, and behind parts of a group; a window whose edges lie anywhere in a key tile
+@pytest.mark.parametrize("heads", [16, 8])
+@pytest.mark.parametrize("window", [0, 70])
+def test_neighbours_in_a_step(gpu, heads, window):
+    """Row tiles that share their keys give a token the same bits whichever tokens of its sequence are beside it.  Those whose group has another prompt's tokens in it
+    sum in another order: their weights' two bf16 halves are off by 2^-16 on either side, as in test_position_without_keys, and the f32 sums of
+    280 products by as many roundings."""
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    R, RD, bs, scale, n = 512, 64, 16, 0.06, 280
+    g = torch.Generator(device="cuda").manual_seed(heads + window)
+    mb = (n + 15) // bs + 1
+    bt = torch.randperm(2 * mb, device="cuda", generator=g).to(torch.int32).view(2, mb)
+    cache = torch.randn((2 * mb * bs, R + RD), device="cuda", generator=g).to(torch.bfloat16)
+    qa = torch.randn((2 * n, heads, R), device="cuda", generator=g)
+    qr = torch.randn((2 * n, heads, RD), device="cuda", generator=g)
+
+    def run(before):   # `before` tokens of sequence 1, then the n of sequence 0
+        T = before + n
+        pos = torch.cat([torch.arange(before), torch.arange(n)]).to(torch.int32).cuda()
+        sid = torch.tensor([1] * before + [0] * n, dtype=torch.int32, device="cuda")
+        a, r = (torch.cat([q[n:n + before], q[:n]]).contiguous() for q in (qa, qr))
+        out = torch.full((T, heads, R), float("nan"), device="cuda")
+        check(lib.vmx_latent_attention(out.data_ptr(), a.data_ptr(), r.data_ptr(), cache.data_ptr(), 1, bt.data_ptr(), mb, sid.data_ptr(), pos.data_ptr(),
+                                       None, scale, window, T, heads, R, RD, bs, None, 0, None))
+        torch.cuda.synchronize()
+        return out[before:]
+
+    group = 4 * (16 // heads)   # tokens of four row tiles
+    alone = run(0)
+    for before in (group, group + 1, 2 * group - 1, 33):
+        got = run(before)
+        mixed = -before % group   # tokens in the group with the other prompt's last ones
+        assert torch.equal(got[mixed:], alone[mixed:])
+        assert float((got[:mixed] - alone[:mixed]).abs().max() if mixed else 0.0) <= (2.0 ** -15 + 280 * 2.0 ** -23) * float(cache.abs().max())

@@ -12,8 +12,10 @@
 // constant), queries straight from the input or through an RMS-normed latent of their own, sizes, cache element type (bf16 / f32).
 // Layers may attend over another layer's cache: preparation then skips the key/value part.
 // Scores, softmax, the weighted sum, norms and angles are f32.  Queries are packed: token t belongs to sequence seq_ids[t] at
-// position positions[t], so prompts of different lengths, prompt portions and single decode tokens are the same launch, and a
-// token's result depends only on its own query and the cache rows of its window.
+// position positions[t], so prompts of different lengths, prompt portions and single decode tokens are the same launch.  A
+// token's result depends only on its own query and the cache rows of its window, beyond rounding: how its keys are cut into partitions and tiles, and so the order of
+// its sums, depends on how many row tiles the launch has and on whether those beside its own belong to its sequence.  (With fewer than 16 heads a row tile
+// holds several tokens; an infinity or a NaN in the cache row of one reaches the others of its tile.)
 #include "tile_gemm.h"
 #include "vmx_kernels.h"
 #include <float.h>
@@ -506,7 +508,8 @@ __global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const Latent
     int hi = a.positions[t0 + min(lane, n - 1)], lo = hi < 0 ? INT_MAX : a.window > 0 ? max(0, hi - a.window + 1) : 0;
     for (int m = 1; m < 64; m <<= 1) hi = max(hi, __shfl_xor(hi, m)), lo = min(lo, __shfl_xor(lo, m));
     hi = __builtin_amdgcn_readfirstlane(hi), lo = __builtin_amdgcn_readfirstlane(lo);
-    const int ntiles = hi < lo ? 0 : (hi - lo) / LS_KT + 1;
+    // Tiles start at multiples of 32 keys, wherever `lo` lies: a row's sums are cut at the same keys whatever tokens share its workgroup
+    const int key0 = lo / LS_KT * LS_KT, ntiles = hi < lo ? 0 : (hi - key0) / LS_KT + 1;
     // the lane's row
     const int tq = t0 + wave * a.TPT + fl / a.HPT, hq = hg * a.HPT + fl % a.HPT;
     const bool act = fl < a.TPT * a.HPT && tq < a.T && hq < a.H;
@@ -528,9 +531,9 @@ __global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const Latent
         const int c = 64 * q + lane, r = c / (LS_ROW / 16), at = c % (LS_ROW / 16);
         piece[q] = (uint32_t)((at ^ la_swizzle(8 * wave + r)) * 16) | (uint32_t)(4 * r) << 16;
     }
-    // Key 8 wave + lane % 8 of a tile (keys past `hi` repeat its row, and their weights are 0) and its block's table entry, which is not looked at
+    // Key 8 wave + lane % 8 of a tile (keys below `lo` and past `hi`, whose blocks may be another sequence's by now, repeat their rows) and its block's table entry, which is not looked at
     // before the next tile's turn: a wait for it would be one for the rows requested before it
-    auto key_of = [&](int kt) { return min(lo + LS_KT * kt + 8 * wave + (lane & 7), hi); };
+    auto key_of = [&](int kt) { return min(max(key0 + LS_KT * kt + 8 * wave + (lane & 7), lo), hi); };
     auto entry_of = [&](int kt) { return bt[key_of(kt) / a.block_size]; };
     const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)la_smem;
     auto request = [&](int kt, int entry, int stage) {
@@ -561,7 +564,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const Latent
         next_entry = entry_of(1);
     }
     for (int kt = 0; kt < ntiles; kt++) {
-        const int stage = kt & 1, kbase = lo + LS_KT * kt;
+        const int stage = kt & 1, kbase = key0 + LS_KT * kt;
         asm volatile("s_waitcnt vmcnt(0)" : "+v"(next_entry) : : "memory");
         __builtin_amdgcn_s_barrier();   // this tile is whole, and nobody reads the one before it any more
         asm volatile("" ::: "memory");
