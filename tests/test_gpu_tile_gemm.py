@@ -182,6 +182,26 @@ def test_iq_prompt_decoded(gpu, M, ggml_type, N, K, start, room):
     assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all()) and bool((ws[need:] == 7).all())
 
 
+# rows beyond what the least workspace holds in the integer form: the two-term bf16 split, whose activations stay bf16
+@pytest.mark.parametrize("size", [1.0, 3e5, 2.0 ** -40])
+def test_iq_gemm_rows_outside_fp16(gpu, size):
+    """Activations above fp16's largest value and below its smallest.  A weight's two bf16 halves are off by at most 2^-17 of it (2^-9 of a remainder of
+    2^-8); the f32 sums of two products a weight add (2 K + 8) 2^-24 of the sum of magnitudes."""
+    vmx, torch = gpu
+    from tests.helpers import random_iq_blocks
+    from vllm_rust_amd._lib import check, lib
+    M, N, K, t = 1500, 1024, 8192, 18
+    raw = torch.from_numpy(np.ascontiguousarray(random_iq_blocks(np.random.default_rng(3), vmx.iq_type_size(t), N * K // 256))).reshape(-1).cuda()
+    x = (torch.randn((M, K), device="cuda", generator=torch.Generator(device="cuda").manual_seed(3)) * size).to(torch.bfloat16)
+    ws = torch.empty(4 * N * K, dtype=torch.uint8, device="cuda")
+    y = torch.full((M, N), float("nan"), device="cuda")
+    check(lib.vmx_iq_gemm_f32(t, raw.data_ptr(), x.data_ptr(), y.data_ptr(), M, N, K, ws.data_ptr(), ws.numel(), None))
+    torch.cuda.synchronize()
+    w = vmx.iq_dequantize(t, raw, N * K // 256).reshape(N, K).double()
+    bound = (2.0 ** -17 + (2 * K + 8) * 2.0 ** -24) * (x.double().abs() @ w.abs().T)
+    assert bool(((y.double() - x.double() @ w.T).abs() <= bound).all())
+
+
 class _Seg(C.Structure):
     _fields_ = [("w", C.c_void_p), ("ggml_type", C.c_int), ("n_out", C.c_int), ("y_off", C.c_int)]
 

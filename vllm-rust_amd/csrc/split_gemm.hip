@@ -409,13 +409,15 @@ extern "C" int vmx_iq_gemm_f32(int ggml_type, const void *blocks, const uint16_t
                 vmx_iq_gemm_workspace(n_out, n_in));
     if (m == 0) return VMX_OK;
     hipStream_t st = vmx_stream(stream);
+    // Activations go to fp16 (which saturates and loses small values) only where the workspace has always allowed it, whichever of the two products then runs
+    const bool int_form = vmx_iq_int_form_ok(ggml_type) && workspace_bytes >= vmx_iq_gemm_int_workspace(m, n_out, n_in) && vmx_int_gemm_ok(m, n_out, n_in);
     const VmxMmvqSeg seg = {blocks, ggml_type, n_out, 0};
-    const size_t rows = ((size_t)m * n_in * 2 + 255) & ~(size_t)255;
-    if (vmx_iq_prompt_ok(&seg, 1, m, n_in) && workspace_bytes >= rows) {   // decoded inside the product: the workspace holds the rows, then slice sums
+    if (int_form && vmx_iq_prompt_ok(&seg, 1, m, n_in)) {   // decoded inside the product: the workspace holds the rows, then slice sums
+        const size_t rows = ((size_t)m * n_in * 2 + 255) & ~(size_t)255;   // fewer than the weights' integer form takes, besides these rows
         if (int rc = vmx_bf16_rows_to_f16(x, (uint16_t *)workspace, (int64_t)m * n_in, st)) return rc;
         return vmx_iq_prompt_f32(&seg, 1, (const uint16_t *)workspace, y, m, n_in, n_out, (float *)((char *)workspace + rows), workspace_bytes - rows, st);
     }
-    if (vmx_iq_int_form_ok(ggml_type) && workspace_bytes >= vmx_iq_gemm_int_workspace(m, n_out, n_in) && vmx_int_gemm_ok(m, n_out, n_in)) {
+    if (int_form) {
         // exact one-pass form: integer weights in fp16, one f32 scale per super-block; slice sums where the workspace has room for them
         uint16_t *a16 = (uint16_t *)((char *)workspace + vmx_iq_gemm_int_workspace(0, n_out, n_in));
         const size_t used = (vmx_iq_gemm_int_workspace(m, n_out, n_in) + 255) & ~(size_t)255;
