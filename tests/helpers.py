@@ -1,4 +1,5 @@
 """Shared test inputs: the reference tests' deterministic generators."""
+import ctypes
 import json
 from pathlib import Path
 
@@ -112,3 +113,41 @@ def spawn_ranks(world, target, extra_args=(), timeout=240):
                 p.kill()
     assert set(results) == set(range(world)), f"ranks that reported: {sorted(results)}"
     return results
+
+
+class _Dim3(ctypes.Structure):
+    _fields_ = [("x", ctypes.c_uint32), ("y", ctypes.c_uint32), ("z", ctypes.c_uint32)]
+
+
+class _KernelNode(ctypes.Structure):   # hipKernelNodeParams
+    _fields_ = [("block", _Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", _Dim3), ("params", ctypes.c_void_p), ("lds", ctypes.c_uint)]
+
+
+class _FuncAttributes(ctypes.Structure):   # hipFuncAttributes
+    _fields_ = [("binary_version", ctypes.c_int), ("cache_mode", ctypes.c_int), ("const_bytes", ctypes.c_size_t), ("local_bytes", ctypes.c_size_t),
+                ("max_dynamic_lds", ctypes.c_int), ("max_threads", ctypes.c_int), ("registers", ctypes.c_int), ("carveout", ctypes.c_int),
+                ("ptx_version", ctypes.c_int), ("shared_bytes", ctypes.c_size_t)]
+
+
+def launched_kernels(torch, run):
+    """Kernels that run() launches on the current stream, captured and not executed: (mangled name, grid x, bytes of dynamic LDS, the most its
+    attribute allows) of each."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        run()
+    raw, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+    out = []
+    for node in nodes:
+        kind, p, a = ctypes.c_int(-1), _KernelNode(), _FuncAttributes()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+        if kind.value != 0:
+            continue
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        assert hip.hipFuncGetAttributes(ctypes.byref(a), ctypes.c_void_p(p.func)) == 0
+        out.append((hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), None).decode(), p.grid.x, p.lds, a.max_dynamic_lds))
+    return out

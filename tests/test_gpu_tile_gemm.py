@@ -202,6 +202,30 @@ def test_iq_gemm_rows_outside_fp16(gpu, size):
     assert bool(((y.double() - x.double() @ w.T).abs() <= bound).all())
 
 
+def test_iq_prompt_lds_of_all_types(gpu):
+    """The types share a kernel and differ in the LDS they take.  What a launch sets the kernel's limit to is the same for all of them, or
+    a thread with one type could lower it between another's setting and its launch."""
+    vmx, torch = gpu
+    from tests.helpers import launched_kernels
+    from vllm_rust_amd._lib import check, lib
+    M, N, K = 256, 8192, 1024
+    x, y = torch.zeros((M, K), dtype=torch.bfloat16, device="cuda"), torch.empty((M, N), device="cuda")
+    ws = torch.empty(8 * N * K, dtype=torch.uint8, device="cuda")
+    seen = {}
+    for t in (22, 18, 21, 17):
+        raw = torch.zeros(vmx.iq_type_size(t) * N * K // 256, dtype=torch.uint8, device="cuda")
+        run = lambda: check(lib.vmx_iq_gemm_f32(t, raw.data_ptr(), x.data_ptr(), y.data_ptr(), M, N, K, ws.data_ptr(), ws.numel(),   # noqa: E731, B023
+                                                torch.cuda.current_stream().cuda_stream))
+        run()
+        torch.cuda.synchronize()
+        for name, _, lds, most in launched_kernels(torch, run):
+            if "iq_prompt_kernel" in name:
+                seen.setdefault(name, []).append((lds, most))
+    (of_types,) = seen.values()
+    assert len(of_types) == 4 and len({lds for lds, _ in of_types}) > 1
+    assert len({most for _, most in of_types}) == 1 and of_types[0][1] >= max(lds for lds, _ in of_types)
+
+
 class _Seg(C.Structure):
     _fields_ = [("w", C.c_void_p), ("ggml_type", C.c_int), ("n_out", C.c_int), ("y_off", C.c_int)]
 

@@ -416,7 +416,9 @@ int iqp_launch(IqpArgs p, int slices, hipStream_t st) {
     p.tiles = tiles * p.row_tiles;
     const int nsb = p.K / 256;
     p.per_slice = (nsb + slices - 1) / slices;
-    VMX_CHECK_HIP(hipFuncSetAttribute((const void *)iq_prompt_kernel<S, GEGLU>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+    // one kernel serves all types: what it may be given is the most that any of them takes, whichever thread asks
+    constexpr int most = std::max({iqp_lds<S, 17>(), iqp_lds<S, 18>(), iqp_lds<S, 21>(), iqp_lds<S, 22>()});
+    VMX_CHECK_HIP(hipFuncSetAttribute((const void *)iq_prompt_kernel<S, GEGLU>, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     hipLaunchKernelGGL((iq_prompt_kernel<S, GEGLU>), dim3(tg_grid(p.tiles), (nsb + p.per_slice - 1) / p.per_slice), dim3(IQP_THREADS), bytes, st, p);
     VMX_CHECK_LAUNCH("iq_prompt");
     return VMX_OK;
