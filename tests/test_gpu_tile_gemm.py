@@ -202,6 +202,22 @@ def test_iq_gemm_rows_outside_fp16(gpu, size):
     assert bool(((y.double() - x.double() @ w.T).abs() <= bound).all())
 
 
+# decoded inside the product, or dequantised first where that leaves less of the last round of tiles empty
+@pytest.mark.parametrize("M,N,K,inside", [(256, 30720, 3840, True), (2048, 30720, 3840, True), (1000, 13862, 3328, True), (2825, 13862, 3328, False),
+                                          (2825, 8192, 3840, False), (8192, 8192, 3840, True), (1000, 4096, 4096, False), (2047, 12288, 1024, False), (333, 3840, 15360, True)])
+def test_iq_prompt_or_dequantised(gpu, M, N, K, inside):
+    """Which of the two products a call takes, on 256 compute units."""
+    vmx, torch = gpu
+    from tests.helpers import launched_kernels
+    from vllm_rust_amd._lib import check, lib
+    raw = torch.zeros(vmx.iq_type_size(18) * N * K // 256, dtype=torch.uint8, device="cuda")
+    x, y = torch.zeros((M, K), dtype=torch.bfloat16, device="cuda"), torch.empty((M, N), device="cuda")
+    ws = torch.empty(4 * N * K + 4 * M * K, dtype=torch.uint8, device="cuda")
+    names = [name for name, *_ in launched_kernels(torch, lambda: check(lib.vmx_iq_gemm_f32(
+        18, raw.data_ptr(), x.data_ptr(), y.data_ptr(), M, N, K, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)))]
+    assert any("iq_prompt_kernel" in n for n in names) == inside
+
+
 def test_iq_prompt_lds_of_all_types(gpu):
     """The types share a kernel and differ in the LDS they take.  What a launch sets the kernel's limit to is the same for all of them, or
     a thread with one type could lower it between another's setting and its launch."""
