@@ -699,6 +699,32 @@ def test_other_sizes(gpu, dtype, name):
     want.check(feed(eng, "c", toks, [2]))
 
 
+# 16 heads over latents of 512 + 64: from 129 tokens a step on, the attention is not partitioned.  Prompts of lengths that leave groups of four tokens over two of them
+@pytest.mark.parametrize("window", [0, 40])
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 128)])
+def test_packed_prompts_with_wide_latents(gpu, window, dim, vdim):
+    """Three prompts in one step, and the rest of one behind a decoding row of another, against the oracle."""
+    from vllm_rust_amd._lib import lib
+    layers = [att_layer(heads=16, dim=dim, rot_dim=64, vdim=vdim, kv_rank=512, scale=0.05, mask=window, rot=rot(64, 1e4), ff=64) for _ in range(2)]
+    spec = small_spec(layers=layers, width=128)
+    model, eng, w = build(spec, "bfloat16", block_size=16, num_blocks=64, max_tokens=320)
+    toks = [tokens_for(spec, n, 3 + n) for n in (130, 71, 102)]
+    want = [Expected(spec, w, t, "bfloat16") for t in toks]
+    assert all(lib.vmx_latent_attention_workspace_bytes(t, 16, 512, window, 64, 16) == 0 for t in (303, 131))
+    lg, _, _ = eng.step([(str(i), t, list(range(len(t)))) for i, t in enumerate(toks)])
+    lg, at = lg.cpu().numpy(), 0
+    for t, e in zip(toks, want):
+        e.check(lg[at:at + len(t)], what=len(t))
+        at += len(t)
+    eng.finish("0")
+    eng.finish("2")
+    again = tokens_for(spec, 72, 3 + 71)
+    assert list(again[:71]) == list(toks[1])
+    lg, _, _ = eng.step([("1", again[71:], [0]), ("3", toks[0], list(range(130)))])
+    Expected(spec, w, again, "bfloat16").check(lg[:1].cpu().numpy(), rows=slice(71, 72))
+    want[0].check(lg[1:].cpu().numpy())
+
+
 def random_spec(rng):
     pick = lambda *a: a[int(rng.integers(0, len(a)))]   # noqa: E731
     layers = []

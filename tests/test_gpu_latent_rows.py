@@ -215,3 +215,48 @@ def test_neighbours_in_a_step(gpu, heads, window):
         mixed = -before % group   # tokens in the group with the other prompt's last ones
         assert torch.equal(got[mixed:], alone[mixed:])
         assert float((got[:mixed] - alone[:mixed]).abs().max() if mixed else 0.0) <= (2.0 ** -15 + 280 * 2.0 ** -23) * float(cache.abs().max())
+
+
+# (R, RD, contexts, new tokens, heads, window): row tiles that share their keys, that lie in several sequences (prompts' ends, decode steps), partitions and their
+# merge, and rows of other sizes
+@pytest.mark.parametrize("R,RD,contexts,new,heads,window,parts", [
+    (512, 64, [270], 270, 20, 0, False), (512, 64, [97, 66, 111], 111, 16, 33, False), (512, 64, [33] * 259, 1, 16, 0, False), (512, 64, [300, 301], 300, 5, 0, False),
+    (512, 64, [128, 129, 700], 1, 16, 0, True), (256, 32, [70, 41], 60, 16, 0, True), (96, 32, [90, 41], 90, 3, 0, True),
+])
+def test_bf16_queries_and_results(gpu, R, RD, contexts, new, heads, window, parts):
+    """Queries that are bf16 already, handed over as bf16 and as f32: the bf16 results are the f32 ones (which the tests above hold against float64)
+    rounded, bit by bit.  Nothing is written beside them."""
+    import ctypes as C
+    vmx, torch = gpu
+    from vllm_rust_amd._lib import check, lib
+    bs, scale = 16, 0.06
+    g = torch.Generator(device="cuda").manual_seed(sum(contexts) + heads + R)
+    n = len(contexts)
+    mb = (max(contexts) + bs - 1) // bs
+    bt = torch.randperm(n * mb, device="cuda", generator=g).to(torch.int32).view(n, mb)
+    cache = torch.randn((n * mb * bs, R + RD), device="cuda", generator=g).to(torch.bfloat16)
+    sid, pos = [], []
+    for b, c in enumerate(contexts):
+        k = min(new, c)
+        sid += [b] * k
+        pos += list(range(c - k, c))
+    pos[1] = -1                     # a row without keys
+    T = len(pos)
+    qa = torch.randn((T, heads, R), device="cuda", generator=g).to(torch.bfloat16)
+    qr = torch.randn((T, heads, RD), device="cuda", generator=g)
+    sink = torch.randn(heads, device="cuda", generator=g).to(torch.bfloat16)
+    ts, tp = (torch.tensor(v, device="cuda", dtype=torch.int32) for v in (sid, pos))
+    need = lib.vmx_latent_attention_workspace_bytes(T, heads, R, window, mb, bs)
+    assert (need > 0) == parts
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    got = {}
+    for io16, dt in ((0, torch.float32), (1, torch.bfloat16)):
+        q, held = qa.to(dt), torch.full((T + 2, heads, R), 7.0, dtype=dt, device="cuda")
+        p = lambda t: C.c_void_p(t.data_ptr())   # noqa: E731
+        check(lib.vmx_latent_attention_launch(p(held[1:]), p(q), io16, p(qr), p(cache), 1, p(bt), mb, p(ts), p(tp), p(sink), C.c_float(scale), window, T, heads, R, RD, bs,
+                                              p(ws), C.c_size_t(ws.numel()), None))
+        torch.cuda.synchronize()
+        assert bool((held[0] == 7.0).all()) and bool((held[T + 1] == 7.0).all())
+        got[io16] = held[1:T + 1]
+    assert bool((got[0][1] == 0).all()) and bool(got[0].isfinite().all())
+    assert torch.equal(got[1], got[0].to(torch.bfloat16))

@@ -42,14 +42,26 @@ def test_bf16_linear_tiles(gpu, M, N, K, out):
     assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all())
 
 
-# on 256 compute units, in this order: 64 x 128 tiles, 128 x 128 two a unit, 128 x 128 one a unit, 192 x 128 (rows and columns past the last whole
-# tile; whole tiles, whose bf16 results go out in pairs), 256 x 128 (the same two)
-@pytest.mark.parametrize("M,N,K", [(129, 12801, 128), (513, 11001, 320), (1023, 2049, 2048), (383, 12281, 1024), (384, 12288, 1024), (511, 12281, 2048),
-                                   (512, 12288, 2048)])
+_LINEAR_SHAPES = {"64 x 64": (2, 2, 1, 1, 5), "64 x 128": (2, 2, 1, 2, 3), "128 x 128, two a unit": (2, 2, 2, 2, 2), "128 x 128, one a unit": (2, 4, 2, 1, 4), "192 x 128": (2, 2, 3, 2, 3),
+                  "256 x 128": (4, 2, 2, 2, 3)}
+
+
+# every tile shape of 256 compute units; rows and columns past the last whole tile, and whole tiles, whose bf16 results go out in pairs
+@pytest.mark.parametrize("M,N,K,shape", [(100, 300, 64, "64 x 64"), (64, 64, 320, "64 x 64"), (129, 12801, 128, "64 x 128"), (128, 12800, 128, "64 x 128"),
+                                         (513, 11001, 320, "128 x 128, two a unit"), (1023, 2049, 2048, "128 x 128, one a unit"), (383, 12281, 1024, "192 x 128"),
+                                         (384, 12288, 1024, "192 x 128"), (511, 12281, 2048, "256 x 128"), (512, 12288, 2048, "256 x 128")])
 @pytest.mark.parametrize("out", ["f32", "bf16"])
-def test_bf16_linear_tile_shapes(gpu, M, N, K, out):
-    """As test_bf16_linear_tiles, the same bounds."""
+def test_bf16_linear_tile_shapes(gpu, M, N, K, shape, out):
+    """As test_bf16_linear_tiles, the same bounds; and the shape that the call launches is the one named."""
+    vmx, torch = gpu
+    from tests.helpers import launched_kernels
+    from vllm_rust_amd._lib import check, lib
     test_bf16_linear_tiles(gpu, M, N, K, out)
+    x, w = (torch.zeros((n, K), dtype=torch.bfloat16, device="cuda") for n in (M, N))
+    y = torch.empty((M, N), device="cuda", dtype=torch.float32 if out == "f32" else torch.bfloat16)
+    (name,) = [k for k, *_ in launched_kernels(torch, lambda: check(lib.vmx_linear_bf16w(
+        y.data_ptr(), 0 if out == "f32" else 1, x.data_ptr(), 1, w.data_ptr(), M, N, K, 0, torch.cuda.current_stream().cuda_stream)))]
+    assert "linear_tile_kernel" in name and "TgShapeI%sLb0E" % "".join("Li%dE" % v for v in _LINEAR_SHAPES[shape]) in name, name
 
 
 # f32 rows (64 x 128 tiles in two stages): rows and columns one below, at and one above a tile, one to many stages
@@ -73,6 +85,96 @@ def test_f32_row_linear_tiles(gpu, M, N, K, out):
         bound = bound + 2.0 ** -8 * ref.abs()
     assert bool(((y.double() - ref).abs() <= bound).all())
     assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all())
+
+
+class _Linear(C.Structure):   # VmxLinear
+    _fields_ = [("A", C.c_void_p), ("a_f32", C.c_int), ("lda", C.c_int64), ("W", C.c_void_p), ("w_sn", C.c_int64), ("w_sk", C.c_int64), ("C", C.c_void_p), ("c_f32", C.c_int),
+                ("ldc", C.c_int64), ("M", C.c_int), ("N", C.c_int), ("K", C.c_int), ("batch", C.c_int), ("a_bs", C.c_int64), ("w_bs", C.c_int64), ("c_bs", C.c_int64),
+                ("aux_bs", C.c_int64), ("row_ids", C.c_void_p), ("row_div", C.c_int), ("row_limit", C.c_int), ("block_expert", C.c_void_p), ("expert_stride", C.c_int64),
+                ("block_rows", C.c_int), ("total_rows", C.c_void_p), ("bias", C.c_void_p), ("bias_bs", C.c_int64), ("epilogue", C.c_int), ("aux", C.c_void_p), ("ldaux", C.c_int64),
+                ("aux_sn", C.c_int), ("silu_begin", C.c_int), ("silu_end", C.c_int), ("out_scale", C.c_float), ("exact", C.c_int)]
+
+
+def _launch_linear(torch, shape, **kw):
+    """One vmx_linear_launch, which must run as a linear_tile_kernel of that shape (None: of any)."""
+    from tests.helpers import launched_kernels
+    from vllm_rust_amd._lib import check, lib
+    given = dict(w_sk=1, batch=1, row_div=1, aux_sn=1, out_scale=1.0) | kw
+    p = _Linear(**{k: v.data_ptr() if hasattr(v, "data_ptr") else v for k, v in given.items()})
+    run = lambda: check(lib.vmx_linear_launch(C.byref(p), C.c_void_p(torch.cuda.current_stream().cuda_stream)))   # noqa: E731
+    (name,) = [k for k, *_ in launched_kernels(torch, run)]
+    assert "linear_tile_kernel" in name and (shape is None or "TgShapeI%sE" % shape in name), name
+    run()
+    torch.cuda.synchronize()
+
+
+_MUL_SIGMOID = 3   # VMX_EP_MUL_SIGMOID
+_F32_ROWS = "Li2ELi2ELi1ELi2ELi2ELb1E"
+
+
+# heads side by side in a wider row, as latent attention has them; whole 64 x 128 tiles and not; results in rows of an odd length (no pairs); the gate of a row and
+# head, or of every output
+@pytest.mark.parametrize("M,N,K,pad", [(70, 130, 128, 8), (128, 128, 64, 0), (128, 128, 64, 1), (17, 512, 192, 8)])
+@pytest.mark.parametrize("gate", [None, "head", "element"])
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("rows", ["f32", "bf16"])
+def test_batched_linear_tiles(gpu, M, N, K, pad, gate, out, rows):
+    """Against float64 on the rows rounded to bf16.  An f32 sum of K exact products is off by at most (K + 8) 2^-24 sum |x w|; a sigmoid and the
+    multiplication by it by a few units of 2^-24 of the result; a bf16 result by half an ulp more.  Nothing is written between the rows."""
+    vmx, torch = gpu
+    B = 3
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    lda, ldc = B * (K + 64) + 8, B * N + pad
+    x = torch.randn((M, lda), device="cuda", generator=g)
+    x = x if rows == "f32" else x.to(torch.bfloat16)
+    w = torch.randn((B, N, K), device="cuda", generator=g).to(torch.bfloat16)
+    aux = torch.randn((M, B * N), device="cuda", generator=g) * 2
+    y = torch.full((M, ldc), 7.0, device="cuda", dtype=torch.float32 if out == "f32" else torch.bfloat16)
+    gates = {} if gate is None else dict(epilogue=_MUL_SIGMOID, aux=aux, ldaux=B * N, aux_sn=0 if gate == "head" else 1, aux_bs=1 if gate == "head" else N)
+    _launch_linear(torch, _F32_ROWS if rows == "f32" else None, A=x, a_f32=rows == "f32", lda=lda, a_bs=K + 64, W=w, w_sn=K, w_bs=N * K, C=y, c_f32=out == "f32", ldc=ldc, c_bs=N,
+                   M=M, N=N, K=K, batch=B, **gates)
+    for b in range(B):
+        xr = x[:, b * (K + 64):b * (K + 64) + K].to(torch.bfloat16).double()
+        ref, size = xr @ w[b].double().T, xr.abs() @ w[b].double().abs().T
+        if gate:
+            f = torch.sigmoid(aux[:, b:b + 1] if gate == "head" else aux[:, b * N:(b + 1) * N]).double()
+            ref, size = ref * f, size * f
+        bound = (K + 8 + 16) * 2.0 ** -24 * size + (2.0 ** -8 * ref.abs() if out == "bf16" else 0.0)
+        assert bool(((y[:, b * N:(b + 1) * N].double() - ref).abs() <= bound).all()), b
+    assert bool((y[:, B * N:] == 7.0).all())
+
+
+# gathered rows, two outputs a source row, with ids that are padding (negative, past the limit); and the same in 64-row blocks of three experts, of which the last
+# lies past the count of rows
+@pytest.mark.parametrize("experts", [False, True])
+@pytest.mark.parametrize("N,K", [(130, 128), (256, 64)])
+@pytest.mark.parametrize("rows", ["f32", "bf16"])
+def test_gathered_linear_tiles(gpu, experts, N, K, rows):
+    """Against float64 as above; rows of padding and of blocks past the count stay as they were."""
+    vmx, torch = gpu
+    M, T = 256, 90
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    x = torch.randn((T, K + 8), device="cuda", generator=g)
+    x = x if rows == "f32" else x.to(torch.bfloat16)
+    w = torch.randn((3, N, K), device="cuda", generator=g).to(torch.bfloat16)
+    ids = torch.randint(0, 2 * T, (M,), device="cuda", generator=g, dtype=torch.int32)
+    ids[5::16] = -1
+    ids[70] = 2 * T
+    y = torch.full((M, N), 7.0, device="cuda")
+    of = torch.tensor([2, 0, 0, 1], dtype=torch.int32, device="cuda")
+    total = torch.tensor([192], dtype=torch.int32, device="cuda")
+    more = dict(block_expert=of, expert_stride=N * K, block_rows=64, total_rows=total) if experts else {}
+    _launch_linear(torch, _F32_ROWS if rows == "f32" else None, A=x, a_f32=rows == "f32", lda=K + 8, W=w, w_sn=K, C=y, c_f32=1, ldc=N, M=M, N=N, K=K, row_ids=ids, row_div=2, row_limit=2 * T,
+                   **more)
+    live = (ids >= 0) & (ids < 2 * T)
+    if experts:
+        live[192:] = False
+    xr = x[(ids.long().clamp(0, 2 * T - 1) // 2), :K].to(torch.bfloat16).double()
+    pick = (of.long() if experts else torch.zeros(4, dtype=torch.long, device="cuda")).repeat_interleave(64)
+    ref = torch.stack([xr[m] @ w[pick[m]].double().T for m in range(M)])
+    size = torch.stack([xr[m].abs() @ w[pick[m]].double().abs().T for m in range(M)])
+    assert bool(((y.double() - ref).abs() <= (K + 8) * 2.0 ** -24 * size)[live].all())
+    assert bool((y[~live] == 7.0).all())
 
 
 # rows around the 64- and 128-row tiles; columns around the 128-wide ones; K of one super-block, an odd number of them, and enough with
@@ -155,7 +257,7 @@ def test_iq_prompt_linear_short(gpu, M, N, K, sliced):
     assert n.value == (4 if sliced else 3)
 
 
-# raw blocks decoded inside the product: rows at and past every tile height; an odd number of super-blocks (block starts alternate between
+# raw blocks decoded inside the product (tiles of 64, 128 and 192 rows; every height by name in test_iq_prompt_tile_heights): an odd number of super-blocks (block starts alternate between
 # the halves of a dword along a row and from row to row) and an even one; columns past a tile; a weight that starts in the middle of a dword; room for
 # slices of k and none
 @pytest.mark.parametrize("M", [17, 64, 65, 129, 192, 256, 333])
@@ -246,7 +348,7 @@ class _Seg(C.Structure):
     _fields_ = [("w", C.c_void_p), ("ggml_type", C.c_int), ("n_out", C.c_int), ("y_off", C.c_int)]
 
 
-# three projections of three types as one product, none of whose widths is whole tiles; rows in one tile height and in two, in slices and in none
+# three projections of three types as one product, none of whose widths is whole tiles; in slices and in none
 @pytest.mark.parametrize("M", [33, 130, 300])
 @pytest.mark.parametrize("K,room", [(1280, 0), (4096, 64 << 20)])
 def test_iq_prompt_projections(gpu, M, K, room):
@@ -262,8 +364,7 @@ def test_iq_prompt_projections(gpu, M, K, room):
     segs = (_Seg * 3)(*[_Seg(r.data_ptr(), t, n, o) for r, t, n, o in zip(raws, types, widths, off)])
     y = torch.full((M, N + 3), 7.0, device="cuda")
     part = torch.empty(max(room, 1), dtype=torch.uint8, device="cuda")
-    check(lib._Z17vmx_iq_prompt_f32PK10VmxMmvqSegiPKtPfiilS4_mP12ihipStream_t(segs, 3, C.c_void_p(x.data_ptr()), C.c_void_p(y.data_ptr()), M, K, C.c_int64(N + 3),
-                                                                              C.c_void_p(part.data_ptr()), C.c_size_t(room), None))
+    check(lib.vmx_iq_prompt_f32(segs, 3, C.c_void_p(x.data_ptr()), C.c_void_p(y.data_ptr()), M, K, C.c_int64(N + 3), C.c_void_p(part.data_ptr()), C.c_size_t(room), None))
     torch.cuda.synchronize()
     w = torch.cat([vmx.iq_dequantize(t, r, n * K // 256).reshape(n, K).double() for r, t, n in zip(raws, types, widths)])
     bound = (264 + K // 256 + 8) * 2.0 ** -24 * (x.double().abs() @ w.abs().T)
@@ -271,12 +372,18 @@ def test_iq_prompt_projections(gpu, M, K, room):
     assert bool((y[:, N:] == 7.0).all())
 
 
-# gate columns below, at and past the 64 that a tile takes; rows in every tile height
+# gate columns below, at and past the 64 that a tile takes (tiles of 64 rows: too few columns for others)
 @pytest.mark.parametrize("M", [17, 65, 129, 192, 256])
 @pytest.mark.parametrize("ggml_type,inter,K", [(18, 40, 256), (21, 64, 512), (22, 200, 1280), (17, 130, 768)])
 def test_iq_prompt_geglu(gpu, M, ggml_type, inter, K):
     """act = bf16(bf16(gelu(gate)) * up), gate and up rounded to bf16, against float64 on the dequantised weights.  The f32 sums may fall on the
     other side of a bf16 rounding: one step (2^-8 relative) of gate and of up, and one of each product behind."""
+    err, by_gate, ref = _geglu(gpu, M, ggml_type, inter, K, 64)
+    assert bool((err <= 2.0 ** -8 * (by_gate + 3 * ref) + 2.0 ** -20).all())
+
+
+def _geglu(gpu, M, ggml_type, inter, K, height):
+    """|act - exact| of a product that must take tiles of that height, |d exact / d gate * gate| and |exact|."""
     vmx, torch = gpu
     from tests.helpers import random_iq_blocks
     from vllm_rust_amd._lib import check, lib
@@ -288,15 +395,64 @@ def test_iq_prompt_geglu(gpu, M, ggml_type, inter, K):
     guard = torch.full((M + 2, inter), 7.0, dtype=torch.float16, device="cuda")
     act = guard[1:M + 1]
     gate, up = [_Seg(r.data_ptr(), ggml_type, inter, 0) for r in raw]
-    check(lib._Z19vmx_iq_prompt_gegluRK10VmxMmvqSegS1_PKtPtiiP12ihipStream_t(C.byref(gate), C.byref(up), C.c_void_p(x.data_ptr()), C.c_void_p(act.data_ptr()), M, K, None))
+    run = lambda: check(lib.vmx_iq_prompt_geglu(C.byref(gate), C.byref(up), C.c_void_p(x.data_ptr()), C.c_void_p(act.data_ptr()), M, K,   # noqa: E731
+                                                C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert _iq_tile(torch, run) == (height, True)
+    run()
     torch.cuda.synchronize()
     gate, up = [(x.double() @ m.T).to(torch.bfloat16).double() for m in w]
     cdf = 0.5 * (1 + torch.erf(gate / 2 ** 0.5))
     slope = cdf + gate * torch.exp(-gate * gate / 2) / (2 * np.pi) ** 0.5
     ref = gate * cdf * up
-    bound = 2.0 ** -8 * ((slope * gate * up).abs() + 3 * ref.abs()) + 2.0 ** -20
-    assert bool(((act.double() - ref).abs() <= bound).all())
     assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all())
+    return (act.double() - ref).abs(), (slope * gate * up).abs(), ref.abs()
+
+
+_IQ_SHAPES = {64: (2, 4, 1, 1), 128: (4, 2, 1, 2), 192: (2, 4, 3, 1), 256: (4, 2, 2, 2)}
+
+
+def _iq_tile(torch, run):
+    """Rows of the tile of the one iq_prompt_kernel that run() launches, and whether its epilogue is GeGLU."""
+    from tests.helpers import launched_kernels
+    (name,) = [k for k, *_ in launched_kernels(torch, run) if "iq_prompt_kernel" in k]
+    (rows,) = [r for r, s in _IQ_SHAPES.items() if "IqpShapeI%sEE" % "".join("Li%dE" % v for v in s) in name]
+    return rows, "EELb1EE" in name
+
+
+# every height with columns for more than half of 256 units (129 .. 131 tiles), its last rows missing or not, and with its results in slices
+@pytest.mark.parametrize("ggml_type", [17, 18, 21, 22])
+@pytest.mark.parametrize("M,N,K,room,height", [(50, 16700, 512, 0, 64), (64, 16640, 512, 0, 64), (127, 16700, 512, 0, 128), (128, 16640, 768, 0, 128), (190, 16700, 512, 0, 192), (192, 16640, 768, 0, 192),
+                                               (250, 16700, 512, 0, 256), (256, 16640, 768, 0, 256), (1000, 1060, 8192, 64 << 20, 256), (290, 1060, 8192, 64 << 20, 192)])
+def test_iq_prompt_tile_heights(gpu, ggml_type, M, N, K, room, height):
+    """Against float64 on the dequantised weight, bounds as in test_iq_prompt_linear_tiles; and the tile is of the height named."""
+    vmx, torch = gpu
+    from tests.helpers import random_iq_blocks
+    from vllm_rust_amd._lib import check, lib
+    raw = torch.from_numpy(np.ascontiguousarray(random_iq_blocks(np.random.default_rng(N + K), vmx.iq_type_size(ggml_type), N * K // 256))).reshape(-1).cuda()
+    x = torch.randn((M, K), device="cuda", generator=torch.Generator(device="cuda").manual_seed(M + N)).to(torch.float16)
+    seg = (_Seg * 1)(_Seg(raw.data_ptr(), ggml_type, N, 0))
+    guard = torch.full((M + 2, N), 7.0, device="cuda")
+    y = guard[1:M + 1]
+    part = torch.empty(max(room, 1), dtype=torch.uint8, device="cuda")
+    run = lambda: check(lib.vmx_iq_prompt_f32(seg, 1, C.c_void_p(x.data_ptr()), C.c_void_p(y.data_ptr()), M, K, C.c_int64(N), C.c_void_p(part.data_ptr()),   # noqa: E731
+                                              C.c_size_t(room), C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert _iq_tile(torch, run) == (height, False)
+    run()
+    torch.cuda.synchronize()
+    w = vmx.iq_dequantize(ggml_type, raw, N * K // 256).reshape(N, K).double()
+    bound = (264 + K // 256 + 8) * 2.0 ** -24 * (x.double().abs() @ w.abs().T)
+    assert bool(((y.double() - x.double() @ w.T).abs() <= bound).all())
+    assert bool((guard[0] == 7.0).all()) and bool((guard[M + 1] == 7.0).all())
+
+
+# the same with the GeGLU epilogue: 130 tiles of 64 gate and 64 up columns
+@pytest.mark.parametrize("ggml_type", [17, 18, 21, 22])
+@pytest.mark.parametrize("M,inter,K,height", [(64, 8300, 512, 64), (127, 8300, 512, 128), (128, 8320, 768, 128), (190, 8300, 512, 192), (192, 8320, 768, 192), (250, 8300, 512, 256), (256, 8320, 768, 256)])
+def test_iq_prompt_geglu_tile_heights(gpu, ggml_type, M, inter, K, height):
+    """As test_iq_prompt_geglu.  Among millions of results some have a gate or an up whose f32 sum falls on the other side of a rounding where the step is
+    widest, 2^-7 of the value (8 bits from 1.0 on); gelu and the product behind are rounded to the nearest, 2^-8 each; 2^-6 of all that for their products."""
+    err, by_gate, ref = _geglu(gpu, M, ggml_type, inter, K, height)
+    assert bool((err <= (1 + 2.0 ** -6) * 2.0 ** -7 * (by_gate + 2 * ref) + 2.0 ** -20).all())
 
 
 # 256-column blocks; one k-block, odd numbers of them (17; 33 in slices) and groups wider than a

@@ -190,10 +190,10 @@ int vmx_int_gemm_geglu(const uint16_t *a16, const void *workspace, uint16_t *act
 int vmx_int_slices(const float *part, float *y, int slices, int M, int N, int64_t ldy, hipStream_t st);   // y = part [slices][M][N] in slice order
 // iq_prompt.hip: the same product with the raw blocks decoded inside it (a segment's `w` = its raw blocks)
 bool vmx_iq_prompt_ok(const VmxMmvqSeg *segs, int nseg, int M, int K);
-int vmx_iq_prompt_f32(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st);
+extern "C" int vmx_iq_prompt_f32(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st);
 int vmx_iq_prompt_slices(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st,
                          int *left);
-int vmx_iq_prompt_geglu(const VmxMmvqSeg &gate, const VmxMmvqSeg &up, const uint16_t *a16, uint16_t *act16, int M, int K, hipStream_t st);
+extern "C" int vmx_iq_prompt_geglu(const VmxMmvqSeg &gate, const VmxMmvqSeg &up, const uint16_t *a16, uint16_t *act16, int M, int K, hipStream_t st);
 int vmx_dense_gemv_launch(uint16_t *y, const uint16_t *x, const uint16_t *W, const uint16_t *bias, int M, int N, int K, hipStream_t st,
                           int f16 = 0);   // f16: x, W, bias and y hold fp16 (same f32 accumulation, fp16 matrix / dot instructions)
 // bf16 matrix-core GEMM y = bf16(bf16(x @ W^T) + bias), W [N, K] bf16 (fp8_kernels.hip)
@@ -234,14 +234,14 @@ struct VmxLinear {
     float out_scale = 1.0f;            // what is stored or added is this times the epilogue's value (C += out_scale * v)
     int exact = 0;                     // 1: multiply in f32 on the vector ALU even where the matrix cores could take bf16 operands
 };
-int vmx_linear_launch(const VmxLinear &p, hipStream_t st);
+extern "C" int vmx_linear_launch(const VmxLinear &p, hipStream_t st);
 
 // latent_attn.hip: out[h][r][d] = in[h][d][r], the key up-projection turned for q_abs = U_h^T q_h
 int vmx_latent_transpose_heads(uint16_t *out, const uint16_t *in, int heads, int dim, int kv_rank, hipStream_t st);
 // vmx_latent_attention with latent-space queries and results both f32 or (io_bf16, where vmx_latent_attention_takes_bf16) both bf16: the kernel rounds its
 // queries to bf16 anyway, so a caller whose next product rounds its rows as well gets the same bits with half the traffic.
 bool vmx_latent_attention_takes_bf16(int cache_dtype, int kv_rank, int rot_dim);
-int vmx_latent_attention_launch(void *out_latent, const void *q_abs, int io_bf16, const float *q_rot, const void *cache, int cache_dtype,
+extern "C" int vmx_latent_attention_launch(void *out_latent, const void *q_abs, int io_bf16, const float *q_rot, const void *cache, int cache_dtype,
                                 const int32_t *block_tables, int max_blocks_per_seq, const int32_t *seq_ids, const int32_t *positions,
                                 const uint16_t *sink_bf16, float scale, int window, int tokens, int heads, int kv_rank, int rot_dim, int block_size,
                                 void *workspace, size_t workspace_bytes, hipStream_t st);
