@@ -140,7 +140,8 @@ __global__ __launch_bounds__(64) void exl3_out_had_kernel(const float *__restric
 // LDS holds each tile's bit stream word-reversed: stream word i at slot W-1-i, plus a copy of word W-1 at slot W, so that
 // the <= 24-bit window pair of weights (t, t+1) is always inside the two consecutive slots {s, s+1} = stream words
 // {i, i-1 (cyclic)}: one two-dword LDS read and one funnel shift per pair, with per-lane slot/shift constants computed
-// once.  (The first version moved words between lanes with 16 wave permutes per k-step.)
+// once (4 bits: two reads for a lane's four pairs, see the kernel's step).  (The first version moved words between lanes with 16 wave permutes per k-step.)
+
 // Decoded weights of four windows, each the low 16 bits of w[i] (whatever lies above them is not looked at), as two packed fp16 pairs (even window low).
 // A 32-bit product is quarter rate on CDNA, so w * C + ADD mod 2^32 is w * (C & 0xFFFF) + ADD in 32 bits and then w * (C >> 16) added to the upper
 // half alone: two full-rate instructions that read half registers, so that a window needs no mask either (two 24-bit products took three and a mask).

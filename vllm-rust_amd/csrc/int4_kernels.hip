@@ -1268,11 +1268,11 @@ __global__ __launch_bounds__(256) void int4_gemm_tiled_kernel(const uint4 *__res
 //     either sign: the instruction cuts small products off towards zero beside a large accumulator, which with parts of one sign adds up.  bf16 results that differ from the rounded exact ones: 0.8e-4 .. 2.3e-4 of all
 //     (4096 and 12288 deep, rows of mean 0, 1 and 5), 2.0e-4 .. 3.4e-4 with the term of two-part factors on the scaled result a block later;
 //   * the scales of a finished k-block are applied between the first products of the next one.
-// What is left: matrix cores busy 0.59 of the time at 1.94 GHz and the vector ALU (unpacking 128, scales 64 of 250 instructions a k-block) about as long; the two
-// waves of a SIMD hardly overlap them.  One wave a SIMD with 96 rows of accumulators 570 us where this takes 385 (an instruction every 4.5 clocks is
+// What is left (gate|up of a 2048-token prompt): matrix cores busy 0.60 of the clocks and vector instructions (unpacking 128, scales 64 of 250 a k-block) 0.54, at 1.8 to
+// 2.0 GHz; the two waves of a SIMD hardly overlap them.  One wave a SIMD with 96 rows of accumulators 570 us where this takes 385 (an instruction every 4.5 clocks is
 // what one wave issues); clusters of four products behind the unpacking, with or without a raised priority, 1 % slower than one by one.
 // us against the form before (one pair of column tiles after the other, so that every fragment of x was read twice; everything waited for at
-// the block's head), rows x columns x depth, weights in HBM: 2048 x 24576 x 4096 419 -> 385 (1070 TFLOP/s), 2048 x 6144 x 4096 109 -> 102, 333 x 24576 x 4096 106 -> 100,
+// the block's head), rows x columns x depth, each launch alone, weights in HBM: 2048 x 24576 x 4096 419 -> 385 (1070 TFLOP/s; 394 .. 427 inside a prompt pass, by the clock), 2048 x 6144 x 4096 109 -> 102, 333 x 24576 x 4096 106 -> 100,
 // 8 experts of 64 rows x 28672 x 4096 230 -> 211, x 4096 x 14336 125 -> 106.  N % 256 == 0.
 template <bool GLU, bool GROUPED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void int4_gemm_prompt_kernel(
@@ -1865,13 +1865,14 @@ static void launch_tiled(const uint4 *W, const uint32_t *SZ, const uint16_t *x, 
 int vmx_int4_splits(int N, int K) { return plan_gemm(N, K).splits; }
 
 // Slices of k for a product of M rows on the prompt-shaped kernel, at most the plan's: the count with the least estimated time.
-//   * a k-block takes a compute unit that holds one workgroup 1.15 us and one that holds two 1.95, so w workgroups a unit cost what 1.7 (w / 2) + w % 2
+//   * a k-block takes a compute unit that holds one workgroup 1.15 us and one that holds two 1.95 (1.0 .. 1.13 and 1.97 .. 2.1 in the calls below), so w workgroups a unit cost what 1.7 (w / 2) + w % 2
 //     cost alone;
 //   * a slice is M N f32 written and read again, at 4.5 TB/s.  `own_pass`: the slices are added in a pass of their own (3 us), and one
 //     slice is stored as bf16 by the product itself; else the reader of the rows adds them, one slice as well.
-// Whole call in us with 1 / 2 / 3 / 4 slices, the taken one last:  4096 x 4096, 200 rows 39 / 29 / 25 / 24: 4; 333 rows 40 / 33 / 35 / 34: 2; 512 rows
-// 42 / 34 / 35 / 38: 2; 1024 rows 44 / 51 / 56 / 59: 1;  4096 x 12288, 333 rows 112 / 66 / 68: 2; 640 rows 112 / 98 / 79: 3; 800 rows 113 / 105 / 113: 2; 2048 rows
-// 203 / 225 / 232: 1;  2048 x 4096, 640 rows 42 / 32 / 29 / 33: 3;  6144 x 4096, 256 rows 40 / 33: 2; 640 rows 43 / 50: 1; 2048 rows 108 / 137: 1.
+// Whole call in us with 1 / 2 / 3 / 4 slices, the taken one last:  4096 x 4096, 200 rows 36 / 28 / 25 / 25: 4; 333 rows 36 / 31 / 34 / 34: 2; 512 rows
+// 36 / 32 / 34 / 36: 2; 1024 rows 39 / 49 / 55 / 58: 1;  4096 x 12288, 333 rows 95 / 59 / 64: 2; 640 rows 97 / 91 / 75: 3; 800 rows 97 / 98 / 107: 2; 2048 rows
+// 189 / 212 / 219: 1;  2048 x 4096, 640 rows 36 / 30 / 27 / 32: 3;  6144 x 4096, 256 rows 36 / 31: 2; 640 rows 38 / 48: 1; 2048 rows 100 / 131: 1.  Over 140 shapes of
+// 49 .. 2048 rows the taken count is within 4 % of the best but for eight, five of them 2048 deep (2048 x 2048, 800 rows 22 / 25 / 28 / 30: 2).
 static int prompt_slices(int M, int N, int K, bool own_pass) {
     const int plan = plan_gemm(N, K).splits, kblocks = K / KB, cus = vmx_num_cus();
     if (plan == 1 || !tiled_ok(M, N, K) || !tiled_wide_ok(M, N, K)) return plan;

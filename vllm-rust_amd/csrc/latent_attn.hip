@@ -261,13 +261,11 @@ typedef __attribute__((address_space(3))) uint16_t la_lds;
 typedef short la_s16x4 __attribute__((ext_vector_type(4)));
 typedef short la_s16x8 __attribute__((ext_vector_type(8)));
 
-// WHOLE > 0: rows of exactly 32 KSMAX values with 64 DTW latents (512 + 64).  Every size is then a constant, which leaves the registers for
-// requesting a tile's rows while the one before it is worked on, and with WHOLE = 2 (inside latent_attn_shared_kernel) for two workgroups per compute unit: 1500
-// tokens of 16 heads 270 -> 178 us.  Two workgroups cap the registers at 256, and 52 more (212 bytes a lane of scratch memory) are spilled while the
-// queries and rows are set up and read back there and behind the loop; the loop over key tiles itself touches no scratch.  A partitioned
-// launch (decode steps: one workgroup per compute unit, a tile or two each) is mostly setup, so it has WHOLE = 1 without the cap and without
-// spills: 16 rows of 1000 tokens 22.3 -> 17.9 us (WHOLE = 2: 29.7).  Other sizes (0) request a tile's rows when its turn comes.
-template <int KSMAX, int DTW, int WHOLE>
+// WHOLE: rows of exactly 32 KSMAX values with 64 DTW latents (512 + 64).  Every size is then a constant, which leaves the registers for
+// requesting a tile's rows while the one before it is worked on; other sizes request a tile's rows when its turn comes.  A partitioned
+// launch (decode steps: one workgroup per compute unit, a tile or two each) is mostly setup, so latent_attn_mfma_kernel has no cap on its registers and no
+// spills: 16 rows of 1000 tokens 22.3 -> 17.9 us (29.7 with the registers of two workgroups a compute unit, which latent_attn_shared_kernel has).
+template <int KSMAX, int DTW, bool WHOLE>
 __device__ __forceinline__ void latent_row_tile(const LatentAttnArgs &a, int tb, int hg, int part) {
     extern __shared__ __align__(256) unsigned char la_smem[];
     const int R = WHOLE ? 64 * DTW : a.R, RW = WHOLE ? 32 * KSMAX : a.R + a.rd;
@@ -459,7 +457,7 @@ __device__ __forceinline__ void latent_row_tile(const LatentAttnArgs &a, int tb,
     }
 }
 
-template <int KSMAX, int DTW, int WHOLE>
+template <int KSMAX, int DTW, bool WHOLE>
 __global__ __launch_bounds__(256, 1) void latent_attn_mfma_kernel(const LatentAttnArgs a) {
     latent_row_tile<KSMAX, DTW, WHOLE>(a, blockIdx.x / a.NHG, blockIdx.x % a.NHG, blockIdx.y);
 }
@@ -474,9 +472,10 @@ __global__ __launch_bounds__(256, 1) void latent_attn_mfma_kernel(const LatentAt
 //     the weights go straight into the second product O^T = C^T P^T, whose k slots are assigned to the keys a lane already holds;
 //   * the 128 accumulators are rescaled only on tiles where a row's maximum grew.  (Leaving it behind by up to 8 saves little and costs precision: the largest
 //     weight is then no longer 1, which its two bf16 halves hold exactly.)
-// us, 16 heads, one row tile a workgroup -> this: 600 + 500 + 400 tokens packed 177 -> 68, 1000 tokens 175 -> 86, 4000 tokens 1667 -> 499, 130 tokens 27 -> 19;
-// 32 heads, 500 + 400 tokens 185 -> 62; 3 heads, 700 + 300 tokens 68 -> 58; decode steps of 300 sequences 117 -> 110.  Error against 64 bits as before (1.2e-6).
-// The queries (72 registers) and the accumulators (128) leave two waves a SIMD.  Blocks are numbered from the last token backwards: later tokens have
+// us, 16 heads, one row tile a workgroup -> this: 600 + 500 + 400 tokens packed 177 -> 70, 599 + 501 + 401 173 -> 80, 4000 tokens 1654 -> 466, 130 tokens 29 -> 22, 1500 tokens with a
+// window of 200 137 -> 49; 3 heads, 700 + 300 tokens 71 -> 63; 300 decode rows of 700 keys 97 -> 101.  (1 to 4 % of it are the zeros for other tokens' keys.)  Error against 64 bits as before (1.2e-6).
+// The queries (72 registers) and the accumulators (128) leave two waves a SIMD, which cap the registers at 256; 85 more (332 bytes a lane of scratch memory) are
+// spilled where queries and rows are set up and read back behind the loops; neither loop over key tiles touches scratch.  Blocks are numbered from the last token backwards: later tokens have
 // more keys.  A group of row tiles over several sequences (a large decode step) has no keys to share: its tiles go the way above, one a workgroup,
 // the first by the group's own workgroup and the others by those behind the groups.
 __device__ __forceinline__ int la_swizzle(int r) { return ((((r >> 2) ^ (r >> 3)) & 1) << 2) | (r & 2) | ((r >> 3) & 1); }
@@ -500,7 +499,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_shared_kernel(const Latent
     const int t0 = group * 4 * a.TPT, n = min(4 * a.TPT, a.T - t0);   // at most 64 tokens
     const int seq = a.seq_ids[t0];
     if (!__all(a.seq_ids[t0 + min(lane, n - 1)] == seq)) {
-        if (4 * group + which < row_tiles) latent_row_tile<KS, R / 64, 2>(a, 4 * group + which, hg, 0);
+        if (4 * group + which < row_tiles) latent_row_tile<KS, R / 64, true>(a, 4 * group + which, hg, 0);
         return;
     }
     if (!leader) return;
@@ -778,14 +777,14 @@ int vmx_latent_attention_launch(void *out_latent, const void *q_abs, int io_bf16
         const size_t lds = ((size_t)LA_KT * ((small ? 128 : 512) + LA_PAD) + 2 * 16 * LA_LD) * 2 + (64 + 64) * 4;
         static_assert(2 * LS_TILE + LS_ZEROS <= (LA_KT * (512 + LA_PAD) + 2 * 16 * LA_LD) * 2 + (64 + 64) * 4, "the shared form fits the row tiles' memory");
         const bool whole = kv_rank == 512 && rot_dim == 64;
-        const void *fn = small              ? (const void *)latent_attn_mfma_kernel<5, 2, 0>
-                         : !whole           ? (const void *)latent_attn_mfma_kernel<18, 8, 0>
-                         : a.NP > 1         ? (const void *)latent_attn_mfma_kernel<18, 8, 1>
+        const void *fn = small              ? (const void *)latent_attn_mfma_kernel<5, 2, false>
+                         : !whole           ? (const void *)latent_attn_mfma_kernel<18, 8, false>
+                         : a.NP > 1         ? (const void *)latent_attn_mfma_kernel<18, 8, true>
                                             : (const void *)latent_attn_shared_kernel;
         if (lds > 64 * 1024) VMX_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        if (small) hipLaunchKernelGGL((latent_attn_mfma_kernel<5, 2, 0>), grid, dim3(256), lds, st, a);
-        else if (!whole) hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8, 0>), grid, dim3(256), lds, st, a);
-        else if (a.NP > 1) hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8, 1>), grid, dim3(256), lds, st, a);
+        if (small) hipLaunchKernelGGL((latent_attn_mfma_kernel<5, 2, false>), grid, dim3(256), lds, st, a);
+        else if (!whole) hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8, false>), grid, dim3(256), lds, st, a);
+        else if (a.NP > 1) hipLaunchKernelGGL((latent_attn_mfma_kernel<18, 8, true>), grid, dim3(256), lds, st, a);
         else hipLaunchKernelGGL(latent_attn_shared_kernel, dim3((unsigned)(((tokens + a.TPT - 1) / a.TPT + 3) / 4 * 4 * a.NHG)), dim3(256), lds, st, a);
         VMX_CHECK_LAUNCH("latent_attention (matrix cores)");
         if (a.NP > 1) {

@@ -8,8 +8,9 @@
 //   * the requests are issued by an instruction the compiler does not track (tg_request_1k), because behind one that it does it
 //     makes every LDS read wait for all requests under way, the other stage's included.  The waits are written out instead;
 //   * a request occupies the address path of the compute unit for 16 clocks and a wave that issues several in a row stands still while the
-//     path is busy, its products included.  tg_product therefore spreads the requests of the stage two ahead between the products of the
-//     stage in use (three stages in LDS), and reads a stage's first fragments under the last products of the one before it.  Against all requests at the
+//     path is busy, its products included.  In shapes of three or more stages tg_product therefore spreads the requests of the stage STAGES - 1 ahead between
+//     the products of the stage in use, and reads a stage's first fragments under the last products of the one before it.  (Two stages: two workgroups a
+//     compute unit, of which one multiplies while the other issues.)  Against all requests at the
 //     head of a stage, bf16, rows x columns x depth: 128 x 128 tiles 1500 x 2048 x 6144 51 -> 43 us (727 -> 889 TFLOP/s), 256 x 128 tiles 2048 x 24576 x
 //     4096 404 -> 369 us (1116 TFLOP/s; products alone, no memory: 1550 on random numbers, where the clock falls to 1.6 GHz);
 //   * tiles are numbered row-fastest and dealt to the eight XCDs in contiguous runs (workgroup i runs on XCD i % 8), so the rows of a
