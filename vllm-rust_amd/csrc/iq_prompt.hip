@@ -465,33 +465,41 @@ int iqp_launch_rows(const IqpArgs &p, const IqpPlan &plan, hipStream_t st) {
 
 }  // namespace
 
-// Estimated ns of the other way on 128 x 128 tiles, two a compute unit: 2.4 bytes a weight at 4.3 TB/s and a launch, then rounds of 1080 ns a 64-deep step (1280 in
-// products of 280 steps and more, under which the clock falls; 650 with at most one tile a unit)
-static int64_t dequantised_ns(int M, int64_t N, int K) {
-    const int64_t tiles = (M + 127) / 128 * ((N + 127) / 128), places = 2 * vmx_num_cus(), steps = K / 64;
-    const int64_t full = steps * (tiles * steps > 280 * places ? 1280 : 1080), rounds = tiles / places, rest = tiles % places;
-    const int64_t last = rest == 0 ? 0 : rounds == 0 ? full * (4 * places + rest) / (5 * places) : full * (2 * places + 3 * rest) / (5 * places);
-    return 4000 + N * K * 24 / 43000 + (tiles <= places / 2 ? steps * 650 : rounds * full + last) + M * N * 4 / 18400;
-}
-
 // Types with the integer form, operands inside 32-bit byte offsets, blocks at even addresses; and where the other way (vmx_iq_dequant_int, then
 // vmx_int_gemm_f32) is not as fast.  IQ3_XXS with the rows' conversion, that way / this one in us:  65 x 30720 x 3840 118 / 46, 256 162 / 76, 600 250 / 195,
 // 2048 655 / 515;  200 x 3840 x 15360 75 / 52, 1500 231 / 208;  65 x 8192 x 3840 39 / 23, 2048 135 / 136;  65 x 2048 x 4096 31 / 20, 1000 41 / 40, 2048
 // 59 / 63.  Of fewer than 8 M weights the other way writes and reads little and both are a handful of short launches: 65 x 512 x 2048 15 / 13, 400 x
-// 1024 x 1024 16 / 15, 800 x 2048 x 2048 28.3 / 28.5, 800 x 512 x 8192 31 / 41.  With 128 x 128 tiles for four units of
-// five the dequantised weight costs little and the other way's smaller tiles leave less of the last round empty, so the estimates decide (IQ3 codebooks take 2 % more
-// than they say).  IQ3_XXS:  1000 x 4096 x 4096 62 / 65 .. 68, 1500 79 / 75;  1000 x 13862 x 3328 134 / 132, 2047 243 / 264, 2825 341 / 406, 4096 503 /
-// 477;  2047 x 12288 x 1024 79 / 85;  2825 x 8192 x 3840 217 / 233, 8192 673 / 639.
+// 1024 x 1024 16 / 15, 800 x 2048 x 2048 28.3 / 28.5, 800 x 512 x 8192 31 / 41.
 bool vmx_iq_prompt_ok(const VmxMmvqSeg *segs, int nseg, int M, int K) {
-    int64_t total = 0, tiles = 0, percent = 100;
+    int64_t total = 0;
     for (int i = 0; i < nseg; i++) {
         if (!vmx_iq_int_form_ok(segs[i].ggml_type) || ((uintptr_t)segs[i].w & 1) || (int64_t)segs[i].n_out * (K / 256) * 128 >= (int64_t)1 << 32) return false;
-        total += segs[i].n_out, tiles += (segs[i].n_out + IQP_BN - 1) / IQP_BN;
-        if (segs[i].ggml_type == 18 || segs[i].ggml_type == 21) percent = 98;
+        total += segs[i].n_out;
     }
-    if ((int64_t)M * K * 2 >= (int64_t)1 << 32 || total * K < (M < 2048 ? 8 << 20 : 24 << 20)) return false;
-    if (5 * ((M + 127) / 128 * tiles) < 4 * vmx_num_cus()) return true;
-    return 100 * (iqp_plan((int)tiles, M, (int)total, K / 256, 1).ns + M * total * 4 / 9200) <= percent * dequantised_ns(M, total, K);
+    return (int64_t)M * K * 2 < (int64_t)1 << 32 && total * K >= (M < 2048 ? 8 << 20 : 24 << 20);
+}
+
+// Estimated ns of the other way on 128 x 128 tiles, two a compute unit: 2.4 bytes a weight at 4.3 TB/s (3.4 where 16 bits a weight are more than the caches
+// keep) and a launch, then rounds of 1080 ns a 64-deep step (1280 in products of 280 steps and more, under which the clock falls; 700 with at most one tile a unit)
+static int64_t dequantised_ns(int M, int64_t N, int K) {
+    const int64_t tiles = (M + 127) / 128 * ((N + 127) / 128), places = 2 * vmx_num_cus(), steps = K / 64;
+    const int64_t full = steps * (tiles * steps > 280 * places ? 1280 : 1080), rounds = tiles / places, rest = tiles % places;
+    const int64_t last = rest == 0 ? 0 : rounds == 0 ? full * (4 * places + rest) / (5 * places) : full * (2 * places + 3 * rest) / (5 * places);
+    return 4000 + N * K * (N * K > 64 << 20 ? 34 : 24) / 43000 + (tiles <= places / 2 ? steps * 700 : rounds * full + last) + M * N * 4 / 18400;
+}
+
+// vmx_iq_prompt_ok for a product that is called by itself.  With 128 x 128 tiles for four units of five the dequantised weight costs little and the other way's smaller
+// tiles leave less of the last round empty, so the estimates decide (IQ3 codebooks take 4 % more than they say).  IQ3_XXS, weights out of HBM, that way / this one in us:  850 x
+// 9216 x 3840 94 / 120, 2000 194 / 216;  1000 x 13862 x 3328 140 / 139, 2400 296 / 347;  1000 x 4096 x 4096 63 / 68, 1500 79 / 76;  2000 x 10240 x 5120 260 / 291;  but 1000 x
+// 30720 x 3840 374 / 292, 1000 x 3840 x 15360 173 / 162.  Of 330 calls of 256 .. 4000 rows the estimates lose 0.4 % in the mean against the better way, always this way 1.5 %, always the
+// other 10 %.  A model's prompt, whose norms add the slices, is faster without them: Gemma-4-12B (12 layers), 1000 tokens 8.57 ms, with the estimates 9.13; 2000 16.3 / 17.1.
+bool vmx_iq_prompt_alone_ok(const VmxMmvqSeg &seg, int M, int K) {
+    if (!vmx_iq_prompt_ok(&seg, 1, M, K)) return false;
+    const int N = seg.n_out, tiles = (N + IQP_BN - 1) / IQP_BN;
+    if (5 * ((int64_t)(M + 127) / 128 * tiles) < 4 * vmx_num_cus()) return true;
+    const int64_t slices = (int64_t)(vmx_int_gemm_part_bytes() / ((size_t)M * N * 4));   // as many as the public workspace has room for
+    const int64_t inside = iqp_plan(tiles, M, N, K / 256, slices).ns + (int64_t)M * N * 4 / 9200;
+    return 100 * inside <= (seg.ggml_type == 18 || seg.ggml_type == 21 ? 96 : 100) * dequantised_ns(M, N, K);
 }
 
 // y[:, y_off of a segment ..] (f32, rows ldy apart) = a16 [M][K] times the segments' raw blocks, one product.  The segments' columns lie one behind the

@@ -412,7 +412,7 @@ extern "C" int vmx_iq_gemm_f32(int ggml_type, const void *blocks, const uint16_t
     // Activations go to fp16 (which saturates and loses small values) only where the workspace has always allowed it, whichever of the two products then runs
     const bool int_form = vmx_iq_int_form_ok(ggml_type) && workspace_bytes >= vmx_iq_gemm_int_workspace(m, n_out, n_in) && vmx_int_gemm_ok(m, n_out, n_in);
     const VmxMmvqSeg seg = {blocks, ggml_type, n_out, 0};
-    if (int_form && vmx_iq_prompt_ok(&seg, 1, m, n_in)) {   // decoded inside the product: the workspace holds the rows, then slice sums
+    if (int_form && vmx_iq_prompt_alone_ok(seg, m, n_in)) {   // decoded inside the product: the workspace holds the rows, then slice sums
         const size_t rows = ((size_t)m * n_in * 2 + 255) & ~(size_t)255;   // fewer than the weights' integer form takes, besides these rows
         if (int rc = vmx_bf16_rows_to_f16(x, (uint16_t *)workspace, (int64_t)m * n_in, st)) return rc;
         return vmx_iq_prompt_f32(&seg, 1, (const uint16_t *)workspace, y, m, n_in, n_out, (float *)((char *)workspace + rows), workspace_bytes - rows, st);

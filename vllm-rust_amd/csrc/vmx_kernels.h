@@ -190,6 +190,7 @@ int vmx_int_gemm_geglu(const uint16_t *a16, const void *workspace, uint16_t *act
 int vmx_int_slices(const float *part, float *y, int slices, int M, int N, int64_t ldy, hipStream_t st);   // y = part [slices][M][N] in slice order
 // iq_prompt.hip: the same product with the raw blocks decoded inside it (a segment's `w` = its raw blocks)
 bool vmx_iq_prompt_ok(const VmxMmvqSeg *segs, int nseg, int M, int K);
+bool vmx_iq_prompt_alone_ok(const VmxMmvqSeg &seg, int M, int K);
 extern "C" int vmx_iq_prompt_f32(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st);
 int vmx_iq_prompt_slices(const VmxMmvqSeg *segs, int nseg, const uint16_t *a16, float *y, int M, int K, int64_t ldy, float *part, size_t part_bytes, hipStream_t st,
                          int *left);
