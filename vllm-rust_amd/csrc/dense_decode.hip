@@ -4,7 +4,7 @@
 // Such a step is a chain of short launches over weights that are read once (Qwen3-0.6B: 4 .. 13 MB each), so what bounds it is the
 // latency of each link: the weights of a workgroup are requested before anything they wait for is computed, and no result is converted
 // by a launch of its own.  Qwen3-0.6B at one row, 128 tokens: 12 launches and 43 us a layer as norm, GEMV, widening, activation kernels;
-// 5 launches and 28 us now (q|k|v 4.9 us, attention 7.6, o 4.7, gate|up 6.4 = 2.0 TB/s, down 4.5); the whole step 1269 -> 819 us.
+// 5 launches and 27 us now (q|k|v 4.9 us, attention 7.6, o 4.7, gate|up 6.4 = 2.0 TB/s, down 4.5); the whole step 1269 -> 795 us.
 #include "vmx_kernels.h"
 
 namespace {
@@ -54,14 +54,21 @@ constexpr int DD_STAGE = 16 * 1032;   // values that the norm and the merge stag
 // Rows that have to be normed or merged are worked out once per workgroup, spread over its threads, and staged in LDS: computed by
 // each lane for its own operands, one live row of sixteen kept four lanes of a wave busy (q|k|v 6.7 -> 5.0 us, gate|up 9.1 -> 8.1).
 // Their inputs come from the caches and are requested ahead of the weights of the first DEPTH blocks, because loads return in order.
+// What the first requests need comes as arguments of its own, which are in registers when a wave starts (members of a struct are not): a step of Qwen3-0.6B at
+// one row, 128 tokens, 821 -> 795 us, 0.2 us a launch.
 template <int NW, int CW, int DEPTH, int SRC, int DST>
-__global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const DenseDecode p) {
+__global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W, const void *first, const void *second, const void *third, int M, int N, int K,
+                                                                int fourth, const DenseDecode rest) {
+    DenseDecode p = rest;
+    p.W = W, p.M = M, p.N = N, p.K = K;
+    if constexpr (SRC == DD_MERGE) p.part = static_cast<const float *>(first), p.part_max = static_cast<const float *>(second), p.part_sum = static_cast<const float *>(third), p.P = fourth;
+    else p.x = static_cast<const uint16_t *>(first), p.norm_w = static_cast<const uint16_t *>(second), p.ssq = static_cast<const float *>(third), p.tiles = fourth;
     constexpr int PARTS = 16 / CW, DEEP = 128 * PARTS;
     constexpr bool STAGED = SRC == DD_NORM || SRC == DD_MERGE, NORM = SRC == DD_NORM || SRC == DD_NORM_REG;
     __shared__ float red[NW][64][4];
     __shared__ __align__(16) uint16_t rows_lds[STAGED ? DD_STAGE : 8];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & (CW - 1), part = (lane & 15) / CW, g = lane >> 4, nt = blockIdx.x;
-    const int K = p.K, nblk = (K + DEEP - 1) / DEEP, row = min(c, p.M - 1);
+    const int nblk = (K + DEEP - 1) / DEEP, row = min(c, p.M - 1);
     const bool live = c < p.M;
     const uint16_t *wrow = p.W + (int64_t)(DST == DD_GLU ? (c < CW / 2 ? 0 : p.N / 2) + nt * (CW / 2) + (c & (CW / 2 - 1)) : nt * CW + c) * K;
     const int k0 = 128 * part + 8 * g;
@@ -126,6 +133,11 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const DenseDecode
         n0 = *reinterpret_cast<const dd_u32x4 *>(p.norm_w + chunk0 % (K / 8) * 8);
     }
     if constexpr (SRC == DD_MERGE) load_parts(chunk0);
+    // DD_RESID: the thread's value of the stream, asked for ahead of the weights as everything that is not theirs
+    const int om = CW == 16 ? (tid >> 4) & 15 : (tid >> 2) & 3, on = tid & (CW - 1);
+    const int64_t out_at = (int64_t)min(om, p.M - 1) * p.N + nt * CW + on;
+    uint16_t hold = 0;
+    if constexpr (DST == DD_RESID) hold = p.h[out_at];
 #pragma unroll
     for (int d = 0; d < DEPTH; d++)
         if (wave + d * NW < nblk) load_rows(wave + d * NW, xr[d], nr[d]);
@@ -204,7 +216,7 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const DenseDecode
     if (tid >= (CW == 4 ? 64 : 256)) return;
     // CW 16: thread -> row tid / 16, column tid % 16 (element (4 g + r, c) of a tile sits with lane 16 g + c); CW 4: thread -> part
     // tid / 16, row tid / 4 % 4, column tid % 4, the square of part i at rows and columns 4 i ..
-    const int m = CW == 16 ? tid >> 4 : (tid >> 2) & 3, n = tid & (CW - 1);
+    const int m = om, n = on;
     const int from = CW == 16 ? (m >> 2) * 16 + n : (tid >> 4) * 20 + n, r = m & 3;
     float v = 0.f;
 #pragma unroll
@@ -223,8 +235,7 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const DenseDecode
             p.act[(int64_t)m * (p.N / 2) + nt * (CW / 2) + n] = vmx_f32_to_bf16((gg / (1.0f + expf(-gg))) * uu);
         }
     } else {
-        const int64_t at = (int64_t)min(m, p.M - 1) * p.N + nt * CW + n;
-        const uint16_t hn = vmx_f32_to_bf16(vmx_bf16_to_f32(p.h[at]) + vmx_bf16_to_f32(vmx_f32_to_bf16(v)));
+        const uint16_t hn = vmx_f32_to_bf16(vmx_bf16_to_f32(hold) + vmx_bf16_to_f32(vmx_f32_to_bf16(v)));
         const float f = vmx_bf16_to_f32(hn);
         float s = f * f;
         s += vmx_lane_xor<1>(s);
@@ -234,7 +245,7 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const DenseDecode
             s += vmx_lane_xor<8>(s);
         }
         if (keep) {
-            p.h[at] = hn;
+            p.h[out_at] = hn;
             if (n == 0) p.ssq_out[m * (p.N / CW) + nt] = s;
         }
     }
@@ -244,10 +255,13 @@ template <int CW, int SRC, int DST>
 int dd_launch(const DenseDecode &p, hipStream_t st) {
     const int nblk = (p.K + 128 * (16 / CW) - 1) / (128 * (16 / CW));
     const dim3 grid((unsigned)(p.N / CW));
-    if (nblk <= 4) hipLaunchKernelGGL((dense_decode_kernel<4, CW, 1, SRC, DST>), grid, dim3(256), 0, st, p);
-    else if (nblk <= 8) hipLaunchKernelGGL((dense_decode_kernel<8, CW, 1, SRC, DST>), grid, dim3(512), 0, st, p);
-    else if (nblk <= 16 || SRC == DD_NORM_REG) hipLaunchKernelGGL((dense_decode_kernel<8, CW, 2, SRC, DST>), grid, dim3(512), 0, st, p);
-    else hipLaunchKernelGGL((dense_decode_kernel<SRC == DD_NORM_REG ? 8 : 16, CW, 2, SRC, DST>), grid, dim3(1024), 0, st, p);
+    const void *first = p.x, *second = p.norm_w, *third = p.ssq;
+    int fourth = p.tiles;
+    if (SRC == DD_MERGE) first = p.part, second = p.part_max, third = p.part_sum, fourth = p.P;
+    if (nblk <= 4) hipLaunchKernelGGL((dense_decode_kernel<4, CW, 1, SRC, DST>), grid, dim3(256), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
+    else if (nblk <= 8) hipLaunchKernelGGL((dense_decode_kernel<8, CW, 1, SRC, DST>), grid, dim3(512), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
+    else if (nblk <= 16 || SRC == DD_NORM_REG) hipLaunchKernelGGL((dense_decode_kernel<8, CW, 2, SRC, DST>), grid, dim3(512), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
+    else hipLaunchKernelGGL((dense_decode_kernel<SRC == DD_NORM_REG ? 8 : 16, CW, 2, SRC, DST>), grid, dim3(1024), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
     VMX_CHECK_LAUNCH("dense_decode");
     return VMX_OK;
 }
