@@ -181,7 +181,7 @@ __device__ __forceinline__ float chunk_sum16(const uint4 v) {
 template <bool GLU>
 __device__ __forceinline__ void int4_gemm_tile_store(const float *red, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
                                                      float *__restrict__ partial, int64_t slice_stride, int M, int N, int nt, int ks,
-                                                     const int32_t *omap);
+                                                     const int32_t *omap, const float *row_by = nullptr);
 
 // Sum of the 4 waves' accumulators and the store.  Lane holds rows m = 4h + r, column n = nt*16 + nl.
 // omap (token-grouped experts): output row of block row m (LDS), instead of m itself.
@@ -200,7 +200,7 @@ __device__ __forceinline__ void int4_gemm_epilogue(float *red, const vmx_f32x4 f
 template <bool GLU>
 __device__ __forceinline__ void int4_gemm_tile_store(const float *red, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y,
                                                      float *__restrict__ partial, int64_t slice_stride, int M, int N, int nt, int ks,
-                                                     const int32_t *omap) {
+                                                     const int32_t *omap, const float *row_by) {
     const int lane = threadIdx.x & 63, nl = lane & 15, h = lane >> 4;
     float4 a = *reinterpret_cast<const float4 *>(red + lane * 4);
 #pragma unroll
@@ -208,7 +208,11 @@ __device__ __forceinline__ void int4_gemm_tile_store(const float *red, const uin
         const float4 b = *reinterpret_cast<const float4 *>(red + (wv * 64 + lane) * 4);
         a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
     }
-    const float out4[4] = {a.x, a.y, a.z, a.w};
+    float out4[4] = {a.x, a.y, a.z, a.w};
+    if (row_by) {   // rows whose factor (one over their root mean square) was left out of the operand
+#pragma unroll
+        for (int r = 0; r < 4; r++) out4[r] *= row_by[4 * h + r];
+    }
     const int n = nt * NT + nl;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -537,6 +541,7 @@ template <int N, class F> __device__ __forceinline__ void ring_static_for(F &&f)
 #define VMX_RING_D 3
 #endif
 constexpr int RING_D = VMX_RING_D;   // passes a request runs ahead of its use
+constexpr size_t RING_LDS = 2 * 16 * 4 * KB * 2;   // two stages of four waves
 // 5..16 activation rows, ring form.  The looped body above waits for an L2 round trip per staging batch (8 of them on a
 // 4096-deep slice at 16 rows) with its matrix work in between: a wave spends most of its life waiting.  Here
 //   * a pass is 4 k-blocks (one per wave); its 16 x 512 activation tile is requested D passes ahead into registers (16 per
@@ -548,34 +553,30 @@ constexpr int RING_D = VMX_RING_D;   // passes a request runs ahead of its use
 //   * a row is 1 KiB unpadded; position p of row r holds the row's 16-byte chunk p ^ (r & 15), so the 16 rows a fragment read
 //     touches lie in 16 different bank groups;
 //   * the row sums of the zero-point term come from the matrix cores (the tile times a matrix of ones).
-// K % (512 * UPW) == 0, (N / 16) % CT == 0; rows past M replicate row M - 1 (never stored).
-// xmap / omap (token-grouped experts, LDS): activation row and output row of block row m.
-template <int UPW, bool GLU, int CT>
-__device__ __forceinline__ void int4_gemm_ring_body(const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ,
-                                                    const uint16_t *__restrict__ x, const uint16_t *__restrict__ bias,
-                                                    uint16_t *__restrict__ y, float *__restrict__ partial, int64_t slice_stride, int M,
-                                                    int N, int K, int group, int block, const int32_t *xmap = nullptr,
-                                                    const int32_t *omap = nullptr) {
-    constexpr int PASSES = UPW, D = RING_D, ROWB = 4 * KB * 2;   // bytes per staged row
-    extern __shared__ __align__(16) unsigned char smem[];
+// A workgroup has NWV waves (a pass is NWV k-blocks, a stage 4 NWV KB); the sums of column tile nt0 + t over the k-blocks of slice ks end in
+// red [CT][NWV][64][4] at the head of smem, behind a barrier.  K % (128 NWV PASSES) == 0, (N / 16) % CT == 0; rows past M replicate row M - 1
+// (never stored).  xmap (token-grouped experts, LDS): activation row of block row m.  meanwhile(): called once the first requests are out.
+template <int PASSES, int CT, int NWV, class F>
+__device__ __forceinline__ void int4_gemm_ring_sums(unsigned char *smem, const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ,
+                                                    const uint16_t *__restrict__ x, int M, int K, int group, int nt0, int ks, const int32_t *xmap,
+                                                    F &&meanwhile) {
+    constexpr int D = RING_D, ROWB = NWV * KB * 2;   // bytes per staged row
     unsigned char *xs = smem;                                        // [2][16][ROWB]
-    float *red = reinterpret_cast<float *>(smem);                    // [CT][4][64][4], after the last pass
+    float *red = reinterpret_cast<float *>(smem);                    // [CT][NWV][64][4], after the last pass
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nl = lane & 15, h = lane >> 4;
-    const int n_tiles = N / NT, kblocks = K / KB, G = K / group;
-    const int n_groups = n_tiles / CT;
-    const int nt0 = (block % n_groups) * CT, ks = block / n_groups;
-    const int kb_wg = ks * 4 * UPW;
+    const int kblocks = K / KB, G = K / group;
+    const int kb_wg = ks * NWV * PASSES;
 
-    // staging: request j of a wave is row 4 j + wave of the tile, lane l its chunk l.  Every address is a wave-uniform base
-    // plus a 32-bit lane offset.
+    // staging: request j of a wave is the 1 KiB piece NWV j + wave of the tile (NWV / 4 pieces a row), lane l its chunk l.  Every address is a
+    // wave-uniform base plus a 32-bit lane offset.
     const char *xrow_u[4];
     uint32_t xdst[4];   // byte offset of the lane's chunk inside a stage
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const int row = 4 * j + wave, rsrc = min(row, M - 1);
-        xrow_u[j] = reinterpret_cast<const char *>(x + (int64_t)(xmap ? __builtin_amdgcn_readfirstlane(xmap[rsrc]) : rsrc) * K + (int64_t)kb_wg * KB);
-        xdst[j] = (uint32_t)(row * ROWB + ((lane ^ (row & 15)) << 4));
+        const int piece = NWV * j + wave, row = piece / (NWV / 4), at = piece % (NWV / 4), rsrc = min(row, M - 1);
+        xrow_u[j] = reinterpret_cast<const char *>(x + (int64_t)(xmap ? __builtin_amdgcn_readfirstlane(xmap[rsrc]) : rsrc) * K + (int64_t)kb_wg * KB + at * 512);
+        xdst[j] = (uint32_t)(row * ROWB + (((at * 64 + lane) ^ (row & 15)) << 4));
     }
     const char *w_u[CT];
     const char *z_u[CT];
@@ -595,8 +596,8 @@ __device__ __forceinline__ void int4_gemm_ring_body(const uint4 *__restrict__ W,
         for (int j = 0; j < 4; j++) tq[r][j] = *reinterpret_cast<const ring_u32x4 *>(xrow_u[j] + (size_t)p * ROWB + woff);
 #pragma unroll
         for (int t = 0; t < CT; t++) {
-            wq[r][t] = ld_weights(reinterpret_cast<const uint4 *>(w_u[t] + (size_t)p * 4 * 64 * 16 + woff));
-            zq[r][t] = *reinterpret_cast<const uint32_t *>(z_u[t] + (size_t)((((kb_wg + 4 * p + wave) * KB) / group) * 16) * 4 + zoff);
+            wq[r][t] = ld_weights(reinterpret_cast<const uint4 *>(w_u[t] + (size_t)p * NWV * 64 * 16 + woff));
+            zq[r][t] = *reinterpret_cast<const uint32_t *>(z_u[t] + (size_t)((((kb_wg + NWV * p + wave) * KB) / group) * 16) * 4 + zoff);
         }
     };
     auto write_tile = [&](auto pc) {
@@ -605,6 +606,7 @@ __device__ __forceinline__ void int4_gemm_ring_body(const uint4 *__restrict__ W,
         for (int j = 0; j < 4; j++) *reinterpret_cast<ring_u32x4 *>(xs + (p & 1) * 16 * ROWB + xdst[j]) = tq[r][j];
     };
     ring_static_for<(D < PASSES ? D : PASSES)>([&](auto pc) { issue(pc); });
+    meanwhile();
     write_tile(std::integral_constant<int, 0>{});
     const int rowc = min(nl, M - 1);
     uint32_t fa[4];   // byte offsets of this lane's four A fragments inside a stage
@@ -652,10 +654,85 @@ __device__ __forceinline__ void int4_gemm_ring_body(const uint4 *__restrict__ W,
     __syncthreads();   // the last tile has been read: the stages become the waves' exchange buffer
 #pragma unroll
     for (int t = 0; t < CT; t++)
-        *reinterpret_cast<float4 *>(red + ((t * 4 + wave) * 64 + lane) * 4) = make_float4(fin[t][0], fin[t][1], fin[t][2], fin[t][3]);
+        *reinterpret_cast<float4 *>(red + ((t * NWV + wave) * 64 + lane) * 4) = make_float4(fin[t][0], fin[t][1], fin[t][2], fin[t][3]);
     __syncthreads();
+}
+
+// One over the root mean square of the rows of a stream, from the sums of squares of its 16-column tiles, ssq [M][K / 16], into by [16]: by 16 threads a
+// row.  The requests go out with the constructor, the sums are for when they have come.
+struct RingRowScale {
+    static constexpr int Q = 8;   // float4 a thread: K <= 8192
+    float4 v[Q];
+    int quads;
+    __device__ __forceinline__ RingRowScale(const float *ssq, int M, int K) : quads(K / 64) {
+        const float4 *row = reinterpret_cast<const float4 *>(ssq) + (int64_t)min((int)(threadIdx.x >> 4), M - 1) * quads;
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            if (16 * q < quads) v[q] = row[min(16 * q + (int)(threadIdx.x & 15), quads - 1)];
+    }
+    __device__ __forceinline__ void store(float *by, int K, float eps) const {
+        float s = 0.f;
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            if (16 * q < quads) s += 16 * q + (int)(threadIdx.x & 15) < quads ? (v[q].x + v[q].y) + (v[q].z + v[q].w) : 0.f;
+        s = vmx_row16_sum(s);
+        if ((threadIdx.x & 15) == 0) by[threadIdx.x >> 4] = rsqrtf(s / (float)K + eps);
+    }
+};
+
+// NORM: x is a stream's rows times the norm's gains, without the factor of the row, which comes from ssq and multiplies the sums (RingRowScale).
+template <int UPW, bool GLU, int CT, bool NORM = false>
+__device__ __forceinline__ void int4_gemm_ring_body(const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ,
+                                                    const uint16_t *__restrict__ x, const uint16_t *__restrict__ bias,
+                                                    uint16_t *__restrict__ y, float *__restrict__ partial, int64_t slice_stride, int M,
+                                                    int N, int K, int group, int block, const int32_t *xmap = nullptr,
+                                                    const int32_t *omap = nullptr, const float *ssq = nullptr, float eps = 0.f) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int n_groups = N / NT / CT, nt0 = (block % n_groups) * CT, ks = block / n_groups;
+    float *by = nullptr;
+    if constexpr (NORM) {
+        by = reinterpret_cast<float *>(smem + RING_LDS);
+        RingRowScale rs(ssq, M, K);
+        int4_gemm_ring_sums<UPW, CT, 4>(smem, W, SZ, x, M, K, group, nt0, ks, xmap, [&] { rs.store(by, K, eps); });
+    } else {
+        int4_gemm_ring_sums<UPW, CT, 4>(smem, W, SZ, x, M, K, group, nt0, ks, xmap, [] {});
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int t = wave; t < CT; t += 4)
-        int4_gemm_tile_store<GLU>(red + t * 4 * 64 * 4, bias, y, partial, slice_stride, M, N, nt0 + t, ks, omap);
+        int4_gemm_tile_store<GLU>(reinterpret_cast<float *>(smem) + t * 4 * 64 * 4, bias, y, partial, slice_stride, M, N, nt0 + t, ks, omap, by);
+}
+
+// The linears of 5 .. 16 rows whose result goes back into the residual stream: a workgroup of eight waves owns a column tile over all of K, so the sum is
+// whole and the epilogue does what a launch of its own did: h = bf16(h + bf16(sum)), the sums of squares of its 16-column tile, and hg = bf16(h gain), the
+// operand of the next norm's consumer (NORM above; one rounding, as bf16(h factor gain) has).  N / 16 workgroups.
+template <int PASSES>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void int4_gemm_ring_resid_kernel(
+    const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ, const uint16_t *__restrict__ x, uint16_t *__restrict__ h, const uint16_t *__restrict__ gain,
+    int M, int N, int K, int group, uint16_t *__restrict__ hg, float *__restrict__ ssq) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int tid = threadIdx.x, nt = blockIdx.x, row = (tid >> 4) & 15, n = nt * NT + (tid & 15);   // of the first four waves' threads
+    const int64_t at = (int64_t)min(row, M - 1) * N + n;
+    const uint16_t hold = h[at], gn = gain[n];
+    int4_gemm_ring_sums<PASSES, 1, 8>(smem, W, SZ, x, M, K, group, nt, 0, nullptr, [] {});
+    if (tid >= 256) return;
+    const float *red = reinterpret_cast<const float *>(smem) + ((row >> 2) * 16 + (tid & 15)) * 4 + (row & 3);   // element (row, column) of a wave's tile
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; w++) v += red[w * 256];
+    const float hn = vmx_bf16_to_f32(vmx_f32_to_bf16(vmx_bf16_to_f32(hold) + vmx_bf16_to_f32(vmx_f32_to_bf16(v))));
+    const float sq = vmx_row16_sum(hn * hn);
+    if (row < M) {
+        h[at] = vmx_f32_to_bf16(hn);
+        hg[at] = vmx_f32_to_bf16(hn * vmx_bf16_to_f32(gn));
+        if ((tid & 15) == 0) ssq[row * (N / NT) + nt] = sq;
+    }
+}
+
+template <int UPW, bool GLU, int CT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 3))) void int4_gemm_ring_norm_kernel(
+    const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ, const uint16_t *__restrict__ hg, const float *__restrict__ ssq, int M, int N, int K, int group,
+    float eps, uint16_t *__restrict__ act, float *__restrict__ partial) {
+    int4_gemm_ring_body<UPW, GLU, CT, true>(W, SZ, hg, nullptr, act, partial, (int64_t)M * N, M, N, K, group, (int)blockIdx.x, nullptr, nullptr, ssq, eps);
 }
 
 template <int UPW, bool GLU, int CT>
@@ -1680,7 +1757,6 @@ inline int looped_ct(int M, int N) {
 // Ring form (5..16 rows, whole passes of 512 k): column tiles per workgroup, 0 = not eligible.  The most tiles (at most 3:
 // registers) that still leave a workgroup for every compute unit (Qwen3-8B AWQ at 16 rows, same box: 3 / 2 / 1 tiles
 // 6367 / 6155 / 5821 tok/s aggregate).
-constexpr size_t RING_LDS = 2 * 16 * 4 * KB * 2;
 inline int ring_ct(int M, int N, int K, const GemmPlan &p) {
     static const int on = vmx_tune("VMX_INT4_RING", 1), force_ct = vmx_tune("VMX_INT4_RING_CT", 0);
     if (!on || M < 5 || M > 16 || (p.upw != 2 && p.upw != 4 && p.upw != 8) || (K / KB) % (4 * p.upw) != 0) return 0;
@@ -1906,6 +1982,61 @@ int vmx_int4_gemm_partial(const void *packed, const uint16_t *x, float *partial,
         const int mm = M - m0 < 16 ? M - m0 : 16;
         if (int rc = launch_gemm(p, W, SZ, x + (int64_t)m0 * K, nullptr, nullptr, partial + (int64_t)m0 * N, mm, N, K, group, st, M)) return rc;
     }
+    return VMX_OK;
+}
+
+// ---- 5 .. 16 rows: the residual add and the next norm's gains in the epilogue, the norm's row factor behind the consumer's sums
+// (int4_gemm_ring_resid_kernel, int4_gemm_ring_norm_kernel)
+bool vmx_int4_ring_resid_ok(int M, int N, int K) {
+    const int passes = K % (8 * KB) == 0 ? K / (8 * KB) : 0;
+    return M >= 5 && M <= 16 && N % NT == 0 && (passes == 2 || passes == 4 || passes == 6 || passes == 8 || passes == 12);
+}
+// slices the consumer leaves (1 with glu), 0: not covered
+int vmx_int4_ring_norm_splits(int M, int N, int K, int glu) {
+    const GemmPlan p = plan_gemm(N, K);
+    if (K > 8192 || !ring_ct(M, N, K, p) || (glu && (N % 32 || p.splits != 1 || p.upw < 4))) return 0;
+    return p.splits;
+}
+
+// h [M][N] = bf16(h + bf16(x W)), ssq [M][N / 16] = sums of squares of the tiles of the new h, hg = bf16(h gain)
+int vmx_int4_ring_resid(const void *packed, const uint16_t *x, uint16_t *h, uint16_t *hg, const uint16_t *gain, float *ssq, int M, int N, int K, int group,
+                        hipStream_t st) {
+    VMX_REQUIRE(vmx_int4_ring_resid_ok(M, N, K), "int4_ring_resid: shape [%d x %d -> %d] not supported", M, K, N);
+    const uint4 *W = (const uint4 *)packed;
+    const uint32_t *SZ = (const uint32_t *)((const char *)packed + sz_offset_bytes(K, N));
+#define RRES(P) hipLaunchKernelGGL((int4_gemm_ring_resid_kernel<P>), dim3((unsigned)(N / NT)), dim3(512), 2 * RING_LDS, st, W, SZ, x, h, gain, M, N, K, group, hg, ssq)
+    switch (K / (8 * KB)) {
+        case 2: RRES(2); break;
+        case 4: RRES(4); break;
+        case 6: RRES(6); break;
+        case 8: RRES(8); break;
+        default: RRES(12); break;
+    }
+#undef RRES
+    VMX_CHECK_LAUNCH("int4_gemm(ring, residual)");
+    return VMX_OK;
+}
+
+// The linear of rms_norm(h) from what vmx_int4_ring_resid left: partial [slices][M][N], or act [M][N / 2] of a gate|up linear
+int vmx_int4_ring_norm(const void *packed, const uint16_t *hg, const float *ssq, float eps, float *partial, uint16_t *act, int M, int N, int K, int group,
+                       hipStream_t st) {
+    VMX_REQUIRE(vmx_int4_ring_norm_splits(M, N, K, act != nullptr) > 0, "int4_ring_norm: shape [%d x %d -> %d] not supported", M, K, N);
+    const GemmPlan p = plan_gemm(N, K);
+    const int ct = ring_ct(M, N, K, p);
+    const uint4 *W = (const uint4 *)packed;
+    const uint32_t *SZ = (const uint32_t *)((const char *)packed + sz_offset_bytes(K, N));
+    const dim3 grid((unsigned)((N / NT / ct) * p.splits));
+#define RN_C(U, G, C) hipLaunchKernelGGL((int4_gemm_ring_norm_kernel<U, G, C>), grid, dim3(256), RING_LDS + 64, st, W, SZ, hg, ssq, M, N, K, group, eps, act, partial)
+#define RN(U, G) do { if (ct == 3) RN_C(U, G, 3); else if (ct == 2) RN_C(U, G, 2); else RN_C(U, G, 1); } while (0)
+    if (act) {
+        if (p.upw == 8) RN(8, true);
+        else RN(4, true);
+    } else if (p.upw == 8) RN(8, false);
+    else if (p.upw == 4) RN(4, false);
+    else RN(2, false);
+#undef RN
+#undef RN_C
+    VMX_CHECK_LAUNCH("int4_gemm(ring, norm)");
     return VMX_OK;
 }
 

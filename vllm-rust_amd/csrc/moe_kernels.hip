@@ -19,7 +19,9 @@ __device__ __forceinline__ float rb(float v) { return vmx_bf16_to_f32(vmx_f32_to
 __global__ __launch_bounds__(256) void moe_combine_kernel(uint16_t *__restrict__ out, const float *__restrict__ partial, int splits,
                                                            int pairs, const float *__restrict__ w, int k, int hidden,
                                                            const void *const *__restrict__ w2_table, const int32_t *__restrict__ ids,
-                                                           int num_experts, uint16_t *__restrict__ h_resid, float *__restrict__ ssq) {
+                                                           int num_experts, uint16_t *__restrict__ h_resid, float *__restrict__ ssq,
+                                                           uint16_t *__restrict__ hg, const uint16_t *__restrict__ gain) {
+    // hg != NULL (with h_resid): also bf16(h * gain), the operand of the next norm's consumer without the row's factor.
     // h_resid != NULL: the layer's residual add happens here as well, h = bf16(h + out), and ssq[t][hidden / 16] receives the
     // sums of squares of the 16-column tiles of the new h (what the norm prologue of the next layer's q|k|v GEMM reads);
     // the launch then has one thread per column (hidden % 256 == 0), so a tile is 16 consecutive lanes.
@@ -27,7 +29,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(uint16_t *__restrict__
     for (int i = blockIdx.x * 256 + threadIdx.x; i < hidden; i += gridDim.x * 256) {
         // The launch is a chain of memory round trips, so the loads of two experts and eight split-K slices go out together
         // (branch-free: a slot past the end re-reads the last valid one and is not added); sums in slice order, experts in j order.
-        const uint16_t hold = h_resid ? h_resid[(int64_t)t * hidden + i] : (uint16_t)0;
+        const uint16_t hold = h_resid ? h_resid[(int64_t)t * hidden + i] : (uint16_t)0, gn = hg ? gain[i] : (uint16_t)0;
         float acc = 0.f;
         for (int j0 = 0; j0 < k; j0 += 2) {
             int p[2];
@@ -60,6 +62,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(uint16_t *__restrict__
         if (h_resid) {
             const uint16_t hn = vmx_f32_to_bf16(vmx_bf16_to_f32(hold) + acc);
             h_resid[(int64_t)t * hidden + i] = hn;
+            if (hg) hg[(int64_t)t * hidden + i] = vmx_f32_to_bf16(vmx_bf16_to_f32(hn) * vmx_bf16_to_f32(gn));
             float sq = vmx_bf16_to_f32(hn);
             sq *= sq;
             sq = vmx_row16_sum(sq);
@@ -123,13 +126,13 @@ extern "C" int vmx_moe_int4_forward(uint16_t *out, const uint16_t *x, const floa
                                     const void *const *w13_packed, const void *const *w2_packed, int tokens, int k, int num_experts,
                                     int hidden, int inter, int group, void *workspace, size_t workspace_bytes, void *stream) {
     return vmx_moe_int4_forward_glu(out, x, topk_weights, topk_ids, w13_packed, w2_packed, tokens, k, num_experts, hidden, inter, group,
-                                    workspace, workspace_bytes, 0, vmx_stream(stream), nullptr, nullptr);
+                                    workspace, workspace_bytes, 0, vmx_stream(stream), nullptr, nullptr, nullptr, nullptr);
 }
 
 int vmx_moe_int4_forward_glu(uint16_t *out, const uint16_t *x, const float *topk_weights, const int32_t *topk_ids,
                              const void *const *w13_packed, const void *const *w2_packed, int tokens, int k, int num_experts, int hidden,
                              int inter, int group, void *workspace, size_t workspace_bytes, int w13_glu, hipStream_t st, uint16_t *h_resid,
-                             float *ssq) {
+                             float *ssq, uint16_t *hg, const uint16_t *gain) {
     VMX_REQUIRE(!h_resid || (ssq && hidden % 256 == 0), "moe_int4_forward: the residual epilogue needs ssq and hidden %% 256 == 0");
     VMX_REQUIRE(out && x && topk_weights && topk_ids && w13_packed && w2_packed && workspace, "moe_int4_forward: null pointer");
     VMX_REQUIRE(tokens >= 1 && k >= 1 && num_experts >= 1, "moe_int4_forward: bad counts");
@@ -169,7 +172,7 @@ int vmx_moe_int4_forward_glu(uint16_t *out, const uint16_t *x, const float *topk
                                                  pairs, hidden, inter, group, st))
             return rc;
         hipLaunchKernelGGL(moe_combine_kernel, dim3((hidden + 255) / 256, tokens), dim3(256), 0, st, out, p2, s2, pairs, topk_weights, k, hidden,
-                           w2_packed, topk_ids, num_experts, h_resid, ssq);
+                           w2_packed, topk_ids, num_experts, h_resid, ssq, hg, gain);
         VMX_CHECK_LAUNCH("moe_combine");
         return VMX_OK;
     }
@@ -185,7 +188,7 @@ int vmx_moe_int4_forward_glu(uint16_t *out, const uint16_t *x, const float *topk
     // down projection; x row = pair
     if (int rc = vmx_int4_gemm_grouped(w2_packed, topk_ids, num_experts, act, 1, p2, pairs, hidden, inter, group, st)) return rc;
     hipLaunchKernelGGL(moe_combine_kernel, dim3((hidden + 255) / 256, tokens), dim3(256), 0, st, out, p2, s2, pairs, topk_weights, k, hidden, w2_packed, topk_ids,
-                       num_experts, h_resid, ssq);
+                       num_experts, h_resid, ssq, hg, gain);
     VMX_CHECK_LAUNCH("moe_combine");
     return VMX_OK;
 }

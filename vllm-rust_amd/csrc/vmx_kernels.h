@@ -24,7 +24,8 @@ bool vmx_int4_token_grouped16_ok(int N, int K);
 int vmx_moe_int4_forward_glu(uint16_t *out, const uint16_t *x, const float *topk_weights, const int32_t *topk_ids,
                              const void *const *w13_packed, const void *const *w2_packed, int tokens, int k, int num_experts, int hidden,
                              int inter, int group, void *workspace, size_t workspace_bytes, int w13_glu, hipStream_t st,
-                             uint16_t *h_resid = nullptr, float *ssq = nullptr);   // h_resid: also h = bf16(h + out) and its tile sums of squares
+                             uint16_t *h_resid = nullptr, float *ssq = nullptr, uint16_t *hg = nullptr, const uint16_t *gain = nullptr);
+// h_resid: also h = bf16(h + out) and its tile sums of squares, and with hg also bf16(h gain)
 int vmx_int4_gemm_glu(const void *packed, const uint16_t *x, uint16_t *act, int M, int N, int K, int group, hipStream_t st);
 // decode rows (M <= 4): RMSNorm of the residual stream in the prologue (q|k|v, gate|up) and the residual add in the epilogue
 // (o_proj, down_proj), so that a dense int4 layer is five launches
@@ -35,6 +36,14 @@ int vmx_int4_gemm_partial_norm(const void *packed, const uint16_t *h, const uint
                                int M, int N, int K, int group, hipStream_t st);
 int vmx_int4_gemm_glu_norm(const void *packed, const uint16_t *h, const uint16_t *norm_w, float eps, const float *ssq, uint16_t *act, int M,
                            int N, int K, int group, hipStream_t st);
+// 5 .. 16 rows (ring form): h = bf16(h + bf16(x W)) with the sums of squares of its 16-column tiles and hg = bf16(h gain); the linear of rms_norm(h) from
+// those (hg carries the gains, the row factor comes from ssq and multiplies the sums)
+bool vmx_int4_ring_resid_ok(int M, int N, int K);
+int vmx_int4_ring_norm_splits(int M, int N, int K, int glu);
+int vmx_int4_ring_resid(const void *packed, const uint16_t *x, uint16_t *h, uint16_t *hg, const uint16_t *gain, float *ssq, int M, int N, int K, int group,
+                        hipStream_t st);
+int vmx_int4_ring_norm(const void *packed, const uint16_t *hg, const float *ssq, float eps, float *partial, uint16_t *act, int M, int N, int K, int group,
+                       hipStream_t st);
 int vmx_int4_gemm_resid(const void *packed, const uint16_t *x, uint16_t *h, float *ssq, int M, int N, int K, int group, hipStream_t st);
 int vmx_awq_convert_into(const uint32_t *awq_qweight, const uint32_t *awq_qzeros, uint32_t *qweight_out, uint32_t *qzeros_out, int K,
                          int N, int group, int Ntot, int col0, hipStream_t st);
