@@ -46,3 +46,25 @@ def test_layers_match_oracle(models, rows):
             rel = np.sqrt(err.sum() / norm.sum() if spec.num_experts else (err / norm).max())
             assert rel <= 3e-2, (p, rel)
         ids = out.cpu().numpy().astype(np.int32)
+
+
+@pytest.mark.parametrize("rows", [49, 64, 65, 130])
+def test_one_slice_prompts_match_the_decode_path(rows):
+    """Prompts whose linears take all of k in one slice pass bf16 sums on; 256 and 512 wide, so that every projection does."""
+    import torch
+    import vllm_rust_amd as vmx
+    from vllm_rust_amd.qwen3 import QuantizedQwen3ForCausalLM, Qwen3Spec
+    vmx.init(0)
+    spec = Qwen3Spec(hidden_size=256, num_layers=2, num_heads=4, num_kv_heads=2, head_dim=64, intermediate_size=512, vocab_size=1000, max_position=256,
+                     num_blocks=16, max_batch=4, max_seq_len=160, max_prefill_tokens=130)
+    model = QuantizedQwen3ForCausalLM(spec)
+    model.load_synthetic(seed=9)
+    prompt = torch.randint(0, spec.vocab_size, (rows,), dtype=torch.int32, device="cuda", generator=torch.Generator(device="cuda").manual_seed(rows))
+    bt = torch.randperm(16, dtype=torch.int32, device="cuda")
+    got = torch.empty(spec.vocab_size, dtype=torch.bfloat16, device="cuda")
+    _, want = model.forward(prompt, 0, bt)
+    model.prefill(prompt, 0, bt, logits_last=got)
+    torch.cuda.synchronize()
+    want = want[-1].float()
+    assert float((got.float() - want).norm() / want.norm()) <= 2e-2   # the decoder tests' bar
+    model.close()

@@ -364,7 +364,8 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(const float *__restrict__
     const int64_t slice = (int64_t)tokens * heads * HD, base = ((int64_t)t * heads + head) * HD + 8 * l;
     const bool is_q = head < Hq, is_k = !is_q && head < Hq + Hkv;
     float v[8];
-    sum_partials8(partial, splits, slice, base, v);
+    if (splits < 0) vmx_unpack16x8<F16>(*reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(partial) + base), v);   // the rounded sums themselves
+    else sum_partials8(partial, splits, slice, base, v);
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
@@ -687,6 +688,13 @@ double int4_alg_bytes(const Int4Linear &l, int M) {
 
 int run_linear(vmx_qwen3 *, const Int4Linear &l, const uint16_t *xin, float *partial, int M, hipStream_t st) {
     return l.forward_partial(xin, partial, M, st);
+}
+// A prompt's linear, for readers that round the sum to bf16 before anything else: *splits slices in f32, or (-1) where one slice is the whole sum the bf16
+// values themselves, in half the bytes (2048 rows of Qwen3-8B, 9 layers: 8190 -> 8055 us)
+int run_prompt_linear(vmx_qwen3 *m, const Int4Linear &l, const uint16_t *xin, float *partial, int *splits, int M, hipStream_t st) {
+    if (!vmx_int4_gemm_y_ok(M, l.out_features, l.in_features)) return run_linear(m, l, xin, partial, M, st);
+    *splits = -1;
+    return vmx_int4_gemm_y(l.packed.p, xin, reinterpret_cast<uint16_t *>(partial), M, l.out_features, l.in_features, l.group, st);
 }
 
 int8_t *q8_aq(vmx_qwen3 *m) { return (int8_t *)m->q8.p; }
@@ -1323,7 +1331,8 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
         const bool iq = !moe && !L.int4_ready() && !ex && !dn;       // GGUF I-quant layer: every projection is an IqLinear
         const bool one = iq || ex || dn;                             // linear outputs arrive as one f32 slice
         int s_qkv = one ? 1 : L.qkv.splits(B);
-        const int s_o = one ? 1 : L.o.splits(B), s_gu = one ? 1 : L.gate_up.splits(B), s_down = one ? 1 : L.down.splits(B);
+        int s_o = one ? 1 : L.o.splits(B), s_gu = one ? 1 : L.gate_up.splits(B), s_down = one ? 1 : L.down.splits(B);
+        const bool prompt = prefill_offset >= 0 && !tp;
         // h += pending; x = rms_norm(h);  q|k|v = linear(x)
         // EXL3 decode rows: the consumers of o, gate|up and down apply the output transform themselves (one launch less each)
         const bool ex_fold = ex && B <= 4 && !tp && H % 128 == 0 && I % 128 == 0 && L.ex_svh_gu.p;
@@ -1412,7 +1421,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
             if (int rc = iq_forward(m, L.iq[VMX_L_Q], PA, NQKV_, B, st)) return rc;
             if (int rc = iq_forward(m, L.iq[VMX_L_K], PA + NQ, NQKV_, B, st)) return rc;
             if (int rc = iq_forward(m, L.iq[VMX_L_V], PA + NQ + NKV, NQKV_, B, st)) return rc;
-        } else if (int rc = run_linear(m, L.qkv, x, PA, B, st)) return rc;
+        } else if (int rc = prompt ? run_prompt_linear(m, L.qkv, x, PA, &s_qkv, B, st) : run_linear(m, L.qkv, x, PA, B, st)) return rc;
         const float *ks = (const float *)L.kv_scales.p;
         // five-launch layers: attention spread over several workgroups per KV head, merged by o_proj while it stages its activations
         const int split_p = vmx_split_decode_attention_parts(hd, Hq / Hkv, hd, max_seq_len, 0);
@@ -1558,7 +1567,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
             if (int rc = dense_forward(L.dn[1].p, attn, PB, H, NQ, B, st)) return rc;
         } else if (iq) {
             if (int rc = iq_forward(m, L.iq[VMX_L_O], PB, H, B, st)) return rc;
-        } else if (int rc = run_linear(m, L.o, attn, PB, B, st)) return rc;
+        } else if (int rc = prompt ? run_prompt_linear(m, L.o, attn, PB, &o_splits, B, st) : run_linear(m, L.o, attn, PB, B, st)) return rc;
         // h += o; x = rms_norm(h);  gate|up = linear(x);  act = silu(gate) * up;  down = linear(act)
         if (tp) {  // row-parallel: local bf16 output, summed over the ranks
             if (int rc = tp_reduce(m, PB, o_splits, B, H, st)) return rc;
@@ -1638,7 +1647,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
             if (int rc = dense_forward(L.dn[3].p, act, PB, H, I, B, st)) return rc;
         } else if (iq) {
             if (int rc = iq_forward(m, L.iq[VMX_L_DOWN], PB, H, B, st)) return rc;
-        } else if (int rc = run_linear(m, L.down, act, PB, B, st)) return rc;
+        } else if (int rc = prompt ? run_prompt_linear(m, L.down, act, PB, &s_down, B, st) : run_linear(m, L.down, act, PB, B, st)) return rc;
         pending = PB;
         pending_splits = s_down;
         if (tp) {

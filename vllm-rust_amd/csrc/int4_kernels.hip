@@ -1985,6 +1985,16 @@ int vmx_int4_gemm_partial(const void *packed, const uint16_t *x, float *partial,
     return VMX_OK;
 }
 
+// y [M][N] = bf16(x W) where the prompt-shaped kernel takes all of k in one slice
+bool vmx_int4_gemm_y_ok(int M, int N, int K) { return tiled_ok(M, N, K) && tiled_wide_ok(M, N, K) && prompt_slices(M, N, K, false) == 1; }
+int vmx_int4_gemm_y(const void *packed, const uint16_t *x, uint16_t *y, int M, int N, int K, int group, hipStream_t st) {
+    VMX_REQUIRE(vmx_int4_gemm_y_ok(M, N, K), "int4_gemm_y: shape [%d x %d -> %d] takes slices", M, K, N);
+    launch_tiled<false, false>((const uint4 *)packed, (const uint32_t *)((const char *)packed + sz_offset_bytes(K, N)), x, nullptr, nullptr, M, N, K, group,
+                               K / KB, M, Int4GroupedArgs{}, (M + PF_BM - 1) / PF_BM, 1, st, y);
+    VMX_CHECK_LAUNCH("int4_gemm(tiled, bf16)");
+    return VMX_OK;
+}
+
 // ---- 5 .. 16 rows: the residual add and the next norm's gains in the epilogue, the norm's row factor behind the consumer's sums
 // (int4_gemm_ring_resid_kernel, int4_gemm_ring_norm_kernel)
 bool vmx_int4_ring_resid_ok(int M, int N, int K) {

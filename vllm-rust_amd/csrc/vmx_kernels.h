@@ -36,6 +36,8 @@ int vmx_int4_gemm_partial_norm(const void *packed, const uint16_t *h, const uint
                                int M, int N, int K, int group, hipStream_t st);
 int vmx_int4_gemm_glu_norm(const void *packed, const uint16_t *h, const uint16_t *norm_w, float eps, const float *ssq, uint16_t *act, int M,
                            int N, int K, int group, hipStream_t st);
+bool vmx_int4_gemm_y_ok(int M, int N, int K);
+int vmx_int4_gemm_y(const void *packed, const uint16_t *x, uint16_t *y, int M, int N, int K, int group, hipStream_t st);   // y = bf16(x W), one slice of k
 // 5 .. 16 rows (ring form): h = bf16(h + bf16(x W)) with the sums of squares of its 16-column tiles and hg = bf16(h gain); the linear of rms_norm(h) from
 // those (hg carries the gains, the row factor comes from ssq and multiplies the sums)
 bool vmx_int4_ring_resid_ok(int M, int N, int K);
