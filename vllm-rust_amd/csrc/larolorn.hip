@@ -408,8 +408,14 @@ int chunked_lightning(vmx_larolorn *m, Layer &L, const Layer &w, const Step &s) 
 // m->y = ff(x)
 int clamped_glu(vmx_larolorn *m, const Layer &w, const Step &s) {
     const int W = m->cfg.width, F = w.c.ff, f32 = m->f32() ? 1 : 0;
-    if (int rc = vmx_linear_launch(product(m->input(), f32, W, w.wgu, 2 * F, m->fused.p, 1, s.T, f32), s.st)) return rc;
-    if (int rc = vmx_glu_clamped_rows(m->act.p, f32, m->fused.as<float>(), s.T, F, GLU_SLOPE, w.c.limit, s.st)) return rc;
+    VmxLinear gu = product(m->input(), f32, W, w.wgu, 2 * F, m->act.p, f32, s.T, f32);
+    gu.ldc = F;
+    if (vmx_linear_glu_ok(gu)) {   // the activation behind the sums: no f32 rows of gate and up in memory
+        if (int rc = vmx_linear_glu(gu, GLU_SLOPE, w.c.limit, s.st)) return rc;
+    } else {
+        if (int rc = vmx_linear_launch(product(m->input(), f32, W, w.wgu, 2 * F, m->fused.p, 1, s.T, f32), s.st)) return rc;
+        if (int rc = vmx_glu_clamped_rows(m->act.p, f32, m->fused.as<float>(), s.T, F, GLU_SLOPE, w.c.limit, s.st)) return rc;
+    }
     return vmx_linear_launch(product(m->act, f32, F, w.wdown, W, m->y.p, 1, s.T, f32), s.st);
 }
 

@@ -291,9 +291,16 @@ __device__ __forceinline__ void linear_tile_store(const VmxLinear &p, int z, int
 // finished sums are stored as they are, with a bias and a SiLU range, times the sigmoids of a gate, or through linear_store (whose run-time choices per
 // element cost a 1500 x 12288 output as much as half of its product: 159 against 101 us; gates read there wait for the store before them, each in
 // turn: 16 products of 1500 x 128 x 512 33 -> 27 us).
-enum { TILE_PLAIN, TILE_BIAS_SILU, TILE_GATE, TILE_ANY };
-template <class S, int EP>
-__global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(const VmxLinear p, int row_tiles, int tiles) {
+// TILE_GLU: of a wave's pairs of 32 columns the first are gate columns and the second the up columns that belong to them, so a lane holds both.
+enum { TILE_PLAIN, TILE_BIAS_SILU, TILE_GATE, TILE_ANY, TILE_GLU };
+template <class S> struct HalfColumns { static constexpr int MI = S::MI, NJ = S::NJ / 2; };
+struct GluLinear : VmxLinear { float slope, limit; };   // vmx_linear_glu
+__device__ __forceinline__ float linear_glu(const GluLinear &p, float g, float u) {
+    g = fminf(g, p.limit);
+    return g / (1.0f + expf(-p.slope * g)) * (fminf(fmaxf(u, -p.limit), p.limit) + 1.0f);
+}
+template <class S, int EP, class P = VmxLinear>
+__global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(const P p, int row_tiles, int tiles) {
     extern __shared__ __align__(1024) uint16_t tg_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tile = tg_tile(blockIdx.x, tiles), z = blockIdx.y;
@@ -312,7 +319,15 @@ __global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(co
     }
 #pragma unroll
     for (int q = 0; q < S::BQ; q++)
-        b_src[q] = (uint32_t)((int64_t)min(n0 + tg_src_row<S::BQ>(wave, lane, q), p.N - 1) * p.w_sn * 2) + tg_src_byte(lane);
+    {
+        const int c = tg_src_row<S::BQ>(wave, lane, q);   // column of the tile
+        int n = min(n0 + c, p.N - 1);
+        if constexpr (EP == TILE_GLU) {
+            const int half = p.N / 2, j = c / 32 % S::NJ;
+            n = (j & 1 ? half : 0) + min(n0 / 2 + c / (32 * S::NJ) * (16 * S::NJ) + j / 2 * 32 + (c & 31), half - 1);
+        }
+        b_src[q] = (uint32_t)((int64_t)n * p.w_sn * 2) + tg_src_byte(lane);
+    }
     tg_f32x16 acc[S::MI][S::NJ];
 #pragma unroll
     for (int i = 0; i < S::MI; i++)
@@ -360,6 +375,20 @@ __global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(co
                 for (int j = 0; j < S::NJ; j++) acc[i][j][r] *= 1.0f / (1.0f + expf(-gate[(int64_t)min(wn + 32 * j + col, p.N - 1) * p.aux_sn]));
             }
     }
+    if constexpr (EP == TILE_GLU) {
+        tg_f32x16 act[S::MI][S::NJ / 2];
+#pragma unroll
+        for (int i = 0; i < S::MI; i++)
+#pragma unroll
+            for (int j = 0; j < S::NJ / 2; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) act[i][j][r] = linear_glu(p, acc[i][2 * j][r], acc[i][2 * j + 1][r]);
+        VmxLinear out = p;
+        out.N = p.N / 2;
+        if (p.c_f32) linear_tile_store<HalfColumns<S>, float>(out, z, wm, wn / 2, lane, act);
+        else linear_tile_store<HalfColumns<S>, uint16_t>(out, z, wm, wn / 2, lane, act);
+        return;
+    }
     if (p.c_f32) linear_tile_store<S, float>(p, z, wm, wn, lane, acc);
     else linear_tile_store<S, uint16_t>(p, z, wm, wn, lane, acc);
 }
@@ -370,8 +399,11 @@ __global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(co
 // of 128 values a part.  Lane (c, g) reads 16 of the 64 consecutive bytes that the four lanes g share of a column, straight from memory
 // and DEPTH blocks ahead, and the activation fragment at the same k from the (cache-resident) rows.  The waves' tiles are added in
 // wave order through LDS.
-template <int NW, int PARTS, int DEPTH>
-__global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const VmxLinear p) {
+// GluLinear: the sixteen columns are eight gate columns and the up columns that belong to them.
+template <int NW, int PARTS, int DEPTH, class P = VmxLinear>
+__global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const P p) {
+    constexpr bool GLU = std::is_same<P, GluLinear>::value;
+    static_assert(!GLU || PARTS == 1, "eight gate and eight up columns a workgroup");
     constexpr int CW = 16 / PARTS, DEEP = 128 * PARTS;
     __shared__ float red[NW][64][4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fl = lane & 15, c = fl & (CW - 1), part = fl / CW, fg = lane >> 4;
@@ -379,7 +411,8 @@ __global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const VmxLinear 
     if (p.total_rows && m0 >= *p.total_rows) return;
     const uint16_t *W = p.W + z * p.w_bs;
     if (p.block_expert) W += (int64_t)p.block_expert[m0 / p.block_rows] * p.expert_stride;
-    const uint16_t *wrow = W + (int64_t)min(n0 + c, p.N - 1) * p.w_sn;
+    const int wn = GLU ? (c < 8 ? 0 : p.N / 2) + min(n0 / 2 + (c & 7), p.N / 2 - 1) : min(n0 + c, p.N - 1);
+    const uint16_t *wrow = W + (int64_t)wn * p.w_sn;
     const int64_t ar = linear_src_row(p, m0 + fl), a_at = z * p.a_bs + (ar < 0 ? 0 : ar) * p.lda;
     const int nblk = (p.K + DEEP - 1) / DEEP;
     tg_u32x4 w[DEPTH][4], a[DEPTH][PARTS][4];
@@ -455,13 +488,23 @@ __global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const VmxLinear 
     for (int q = 0; q < PARTS; q++)
 #pragma unroll
         for (int i = 0; i < NW; i++) v += red[i][(ml >> 2) * 16 + CW * q + nl][ml & 3];
+    if constexpr (GLU) {
+        const float up = vmx_lane_xor<8>(v);
+        const int n = n0 / 2 + nl;
+        if (m < p.M && nl < 8 && n < p.N / 2) {
+            const float y = linear_glu(p, v, up);
+            if (p.c_f32) ((float *)p.C)[(int64_t)m * p.ldc + n] = y;
+            else ((uint16_t *)p.C)[(int64_t)m * p.ldc + n] = vmx_f32_to_bf16(y);
+        }
+        return;
+    }
     if (m < p.M && n0 + nl < p.N && !(p.row_ids && linear_src_row(p, m) < 0)) linear_store(p, z, m, n0 + nl, v);
 }
 
-template <int NW, int PARTS, int DEPTH>
-void launch_skinny_as(const VmxLinear &p, hipStream_t st) {
+template <int NW, int PARTS, int DEPTH, class P>
+void launch_skinny_as(const P &p, hipStream_t st) {
     constexpr int CW = 16 / PARTS;
-    hipLaunchKernelGGL((linear_skinny_kernel<NW, PARTS, DEPTH>), dim3((p.N + CW - 1) / CW, (p.M + 15) / 16, p.batch), dim3(64 * NW), 0, st, p);
+    hipLaunchKernelGGL((linear_skinny_kernel<NW, PARTS, DEPTH, P>), dim3((p.N + CW - 1) / CW, (p.M + 15) / 16, p.batch), dim3(64 * NW), 0, st, p);
 }
 
 // What bounds these is the number of requests under way, so the split follows the number of 16-column groups (and K, never M: a row's
@@ -483,6 +526,11 @@ void launch_skinny(const VmxLinear &p, hipStream_t st) {
     if (nblk <= 4) return launch_skinny_as<4, 2, 1>(p, st);
     if (nblk <= 8) return launch_skinny_as<8, 2, 1>(p, st);
     launch_skinny_as<8, 2, 2>(p, st);
+}
+void launch_skinny_glu(const GluLinear &p, hipStream_t st) {   // sixteen columns a workgroup
+    const int nblk = (p.K + 127) / 128;
+    if (p.N / 16 >= 2 * vmx_num_cus()) return launch_skinny_as<4, 1, 2>(p, st);
+    return nblk <= 4 ? launch_skinny_as<4, 1, 1>(p, st) : nblk <= 8 ? launch_skinny_as<8, 1, 1>(p, st) : launch_skinny_as<8, 1, 2>(p, st);
 }
 
 // A few output columns in true f32 (router logits): one workgroup per row and group of 16 columns; a thread walks its k with
@@ -518,11 +566,11 @@ bool tile_ok(const VmxLinear &p, bool direct) {
            p.lda >= 0 && p.w_sn >= 0;
 }
 
-template <class S, int EP>
-int launch_tile_as(const VmxLinear &p, hipStream_t st) {
+template <class S, int EP, class P>
+int launch_tile_as(const P &p, hipStream_t st) {
     const int row_tiles = (p.M + S::BM - 1) / S::BM, tiles = row_tiles * ((p.N + S::BN - 1) / S::BN);
-    VMX_CHECK_HIP(hipFuncSetAttribute((const void *)linear_tile_kernel<S, EP>, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS));
-    hipLaunchKernelGGL((linear_tile_kernel<S, EP>), dim3(tg_grid(tiles), p.batch), dim3(S::THREADS), S::LDS, st, p, row_tiles, tiles);
+    VMX_CHECK_HIP(hipFuncSetAttribute((const void *)linear_tile_kernel<S, EP, P>, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS));
+    hipLaunchKernelGGL((linear_tile_kernel<S, EP, P>), dim3(tg_grid(tiles), p.batch), dim3(S::THREADS), S::LDS, st, p, row_tiles, tiles);
     return VMX_OK;
 }
 
@@ -579,8 +627,42 @@ int launch_tile(const VmxLinear &p, hipStream_t st) {
     if (least == t192) return launch_tile_shape<Tile192>(p, st);
     return least == t256 ? launch_tile_shape<Tile256>(p, st) : launch_tile_shape<Tile128two>(p, st);
 }
+// ... of those whose waves own pairs of 32 columns
+int launch_tile_glu(const GluLinear &p, hipStream_t st) {
+    const int64_t t64w = tile_ns<Tile64w>(p, 700, 450), two = tile_ns<Tile128two>(p, 1130, 800), t192 = tile_ns<Tile192>(p, 850, 0), t256 = tile_ns<Tile256>(p, 1000, 0),
+                  least = std::min({t64w, two, t192, t256});
+    if (least == t64w) return launch_tile_as<Tile64w, TILE_GLU>(p, st);
+    if (least == t192) return launch_tile_as<Tile192, TILE_GLU>(p, st);
+    return least == t256 ? launch_tile_as<Tile256, TILE_GLU>(p, st) : launch_tile_as<Tile128two, TILE_GLU>(p, st);
+}
+
+// 16-byte loads straight from the operands: whole 8-element chunks, aligned rows
+bool direct_ok(const VmxLinear &p) {
+    return p.w_sk == 1 && p.K % 8 == 0 && p.w_sn % 8 == 0 && p.lda % 8 == 0 && p.a_bs % 8 == 0 && p.w_bs % 8 == 0 && p.expert_stride % 8 == 0 &&
+           ((uintptr_t)p.W & 15) == 0 && ((uintptr_t)p.A & 31) == 0;
+}
 
 }  // namespace
+
+// A plain product with bf16 rows (a few rows: f32 as well) whose kernel ends in TILE_GLU or its counterpart for up to 16 rows.  Against f32 rows of gate and up
+// and a kernel of its own for the activation (the same bits): 1500 x 12288 x 2048 89.5 + 17.8 -> 91.6 us, 16 rows 17.0 + 4.6 -> 16.2.
+bool vmx_linear_glu_ok(const VmxLinear &p) {
+    const bool plain = !p.exact && p.batch == 1 && !p.row_ids && !p.block_expert && !p.bias && p.silu_end <= p.silu_begin && p.epilogue == VMX_EP_STORE &&
+                       p.out_scale == 1.0f;
+    if (!plain || p.M < 1 || p.N % 16 || !direct_ok(p)) return false;
+    return p.M <= 16 || (!p.a_f32 && tile_ok(p, true));
+}
+
+int vmx_linear_glu(const VmxLinear &p, float slope, float limit, hipStream_t st) {
+    VMX_REQUIRE(p.A && p.W && p.C && p.N > 0 && p.K > 0 && vmx_linear_glu_ok(p), "linear_glu: no gated epilogue for %d rows, [%d, %d]", p.M, p.N, p.K);
+    GluLinear g;
+    static_cast<VmxLinear &>(g) = p;
+    g.slope = slope, g.limit = limit;
+    if (p.M <= 16) launch_skinny_glu(g, st);
+    else if (int rc = launch_tile_glu(g, st)) return rc;
+    VMX_CHECK_LAUNCH("linear (gated)");
+    return VMX_OK;
+}
 
 int vmx_linear_launch(const VmxLinear &p, hipStream_t st) {
     VMX_REQUIRE(p.A && p.W && p.C, "linear: null pointer");
@@ -602,9 +684,7 @@ int vmx_linear_launch(const VmxLinear &p, hipStream_t st) {
         if (bm == 16) hipLaunchKernelGGL(linear_fma_kernel<16>, grid, dim3(256), 0, st, p);
         else hipLaunchKernelGGL(linear_fma_kernel<64>, grid, dim3(256), 0, st, p);
     } else {
-        // 16-byte loads straight from the operands: whole 8-element chunks, aligned rows
-        const bool direct = p.w_sk == 1 && p.K % 8 == 0 && p.w_sn % 8 == 0 && p.lda % 8 == 0 && p.a_bs % 8 == 0 && p.w_bs % 8 == 0 &&
-                            p.expert_stride % 8 == 0 && ((uintptr_t)p.W & 15) == 0 && ((uintptr_t)p.A & 31) == 0;
+        const bool direct = direct_ok(p);
         if (bm == 64 && tile_ok(p, direct)) {
             if (int rc = launch_tile(p, st)) return rc;
         } else if (bm == 16 && direct) {

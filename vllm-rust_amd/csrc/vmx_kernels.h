@@ -247,6 +247,10 @@ struct VmxLinear {
     int exact = 0;                     // 1: multiply in f32 on the vector ALU even where the matrix cores could take bf16 operands
 };
 extern "C" int vmx_linear_launch(const VmxLinear &p, hipStream_t st);
+// The product with a clamped gated activation behind its sums: W's rows are N / 2 gate rows and as many up rows, C is [M, N / 2] = g sigmoid(slope g) (u + 1) with
+// g = min(gate, limit) and u = the up product clamped to +- limit; for products that vmx_linear_glu_ok takes
+bool vmx_linear_glu_ok(const VmxLinear &p);
+extern "C" int vmx_linear_glu(const VmxLinear &p, float slope, float limit, hipStream_t st);
 
 // latent_attn.hip: out[h][r][d] = in[h][d][r], the key up-projection turned for q_abs = U_h^T q_h
 int vmx_latent_transpose_heads(uint16_t *out, const uint16_t *in, int heads, int dim, int kv_rank, hipStream_t st);
