@@ -48,19 +48,23 @@ def test_layers_match_oracle(models, rows):
         ids = out.cpu().numpy().astype(np.int32)
 
 
-@pytest.mark.parametrize("rows", [49, 64, 65, 130])
-def test_one_slice_prompts_match_the_decode_path(rows):
-    """Prompts whose linears take all of k in one slice pass bf16 sums on; 256 and 512 wide, so that every projection does."""
+_SMALL = dict(hidden_size=256, num_heads=4, num_kv_heads=2, head_dim=64, intermediate_size=512)
+_WIDE = dict(hidden_size=2048, num_heads=32, num_kv_heads=8, head_dim=128, intermediate_size=12288)
+
+
+@pytest.mark.parametrize("sizes,rows", [(_SMALL, 49), (_SMALL, 64), (_SMALL, 65), (_SMALL, 130), (_WIDE, 320), (_WIDE, 321), (_WIDE, 333), (_WIDE, 336), (_WIDE, 337)])
+def test_prompts_match_the_decode_path(sizes, rows):
+    """Prompts whose linears take all of k in one slice pass bf16 sums on (256 and 512 wide, so that every projection does); 1 to 16 rows behind the last
+    whole tile take a pass of their own (gate|up, q|k|v), none and 17 do not."""
     import torch
     import vllm_rust_amd as vmx
     from vllm_rust_amd.qwen3 import QuantizedQwen3ForCausalLM, Qwen3Spec
     vmx.init(0)
-    spec = Qwen3Spec(hidden_size=256, num_layers=2, num_heads=4, num_kv_heads=2, head_dim=64, intermediate_size=512, vocab_size=1000, max_position=256,
-                     num_blocks=16, max_batch=4, max_seq_len=160, max_prefill_tokens=130)
+    spec = Qwen3Spec(**sizes, num_layers=2, vocab_size=1000, max_position=512, num_blocks=24, max_batch=16, max_seq_len=384, max_prefill_tokens=rows)
     model = QuantizedQwen3ForCausalLM(spec)
     model.load_synthetic(seed=9)
     prompt = torch.randint(0, spec.vocab_size, (rows,), dtype=torch.int32, device="cuda", generator=torch.Generator(device="cuda").manual_seed(rows))
-    bt = torch.randperm(16, dtype=torch.int32, device="cuda")
+    bt = torch.randperm(24, dtype=torch.int32, device="cuda")
     got = torch.empty(spec.vocab_size, dtype=torch.bfloat16, device="cuda")
     _, want = model.forward(prompt, 0, bt)
     model.prefill(prompt, 0, bt, logits_last=got)

@@ -631,10 +631,10 @@ __device__ __forceinline__ void int4_gemm_ring_sums(unsigned char *smem, const u
                 const uint4 wv = wq[r][t];
                 const uint32_t w = i == 0 ? wv.x : i == 1 ? wv.y : i == 2 ? wv.z : wv.w;
                 uint4 bu;
-                bu.x = (w & 0x000F000Fu) | 0x43004300u;
-                bu.y = ((w >> 4) & 0x000F000Fu) | 0x43004300u;
-                bu.z = ((w >> 8) & 0x000F000Fu) | 0x43004300u;
-                bu.w = ((w >> 12) & 0x000F000Fu) | 0x43004300u;
+                bu.x = ((w << 3) & 0x00780078u) | 0x41804180u;   // 16 + nibble: sums a sixth the size of those of 128 + nibble
+                bu.y = ((w >> 1) & 0x00780078u) | 0x41804180u;
+                bu.z = ((w >> 5) & 0x00780078u) | 0x41804180u;
+                bu.w = ((w >> 9) & 0x00780078u) | 0x41804180u;
                 acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, au), __builtin_bit_cast(vmx_bf16x8, bu), acc[t], 0, 0, 0);
             }
         }
@@ -642,7 +642,7 @@ __device__ __forceinline__ void int4_gemm_ring_sums(unsigned char *smem, const u
         for (int t = 0; t < CT; t++) {
             const uint32_t szw = zq[r][t];
             const float sc = __uint_as_float(szw << 16);
-            const float zo = __uint_as_float(szw & 0xFFFF0000u);
+            const float zo = __uint_as_float(szw & 0xFFFF0000u) - 112.f;
             fin[t][0] += sc * (acc[t][0] - zo * acc1[0]);
             fin[t][1] += sc * (acc[t][1] - zo * acc1[1]);
             fin[t][2] += sc * (acc[t][2] - zo * acc1[2]);
@@ -1772,9 +1772,9 @@ inline size_t gemm_lds_bytes(int M, int upw) {
 }
 
 int launch_gemm(const GemmPlan &p, const uint4 *W, const uint32_t *SZ, const uint16_t *x, const uint16_t *bias, uint16_t *y,
-                float *partial, int M, int N, int K, int group, hipStream_t st, int slice_rows = 0) {
+                float *partial, int M, int N, int K, int group, hipStream_t st, int slice_rows = 0, bool ring = false) {
     if (slice_rows <= 0) slice_rows = M;
-    if (const int rct = ring_ct(M, N, K, p)) {
+    if (const int rct = ring_ct(ring ? 16 : M, N, K, p)) {   // ring: for fewer rows than it is chosen for as well
         const dim3 rgrid((unsigned)((N / NT / rct) * p.splits));
 #define RING_C(U, C) hipLaunchKernelGGL((int4_gemm_ring_kernel<U, false, C>), rgrid, dim3(256), RING_LDS, st, W, SZ, x, bias, y, partial, M, N, K, group, slice_rows)
 #define RING(U) do { if (rct == 3) RING_C(U, 3); else if (rct == 2) RING_C(U, 2); else RING_C(U, 1); } while (0)
@@ -1949,23 +1949,43 @@ int vmx_int4_splits(int N, int K) { return plan_gemm(N, K).splits; }
 // 36 / 32 / 34 / 36: 2; 1024 rows 39 / 49 / 55 / 58: 1;  4096 x 12288, 333 rows 95 / 59 / 64: 2; 640 rows 97 / 91 / 75: 3; 800 rows 97 / 98 / 107: 2; 2048 rows
 // 189 / 212 / 219: 1;  2048 x 4096, 640 rows 36 / 30 / 27 / 32: 3;  6144 x 4096, 256 rows 36 / 31: 2; 640 rows 38 / 48: 1; 2048 rows 100 / 131: 1.  Over 140 shapes of
 // 49 .. 2048 rows the taken count is within 4 % of the best but for eight, five of them 2048 deep (2048 x 2048, 800 rows 22 / 25 / 28 / 30: 2).
+static int64_t prompt_blocks_ns(int row_tiles, int N, int K, int slices) {   // the products, without their slices' way through memory
+    const int kblocks = K / KB, cus = vmx_num_cus(), kbs = (kblocks + slices - 1) / slices;
+    const int64_t w = ((int64_t)(N >> 8) * row_tiles * slices + cus - 1) / cus;
+    return kbs * (1955 * (w / 2) + 1150 * (w % 2));
+}
+static int64_t prompt_slice_ns(int M, int N) { return (int64_t)M * N * 8 / 4500; }
 static int prompt_slices(int M, int N, int K, bool own_pass) {
-    const int plan = plan_gemm(N, K).splits, kblocks = K / KB, cus = vmx_num_cus();
+    const int plan = plan_gemm(N, K).splits, kblocks = K / KB;
     if (plan == 1 || !tiled_ok(M, N, K) || !tiled_wide_ok(M, N, K)) return plan;
-    const int64_t tiles = (int64_t)(N >> 8) * ((M + PF_BM - 1) / PF_BM), slice_ns = (int64_t)M * N * 8 / 4500;
+    const int64_t slice_ns = prompt_slice_ns(M, N);
     int best = plan;
     int64_t least = INT64_MAX;
     for (int s = 1; s <= plan; s++) {
         const int kbs = (kblocks + s - 1) / s;
         if ((s - 1) * kbs >= kblocks) continue;   // the last slice would be empty
-        const int64_t w = (tiles * s + cus - 1) / cus, ns = kbs * (1955 * (w / 2) + 1150 * (w % 2)) + (own_pass ? (s > 1) * (3000 + s * slice_ns) : s * slice_ns);
+        const int64_t ns = prompt_blocks_ns((M + PF_BM - 1) / PF_BM, N, K, s) + (own_pass ? (s > 1) * (3000 + s * slice_ns) : s * slice_ns);
         if (ns < least) least = ns, best = s;
     }
     return best;
 }
 
+// Up to 16 rows behind the last whole 64-row tile take a pass of the 16-row form instead of a tile that is mostly empty, where that leaves the tiles a round
+// less by the estimates: a k-block takes a tile as long with one row as with 64 (the weights have to come and to be unpacked), the 16-row form streams them at
+// 3 TB/s and more.  It leaves the plan's slices, so the tiles have to as well.  us, 333 rows of Qwen3-8B, tiles alone / with 13 rows apart: gate|up 98.8 /
+// 69.6 + 12.6, down 59 / 39.4 + 9.4, q|k|v 34.0 / 26.6 + 6.0; the prompt (9 layers) 2352 -> 2143.  bf16 results that differ from the rounded exact ones: tiles 0.8e-4 .. 4.7e-4, the
+// 16-row form 1.2e-4 .. 4.6e-4 (rows of mean 0 and 5, of sizes 2^-12 .. 2^12, with outliers of 100; 1.5e-4 .. 25e-4 before its weights became 16 + nibble)
+static int prompt_tail(int M, int N, int K) {
+    const int tail = M % PF_BM, full = M - tail, tiles = full / PF_BM;
+    const GemmPlan p = plan_gemm(N, K);
+    if (tail == 0 || tail > 16 || full == 0 || !tiled_ok(full, N, K) || !tiled_wide_ok(M, N, K) || !ring_ct(16, N, K, p)) return 0;
+    const int now = prompt_slices(M, N, K, false);
+    const int64_t ring = 2500 + (int64_t)K * N / 6000, slices = p.splits == 1 ? 0 : (p.splits - now) * prompt_slice_ns(M, N);
+    return (prompt_blocks_ns(tiles, N, K, p.splits) + ring + slices) * 20 <= prompt_blocks_ns(tiles + 1, N, K, now) * 19 ? tail : 0;
+}
+
 // Slices that vmx_int4_gemm_partial writes for M rows, at most vmx_int4_splits
-int vmx_int4_splits_rows(int M, int N, int K) { return prompt_slices(M, N, K, false); }
+int vmx_int4_splits_rows(int M, int N, int K) { return prompt_tail(M, N, K) ? plan_gemm(N, K).splits : prompt_slices(M, N, K, false); }
 
 // partial[vmx_int4_splits_rows][M][N] f32, also with one slice.  Arguments must already satisfy check_int4_shape.
 int vmx_int4_gemm_partial(const void *packed, const uint16_t *x, float *partial, int M, int N, int K, int group, hipStream_t st) {
@@ -1973,10 +1993,10 @@ int vmx_int4_gemm_partial(const void *packed, const uint16_t *x, float *partial,
     const uint4 *W = (const uint4 *)packed;
     const uint32_t *SZ = (const uint32_t *)((const char *)packed + sz_offset_bytes(K, N));
     if (tiled_ok(M, N, K)) {   // prompt chunk
-        const int splits = vmx_int4_splits_rows(M, N, K), kblocks = K / KB, kbs = (kblocks + splits - 1) / splits;
-        launch_tiled<false, false>(W, SZ, x, partial, nullptr, M, N, K, group, kbs, M, Int4GroupedArgs{}, (M + PF_BM - 1) / PF_BM, splits, st);
+        const int tail = prompt_tail(M, N, K), full = M - tail, splits = vmx_int4_splits_rows(M, N, K), kblocks = K / KB, kbs = (kblocks + splits - 1) / splits;
+        launch_tiled<false, false>(W, SZ, x, partial, nullptr, full, N, K, group, kbs, M, Int4GroupedArgs{}, (full + PF_BM - 1) / PF_BM, splits, st);
         VMX_CHECK_LAUNCH("int4_gemm(tiled)");
-        return VMX_OK;
+        return tail ? launch_gemm(p, W, SZ, x + (int64_t)full * K, nullptr, nullptr, partial + (int64_t)full * N, tail, N, K, group, st, M, true) : VMX_OK;
     }
     for (int m0 = 0; m0 < M; m0 += 16) {   // 16 rows (one MFMA row tile) per launch; every launch re-streams the weights
         const int mm = M - m0 < 16 ? M - m0 : 16;
@@ -1986,7 +2006,7 @@ int vmx_int4_gemm_partial(const void *packed, const uint16_t *x, float *partial,
 }
 
 // y [M][N] = bf16(x W) where the prompt-shaped kernel takes all of k in one slice
-bool vmx_int4_gemm_y_ok(int M, int N, int K) { return tiled_ok(M, N, K) && tiled_wide_ok(M, N, K) && prompt_slices(M, N, K, false) == 1; }
+bool vmx_int4_gemm_y_ok(int M, int N, int K) { return tiled_ok(M, N, K) && tiled_wide_ok(M, N, K) && !prompt_tail(M, N, K) && prompt_slices(M, N, K, false) == 1; }
 int vmx_int4_gemm_y(const void *packed, const uint16_t *x, uint16_t *y, int M, int N, int K, int group, hipStream_t st) {
     VMX_REQUIRE(vmx_int4_gemm_y_ok(M, N, K), "int4_gemm_y: shape [%d x %d -> %d] takes slices", M, K, N);
     launch_tiled<false, false>((const uint4 *)packed, (const uint32_t *)((const char *)packed + sz_offset_bytes(K, N)), x, nullptr, nullptr, M, N, K, group,
@@ -2254,18 +2274,19 @@ int vmx_int4_gemm_glu(const void *packed, const uint16_t *x, uint16_t *act, int 
     VMX_REQUIRE(p.splits == 1, "int4_gemm_glu: linear [%d -> %d] is split over k", K, N);
     const uint4 *W = (const uint4 *)packed;
     const uint32_t *SZ = (const uint32_t *)((const char *)packed + sz_offset_bytes(K, N));
+    int done = 0, apart = 0;
     if (tiled_ok(M, N, K)) {
-        launch_tiled<true, false>(W, SZ, x, nullptr, act, M, N, K, group, K / KB, M, Int4GroupedArgs{}, (M + PF_BM - 1) / PF_BM, 1, st);
+        apart = p.upw >= 4 ? prompt_tail(M, N, K) : 0, done = M - apart;
+        launch_tiled<true, false>(W, SZ, x, nullptr, act, done, N, K, group, K / KB, done, Int4GroupedArgs{}, (done + PF_BM - 1) / PF_BM, 1, st);
         VMX_CHECK_LAUNCH("int4_gemm(tiled glu)");
-        return VMX_OK;
     }
     const bool tail = (K / KB) % (4 * p.upw) != 0;
     const dim3 grid((unsigned)(N / NT)), block(256);
-    for (int m0 = 0; m0 < M; m0 += 16) {
+    for (int m0 = done; m0 < M; m0 += 16) {
         const int mm = M - m0 < 16 ? M - m0 : 16;
         const uint16_t *xc = x + (int64_t)m0 * K;
         uint16_t *ac = act + (int64_t)m0 * (N / 2);
-        if (const int rct = p.upw >= 4 ? ring_ct(mm, N, K, p) : 0) {
+        if (const int rct = p.upw >= 4 ? ring_ct(apart ? 16 : mm, N, K, p) : 0) {
             const dim3 rgrid((unsigned)(N / NT / rct));
 #define GRING_C(U, C) hipLaunchKernelGGL((int4_gemm_ring_kernel<U, true, C>), rgrid, block, RING_LDS, st, W, SZ, xc, nullptr, ac, nullptr, mm, N, K, group, mm)
 #define GRING(U) do { if (rct == 3) GRING_C(U, 3); else if (rct == 2) GRING_C(U, 2); else GRING_C(U, 1); } while (0)
