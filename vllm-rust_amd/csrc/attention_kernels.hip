@@ -12,6 +12,7 @@
 // (details at the kernel).  At most 64 partitions per sequence; a second kernel (or the consumer)
 // merges them.
 #include "tile_gemm.h"
+#include <algorithm>
 #include "vmx_kernels.h"
 #include <float.h>
 #include <mutex>
@@ -1112,21 +1113,23 @@ typedef short vmx_s16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 vmx_f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 vmx_f16x8 __attribute__((ext_vector_type(8)));
 
-template <int HD, int QPK, int FP8>
-__global__ __launch_bounds__(256) void prefill_attn_kernel(uint16_t *__restrict__ out, const uint16_t *__restrict__ q,
+// A workgroup is NG groups of HPW TT waves.  Each group walks every NG-th tile of the same keys for the same queries, in LDS of its own; the first group merges
+// the running sums at the end.  With one group a prompt of 256 tokens is 64 workgroups that walk a chain of up to 16 tiles, 1.7 us each.
+template <int HD, int QPK, int FP8, int TT, int NG>
+__global__ __launch_bounds__(64 * (QPK < 4 ? QPK : 4) * TT * NG) void prefill_attn_kernel(uint16_t *__restrict__ out, const uint16_t *__restrict__ q,
                                                             const void *__restrict__ k_cache, const void *__restrict__ v_cache,
                                                             const int32_t *__restrict__ block_table, int q_len, int offset, float scale,
                                                             int num_heads, int num_kv_heads, int block_size, int window,
                                                             const float *__restrict__ k_scale_ptr, const float *__restrict__ v_scale_ptr,
                                                             int out_f16) {   // out_f16: results rounded to bf16 go out as fp16
     constexpr int HPW = QPK < 4 ? QPK : 4;   // query heads per workgroup
-    constexpr int TT = 4 / HPW;              // 16-token query tiles per workgroup
+    constexpr int GT = 64 * HPW * TT;        // threads of a group; TT 16-token query tiles per workgroup
     constexpr int KSTEPS = HD / 32, DT = HD / 16;
     constexpr int KROW = HD + 8;             // bf16 per K row in LDS (16 B pad)
     constexpr int VROW = 20;                 // bf16 per V^T row: 16 tokens + pad (rows stay 8-byte aligned)
-    constexpr int BUF = 16 * KROW + HD * VROW, CHUNKS = HD / 128;   // 16 x HD / 8 pieces of eight elements, CHUNKS a thread
-    extern __shared__ __align__(16) uint16_t pf_lds[];              // two tiles, written and read in turn
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int BUF = 16 * KROW + HD * VROW, CHUNKS = 2 * HD / GT;   // 16 x HD / 8 pieces of eight elements, CHUNKS a thread (0: one for the first 2 HD)
+    extern __shared__ __align__(16) uint16_t pf_lds[];              // two tiles a group, written and read in turn
+    const int group = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / GT) : 0, tid = threadIdx.x - group * GT, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, n = lane & 15;
     const int hh = wave % HPW, tt = wave / HPW;
     constexpr int HGROUPS = QPK / HPW;
@@ -1169,20 +1172,22 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(uint16_t *__restrict_
 #pragma unroll
         for (int i = 0; i < (CHUNKS > 0 ? CHUNKS : 1); i++)
             if (CHUNKS > 0 || tid < 2 * HD) {
-                kr[i] = load8_raw<FP8>(k_cache, base + (dc0 + 16 * i) * 8);
-                vr[i] = load8_raw<FP8>(v_cache, base + (dc0 + 16 * i) * 8);
+                kr[i] = load8_raw<FP8>(k_cache, base + (dc0 + GT / 16 * i) * 8);
+                vr[i] = load8_raw<FP8>(v_cache, base + (dc0 + GT / 16 * i) * 8);
             }
     };
     int blk_next = 0, turn = 0;
+    constexpr int STEP = 16 * NG;   // of a group
     if (lo < hi) {
-        request(lo, entry(lo));
-        blk_next = entry(lo + 16);
+        request(lo + 16 * group, entry(lo + 16 * group));
+        blk_next = entry(lo + 16 * group + STEP);
     }
-    for (int t0 = lo; t0 < hi; t0 += 16, turn ^= 1) {
-        uint16_t *Ks = pf_lds + turn * BUF, *Vt = Ks + 16 * KROW;
+    for (int first = lo; first < hi; first += STEP, turn ^= 1) {   // the same count in every group: a tile past the end is nobody's need
+        const int t0 = first + 16 * group;
+        uint16_t *Ks = pf_lds + (2 * group + turn) * BUF, *Vt = Ks + 16 * KROW;
 #pragma unroll
         for (int i = 0; i < (CHUNKS > 0 ? CHUNKS : 1); i++) {
-            const int dc = dc0 + 16 * i;
+            const int dc = dc0 + GT / 16 * i;
             if (CHUNKS == 0 && tid >= 2 * HD) continue;
             if constexpr (kv16<FP8>()) {   // bf16 or fp16 rows: the bits go to LDS as they are
                 *reinterpret_cast<uint4 *>(&Ks[tok * KROW + dc * 8]) = kr[i];
@@ -1201,9 +1206,9 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(uint16_t *__restrict_
                 for (int e = 0; e < 8; e++) Vt[(dc * 8 + e) * VROW + tok] = (uint16_t)(__float_as_uint(vf[e]) >> 16);
             }
         }
-        if (t0 + 16 < hi) {
-            request(t0 + 16, blk_next);
-            blk_next = entry(t0 + 32);
+        if (first + STEP < hi) {
+            request(t0 + STEP, blk_next);
+            blk_next = entry(t0 + 2 * STEP);
         }
         __syncthreads();   // one a tile: a wave that is a tile ahead writes the other buffer
         // wave-uniform: does this KV tile intersect the wave's causal / window range at all
@@ -1255,6 +1260,31 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(uint16_t *__restrict_
     }
     float l = l_part + vmx_lane_xor<16>(l_part);
     l += vmx_lane_xor<32>(l);
+    if constexpr (NG > 1) {
+        __syncthreads();   // the last tiles have been read
+        constexpr int PER = 4 * DT + 2;   // a lane's sums, maximum and weight sum, [wave][value][lane]
+        float *parts = reinterpret_cast<float *>(pf_lds) + (int64_t)(group - 1) * (GT * PER) + wave * 64 * PER + lane;
+        if (group > 0) {
+#pragma unroll
+            for (int d = 0; d < DT; d++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) parts[64 * (4 * d + i)] = acc[d][i];
+            parts[64 * (PER - 2)] = m_run, parts[64 * (PER - 1)] = l;
+        }
+        __syncthreads();
+        if (group > 0) return;
+#pragma unroll
+        for (int gi = 1; gi < NG; gi++) {
+            const float *from = reinterpret_cast<const float *>(pf_lds) + (int64_t)(gi - 1) * (GT * PER) + wave * 64 * PER + lane;
+            const float m_other = from[64 * (PER - 2)], m_new = fmaxf(m_run, m_other), mine = __expf(m_run - m_new), its = __expf(m_other - m_new);
+            l = l * mine + from[64 * (PER - 1)] * its;
+            m_run = m_new;
+#pragma unroll
+            for (int d = 0; d < DT; d++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[d][i] = acc[d][i] * mine + from[64 * (4 * d + i)] * its;
+        }
+    }
     if (q_valid) {
         const float inv = vsc / l;
         uint16_t *o = out + ((int64_t)qi * num_heads + head) * HD;
@@ -1271,18 +1301,41 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(uint16_t *__restrict_
     }
 }
 
-template <int HD, int QPK, int FP8>
-int launch_prefill(hipStream_t st, uint16_t *out, const uint16_t *q, const void *kc, const void *vc, const int32_t *bt, int q_len, int offset,
-                   float scale, int H, int KVH, int bs, int window, const float *ks, const float *vs, int out_f16) {
-    constexpr int HPW = QPK < 4 ? QPK : 4, TT = 4 / HPW;
+template <int HD, int QPK, int FP8, int TT, int NG>
+int launch_prefill_as(hipStream_t st, uint16_t *out, const uint16_t *q, const void *kc, const void *vc, const int32_t *bt, int q_len, int offset,
+                      float scale, int H, int KVH, int bs, int window, const float *ks, const float *vs, int out_f16) {
+    constexpr int HPW = QPK < 4 ? QPK : 4, GT = 64 * HPW * TT;
     const dim3 grid((q_len + 16 * TT - 1) / (16 * TT), KVH * (QPK / HPW));
-    constexpr size_t lds = 2 * (16 * (HD + 8) + HD * 20) * 2;
+    constexpr size_t tiles = (size_t)NG * 2 * (16 * (HD + 8) + HD * 20) * 2, sums = (size_t)(NG - 1) * GT * (HD / 4 + 2) * 4, lds = tiles > sums ? tiles : sums;
+    static_assert(lds <= 160 * 1024, "the groups' tiles and sums fit");
     if (lds > 64 * 1024)
-        VMX_CHECK_HIP(hipFuncSetAttribute((const void *)prefill_attn_kernel<HD, QPK, FP8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((prefill_attn_kernel<HD, QPK, FP8>), grid, dim3(256), lds, st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window,
+        VMX_CHECK_HIP(hipFuncSetAttribute((const void *)prefill_attn_kernel<HD, QPK, FP8, TT, NG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((prefill_attn_kernel<HD, QPK, FP8, TT, NG>), grid, dim3(GT * NG), lds, st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window,
                        ks, vs, out_f16);
     VMX_CHECK_LAUNCH("prefill_attention");
     return VMX_OK;
+}
+
+// Wide heads, from five key tiles on: several groups share the keys of a workgroup.  256 wide, four groups where the workgroups then still have a compute unit each
+// (the groups' tiles fill its LDS), two up to the workgroups that the units hold, else one.  512 wide, two at any length: a workgroup of one group has a unit's
+// registers to itself as well.  us, one group / this, FP8 cache, no history, tokens 17 / 100 / 256 / 512 / 1024 / 2048 / 4096: 16 heads over 8, 256 wide, window 1024
+// 7.4 14.0 28.2 52.4 101 129 247 / 7.4 12.6 17.6 27.5 60 123 249; 16 heads over one, 512 wide 11.5 22.7 44.3 81 159 537 1660 / 11.4 20.7 33.4 54 99 325 974.
+template <int HD, int QPK, int FP8, class... A>
+int launch_prefill(hipStream_t st, uint16_t *out, const uint16_t *q, const void *kc, const void *vc, const int32_t *bt, int q_len, int offset,
+                   float scale, int H, int KVH, int bs, int window, A... rest) {
+    constexpr int HPW = QPK < 4 ? QPK : 4, TT = 4 / HPW;
+    const int64_t keys = window > 0 ? std::min<int64_t>((int64_t)offset + q_len, (int64_t)window + 16 * TT) : (int64_t)offset + q_len;
+    if constexpr (HD >= 256) {
+        const int64_t tiles = ((int64_t)q_len + 15) / 16, columns = (int64_t)KVH * (QPK / HPW), cus = vmx_num_cus();
+        if constexpr (HD == 256 && HPW < 4) {
+            constexpr int FEW = 2 / HPW;   // 128 threads a group, four groups
+            if (keys > 64 && (tiles + FEW - 1) / FEW * columns <= cus)
+                return launch_prefill_as<HD, QPK, FP8, FEW, 4>(st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window, rest...);
+        }
+        if (keys > 64 && (HD == 512 || (tiles + TT - 1) / TT * columns <= 2 * cus))
+            return launch_prefill_as<HD, QPK, FP8, TT, 2>(st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window, rest...);
+    }
+    return launch_prefill_as<HD, QPK, FP8, TT, 1>(st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window, rest...);
 }
 }  // namespace
 
