@@ -66,12 +66,18 @@ struct WinAttn {
     int window, keep_first, tokens, heads, kv_heads, dim, vdim, block_size;
     const int32_t *seq_starts;   // matrix-core form: sequence s owns the packed rows seq_starts[s] .. seq_starts[s + 1] - 1
     int num_seqs;
-    int bs_shift;                // log2(block_size) when it is a power of two, else -1
+    uint32_t bs_mul;             // 2^32 / block_size, rounded down (one block per key: 2^32 - 1)
     int parts;                   // > 1: the key tiles of a run are dealt to `parts` workgroups, whose results go to `ws` for the merge
     float *ws;                   // [tokens, heads, parts, vdim + 2]: unnormalised sums, running maximum, denominator
     const uint16_t *sink, *r1, *r2, *talk;   // extras, each NULL when absent
     int gate_elem;               // 1: gate rows hold heads * vdim numbers
     int chunk;                   // > 0: only keys of the query's own chunk of positions
+    // block and offset of position j.  The product is j / block_size or one less: j (2^32 / block_size - bs_mul) < j < 2^31
+    __device__ __forceinline__ void place(int j, int &block, int &offset) const {
+        block = (int)__umulhi((uint32_t)j, bs_mul);
+        offset = j - block * block_size;
+        if (offset >= block_size) offset -= block_size, block++;
+    }
     // first key of the run that ends at position i
     __device__ __forceinline__ int first_key(int i) const {
         const int lo = window > 0 ? max(0, i - window + 1) : 0;
@@ -437,8 +443,11 @@ __global__ __launch_bounds__(512) void window_attn_talk_kernel(const WinAttn p) 
 //   O^T += V^T P^T (A = transposed value rows from LDS, B = those scores after the softmax, as a bf16 pair hi + lo so that the
 //                 weights keep f32 precision): lane (c, g) accumulates value columns 16 vs + 4 g + r of query c.
 // Every statistic of a query therefore lives in the four lanes (c, 0..3): the softmax needs two lane exchanges per tile.
+// Latency bounds it, the trips to the block table most: a branch around each of a thread's eight lookups a tile made eight trips of them, one after
+// another.  Without branches they are one trip, a thread's value chunks share theirs, and a tile that every row sees whole is not masked: 16 heads
+// over 4 of 128, a prompt of 1500 rows 66 -> 45 us, 16 rows at 1000 keys 28 -> 22.
 template <int DS, int VS>
-__global__ __launch_bounds__(256) void window_attn_mfma_kernel(const WinAttn p) {
+__global__ __launch_bounds__(256, DS <= 4 ? 3 : 2) void window_attn_mfma_kernel(const WinAttn p) {
     constexpr int KT = 64, LDK = 32 * DS + 8, LDV = KT + 8, KCH = DS, VCH = (VS + 1) / 2;
     __shared__ __align__(16) uint16_t Ks[KT * LDK];
     __shared__ __align__(16) uint16_t Vt[16 * VS * LDV];
@@ -468,6 +477,7 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(const WinAttn p) 
     const uint16_t *kc = (const uint16_t *)p.kc, *vc = (const uint16_t *)p.vc;
     const int qrow = 16 * sub + fl, qi = i0 + qrow, qlo = p.first_key(qi);
     const bool qlive = active && qrow < nrows;
+    const int last_lo = p.first_key(i0 + min(16 * sub + 15, nrows - 1));
     // this workgroup's share of the run's key tiles
     const int ntile = (nk + KT - 1) / KT, per = (ntile + p.parts - 1) / p.parts;
     const int kb0 = share * per * KT, kb1 = min(nk, (share + 1) * per * KT);
@@ -494,51 +504,44 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(const WinAttn p) 
     const float inv_cap = p.softcap > 0.f ? 1.0f / p.softcap : 0.f;
     const float dr1 = p.r1 ? vmx_bf16_to_f32(p.r1[head]) : 0.f, dr2 = p.r1 ? vmx_bf16_to_f32(p.r2[head]) : 0.f;
     uint4 kr[KCH], vr[VCH];
-    int krow[KCH], vrow[VCH];    // cache rows of the tile to fetch next: looked up one tile earlier, so that a fetch is one trip to memory
-    auto cache_row = [&](int idx) -> int {
-        if (idx >= nk) return 0;
-        const int j = idx < na ? idx : lo + (idx - na);
-        if (p.bs_shift >= 0) return (bt[j >> p.bs_shift] << p.bs_shift) + (j & (p.block_size - 1));
-        return bt[j / p.block_size] * p.block_size + j % p.block_size;
+    // Block and offset of the keys to fetch next are looked up one tile earlier, so that a fetch is one trip to memory, and without a branch, so that
+    // the table reads of a tile are in flight together: places beyond the last key take that key's.
+    // A thread's chunks of a tile: the keys tid / (4 DS) + c 64 / DS at one part of the head, and the value parts tid / 64 + 4 c of one key.
+    static_assert(KT == 64 && 256 % (4 * DS) == 0 && 2 * VS == 4 * VCH, "whole chunks of 16 bytes for every thread");
+    const int kkey = tid / (4 * DS), kpart = tid % (4 * DS), vkey = tid % KT, vpart = tid / KT;
+    const bool kin = 8 * kpart < D;
+    const uint16_t *kbase = kc + (int64_t)kvh * D + (kin ? 8 * kpart : 0), *vbase = vc + (int64_t)kvh * V;
+    int kblock[KCH], koff[KCH], vblock, voff;
+    auto place = [&](int idx, int &block, int &offset) {
+        idx = min(idx, nk - 1);
+        p.place(idx < na ? idx : lo + (idx - na), block, offset);
+        block = bt[block];
     };
     auto lookup = [&](int kb) {
 #pragma unroll
-        for (int c = 0; c < KCH; c++) krow[c] = cache_row(kb + (tid + 256 * c) / (4 * DS));
-#pragma unroll
-        for (int c = 0; c < VCH; c++) vrow[c] = cache_row(kb + (tid + 256 * c) % KT);
+        for (int c = 0; c < KCH; c++) place(kb + kkey + c * (64 / DS), kblock[c], koff[c]);
+        place(kb + vkey, vblock, voff);
     };
-    auto fetch = [&](int kb) {
+    auto fetch = [&]() {
 #pragma unroll
-        for (int c = 0; c < KCH; c++) {
-            const int ch = tid + 256 * c, kk = ch / (4 * DS), part = ch % (4 * DS);
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (kb + kk < kb1 && 8 * part < D) v = *reinterpret_cast<const uint4 *>(kc + (int64_t)krow[c] * kw + (int64_t)kvh * D + 8 * part);
-            kr[c] = v;
-        }
+        for (int c = 0; c < KCH; c++) kr[c] = *reinterpret_cast<const uint4 *>(kbase + (int64_t)(kblock[c] * p.block_size + koff[c]) * kw);
+        const uint16_t *row = vbase + (int64_t)(vblock * p.block_size + voff) * vw;
 #pragma unroll
         for (int c = 0; c < VCH; c++) {
-            const int ch = tid + 256 * c, kk = ch % KT, part = ch / KT;   // a wave's lanes: 64 keys, so that their LDS columns differ
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (ch < KT * 2 * VS && kb + kk < kb1 && 8 * part < V) v = *reinterpret_cast<const uint4 *>(vc + (int64_t)vrow[c] * vw + (int64_t)kvh * V + 8 * part);
-            vr[c] = v;
+            const int at = 8 * (vpart + 4 * c);
+            vr[c] = *reinterpret_cast<const uint4 *>(row + (at < V ? at : 0));   // columns beyond the head: of sums that nobody stores
         }
     };
     auto stash = [&]() {
 #pragma unroll
-        for (int c = 0; c < KCH; c++) {
-            const int ch = tid + 256 * c, kk = ch / (4 * DS), part = ch % (4 * DS);
-            *reinterpret_cast<uint4 *>(Ks + kk * LDK + 8 * part) = kr[c];
-        }
+        for (int c = 0; c < KCH; c++) *reinterpret_cast<uint4 *>(Ks + (kkey + c * (64 / DS)) * LDK + 8 * kpart) = kin ? kr[c] : make_uint4(0, 0, 0, 0);
+        // a key of the tile sits in k slot `col`: the order in which the score registers of a lane line up as an operand
+        const int col = 32 * (vkey >> 5) + 8 * ((vkey & 15) >> 2) + (vkey & 3) + 4 * ((vkey >> 4) & 1);   // a wave's lanes: 64 keys, so that their LDS columns differ
 #pragma unroll
         for (int c = 0; c < VCH; c++) {
-            const int ch = tid + 256 * c, kk = ch % KT, part = ch / KT;
-            if (ch < KT * 2 * VS) {
-                // key kk of the tile sits in k slot `col`: the order in which the score registers of a lane line up as an operand
-                const int col = 32 * (kk >> 5) + 8 * ((kk & 15) >> 2) + (kk & 3) + 4 * ((kk >> 4) & 1);
-                const uint32_t w[4] = {vr[c].x, vr[c].y, vr[c].z, vr[c].w};
+            const uint32_t w[4] = {vr[c].x, vr[c].y, vr[c].z, vr[c].w};
 #pragma unroll
-                for (int e = 0; e < 8; e++) Vt[(8 * part + e) * LDV + col] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
-            }
+            for (int e = 0; e < 8; e++) Vt[(8 * (vpart + 4 * c) + e) * LDV + col] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
         }
     };
     float m = -FLT_MAX, den = 0.f;
@@ -546,13 +549,13 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(const WinAttn p) 
 #pragma unroll
     for (int v = 0; v < VS; v++) o[v] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
     lookup(kb0);
-    fetch(kb0);
+    fetch();
     lookup(kb0 + KT);
     stash();
     __syncthreads();
     for (int kb = kb0; kb < kb1; kb += KT) {
         if (kb + KT < kb1) {
-            fetch(kb + KT);
+            fetch();
             lookup(kb + 2 * KT);
         }
         if (active) {
@@ -567,17 +570,37 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(const WinAttn p) 
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, a), __builtin_bit_cast(vmx_bf16x8, qf[s]), acc, 0, 0, 0);
                 }
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int idx = kb + 16 * kt + 4 * fg + r;
-                    const int j = idx < na ? idx : lo + (idx - na);
-                    const bool vis = qlive && idx < kb1 && j <= qi && (j >= qlo || j < p.keep_first);
-                    float x = acc[r] * smul;
-                    if (p.softcap > 0.f) x = p.softcap * tanh_fast(x * inv_cap);
-                    if (p.r1) x -= dr1 * __logf(1.0f + dr2 * (float)max(qi - j, 0));
-                    sc[kt][r] = vis ? x : -FLT_MAX;
-                    tmax = fmaxf(tmax, sc[kt][r]);
-                }
+                for (int r = 0; r < 4; r++) sc[kt][r] = acc[r] * smul;
             }
+            if (p.softcap > 0.f) {
+#pragma unroll
+                for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) sc[kt][r] = p.softcap * tanh_fast(sc[kt][r] * inv_cap);
+            }
+            auto key_at = [&](int idx) { return idx < na ? idx : lo + (idx - na); };
+            if (p.r1) {
+#pragma unroll
+                for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) sc[kt][r] -= dr1 * __logf(1.0f + dr2 * (float)max(qi - key_at(kb + 16 * kt + 4 * fg + r), 0));
+            }
+            // every row of the wave sees every key of the tile: the first row its last, the last row its first
+            const bool whole = kb >= na && kb + KT <= kb1 && key_at(kb + KT - 1) <= i0 + 16 * sub && key_at(kb) >= last_lo;
+            if (!whole) {
+#pragma unroll
+                for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const int idx = kb + 16 * kt + 4 * fg + r, j = key_at(idx);
+                        const bool vis = qlive && idx < kb1 && j <= qi && (j >= qlo || j < p.keep_first);
+                        sc[kt][r] = vis ? sc[kt][r] : -FLT_MAX;
+                    }
+            }
+#pragma unroll
+            for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) tmax = fmaxf(tmax, sc[kt][r]);
             tmax = fmaxf(tmax, vmx_lane_xor<16>(tmax));
             tmax = fmaxf(tmax, vmx_lane_xor<32>(tmax));
             const float mn = fmaxf(m, tmax);
@@ -737,11 +760,11 @@ __global__ __launch_bounds__(TM_NT) void talk_attn_mfma_kernel(const WinAttn p) 
     const int nKch = KT * G * 4 * DS, nVch = KT * G * 2 * VS;
     uint4 kr[MAXCH], vr[MAXCH];
     int krow[MAXCH], vrow[MAXCH];
-    auto cache_row = [&](int idx) -> int {
-        if (idx >= nk) return 0;
-        const int j = idx < na ? idx : lo + (idx - na);
-        if (p.bs_shift >= 0) return (bt[j >> p.bs_shift] << p.bs_shift) + (j & (p.block_size - 1));
-        return bt[j / p.block_size] * p.block_size + j % p.block_size;
+    auto cache_row = [&](int idx) -> int {   // places beyond the last key take that key's: no branch, so a tile's table reads are in flight together
+        idx = min(idx, nk - 1);
+        int block, offset;
+        p.place(idx < na ? idx : lo + (idx - na), block, offset);
+        return bt[block] * p.block_size + offset;
     };
     auto lookup = [&](int kb) {
 #pragma unroll
@@ -1112,7 +1135,7 @@ extern "C" int vmx_window_attention_ex(void *out, int out_dtype, const float *q,
     if (tokens <= 0) return VMX_OK;
     WinAttn p{out, out_dtype == VMX_F32, q, ldq, k_cache, v_cache, block_tables, seq_ids, positions, max_blocks_per_seq, head_temp_bf16,
               gate, ldgate, scale, softcap, window, keep_first, tokens, heads, kv_heads, dim, vdim, block_size, seq_starts, num_seqs,
-              (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1, 1, (float *)workspace,
+              block_size > 1 ? (uint32_t)((1ull << 32) / (uint32_t)block_size) : ~0u, 1, (float *)workspace,
               ex.sink_bf16, ex.dist_r1_bf16, ex.dist_r2_bf16, ex.talk_bf16, ex.gate_per_element ? 1 : 0, ex.chunk};
     hipStream_t st = vmx_stream(stream);
     const bool f32 = cache_dtype == VMX_F32;
@@ -1177,12 +1200,14 @@ extern "C" int vmx_window_attention_ex(void *out, int out_dtype, const float *q,
         const int qpk = heads / kv_heads, hq = qpk < 4 ? qpk : 4, rt = 16 * (4 / hq);
         const int runs = tokens / rt + num_seqs;                              // at most one partly filled run per sequence
         const int base = runs * kv_heads * ((qpk + 3) / 4);
-        // few workgroups: deal each run's key tiles to several, up to the two workgroups that a compute unit holds.  Decode of a model with 16
-        // heads over 4, rows x tokens, attention and merge, up to one -> up to two workgroups: 16 x 1000 40.0 -> 29.8 us, 16 x 300 19.5 -> 16.8,
-        // 12 x 700 24.0 -> 19.4, 8 x 1500 25.0 -> 23.6, 16 x 100 14.7 -> 14.6.  Tables say how long a sequence can be, not how long it is: shares beyond
-        // its tiles leave at once and are launched last (16 x 100 in tables of 4096: 14.7; as whole shares among the others 15.9)
+        // few workgroups: deal each run's key tiles to several, up to the workgroups that a compute unit holds (three; two of heads wider than 128).
+        // Decode of a model with 16 heads over 4, rows x tokens, attention and merge, up to one -> up to two workgroups a compute unit: 16 x 1000
+        // 40.0 -> 29.8 us, 16 x 300 19.5 -> 16.8, 12 x 700 24.0 -> 19.4, 8 x 1500 25.0 -> 23.6, 16 x 100 14.7 -> 14.6; up to three: a step of 16 x 1000
+        // 476.7 -> 474.7.  Tables say how long a sequence can be, not how long it is: shares beyond its tiles leave at once and are launched last
+        // (16 x 100 in tables of 4096: 14.7; as whole shares among the others 15.9)
         if (workspace && base < 128) {
-            int parts = 512 / base < 16 ? 512 / base : 16;
+            const int held = dim <= 128 ? 768 : 512;
+            int parts = held / base < 16 ? held / base : 16;
             if (span > 0) parts = std::min(parts, (span + keep_first + rt + 63) / 64);
             parts = (int)std::min<int64_t>(parts, ((int64_t)max_blocks_per_seq * block_size + 63) / 64);   // no sequence is longer than its table
             parts = std::min<size_t>(parts, workspace_bytes / ((size_t)tokens * heads * (vdim + 2) * 4));
