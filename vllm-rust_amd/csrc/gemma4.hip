@@ -265,6 +265,89 @@ __global__ __launch_bounds__(64) void g4_qkv_post_kernel(const float *__restrict
     }
 }
 
+// The same with E = hd / 64 neighbouring elements a lane, four heads a workgroup of 256: reads and writes of 16 bytes, the partner of a rotated
+// element from its lane.  Memory bounds it (a prompt's slices, 33 MB at 256 rows), and 4-byte reads a few at a time
+// did not fill it: 256 rows, 16 heads over 8 of 256 in four slices 12.4 -> 8.5 us, over one of 512 13.5 -> 9.6 (a pass of 12 layers 2789 -> 2746).
+template <int E>
+__global__ __launch_bounds__(256) void g4_qkv_post_wide_kernel(const float *__restrict__ proj, int ntot, uint16_t *__restrict__ q_out,
+                                                               void *__restrict__ k_cache, void *__restrict__ v_cache,
+                                                               const uint16_t *__restrict__ q_norm_w, const uint16_t *__restrict__ k_norm_w,
+                                                               float eps, const float *__restrict__ cos_sin,
+                                                               const int32_t *__restrict__ positions, const int32_t *__restrict__ slots, int Hq,
+                                                               int Hkv, int rot_dim, int v_from_k, int fp8,
+                                                               const float *__restrict__ k_scale, const float *__restrict__ v_scale,
+                                                               uint16_t *__restrict__ stage, int slices, int tokens, int nheads) {
+    constexpr int hd = 64 * E;
+    const int w = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, i0 = E * lane;
+    const int t = __builtin_amdgcn_readfirstlane(w / nheads), head = __builtin_amdgcn_readfirstlane(w - w / nheads * nheads);
+    if (t >= tokens) return;
+    const bool is_q = head < Hq, is_k = !is_q && head < Hq + Hkv;
+    const int src_head = !is_q && !is_k && v_from_k ? head - Hkv : head;
+    const float *src = proj + (int64_t)t * ntot + (int64_t)src_head * hd + i0;
+    const uint16_t *nw = is_q ? q_norm_w : (is_k ? k_norm_w : nullptr);
+    const int pos = positions[t];
+    const int slot = (is_q || stage) ? 0 : slots[t];
+    const float kv_sc = (!is_q && !stage && fp8) ? (is_k ? *k_scale : *v_scale) : 1.0f;
+    float pv[E], wv[E], cv[E], sv[E];
+    auto load = [](float *to, const float *from) {
+#pragma unroll
+        for (int j = 0; j < E; j += 4) *reinterpret_cast<float4 *>(to + j) = *reinterpret_cast<const float4 *>(from + j);
+    };
+    load(pv, src);
+#pragma unroll
+    for (int j = 0; j < E; j++) wv[j] = nw ? vmx_bf16_to_f32(nw[i0 + j]) : 1.0f;
+#pragma unroll 4
+    for (int s = 1; s < slices; s++) {   // in slice order
+        float more[E];
+        load(more, src + (int64_t)s * tokens * ntot);
+#pragma unroll
+        for (int j = 0; j < E; j++) pv[j] += more[j];
+    }
+    const int half = rot_dim >> 1;
+    const bool rot = (is_q || is_k) && i0 < rot_dim, second = i0 >= half;   // whole lanes: half is a multiple of E
+    const float *cs = cos_sin + (int64_t)pos * rot_dim + (rot ? (second ? i0 - half : i0) : 0);
+    if (half > 0) load(cv, cs), load(sv, cs + half);
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < E; j++) {
+        pv[j] = rbf(pv[j]);
+        ss += pv[j] * pv[j];
+    }
+    ss = vmx_wave_sum(ss);
+    const float inv = rsqrtf(ss / (float)hd + eps);
+#pragma unroll
+    for (int j = 0; j < E; j++) pv[j] = rbf(pv[j] * inv * wv[j]);
+    if (half > 0) {
+        const int partner = rot ? (second ? lane - half / E : lane + half / E) : lane;
+#pragma unroll
+        for (int j = 0; j < E; j++) {
+            const float other = __shfl(pv[j], partner);
+            if (rot) pv[j] = rbf(second ? pv[j] * cv[j] + other * sv[j] : pv[j] * cv[j] - other * sv[j]);
+        }
+    }
+    auto store = [&](uint16_t *to) {
+        if constexpr (E == 8) *reinterpret_cast<uint4 *>(to) = pack8(pv);
+        else
+            *reinterpret_cast<uint2 *>(to) = make_uint2((uint32_t)vmx_f32_to_bf16(pv[0]) | ((uint32_t)vmx_f32_to_bf16(pv[1]) << 16),
+                                                        (uint32_t)vmx_f32_to_bf16(pv[2]) | ((uint32_t)vmx_f32_to_bf16(pv[3]) << 16));
+    };
+    if (is_q) return store(q_out + ((int64_t)t * Hq + head) * hd + i0);
+    const int kvh = is_k ? head - Hq : head - Hq - Hkv;
+    if (stage) return store(stage + ((int64_t)(is_k ? 0 : tokens) + t) * Hkv * hd + (int64_t)kvh * hd + i0);
+    if (slot < 0) return;
+    const int64_t dst = ((int64_t)slot * Hkv + kvh) * hd + i0;
+    void *cache = is_k ? k_cache : v_cache;
+    if (!fp8) return store((uint16_t *)cache + dst);
+#pragma unroll
+    for (int j = 0; j < E; j += 4) {
+        float a[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) a[e] = rbf(fminf(fmaxf(pv[j + e] / kv_sc, -448.0f), 448.0f));
+        const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(a[0], a[1], 0, false);
+        *reinterpret_cast<uint32_t *>((uint8_t *)cache + dst + j) = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a[2], a[3], lo, true);
+    }
+}
+
 // act[t, i] = bf16(bf16(gelu_erf(bf16(gate))) * bf16(up)) from f32 [tokens][2*inter] (gate columns first), 8 elements per
 // thread, plus the q8_1 form of the result for the down projection.
 __global__ __launch_bounds__(256) void g4_geglu_kernel(const float *__restrict__ gu, int tokens, uint16_t *__restrict__ act, int inter,
@@ -1056,11 +1139,20 @@ int g4_run_layers(vmx_gemma4 *m, const int32_t *input_ids, const int32_t *positi
                 return rc;
         } else {
             // a KV-shared layer launches the query heads only: its K/V for these tokens were written by the target layer
-            const auto post = qkv_left > 1 ? g4_qkv_post_kernel<true> : g4_qkv_post_kernel<false>;
-            hipLaunchKernelGGL(post, dim3(L.kv_shared ? Hq : Hq + 2 * Hkv, B), dim3(64), 0, st, qkv_left > 1 ? (const float *)m->gemm_part.p : proj, ntot, q, KV.k_cache.p,
-                               KV.v_cache.p, (const uint16_t *)L.q_norm.p, (const uint16_t *)L.k_norm.p, c.rms_norm_eps,
-                               (const float *)(L.sliding ? m->cos_sin_s.p : m->cos_sin_f.p), positions, slot_mapping, Hq, Hkv, hd, L.rot,
-                               L.k_eq_v ? 1 : 0, fp8, ks, ks + 1, first_write ? stage : nullptr, qkv_left);
+            const float *qkv = qkv_left > 1 ? (const float *)m->gemm_part.p : proj;
+            const float *cos_sin = (const float *)(L.sliding ? m->cos_sin_s.p : m->cos_sin_f.p);
+            const int nheads = L.kv_shared ? Hq : Hq + 2 * Hkv;
+            if ((hd == 256 || hd == 512) && L.rot % (hd / 32) == 0) {   // a rotated half ends with a lane, rows start on 16 bytes
+                const auto post = hd == 256 ? g4_qkv_post_wide_kernel<4> : g4_qkv_post_wide_kernel<8>;
+                hipLaunchKernelGGL(post, dim3(((int64_t)nheads * B + 3) / 4), dim3(256), 0, st, qkv, ntot, q, KV.k_cache.p, KV.v_cache.p,
+                                   (const uint16_t *)L.q_norm.p, (const uint16_t *)L.k_norm.p, c.rms_norm_eps, cos_sin, positions, slot_mapping, Hq, Hkv, L.rot,
+                                   L.k_eq_v ? 1 : 0, fp8, ks, ks + 1, first_write ? stage : nullptr, qkv_left, B, nheads);
+            } else {
+                const auto post = qkv_left > 1 ? g4_qkv_post_kernel<true> : g4_qkv_post_kernel<false>;
+                hipLaunchKernelGGL(post, dim3(nheads, B), dim3(64), 0, st, qkv, ntot, q, KV.k_cache.p, KV.v_cache.p, (const uint16_t *)L.q_norm.p,
+                                   (const uint16_t *)L.k_norm.p, c.rms_norm_eps, cos_sin, positions, slot_mapping, Hq, Hkv, hd, L.rot, L.k_eq_v ? 1 : 0, fp8, ks,
+                                   ks + 1, first_write ? stage : nullptr, qkv_left);
+            }
             if (first_write) {
                 const int64_t n = (int64_t)B * NKV;
                 if (int rc = vmx_kv_scales_calibrate_if_needed(L.kv_scales.p, stage, n, stage + n, n, m->kv_headroom, st)) return rc;
