@@ -61,20 +61,33 @@ __device__ __forceinline__ uint4 bf16_rows_as_f16(const uint4 v) {
     return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// One workgroup per token; thread t owns the 8-element chunks t, t+256, ... (CH of them) in registers.
+// One workgroup of NT per token; thread t owns the 8-element chunks t, t + NT, ... (CH of them) in registers.
 // PROMPT: o may lie in slices [slices][tokens][hidden], whose sum it is; x16 != nullptr: x as fp16 as well, what the products behind it read.  (Decode steps
 // have a form without either: their 5.2 us, four a step, were 6.2 with the choices in it.)  A 256-token prompt of Gemma-4-12B, where sums and conversions were
 // launches of their own: 3204 -> 2925 us for 12 layers.
+// NT: threads a row.  A prompt has a workgroup a row, so fewer rows than the chip has room for waves: 512 where a row has chunks for them (256 rows of
+// 3840 in four slices 8.64 -> 8.36 us, two a layer).
 //   o given:  o_r = bf16(o);  n = bf16(o_r * rsqrt(mean(o_r^2) + eps) * w_post);  h = bf16(n + h_in);
 //             scalar given: h = bf16(h * scalar)                       (post-norm, residual add, layer_scalar)
 //   always:   x = bf16(h * rsqrt(mean(h^2) + eps) * w_next)  (+ its q8_1 form)   (the next sub-block's pre-norm);
 //             w_next == nullptr: x = h (the per-layer-input gate projects the residual stream itself)
-template <int CH, bool PROMPT>
-__global__ __launch_bounds__(256) void g4_norm_kernel(uint16_t *__restrict__ h, const uint16_t *__restrict__ h_in, uint16_t *__restrict__ x, const float *__restrict__ o,
+template <int NT> __device__ __forceinline__ float g4_block_sum(float v, float *red) {
+    if constexpr (NT == 256) return vmx_block_sum_256(v, red);
+    v = vmx_wave_sum(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    float r = red[0];
+#pragma unroll
+    for (int i = 1; i < NT / 64; i++) r += red[i];
+    __syncthreads();
+    return r;
+}
+template <int CH, bool PROMPT, int NT>
+__global__ __launch_bounds__(NT) void g4_norm_kernel(uint16_t *__restrict__ h, const uint16_t *__restrict__ h_in, uint16_t *__restrict__ x, const float *__restrict__ o,
                                                        const uint16_t *__restrict__ w_post, const uint16_t *__restrict__ scalar,
                                                        const uint16_t *__restrict__ w_next, float eps, int hidden,
                                                        int8_t *__restrict__ aq, float *__restrict__ ad, int slices, uint16_t *__restrict__ x16) {
-    __shared__ float red[4];
+    __shared__ float red[NT / 64];
     const int64_t row = (int64_t)blockIdx.x * hidden;
     const int nchunk = hidden >> 3;
     // every global load of the kernel is requested here, before the first reduction (the kernel is a chain of latencies)
@@ -82,7 +95,7 @@ __global__ __launch_bounds__(256) void g4_norm_kernel(uint16_t *__restrict__ h, 
     uint4 hraw[CH], wp[CH], wn[CH];
 #pragma unroll
     for (int c = 0; c < CH; c++) {
-        const int ci = min(threadIdx.x + 256 * c, nchunk - 1);
+        const int ci = min(threadIdx.x + NT * c, nchunk - 1);
         if (o) {
             oa[c] = *reinterpret_cast<const float4 *>(o + row + 8 * ci);
             ob[c] = *reinterpret_cast<const float4 *>(o + row + 8 * ci + 4);
@@ -98,7 +111,7 @@ __global__ __launch_bounds__(256) void g4_norm_kernel(uint16_t *__restrict__ h, 
         for (int s = 1; s < slices; s++) {   // in slice order
 #pragma unroll
             for (int c = 0; c < CH; c++) {
-                const float *at = o + (int64_t)s * gridDim.x * hidden + row + 8 * min((int)threadIdx.x + 256 * c, nchunk - 1);
+                const float *at = o + (int64_t)s * gridDim.x * hidden + row + 8 * min((int)threadIdx.x + NT * c, nchunk - 1);
                 const float4 a4 = *reinterpret_cast<const float4 *>(at), b4 = *reinterpret_cast<const float4 *>(at + 4);
                 oa[c] = make_float4(oa[c].x + a4.x, oa[c].y + a4.y, oa[c].z + a4.z, oa[c].w + a4.w);
                 ob[c] = make_float4(ob[c].x + b4.x, ob[c].y + b4.y, ob[c].z + b4.z, ob[c].w + b4.w);
@@ -110,17 +123,17 @@ __global__ __launch_bounds__(256) void g4_norm_kernel(uint16_t *__restrict__ h, 
         float v1 = 0.f;
 #pragma unroll
         for (int c = 0; c < CH; c++) {
-            if ((int)threadIdx.x + 256 * c < nchunk) {
+            if ((int)threadIdx.x + NT * c < nchunk) {
                 const float t8[8] = {oa[c].x, oa[c].y, oa[c].z, oa[c].w, ob[c].x, ob[c].y, ob[c].z, ob[c].w};
 #pragma unroll
                 for (int j = 0; j < 8; j++) { ov[c][j] = rbf(t8[j]); v1 += ov[c][j] * ov[c][j]; }
             }
         }
-        v1 = vmx_block_sum_256(v1, red);
+        v1 = g4_block_sum<NT>(v1, red);
         const float inv1 = rsqrtf(v1 / (float)hidden + eps);
 #pragma unroll
         for (int c = 0; c < CH; c++) {
-            const int ci = threadIdx.x + 256 * c;
+            const int ci = threadIdx.x + NT * c;
             if (ci < nchunk) {
                 float wv[8], hr[8];
                 unpack8(wp[c], wv);
@@ -141,16 +154,16 @@ __global__ __launch_bounds__(256) void g4_norm_kernel(uint16_t *__restrict__ h, 
     float v2 = 0.f;
 #pragma unroll
     for (int c = 0; c < CH; c++) {
-        if ((int)threadIdx.x + 256 * c < nchunk) {
+        if ((int)threadIdx.x + NT * c < nchunk) {
 #pragma unroll
             for (int j = 0; j < 8; j++) v2 += hv[c][j] * hv[c][j];
         }
     }
-    v2 = vmx_block_sum_256(v2, red);
+    v2 = g4_block_sum<NT>(v2, red);
     const float inv2 = rsqrtf(v2 / (float)hidden + eps);
 #pragma unroll
     for (int c = 0; c < CH; c++) {
-        const int ci = threadIdx.x + 256 * c;
+        const int ci = threadIdx.x + NT * c;
         if (ci < nchunk) {
             float wv[8], out[8];
             unpack8(wn[c], wv);
@@ -686,17 +699,19 @@ int g4_tp_reduce(vmx_gemma4 *m, float *out, int tokens, int hidden, hipStream_t 
 void launch_norm(hipStream_t st, int tokens, uint16_t *h, uint16_t *x, const float *o, const uint16_t *w_post, const uint16_t *scalar,
                  const uint16_t *w_next, float eps, int hidden, int8_t *aq, float *ad, const uint16_t *h_in = nullptr, int slices = 1, uint16_t *x16 = nullptr) {
     if (!h_in) h_in = h;
-#define G4_NORM(CH)                                                                                                                                \
-    do {                                                                                                                                           \
-        if (slices > 1 || x16) hipLaunchKernelGGL((g4_norm_kernel<CH, true>), dim3(tokens), dim3(256), 0, st, h, h_in, x, o, w_post, scalar, w_next, eps, \
-                                           hidden, aq, ad, slices, x16);                                                                           \
-        else hipLaunchKernelGGL((g4_norm_kernel<CH, false>), dim3(tokens), dim3(256), 0, st, h, h_in, x, o, w_post, scalar, w_next, eps, hidden,   \
-                                aq, ad, 1, nullptr);                                                                                                   \
-    } while (0)
-    if (hidden <= 2048) G4_NORM(1);
-    else if (hidden <= 4096) G4_NORM(2);
-    else if (hidden <= 8192) G4_NORM(4);
-    else G4_NORM(8);
+#define G4_NORM(CH, PROMPT, NT, ...) hipLaunchKernelGGL((g4_norm_kernel<CH, PROMPT, NT>), dim3(tokens), dim3(NT), 0, st, h, h_in, x, o, w_post, scalar, w_next, eps, \
+                                                        hidden, aq, ad, __VA_ARGS__)
+    if (slices > 1 || x16) {
+        if (hidden <= 2048) G4_NORM(1, true, 256, slices, x16);
+        else if (hidden <= 4096) G4_NORM(1, true, 512, slices, x16);
+        else if (hidden <= 8192) G4_NORM(2, true, 512, slices, x16);
+        else G4_NORM(4, true, 512, slices, x16);
+    } else {
+        if (hidden <= 2048) G4_NORM(1, false, 256, 1, nullptr);
+        else if (hidden <= 4096) G4_NORM(2, false, 256, 1, nullptr);
+        else if (hidden <= 8192) G4_NORM(4, false, 256, 1, nullptr);
+        else G4_NORM(8, false, 256, 1, nullptr);
+    }
 #undef G4_NORM
 }
 }  // namespace
