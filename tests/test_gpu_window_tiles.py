@@ -78,3 +78,36 @@ def test_prompt_tiles(gpu, block, heads, groups, dim, vdim, window, keep, chunk,
             bound = (2 * d + 2.0 ** -15 + 512 * 2.0 ** -24) * float(v.abs().max())
             got = out[int(starts[b]):int(starts[b + 1]), h].double()
             assert float((got - exact).abs().max()) <= bound, (b, h)
+
+
+@pytest.mark.parametrize("talk", [False, True])
+@pytest.mark.parametrize("block", [16, 7])
+def test_rows_without_keys(gpu, block, talk):
+    """A row at position -1 sees no key: its block table, which holds no block, is not followed, and the other rows are what they are without it."""
+    vmx, torch = gpu
+    import ctypes as C
+    from vllm_rust_amd._lib import WindowAttnExtras, check, lib
+    heads, dim, T = 4, 64, 70
+    g = torch.Generator(device="cuda").manual_seed(block)
+    mb = (T + block - 1) // block
+    bt = torch.zeros((2, mb), dtype=torch.int32, device="cuda")
+    bt[0] = torch.randperm(mb, device="cuda", generator=g).to(torch.int32)
+    bt[1] = -1
+    kc, vc = (torch.randn((mb * block, 1, dim), device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn((T + 1, heads, dim), device="cuda", generator=g)
+    mix = torch.randn((heads, heads), device="cuda", generator=g).to(torch.bfloat16)
+    ex = WindowAttnExtras()
+    if talk:
+        ex.talk_bf16 = mix.data_ptr()
+    sid = torch.tensor([0] * T + [1], dtype=torch.int32, device="cuda")
+    pos = torch.tensor(list(range(T)) + [-1], dtype=torch.int32, device="cuda")
+    starts = torch.tensor([0, T, T + 1], dtype=torch.int32, device="cuda")
+
+    def run(rows, seqs):
+        out = torch.empty((T + 1, heads, dim), device="cuda")
+        check(lib.vmx_window_attention_ex(out.data_ptr(), 0, q.data_ptr(), heads * dim, kc.data_ptr(), vc.data_ptr(), 1, bt.data_ptr(), mb, sid.data_ptr(),
+                                          pos.data_ptr(), None, None, 0, 0.1, 0.0, 0, 0, rows, heads, 1, dim, dim, block, starts.data_ptr(), seqs, None, 0,
+                                          C.byref(ex), None))
+        torch.cuda.synchronize()
+        return out[:T]
+    assert torch.equal(run(T + 1, 2), run(T, 1))

@@ -548,10 +548,12 @@ __global__ __launch_bounds__(256, DS <= 4 ? 3 : 2) void window_attn_mfma_kernel(
     vmx_f32x4 o[VS];
 #pragma unroll
     for (int v = 0; v < VS; v++) o[v] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
-    lookup(kb0);
-    fetch();
-    lookup(kb0 + KT);
-    stash();
+    if (kb0 < kb1) {   // no keys (a row at position -1): no table entry is read
+        lookup(kb0);
+        fetch();
+        lookup(kb0 + KT);
+        stash();
+    }
     __syncthreads();
     for (int kb = kb0; kb < kb1; kb += KT) {
         if (kb + KT < kb1) {
@@ -817,10 +819,12 @@ __global__ __launch_bounds__(TM_NT) void talk_attn_mfma_kernel(const WinAttn p) 
 #pragma unroll
         for (int v = 0; v < VS; v++) o[a][v] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    lookup(kb0);
-    fetch(kb0);
-    lookup(kb0 + KT);
-    stash();
+    if (kb0 < kb1) {   // no keys (a row at position -1): no table entry is read
+        lookup(kb0);
+        fetch(kb0);
+        lookup(kb0 + KT);
+        stash();
+    }
     __syncthreads();
     for (int kb = kb0; kb < kb1; kb += KT) {
         if (kb + KT < kb1) {
