@@ -237,7 +237,7 @@ extern "C" int vmx_larolorn_create(const vmx_larolorn_config *cfg, const vmx_lar
     GA(m->hsel, T * W * m->esz());
     GA(m->y, T * W * 4);
     GA(m->side, T * W * 4);
-    GA(m->fused, T * std::max(nf, (size_t)c.vocab) * 4);   // also gate | up of the feed-forward and the logits of a greedy-only step
+    GA(m->fused, T * std::max(nf, (size_t)c.vocab) * 4);   // also gate | up of a feed-forward in two launches and the logits of a greedy-only step
     GA(m->q, T * nq * 4);
     GA(m->qabs, T * hr * 4);
     GA(m->olat, T * hr * 4);
@@ -410,7 +410,7 @@ int clamped_glu(vmx_larolorn *m, const Layer &w, const Step &s) {
     const int W = m->cfg.width, F = w.c.ff, f32 = m->f32() ? 1 : 0;
     VmxLinear gu = product(m->input(), f32, W, w.wgu, 2 * F, m->act.p, f32, s.T, f32);
     gu.ldc = F;
-    if (vmx_linear_glu_ok(gu)) {   // the activation behind the sums: no f32 rows of gate and up in memory
+    if (vmx_linear_glu_ok(gu) && vmx_linear_glu_pays(gu)) {   // the activation behind the sums: no f32 rows of gate and up in memory
         if (int rc = vmx_linear_glu(gu, GLU_SLOPE, w.c.limit, s.st)) return rc;
     } else {
         if (int rc = vmx_linear_launch(product(m->input(), f32, W, w.wgu, 2 * F, m->fused.p, 1, s.T, f32), s.st)) return rc;

@@ -615,12 +615,17 @@ int64_t tile_ns(const VmxLinear &p, int full, int few) {
 // 1500 x 2048 x 6144 74 / 61 / 81 / 53 / 65 / 73.  The call before (128 x 128 two a unit, or 64 x 64 in two or three stages, requests at the head of a
 // stage, results element by element) and now:  1500 x 12288 x 2048 107 -> 85, 1500 x 3664 x 2048 36 -> 28, 1500 x 2048 x 6144 72 -> 53, 500 x 12288 x
 // 2048 42 -> 33, 333 x 2048 x 6144 35 -> 25, 100 x 3664 x 2048 14.6 -> 11.2.  Expert blocks bring 64 rows each.
+int64_t ns64(const VmxLinear &p) { return tile_ns<Tile64>(p, 490, 280); }
+int64_t ns64w(const VmxLinear &p) { return tile_ns<Tile64w>(p, 700, 450); }
+int64_t ns128two(const VmxLinear &p) { return tile_ns<Tile128two>(p, 1130, 800); }
+int64_t ns128(const VmxLinear &p) { return tile_ns<Tile128>(p, 640, 0); }
+int64_t ns192(const VmxLinear &p) { return tile_ns<Tile192>(p, 850, 0); }
+int64_t ns256(const VmxLinear &p) { return tile_ns<Tile256>(p, 1000, 0); }
 int launch_tile(const VmxLinear &p, hipStream_t st) {
     if (p.a_f32) return launch_tile_shape<Tile64f>(p, st);
-    const int64_t t64 = tile_ns<Tile64>(p, 490, 280), t64w = tile_ns<Tile64w>(p, 700, 450);
+    const int64_t t64 = ns64(p), t64w = ns64w(p);
     if (p.block_expert) return t64 <= t64w ? launch_tile_shape<Tile64>(p, st) : launch_tile_shape<Tile64w>(p, st);
-    const int64_t two = tile_ns<Tile128two>(p, 1130, 800), t128 = tile_ns<Tile128>(p, 640, 0), t192 = tile_ns<Tile192>(p, 850, 0),
-                  t256 = tile_ns<Tile256>(p, 1000, 0), least = std::min({t64, t64w, two, t128, t192, t256});
+    const int64_t two = ns128two(p), t128 = ns128(p), t192 = ns192(p), t256 = ns256(p), least = std::min({t64, t64w, two, t128, t192, t256});
     if (least == t64) return launch_tile_shape<Tile64>(p, st);
     if (least == t64w) return launch_tile_shape<Tile64w>(p, st);
     if (least == t128) return launch_tile_shape<Tile128>(p, st);
@@ -629,8 +634,7 @@ int launch_tile(const VmxLinear &p, hipStream_t st) {
 }
 // ... of those whose waves own pairs of 32 columns
 int launch_tile_glu(const GluLinear &p, hipStream_t st) {
-    const int64_t t64w = tile_ns<Tile64w>(p, 700, 450), two = tile_ns<Tile128two>(p, 1130, 800), t192 = tile_ns<Tile192>(p, 850, 0), t256 = tile_ns<Tile256>(p, 1000, 0),
-                  least = std::min({t64w, two, t192, t256});
+    const int64_t t64w = ns64w(p), two = ns128two(p), t192 = ns192(p), t256 = ns256(p), least = std::min({t64w, two, t192, t256});
     if (least == t64w) return launch_tile_as<Tile64w, TILE_GLU>(p, st);
     if (least == t192) return launch_tile_as<Tile192, TILE_GLU>(p, st);
     return least == t256 ? launch_tile_as<Tile256, TILE_GLU>(p, st) : launch_tile_as<Tile128two, TILE_GLU>(p, st);
@@ -651,6 +655,23 @@ bool vmx_linear_glu_ok(const VmxLinear &p) {
                        p.out_scale == 1.0f;
     if (!plain || p.M < 1 || p.N % 16 || !direct_ok(p)) return false;
     return p.M <= 16 || (!p.a_f32 && tile_ok(p, true));
+}
+
+// Whether that is faster than a plain product into f32 rows and a kernel of its own for the activation.  Up to 16 rows it is.  Tiles: pairs of columns leave out the
+// shapes of 64 x 64 and of 128 x 128 with one workgroup a unit, and where those are the plain product's, two launches can be done first.  Both sides by
+// the shapes' estimates and what these leave out: shapes with two workgroups a unit wait for weights out of memory (the bytes at 8 TB/s); the activation's launch, and its
+// rows at 4.5 TB/s.  us, two launches / this, weights out of memory:  12288 x 2048, 17 rows 15.8 / 20.2, 64 17.1 / 20.8, 65 21.1 / 19.8, 128 23.1 / 20.6, 129 22.6 / 26.9,
+// 256 28.1 / 30.3, 257 33.0 / 28.1, 1500 102 / 87;  16384 x 3072, 64 24.8 / 31.8, 65 30.7 / 28.9, 192 38.1 / 47.0, 257 46.3 / 41.5;  24576 x 4096, 64 50.7 / 47.5, 128 58.8 /
+// 62.6, 129 60.0 / 56.5;  6144 x 1024, 128 10.8 / 11.8, 129 13.1 / 11.4;  2816 x 2048, 300 14.8 / 18.5, 400 20.3 / 18.2.  Of six widths at 27 counts of 17 .. 2000 rows all but
+// one (2816 x 2048, 333 rows: 16.1 / 18.3) take the faster side or are within 3 % of it.
+int vmx_linear_glu_pays(const VmxLinear &p) {
+    if (p.M <= 16) return 1;
+    VmxLinear rows = p;   // of gate and up
+    rows.c_f32 = 1;
+    const int64_t fetch = (int64_t)p.N * p.K * 2 / 8000, activation = 800 + (int64_t)p.M * p.N / 2 * 10 / 4500;
+    auto least = [&](int64_t two_a_unit, int64_t one_a_unit) { return two_a_unit <= one_a_unit ? two_a_unit + fetch : one_a_unit; };
+    const int64_t apart = least(std::min({ns64(rows), ns64w(rows), ns128two(rows)}), std::min({ns128(rows), ns192(rows), ns256(rows)}));
+    return least(std::min(ns64w(p), ns128two(p)), std::min(ns192(p), ns256(p))) <= apart + activation;
 }
 
 int vmx_linear_glu(const VmxLinear &p, float slope, float limit, hipStream_t st) {

@@ -248,8 +248,9 @@ struct VmxLinear {
 };
 extern "C" int vmx_linear_launch(const VmxLinear &p, hipStream_t st);
 // The product with a clamped gated activation behind its sums: W's rows are N / 2 gate rows and as many up rows, C is [M, N / 2] = g sigmoid(slope g) (u + 1) with
-// g = min(gate, limit) and u = the up product clamped to +- limit; for products that vmx_linear_glu_ok takes
+// g = min(gate, limit) and u = the up product clamped to +- limit; for products that vmx_linear_glu_ok takes, worth it where vmx_linear_glu_pays (host arithmetic)
 bool vmx_linear_glu_ok(const VmxLinear &p);
+extern "C" int vmx_linear_glu_pays(const VmxLinear &p);
 extern "C" int vmx_linear_glu(const VmxLinear &p, float slope, float limit, hipStream_t st);
 
 // latent_attn.hip: out[h][r][d] = in[h][d][r], the key up-projection turned for q_abs = U_h^T q_h
