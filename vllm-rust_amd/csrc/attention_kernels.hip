@@ -1101,7 +1101,7 @@ static int parts_for_impl(int max_seq_len) {
 // Causal (optionally windowed) attention of q_len new tokens at positions offset .. offset + q_len - 1 over everything the
 // paged cache holds for the sequence up to and including themselves (the caller wrote the new K/V rows first, as the
 // reference's naive backend does: write, read back, softmax(QK^T * scale + mask) V; layers/attention/naive.rs:38-83).
-// Flash-style on the matrix cores.  A workgroup = 4 waves = up to 4 query heads of one KV head x 16-token query tiles;
+// Flash-style on the matrix cores.  A workgroup takes up to 4 query heads of one KV head x 16-token query tiles, a wave each (several groups of such waves: below);
 // KV tiles of 16 tokens are staged through LDS once per workgroup (K row-major, V transposed; the next tile's rows are under way while a
 // tile is multiplied: 256 tokens of Gemma-4-12B, a chain of up to 16 tiles in 64 workgroups that its latency bounds, 48.7 -> 28.6 us
 // with 256-wide and 74 -> 46 us with 512-wide heads), then per wave
@@ -1316,28 +1316,37 @@ int launch_prefill_as(hipStream_t st, uint16_t *out, const uint16_t *q, const vo
     return VMX_OK;
 }
 
-// Wide heads, from five key tiles on: several groups share the keys of a workgroup.  256 wide, four groups where the workgroups then still have a compute unit each
-// (the groups' tiles fill its LDS), two up to the workgroups that the units hold, else one.  512 wide, two at any length: a workgroup of one group has a unit's
-// registers to itself as well.  us, one group / this, FP8 cache, no history, tokens 17 / 100 / 256 / 512 / 1024 / 2048 / 4096: 16 heads over 8, 256 wide, window 1024
-// 7.4 14.0 28.2 52.4 101 129 247 / 7.4 12.6 17.6 27.5 60 123 249; 16 heads over one, 512 wide 11.5 22.7 44.3 81 159 537 1660 / 11.4 20.7 33.4 54 99 325 974.
 template <int HD, int QPK, int FP8, class... A>
 int launch_prefill(hipStream_t st, uint16_t *out, const uint16_t *q, const void *kc, const void *vc, const int32_t *bt, int q_len, int offset,
                    float scale, int H, int KVH, int bs, int window, A... rest) {
     constexpr int HPW = QPK < 4 ? QPK : 4, TT = 4 / HPW;
-    const int64_t keys = window > 0 ? std::min<int64_t>((int64_t)offset + q_len, (int64_t)window + 16 * TT) : (int64_t)offset + q_len;
     if constexpr (HD >= 256) {
-        const int64_t tiles = ((int64_t)q_len + 15) / 16, columns = (int64_t)KVH * (QPK / HPW), cus = vmx_num_cus();
-        if constexpr (HD == 256 && HPW < 4) {
-            constexpr int FEW = 2 / HPW;   // 128 threads a group, four groups
-            if (keys > 64 && (tiles + FEW - 1) / FEW * columns <= cus)
-                return launch_prefill_as<HD, QPK, FP8, FEW, 4>(st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window, rest...);
-        }
-        if (keys > 64 && (HD == 512 || (tiles + TT - 1) / TT * columns <= 2 * cus))
-            return launch_prefill_as<HD, QPK, FP8, TT, 2>(st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window, rest...);
+        const int groups = vmx_prefill_attention_groups(HD, QPK, KVH, FP8, q_len, offset, window);
+        if constexpr (HD == 256 && HPW < 4)
+            if (groups == 4) return launch_prefill_as<HD, QPK, FP8, 2 / HPW, 4>(st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window, rest...);   // 128 threads a group
+        if (groups == 2) return launch_prefill_as<HD, QPK, FP8, TT, 2>(st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window, rest...);
     }
     return launch_prefill_as<HD, QPK, FP8, TT, 1>(st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH, bs, window, rest...);
 }
 }  // namespace
+
+// Groups that share the keys of a workgroup of 256- and 512-wide heads (host arithmetic); qpk: the compiled head ratio, cache 1: FP8.  256 wide, four groups where
+// the workgroups then still have a compute unit each (the groups' tiles fill its LDS), two up to the workgroups that the units hold, else one.  512 wide, two at any
+// length: a workgroup of one group has a unit's registers to itself as well.  us, one group / this, FP8 cache, no history, tokens 17 / 256 / 512 / 1024 / 2048 / 4096:
+// 16 heads over 8, 256 wide, window 1024 7.4 28.2 52.4 101 129 247 / 7.4 17.6 27.5 60 123 249; 16 heads over one, 512 wide 11.5 44.3 81 159 537 1660 / 11.4 33.4 54 99
+// 325 974.  A few tiles take as long as the merge: time of one group over that of several, at 65 / 80 / 81 / 97 / 113 / 129 keys, bf16 and FP8 cache: 16 heads over 8, 256
+// wide 0.93 0.88 1.01 1.02 1.21 1.17 and 1.00 0.94 1.08 1.09 1.28 1.25; 32 over 8 (two groups of four heads) 1.06 1.04 1.06 1.16 1.18 1.21 and 1.10 1.09 1.16
+// 1.23 1.24 1.26; 16 over one, 512 wide 0.93 0.93 0.95 0.99 1.01 1.03 and 0.98 0.98 1.02 1.07 1.10 1.16.
+int vmx_prefill_attention_groups(int head_dim, int qpk, int kv_heads, int cache, int q_len, int offset, int window) {
+    if (head_dim < 256) return 1;
+    const int hpw = qpk < 4 ? qpk : 4, tt = 4 / hpw;
+    const int64_t keys = window > 0 ? std::min<int64_t>((int64_t)offset + q_len, (int64_t)window + 16 * tt) : (int64_t)offset + q_len;
+    if (keys <= (head_dim == 512 ? (cache == 1 ? 80 : 112) : hpw < 4 ? 80 : 64)) return 1;
+    if (head_dim == 512) return 2;
+    const int64_t tiles = ((int64_t)q_len + 15) / 16, columns = (int64_t)kv_heads * (qpk / hpw), cus = vmx_num_cus();
+    if (hpw < 4 && (tiles + 2 / hpw - 1) / (2 / hpw) * columns <= cus) return 4;
+    return (tiles + tt - 1) / tt * columns <= 2 * cus ? 2 : 1;
+}
 
 static int prefill_attention_impl(uint16_t *out, const uint16_t *q, const void *k_cache, const void *v_cache,
                                   const int32_t *block_table, int q_len, int seqlen_offset, float scale, int num_heads,

@@ -191,6 +191,7 @@ size_t vmx_iq_gemm_int_weight_bytes(int N, int K);
 int vmx_iq_dequant_int(int ggml_type, const void *blocks, void *workspace, int row0, int rows, int N, int K, hipStream_t st);
 int vmx_bf16_rows_to_f16(const uint16_t *A, uint16_t *a16, int64_t n, hipStream_t st);
 bool vmx_prefill_attention_gives_f16(int head_dim);
+int vmx_prefill_attention_groups(int head_dim, int qpk, int kv_heads, int cache, int q_len, int offset, int window);
 int vmx_prefill_attention_rows(uint16_t *out, const uint16_t *q, const void *k_cache, const void *v_cache, const int32_t *block_table, int q_len, int seqlen_offset,
                                float scale, int num_heads, int num_kv_heads, int head_dim, int block_size, int window, int kv_dtype, const float *k_scale,
                                const float *v_scale, bool out_f16, hipStream_t st);
