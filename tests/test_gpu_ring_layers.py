@@ -18,7 +18,7 @@ def models(request):
     moe = request.param
     # q|k|v 2048 -> 6144 in two slices, o 4096 deep (four passes), gate|up 2048 -> 12288, down 6144 deep (six): the smallest widths the form takes
     spec = Qwen3Spec(hidden_size=2048, num_layers=2, num_heads=32, num_kv_heads=8, head_dim=128, intermediate_size=512 if moe else 6144, vocab_size=500,
-                     max_position=128, num_blocks=32, max_batch=16, max_seq_len=64, qk_norm=not moe, num_experts=4 if moe else 0, experts_per_tok=4 if moe else 0)   # all experts: no row can land on another choice
+                     max_position=128, num_blocks=32, max_batch=16, max_seq_len=64, max_prefill_tokens=16, qk_norm=not moe, num_experts=4 if moe else 0, experts_per_tok=4 if moe else 0)   # all experts: no row can land on another choice
     model = QuantizedQwen3ForCausalLM(spec)
     ck = (model.load_synthetic_moe if moe else model.load_synthetic)(seed=5, keep_host_copy=True)
     yield torch, spec, model, lambda: OracleQwen3(spec, ck, rope_cos_sin_cache(spec.head_dim, spec.max_position, spec.rope_theta))
@@ -46,6 +46,26 @@ def test_layers_match_oracle(models, rows):
             rel = np.sqrt(err.sum() / norm.sum() if spec.num_experts else (err / norm).max())
             assert rel <= 3e-2, (p, rel)
         ids = out.cpu().numpy().astype(np.int32)
+
+
+@pytest.mark.parametrize("rows", [5, 16])
+def test_short_prompts_match_oracle(models, rows):
+    """Prompts of as many rows take the same layers: a first part and one with history, every row of the residual stream and the last row's logits."""
+    from oracle import oracle as orc
+    torch, spec, model, oracle = models
+    ref = oracle()
+    bt = np.random.default_rng(rows).permutation(spec.num_blocks)[:2 * rows // spec.block_size + 1].astype(np.int32)
+    for part in range(2):
+        ids = np.random.default_rng(10 * rows + part).integers(0, spec.vocab_size, rows).astype(np.int32)
+        pos = np.arange(part * rows, (part + 1) * rows, dtype=np.int32)
+        last = torch.empty(spec.vocab_size, dtype=torch.bfloat16, device="cuda")
+        model.prefill(torch.from_numpy(ids).cuda(), part * rows, torch.from_numpy(bt).cuda(), logits_last=last)
+        got_h = model.debug_read(0, (rows, spec.hidden_size)).double().cpu().numpy()
+        slots = (bt[pos // spec.block_size] * spec.block_size + pos % spec.block_size).astype(np.int32)
+        exp, exp_h, _ = ref.decode(ids, pos, slots, np.repeat(bt[None], rows, axis=0), pos + 1)
+        for g, e in ((last.double().cpu().numpy()[None], orc.bf16_to_f32(exp[-1:])), (got_h, orc.bf16_to_f32(exp_h))):   # the decoder tests' bar
+            err, norm = ((g - e) ** 2).sum(1), (e.astype(np.float64) ** 2).sum(1)
+            assert np.sqrt(err.sum() / norm.sum() if spec.num_experts else (err / norm).max()) <= 3e-2, part
 
 
 _SMALL = dict(hidden_size=256, num_heads=4, num_kv_heads=2, head_dim=64, intermediate_size=512)

@@ -80,10 +80,12 @@ def test_prompt_tiles(gpu, block, heads, groups, dim, vdim, window, keep, chunk,
             assert float((got - exact).abs().max()) <= bound, (b, h)
 
 
-@pytest.mark.parametrize("talk", [False, True])
+@pytest.mark.parametrize("talk,sink", [(False, False), (False, True), (True, False)])
+@pytest.mark.parametrize("shares", [False, True])
 @pytest.mark.parametrize("block", [16, 7])
-def test_rows_without_keys(gpu, block, talk):
-    """A row at position -1 sees no key: its block table, which holds no block, is not followed, and the other rows are what they are without it."""
+def test_rows_without_keys(gpu, block, shares, talk, sink):
+    """A row at position -1 sees no key: it is what a softmax over nothing gives (zeros with a sink, else not a number), with and without shares of keys and their merge, and
+    the other rows are what they are without it.  (Whether its block table is read shows in no result: all it could bring is hidden.)"""
     vmx, torch = gpu
     import ctypes as C
     from vllm_rust_amd._lib import WindowAttnExtras, check, lib
@@ -95,19 +97,26 @@ def test_rows_without_keys(gpu, block, talk):
     bt[1] = -1
     kc, vc = (torch.randn((mb * block, 1, dim), device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
     q = torch.randn((T + 1, heads, dim), device="cuda", generator=g)
-    mix = torch.randn((heads, heads), device="cuda", generator=g).to(torch.bfloat16)
+    mix, sinks = torch.randn((heads, heads), device="cuda", generator=g).to(torch.bfloat16), torch.randn(heads, device="cuda", generator=g).to(torch.bfloat16)
     ex = WindowAttnExtras()
     if talk:
         ex.talk_bf16 = mix.data_ptr()
+    if sink:
+        ex.sink_bf16 = sinks.data_ptr()
     sid = torch.tensor([0] * T + [1], dtype=torch.int32, device="cuda")
     pos = torch.tensor(list(range(T)) + [-1], dtype=torch.int32, device="cuda")
     starts = torch.tensor([0, T, T + 1], dtype=torch.int32, device="cuda")
+    size = lib.vmx_window_attention_workspace_bytes(T + 1, heads, dim) if shares else 0
+    ws = torch.full((size // 4,), float("nan"), device="cuda")
 
     def run(rows, seqs):
-        out = torch.empty((T + 1, heads, dim), device="cuda")
+        out = torch.full((T + 2, heads, dim), 3.0, device="cuda")
         check(lib.vmx_window_attention_ex(out.data_ptr(), 0, q.data_ptr(), heads * dim, kc.data_ptr(), vc.data_ptr(), 1, bt.data_ptr(), mb, sid.data_ptr(),
-                                          pos.data_ptr(), None, None, 0, 0.1, 0.0, 0, 0, rows, heads, 1, dim, dim, block, starts.data_ptr(), seqs, None, 0,
-                                          C.byref(ex), None))
+                                          pos.data_ptr(), None, None, 0, 0.1, 0.0, 0, 0, rows, heads, 1, dim, dim, block, starts.data_ptr(), seqs,
+                                          ws.data_ptr() if shares else None, size, C.byref(ex), None))
         torch.cuda.synchronize()
-        return out[:T]
-    assert torch.equal(run(T + 1, 2), run(T, 1))
+        assert bool((out[rows:] == 3.0).all())
+        return out
+    both, alone = run(T + 1, 2), run(T, 1)
+    assert torch.equal(both[:T], alone[:T]) and bool(both[:T].isfinite().all())
+    assert bool((both[T] == 0).all()) if sink else bool(both[T].isnan().all())
