@@ -1355,9 +1355,9 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
         // -> 6.0, down 11.6 + 4.9 -> 12.4, q|k|v and gate|up 0.3 .. 0.6 more); 8 rows of Mixtral, 4 layers, whose router joins the norm as well: 846 -> 804
         const bool rfold = folded_layers_enabled() && !tp && !moe && !one && L.int4_ready() && L.gate_up.glu && !pending &&
                            vmx_int4_ring_norm_splits(B, NQKV_, H, 0) > 0 && vmx_int4_ring_norm_splits(B, 2 * I, H, 1) == 1 &&
-                           vmx_int4_ring_resid_ok(B, H, NQ) && vmx_int4_ring_resid_ok(B, H, I);
+                           vmx_int4_ring_resid_pays(B, H, NQ) && vmx_int4_ring_resid_pays(B, H, I);
         const bool mrfold = moe && folded_layers_enabled() && !tp && !pending && L.int4_attn_ready() && H % 256 == 0 &&
-                            vmx_int4_ring_norm_splits(B, NQKV_, H, 0) > 0 && vmx_int4_ring_resid_ok(B, H, NQ);
+                            vmx_int4_ring_norm_splits(B, NQKV_, H, 0) > 0 && vmx_int4_ring_resid_pays(B, H, NQ);
         const bool ring_in = (rfold || mrfold) && hg_in_x;
         // the first layer's h comes from the embedding: no tile sums yet
         const bool fold_in = ((fold || mfold) && ssq_tiles == H / 16) || (dfold && ssq_tiles > 0 && ssq_tiles % 4 == 0);
@@ -1836,7 +1836,7 @@ extern "C" int vmx_qwen3_linears_only(vmx_qwen3 *m, int batch, void *stream) {
             continue;
         }
         if (folded_layers_enabled() && !m->comm && c.tp_size <= 1 && c.num_experts == 0 && L.gate_up.glu && vmx_int4_ring_norm_splits(batch, NQKV_, H, 0) > 0 &&
-            vmx_int4_ring_norm_splits(batch, 2 * I, H, 1) == 1 && vmx_int4_ring_resid_ok(batch, H, NQ) && vmx_int4_ring_resid_ok(batch, H, I)) {
+            vmx_int4_ring_norm_splits(batch, 2 * I, H, 1) == 1 && vmx_int4_ring_resid_pays(batch, H, NQ) && vmx_int4_ring_resid_pays(batch, H, I)) {
             float *ssq = (float *)m->ssq.p;
             uint16_t *hg = (uint16_t *)m->x.p;
             if (mk & 1)

@@ -2017,9 +2017,18 @@ int vmx_int4_gemm_y(const void *packed, const uint16_t *x, uint16_t *y, int M, i
 
 // ---- 5 .. 16 rows: the residual add and the next norm's gains in the epilogue, the norm's row factor behind the consumer's sums
 // (int4_gemm_ring_resid_kernel, int4_gemm_ring_norm_kernel)
+// Depths: the passes are unrolled, and the kernel is built for these counts.
 bool vmx_int4_ring_resid_ok(int M, int N, int K) {
     const int passes = K % (8 * KB) == 0 ? K / (8 * KB) : 0;
     return M >= 5 && M <= 16 && N % NT == 0 && (passes == 2 || passes == 4 || passes == 6 || passes == 8 || passes == 12);
+}
+// Whether a layer gains by it.  A compute unit holds one workgroup, which walks all of K: one round of workgroups pays, of sums deeper than eight passes if it is more than
+// half of one, two rounds only of short sums.  Steps, 5 / 8 / 16 rows, time without over time with it (o_proj N x K, then down):  dense 4096 x 4096, x 12288
+// 1.083 1.082 1.075;  x 8192 1.070 1.071 1.072;  2048 x 4096, x 6144 1.021 1.021 1.025;  x 12288 0.995 0.995 0.994;  experts' layers 4096 x 4096 1.095 1.089 1.091;
+// 2048 x 4096 1.098 1.081 1.066;  two rounds: 6144 x 2048 1.013 1.019 1.016, x 4096 1.017 0.988 0.991;  8192 x 4096 1.003 1.015 1.016, x 8192 0.991 0.994 0.985.
+bool vmx_int4_ring_resid_pays(int M, int N, int K) {
+    const int tiles = N / NT, cus = vmx_num_cus();
+    return vmx_int4_ring_resid_ok(M, N, K) && (tiles <= cus ? K <= 8 * 8 * KB || 2 * tiles > cus : tiles <= 2 * cus && 2 * K <= N);
 }
 // slices the consumer leaves (1 with glu), 0: not covered
 int vmx_int4_ring_norm_splits(int M, int N, int K, int glu) {

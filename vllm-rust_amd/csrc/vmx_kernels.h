@@ -41,6 +41,7 @@ int vmx_int4_gemm_y(const void *packed, const uint16_t *x, uint16_t *y, int M, i
 // 5 .. 16 rows (ring form): h = bf16(h + bf16(x W)) with the sums of squares of its 16-column tiles and hg = bf16(h gain); the linear of rms_norm(h) from
 // those (hg carries the gains, the row factor comes from ssq and multiplies the sums)
 bool vmx_int4_ring_resid_ok(int M, int N, int K);
+bool vmx_int4_ring_resid_pays(int M, int N, int K);
 int vmx_int4_ring_norm_splits(int M, int N, int K, int glu);
 int vmx_int4_ring_resid(const void *packed, const uint16_t *x, uint16_t *h, uint16_t *hg, const uint16_t *gain, float *ssq, int M, int N, int K, int group,
                         hipStream_t st);
