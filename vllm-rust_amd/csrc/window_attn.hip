@@ -446,8 +446,11 @@ __global__ __launch_bounds__(512) void window_attn_talk_kernel(const WinAttn p) 
 // Latency bounds it, the trips to the block table most: a branch around each of a thread's eight lookups a tile made eight trips of them, one after
 // another.  Without branches they are one trip, a thread's value chunks share theirs, and a tile that every row sees whole is not masked: 16 heads
 // over 4 of 128, a prompt of 1500 rows 66 -> 45 us, 16 rows at 1000 keys 28 -> 22.
+// Registers: heads up to 128 leave room for a third workgroup a compute unit (two / three: 16 rows at 1000 keys 23.6 / 21.5 us, 64 wide 17.3 / 15.4; a prompt of 2000 rows 118.5 /
+// 114.3, 64 wide 83.8 / 77.9; one row of 60 keys 11.2 / 11.8); wider ones keep what they want (bound to two / not: 32 rows at 3000 keys, 192 wide 163 / 156 us, 256 wide 177 / 168;
+// a prompt of 500 rows, 160 wide 22.8 / 20.8).
 template <int DS, int VS>
-__global__ __launch_bounds__(256, DS <= 4 ? 3 : 2) void window_attn_mfma_kernel(const WinAttn p) {
+__global__ __launch_bounds__(256, DS <= 4 ? 3 : 1) void window_attn_mfma_kernel(const WinAttn p) {
     constexpr int KT = 64, LDK = 32 * DS + 8, LDV = KT + 8, KCH = DS, VCH = (VS + 1) / 2;
     __shared__ __align__(16) uint16_t Ks[KT * LDK];
     __shared__ __align__(16) uint16_t Vt[16 * VS * LDV];
@@ -1206,11 +1209,11 @@ extern "C" int vmx_window_attention_ex(void *out, int out_dtype, const float *q,
         const int base = runs * kv_heads * ((qpk + 3) / 4);
         // few workgroups: deal each run's key tiles to several, up to the workgroups that a compute unit holds (three; two of heads wider than 128).
         // Decode of a model with 16 heads over 4, rows x tokens, attention and merge, up to one -> up to two workgroups a compute unit: 16 x 1000
-        // 40.0 -> 29.8 us, 16 x 300 19.5 -> 16.8, 12 x 700 24.0 -> 19.4, 8 x 1500 25.0 -> 23.6, 16 x 100 14.7 -> 14.6; up to three: a step of 16 x 1000
-        // 476.7 -> 474.7.  Tables say how long a sequence can be, not how long it is: shares beyond its tiles leave at once and are launched last
+        // 40.0 -> 29.8 us, 16 x 300 19.5 -> 16.8, 12 x 700 24.0 -> 19.4, 8 x 1500 25.0 -> 23.6, 16 x 100 14.7 -> 14.6; up to three: above, at the
+        // kernel.  Tables say how long a sequence can be, not how long it is: shares beyond its tiles leave at once and are launched last
         // (16 x 100 in tables of 4096: 14.7; as whole shares among the others 15.9)
         if (workspace && base < 128) {
-            const int held = dim <= 128 ? 768 : 512;
+            const int held = (dim <= 128 ? 3 : 2) * vmx_num_cus();
             int parts = held / base < 16 ? held / base : 16;
             if (span > 0) parts = std::min(parts, (span + keep_first + rt + 63) / 64);
             parts = (int)std::min<int64_t>(parts, ((int64_t)max_blocks_per_seq * block_size + 63) / 64);   // no sequence is longer than its table
