@@ -1352,7 +1352,7 @@ int run_layers(vmx_qwen3 *m, const int32_t *input_ids, const int32_t *positions,
                            vmx_dense_decode_ok(B, H, NQ) && vmx_dense_decode_ok(B, 2 * I, H) && vmx_dense_decode_ok(B, H, I);
         // 5 .. 16 rows, int4: the residual adds and the norms' gains move into the epilogues of o_proj and down (or of the expert combine), the norms' row
         // factors behind the sums of the consumers: two launches a layer less.  16 rows of Qwen3-8B AWQ, 1500 tokens, 9 layers: 749 -> 696 us (o 4.9 + 4.9
-        // -> 6.0, down 11.6 + 4.9 -> 12.4, q|k|v and gate|up 0.3 .. 0.6 more); 8 rows of Mixtral, 4 layers, whose router joins the norm as well: 846 -> 804
+        // -> 6.0, down 11.6 + 4.9 -> 12.4, q|k|v and gate|up 0.3 .. 0.6 more); experts' layers of that width, whose router joins the norm as well, 8 rows, 3 layers 307 -> 282
         const bool rfold = folded_layers_enabled() && !tp && !moe && !one && L.int4_ready() && L.gate_up.glu && !pending &&
                            vmx_int4_ring_norm_splits(B, NQKV_, H, 0) > 0 && vmx_int4_ring_norm_splits(B, 2 * I, H, 1) == 1 &&
                            vmx_int4_ring_resid_pays(B, H, NQ) && vmx_int4_ring_resid_pays(B, H, I);

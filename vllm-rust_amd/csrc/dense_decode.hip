@@ -4,7 +4,7 @@
 // Such a step is a chain of short launches over weights that are read once (Qwen3-0.6B: 4 .. 13 MB each), so what bounds it is the
 // latency of each link: the weights of a workgroup are requested before anything they wait for is computed, and no result is converted
 // by a launch of its own.  Qwen3-0.6B at one row, 128 tokens: 12 launches and 43 us a layer as norm, GEMV, widening, activation kernels;
-// 5 launches and 27 us now (q|k|v 4.9 us, attention 7.6, o 4.7, gate|up 6.4 = 2.0 TB/s, down 4.5); the whole step 1269 -> 795 us.
+// 5 launches and 26 us now (q|k|v 4.2 us, attention 7.4, o 4.2, gate|up 5.8 = 2.2 TB/s, down 4.6); the whole step 1269 -> 795 us.
 #include "vmx_kernels.h"
 
 namespace {

@@ -1975,6 +1975,9 @@ static int prompt_slices(int M, int N, int K, bool own_pass) {
 // 3 TB/s and more.  It leaves the plan's slices, so the tiles have to as well.  us, 333 rows of Qwen3-8B, tiles alone / with 13 rows apart: gate|up 98.8 /
 // 69.6 + 12.6, down 59 / 39.4 + 9.4, q|k|v 34.0 / 26.6 + 6.0; the prompt (9 layers) 2352 -> 2143.  bf16 results that differ from the rounded exact ones: tiles 0.8e-4 .. 4.7e-4, the
 // 16-row form 1.2e-4 .. 4.6e-4 (rows of mean 0 and 5, of sizes 2^-12 .. 2^12, with outliers of 100; 1.5e-4 .. 25e-4 before its weights became 16 + nibble)
+// One and sixteen rows behind 1 .. 32 tiles, prompts of four sizes, before / with the pass apart (and slices of one k slice in bf16, below 1 %):  width 4096, gate and up 2 x 12288
+// (4 layers) 321 rows 1020 / 913, 513 1262 / 1207, 641 1597 / 1450, 1025 2210 / 2099, 1040 2212 / 2107;  2048, 2 x 6144 (6) 321 734 / 704, 641 1053 / 965, 1025 1393 / 1321;
+// 4096, 2 x 14336 (4) 257 915 / 850, 272 922 / 861, 641 1625 / 1583;  8192, 2 x 12288 (1) 513 682 / 653.  Of 104 prompts of 17 .. 2049 rows none took longer.
 static int prompt_tail(int M, int N, int K) {
     const int tail = M % PF_BM, full = M - tail, tiles = full / PF_BM;
     const GemmPlan p = plan_gemm(N, K);
