@@ -690,7 +690,7 @@ int run_linear(vmx_qwen3 *, const Int4Linear &l, const uint16_t *xin, float *par
     return l.forward_partial(xin, partial, M, st);
 }
 // A prompt's linear, for readers that round the sum to bf16 before anything else: *splits slices in f32, or (-1) where one slice is the whole sum the bf16
-// values themselves, in half the bytes (2048 rows of Qwen3-8B, 9 layers: 8190 -> 8055 us)
+// values themselves, in half the bytes (2048 rows of Qwen3-8B: the norms behind them 15.4 -> 13.0 us, q|k|v's post-processing 19.4 -> 15.0)
 int run_prompt_linear(vmx_qwen3 *m, const Int4Linear &l, const uint16_t *xin, float *partial, int *splits, int M, hipStream_t st) {
     if (!vmx_int4_gemm_y_ok(M, l.out_features, l.in_features)) return run_linear(m, l, xin, partial, M, st);
     *splits = -1;
