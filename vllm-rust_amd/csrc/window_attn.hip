@@ -445,9 +445,10 @@ __global__ __launch_bounds__(512) void window_attn_talk_kernel(const WinAttn p) 
 // Every statistic of a query therefore lives in the four lanes (c, 0..3): the softmax needs two lane exchanges per tile.
 // Latency bounds it, the trips to the block table most: a branch around each of a thread's eight lookups a tile made eight trips of them, one after
 // another.  Without branches they are one trip, a thread's value chunks share theirs, and a tile that every row sees whole is not masked: 16 heads
-// over 4 of 128, a prompt of 1500 rows 66 -> 45 us, 16 rows at 1000 keys 28 -> 22.
+// over 4 of 128, a prompt of 1500 rows 66 -> 45 us, 16 rows at 1000 keys 28 -> 22, but one row of 60 keys, a single tile, 11.1 -> 11.4 (64 wide 7.9 -> 7.7); a branch
+// around the lookups of a second tile that is not there: 11.7, 64 wide 8.3.
 // Registers: heads up to 128 leave room for a third workgroup a compute unit (two / three: 16 rows at 1000 keys 23.6 / 21.5 us, 64 wide 17.3 / 15.4; a prompt of 2000 rows 118.5 /
-// 114.3, 64 wide 83.8 / 77.9; one row of 60 keys 11.2 / 11.8); wider ones keep what they want (bound to two / not: 32 rows at 3000 keys, 192 wide 163 / 156 us, 256 wide 177 / 168;
+// 114.3, 64 wide 83.8 / 77.9); wider ones keep what they want (bound to two / not: 32 rows at 3000 keys, 192 wide 163 / 156 us, 256 wide 177 / 168;
 // a prompt of 500 rows, 160 wide 22.8 / 20.8).
 template <int DS, int VS>
 __global__ __launch_bounds__(256, DS <= 4 ? 3 : 1) void window_attn_mfma_kernel(const WinAttn p) {
