@@ -208,3 +208,38 @@ def test_moe_int4_forward_matches_reference_loop(gpu, T):
     assert np.abs(got - ref).max() <= 2 ** -6 * np.abs(ref).max()
     rel = np.sqrt(((got - ref) ** 2).sum() / (ref ** 2).sum())
     assert rel <= 1e-2
+
+
+@pytest.mark.parametrize("H,I", [(4096, 14336), (2048, 8192)])
+@pytest.mark.parametrize("T,pick", [(6, "mixed"), (8, "mixed"), (8, "one expert"), (9, "two experts"), (16, "two experts"), (16, "mixed"), (40, "mixed")])
+def test_moe_blocks_of_16_rows_match_one_pass_per_pair(gpu, H, I, T, pick):
+    """The staged forms of the 16-row blocks (8 rows, 16 rows with four column tiles, 16 rows with two) beside the form with one pass per
+    (token, slot) pair, which the oracle checks above: few rows, full blocks, and a block of more than 8 rows where 8 are staged (tokens that
+    name one expert twice).  Both round to bf16 at the same points from f32 sums of another order: a hidden value that lands on the
+    other side of a rounding moves by 2^-8 of itself, so rel <= 2^-8 and no element by more than 2^-5 of the largest."""
+    from vllm_rust_amd._lib import lib
+    vmx, torch = gpu
+    g, E, k = 128, 4, 2
+    gen = torch.Generator(device="cuda").manual_seed(5 * T + H)
+    def mk(K, N):
+        qw = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 8, N), dtype=torch.int32, device="cuda", generator=gen)
+        sc = ((torch.rand(K // g, N, device="cuda", generator=gen) * 0.5 + 0.75) / (6.5 * K ** 0.5)).to(torch.bfloat16).view(torch.int16)
+        return vmx.int4_pack(qw, sc, None, K, N, g)
+    p13, p2 = [mk(H, 2 * I) for _ in range(E)], [mk(I, H) for _ in range(E)]
+    t13, t2 = (torch.tensor([p.data_ptr() for p in ps], dtype=torch.int64, device="cuda") for ps in (p13, p2))
+    x = torch.randn(T, H, device="cuda", generator=gen).to(torch.bfloat16)
+    w = torch.rand(T, k, device="cuda", generator=gen) + 0.25
+    first = torch.randint(0, E, (T,), device="cuda", generator=gen)
+    ids = {"mixed": torch.stack([first, (first + 1 + torch.arange(T, device="cuda") % (E - 1)) % E], 1), "one expert": torch.full((T, k), 2, device="cuda"),
+           "two experts": torch.tensor([1, 3], device="cuda").expand(T, k)}[pick].to(torch.int32).contiguous()
+    got = {}
+    try:
+        for rows in (0, 16):
+            lib.vmx_debug_moe_block_rows(rows)
+            got[rows] = vmx.moe_int4_forward(x, w, ids, t13, t2, E, H, I, g).float()
+    finally:
+        lib.vmx_debug_moe_block_rows(-1)
+    d, ref = got[16] - got[0], got[0]
+    assert torch.isfinite(got[16]).all()
+    assert (d.norm() / ref.norm()).item() <= 2 ** -8, (d.norm() / ref.norm()).item()
+    assert d.abs().max().item() <= 2 ** -5 * ref.abs().max().item()

@@ -542,9 +542,10 @@ template <int N, class F> __device__ __forceinline__ void ring_static_for(F &&f)
 #endif
 constexpr int RING_D = VMX_RING_D;   // passes a request runs ahead of its use
 constexpr size_t RING_LDS = 2 * 16 * 4 * KB * 2;   // two stages of four waves
+struct RingOwnRow { __device__ __forceinline__ int operator()(int m) const { return m; } };
 // 5..16 activation rows, ring form.  The looped body above waits for an L2 round trip per staging batch (8 of them on a
 // 4096-deep slice at 16 rows) with its matrix work in between: a wave spends most of its life waiting.  Here
-//   * a pass is 4 k-blocks (one per wave); its 16 x 512 activation tile is requested D passes ahead into registers (16 per
+//   * a pass is 4 k-blocks (one per wave); its 16 x 512 activation tile is requested D (RING_D) passes ahead into registers (16 per
 //     lane and pass) and written to one of two 16 KB LDS stages one pass ahead, so the round trips overlap each other and
 //     the matrix work; one barrier per pass;
 //   * weights and scale|zero words are requested D passes ahead as well; the loop is fully unrolled, every request is a plain
@@ -555,13 +556,16 @@ constexpr size_t RING_LDS = 2 * 16 * 4 * KB * 2;   // two stages of four waves
 //   * the row sums of the zero-point term come from the matrix cores (the tile times a matrix of ones).
 // A workgroup has NWV waves (a pass is NWV k-blocks, a stage 4 NWV KB); the sums of column tile nt0 + t over the k-blocks of slice ks end in
 // red [CT][NWV][64][4] at the head of smem, behind a barrier.  K % (128 NWV PASSES) == 0, (N / 16) % CT == 0; rows past M replicate row M - 1
-// (never stored).  xmap (token-grouped experts, LDS): activation row of block row m.  meanwhile(): called once the first requests are out.
-template <int PASSES, int CT, int NWV, class F>
+// (never stored).  ROWS (8 or 16, M <= ROWS) rows are staged.  xrow(m): activation row of block row m < M, the same in every lane of a wave.
+// meanwhile(): called once the first requests are out.
+template <int PASSES, int CT, int NWV, int ROWS, int D, class X, class F>
 __device__ __forceinline__ void int4_gemm_ring_sums(unsigned char *smem, const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ,
-                                                    const uint16_t *__restrict__ x, int M, int K, int group, int nt0, int ks, const int32_t *xmap,
+                                                    const uint16_t *__restrict__ x, int M, int K, int group, int nt0, int ks, X &&xrow,
                                                     F &&meanwhile) {
-    constexpr int D = RING_D, ROWB = NWV * KB * 2;   // bytes per staged row
-    unsigned char *xs = smem;                                        // [2][16][ROWB]
+    constexpr int ROWB = NWV * KB * 2;   // bytes per staged row
+    static_assert(D >= 2 && CT * NWV * 1024 <= 2 * ROWS * ROWB, "a pass is written to its stage while the one before it is multiplied; the exchange fits the stages");
+    constexpr int PIECES = ROWS / 4;                 // a wave's requests a pass
+    unsigned char *xs = smem;                                        // [2][ROWS][ROWB]
     float *red = reinterpret_cast<float *>(smem);                    // [CT][NWV][64][4], after the last pass
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nl = lane & 15, h = lane >> 4;
@@ -570,12 +574,12 @@ __device__ __forceinline__ void int4_gemm_ring_sums(unsigned char *smem, const u
 
     // staging: request j of a wave is the 1 KiB piece NWV j + wave of the tile (NWV / 4 pieces a row), lane l its chunk l.  Every address is a
     // wave-uniform base plus a 32-bit lane offset.
-    const char *xrow_u[4];
-    uint32_t xdst[4];   // byte offset of the lane's chunk inside a stage
+    const char *xrow_u[PIECES];
+    uint32_t xdst[PIECES];   // byte offset of the lane's chunk inside a stage
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int piece = NWV * j + wave, row = piece / (NWV / 4), at = piece % (NWV / 4), rsrc = min(row, M - 1);
-        xrow_u[j] = reinterpret_cast<const char *>(x + (int64_t)(xmap ? __builtin_amdgcn_readfirstlane(xmap[rsrc]) : rsrc) * K + (int64_t)kb_wg * KB + at * 512);
+    for (int j = 0; j < PIECES; j++) {
+        const int piece = NWV * j + wave, row = piece / (NWV / 4), at = piece % (NWV / 4);
+        xrow_u[j] = reinterpret_cast<const char *>(x + (int64_t)xrow(min(row, M - 1)) * K + (int64_t)kb_wg * KB + at * 512);
         xdst[j] = (uint32_t)(row * ROWB + (((at * 64 + lane) ^ (row & 15)) << 4));
     }
     const char *w_u[CT];
@@ -587,13 +591,13 @@ __device__ __forceinline__ void int4_gemm_ring_sums(unsigned char *smem, const u
     }
     const uint32_t woff = (uint32_t)lane << 4, zoff = (uint32_t)nl << 2;
     typedef unsigned int ring_u32x4 __attribute__((ext_vector_type(4)));
-    ring_u32x4 tq[D][4];
+    ring_u32x4 tq[D][PIECES];
     uint4 wq[D][CT];
     uint32_t zq[D][CT];
     auto issue = [&](auto pc) {
         constexpr int p = decltype(pc)::value, r = p % D;
 #pragma unroll
-        for (int j = 0; j < 4; j++) tq[r][j] = *reinterpret_cast<const ring_u32x4 *>(xrow_u[j] + (size_t)p * ROWB + woff);
+        for (int j = 0; j < PIECES; j++) tq[r][j] = *reinterpret_cast<const ring_u32x4 *>(xrow_u[j] + (size_t)p * ROWB + woff);
 #pragma unroll
         for (int t = 0; t < CT; t++) {
             wq[r][t] = ld_weights(reinterpret_cast<const uint4 *>(w_u[t] + (size_t)p * NWV * 64 * 16 + woff));
@@ -603,7 +607,7 @@ __device__ __forceinline__ void int4_gemm_ring_sums(unsigned char *smem, const u
     auto write_tile = [&](auto pc) {
         constexpr int p = decltype(pc)::value, r = p % D;
 #pragma unroll
-        for (int j = 0; j < 4; j++) *reinterpret_cast<ring_u32x4 *>(xs + (p & 1) * 16 * ROWB + xdst[j]) = tq[r][j];
+        for (int j = 0; j < PIECES; j++) *reinterpret_cast<ring_u32x4 *>(xs + (p & 1) * ROWS * ROWB + xdst[j]) = tq[r][j];
     };
     ring_static_for<(D < PASSES ? D : PASSES)>([&](auto pc) { issue(pc); });
     meanwhile();
@@ -624,7 +628,7 @@ __device__ __forceinline__ void int4_gemm_ring_sums(unsigned char *smem, const u
         for (int t = 0; t < CT; t++) acc[t] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const uint4 au = *reinterpret_cast<const uint4 *>(xs + (p & 1) * 16 * ROWB + fa[i]);
+            const uint4 au = *reinterpret_cast<const uint4 *>(xs + (p & 1) * ROWS * ROWB + fa[i]);
             acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, au), __builtin_bit_cast(vmx_bf16x8, ones), acc1, 0, 0, 0);
 #pragma unroll
             for (int t = 0; t < CT; t++) {
@@ -681,11 +685,11 @@ struct RingRowScale {
 };
 
 // NORM: x is a stream's rows times the norm's gains, without the factor of the row, which comes from ssq and multiplies the sums (RingRowScale).
-template <int UPW, bool GLU, int CT, bool NORM = false>
+template <int UPW, bool GLU, int CT, bool NORM = false, int ROWS = 16, int D = RING_D, class X = RingOwnRow>
 __device__ __forceinline__ void int4_gemm_ring_body(const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ,
                                                     const uint16_t *__restrict__ x, const uint16_t *__restrict__ bias,
                                                     uint16_t *__restrict__ y, float *__restrict__ partial, int64_t slice_stride, int M,
-                                                    int N, int K, int group, int block, const int32_t *xmap = nullptr,
+                                                    int N, int K, int group, int block, X &&xrow = X(),
                                                     const int32_t *omap = nullptr, const float *ssq = nullptr, float eps = 0.f) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int n_groups = N / NT / CT, nt0 = (block % n_groups) * CT, ks = block / n_groups;
@@ -693,9 +697,9 @@ __device__ __forceinline__ void int4_gemm_ring_body(const uint4 *__restrict__ W,
     if constexpr (NORM) {
         by = reinterpret_cast<float *>(smem + RING_LDS);
         RingRowScale rs(ssq, M, K);
-        int4_gemm_ring_sums<UPW, CT, 4>(smem, W, SZ, x, M, K, group, nt0, ks, xmap, [&] { rs.store(by, K, eps); });
+        int4_gemm_ring_sums<UPW, CT, 4, ROWS, D>(smem, W, SZ, x, M, K, group, nt0, ks, xrow, [&] { rs.store(by, K, eps); });
     } else {
-        int4_gemm_ring_sums<UPW, CT, 4>(smem, W, SZ, x, M, K, group, nt0, ks, xmap, [] {});
+        int4_gemm_ring_sums<UPW, CT, 4, ROWS, D>(smem, W, SZ, x, M, K, group, nt0, ks, xrow, [] {});
     }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int t = wave; t < CT; t += 4)
@@ -713,7 +717,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int tid = threadIdx.x, nt = blockIdx.x, row = (tid >> 4) & 15, n = nt * NT + (tid & 15);   // of the first four waves' threads
     const int64_t at = (int64_t)min(row, M - 1) * N + n;
     const uint16_t hold = h[at], gn = gain[n];
-    int4_gemm_ring_sums<PASSES, 1, 8>(smem, W, SZ, x, M, K, group, nt, 0, nullptr, [] {});
+    int4_gemm_ring_sums<PASSES, 1, 8, 16, RING_D>(smem, W, SZ, x, M, K, group, nt, 0, RingOwnRow(), [] {});
     if (tid >= 256) return;
     const float *red = reinterpret_cast<const float *>(smem) + ((row >> 2) * 16 + (tid & 15)) * 4 + (row & 3);   // element (row, column) of a wave's tile
     float v = 0.f;
@@ -732,7 +736,7 @@ template <int UPW, bool GLU, int CT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 3))) void int4_gemm_ring_norm_kernel(
     const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ, const uint16_t *__restrict__ hg, const float *__restrict__ ssq, int M, int N, int K, int group,
     float eps, uint16_t *__restrict__ act, float *__restrict__ partial) {
-    int4_gemm_ring_body<UPW, GLU, CT, true>(W, SZ, hg, nullptr, act, partial, (int64_t)M * N, M, N, K, group, (int)blockIdx.x, nullptr, nullptr, ssq, eps);
+    int4_gemm_ring_body<UPW, GLU, CT, true>(W, SZ, hg, nullptr, act, partial, (int64_t)M * N, M, N, K, group, (int)blockIdx.x, RingOwnRow(), nullptr, ssq, eps);
 }
 
 template <int UPW, bool GLU, int CT>
@@ -1640,33 +1644,38 @@ __global__ __launch_bounds__(256) void int4_gemm_grouped16_kernel(Int4GroupedArg
 
 // The same row blocks through the ring form (slices of whole 512-deep passes): the looped body waits for an L2 round trip per
 // staging pass, and a 16-sequence decode step of an 8-expert model is thousands of such workgroups in a dozen rounds.
-template <int UPW, bool GLU, int CT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 3))) void int4_gemm_grouped16_ring_kernel(
-    Int4GroupedArgs ga, const uint16_t *__restrict__ x, float *__restrict__ partial, uint16_t *__restrict__ act, int N, int K, int group) {
-    __shared__ int32_t xmap[16], omap[16];
-    __shared__ int m_s;
+// So a compute unit always has workgroups that start (their expert, its rows, the first requests: four round trips) and workgroups that end, and what counts is
+// how many it holds: requests go two passes ahead instead of three, and ROWS = 8 halves stages and staging registers (96 registers: five workgroups, where three
+// passes ahead of 16 rows held three).  Or CT = 4 column tiles make a workgroup's stream longer.  A block of more than ROWS rows takes another pass over its
+// weights.  Mixtral-8x7B, gate|up 4096 x 28672 and down 14336 x 4096 of the 7 experts that 8 rows hit (420 and 210 MB), us: 113 + 62 before, 88 + 49.5
+// with <2, 8> (4.8 TB/s), 86 + 49 with <4, 8> (not kept: one more form), 91 + 51 with <4, 8> three passes ahead.
+// Decode steps of four layers, before / now: 6 rows 680 / 593, 8 rows 818 / 706, 12 rows 847 / 742, 16 rows 860 / 752.
+template <int UPW, bool GLU, int CT, int ROWS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ROWS == 8 ? 5 : CT == 4 ? 2 : 3, ROWS == 8 ? 7 : CT == 4 ? 3 : 5))) void int4_gemm_grouped16_ring_kernel(
+    const void *const *__restrict__ table, const int32_t *__restrict__ sorted, const int32_t *__restrict__ block_expert,
+    const int32_t *__restrict__ total_post_pad, const uint16_t *__restrict__ x, int numel, int num_experts, int N, int K, int group, int x_row_div,
+    float *__restrict__ partial, uint16_t *__restrict__ act) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int32_t omap[16];
     const int row0 = blockIdx.y * 16, tid = threadIdx.x;
-    if (row0 >= ga.total_post_pad[0]) return;
-    int e = ga.block_expert[blockIdx.y];
-    e = e < 0 ? 0 : (e >= ga.num_experts ? ga.num_experts - 1 : e);
-    const char *packed = static_cast<const char *>(ga.table[e]);
+    int e = block_expert[blockIdx.y];
+    if (row0 >= total_post_pad[0]) return;
+    const int p = sorted[row0 + (tid & 15)];
+    e = e < 0 ? 0 : (e >= num_experts ? num_experts - 1 : e);
+    const char *packed = static_cast<const char *>(table[e]);
     if (!packed) return;   // expert held by another rank
-    if (tid < 64) {
-        const int p = tid < 16 ? ga.sorted[row0 + tid] : -1;
-        const bool valid = tid < 16 && p >= 0 && p < ga.numel;
-        if (tid < 16) {
-            xmap[tid] = valid ? p / ga.x_row_div : 0;
-            omap[tid] = valid ? p : 0;
-        }
-        const unsigned long long mask = __ballot(valid);   // the valid pairs of a block come first
-        if (tid == 0) m_s = __popcll(mask);
-    }
-    __syncthreads();
-    const int M = m_s;
+    const bool valid = p >= 0 && p < numel;
+    if (tid < 16) omap[tid] = valid ? p : 0;                               // read behind the barriers of the sums
+    const int M = __popcll(__ballot(valid) & 0xFFFFull);                   // the valid pairs of a block come first
     if (M == 0) return;
+    const int xr = valid ? p / x_row_div : 0;
     const uint4 *W = reinterpret_cast<const uint4 *>(packed);
     const uint32_t *SZ = reinterpret_cast<const uint32_t *>(packed + sz_offset_bytes(K, N));
-    int4_gemm_ring_body<UPW, GLU, CT>(W, SZ, x, nullptr, act, partial, (int64_t)ga.numel * N, M, N, K, group, (int)blockIdx.x, xmap, omap);
+    for (int m0 = 0; m0 < M; m0 += ROWS) {
+        if (m0) __syncthreads();
+        int4_gemm_ring_body<UPW, GLU, CT, false, ROWS, 2>(W, SZ, x, nullptr, act, partial, (int64_t)numel * N, min(M - m0, ROWS), N, K, group, (int)blockIdx.x,
+                                                       [&](int m) { return __builtin_amdgcn_readlane(xr, m0 + m); }, omap + m0);
+    }
 }
 
 // Grouped form for mixture-of-experts decode: blockIdx.y = p selects one (token, expert slot) pair;
@@ -2389,12 +2398,13 @@ int vmx_int4_gemm_grouped_glu(const void *const *packed_table, const int32_t *ex
 }
 
 // Token-grouped form: `sorted` / `block_expert` / `total_post_pad` as vmx_moe_align_block_size(block_size = 64) leaves them;
-// max_blocks = the host-side bound on the block count (blocks past total_post_pad exit at once).  act != NULL: experts packed
+// max_blocks = the host-side bound on the block count (blocks past total_post_pad exit at once); max_rows = how many rows an expert gets at most where no
+// token names it twice (a choice of form only).  act != NULL: experts packed
 // with glu = 1, act [pairs][N/2]; else partial [splits][pairs][N].
 bool vmx_int4_token_grouped16_ok(int N, int K) { return N % NT == 0 && K % KB == 0; }
 
 int vmx_int4_gemm_token_grouped(const void *const *packed_table, const int32_t *sorted, const int32_t *block_expert,
-                                const int32_t *total_post_pad, int max_blocks, int block_rows, int num_experts, const uint16_t *x,
+                                const int32_t *total_post_pad, int max_blocks, int block_rows, int max_rows, int num_experts, const uint16_t *x,
                                 int x_row_div, float *partial, uint16_t *act, int pairs, int N, int K, int group, hipStream_t st) {
     VMX_REQUIRE(block_rows == 16 || block_rows == 64, "int4_gemm_token_grouped: block_rows %d (16 or 64)", block_rows);
     const GemmPlan p = plan_gemm(N, K);
@@ -2407,15 +2417,19 @@ int vmx_int4_gemm_token_grouped(const void *const *packed_table, const int32_t *
         const int per_slice = kblocks % p.splits == 0 ? kblocks / p.splits : 0;
         const int rupw = per_slice % 4 == 0 ? per_slice / 4 : 0;
         if (ring_on && vmx_tune("VMX_INT4_RING", 1) && (rupw == 4 || rupw == 7 || rupw == 8) && (N / NT) % 2 == 0) {
-            const dim3 rgrid((unsigned)((N / NT / 2) * p.splits), (unsigned)max_blocks);
-#define G16R(U)                                                                                                                       \
-            do {                                                                                                                      \
-                if (act) hipLaunchKernelGGL((int4_gemm_grouped16_ring_kernel<U, true, 2>), rgrid, dim3(256), RING_LDS, st, ga, x, partial, act, N, K, group); \
-                else hipLaunchKernelGGL((int4_gemm_grouped16_ring_kernel<U, false, 2>), rgrid, dim3(256), RING_LDS, st, ga, x, partial, act, N, K, group);    \
-            } while (0)
+            // 8 staged rows where no expert can have more.  Above, four tiles a workgroup where that leaves one for every compute unit (Mixtral, 12 and 16 rows:
+            // 742 and 752 us a step against 799 and 814 with two); 8 staged rows there too were 728 and 746, but a full block would be read twice.
+            const int tiles = N / NT, ct = max_rows <= 8 || tiles % 4 != 0 || tiles / 4 * p.splits < vmx_num_cus() ? 2 : 4;
+            const dim3 rgrid((unsigned)(tiles / ct * p.splits), (unsigned)max_blocks);
+#define G16R_T(U, G, C, R) hipLaunchKernelGGL((int4_gemm_grouped16_ring_kernel<U, G, C, R>), rgrid, dim3(256), RING_LDS * R / 16, st, packed_table, sorted, \
+                                              block_expert, total_post_pad, x, pairs, num_experts, N, K, group, x_row_div, partial, act)
+#define G16R_F(U, G) do { if (max_rows <= 8) G16R_T(U, G, 2, 8); else if (ct == 4) G16R_T(U, G, 4, 16); else G16R_T(U, G, 2, 16); } while (0)
+#define G16R(U) do { if (act) G16R_F(U, true); else G16R_F(U, false); } while (0)
             if (rupw == 8) G16R(8);
             else if (rupw == 7) G16R(7);
             else G16R(4);
+#undef G16R_T
+#undef G16R_F
 #undef G16R
             VMX_CHECK_LAUNCH("int4_gemm(token grouped, ring)");
             return VMX_OK;

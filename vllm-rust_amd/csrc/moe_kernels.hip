@@ -157,18 +157,18 @@ int vmx_moe_int4_forward_glu(uint16_t *out, const uint16_t *x, const float *topk
         int32_t *sorted = (int32_t *)ws, *block_expert = sorted + ((cap + 63) & ~63), *total = block_expert + ((max_blocks + 63) & ~63);
         if (int rc = vmx_moe_align_block_size(topk_ids, sorted, block_expert, total, pairs, num_experts, brows, cap, st)) return rc;
         if (w13_glu) {
-            if (int rc = vmx_int4_gemm_token_grouped(w13_packed, sorted, block_expert, total, max_blocks, brows, num_experts, x, k, nullptr, act,
+            if (int rc = vmx_int4_gemm_token_grouped(w13_packed, sorted, block_expert, total, max_blocks, brows, tokens, num_experts, x, k, nullptr, act,
                                                      pairs, 2 * inter, hidden, group, st))
                 return rc;
         } else {
-            if (int rc = vmx_int4_gemm_token_grouped(w13_packed, sorted, block_expert, total, max_blocks, brows, num_experts, x, k, p1, nullptr,
+            if (int rc = vmx_int4_gemm_token_grouped(w13_packed, sorted, block_expert, total, max_blocks, brows, tokens, num_experts, x, k, p1, nullptr,
                                                      pairs, 2 * inter, hidden, group, st))
                 return rc;
             int64_t blocks = ((int64_t)pairs * inter + 255) / 256;
             hipLaunchKernelGGL(moe_act_kernel, dim3((unsigned)(blocks > 2048 ? 2048 : blocks)), dim3(256), 0, st, p1, s1, pairs, act, inter);
             VMX_CHECK_LAUNCH("moe_act");
         }
-        if (int rc = vmx_int4_gemm_token_grouped(w2_packed, sorted, block_expert, total, max_blocks, brows, num_experts, act, 1, p2, nullptr,
+        if (int rc = vmx_int4_gemm_token_grouped(w2_packed, sorted, block_expert, total, max_blocks, brows, tokens, num_experts, act, 1, p2, nullptr,
                                                  pairs, hidden, inter, group, st))
             return rc;
         hipLaunchKernelGGL(moe_combine_kernel, dim3((hidden + 255) / 256, tokens), dim3(256), 0, st, out, p2, s2, pairs, topk_weights, k, hidden,
@@ -369,18 +369,18 @@ extern "C" int vmx_moe_ep_int4_forward(uint16_t *out, const uint16_t *x, const f
         int32_t *sorted = (int32_t *)mws, *block_expert = sorted + ((cap + 63) & ~63), *total = block_expert + ((max_blocks + 63) & ~63);
         if (int rc = vmx_moe_align_block_size(recv_e, sorted, block_expert, total, cap_rows, per, brows, cap, st)) return rc;
         if (w13_glu) {
-            if (int rc = vmx_int4_gemm_token_grouped(w13_local, sorted, block_expert, total, max_blocks, brows, per, recv_x, 1, nullptr, act, cap_rows,
+            if (int rc = vmx_int4_gemm_token_grouped(w13_local, sorted, block_expert, total, max_blocks, brows, (int)cap_rows, per, recv_x, 1, nullptr, act, cap_rows,
                                                      2 * inter, hidden, group, st))
                 return rc;
         } else {
-            if (int rc = vmx_int4_gemm_token_grouped(w13_local, sorted, block_expert, total, max_blocks, brows, per, recv_x, 1, p1, nullptr, cap_rows,
+            if (int rc = vmx_int4_gemm_token_grouped(w13_local, sorted, block_expert, total, max_blocks, brows, (int)cap_rows, per, recv_x, 1, p1, nullptr, cap_rows,
                                                      2 * inter, hidden, group, st))
                 return rc;
             int64_t blocks = ((int64_t)cap_rows * inter + 255) / 256;
             hipLaunchKernelGGL(moe_act_kernel, dim3((unsigned)(blocks > 2048 ? 2048 : blocks)), dim3(256), 0, st, p1, s1, cap_rows, act, inter);
             VMX_CHECK_LAUNCH("moe_act");
         }
-        if (int rc = vmx_int4_gemm_token_grouped(w2_local, sorted, block_expert, total, max_blocks, brows, per, act, 1, p2, nullptr, cap_rows, hidden,
+        if (int rc = vmx_int4_gemm_token_grouped(w2_local, sorted, block_expert, total, max_blocks, brows, (int)cap_rows, per, act, 1, p2, nullptr, cap_rows, hidden,
                                                  inter, group, st))
             return rc;
         hipLaunchKernelGGL(ep_rows_finish_kernel, dim3((hidden + 255) / 256, cap_rows), dim3(256), 0, st, p2, s2, cap_rows, hidden, recv_e, y);

@@ -17,7 +17,7 @@ int vmx_int4_gemm_grouped_glu(const void *const *packed_table, const int32_t *ex
 // token-grouped matrix-core form: pairs sorted by expert in blocks of 64 rows (vmx_moe_align_block_size); act != NULL = gated epilogue
 // block_rows 64: the 64 x 128-tile kernel (prompts); 16: the small-M kernel with gathered rows (decode batches)
 int vmx_int4_gemm_token_grouped(const void *const *packed_table, const int32_t *sorted, const int32_t *block_expert,
-                                const int32_t *total_post_pad, int max_blocks, int block_rows, int num_experts, const uint16_t *x,
+                                const int32_t *total_post_pad, int max_blocks, int block_rows, int max_rows, int num_experts, const uint16_t *x,
                                 int x_row_div, float *partial, uint16_t *act, int pairs, int N, int K, int group, hipStream_t st);
 bool vmx_int4_token_grouped16_ok(int N, int K);
 // moe_kernels.hip: vmx_moe_int4_forward with the experts' gate|up tensors packed for the fused activation (w13_glu != 0)
