@@ -802,98 +802,317 @@ __device__ unsigned long long vmx_attn_stamp_buf[4096 * 8];
 #else
 #define ATTN_STAMP(i) do {} while (0)
 #endif
+// ---- tiles of 16 tokens with both products on the matrix cores (up to four query heads per KV head)
+// The scores are formed transposed, S^T = K Q^T: lane (dg, n) ends up with four tokens 4 dg + r of head n & 3, so the softmax of a tile is three
+// maxima in the lane and two across lanes, its sum stays in the lane until the end, and the probabilities lie as the second product takes them as its
+// left operand.  That product has 16 rows and only four heads, so the rows hold each probability in three bf16 terms of 8 bits (row 4 term + head:
+// together the 24 bits of the f32 number; fp16 caches: terms of 11 bits of 2^15 p) and the three sums are added at the end: no bit of p is lost.  (An infinite
+// value makes its number NaN, 0 inf in a term, where it was infinite: the projection behind makes NaN of either.)
+// V takes the way K takes (one address for both), goes through the wave's own rows in LDS and comes back transposed (ds_read_b64_tr_b16).
+// Against p broadcast lane by lane and a multiply-add per number (447 vector instructions a tile, a branch a token): see the kernel.
+template <int HD, int FP8> struct DecTile {
+    typename Raw8<FP8>::T k[HD / 32], v[HD / 32];
+};
+constexpr int dec_vld(int hd) { return hd + 16; }   // elements a staged V row: rows 8 banks apart
+
+// Where the rows of tile [t0, min(t0 + 16, p1)) lie: lane (tl, dg) addresses token tl; past the end the last valid one again.
+struct DecPages {   // the sequence's block-table row; BTREG: lane l of reg holds entry base + l
+    const int32_t *row;
+    int reg, base;
+    uint32_t size, recip;   // tokens a page, dec_recip of it
+};
+// n / d for n < 2^31 with recip = dec_recip(d): floor(n recip / 2^32) is the quotient or one less.
+__device__ __forceinline__ uint32_t dec_div(uint32_t n, uint32_t d, uint32_t recip) {
+    const uint32_t q = __umulhi(n, recip);
+    return n - q * d >= d ? q + 1 : q;
+}
+inline uint32_t dec_recip(uint32_t d) { return d <= 1 ? 0xFFFFFFFFu : (uint32_t)(((uint64_t)1 << 32) / d); }
+template <bool BTREG>
+__device__ __forceinline__ int64_t dec_tile_row(const DecPages &pg, int t0, int p1, int lane) {   // cache row (token slot) of the lane's token
+    const uint32_t tok = (uint32_t)(t0 + min(lane & 15, min(16, p1 - t0) - 1)), page = dec_div(tok, pg.size, pg.recip);
+    int blk = 0;
+    if constexpr (BTREG) blk = __shfl(pg.reg, (int)page - pg.base, 64);
+    else {
+        blk = pg.row[page];
+        asm volatile("" : "+v"(blk));   // waited for here, not where this branch meets the other
+    }
+    return (int64_t)blk * (int)pg.size + (tok - page * pg.size);
+}
+template <int HD> __device__ __forceinline__ int64_t dec_row_at(int64_t row, int64_t tok_stride, int kvh, int lane) {
+    return row * tok_stride + (int64_t)kvh * HD + 8 * (lane >> 4);
+}
+template <int HD, int FP8>
+__device__ __forceinline__ void dec_rows_load(typename Raw8<FP8>::T (&r)[HD / 32], const void *__restrict__ cache, int64_t base) {
+#pragma unroll
+    for (int i = 0; i < HD / 32; i++) r[i] = load8_raw<FP8>(cache, base + 32 * i);
+}
+// Eight cached numbers as the matrix instructions take them: e4m3 -> bf16 is exact, 16-bit caches as they are.
+template <int FP8> __device__ __forceinline__ uint4 dec_operand(const typename Raw8<FP8>::T raw) {
+    if constexpr (kv16<FP8>()) return raw;
+    else {
+        float f[8];
+        cvt8<FP8>(raw, 1.0f, f);
+        return make_uint4(__builtin_amdgcn_perm(__float_as_uint(f[1]), __float_as_uint(f[0]), 0x07060302u), __builtin_amdgcn_perm(__float_as_uint(f[3]), __float_as_uint(f[2]), 0x07060302u),
+                          __builtin_amdgcn_perm(__float_as_uint(f[5]), __float_as_uint(f[4]), 0x07060302u), __builtin_amdgcn_perm(__float_as_uint(f[7]), __float_as_uint(f[6]), 0x07060302u));
+    }
+}
+typedef short dec_s16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 dec_f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 dec_f16x8 __attribute__((ext_vector_type(8)));
+template <int FP8> __device__ __forceinline__ vmx_f32x4 dec_scores(uint4 a, uint4 b, vmx_f32x4 c) {
+    if constexpr (FP8 == 3) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(dec_f16x8, a), __builtin_bit_cast(dec_f16x8, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, a), __builtin_bit_cast(vmx_bf16x8, b), c, 0, 0, 0);
+}
+
+// State of a wave: running maximum (of head lane & 3, the same in the four lane groups), this lane's share of its sum, and o[b][r] = term dg of head r,
+// number 16 b + (lane & 15).
+template <int HD> struct DecState {
+    float m = -FLT_MAX, s = 0.f;
+    vmx_f32x4 o[HD / 16];
+};
+
+template <int HD, int FP8, bool BTREG>
+__device__ __forceinline__ void dec_walk(DecState<HD> &st, const uint16_t *q_row, uint16_t *vs, const void *__restrict__ k_cache, const void *__restrict__ v_cache,
+                                         const DecPages &pg, int p0, int p1, int64_t tok_stride, int kvh, float lscale, int lane, DecTile<HD, FP8> &t) {
+    constexpr int KS = HD / 32, NB = HD / 16, VLD = dec_vld(HD);
+    constexpr uint32_t HEAD_BITS = FP8 == 3 ? 0xFFFFE000u : 0xFFFF0000u;   // sign, exponent and the leading bits of a term
+    const int tl = lane & 15, dg = lane >> 4, term = tl >> 2;
+    const uint32_t cut1 = term >= 1 ? HEAD_BITS : 0u, cut2 = term >= 2 ? HEAD_BITS : 0u, live = term < 3 ? 0xFFFFFFFFu : 0u;
+    uint16_t *const v_to = vs + tl * VLD + 8 * dg;
+    const uint16_t *const v_from = vs + (4 * dg + (tl >> 2)) * VLD + 4 * (tl & 3);
+#pragma unroll
+    for (int b = 0; b < NB; b++) st.o[b] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto scores = [&](int ntok) {   // of the tile, whose V rows go to LDS: its registers are free afterwards
+        vmx_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < KS; i++) acc = dec_scores<FP8>(dec_operand<FP8>(t.k[i]), *reinterpret_cast<const uint4 *>(q_row + 32 * i), acc);   // q from LDS: 16 registers less
+#pragma unroll
+        for (int i = 0; i < KS; i++) {   // rows past the end count for nothing, whatever the last valid one holds
+            uint4 x = dec_operand<FP8>(t.v[i]);
+            if (ntok < 16 && tl >= ntok) x = make_uint4(0, 0, 0, 0);
+            *reinterpret_cast<uint4 *>(v_to + 32 * i) = x;
+        }
+        return acc;
+    };
+    auto fold = [&](const vmx_f32x4 acc, int ntok) {
+        float l[4], x[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) l[r] = 4 * dg + r < ntok ? acc[r] * lscale : -FLT_MAX;
+        float mx = fmaxf(fmaxf(l[0], l[1]), fmaxf(l[2], l[3])), a, b2;
+        vmx_swap_pair<16>(mx, a, b2); mx = fmaxf(a, b2);
+        vmx_swap_pair<32>(mx, a, b2); mx = fmaxf(a, b2);
+        const float m_new = fmaxf(st.m, mx), corr = __expf(st.m - m_new);   // 0 on the first tile (m = -FLT_MAX)
+        st.m = m_new;
+        st.s *= corr;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float e = 4 * dg + r < ntok ? __expf(l[r] - m_new) : 0.f;
+            st.s += e;
+            x[r] = FP8 == 3 ? e * 32768.f : e;
+            x[r] -= __uint_as_float(__float_as_uint(x[r]) & cut1);
+            x[r] -= __uint_as_float(__float_as_uint(x[r]) & cut2);
+        }
+        uint2 pa;
+        if constexpr (FP8 == 3) {
+            pa.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x[0], x[1])) & live;
+            pa.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x[2], x[3])) & live;
+        } else {
+            pa.x = __builtin_amdgcn_perm(__float_as_uint(x[1]), __float_as_uint(x[0]), 0x07060302u) & live;
+            pa.y = __builtin_amdgcn_perm(__float_as_uint(x[3]), __float_as_uint(x[2]), 0x07060302u) & live;
+        }
+        if (__ballot(corr != 1.0f)) {   // a quad of lanes holds the four heads
+            const float c[4] = {vmx_dpp<0x00>(corr), vmx_dpp<0x55>(corr), vmx_dpp<0xAA>(corr), vmx_dpp<0xFF>(corr)};
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) st.o[b][r] *= c[r];
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const dec_s16x4 vb = __builtin_amdgcn_ds_read_tr16_b64_v4i16((dec_s16x4 __attribute__((address_space(3))) *)(v_from + 16 * b));
+            if constexpr (FP8 == 3)
+                st.o[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(dec_f16x4, pa), __builtin_bit_cast(dec_f16x4, vb), st.o[b], 0, 0, 0);
+            else
+                st.o[b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(dec_s16x4, pa), vb, st.o[b], 0, 0, 0);
+        }
+    };
+    int t0 = p0;
+    for (; t0 + 16 < p1; t0 += 16) {
+        const int64_t base = dec_row_at<HD>(dec_tile_row<BTREG>(pg, t0 + 16, p1, lane), tok_stride, kvh, lane);
+        const vmx_f32x4 acc = scores(16);
+        dec_rows_load<HD, FP8>(t.k, k_cache, base);
+        dec_rows_load<HD, FP8>(t.v, v_cache, base);
+        fold(acc, 16);
+    }
+    fold(scores(p1 - t0), p1 - t0);
+}
+
+// Lanes 32 .. 63 of a and 0 .. 31 of b (MASK 32), odd rows of a and even rows of b (MASK 16) change places.
+template <int MASK> __device__ __forceinline__ void dec_swap(float &a, float &b) {
+    if constexpr (MASK == 32) asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    else asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+// The three terms' sums added up, out[e][r]: head r, number 16 (4 e + dec_block(dg)) + (lane & 15).
+__device__ __forceinline__ int dec_block(int dg) { return (dg >> 1) | ((dg & 1) << 1); }
+template <int HD> __device__ __forceinline__ void dec_add_terms(const vmx_f32x4 (&o)[HD / 16], float (&out)[HD / 64][4]) {
+#pragma unroll
+    for (int e = 0; e < HD / 64; e++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            float s[2];
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                float a = o[4 * e + 2 * c][r], b = o[4 * e + 2 * c + 1][r];
+                dec_swap<32>(a, b);
+                s[c] = a + b;
+            }
+            dec_swap<16>(s[0], s[1]);
+            out[e][r] = s[0] + s[1];
+        }
+}
+
+constexpr bool split_on_mfma(int qpk) { return qpk <= 4; }
+constexpr int split_wave_floats(int hd, int qpk) { return split_on_mfma(qpk) ? 8 * dec_vld(hd) : qpk * hd; }   // 16 staged rows hold four heads' results
+// The launch is a chain of trips to memory, so its prologue is one straight line: whatever has an address known at entry (the first eight arguments are there when
+// a wave starts) is requested first -- the block-table row (lane l = entry l, tile lookups are lane exchanges), the wave's head of the qkv sums, three scalars,
+// norm weights and scales (of partial's own memory where there are none: no branch) -- then rotation factors and the first tile, and only then is anything waited
+// for.  The tile of the new token is requested with the others; its own row, which this workgroup derives, is put in from LDS.
+// Before (loads behind branches, each waited for; 64-bit divisions; that tile behind the barrier; p broadcast lane by lane) / now, us a launch, 8 KV heads:
+// Qwen3-0.6B, one row of 128 tokens 7.5 / 5.4; Qwen3-8B of 300 8.9 / 6.8 (fp16 9.2 / 6.7); 256-wide FP8 heads 10.1 / 6.9; 16 rows of 1500 to 800 tokens 25.8 / 21.1
+// (75 MB of K and V; the tiles requested and not multiplied: 22.1 with the prologue as it was).  Steps: 770 / 718, 442 / 419, 747 / 725, 742 / 706, 713 / 674.
 template <int HD, int QPK, int FP8, int NW>
-__global__ __launch_bounds__(64 * NW) void split_decode_attn_kernel(
-    float *__restrict__ tmp_out, float *__restrict__ exp_sums, float *__restrict__ max_logits, const float *__restrict__ partial, int splits,
-    int tokens, void *__restrict__ k_cache, void *__restrict__ v_cache, const uint16_t *__restrict__ q_norm_w,
-    const uint16_t *__restrict__ k_norm_w, float eps, const float *__restrict__ cos_sin, const int32_t *__restrict__ positions,
-    const int32_t *__restrict__ slots, const int32_t *__restrict__ block_tables, const int32_t *__restrict__ seq_lens, float scale, int Hq,
-    int Hkv, int rot_dim, int max_blocks_per_seq, int block_size, int window, const float *__restrict__ k_scale_ptr,
-    const float *__restrict__ v_scale_ptr, int v_norm, const uint16_t *__restrict__ had_svh) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HD == 256 ? 2 : 4))) void split_decode_attn_kernel(
+    const float *__restrict__ partial, const int32_t *__restrict__ seq_lens, const int32_t *__restrict__ block_tables, const int32_t *__restrict__ positions,
+    const int32_t *__restrict__ slots, int heads, int splits_tokens, int max_blocks_per_seq, void *__restrict__ k_cache, void *__restrict__ v_cache,
+    const uint16_t *__restrict__ q_norm_w, const uint16_t *__restrict__ k_norm_w, const float *__restrict__ cos_sin, const uint16_t *__restrict__ had_svh,
+    int block_size, uint32_t page_recip, int P, uint32_t parts_recip, int rot_dim, int window, float eps, float scale, const float *__restrict__ k_scale_ptr,
+    const float *__restrict__ v_scale_ptr, int v_norm, float *__restrict__ tmp_out, float *__restrict__ exp_sums, float *__restrict__ max_logits) {
+    // heads = query heads per KV head | KV heads << 8; splits_tokens = split-K slices of the sums | rows << 8
     constexpr int KSTEPS = HD / 32, NP = HD >= 128 ? HD / 128 : 1, EPL = HD / 64;
-    const int nq = Hq / Hkv, P = gridDim.z;
+    constexpr bool MX = split_on_mfma(QPK);
+    constexpr int MOW = split_wave_floats(HD, QPK);                              // floats a wave owns: its results, before them its staged V rows
+    const int nq = heads & 255, Hkv = heads >> 8, Hq = nq * Hkv, splits = splits_tokens & 255, tokens = splits_tokens >> 8;
     extern __shared__ __align__(16) unsigned char smem_attn[];
-    uint16_t *qs = reinterpret_cast<uint16_t *>(smem_attn);                      // [QPK][HD] bf16
-    float *mo = reinterpret_cast<float *>(smem_attn + QPK * HD * 2);             // [NW][QPK][HD]
-    float *mm = mo + NW * QPK * HD;                                              // [NW][QPK] max
+    uint16_t *qs = reinterpret_cast<uint16_t *>(smem_attn);                      // [QPK][HD] 16-bit
+    uint16_t *kvs = qs + QPK * HD;                                               // [2][HD] the new token's k and v rows as the cache holds them
+    float *mo = reinterpret_cast<float *>(smem_attn + (QPK + 2) * HD * 2);       // [NW][MOW]: [QPK][HD] each
+    float *mm = mo + NW * MOW;                                                   // [NW][QPK] max
     float *ms = mm + NW * QPK;                                                   // [NW][QPK] sum
-    const int kvh = blockIdx.x, seq = blockIdx.y, part = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int kvh = blockIdx.x, seq = blockIdx.y, part = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tl = lane & 15, dg = lane >> 4;
-    // The launch is a chain of memory round trips, so whatever has a known address is requested at once: the three per-row
-    // scalars, the block-table row (lane l = entry l; tile lookups are then lane exchanges), and below the wave's head of the
-    // qkv sums with its norm weights -- none of them waits for seq_len.
+    ATTN_STAMP(0);
     const int seq_len = seq_lens[seq];
     const int pos = positions[seq];
     const int slot = slots[seq];
     const int32_t *bt_row = block_tables + (int64_t)seq * max_blocks_per_seq;
     int bt_reg = bt_row[min(lane, max_blocks_per_seq - 1)], bt_base = 0;
-    const float ksc = (FP8 && k_scale_ptr) ? *k_scale_ptr : 1.0f;
-    const float vsc = (FP8 && v_scale_ptr) ? *v_scale_ptr : 1.0f;
 
-    ATTN_STAMP(0);
     // ---- A (loads): head `wave` of this KV head's q heads, then k, then v (NW >= nq + 2 waves, checked on the host)
     const bool has_head = wave < nq + 2;
     const bool is_q = wave < nq, is_k = wave == nq;
-    float v[EPL], nwf[EPL];
-    uint16_t sv0 = 0x3c00, sv1 = 0x3c00;   // EXL3 output scales of this lane's two elements (HD == 128)
-    {
-        const int head = is_q ? kvh * nq + wave : (is_k ? Hq + kvh : Hq + Hkv + kvh);
-        if constexpr (HD == 128) {
-            if (had_svh) { sv0 = had_svh[(int64_t)(has_head ? head : 0) * HD + lane]; sv1 = had_svh[(int64_t)(has_head ? head : 0) * HD + lane + 64]; }
-        }
-        const int ntot = (Hq + 2 * Hkv) * HD;
-        const int64_t slice = (int64_t)tokens * ntot, base = (int64_t)seq * ntot + (int64_t)(has_head ? head : 0) * HD;
-        const uint16_t *nw = is_q ? q_norm_w : (is_k ? k_norm_w : nullptr);
+    const int head = is_q ? kvh * nq + wave : is_k ? Hq + kvh : has_head ? Hq + Hkv + kvh : 0;
+    const int ntot = (Hq + 2 * Hkv) * HD;
+    const int64_t slice = (int64_t)tokens * ntot;
+    const float *src = partial + (int64_t)seq * ntot + (int64_t)head * HD;
+    float raw[4][EPL];
 #pragma unroll
-        for (int j = 0; j < EPL; j++) nwf[j] = nw ? vmx_ld16<FP8 == 3>(nw[lane + 64 * j]) : 1.0f;
-        attn_sum_splits<EPL>(partial + base + lane, splits, slice, v);
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int j = 0; j < EPL; j++) raw[u][j] = src[min(u, splits - 1) * slice + lane + 64 * j];
+    __builtin_amdgcn_sched_barrier(0);
+    const uint16_t *none = reinterpret_cast<const uint16_t *>(partial);
+    const uint16_t *nw = is_q ? q_norm_w : (is_k ? k_norm_w : nullptr), *nw_at = nw ? nw : none;
+    uint16_t nw16[EPL];
+#pragma unroll
+    for (int j = 0; j < EPL; j++) nw16[j] = nw_at[lane + 64 * j];
+    uint16_t sv0 = 0, sv1 = 0;   // EXL3 output scales of this lane's two elements (HD == 128)
+    if constexpr (HD == 128 && FP8 != 1) {
+        const uint16_t *sv_at = (had_svh ? had_svh : none) + (int64_t)head * HD + lane;
+        sv0 = sv_at[0];
+        sv1 = sv_at[64];
     }
-    asm volatile("" ::"v"(v[0]));   // the split sums have landed
-    ATTN_STAMP(1);
-    // rotation factors of this lane's pairs (position known after the first round trip)
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::"s"(seq_len), "s"(pos), "s"(slot), "s"(k_cache), "s"(v_cache));   // the scalars were requested before the sums, not where they are used
+    float ksc = 1.0f, vsc = 1.0f;
+    if constexpr (FP8 == 1) {
+        const float k1 = *(k_scale_ptr ? k_scale_ptr : partial), v1 = *(v_scale_ptr ? v_scale_ptr : partial);
+        ksc = k_scale_ptr ? k1 : 1.0f;
+        vsc = v_scale_ptr ? v1 : 1.0f;
+    }
+    // rotation factors of this lane's pairs: half a multiple of 64: cos / sin of pair lane + 64 j, j < half / 64; half == 32: of pair lane & 31
     const int half = rot_dim >> 1;
     const float *cs = cos_sin + (int64_t)pos * rot_dim;
-    float rc[EPL], rs[EPL];   // (half & 63) == 0: cos / sin of pair j < half/64; half == 32: of pair lane & 31 in [0]
+    const int cs_lane = (half & 63) == 0 ? lane : lane & 31;
+    float rc[EPL], rs[EPL];
 #pragma unroll
     for (int j = 0; j < EPL; j++) { rc[j] = 1.f; rs[j] = 0.f; }
-    if ((half & 63) == 0) {
 #pragma unroll
-        for (int j = 0; j < EPL / 2; j++)
-            if (j < (half >> 6)) { rc[j] = cs[lane + 64 * j]; rs[j] = cs[half + lane + 64 * j]; }
-    } else {
-        rc[0] = cs[lane & 31];
-        rs[0] = cs[32 + (lane & 31)];
+    for (int j = 0; j < (EPL > 1 ? EPL / 2 : 1); j++) {
+        const int i = min(cs_lane + 64 * j, half - 1);
+        rc[j] = cs[i];
+        rs[j] = cs[half + i];
     }
 
-    // ---- tiles of this workgroup / wave (needs seq_len), and the wave's first tile if it lies before the new token
+    // ---- tiles of this workgroup / wave, and the wave's first tile
     const int start = (window > 0 && seq_len > window) ? seq_len - window : 0;
     const int T = (seq_len - start + 15) >> 4;                  // tiles of this sequence
     // this workgroup's tiles: P contiguous ranges of T/P tiles, rounded down or up (fewer tiles than workgroups: one each for
     // the first T); inside the workgroup the same deal over its waves, so no wave walks more than one tile above the average
-    const int g0 = T >= P ? (int)((int64_t)part * T / P) : min(part, T), g1 = T >= P ? (int)((int64_t)(part + 1) * T / P) : min(part + 1, T);
+    const uint32_t each = dec_div((uint32_t)T, (uint32_t)P, parts_recip), over = (uint32_t)T - each * (uint32_t)P;   // part T / P = part each + part over / P
+    const int g0 = T >= P ? (int)(part * each + dec_div(part * over, (uint32_t)P, parts_recip)) : min(part, T);
+    const int g1 = T >= P ? (int)((part + 1) * each + dec_div((part + 1) * over, (uint32_t)P, parts_recip)) : min(part + 1, T);
     const bool owner = seq_len > 0 && g0 < T && g1 == T;        // its range ends with the tile of the new token
     const int ng = g1 - g0;
     const int w0 = ng >= NW ? g0 + wave * ng / NW : g0 + min(wave, ng), w1 = ng >= NW ? g0 + (wave + 1) * ng / NW : g0 + min(wave + 1, ng);
     const bool active = seq_len > 0 && w0 < w1;
     const int p0 = start + 16 * w0, p1 = min(start + 16 * w1, seq_len);
     // block-table entries in a register: every token of the walk lies in the first 64 blocks, or else in 64 of the wave's own
-    bool bt_regs = (seq_len + block_size - 1) / block_size <= 64;
+    bool bt_regs = seq_len <= 64 * (int64_t)block_size;
     if (!bt_regs && active && (p1 - 1) / block_size - p0 / block_size < 64) {
         bt_base = p0 / block_size;
         bt_reg = bt_row[min(bt_base + lane, max_blocks_per_seq - 1)];
+        asm volatile("" : "+v"(bt_reg));   // waited for here: behind the branch the lookup waits for the first load only
         bt_regs = true;
     }
-    AttnTile<HD, FP8> tile;
+    std::conditional_t<MX, DecTile<HD, FP8>, AttnTile<HD, FP8>> tile;
+    const DecPages pages{bt_row, bt_reg, bt_base, (uint32_t)block_size, page_recip};
     const bool pre = active && p0 + 16 < seq_len;
-    if (pre) {
+    bool fresh = false;   // the lane's token is the new one: its row is not in the cache yet
+    if constexpr (MX) {
+        if (active) {
+            const int64_t row = bt_regs ? dec_tile_row<true>(pages, p0, p1, lane) : dec_tile_row<false>(pages, p0, p1, lane);
+            const int64_t base = dec_row_at<HD>(row, (int64_t)Hkv * HD, kvh, lane);
+            dec_rows_load<HD, FP8>(tile.k, k_cache, base);
+            dec_rows_load<HD, FP8>(tile.v, v_cache, base);
+            fresh = !pre && row == slot;
+        }
+    } else if (pre) {
         if (bt_regs) attn_tile_load<HD, FP8, true>(tile, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, lane, bt_reg, bt_base);
         else attn_tile_load<HD, FP8, false>(tile, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, lane);
+    }
+    float v[EPL], nwf[EPL];
+#pragma unroll
+    for (int j = 0; j < EPL; j++) {
+        nwf[j] = nw ? vmx_ld16<FP8 == 3>(nw16[j]) : 1.0f;
+        v[j] = 0.f;
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[j] += u < splits ? raw[u][j] : 0.f;   // slices added in index order
+    }
+    for (int s0 = 4; s0 < splits; s0 += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int j = 0; j < EPL; j++) raw[u][j] = src[min(s0 + u, splits - 1) * slice + lane + 64 * j];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int j = 0; j < EPL; j++) v[j] += s0 + u < splits ? raw[u][j] : 0.f;
     }
 
     ATTN_STAMP(2);
     // ---- A (arithmetic): bf16 round, optional per-head RMSNorm, NeoX RoPE; q -> LDS, k and v -> cache (owner only)
     if (has_head && g0 < T && (is_q || owner)) {
-        if constexpr (HD == 128) {   // EXL3: the sums are the trellis GEMM before its output transform; a head is one Hadamard block
+        if constexpr (HD == 128 && FP8 != 1) {   // EXL3: the sums are the trellis GEMM before its output transform; a head is one Hadamard block
             if (had_svh) attn_exl3_out_transform(v, lane, sv0, sv1);
         }
         float ss = 0.f;
@@ -933,7 +1152,11 @@ __global__ __launch_bounds__(64 * NW) void split_decode_attn_kernel(
             void *cache = is_k ? k_cache : v_cache;
             if constexpr (kv16<FP8>()) {
 #pragma unroll
-                for (int j = 0; j < EPL; j++) ((uint16_t *)cache)[dst + lane + 64 * j] = vmx_st16<FP8 == 3>(v[j]);
+                for (int j = 0; j < EPL; j++) {
+                    const uint16_t b = vmx_st16<FP8 == 3>(v[j]);
+                    ((uint16_t *)cache)[dst + lane + 64 * j] = b;
+                    kvs[(is_k ? 0 : HD) + lane + 64 * j] = b;
+                }
             } else {
                 const float sc = is_k ? ksc : vsc;
 #pragma unroll
@@ -941,7 +1164,9 @@ __global__ __launch_bounds__(64 * NW) void split_decode_attn_kernel(
                     float a = v[j] / sc;
                     a = fminf(fmaxf(a, -448.0f), 448.0f);
                     a = vmx_bf16_to_f32(vmx_f32_to_bf16(a));
-                    ((uint8_t *)cache)[dst + lane + 64 * j] = (uint8_t)(__builtin_amdgcn_cvt_pk_fp8_f32(a, a, 0, false) & 0xFFu);
+                    const uint8_t b = (uint8_t)(__builtin_amdgcn_cvt_pk_fp8_f32(a, a, 0, false) & 0xFFu);
+                    ((uint8_t *)cache)[dst + lane + 64 * j] = b;
+                    reinterpret_cast<uint8_t *>(kvs)[(is_k ? 0 : HD) + lane + 64 * j] = b;
                 }
             }
         }
@@ -951,38 +1176,74 @@ __global__ __launch_bounds__(64 * NW) void split_decode_attn_kernel(
 
     // ---- B
     ATTN_STAMP(4);
-    float m_run[4], s_run[4];
-    float o[QPK][NP][2];
-    if (active) {   // wave-uniform
-        uint4 qa[KSTEPS];
+    if constexpr (MX) {
+        DecState<HD> st;
+        if (active) {   // wave-uniform
+            const uint16_t *q_row = qs + min(lane & 3, nq - 1) * HD + 8 * dg;
+            uint16_t *vs = reinterpret_cast<uint16_t *>(mo + wave * MOW);
+            if (!pre && fresh) {
 #pragma unroll
-        for (int i = 0; i < KSTEPS; i++) {
-            qa[i] = make_uint4(0, 0, 0, 0);
-            if (tl < nq) qa[i] = *reinterpret_cast<const uint4 *>(qs + tl * HD + 32 * i + 8 * dg);
+                for (int i = 0; i < KSTEPS; i++) {
+                    tile.k[i] = load8_raw<FP8>(kvs, 32 * i + 8 * dg);
+                    tile.v[i] = load8_raw<FP8>(kvs, HD + 32 * i + 8 * dg);
+                }
+            }
+            if (bt_regs) dec_walk<HD, FP8, true>(st, q_row, vs, k_cache, v_cache, pages, p0, p1, (int64_t)Hkv * HD, kvh, scale * ksc, lane, tile);
+            else dec_walk<HD, FP8, false>(st, q_row, vs, k_cache, v_cache, pages, p0, p1, (int64_t)Hkv * HD, kvh, scale * ksc, lane, tile);
         }
-        if (bt_regs)
-            attn_walk<HD, QPK, FP8, true>(qa, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, scale * ksc, vsc, lane,
-                                          m_run, s_run, o, tile, pre, bt_reg, bt_base);
-        else
-            attn_walk<HD, QPK, FP8, false>(qa, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, scale * ksc, vsc, lane,
-                                           m_run, s_run, o, tile, pre);
-    }
-    asm volatile("" ::"v"(o[0][0][0]), "v"(s_run[0]));
-    ATTN_STAMP(5);
-    const bool lane_live = (HD >= 128) || (lane < 32);
-#pragma unroll
-    for (int h = 0; h < QPK; h++) {
-        float sh = 0.f, mh = -FLT_MAX;
+        ATTN_STAMP(5);
         if (active) {
-            sh = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s_run[h & 3]), 16 * (h >> 2)));
-            mh = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m_run[h & 3]), 16 * (h >> 2)));
-        }
-        if (lane == 0) { mm[wave * QPK + h] = mh; ms[wave * QPK + h] = sh; }
-        if (active && lane_live) {
-            const float inv = 1.0f / (sh + 1e-6f);
+            float a, b2;
+            vmx_swap_pair<16>(st.s, a, b2); st.s = a + b2;
+            vmx_swap_pair<32>(st.s, a, b2); st.s = a + b2;
+            float out[HD / 64][4];
+            dec_add_terms<HD>(st.o, out);
+            const float inv = vsc * (FP8 == 3 ? 0x1p-15f : 1.0f) / (st.s + 1e-6f);
+            const float c[4] = {vmx_dpp<0x00>(inv), vmx_dpp<0x55>(inv), vmx_dpp<0xAA>(inv), vmx_dpp<0xFF>(inv)};
+            float *to = mo + wave * MOW + 16 * dec_block(dg) + tl;   // the staged rows have been read
 #pragma unroll
-            for (int p = 0; p < NP; p++)
-                *reinterpret_cast<float2 *>(mo + (wave * QPK + h) * HD + 2 * lane + 128 * p) = make_float2(o[h][p][0] * inv, o[h][p][1] * inv);
+            for (int e = 0; e < HD / 64; e++)
+#pragma unroll
+                for (int r = 0; r < QPK; r++) to[r * HD + 64 * e] = out[e][r] * c[r];
+        }
+        if (lane < QPK) {
+            mm[wave * QPK + lane] = active ? st.m : -FLT_MAX;
+            ms[wave * QPK + lane] = active ? st.s : 0.f;
+        }
+    } else {
+        float m_run[4], s_run[4];
+        float o[QPK][NP][2];
+        if (active) {   // wave-uniform
+            uint4 qa[KSTEPS];
+#pragma unroll
+            for (int i = 0; i < KSTEPS; i++) {
+                qa[i] = make_uint4(0, 0, 0, 0);
+                if (tl < nq) qa[i] = *reinterpret_cast<const uint4 *>(qs + tl * HD + 32 * i + 8 * dg);
+            }
+            if (bt_regs)
+                attn_walk<HD, QPK, FP8, true>(qa, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, scale * ksc, vsc, lane,
+                                              m_run, s_run, o, tile, pre, bt_reg, bt_base);
+            else
+                attn_walk<HD, QPK, FP8, false>(qa, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, scale * ksc, vsc, lane,
+                                               m_run, s_run, o, tile, pre);
+        }
+        asm volatile("" ::"v"(o[0][0][0]), "v"(s_run[0]));
+        ATTN_STAMP(5);
+        const bool lane_live = (HD >= 128) || (lane < 32);
+#pragma unroll
+        for (int h = 0; h < QPK; h++) {
+            float sh = 0.f, mh = -FLT_MAX;
+            if (active) {
+                sh = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s_run[h & 3]), 16 * (h >> 2)));
+                mh = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m_run[h & 3]), 16 * (h >> 2)));
+            }
+            if (lane == 0) { mm[wave * QPK + h] = mh; ms[wave * QPK + h] = sh; }
+            if (active && lane_live) {
+                const float inv = 1.0f / (sh + 1e-6f);
+#pragma unroll
+                for (int p = 0; p < NP; p++)
+                    *reinterpret_cast<float2 *>(mo + wave * MOW + h * HD + 2 * lane + 128 * p) = make_float2(o[h][p][0] * inv, o[h][p][1] * inv);
+            }
         }
     }
     __syncthreads();
@@ -1004,7 +1265,7 @@ __global__ __launch_bounds__(64 * NW) void split_decode_attn_kernel(
                 const bool on = w < nwv;
                 mw[w] = on ? mm[w * QPK + h] : -FLT_MAX;
                 sw[w] = on ? ms[w * QPK + h] : 0.f;
-                ow[w] = on ? mo[(w * QPK + h) * HD + d] : 0.f;
+                ow[w] = on ? mo[w * MOW + h * HD + d] : 0.f;
             }
 #pragma unroll
             for (int w = 0; w < NW; w++) gmax = fmaxf(gmax, mw[w]);
@@ -1051,13 +1312,15 @@ int launch_split(dim3 grid, hipStream_t st, float *tmp_out, float *exp_sums, flo
                  void *kc, void *vc, const uint16_t *qn, const uint16_t *kn, float eps, const float *cos_sin, const int32_t *positions,
                  const int32_t *slots, const int32_t *bt, const int32_t *sl, float scale, int Hq, int Hkv, int rot_dim, int mbps, int bs,
                  int window, const float *ks, const float *vs, int v_norm, const uint16_t *had_svh) {
-    const size_t lds = (size_t)QPK * HD * 2 + (size_t)NW * QPK * HD * 4 + (size_t)2 * NW * QPK * 4;
+    const int nq = Hq / Hkv, P = (int)grid.z;
+    VMX_REQUIRE(nq <= 255 && Hkv < 1 << 23 && splits >= 1 && splits <= 255 && tokens < 1 << 23, "split_decode_attention: %d heads, %d slices, %d rows", Hq, splits, tokens);
+    const size_t lds = (size_t)(QPK + 2) * HD * 2 + (size_t)NW * split_wave_floats(HD, QPK) * 4 + (size_t)2 * NW * QPK * 4;
     if (lds > 64 * 1024)
         VMX_CHECK_HIP(hipFuncSetAttribute((const void *)split_decode_attn_kernel<HD, QPK, FP8, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                           (int)lds));
-    hipLaunchKernelGGL((split_decode_attn_kernel<HD, QPK, FP8, NW>), grid, dim3(64 * NW), lds, st, tmp_out, exp_sums, max_logits, partial,
-                       splits, tokens, kc, vc, qn, kn, eps, cos_sin, positions, slots, bt, sl, scale, Hq, Hkv, rot_dim, mbps, bs, window, ks,
-                       vs, v_norm, had_svh);
+    hipLaunchKernelGGL((split_decode_attn_kernel<HD, QPK, FP8, NW>), grid, dim3(64 * NW), lds, st, partial, sl, bt, positions, slots, nq | Hkv << 8, splits | tokens << 8,
+                       mbps, kc, vc, qn, kn, cos_sin, had_svh, bs, dec_recip((uint32_t)bs), P, dec_recip((uint32_t)P), rot_dim, window, eps, scale, ks, vs, v_norm,
+                       tmp_out, exp_sums, max_logits);
     VMX_CHECK_LAUNCH("split_decode_attention");
     return VMX_OK;
 }
