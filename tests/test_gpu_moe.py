@@ -211,9 +211,10 @@ def test_moe_int4_forward_matches_reference_loop(gpu, T):
 
 
 @pytest.mark.parametrize("H,I", [(4096, 14336), (2048, 8192)])
-@pytest.mark.parametrize("T,pick", [(6, "mixed"), (8, "mixed"), (8, "one expert"), (9, "two experts"), (16, "two experts"), (16, "mixed"), (40, "mixed")])
-def test_moe_blocks_of_16_rows_match_one_pass_per_pair(gpu, H, I, T, pick):
-    """The staged forms of the 16-row blocks (8 rows, 16 rows with four column tiles, 16 rows with two) beside the form with one pass per
+@pytest.mark.parametrize("T,pick", [(6, "mixed"), (8, "mixed"), (8, "one expert"), (9, "two experts"), (16, "two experts"), (16, "mixed"), (40, "mixed"), (70, "two experts"),
+                                    (80, "mixed")])
+def test_moe_blocks_of_rows_match_one_pass_per_pair(gpu, H, I, T, pick):
+    """The staged forms of the 16-row blocks (8 rows, 16 rows with four column tiles, 16 rows with two), and 64-row blocks whole, of up to 16 rows and between, beside the form with one pass per
     (token, slot) pair, which the oracle checks above: few rows, full blocks, and a block of more than 8 rows where 8 are staged (tokens that
     name one expert twice).  Both round to bf16 at the same points from f32 sums of another order: a hidden value that lands on the
     other side of a rounding moves by 2^-8 of itself, so rel <= 2^-8 and no element by more than 2^-5 of the largest."""
@@ -234,12 +235,13 @@ def test_moe_blocks_of_16_rows_match_one_pass_per_pair(gpu, H, I, T, pick):
            "two experts": torch.tensor([1, 3], device="cuda").expand(T, k)}[pick].to(torch.int32).contiguous()
     got = {}
     try:
-        for rows in (0, 16):
+        for rows in (0, 16, 64):
             lib.vmx_debug_moe_block_rows(rows)
             got[rows] = vmx.moe_int4_forward(x, w, ids, t13, t2, E, H, I, g).float()
     finally:
         lib.vmx_debug_moe_block_rows(-1)
-    d, ref = got[16] - got[0], got[0]
-    assert torch.isfinite(got[16]).all()
-    assert (d.norm() / ref.norm()).item() <= 2 ** -8, (d.norm() / ref.norm()).item()
-    assert d.abs().max().item() <= 2 ** -5 * ref.abs().max().item()
+    for rows in (16, 64):
+        d, ref = got[rows] - got[0], got[0]
+        assert torch.isfinite(got[rows]).all()
+        assert (d.norm() / ref.norm()).item() <= 2 ** -8, (rows, (d.norm() / ref.norm()).item())
+        assert d.abs().max().item() <= 2 ** -5 * ref.abs().max().item(), rows

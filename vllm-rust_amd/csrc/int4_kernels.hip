@@ -132,6 +132,10 @@ __global__ __launch_bounds__(256) void int4_dequant_kernel(const uint32_t *__res
     }
 }
 
+// An expert's weights, whose address comes from a table: said to lie in global memory, or every load through it is a flat one, which may also go to LDS, so that each
+// wait for it is a wait for everything on the way (Mixtral-8x7B, four layers, 8 decode rows 711 -> 680 us).
+__device__ __forceinline__ const char *i4_expert(const void *p) { return (const char *)(const __attribute__((address_space(1))) char *)(uintptr_t)p; }
+
 // ---------------------------------------------------------------- small-M GEMM
 // Workgroup = 4 waves = one 16-column tile x (4*UPW) consecutive k-blocks (one split-K slice);
 // wave w owns k-blocks [w*UPW, (w+1)*UPW) of the slice.  One work item per workgroup and every
@@ -1214,7 +1218,7 @@ __global__ __launch_bounds__(256) void int4_gemm_tiled_kernel(const uint4 *__res
         if (row0 >= ga.total_post_pad[0]) return;
         int e = ga.block_expert[blockIdx.y];
         e = e < 0 ? 0 : (e >= ga.num_experts ? ga.num_experts - 1 : e);
-        const char *packed = static_cast<const char *>(ga.table[e]);
+        const char *packed = i4_expert(ga.table[e]);
         if (!packed) return;
         W = reinterpret_cast<const uint4 *>(packed);
         SZ = reinterpret_cast<const uint32_t *>(packed + sz_offset_bytes(K, N));
@@ -1332,6 +1336,96 @@ __global__ __launch_bounds__(256) void int4_gemm_tiled_kernel(const uint4 *__res
             }
 }
 
+// Up to 16 rows of an expert (its last block, or all it has) by a workgroup of the kernel below, which for that many would still bring and unpack every weight
+// for 64 and take as long: a k-block is 16 rows in LDS for the four waves, a wave multiplies its four column tiles by it with the 16-row instruction and the
+// arithmetic of the ring form, its weights four k-blocks and the rows two passes of four ahead.  What bounds it is the stream of the weights.  They are not
+// loaded past the caches: the workgroup of the expert's 64 rows in front reads the same ones (below, 256 tokens: 193 + 114 us with loads that are).
+// Mixtral-8x7B, a layer's gate|up + down, us, before / now: 50 tokens (12 rows an expert) 151 + 74 / 115 + 58, 256 (64, four experts have 1 to 11 more) 212 + 108 / 187 + 109;
+// prompts of four layers 1193 / 1047, 1710 / 1616 (with plain global loads of all weights, i4_expert; 100, 180, 400, 512 tokens 1252 / 1217, 1328 / 1284, 2137 / 2048, 2574 / 2417).  Not kept: whole tiles first and these behind them, 195 + 105; 17 to 32 rows in two row tiles, 100 tokens (25 rows)
+// 146 + 72 as with a tile; the rows behind a dense prompt's last whole tile this way, 333 rows' gate|up 93 where the tiles and a launch of the ring form take 84.
+// xs: 2 x 16 rows x 1 KiB, position p of row r holds the row's 16-byte chunk p ^ r.  xrow(m): row of x that block row m < M reads; store(tile, sums): the
+// sums of tile nt0 + tile, rows 4 (lane / 16) + 0 .. 3, column lane & 15.
+template <class X, class F>
+__device__ __forceinline__ void int4_prompt_few_rows(uint16_t *xs, const uint4 *__restrict__ W, const uint32_t *__restrict__ SZ, const uint16_t *__restrict__ x, int M, int K,
+                                                     int group, int nt0, int kb_begin, int kb_end, X &&xrow, F &&store) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nl = lane & 15, h = lane >> 4;
+    const int kblocks = K / KB, G = K / group, gkb = group / KB, last = kb_end - 1;
+    typedef unsigned int few_u32x4 __attribute__((ext_vector_type(4)));
+    few_u32x4 tq[4];
+    uint4 wq[4][4];
+    uint32_t zq[4][4];
+    const char *xr[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) xr[j] = reinterpret_cast<const char *>(x + (int64_t)xrow(min(4 * wave + j, M - 1)) * K);
+    unsigned char *const stage = reinterpret_cast<unsigned char *>(xs);
+    auto fetch_x = [&](int kb) {   // of rows 4 wave ..: lane l the chunk that goes to position l
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int chunk = lane ^ (4 * wave + j);
+            tq[j] = *reinterpret_cast<const few_u32x4 *>(xr[j] + (uint32_t)min(kb + (chunk >> 4), last) * (KB * 2) + ((chunk & 15) << 4));
+        }
+    };
+    auto write_x = [&](int turn) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) *reinterpret_cast<few_u32x4 *>(stage + turn * 16384 + (4 * wave + j) * 1024 + (lane << 4)) = tq[j];
+    };
+    auto fetch_w = [&](int kb, int r) {
+        kb = min(kb, last);
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            wq[r][t] = W[((int64_t)(nt0 + t) * kblocks + kb) * 64 + lane];
+            zq[r][t] = SZ[((int64_t)(nt0 + t) * G + kb / gkb) * 16 + nl];
+        }
+    };
+    vmx_f32x4 fin[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) fin[t] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+    const int rowc = min(nl, M - 1);
+    fetch_x(kb_begin);
+#pragma unroll
+    for (int r = 0; r < 4; r++) fetch_w(kb_begin + r, r);
+    write_x(0);
+    fetch_x(kb_begin + 4);
+    int turn = 0;
+    for (int kb0 = kb_begin; kb0 < kb_end; kb0 += 4, turn ^= 1) {
+        __syncthreads();   // the pass's rows are in their stage; every wave has left the other one
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (kb0 + i >= kb_end) break;
+            vmx_f32x4 acc[4], acc1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < 4; t++) acc[t] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const uint4 au = *reinterpret_cast<const uint4 *>(stage + turn * 16384 + rowc * 1024 + (((i * 16 + 4 * s + h) ^ rowc) << 4));
+                acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, au), __builtin_bit_cast(vmx_bf16x8, ones), acc1, 0, 0, 0);
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const uint4 wv = wq[i][t];
+                    const uint32_t w = s == 0 ? wv.x : s == 1 ? wv.y : s == 2 ? wv.z : wv.w;
+                    const uint4 bu = make_uint4(((w << 3) & 0x00780078u) | 0x41804180u, ((w >> 1) & 0x00780078u) | 0x41804180u,
+                                                ((w >> 5) & 0x00780078u) | 0x41804180u, ((w >> 9) & 0x00780078u) | 0x41804180u);
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, au), __builtin_bit_cast(vmx_bf16x8, bu), acc[t], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const float sc = __uint_as_float(zq[i][t] << 16), zo = __uint_as_float(zq[i][t] & 0xFFFF0000u) - 112.f;
+#pragma unroll
+                for (int r = 0; r < 4; r++) fin[t][r] += sc * (acc[t][r] - zo * acc1[r]);
+            }
+            if (kb0 + 4 + i < kb_end) fetch_w(kb0 + 4 + i, i);
+        }
+        if (kb0 + 4 < kb_end) {
+            write_x(turn ^ 1);
+            if (kb0 + 8 < kb_end) fetch_x(kb0 + 8);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++) store(t, fin[t]);
+}
+
 // The same product with a 64-row x 256-column workgroup tile: a wave owns 64 x 64 outputs in 2 x 2 accumulators of
 // v_mfma_f32_32x32x16_bf16, two workgroups share a compute unit.  The vector ALU (unpacking, group scales) and the matrix cores both
 // need most of the time a k-block takes, so what counts is that neither waits:
@@ -1390,7 +1484,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (row0 >= ga.total_post_pad[0]) return;
         int e = ga.block_expert[rt];
         e = e < 0 ? 0 : (e >= ga.num_experts ? ga.num_experts - 1 : e);
-        const char *packed = static_cast<const char *>(ga.table[e]);
+        const char *packed = i4_expert(ga.table[e]);
         if (!packed) return;
         W = reinterpret_cast<const uint4 *>(packed);
         SZ = reinterpret_cast<const uint32_t *>(packed + sz_offset_bytes(K, N));
@@ -1399,6 +1493,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             prow_s[tid] = p >= 0 && p < ga.numel ? p : -1;
         }
         __syncthreads();
+    }
+    if constexpr (GROUPED) {
+        if (prow_s[16] < 0 && kb_begin < kb_end) {   // an expert's pairs come first in its block
+            const int rows = __popcll(__ballot(prow_s[lane & 15] >= 0) & 0xFFFFull), own = max(prow_s[lane & 15], 0);
+            if (rows == 0) return;
+            int4_prompt_few_rows(xs[0], W, SZ, x, rows, K, group, nt0, kb_begin, kb_end, [&](int m) { return __builtin_amdgcn_readlane(own, m) / ga.x_row_div; },
+                                 [&](int t, const vmx_f32x4 &v) {
+#pragma unroll
+                                     for (int r = 0; r < 4; r++) {
+                                         const int64_t p = prow_s[4 * (lane >> 4) + r];   // -1: no pair
+                                         if constexpr (GLU) {
+                                             const float up = vmx_lane_xor<8>(v[r]);
+                                             const float gg = vmx_bf16_to_f32(vmx_f32_to_bf16(v[r])), uu = vmx_bf16_to_f32(vmx_f32_to_bf16(up));
+                                             if (p >= 0 && nl < 8) act[p * (N >> 1) + (nt0 + t) * 8 + nl] = vmx_f32_to_bf16((gg / (1.0f + expf(-gg))) * uu);
+                                         } else if (p >= 0) {
+                                             partial[((int64_t)ks * slice_rows + p) * N + (nt0 + t) * 16 + nl] = v[r];
+                                         }
+                                     }
+                                 });
+            return;
+        }
     }
     // The four 1 KiB pieces of the activation tile this wave requests per k-block: piece q = rows 16 wave + 4 q .. + 3.  A row
     // past the end (or a padding pair) reads row 0: its outputs are never stored.
@@ -1622,7 +1737,7 @@ __global__ __launch_bounds__(256) void int4_gemm_grouped16_kernel(Int4GroupedArg
     if (row0 >= ga.total_post_pad[0]) return;
     int e = ga.block_expert[blockIdx.y];
     e = e < 0 ? 0 : (e >= ga.num_experts ? ga.num_experts - 1 : e);
-    const char *packed = static_cast<const char *>(ga.table[e]);
+    const char *packed = i4_expert(ga.table[e]);
     if (!packed) return;   // expert held by another rank
     if (tid < 64) {
         const int p = tid < 16 ? ga.sorted[row0 + tid] : -1;
@@ -1649,7 +1764,7 @@ __global__ __launch_bounds__(256) void int4_gemm_grouped16_kernel(Int4GroupedArg
 // passes ahead of 16 rows held three).  Or CT = 4 column tiles make a workgroup's stream longer.  A block of more than ROWS rows takes another pass over its
 // weights.  Mixtral-8x7B, gate|up 4096 x 28672 and down 14336 x 4096 of the 7 experts that 8 rows hit (420 and 210 MB), us: 113 + 62 before, 88 + 49.5
 // with <2, 8> (4.8 TB/s), 86 + 49 with <4, 8> (not kept: one more form), 91 + 51 with <4, 8> three passes ahead.
-// Decode steps of four layers, before / now: 6 rows 680 / 593, 8 rows 818 / 706, 12 rows 847 / 742, 16 rows 860 / 752.
+// Decode steps of four layers, before / now (flat loads still on both sides, see i4_expert): 6 rows 680 / 593, 8 rows 818 / 706, 12 rows 847 / 742, 16 rows 860 / 752.
 template <int UPW, bool GLU, int CT, int ROWS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ROWS == 8 ? 5 : CT == 4 ? 2 : 3, ROWS == 8 ? 7 : CT == 4 ? 3 : 5))) void int4_gemm_grouped16_ring_kernel(
     const void *const *__restrict__ table, const int32_t *__restrict__ sorted, const int32_t *__restrict__ block_expert,
@@ -1662,7 +1777,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ROWS == 8 ?
     if (row0 >= total_post_pad[0]) return;
     const int p = sorted[row0 + (tid & 15)];
     e = e < 0 ? 0 : (e >= num_experts ? num_experts - 1 : e);
-    const char *packed = static_cast<const char *>(table[e]);
+    const char *packed = i4_expert(table[e]);
     if (!packed) return;   // expert held by another rank
     const bool valid = p >= 0 && p < numel;
     if (tid < 16) omap[tid] = valid ? p : 0;                               // read behind the barriers of the sums
@@ -1689,7 +1804,7 @@ __global__ __launch_bounds__(256) void int4_gemm_grouped_kernel(const void *cons
     const int p = blockIdx.y;
     int e = expert_ids[p];
     e = e < 0 ? 0 : (e >= num_experts ? num_experts - 1 : e);  // ids come from top-k over num_experts
-    const char *packed = static_cast<const char *>(packed_table[e]);
+    const char *packed = i4_expert(packed_table[e]);
     if (!packed) return;   // expert held by another rank (expert parallelism): the combine step skips this pair
     const uint4 *W = reinterpret_cast<const uint4 *>(packed);
     const uint32_t *SZ = reinterpret_cast<const uint32_t *>(packed + sz_offset_bytes(K, N));
@@ -1706,7 +1821,7 @@ __global__ __launch_bounds__(256) void int4_gemm_grouped_glu_kernel(const void *
     const int p = blockIdx.y;
     int e = expert_ids[p];
     e = e < 0 ? 0 : (e >= num_experts ? num_experts - 1 : e);
-    const char *packed = static_cast<const char *>(packed_table[e]);
+    const char *packed = i4_expert(packed_table[e]);
     if (!packed) return;
     const uint4 *W = reinterpret_cast<const uint4 *>(packed);
     const uint32_t *SZ = reinterpret_cast<const uint32_t *>(packed + sz_offset_bytes(K, N));
