@@ -280,18 +280,20 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(const DeltaArgs a
 // that is not a bf16 enters a product as the sum of three bf16 parts (24 bits), so the memory, the weighted scores and the weighted
 // values keep f32 precision.  L is summed in double (a chunk may cross decays of e^-80, whose differences still count).
 // Wave w takes tokens 16 w .. 16 w + 15 of the first two products and rows w, w + 4, ... of 16 of the memory in the last.
+// What bounds it is the chain of chunks (5.5 us each: three barriers, products that wait for one another), so a compute unit should hold two workgroups: the scores
+// stay in registers, without 27 KB of LDS (90 KB in all, one workgroup) and their way through it.  16 heads of 128 x 128, three sequences, us a launch before / now:
+// 1500 tokens 90 / 62.5 (90: two rounds of workgroups), 300 tokens 28.7 / 18.8, 2000 tokens 112.5 / 76.5.
 constexpr int MC_C = 64, MC_LD = MC_C + 8;
 
 struct MemoryChunkLds {   // offsets in bytes
-    int q, k, p, v, wv, s, gates, total, dp, ldq, ldk;
+    int q, k, v, wv, s, gates, total, dp, ldq, ldk;
 };
 __host__ __device__ constexpr MemoryChunkLds memory_chunk_lds(int dt) {
     MemoryChunkLds l{};
     l.dp = 16 * dt, l.ldq = l.dp + 8, l.ldk = l.dp + 32;
     l.q = 0;
     l.k = l.q + MC_C * l.ldq * 2;
-    l.p = l.k + MC_C * l.ldk * 2;
-    l.v = l.p + 3 * MC_C * MC_LD * 2;
+    l.v = l.k + MC_C * l.ldk * 2;
     l.wv = l.v + 16 * MC_LD * 2;
     l.s = l.wv + 3 * 16 * MC_LD * 2;
     l.gates = l.s + 3 * 16 * l.ldq * 2;
@@ -316,7 +318,7 @@ template <int DT> __global__ __launch_bounds__(256) void memory_chunk_kernel(con
     constexpr MemoryChunkLds l = memory_chunk_lds(DT);
     constexpr int DP = l.dp, NQ = MC_C * DP / 4 / 256, ST = DT / 4, KS = DP / 32;
     extern __shared__ __align__(16) unsigned char mc_lds[];
-    uint16_t *Q = (uint16_t *)(mc_lds + l.q), *K = (uint16_t *)(mc_lds + l.k), *P = (uint16_t *)(mc_lds + l.p), *V = (uint16_t *)(mc_lds + l.v),
+    uint16_t *Q = (uint16_t *)(mc_lds + l.q), *K = (uint16_t *)(mc_lds + l.k), *V = (uint16_t *)(mc_lds + l.v),
              *WV = (uint16_t *)(mc_lds + l.wv), *SS = (uint16_t *)(mc_lds + l.s);
     double *gl = (double *)(mc_lds + l.gates);                    // [2][C] L
     float *ga = (float *)(gl + 2 * MC_C), *gw = ga + 2 * MC_C, *gc = gw + 2 * MC_C, *gt = gc + 2 * MC_C;   // [2][C] a, a e^(L_C - L), e^L; [2] e^(L_C)
@@ -412,7 +414,6 @@ template <int DT> __global__ __launch_bounds__(256) void memory_chunk_kernel(con
         S[j] = vmx_f32x4{f.x, f.y, f.z, f.w};
     }
     split_memory();
-    for (int i = tid; i < 3 * MC_C * MC_LD / 4; i += 256) reinterpret_cast<uint2 *>(P)[i] = make_uint2(0, 0);   // scores after the diagonal block stay 0
     stage();
     if (wave == 0) {
         scan_gates(0);
@@ -437,30 +438,10 @@ template <int DT> __global__ __launch_bounds__(256) void memory_chunk_kernel(con
                 for (int i = 0; i < 3; i++) WV[(i * 16 + vc + e) * MC_LD + vt] = p[i];
             }
         }
-        // scores of this wave's tokens against the chunk's keys up to them, weighted, in three parts
+        // o = e^L q . S (the memory ahead of the chunk) + weighted scores . v
         uint4 qf[KS];
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const uint4 *>(Q + (16 * wave + fl) * l.ldq + 32 * ks + 8 * fg);
-        double Lt[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) Lt[r] = gl[b * MC_C + 16 * wave + 4 * fg + r];
-        for (int j = 0; j <= wave; j++) {
-            vmx_f32x4 sc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) sc = mc_mfma(qf[ks], *reinterpret_cast<const uint4 *>(K + (16 * j + fl) * l.ldk + 32 * ks + 8 * fg), sc);
-            const int sidx = 16 * j + fl;
-            const double Ls = gl[b * MC_C + sidx];
-            const float as = ga[b * MC_C + sidx] * a.q_mul;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int t = 16 * wave + 4 * fg + r;
-                uint16_t p[3];
-                mc_split(sidx <= t ? sc[r] * as * expf((float)(Lt[r] - Ls)) : 0.f, p);
-#pragma unroll
-                for (int i = 0; i < 3; i++) P[(i * MC_C + t) * MC_LD + sidx] = p[i];
-            }
-        }
-        // o = e^L q . S (the memory ahead of the chunk) + weighted scores . v
         vmx_f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 2; i >= 0; i--)
@@ -468,11 +449,26 @@ template <int DT> __global__ __launch_bounds__(256) void memory_chunk_kernel(con
             for (int ks = 0; ks < KS; ks++) o = mc_mfma(qf[ks], *reinterpret_cast<const uint4 *>(SS + (i * 16 + fl) * l.ldq + 32 * ks + 8 * fg), o);
 #pragma unroll
         for (int r = 0; r < 4; r++) o[r] *= gc[b * MC_C + 16 * wave + 4 * fg + r];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the wave's own rows of P
-        for (int ks = 0; ks < (wave >> 1) + 1; ks++) {
-            const uint4 vf = *reinterpret_cast<const uint4 *>(V + fl * MC_LD + 32 * ks + 8 * fg);
+        // Scores of this wave's tokens against the chunk's keys up to them, formed transposed: a lane has keys 16 j + 4 fg + r of token fl, weights them, and hands
+        // each of their three parts on as the left operand of the product with v, without a way through LDS
+        const double Lt = gl[b * MC_C + 16 * wave + fl];
+        for (int j = 0; j <= wave; j++) {
+            const double2 L0 = *reinterpret_cast<const double2 *>(gl + b * MC_C + 16 * j + 4 * fg), L1 = *reinterpret_cast<const double2 *>(gl + b * MC_C + 16 * j + 4 * fg + 2);
+            const float4 al = *reinterpret_cast<const float4 *>(ga + b * MC_C + 16 * j + 4 * fg);
+            const uint2 vf = *reinterpret_cast<const uint2 *>(V + fl * MC_LD + 16 * j + 4 * fg);
+            vmx_f32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 2; i >= 0; i--) o = mc_mfma(*reinterpret_cast<const uint4 *>(P + (i * MC_C + 16 * wave + fl) * MC_LD + 32 * ks + 8 * fg), vf, o);
+            for (int ks = 0; ks < KS; ks++) sc = mc_mfma(*reinterpret_cast<const uint4 *>(K + (16 * j + fl) * l.ldk + 32 * ks + 8 * fg), qf[ks], sc);
+            const double Ls[4] = {L0.x, L0.y, L1.x, L1.y};
+            const float as[4] = {al.x, al.y, al.z, al.w};
+            uint16_t p[4][3];
+#pragma unroll
+            for (int r = 0; r < 4; r++) mc_split(16 * j + 4 * fg + r <= 16 * wave + fl ? sc[r] * (as[r] * a.q_mul) * expf((float)(Lt - Ls[r])) : 0.f, p[r]);
+#pragma unroll
+            for (int i = 2; i >= 0; i--)
+                o = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                    __builtin_bit_cast(mc_s16x4, make_uint2((uint32_t)p[0][i] | ((uint32_t)p[1][i] << 16), (uint32_t)p[2][i] | ((uint32_t)p[3][i] << 16))),
+                    __builtin_bit_cast(mc_s16x4, vf), o, 0, 0, 0);
         }
         const int c = tile * DR_VT + fl;
 #pragma unroll
