@@ -4,7 +4,7 @@
 // Such a step is a chain of short launches over weights that are read once (Qwen3-0.6B: 4 .. 13 MB each), so what bounds it is the
 // latency of each link: the weights of a workgroup are requested before anything they wait for is computed, and no result is converted
 // by a launch of its own.  Qwen3-0.6B at one row, 128 tokens: 12 launches and 43 us a layer as norm, GEMV, widening, activation kernels;
-// 5 launches and 26 us now (q|k|v 4.2 us, attention 7.4, o 4.2, gate|up 5.8 = 2.2 TB/s, down 4.6); the whole step 1269 -> 795 us.
+// 5 launches and 22 us now; the whole step 1269 -> 673 us.
 #include "vmx_kernels.h"
 
 namespace {
@@ -67,26 +67,27 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
     constexpr bool STAGED = SRC == DD_NORM || SRC == DD_MERGE, NORM = SRC == DD_NORM || SRC == DD_NORM_REG;
     __shared__ float red[NW][64][4];
     __shared__ __align__(16) uint16_t rows_lds[STAGED ? DD_STAGE : 8];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & (CW - 1), part = (lane & 15) / CW, g = lane >> 4, nt = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & (CW - 1), part = (lane & 15) / CW, g = lane >> 4, nt = blockIdx.x;
     const int nblk = (K + DEEP - 1) / DEEP, row = min(c, p.M - 1);
-    const bool live = c < p.M;
     const uint16_t *wrow = p.W + (int64_t)(DST == DD_GLU ? (c < CW / 2 ? 0 : p.N / 2) + nt * (CW / 2) + (c & (CW / 2 - 1)) : nt * CW + c) * K;
     const int k0 = 128 * part + 8 * g;
+    // Requests lie behind no condition (where one ends the compiler waits as if they had not been made, or, if it differs between lanes, for each before the next):
+    // what lies past K reads the last values again and is cleared before the product, a wave without a block reads one place (a compute unit is bound by its requests as well: one in
+    // every lane's own row cost down at 16 rows 8.9 -> 10.9 us), rows past M repeat the last
+    // one and are not stored.  Of several rows everything that has to be normed and its statistic come ahead of the weights.
+    // Qwen3-0.6B, a step of 1 / 2 / 4 / 9 / 16 rows: 723 / 774 / 944 / 1147 / 1407 -> 673 / 757 / 890 / 1116 / 1345 us (16 rows' gate|up 9.2 -> 8.0, q|k|v 6.8 -> 6.0).
     dd_u32x4 w[DEPTH][4], xr[DEPTH][4], nr[DEPTH][SRC == DD_NORM_REG ? 4 : 1];
     auto load_w = [&](int b, dd_u32x4 (&d)[4]) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int k = DEEP * b + k0 + 32 * j;
-            d[j] = k < K ? __builtin_nontemporal_load(reinterpret_cast<const dd_u32x4 *>(wrow + k)) : dd_u32x4{0, 0, 0, 0};
-        }
+        for (int j = 0; j < 4; j++) d[j] = __builtin_nontemporal_load(reinterpret_cast<const dd_u32x4 *>(b < nblk ? wrow + min(DEEP * b + k0 + 32 * j, K - 8) : p.W));
     };
     auto load_rows = [&](int b, dd_u32x4 (&x)[4], dd_u32x4 (&n)[SRC == DD_NORM_REG ? 4 : 1]) {
         if constexpr (!STAGED) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int k = DEEP * b + k0 + 32 * j;
-                x[j] = live && k < K ? *reinterpret_cast<const dd_u32x4 *>(p.x + (int64_t)row * K + k) : dd_u32x4{0, 0, 0, 0};
-                if constexpr (SRC == DD_NORM_REG) n[j] = k < K ? *reinterpret_cast<const dd_u32x4 *>(p.norm_w + k) : dd_u32x4{0, 0, 0, 0};
+                const int k = min(DEEP * b + k0 + 32 * j, K - 8);
+                x[j] = *reinterpret_cast<const dd_u32x4 *>(b < nblk ? p.x + (int64_t)row * K + k : p.x);
+                if constexpr (SRC == DD_NORM_REG) n[j] = *reinterpret_cast<const dd_u32x4 *>(b < nblk ? p.norm_w + k : p.norm_w);
             }
         }
     };
@@ -94,8 +95,10 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
     const int chunks = STAGED ? p.M * (K / 8) : 0, chunk0 = min(tid, chunks - 1);
     float4 lo[4], hi[4];
     float most[4], total[4];
+    const float per_row = __builtin_amdgcn_rcpf((float)(K / 8));
+    auto row_of = [&](int i) { return (int)(((float)i + 0.5f) * per_row); };   // i / (K / 8): of at most DD_STAGE / 8 places and 16 rows, so far closer than half a place
     auto load_parts = [&](int i) {
-        const int m = i / (K / 8), k = (i - m * (K / 8)) * 8;
+        const int m = row_of(i), k = (i - m * (K / 8)) * 8;
         const int64_t at = ((int64_t)m * (K / p.head) + k / p.head) * p.P;
 #pragma unroll
         for (int q = 0; q < 4; q++) {   // partitions past P read the last one again; their weight is zero below
@@ -118,35 +121,50 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
         const float scale = 1.0f / (sum + 1e-6f);
 #pragma unroll
         for (int e = 0; e < 8; e++) f[e] *= scale;
-        const int m = i / (K / 8);
+        const int m = row_of(i);
         *reinterpret_cast<dd_u32x4 *>(&rows_lds[m * (K + 8) + (i - m * (K / 8)) * 8]) = dd_pack(f);
     };
 
     // DD_NORM: the wave's lanes share the tiles' sums of its rows out (lane % rows is the row, as it is for c)
-    const int rows = p.M <= 1 ? 1 : p.M <= 2 ? 2 : p.M <= 4 ? 4 : p.M <= 8 ? 8 : 16, quads = NORM ? p.tiles / 4 : 1;
+    const int row_bits = p.M <= 1 ? 0 : p.M <= 2 ? 1 : p.M <= 4 ? 2 : p.M <= 8 ? 3 : 4, rows = 1 << row_bits, quads = NORM ? p.tiles / 4 : 1;
     const float4 *tile = NORM ? reinterpret_cast<const float4 *>(p.ssq + (int64_t)min(lane & (rows - 1), p.M - 1) * p.tiles) : nullptr;
     float4 t0;
-    dd_u32x4 x0, n0;
-    if constexpr (NORM) t0 = tile[min(lane / rows, quads - 1)];
+    constexpr int HELD = 4;   // of several rows' chunks a thread requests ahead of the weights
+    dd_u32x4 xs[SRC == DD_NORM ? HELD : 1], ns[SRC == DD_NORM ? HELD : 1];
+    if constexpr (NORM) t0 = tile[min(lane >> row_bits, quads - 1)];
+    float4 tq[HELD];
     if constexpr (SRC == DD_NORM) {
-        x0 = *reinterpret_cast<const dd_u32x4 *>(p.x + (int64_t)chunk0 * 8);
-        n0 = *reinterpret_cast<const dd_u32x4 *>(p.norm_w + chunk0 % (K / 8) * 8);
+        auto request = [&](int u) {
+            const bool some = 64 * NW * u + 64 * wave < chunks;   // of the wave's
+            const int at = min(tid + 64 * NW * u, chunks - 1);
+            xs[u] = *reinterpret_cast<const dd_u32x4 *>(some ? p.x + (int64_t)at * 8 : p.x);
+            ns[u] = *reinterpret_cast<const dd_u32x4 *>(some ? p.norm_w + (at - row_of(at) * (K / 8)) * 8 : p.norm_w);
+        };
+        request(0);
+        if (p.M > 1) {   // six requests that one row has no use for cost it 0.4 us
+#pragma unroll
+            for (int u = 1; u < HELD; u++) tq[u] = tile[min((lane >> row_bits) + u * (64 >> row_bits), quads - 1)], request(u);
+        }
     }
     if constexpr (SRC == DD_MERGE) load_parts(chunk0);
-    // DD_RESID: the thread's value of the stream, asked for ahead of the weights as everything that is not theirs
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) load_rows(wave + d * NW, xr[d], nr[d]);
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) load_w(wave + d * NW, w[d]);
+    // DD_RESID: the thread's value of the stream, which the end waits for
     const int om = CW == 16 ? (tid >> 4) & 15 : (tid >> 2) & 3, on = tid & (CW - 1);
     const int64_t out_at = (int64_t)min(om, p.M - 1) * p.N + nt * CW + on;
     uint16_t hold = 0;
     if constexpr (DST == DD_RESID) hold = p.h[out_at];
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++)
-        if (wave + d * NW < nblk) load_rows(wave + d * NW, xr[d], nr[d]);
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++) load_w(wave + d * NW, w[d]);   // past the end of K: no request
     float inv = 0.f;
     if constexpr (NORM) {
-        float sq = lane / rows < quads ? (t0.x + t0.y) + (t0.z + t0.w) : 0.f;
-        for (int i = lane / rows + 64 / rows; i < quads; i += 64 / rows) {
+        float sq = lane >> row_bits < quads ? (t0.x + t0.y) + (t0.z + t0.w) : 0.f;
+        const bool held = SRC == DD_NORM && p.M > 1;
+        if (held) {
+#pragma unroll
+            for (int u = 1; u < HELD; u++) sq += (lane >> row_bits) + u * (64 >> row_bits) < quads ? (tq[u].x + tq[u].y) + (tq[u].z + tq[u].w) : 0.f;
+        }
+        for (int i = (lane >> row_bits) + (held ? HELD : 1) * (64 >> row_bits); i < quads; i += 64 >> row_bits) {
             const float4 v = tile[i];
             sq += (v.x + v.y) + (v.z + v.w);
         }
@@ -167,14 +185,20 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
         return dd_pack(f);
     };
     if constexpr (SRC == DD_NORM) {
-        for (int i = tid; i - lane < chunks; i += 64 * NW) {   // whole waves: the statistic of a row is held by the lane of its number
-            const int at = min(i, chunks - 1), m = at / (K / 8), k = (at - m * (K / 8)) * 8;
+        auto stage = [&](int i, dd_u32x4 x, dd_u32x4 n) {   // whole waves: the statistic of a row is held by the lane of its number
+            const int at = min(i, chunks - 1), m = row_of(at);
             const float by = __shfl(inv, m);
-            if (i != tid) {
-                x0 = *reinterpret_cast<const dd_u32x4 *>(p.x + (int64_t)at * 8);
-                n0 = *reinterpret_cast<const dd_u32x4 *>(p.norm_w + k);
-            }
-            if (i < chunks) *reinterpret_cast<dd_u32x4 *>(&rows_lds[m * (K + 8) + k]) = norm8(x0, n0, by);
+            if (i < chunks) *reinterpret_cast<dd_u32x4 *>(&rows_lds[m * (K + 8) + (at - m * (K / 8)) * 8]) = norm8(x, n, by);
+        };
+        if (64 * wave < chunks) stage(tid, xs[0], ns[0]);
+        if (p.M > 1) {
+#pragma unroll
+            for (int u = 1; u < HELD; u++)
+                if (64 * NW * u + 64 * wave < chunks) stage(tid + 64 * NW * u, xs[u], ns[u]);
+        }
+        for (int i = tid + 64 * NW * (p.M > 1 ? HELD : 1); i - lane < chunks; i += 64 * NW) {
+            const int at = min(i, chunks - 1), m = row_of(at);
+            stage(i, *reinterpret_cast<const dd_u32x4 *>(p.x + (int64_t)at * 8), *reinterpret_cast<const dd_u32x4 *>(p.norm_w + (at - m * (K / 8)) * 8));
         }
     }
     if constexpr (SRC == DD_MERGE) {
@@ -187,15 +211,15 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
     if constexpr (STAGED) __syncthreads();
     vmx_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     auto step = [&](int b, dd_u32x4 (&d)[4], dd_u32x4 (&x)[4], dd_u32x4 (&n)[SRC == DD_NORM_REG ? 4 : 1]) {
+        const bool past = DEEP * (b + 1) > K;   // the wave's
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            dd_u32x4 a = x[j];
+            const int k = DEEP * b + k0 + 32 * j;
+            dd_u32x4 a = x[j], v = d[j];
             if constexpr (SRC == DD_NORM_REG) a = norm8(a, n[j], inv);
-            else if constexpr (STAGED) {
-                const int k = DEEP * b + k0 + 32 * j;
-                a = live && k < K ? *reinterpret_cast<const dd_u32x4 *>(&rows_lds[row * (K + 8) + k]) : dd_u32x4{0, 0, 0, 0};
-            }
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, a), __builtin_bit_cast(vmx_bf16x8, d[j]), acc, 0, 0, 0);
+            else if constexpr (STAGED) a = *reinterpret_cast<const dd_u32x4 *>(&rows_lds[row * (K + 8) + min(k, K - 8)]);
+            if (past && k >= K) a = v = dd_u32x4{0, 0, 0, 0};
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, a), __builtin_bit_cast(vmx_bf16x8, v), acc, 0, 0, 0);
         }
         if (DEPTH > 1 && b + DEPTH * NW < nblk) {
             load_w(b + DEPTH * NW, d);
