@@ -400,70 +400,77 @@ __global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(co
 // and DEPTH blocks ahead, and the activation fragment at the same k from the (cache-resident) rows.  The waves' tiles are added in
 // wave order through LDS.
 // GluLinear: the sixteen columns are eight gate columns and the up columns that belong to them.
-template <int NW, int PARTS, int DEPTH, class P = VmxLinear>
-__global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const P p) {
+// What the first requests need comes as arguments of its own (in registers when a wave starts; `plain`: no row list, no blocks, one product).  Requests lie behind no
+// condition, or the compiler waits for each before the next (dense_decode.hip): what lies past K reads the last values again and is cleared before the product, a
+// wave without a block reads one place, rows that do not exist read row 0 and are not stored.  f32 rows (A32) are rounded to bf16 as they are multiplied.
+// 16 rows, us a launch before / now:  gate and up [12288, 2048] 16.5 / 15.9, [32000, 2048] 38.0 / 36.2, [11264, 2048] 16.9 / 15.6, [3664, 2048] 8.7 / 8.3, [2048, 6144] 13.1 /
+// 12.7, [2048, 2048] 6.5 / 5.8; a step of Larolorn's four layers with 1 / 4 / 16 rows 362 / 383 / 468 -> 354 / 371 / 453.
+template <int NW, int PARTS, int DEPTH, bool A32, class P = VmxLinear>
+__global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const uint16_t *W, const void *A, int M, int N, int K, int lda, int w_sn, int plain, const P p) {
     constexpr bool GLU = std::is_same<P, GluLinear>::value;
     static_assert(!GLU || PARTS == 1, "eight gate and eight up columns a workgroup");
-    constexpr int CW = 16 / PARTS, DEEP = 128 * PARTS;
+    constexpr int CW = 16 / PARTS, DEEP = 128 * PARTS, AV = A32 ? 2 : 1;   // 16-byte pieces that hold eight values of a row
     __shared__ float red[NW][64][4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fl = lane & 15, c = fl & (CW - 1), part = fl / CW, fg = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fl = lane & 15, c = fl & (CW - 1), part = fl / CW, fg = lane >> 4;
     const int m0 = blockIdx.y * 16, n0 = blockIdx.x * CW, z = blockIdx.z;
-    if (p.total_rows && m0 >= *p.total_rows) return;
-    const uint16_t *W = p.W + z * p.w_bs;
-    if (p.block_expert) W += (int64_t)p.block_expert[m0 / p.block_rows] * p.expert_stride;
-    const int wn = GLU ? (c < 8 ? 0 : p.N / 2) + min(n0 / 2 + (c & 7), p.N / 2 - 1) : min(n0 + c, p.N - 1);
-    const uint16_t *wrow = W + (int64_t)wn * p.w_sn;
-    const int64_t ar = linear_src_row(p, m0 + fl), a_at = z * p.a_bs + (ar < 0 ? 0 : ar) * p.lda;
-    const int nblk = (p.K + DEEP - 1) / DEEP;
-    tg_u32x4 w[DEPTH][4], a[DEPTH][PARTS][4];
+    int64_t ar = min(fl, M - 1), row_len = lda, col_len = w_sn;
+    if (!plain) {
+        if (p.total_rows && m0 >= *p.total_rows) return;
+        W += z * p.w_bs;
+        if (p.block_expert) W += (int64_t)p.block_expert[m0 / p.block_rows] * p.expert_stride;
+        A = (const char *)A + z * p.a_bs * (A32 ? 4 : 2);
+        ar = max(linear_src_row(p, m0 + fl), (int64_t)0), row_len = p.lda, col_len = p.w_sn;
+    }
+    const int wn = GLU ? (c < 8 ? 0 : N / 2) + min(n0 / 2 + (c & 7), N / 2 - 1) : min(n0 + c, N - 1);
+    const uint16_t *wrow = W + wn * col_len;
+    const char *arow = (const char *)A + ar * row_len * (A32 ? 4 : 2);
+    const int nblk = (K + DEEP - 1) / DEEP;
+    tg_u32x4 w[DEPTH][4], a[DEPTH][PARTS][4][AV];
     auto load_w = [&](int b, tg_u32x4 (&d)[4]) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int k = DEEP * b + 128 * part + 32 * j + 8 * fg;
-            d[j] = k < p.K ? *reinterpret_cast<const tg_u32x4 *>(wrow + k) : tg_u32x4{0, 0, 0, 0};
-        }
+        for (int j = 0; j < 4; j++) d[j] = *reinterpret_cast<const tg_u32x4 *>(b < nblk ? wrow + min(DEEP * b + 128 * part + 32 * j + 8 * fg, K - 8) : W);
     };
-    auto load_a = [&](int b, tg_u32x4 (&d)[PARTS][4]) {
+    auto load_a = [&](int b, tg_u32x4 (&d)[PARTS][4][AV]) {
 #pragma unroll
         for (int q = 0; q < PARTS; q++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int k = DEEP * b + 128 * q + 32 * j + 8 * fg;
-                tg_u32x4 v = {0, 0, 0, 0};
-                if (ar >= 0 && k < p.K) {
-                    if (p.a_f32) {
-                        const float *src = (const float *)p.A + a_at + k;
-                        const float4 f0 = *reinterpret_cast<const float4 *>(src), f1 = *reinterpret_cast<const float4 *>(src + 4);
-                        const float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
-                        v = __builtin_bit_cast(tg_u32x4, vmx_pack16x8<false>(f));
-                    } else {
-                        v = *reinterpret_cast<const tg_u32x4 *>((const uint16_t *)p.A + a_at + k);
-                    }
-                }
-                d[q][j] = v;
-            }
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int e = 0; e < AV; e++)
+                    d[q][j][e] = *reinterpret_cast<const tg_u32x4 *>(b < nblk ? arow + min(DEEP * b + 128 * q + 32 * j + 8 * fg, K - 8) * (A32 ? 4 : 2) + 16 * e : (const char *)A);
     };
     vmx_f32x4 acc[PARTS];
 #pragma unroll
     for (int q = 0; q < PARTS; q++) acc[q] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
-    auto step = [&](int b, tg_u32x4 (&wv)[4], tg_u32x4 (&av)[PARTS][4]) {
+    auto step = [&](int b, tg_u32x4 (&wv)[4], tg_u32x4 (&av)[PARTS][4][AV]) {
+        const bool past = DEEP * (b + 1) > K;   // the wave's
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < 4; j++) {
+            tg_u32x4 x = wv[j];
+            if (past && DEEP * b + 128 * part + 32 * j + 8 * fg >= K) x = tg_u32x4{0, 0, 0, 0};
 #pragma unroll
-            for (int q = 0; q < PARTS; q++)
-                acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, av[q][j]), __builtin_bit_cast(vmx_bf16x8, wv[j]),
-                                                                 acc[q], 0, 0, 0);
+            for (int q = 0; q < PARTS; q++) {
+                tg_u32x4 v = av[q][j][0];
+                if constexpr (A32) {
+                    const tg_u32x4 u = av[q][j][1];
+                    const float f[8] = {__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]),
+                                        __uint_as_float(u[0]), __uint_as_float(u[1]), __uint_as_float(u[2]), __uint_as_float(u[3])};
+                    v = __builtin_bit_cast(tg_u32x4, vmx_pack16x8<false>(f));
+                }
+                if (past && DEEP * b + 128 * q + 32 * j + 8 * fg >= K) v = tg_u32x4{0, 0, 0, 0};
+                acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, v), __builtin_bit_cast(vmx_bf16x8, x), acc[q], 0, 0, 0);
+            }
+        }
         if (DEPTH > 1 && b + DEPTH * NW < nblk) {
             load_w(b + DEPTH * NW, wv);
             load_a(b + DEPTH * NW, av);
         }
     };
 #pragma unroll
-    for (int d = 0; d < DEPTH; d++)
-        if (wave + d * NW < nblk) {
-            load_w(wave + d * NW, w[d]);
-            load_a(wave + d * NW, a[d]);
-        }
+    for (int d = 0; d < DEPTH; d++) {
+        load_w(wave + d * NW, w[d]);
+        load_a(wave + d * NW, a[d]);
+    }
     if constexpr (DEPTH == 1) {   // one block a wave
         if (wave < nblk) step(wave, w[0], a[0]);
     } else {
@@ -504,7 +511,11 @@ __global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const P p) {
 template <int NW, int PARTS, int DEPTH, class P>
 void launch_skinny_as(const P &p, hipStream_t st) {
     constexpr int CW = 16 / PARTS;
-    hipLaunchKernelGGL((linear_skinny_kernel<NW, PARTS, DEPTH, P>), dim3((p.N + CW - 1) / CW, (p.M + 15) / 16, p.batch), dim3(64 * NW), 0, st, p);
+    const dim3 grid((p.N + CW - 1) / CW, (p.M + 15) / 16, p.batch);
+    const int64_t most = 0x7fffffff;
+    const int plain = p.M <= 16 && p.batch == 1 && !p.row_ids && !p.block_expert && !p.total_rows && p.lda >= 0 && p.lda <= most && p.w_sn >= 0 && p.w_sn <= most;
+    if (p.a_f32) hipLaunchKernelGGL((linear_skinny_kernel<NW, PARTS, DEPTH, true, P>), grid, dim3(64 * NW), 0, st, p.W, p.A, p.M, p.N, p.K, (int)p.lda, (int)p.w_sn, plain, p);
+    else hipLaunchKernelGGL((linear_skinny_kernel<NW, PARTS, DEPTH, false, P>), grid, dim3(64 * NW), 0, st, p.W, p.A, p.M, p.N, p.K, (int)p.lda, (int)p.w_sn, plain, p);
 }
 
 // What bounds these is the number of requests under way, so the split follows the number of 16-column groups (and K, never M: a row's
