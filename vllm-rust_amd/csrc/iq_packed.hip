@@ -29,6 +29,7 @@
 //   * a sign entry holds two v_perm selectors: signed activations = perm(-u, u, selector), then one v_dot4 per 4 weights
 //     (instead of xor / and / add on the codebook word, or two dot products).
 #include "iq_common.h"
+#include "tile_gemm.h"
 #include <stdlib.h>
 
 #ifndef VMX_IQ_AHEAD
@@ -152,12 +153,14 @@ template <int T> __global__ __launch_bounds__(256) void pk_build_tables_kernel()
 }
 
 // Request the workgroup's copy of the image: wave w takes the 1 KiB pieces w, w + W, ...; lane l of a piece brings 16 bytes.
-// Asynchronous (counted in vmcnt like any load); issued before the weight requests so that it completes first.
+// Issued before the weight requests so that it completes first, by an instruction that the compiler does not track (tg_request_1k): it took every later wait for a
+// wait for all that is under way, so the norms of the prologue began when the first weights had come from memory.  The caller waits for it (vmcnt 0).
+// With this, a layer scalar's load that no condition stands around and the hot parameters in registers, Gemma-4-12B at one row, us a launch before / now:
+// gate|up 16.3 / 15.0, q|k|v of a sliding layer 10.4 / 9.1; twelve layers 695 / 670.
 template <int T> __device__ __forceinline__ void pk_tables_request(unsigned char *smem, int wave, int W, int lane) {
     const unsigned char *img = pk_table_image<T>();
-    for (int c0 = wave * 64; c0 < PkTab<T>::BYTES / 16; c0 += W * 64)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(img + (c0 + lane) * 16),
-                                         (__attribute__((address_space(3))) void *)(smem + c0 * 16), 16, 0, 0);
+    const uint32_t at = tg_lds_at(smem);
+    for (int c0 = wave * 64; c0 < PkTab<T>::BYTES / 16; c0 += W * 64) tg_request_1k(at + c0 * 16, reinterpret_cast<const char *>(img) + c0 * 16, lane * 16);
 }
 
 // ------------------------------------------------------------------ part registers
@@ -329,13 +332,18 @@ struct PkArgs {
     uint16_t *glu_act;   // bf16 [inter]
     int8_t *glu_aq;      // its q8_1 form for the down projection
     float *glu_ad;
-    // sandwich-norm prologue (NORM = true): the activation row is computed by every workgroup from the previous linear's f32 output
-    // o and the residual stream h instead of being read as q8_1 (see pk_norm_prologue)
-    const float *n_o;
-    const uint16_t *n_h_in, *n_wpost, *n_wnext;
-    uint16_t *n_h_out;
+    uint16_t *n_h_out;   // norm prologue: where workgroup 0 stores the residual stream
     float n_eps;
-    const uint16_t *n_scalar;   // optional layer scalar: h' = bf16(h' * scalar) before the second norm
+    int n_scaled;        // there is a layer scalar
+};
+// Sandwich-norm prologue (NORM = true): the activation row is computed by every workgroup from the previous linear's f32 output o and the residual
+// stream h instead of being read as q8_1 (see pk_norm_prologue).  The kernel takes the five as its first parameters.
+struct PkNorm {
+    const float *o;
+    const uint16_t *h_in, *wpost, *wnext;
+    const uint16_t *scalar;   // optional layer scalar: h' = bf16(h' * scalar) before the second norm
+    uint16_t *h_out;
+    float eps;
 };
 
 __device__ __forceinline__ float pk_rbf(float x) { return vmx_bf16_to_f32(vmx_f32_to_bf16(x)); }
@@ -358,14 +366,14 @@ struct PkNormIn {
     uint16_t sc;
 };
 
-__device__ __forceinline__ void pk_norm_request(PkNormIn &r, const PkArgs &a, int n_in, int tid) {
+__device__ __forceinline__ void pk_norm_request(PkNormIn &r, const PkNorm &a, int n_in, int tid) {
     const int ci = min(tid, (n_in >> 3) - 1);
-    r.oa = *reinterpret_cast<const float4 *>(a.n_o + 8 * ci);
-    r.ob = *reinterpret_cast<const float4 *>(a.n_o + 8 * ci + 4);
-    r.h = *reinterpret_cast<const uint4 *>(a.n_h_in + 8 * ci);
-    r.wp = *reinterpret_cast<const uint4 *>(a.n_wpost + 8 * ci);
-    r.wn = *reinterpret_cast<const uint4 *>(a.n_wnext + 8 * ci);
-    r.sc = a.n_scalar ? a.n_scalar[0] : (uint16_t)0x3f80;
+    r.oa = *reinterpret_cast<const float4 *>(a.o + 8 * ci);
+    r.ob = *reinterpret_cast<const float4 *>(a.o + 8 * ci + 4);
+    r.h = *reinterpret_cast<const uint4 *>(a.h_in + 8 * ci);
+    r.wp = *reinterpret_cast<const uint4 *>(a.wpost + 8 * ci);
+    r.wn = *reinterpret_cast<const uint4 *>(a.wnext + 8 * ci);
+    r.sc = *a.scalar;   // wpost where there is none: not used then, but a condition around the load would wait for all of them
 }
 
 // Gemma's sandwich norms between o_proj and the MLP (gemma4_quantized.rs:1372-1392), with the bf16 rounding points of the
@@ -407,7 +415,7 @@ __device__ __forceinline__ void pk_norm_prologue(const PkNormIn &r, const PkArgs
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             hv[j] = pk_rbf(pk_rbf(ov[j] * inv1 * wv[j]) + hr[j]);
-            if (a.n_scalar) hv[j] = pk_rbf(hv[j] * vmx_bf16_to_f32(r.sc));   // layer_scalar of the layer whose tail this is
+            if (a.n_scaled) hv[j] = pk_rbf(hv[j] * vmx_bf16_to_f32(r.sc));   // layer_scalar of the layer whose tail this is
             v2 += live ? hv[j] * hv[j] : 0.f;
         }
         if (blockIdx.x == 0 && live) *reinterpret_cast<uint4 *>(a.n_h_out + 8 * tid) = pk_pack8(hv);
@@ -433,16 +441,16 @@ __device__ __forceinline__ void pk_norm_prologue(const PkNormIn &r, const PkArgs
 // of a row set sit in one workgroup and are combined through LDS in slice order).
 template <int T, int PPW, bool DBG, int ABL = 0, bool GLU = false, bool NORM = false>
 __device__ __forceinline__ void pk_body(unsigned char *smem, float *part, const PkSeg &sg, int wg, const int8_t *__restrict__ aq,
-                                        const float *__restrict__ ad, int n_in, int S, int32_t *__restrict__ dbg, int issue_barrier,
-                                        const PkArgs &na) {
+                                        const float *__restrict__ ad, int n_in, int S, int32_t *__restrict__ dbg, int W,
+                                        const PkArgs &na, const PkNorm &nm) {
     constexpr int TS = Pk<T>::TS, CPU_ = 4 / PPW, NR = 2 * PPW;   // chunks per unit, rows per item
 #ifndef VMX_IQ_AHEAD_NORM
 #define VMX_IQ_AHEAD_NORM VMX_IQ_AHEAD
 #endif
     // rows requested ahead of the one being decoded (NORM: the requests made before the prologue are all that is in flight during it)
     constexpr int AHEAD = NORM ? VMX_IQ_AHEAD_NORM : VMX_IQ_AHEAD;
-    const int tid = threadIdx.x, nthreads = blockDim.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), W = nthreads >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     unsigned long long ts[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // ABL == 3: shader-clock stamps of this wave
     auto stamp = [&](int i, float dep) {
         if constexpr (ABL == 3) asm volatile("s_memtime %0\n\ts_waitcnt lgkmcnt(0)" : "=s"(ts[i]) : "v"(dep) : "memory");
@@ -455,7 +463,7 @@ __device__ __forceinline__ void pk_body(unsigned char *smem, float *part, const 
     int8_t *aq_s = reinterpret_cast<int8_t *>(part) + 512;                 // [n_in] + 8 spare bytes
     float *ad_s = reinterpret_cast<float *>(aq_s + 4096 + 16);             // [n_in / 32]
     float *nred = ad_s + 128;                                              // [32]
-    if constexpr (NORM) pk_norm_request(nin, na, n_in, tid);
+    if constexpr (NORM) pk_norm_request(nin, nm, n_in, tid);
 #ifndef VMX_IQ_NOTAB
     pk_tables_request<T>(smem, wave, W, lane);
 #endif
@@ -604,26 +612,31 @@ __device__ __forceinline__ void pk_body(unsigned char *smem, float *part, const 
     }
 }
 
+// The first parameters, which arrive in registers, are what the first requests need: x0 / x1 are the q8_1 row and its scales, or with NORM o and h; geom =
+// waves | K-slices << 8 (one slice with GLU or NORM).  The segments are read at once and chosen from: an index into them was a chain of scalar loads.
 template <int PPW, bool DBG, int ABL = 0, bool GLU = false, bool NORM = false>
-__global__ __launch_bounds__(1024) void iq_pk_mmvq_kernel(PkArgs a, const int8_t *__restrict__ aq, const float *__restrict__ ad, int n_in,
-                                                           int S, int32_t *__restrict__ dbg, int lds_tables, int issue_barrier) {
+__global__ __launch_bounds__(1024) void iq_pk_mmvq_kernel(const void *__restrict__ x0, const void *__restrict__ x1, const uint16_t *n_wpost, const uint16_t *n_wnext,
+                                                           const uint16_t *n_scalar, int n_in, int geom, int lds_tables, PkArgs a, int32_t *__restrict__ dbg) {
     // the only LDS object of the kernel, so the tables start at LDS address 0 and a gather needs no base add
     extern __shared__ __align__(16) unsigned char pk_smem[];
-    const int b = blockIdx.x;
-    int si, wg;
+    const int b = blockIdx.x, W = GLU ? 16 : geom & 255, S = GLU || NORM ? 1 : geom >> 8;
+    PkSeg sg = a.seg[0];
+    int wg = b;
     if constexpr (GLU) {
-        si = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 9);   // wave-uniform: waves 8..15 work on the up projection
-        wg = b;
+        if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 9)) sg = a.seg[1];   // wave-uniform: waves 8..15 work on the up projection
     } else {
-        si = (a.nseg > 2 && b >= a.seg[2].wg0) ? 2 : ((a.nseg > 1 && b >= a.seg[1].wg0) ? 1 : 0);
-        wg = b - a.seg[si].wg0;
+        if (a.nseg > 1 && b >= a.seg[1].wg0) sg = a.seg[1];
+        if (a.nseg > 2 && b >= a.seg[2].wg0) sg = a.seg[2];
+        wg = b - sg.wg0;
     }
-    const PkSeg &sg = a.seg[si];
+    const PkNorm nm = {static_cast<const float *>(x0), static_cast<const uint16_t *>(x1), n_wpost, n_wnext, n_scalar, nullptr, 0.f};
+    const int8_t *aq = static_cast<const int8_t *>(x0);
+    const float *ad = static_cast<const float *>(x1);
     float *part = reinterpret_cast<float *>(pk_smem + lds_tables);   // [waves][8] slice sums (512 B) behind the tables, then the compact table copy
-    switch (GLU ? a.seg[0].type : sg.type) {   // workgroup-uniform (GLU: gate and up share a type)
-        case 18: pk_body<18, PPW, DBG, ABL, GLU, NORM>(pk_smem, part, sg, wg, aq, ad, n_in, S, dbg, issue_barrier, a); break;
-        case 21: pk_body<21, PPW, DBG, ABL, GLU, NORM>(pk_smem, part, sg, wg, aq, ad, n_in, S, dbg, issue_barrier, a); break;
-        default: pk_body<22, PPW, DBG, ABL, GLU, NORM>(pk_smem, part, sg, wg, aq, ad, n_in, S, dbg, issue_barrier, a); break;
+    switch (sg.type) {   // workgroup-uniform (GLU: gate and up share a type)
+        case 18: pk_body<18, PPW, DBG, ABL, GLU, NORM>(pk_smem, part, sg, wg, aq, ad, n_in, S, dbg, W, a, nm); break;
+        case 21: pk_body<21, PPW, DBG, ABL, GLU, NORM>(pk_smem, part, sg, wg, aq, ad, n_in, S, dbg, W, a, nm); break;
+        default: pk_body<22, PPW, DBG, ABL, GLU, NORM>(pk_smem, part, sg, wg, aq, ad, n_in, S, dbg, W, a, nm); break;
     }
     if constexpr (GLU) {
         // act = bf16(bf16(gelu_erf(bf16(gate))) * bf16(up)) and its q8_1 form (two 32-wide blocks), as g4_geglu_kernel computes them
@@ -649,8 +662,8 @@ __global__ __launch_bounds__(1024) void iq_pk_mmvq_kernel(PkArgs a, const int8_t
     }
 }
 
-template <int PPW, bool DBG, int ABL = 0, bool GLU = false, bool NORM = false> int pk_launch_ppw(const PkArgs &a, int wgs, int W, int lds, const int8_t *aq, const float *ad, int n_in, int S,
-                                               int32_t *dbg, hipStream_t st) {
+template <int PPW, bool DBG, int ABL = 0, bool GLU = false, bool NORM = false> int pk_launch_ppw(PkArgs a, int wgs, int W, int lds, const int8_t *aq, const float *ad, int n_in, int S,
+                                               int32_t *dbg, hipStream_t st, const PkNorm *norm = nullptr) {
     static bool attr_set = false;
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void *)iq_pk_mmvq_kernel<PPW, DBG, ABL, GLU, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072 + 512 + 8192);
@@ -660,8 +673,18 @@ template <int PPW, bool DBG, int ABL = 0, bool GLU = false, bool NORM = false> i
         }
         attr_set = true;
     }
-    static const int issue_barrier = vmx_tune("VMX_IQ_ISSUE_BARRIER", 1);
-    hipLaunchKernelGGL((iq_pk_mmvq_kernel<PPW, DBG, ABL, GLU, NORM>), dim3(wgs), dim3(64 * W), lds + 512 + 8192, st, a, aq, ad, n_in, S, dbg, lds, issue_barrier);
+    PkNorm nm = {};
+    const void *x0 = aq, *x1 = ad;
+    if constexpr (NORM) {
+        nm = *norm;
+        x0 = nm.o;
+        x1 = nm.h_in;
+        a.n_h_out = nm.h_out;
+        a.n_eps = nm.eps;
+        a.n_scaled = nm.scalar != nullptr;
+    }
+    hipLaunchKernelGGL((iq_pk_mmvq_kernel<PPW, DBG, ABL, GLU, NORM>), dim3(wgs), dim3(64 * W), lds + 512 + 8192, st, x0, x1, nm.wpost, nm.wnext,
+                       nm.scalar ? nm.scalar : nm.wpost, n_in, W | S << 8, lds, a, dbg);
     VMX_CHECK_LAUNCH("iq_mmvq(packed)");
     return VMX_OK;
 }
@@ -670,7 +693,7 @@ bool g_pk_tables_ready[64] = {};   // per device: the table images exist (vmx_in
 void *g_pk_stamps = nullptr;   // measurement: per-wave clock stamps of the next launches (vmx_debug_iq_packed_stamps)
 
 int pk_launch(const VmxMmvqSeg *segs, int nseg, const int8_t *aq, const float *ad, float *y, int n_in, int32_t *dbg, hipStream_t st,
-              const PkArgs *norm = nullptr) {
+              const PkNorm *norm = nullptr) {
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64 || !g_pk_tables_ready[dev]) {
         vmx_set_error("iq_mmvq(packed): vmx_init(%d) has not run on this device (it builds the decode tables)", dev);
@@ -714,11 +737,9 @@ int pk_launch(const VmxMmvqSeg *segs, int nseg, const int8_t *aq, const float *a
             vmx_set_error("iq_mmvq(packed, norm): %d-wave workgroups / %d K-slices cannot hold a row of %d", W, S, n_in);
             return VMX_EUNSUPPORTED;
         }
-        a.n_o = norm->n_o; a.n_h_in = norm->n_h_in; a.n_h_out = norm->n_h_out; a.n_wpost = norm->n_wpost; a.n_wnext = norm->n_wnext;
-        a.n_eps = norm->n_eps; a.n_scalar = norm->n_scalar;
-        if (ppw == 4) return pk_launch_ppw<4, false, 0, false, true>(a, wg, W, lds, nullptr, nullptr, n_in, S, nullptr, st);
-        if (ppw == 2) return pk_launch_ppw<2, false, 0, false, true>(a, wg, W, lds, nullptr, nullptr, n_in, S, nullptr, st);
-        return pk_launch_ppw<1, false, 0, false, true>(a, wg, W, lds, nullptr, nullptr, n_in, S, nullptr, st);
+        if (ppw == 4) return pk_launch_ppw<4, false, 0, false, true>(a, wg, W, lds, nullptr, nullptr, n_in, S, nullptr, st, norm);
+        if (ppw == 2) return pk_launch_ppw<2, false, 0, false, true>(a, wg, W, lds, nullptr, nullptr, n_in, S, nullptr, st, norm);
+        return pk_launch_ppw<1, false, 0, false, true>(a, wg, W, lds, nullptr, nullptr, n_in, S, nullptr, st, norm);
     }
     if (dbg) return pk_launch_ppw<4, true>(a, wg, W, lds, aq, ad, n_in, S, dbg, st);
     static const int abl = vmx_tune("VMX_IQ_ABL", 0);   // measurement only: 1 = stream alone, 2 = decode alone
@@ -862,13 +883,8 @@ int vmx_iq_mmvq_packed_norm_geglu(const VmxMmvqSeg *gate, const VmxMmvqSeg *up, 
     a.glu_act = act;
     a.glu_aq = aq_out;
     a.glu_ad = ad_out;
-    a.n_o = o;
-    a.n_h_in = h_in;
-    a.n_h_out = h_out;
-    a.n_wpost = w_post;
-    a.n_wnext = w_next;
-    a.n_eps = eps;
-    return pk_launch_ppw<4, false, 0, true, true>(a, gate->n_out / 64, 16, pk_lds_bytes(gate->ggml_type), nullptr, nullptr, n_in, 1, nullptr, st);
+    const PkNorm norm = {o, h_in, w_post, w_next, nullptr, h_out, eps};
+    return pk_launch_ppw<4, false, 0, true, true>(a, gate->n_out / 64, 16, pk_lds_bytes(gate->ggml_type), nullptr, nullptr, n_in, 1, nullptr, st, &norm);
 }
 
 bool vmx_iq_packed_norm_geglu_ok(const VmxMmvqSeg *gate, const VmxMmvqSeg *up, int n_in, int m) {
@@ -893,7 +909,7 @@ bool vmx_iq_packed_norm_multi_ok(const VmxMmvqSeg *segs, int nseg, int n_in, int
     const int ppw = units >= 2048 ? 4 : (units >= 1024 ? 2 : 1);
     int W = (units * (4 / ppw) + vmx_num_cus() - 1) / vmx_num_cus();
     W = W < 1 ? 1 : (W > 16 ? 16 : W);
-    // measured on the Gemma-4-12B shapes: with 8-wave workgroups (sliding layers, 1 024 units) the fused launch takes 9.9 us against
+    // measured on the Gemma-4-12B shapes: with 8-wave workgroups (sliding layers, 1 024 units) the fused launch takes 9.1 us against
     // 6.9 + 5.5 us for the raw-layout launch behind a norm kernel; the 9-wave plan of the full-attention layers (1 152 units, one
     // workgroup per compute unit) takes 18.1 us against 8.1 + 5.5 us in the kernel trace, so those keep the two launches (on the
     // whole step the two choices measured within noise of each other: 327-330 vs 328 tok/s)
@@ -907,9 +923,8 @@ int vmx_iq_mmvq_packed_norm_multi(const VmxMmvqSeg *segs, int nseg, const float 
         vmx_set_error("iq_mmvq(packed, norm): not eligible (n_in %d, %d tensors)", n_in, nseg);
         return VMX_EUNSUPPORTED;
     }
-    PkArgs na = {};
-    na.n_o = o; na.n_h_in = h_in; na.n_h_out = h_out; na.n_wpost = w_post; na.n_wnext = w_next; na.n_eps = eps; na.n_scalar = scalar;
-    return pk_launch(segs, nseg, nullptr, nullptr, y, n_in, nullptr, st, &na);
+    const PkNorm norm = {o, h_in, w_post, w_next, scalar, h_out, eps};
+    return pk_launch(segs, nseg, nullptr, nullptr, y, n_in, nullptr, st, &norm);
 }
 
 extern "C" int vmx_iq_mmvq_packed_geglu_bf16(int ggml_type, const void *gate_packed, const void *up_packed, const int8_t *aq, const float *ad,
