@@ -5,8 +5,9 @@
 // crates/core/src/layers/attention/backend.rs:60-71; semantics of naive.rs:38-83).  That kernel walks 16-token KV tiles with a
 // workgroup barrier and scalar LDS stores per tile and keeps the matrix cores ~1.5 % busy; this one is built for them:
 //
-//   workgroup = 4 or 8 waves; a wave owns 32 query rows of ONE query head (HPW heads of one KV head x NW / HPW blocks of
-//   32 query rows per workgroup: every wave of the workgroup shares every KV tile it fetches); 236 registers, two waves per SIMD;
+//   workgroup = 4 or 8 waves, or two groups of 4 that walk every other tile of the same keys for the same queries, in LDS of their own, and merge their
+//   sums at the end (few workgroups: the chain of tiles is what a launch takes); a wave owns 32 query rows of ONE query head (HPW heads of one KV head x NW / HPW blocks of
+//   32 query rows per workgroup: every wave of the workgroup shares every KV tile it fetches); up to 250 registers, two waves per SIMD;
 //   KV tiles of 64 tokens are fetched one tile ahead into registers (16-byte pieces, whole cache rows per wave access) and
 //   written to a two-stage LDS ring: one barrier per tile;
 //   S^T = K Q^T   v_mfma_f32_32x32x16: A = K rows from LDS (ds_read_b128; 16-byte chunk c of row r sits at chunk
@@ -23,6 +24,7 @@
 // once at the end; sums are f32.  Summation order differs (64-token tiles), within the attention tolerance of the tests.
 #include "vmx_kernels.h"
 
+#include <algorithm>
 #include <float.h>
 #include <type_traits>
 
@@ -45,23 +47,24 @@ template <int HD> __device__ __forceinline__ int pa_swz(int r) { return HD == 12
 
 // KV: 0 = bf16 cache and queries, 1 = FP8 e4m3 cache bytes (widened to bf16 on the way into LDS: exact) with bf16 queries,
 // 3 = fp16 cache and queries (fp16 forms of the matrix instructions, P rounded to fp16)
-template <int HD, int HPW, int KV, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_tiled_kernel(uint16_t *__restrict__ out, const uint16_t *__restrict__ q,
+template <int HD, int HPW, int KV, int NW, int NG>
+__global__ __launch_bounds__(64 * NW * NG) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_tiled_kernel(uint16_t *__restrict__ out, const uint16_t *__restrict__ q,
                                                                   const void *__restrict__ k_cache, const void *__restrict__ v_cache,
                                                                   const int32_t *__restrict__ block_table, int q_len, int offset, float scale,
                                                                   int num_heads, int num_kv_heads, int block_size, int window,
                                                                   const float *__restrict__ k_scale_ptr, const float *__restrict__ v_scale_ptr,
-                                                                  int head_groups) {
+                                                                  int head_groups, uint32_t bs_mul) {
     constexpr bool F16 = KV == 3;
     constexpr int TT = NW / HPW;                      // 32-row query blocks per workgroup
     constexpr int CH = HD / 8;                        // 16-byte chunks per row
-    constexpr int NT = 64 * NW;                       // threads
+    constexpr int NT = 64 * NW;                       // threads of a group
     constexpr int NLD = PA_KT * CH / NT;              // chunks per thread per tile and tensor
     constexpr int KS = HD / 16;                       // k-steps of S^T
     constexpr int DT = HD / 32;                       // 32-dim tiles of O^T
     constexpr int KROW = pa_krow<HD>(), VROW = pa_vrow<HD>(), STAGE = pa_stage<HD>();
     extern __shared__ __align__(16) unsigned char pa_smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int grp = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;   // which of the NG tiles of a step is this wave's
+    const int tid = threadIdx.x - grp * NT, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ql = lane & 31, hi = lane >> 5;
     const int hh = wave % HPW, tt = wave / HPW;
     const int nq = num_heads / num_kv_heads;
@@ -96,20 +99,35 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     lo &= ~(PA_KT - 1);
     const int ntiles = (hi_tok - lo + PA_KT - 1) / PA_KT;
     const int64_t tok_stride = (int64_t)num_kv_heads * HD;
-    const int bs_shift = (block_size & (block_size - 1)) == 0 ? __ffs(block_size) - 1 : -1;   // power-of-two blocks: no division per row
 
     // staging registers: chunk id = tid + 256 j -> (row, chunk); a wave access covers whole cache rows
     typedef typename std::conditional<KV == 1, uint2, uint4>::type raw_t;
     raw_t kst[NLD], vst[NLD];
-    auto issue = [&](int tile) {
-        const int t0 = lo + tile * PA_KT;
+    // The block-table entries of a tile are read a tile before its rows, and without a branch: read with the rows, and with a condition between the ways to
+    // divide by the block size, a thread's four rows were four chains of two trips to memory a tile.  32 heads over 8, 128 wide, one group, before / now, us:
+    // 256 tokens 12.8 / 11.0, 1024 35.5 / 29.1, 2048 75.1 / 58.1; 16 behind 2000 62.2 / 47.9.
+    int blk[NLD];
+    // token of chunk j's row in a tile: past the end the last valid one (their weights are 0); its block and its place in it
+    auto place = [&](int tile, int j, int &bi, int &in) {
+        const int t = min(lo + tile * PA_KT + (tid + NT * j) / CH, hi_tok - 1);
+        bi = (int)__umulhi((uint32_t)t, bs_mul);   // t / block_size or one less: t (2^32 / block_size - bs_mul) < t < 2^31
+        in = t - bi * block_size;
+        if (in >= block_size) in -= block_size, bi++;
+    };
+    auto lookup = [&](int tile) {
 #pragma unroll
         for (int j = 0; j < NLD; j++) {
-            const int id = tid + NT * j, row = id / CH, ch = id % CH;
-            const int t = min(t0 + row, hi_tok - 1);   // rows past the end repeat the last valid row (their weights are 0)
-            const int bi = bs_shift >= 0 ? t >> bs_shift : t / block_size;
-            const int blk = block_table[bi];
-            const int64_t base = ((int64_t)blk * block_size + (t - bi * block_size)) * tok_stride + (int64_t)kvh * HD + ch * 8;
+            int bi, in;
+            place(tile, j, bi, in);
+            blk[j] = block_table[bi];
+        }
+    };
+    auto issue = [&](int tile) {
+#pragma unroll
+        for (int j = 0; j < NLD; j++) {
+            int bi, in;
+            place(tile, j, bi, in);
+            const int64_t base = ((int64_t)blk[j] * block_size + in) * tok_stride + (int64_t)kvh * HD + (tid + NT * j) % CH * 8;
             if constexpr (KV == 1) {
                 kst[j] = *reinterpret_cast<const uint2 *>((const uint8_t *)k_cache + base);
                 vst[j] = *reinterpret_cast<const uint2 *>((const uint8_t *)v_cache + base);
@@ -135,7 +153,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
         }
     };
     auto commit = [&](int buf) {
-        unsigned char *kb = pa_smem + buf * STAGE, *vb = kb + PA_KT * KROW;
+        unsigned char *kb = pa_smem + (2 * grp + buf) * STAGE, *vb = kb + PA_KT * KROW;
 #pragma unroll
         for (int j = 0; j < NLD; j++) {
             const int id = tid + NT * j, row = id / CH, ch = id % CH;
@@ -156,17 +174,23 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     const int li = lane & 15, g16 = (lane >> 4) & 1;
     const int vtr_off = (4 * hi + (li >> 2)) * VROW + (16 * g16 + 4 * (li & 3)) * 2;   // + (32 u + 16 ks + 8 h) VROW + 64 dt
 
-    issue(0);
+    const int nsteps = (ntiles + NG - 1) / NG;
+    lookup(grp);   // a tile that there is not takes the last row's block
+    issue(grp);
+    lookup(grp + NG);
     commit(0);
     __syncthreads();
-    for (int tile = 0; tile < ntiles; tile++) {
-        const int t0 = lo + tile * PA_KT;
-        const bool more = tile + 1 < ntiles;
-        if (more) issue(tile + 1);
+    for (int step = 0; step < nsteps; step++) {
+        const int tile = step * NG + grp, t0 = lo + tile * PA_KT;
+        const bool more = tile + NG < ntiles;
+        if (more) {
+            issue(tile + NG);
+            lookup(tile + 2 * NG);
+        }
         // does this tile intersect the wave's causal / window range at all (wave-uniform)
-        const bool need = wave_live && t0 <= qpos_max && (window <= 0 || t0 + PA_KT - 1 > qpos_min - window);
+        const bool need = wave_live && (NG == 1 || tile < ntiles) && t0 <= qpos_max && (window <= 0 || t0 + PA_KT - 1 > qpos_min - window);
         if (__builtin_amdgcn_readfirstlane(need ? 1 : 0)) {
-            const unsigned char *kb = pa_smem + (tile & 1) * STAGE, *vb = kb + PA_KT * KROW;
+            const unsigned char *kb = pa_smem + (2 * grp + (step & 1)) * STAGE, *vb = kb + PA_KT * KROW;
             pa_f32x16 s[2];
 #pragma unroll
             for (int u = 0; u < 2; u++) {
@@ -249,8 +273,29 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
                     }
                 }
         }
-        if (more) commit((tile + 1) & 1);
+        if (more) commit((step + 1) & 1);
         __syncthreads();
+    }
+    if constexpr (NG > 1) {   // the groups' sums meet in LDS (the tiles are done with: the loop ended with a barrier): [wave][number][lane] f32
+        constexpr int NN = 16 * DT + 2;
+        float *at = reinterpret_cast<float *>(pa_smem) + wave * NN * 64 + lane;
+        static_assert(NG == 2 && NW * NN * 256 <= NG * 2 * STAGE, "the other group's sums fit the tiles' place");
+        if (grp == 1) {
+            at[0] = m_run;
+            at[64] = l_run;
+#pragma unroll
+            for (int d = 0; d < DT; d++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) at[64 * (2 + 16 * d + r)] = acc[d][r];
+        }
+        __syncthreads();
+        if (grp == 1) return;
+        const float m1 = at[0], m = fmaxf(m_run, m1), a0 = __builtin_amdgcn_exp2f(m_run - m), a1 = __builtin_amdgcn_exp2f(m1 - m);
+        l_run = l_run * a0 + at[64] * a1;
+#pragma unroll
+        for (int d = 0; d < DT; d++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[d][r] = acc[d][r] * a0 + at[64 * (2 + 16 * d + r)] * a1;
     }
     const float l = l_run + vmx_lane_xor<32>(l_run);
     if (wave_live && qi < q_len) {
@@ -267,17 +312,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     }
 }
 
-template <int HD, int HPW, int KV, int NW>
+template <int HD, int HPW, int KV, int NW, int NG>
 int launch_tiled(hipStream_t st, uint16_t *out, const uint16_t *q, const void *kc, const void *vc, const int32_t *bt, int q_len, int offset,
                  float scale, int H, int KVH, int bs, int window, const float *ks, const float *vs) {
     constexpr int TT = NW / HPW;
     const int nq = H / KVH, groups = (nq + HPW - 1) / HPW;
     const dim3 grid(((q_len + 32 * TT - 1) / (32 * TT)) * KVH * groups);
-    const size_t lds = 2 * (size_t)pa_stage<HD>();
+    const size_t lds = 2 * NG * (size_t)pa_stage<HD>();
     if (lds > 64 * 1024)
-        VMX_CHECK_HIP(hipFuncSetAttribute((const void *)prefill_attn_tiled_kernel<HD, HPW, KV, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((prefill_attn_tiled_kernel<HD, HPW, KV, NW>), grid, dim3(64 * NW), lds, st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH,
-                       bs, window, ks, vs, groups);
+        VMX_CHECK_HIP(hipFuncSetAttribute((const void *)prefill_attn_tiled_kernel<HD, HPW, KV, NW, NG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((prefill_attn_tiled_kernel<HD, HPW, KV, NW, NG>), grid, dim3(64 * NW * NG), lds, st, out, q, kc, vc, bt, q_len, offset, scale, H, KVH,
+                       bs, window, ks, vs, groups, bs == 1 ? 0xFFFFFFFFu : (uint32_t)((1ull << 32) / bs));
     VMX_CHECK_LAUNCH("prefill_attention(32x32 tiles)");
     return VMX_OK;
 }
@@ -298,7 +343,16 @@ int vmx_prefill_attention_tiled(uint16_t *out, const uint16_t *q, const void *k_
     static const int nw_env = vmx_tune("VMX_PREFILL_NW", 0);
     const int64_t wg8 = (int64_t)((q_len + 32 * (8 / hpw) - 1) / (32 * (8 / hpw))) * num_kv_heads * ((nq + hpw - 1) / hpw);
     const bool eight = nw_env ? nw_env == 8 : wg8 >= 2 * vmx_num_cus();
-#define PA_NW(HD, HPW, KVT) return eight ? launch_tiled<HD, HPW, KVT, 8>(PA_ARGS) : launch_tiled<HD, HPW, KVT, 4>(PA_ARGS)
+    // Two groups of four waves share the keys of a workgroup while the workgroups are few (a unit holds one such workgroup, or two of one group) and the longest
+    // chain is six tiles or more; with a shorter one the merge costs what the halved chain gives.  us, one group / two, bf16, no history unless said, tokens
+    // 200 / 256 / 333 / 512 / 1024 / 2048 / 4096: 32 heads over 8, 128 wide 9.6 11.0 12.8 17.1 29.1 58.1 169 / 10.4 11.4 12.9 16.5 26.8 55.3 178 (512 workgroups at 2048);
+    // 8 over 8 10.2 11.1 13.1 17.1 28.5 51.6 98 / 9.6 10.9 11.8 15.4 24.4 41.7 78; 16 over 4, 64 wide 7.2 8.1 9.3 12.1 20.7 37.6 78 / 7.2 7.8 8.7 10.6 16.9 29.1 62;
+    // 16 tokens behind 2000: 47.9 / 40.0; 64 heads over 8, 1024 tokens, window 256 (512 workgroups, chains of 5 tiles) 22.0 / 26.7.
+    const int64_t wg4 = (int64_t)((q_len + 32 * (4 / hpw) - 1) / (32 * (4 / hpw))) * num_kv_heads * ((nq + hpw - 1) / hpw);
+    const int64_t chain = std::min<int64_t>((int64_t)seqlen_offset + q_len, window > 0 ? (int64_t)window + 32 * (4 / hpw) : INT64_MAX);
+    const bool two = nw_env ? nw_env == 2 : wg4 <= 2 * vmx_num_cus() && chain > 5 * PA_KT;
+#define PA_NW(HD, HPW, KVT) return eight ? launch_tiled<HD, HPW, KVT, 8, 1>(PA_ARGS) \
+                                  : two ? launch_tiled<HD, HPW, KVT, 4, 2>(PA_ARGS) : launch_tiled<HD, HPW, KVT, 4, 1>(PA_ARGS)
 #define PA_KV(HD, HPW)                    \
     if (kv == 3) { PA_NW(HD, HPW, 3); }   \
     if (kv == 1) { PA_NW(HD, HPW, 1); }   \
