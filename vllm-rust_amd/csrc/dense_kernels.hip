@@ -80,57 +80,70 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(uint16_t *__restrict__ 
 // A fragment of step j is read from LDS at the matching k (x[m][128 b + 32 g + 8 j .. + 8]): the matrix instruction only needs
 // A and B to agree on which k sits where.  Activations are staged PK = 1024 k at a time (33 KB at 16 rows).  f32 accumulation
 // in k order within a lane group, groups summed by the MFMA: re-associated against the kernel above, same products.
-template <bool F16>
-__global__ __launch_bounds__(256) void dense_gemm16_kernel(uint16_t *__restrict__ y, const uint16_t *__restrict__ x,
+// A pass's activations are requested while the one before it is multiplied and the weights two blocks ahead, all behind no condition (rows and k that there are not
+// read others' words; behind the last pass every lane reads one place): a thread's eight pieces of a pass were eight trips, one after another:
+// 8 rows, 4000 x 4096 on 63 workgroups 32.4 -> 21.0 us; 16 rows, 38000 x 4096 on 594, the stream's time, 76.6 -> 77.  With non-temporal weight loads a step of 672 us took 717 (a lane's 64 bytes are four loads).
+// TAIL: K is no multiple of 1024 (of 128 it is); the last pass's blocks past K are zeros times zeros.
+template <bool F16, bool TAIL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void dense_gemm16_kernel(uint16_t *__restrict__ y, const uint16_t *__restrict__ x,
                                                             const uint16_t *__restrict__ W, const uint16_t *__restrict__ bias, int M,
                                                             int N, int K) {
     constexpr int PK = 1024, XROW = PK + 8;   // k per pass; staged row stride (+16 B against bank conflicts)
     __shared__ __align__(16) uint16_t xs[16 * XROW];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nl = lane & 15, g = lane >> 4;
     const int tiles = (N + 15) >> 4;
     const int waves_total = gridDim.x * 4;
     // every wave of the workgroup walks the same number of tiles (barriers inside): tiles past the end are clamped, not stored
     const int rounds = (tiles + waves_total - 1) / waves_total;
+    const int nblk = K >> 7, passes = (nblk + 7) >> 3;
+    // piece i of a pass: row 2 i + tid / 128, elements 8 (tid % 128) ..
+    uint4 st[8];
+    auto request = [&](int pass, bool real) {
+        const int k = min(pass * PK + 8 * (tid & 127), K - 8);
+#pragma unroll
+        for (int i = 0; i < 8; i++) st[i] = *reinterpret_cast<const uint4 *>(x + (real ? (int64_t)min(2 * i + (tid >> 7), M - 1) * K + k : (int64_t)0));
+    };
+    request(0, true);
     for (int rd = 0; rd < rounds; rd++) {
         const int tile = rd * waves_total + blockIdx.x * 4 + wave;
         const int row = min(tile * 16 + nl, N - 1);
-        const uint16_t *wrow = W + (int64_t)row * K;
+        const uint16_t *wrow = W + (int64_t)row * K + 32 * g;
         vmx_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        // the weights of 128-deep block i + 1 are requested before block i is multiplied: with load and use in the same iteration
-        // a wave has one block (4 KB) in flight and the launch runs at the memory latency, not the memory rate
-        const int nblk = K >> 7;
-        uint4 wn[4];
+        uint4 w[2][4];
+        auto weights = [&](int slot, int blk) {
+            const uint16_t *at = blk < nblk ? wrow + blk * 128 : W;
 #pragma unroll
-        for (int j = 0; j < 4; j++) wn[j] = *reinterpret_cast<const uint4 *>(wrow + 32 * g + 8 * j);
-        for (int blk = 0; blk < nblk; blk++) {
-            const int k0 = (blk >> 3) * PK, b = (blk & 7) * 128;
-            if ((blk & 7) == 0) {
-                const int pk = min(PK, K - k0);   // K % 128 == 0 (checked on the host)
-                if (blk || rd) __syncthreads();   // the previous pass has been read by every wave
-                for (int c = tid; c < 16 * (PK / 8); c += 256) {
-                    const int m = c / (PK / 8), cc = c % (PK / 8);
-                    uint4 v = make_uint4(0, 0, 0, 0);
-                    if (m < M && cc * 8 < pk) v = *reinterpret_cast<const uint4 *>(x + (int64_t)m * K + k0 + cc * 8);
-                    *reinterpret_cast<uint4 *>(xs + m * XROW + cc * 8) = v;
+            for (int j = 0; j < 4; j++) w[slot][j] = *reinterpret_cast<const uint4 *>(at + 8 * j);
+        };
+        weights(0, 0);
+        weights(1, 1);
+        for (int pass = 0; pass < passes; pass++) {
+            if (pass || rd) __syncthreads();   // the previous pass has been read by every wave
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const bool in = !TAIL || pass * PK + 8 * (tid & 127) < K;
+                const uint4 v = make_uint4(in ? st[i].x : 0, in ? st[i].y : 0, in ? st[i].z : 0, in ? st[i].w : 0);
+                *reinterpret_cast<uint4 *>(xs + (2 * i + (tid >> 7)) * XROW + 8 * (tid & 127)) = v;
+            }
+            __syncthreads();
+            const bool last = pass + 1 == passes;
+            request(last ? 0 : pass + 1, !last || rd + 1 < rounds);
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                const int blk = pass * 8 + b;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint4 au = *reinterpret_cast<const uint4 *>(xs + nl * XROW + b * 128 + 32 * g + 8 * j);
+                    uint4 wv = w[b & 1][j];
+                    if (TAIL && blk >= nblk) wv = make_uint4(0, 0, 0, 0);
+                    if constexpr (F16)
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, au), __builtin_bit_cast(f16x8_t, wv), acc, 0, 0, 0);
+                    else
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, au), __builtin_bit_cast(vmx_bf16x8, wv), acc, 0, 0, 0);
                 }
-                __syncthreads();
-            }
-            uint4 wv[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) wv[j] = wn[j];
-            if (blk + 1 < nblk) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) wn[j] = *reinterpret_cast<const uint4 *>(wrow + (blk + 1) * 128 + 32 * g + 8 * j);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint4 au = *reinterpret_cast<const uint4 *>(xs + nl * XROW + b + 32 * g + 8 * j);
-                if constexpr (F16)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, au), __builtin_bit_cast(f16x8_t, wv[j]), acc, 0, 0, 0);
-                else
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, au), __builtin_bit_cast(vmx_bf16x8, wv[j]), acc,
-                                                                  0, 0, 0);
+                weights(b & 1, blk + 2);
+                __builtin_amdgcn_sched_barrier(0);   // or the last two of a pass are requested behind it
             }
         }
         // lane holds activation rows m = 4 g + r of output column (W row) tile * 16 + nl
@@ -210,7 +223,8 @@ static int dense_gemv_launch_t(uint16_t *y, const uint16_t *x, const uint16_t *W
     if (mfma_min_m > 0 && M >= mfma_min_m && K % 128 == 0) {   // GEMM-shaped: matrix cores, activations staged in k-passes
         int g16 = ((N + 15) / 16 + 3) / 4;   // 4 waves x one 16-row tile of W per round
         if (g16 > 4096) g16 = 4096;   // one round of 16-row tiles for vocabularies up to 262144 (151936 rows at 16 activation rows: 286 -> 276 us)
-        hipLaunchKernelGGL((dense_gemm16_kernel<F16>), dim3(g16), dim3(256), 0, st, y, x, W, bias, M, N, K);
+        if (K % 1024) hipLaunchKernelGGL((dense_gemm16_kernel<F16, true>), dim3(g16), dim3(256), 0, st, y, x, W, bias, M, N, K);
+        else hipLaunchKernelGGL((dense_gemm16_kernel<F16, false>), dim3(g16), dim3(256), 0, st, y, x, W, bias, M, N, K);
         VMX_CHECK_LAUNCH("dense_gemm16");
         return VMX_OK;
     }
