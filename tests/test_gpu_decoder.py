@@ -266,6 +266,48 @@ def test_exl3_decoder_matches_oracle(gpu, bits, cb):
     model.close()
 
 
+@pytest.mark.parametrize("B", [1, 4])
+@pytest.mark.parametrize("bound", [300, 900])
+@pytest.mark.parametrize("kv_dtype", [0, 1])
+def test_exl3_wide_heads_transform_in_attention(gpu, kv_dtype, bound, B):
+    """128-wide heads, up to four rows: the output transform of q|k|v is left to the attention kernel, for a bf16 and for an FP8 cache, in the form whose
+    partitions o_proj merges (bounds up to 512) and in the one with a merge of its own.  Without the transform the logits and the cached rows are unrelated to the oracle's.
+    Cached FP8 rows: values 2^-9 apart land on other codes, 2^-4 apart, in up to a sixth of the cases, 2.6 % in all; later layers' inputs differ by ~ 1 % more."""
+    from oracle import oracle as orc
+    from tests.model_oracle import OracleQwen3
+    from vllm_rust_amd.qwen3 import QuantizedQwen3ForCausalLM, rope_cos_sin_cache
+    vmx, torch = gpu
+    spec = _tiny_spec(head_dim=128, num_blocks=64, max_seq_len=bound, max_position=1024, kv_cache_dtype=kv_dtype)
+    model = QuantizedQwen3ForCausalLM(spec)
+    ck = model.load_synthetic_exl3(bits=4, codebook=0, seed=16, keep_host_copy=True)
+    ref = OracleQwen3(spec, ck, rope_cos_sin_cache(spec.head_dim, spec.max_position, spec.rope_theta))
+    rng = np.random.default_rng(B)
+    bt = np.arange(B * 4, dtype=np.int32).reshape(B, 4)[:, ::-1].copy()
+    for step in range(20):   # beyond a tile of 16 tokens
+        ids = rng.integers(0, spec.vocab_size, size=B).astype(np.int32)
+        pos = np.full(B, step, np.int32)
+        slots = (bt[np.arange(B), pos // spec.block_size] * spec.block_size + pos % spec.block_size).astype(np.int32)
+        logits = torch.empty((B, spec.vocab_size), dtype=torch.bfloat16, device="cuda")
+        model.forward_decode_batch(*(torch.from_numpy(a).cuda() for a in (ids, pos, slots, bt, pos + 1)), max_seq_len=bound, logits=logits)
+        torch.cuda.synchronize()
+        exp = orc.bf16_to_f32(ref.decode(ids, pos, slots, bt, pos + 1)[0])
+        got = orc.bf16_to_f32(_u16(torch, logits))
+        rel = np.sqrt(((got - exp) ** 2).sum() / (exp ** 2).sum())
+        assert rel <= (3e-2 if kv_dtype == 0 else 5e-2), (step, rel)
+    shape = (spec.num_blocks * spec.block_size, spec.num_kv_heads, spec.head_dim)
+    for layer in range(spec.num_layers):
+        for which, cache in enumerate((ref.k_cache[layer], ref.v_cache[layer])):
+            t = torch.empty(shape, dtype=torch.uint8 if kv_dtype else torch.bfloat16, device="cuda")
+            model.debug_kv(layer, which, t, False)
+            wide = lambda c: (c.view(torch.float8_e4m3fn) if kv_dtype else c.view(torch.bfloat16)).float().numpy()   # noqa: E731
+            rows = np.concatenate([(bt[b][:, None] * spec.block_size + np.arange(spec.block_size)).reshape(-1)[:20] for b in range(B)])
+            g = wide(t.cpu())[rows]
+            e = wide(torch.from_numpy(cache.view(np.uint8 if kv_dtype else np.int16).reshape(shape)))[rows]
+            rel = np.sqrt(((g - e) ** 2).sum() / (e ** 2).sum())
+            assert rel <= (3e-2 if kv_dtype == 0 else 5e-2), (layer, which, rel)
+    model.close()
+
+
 def test_exl3_decoder_fp16_matches_oracle(gpu):
     """An EXL3 model run in fp16 end to end (vmx_qwen3_set_activation_dtype: fp16 embedding / norms / lm_head, fp16 activations,
     logits and cache) against the composed fp16 oracle; then the native prompt pass against the decode path on the same model."""

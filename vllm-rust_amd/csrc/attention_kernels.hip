@@ -1026,7 +1026,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HD == 2
 #pragma unroll
     for (int j = 0; j < EPL; j++) nw16[j] = nw_at[lane + 64 * j];
     uint16_t sv0 = 0, sv1 = 0;   // EXL3 output scales of this lane's two elements (HD == 128)
-    if constexpr (HD == 128 && FP8 != 1) {
+    if constexpr (HD == 128) {
         const uint16_t *sv_at = (had_svh ? had_svh : none) + (int64_t)head * HD + lane;
         sv0 = sv_at[0];
         sv1 = sv_at[64];
@@ -1112,7 +1112,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HD == 2
     ATTN_STAMP(2);
     // ---- A (arithmetic): bf16 round, optional per-head RMSNorm, NeoX RoPE; q -> LDS, k and v -> cache (owner only)
     if (has_head && g0 < T && (is_q || owner)) {
-        if constexpr (HD == 128 && FP8 != 1) {   // EXL3: the sums are the trellis GEMM before its output transform; a head is one Hadamard block
+        if constexpr (HD == 128) {   // EXL3: the sums are the trellis GEMM before its output transform; a head is one Hadamard block
             if (had_svh) attn_exl3_out_transform(v, lane, sv0, sv1);
         }
         float ss = 0.f;
