@@ -1,0 +1,75 @@
+"""What the compiler made of kernels whose source asks it for something that it does not check, read from the library built here."""
+import re
+import struct
+import subprocess
+from pathlib import Path
+
+import pytest
+
+LIB = Path(__file__).resolve().parent.parent / "vllm-rust_amd" / "lib" / "libvmx.so"
+LLVM = Path("/opt/rocm/llvm/bin")
+
+
+@pytest.fixture(scope="module")
+def attention_code(tmp_path_factory):
+    """The device code object that holds the decode-attention kernels."""
+    data = LIB.read_bytes()
+    at = data.find(b"__CLANG_OFFLOAD_BUNDLE__")
+    while at >= 0:
+        p = at + 32
+        for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
+            off, size, n = struct.unpack_from("<QQQ", data, p)
+            name = data[p + 24:p + 24 + n]
+            p += 24 + n
+            code = data[at + off:at + off + size]
+            if name.endswith(b"gfx950") and b"split_decode_attn_kernel" in code:
+                f = tmp_path_factory.mktemp("code") / "attention.o"
+                f.write_bytes(code)
+                return f
+        at = data.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 1)
+    pytest.fail("no decode-attention kernels in the library")
+
+
+def _kernels(code, names):
+    out = subprocess.run([LLVM / "llvm-objdump", "-d", "--no-show-raw-insn", f"--disassemble-symbols={','.join(names)}", code], check=True, capture_output=True,
+                         text=True).stdout
+    for part in re.split(r"\n(?=[0-9a-f]+ <)", out):
+        m = re.match(r"[0-9a-f]+ <(\S+)>:", part)
+        if m:
+            yield m.group(1), [line.split("//")[0].strip() for line in part.splitlines()[1:]]
+
+
+def _symbols(code):
+    out = subprocess.run([LLVM / "llvm-readelf", "-sW", code], check=True, capture_output=True, text=True).stdout
+    return [w for line in out.splitlines() if " FUNC " in line and "split_decode_attn_kernel" in line for w in line.split() if w.startswith("_Z")]
+
+
+def _registers(text):
+    m = re.match(r"v\[(\d+):(\d+)\]$|v(\d+)$", text)
+    return set() if not m else {int(m.group(3))} if m.group(3) else set(range(int(m.group(1)), int(m.group(2)) + 1))
+
+
+def test_swaps_in_assembly_wait_for_matrix_results(attention_code):
+    """A permlane swap written in assembly that reads what a matrix instruction leaves stands at least 16 wait states behind it: the compiler does not see the reader."""
+    names = [n for n in _symbols(attention_code) if re.search(r"ILi\d+ELi[124]E", n)]
+    assert len(names) >= 20
+    seen = 0
+    for name, lines in _kernels(attention_code, names):
+        for i, line in enumerate(lines):
+            if not line.startswith("v_permlane32_swap"):
+                continue
+            open_regs, states = set().union(*(_registers(r.strip()) for r in line.split(None, 1)[1].split(","))), 0
+            for back in reversed(lines[max(0, i - 200):i]):
+                op, _, rest = back.partition(" ")
+                if op == "s_nop":
+                    states += int(rest) + 1
+                    continue
+                dst = _registers(rest.split(",")[0].strip())
+                if open_regs & dst and op.startswith("v_mfma"):
+                    seen += 1
+                    assert states >= 16, (name, line, back, states)
+                open_regs -= dst if op.startswith("v_") else set()
+                if not open_regs:
+                    break
+                states += 1
+    assert seen >= len(names)   # the test still finds what it looks at

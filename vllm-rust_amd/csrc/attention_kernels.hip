@@ -947,10 +947,21 @@ __device__ __forceinline__ void dec_walk(DecState<HD> &st, const uint16_t *q_row
     fold(scores(p1 - t0), p1 - t0);
 }
 
-// Lanes 32 .. 63 of a and 0 .. 31 of b (MASK 32), odd rows of a and even rows of b (MASK 16) change places.
+// Lanes 32 .. 63 of a and 0 .. 31 of b (MASK 32), odd rows of a and even rows of b (MASK 16) change places.  Not of a matrix instruction's result as it
+// comes: dec_settle.
 template <int MASK> __device__ __forceinline__ void dec_swap(float &a, float &b) {
     if constexpr (MASK == 32) asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
     else asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+// The compiler keeps its own readers of a matrix instruction's result away from it until it is there (a 16x16x16 product: fewer than 16 wait states), but not
+// assembly: the wait for dec_swap's, once a wave.
+template <int HD> __device__ __forceinline__ void dec_settle(vmx_f32x4 (&o)[HD / 16]) {
+    if constexpr (HD == 64) asm volatile("s_nop 15" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
+    else {
+#pragma unroll
+        for (int b = 0; b < HD / 16; b += 8)
+            asm volatile("s_nop 15" : "+v"(o[b]), "+v"(o[b + 1]), "+v"(o[b + 2]), "+v"(o[b + 3]), "+v"(o[b + 4]), "+v"(o[b + 5]), "+v"(o[b + 6]), "+v"(o[b + 7]));
+    }
 }
 // The three terms' sums added up, out[e][r]: head r, number 16 (4 e + dec_block(dg)) + (lane & 15).
 __device__ __forceinline__ int dec_block(int dg) { return (dg >> 1) | ((dg & 1) << 1); }
@@ -1197,6 +1208,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HD == 2
             vmx_swap_pair<16>(st.s, a, b2); st.s = a + b2;
             vmx_swap_pair<32>(st.s, a, b2); st.s = a + b2;
             float out[HD / 64][4];
+            dec_settle<HD>(st.o);
             dec_add_terms<HD>(st.o, out);
             const float inv = vsc * (FP8 == 3 ? 0x1p-15f : 1.0f) / (st.s + 1e-6f);
             const float c[4] = {vmx_dpp<0x00>(inv), vmx_dpp<0x55>(inv), vmx_dpp<0xAA>(inv), vmx_dpp<0xFF>(inv)};
