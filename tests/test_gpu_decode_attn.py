@@ -108,3 +108,17 @@ def test_decode_attention_matches_float64(gpu, heads, kv, hd, fp8, block, lens, 
         rel = ((got[b] - want[b]).norm() / want[b].norm()).item()
         assert rel <= (6e-2 if fp8 else 1.5e-2), (b, lens[b], rel)
     m.close()
+
+
+# Eight query heads a KV head
+EIGHT = [(8, 1, 128, False, 16, [600, 31, 1000], 1100), (8, 1, 128, True, 16, [600, 31, 1000], 1100), (16, 2, 64, False, 5, [701, 15, 511], 1024),
+         (16, 2, 64, True, 16, [701, 15, 511], 1024), (16, 2, 128, False, 1, [150, 950], 1000)]
+# 16 rows over two KV heads have 64 waves each: 4900 tokens on pages of one are 76 pages a wave, more than its lanes hold, so that its lookups go to memory
+LONG = [4900, 4300] + [100 + 311 * i for i in range(14)]
+PAGES = [(4, 2, 64, False, 1, LONG, 5000), (4, 2, 64, True, 1, LONG, 5000), (4, 2, 128, False, 1, LONG, 5000), (16, 2, 64, False, 1, LONG, 5000), (16, 2, 128, True, 1, LONG, 5000)]
+
+
+@pytest.mark.parametrize("heads,kv,hd,fp8,block,lens,bound", EIGHT + PAGES)
+def test_eight_heads_and_long_walks_match_float64(gpu, heads, kv, hd, fp8, block, lens, bound):
+    """As above, with its bounds."""
+    test_decode_attention_matches_float64(gpu, heads, kv, hd, fp8, block, lens, bound)

@@ -73,3 +73,15 @@ def test_swaps_in_assembly_wait_for_matrix_results(attention_code):
                     break
                 states += 1
     assert seen >= len(names)   # the test still finds what it looks at
+
+
+def test_eight_heads_keep_their_values_in_registers(attention_code):
+    """Decode attention of eight query heads a KV head, which walks with two tiles and eight heads' sums in registers, does not go to scratch memory."""
+    out = subprocess.run([LLVM / "llvm-readelf", "--notes", attention_code], check=True, capture_output=True, text=True).stdout
+    sizes = {}
+    for entry in re.split(r"\n  - ", out):
+        name, size = re.search(r"\.name: +(\S*split_decode_attn_kernelILi\d+ELi8E\S*)", entry), re.search(r"\.private_segment_fixed_size: +(\d+)", entry)
+        if name:
+            sizes[name.group(1)] = int(size.group(1))
+    assert len(sizes) >= 6
+    assert not {n: b for n, b in sizes.items() if b}

@@ -132,7 +132,7 @@ template <int HD, int FP8> struct AttnTile {
 // Request tile [t0, min(t0 + 16, p1)): lane (token tl, dim group dg) takes 16-byte pieces of its token's K row, and every
 // V row of the tile is one coalesced wave access (row base broadcast from the lane that owns the token).  Lanes past the
 // end re-read the last valid row; their logits are masked later.
-// BTREG: lane l of bt_reg holds the sequence's block-table entry bt_base + l (read once) and the lookup is a lane exchange
+// BTREG, bt_base >= 0: lane l of bt_reg holds the sequence's block-table entry bt_base + l (read once) and the lookup is a lane exchange
 // instead of a dependent global load -- which, loads returning in order, would also wait for the tile requested before.
 template <int HD, int FP8, bool BTREG = false>
 __device__ __forceinline__ void attn_tile_load(AttnTile<HD, FP8> &t, const void *__restrict__ k_cache, const void *__restrict__ v_cache,
@@ -143,7 +143,12 @@ __device__ __forceinline__ void attn_tile_load(AttnTile<HD, FP8> &t, const void 
     const bool lane_live = (HD >= 128) || (lane < 32);
     const int ntok = min(16, p1 - t0);
     const int tok = t0 + min(tl, ntok - 1);
-    const int blk = BTREG ? __shfl(bt_reg, tok / block_size - bt_base, 64) : bt_row[tok / block_size];
+    int blk;
+    if (BTREG && bt_base >= 0) blk = __shfl(bt_reg, tok / block_size - bt_base, 64);
+    else {
+        blk = bt_row[tok / block_size];
+        if constexpr (BTREG) asm volatile("" : "+v"(blk));   // waited for here, not where this branch meets the other
+    }
     const int64_t base = ((int64_t)blk * block_size + tok % block_size) * tok_stride + (int64_t)kvh * HD;
 #pragma unroll
     for (int i = 0; i < KSTEPS; i++) t.kraw[i] = load8_raw<FP8>(k_cache, base + 32 * i + 8 * dg);
@@ -1085,6 +1090,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HD == 2
         asm volatile("" : "+v"(bt_reg));   // waited for here: behind the branch the lookup waits for the first load only
         bt_regs = true;
     }
+    // Eight heads take one walk whose lookups choose as they come: a walk compiled for each kind spilled 10 to 27 registers (44 .. 104 bytes a lane).  64 heads over 8, 128
+    // wide, 16 rows of 1500 to 800 tokens, us a launch with spills / without: bf16 38.6 / 39.4, FP8 39.4 / 38.0 (the older prologue 41.3 and 41.7); one row of 1500, 64-wide
+    // heads: equal.  Up to four heads keep both walks: theirs spill four or five registers in the walk with lookups in memory alone, and one walk for both kinds, which
+    // spills none, took 21.6 us where this takes 20.7 (16 rows of 32 heads over 8, with K and V from memory; the second trip to the block table in hand: 21.3).
+    if (!MX && !bt_regs) bt_base = -1;
     std::conditional_t<MX, DecTile<HD, FP8>, AttnTile<HD, FP8>> tile;
     const DecPages pages{bt_row, bt_reg, bt_base, (uint32_t)block_size, page_recip};
     const bool pre = active && p0 + 16 < seq_len;
@@ -1098,8 +1108,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HD == 2
             fresh = !pre && row == slot;
         }
     } else if (pre) {
-        if (bt_regs) attn_tile_load<HD, FP8, true>(tile, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, lane, bt_reg, bt_base);
-        else attn_tile_load<HD, FP8, false>(tile, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, lane);
+        attn_tile_load<HD, FP8, true>(tile, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, lane, bt_reg, bt_base);
     }
     float v[EPL], nwf[EPL];
 #pragma unroll
@@ -1232,12 +1241,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HD == 2
                 qa[i] = make_uint4(0, 0, 0, 0);
                 if (tl < nq) qa[i] = *reinterpret_cast<const uint4 *>(qs + tl * HD + 32 * i + 8 * dg);
             }
-            if (bt_regs)
-                attn_walk<HD, QPK, FP8, true>(qa, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, scale * ksc, vsc, lane,
-                                              m_run, s_run, o, tile, pre, bt_reg, bt_base);
-            else
-                attn_walk<HD, QPK, FP8, false>(qa, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, scale * ksc, vsc, lane,
-                                               m_run, s_run, o, tile, pre);
+            attn_walk<HD, QPK, FP8, true>(qa, k_cache, v_cache, bt_row, p0, p1, block_size, (int64_t)Hkv * HD, kvh, scale * ksc, vsc, lane, m_run, s_run, o, tile, pre,
+                                          bt_reg, bt_base);
         }
         asm volatile("" ::"v"(o[0][0][0]), "v"(s_run[0]));
         ATTN_STAMP(5);
