@@ -24,3 +24,11 @@ def test_matches_float64(M, N, K):
         assert torch.equal(y[:, 3].double(), exact[:, 3])
     assert torch.isfinite(y[:, keep]).all()
     assert ((y.double() - exact).abs() <= bound)[:, keep].all()
+
+
+# up to 16384 columns are one workgroup a compute unit at most; one column more and it is the other kernel: last tiles and workgroups that are part empty, odd and even
+# rows, one pass, a pass and some blocks, several
+@pytest.mark.parametrize("M,N,K", [(16, 16384, 256), (5, 16385, 128), (16, 16385, 1024), (8, 16447, 1152), (13, 20001, 896), (7, 33000, 640), (6, 16448, 4096), (11, 270001, 128)])
+def test_more_workgroups_than_compute_units(M, N, K):
+    """As above, with its bound."""
+    test_matches_float64(M, N, K)

@@ -80,15 +80,91 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(uint16_t *__restrict__ 
 // A fragment of step j is read from LDS at the matching k (x[m][128 b + 32 g + 8 j .. + 8]): the matrix instruction only needs
 // A and B to agree on which k sits where.  Activations are staged PK = 1024 k at a time (33 KB at 16 rows).  f32 accumulation
 // in k order within a lane group, groups summed by the MFMA: re-associated against the kernel above, same products.
-// A pass's activations are requested while the one before it is multiplied and the weights two blocks ahead, all behind no condition (rows and k that there are not
-// read others' words; behind the last pass every lane reads one place): a thread's eight pieces of a pass were eight trips, one after another:
-// 8 rows, 4000 x 4096 on 63 workgroups 32.4 -> 21.0 us; 16 rows, 38000 x 4096 on 594, the stream's time, 76.6 -> 77.  With non-temporal weight loads a step of 672 us took 717 (a lane's 64 bytes are four loads).
+constexpr int G16_PK = 1024, G16_XROW = G16_PK + 8;   // k per pass; staged row stride (+16 B against bank conflicts)
+template <bool F16> __device__ __forceinline__ vmx_f32x4 gemm16_mfma(uint4 a, uint4 w, vmx_f32x4 acc) {
+    if constexpr (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, w), acc, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, a), __builtin_bit_cast(vmx_bf16x8, w), acc, 0, 0, 0);
+}
+// lane holds activation rows m = 4 g + r of output column (W row) tile * 16 + nl
+template <bool F16>
+__device__ __forceinline__ void gemm16_store(uint16_t *__restrict__ y, const uint16_t *__restrict__ bias, vmx_f32x4 acc, int tile, int nl, int g, int M, int N) {
+    const int col = tile * 16 + nl;
+    if (col >= N) return;
+    const float bv = bias ? vmx_ld16<F16>(bias[col]) : 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int m = 4 * g + r;
+        if (m < M) y[(int64_t)m * N + col] = vmx_st16<F16>(acc[r] + bv);
+    }
+}
+
+// More workgroups than compute units: one covers for another's wait, and what bounds the launch is the stream of the weights.  A pass's rows are requested where they
+// are needed, in one batch and only those that exist, the weights one block ahead.  5 / 8 / 16 rows, us a launch, rows one after another / as the kernel below does /
+// now: [24000, 4096] 46.7 45.9 52.4 / 48.3 46.8 47.8 / 43.4 43.7 42.2; [30000, 4096] 48.0 47.5 53.9 / 51.8 50.7 52.6 / 48.5 46.9 47.4; [37984, 4096] 70.9 70.0 74.0 /
+// 74.0 72.6 74.6 / 69.4 67.0 69.4 = 4.5 .. 4.6 TB/s; [37984, 4480] 72.4 70.8 73.6 / 80.9 79.2 81.5 / 70.2 69.0 72.9; [65536, 3840] 95.8 92.9 94.8 / 103.4 100 102.8 /
+// 94.1 91.8 94.9; [151936, 1024] 60.9 61.7 64.9 / 59.8 60.9 64.8 / 57.7 57.4 60.9; [32000, 1024] 13.9 14.1 15.4 / 12.9 13.0 13.4 / 13.5 13.6 13.8.
+template <bool F16>
+__global__ __launch_bounds__(256) void dense_gemm16_kernel(uint16_t *__restrict__ y, const uint16_t *__restrict__ x, const uint16_t *__restrict__ W,
+                                                           const uint16_t *__restrict__ bias, int M, int N, int K) {
+    __shared__ __align__(16) uint16_t xs[16 * G16_XROW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nl = lane & 15, g = lane >> 4;
+    const int tiles = (N + 15) >> 4;
+    const int waves_total = gridDim.x * 4;
+    // every wave of the workgroup walks the same number of tiles (barriers inside): tiles past the end are clamped, not stored
+    const int rounds = (tiles + waves_total - 1) / waves_total;
+    for (int rd = 0; rd < rounds; rd++) {
+        const int tile = rd * waves_total + blockIdx.x * 4 + wave;
+        const int row = min(tile * 16 + nl, N - 1);
+        const uint16_t *wrow = W + (int64_t)row * K;
+        vmx_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        // the weights of 128-deep block i + 1 are requested before block i is multiplied: with load and use in the same iteration
+        // a wave has one block (4 KB) in flight and the launch runs at the memory latency, not the memory rate
+        const int nblk = K >> 7;
+        uint4 wn[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) wn[j] = *reinterpret_cast<const uint4 *>(wrow + 32 * g + 8 * j);
+        for (int blk = 0; blk < nblk; blk++) {
+            const int k0 = (blk >> 3) * G16_PK, b = (blk & 7) * 128;
+            if ((blk & 7) == 0) {
+                const int k = k0 + min(8 * (tid & 127), min(G16_PK, K - k0) - 8);   // K % 128 == 0 (checked on the host); what lies past K is not read
+                uint4 st[8];   // piece i: row 2 i + tid / 128, elements 8 (tid % 128) ..
+                if (blk || rd) __syncthreads();   // the previous pass has been read by every wave
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const int m = 2 * i + (wave >> 1);
+                    st[i] = make_uint4(0, 0, 0, 0);
+                    if (m < M) st[i] = *reinterpret_cast<const uint4 *>(x + (int64_t)m * K + k);
+                }
+#pragma unroll
+                for (int i = 0; i < 8; i++) *reinterpret_cast<uint4 *>(xs + (2 * i + (wave >> 1)) * G16_XROW + 8 * (tid & 127)) = st[i];
+                __syncthreads();
+            }
+            uint4 wv[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) wv[j] = wn[j];
+            if (blk + 1 < nblk) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) wn[j] = *reinterpret_cast<const uint4 *>(wrow + (blk + 1) * 128 + 32 * g + 8 * j);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc = gemm16_mfma<F16>(*reinterpret_cast<const uint4 *>(xs + nl * G16_XROW + b + 32 * g + 8 * j), wv[j], acc);
+        }
+        if (tile < tiles) gemm16_store<F16>(y, bias, acc, tile, nl, g, M, N);
+    }
+}
+
+// No more workgroups than compute units: nothing covers for a wait.  A pass's activations are requested while the one before it is multiplied and the weights two blocks ahead,
+// all behind no condition (rows and k that there are not read others' words; behind the last pass every lane reads one place): a thread's eight pieces of a pass were
+// eight trips, one after another.  us a launch, 5 / 16 rows, the kernel above / this one: [4000, 4096] 26.2 26.7 / 17.9 18.6, [12000, 4096] 30.9 31.3 / 21.5 22.5,
+// [16000, 4096] (250 workgroups) 36.1 34.2 / 28.8 28.7, [16000, 1024] 9.3 9.5 / 7.8 7.8; a few more than the units and it is the other way round: [16600, 4096] (260)
+// 38.7 37.5 / 47.9 48.8, [18000, 1024] 10.8 11.2 / 12.0 12.6.  With non-temporal weight loads a step of 672 us took 717 (a lane's 64 bytes are four loads).
 // TAIL: K is no multiple of 1024 (of 128 it is); the last pass's blocks past K are zeros times zeros.
 template <bool F16, bool TAIL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void dense_gemm16_kernel(uint16_t *__restrict__ y, const uint16_t *__restrict__ x,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void dense_gemm16_ahead_kernel(uint16_t *__restrict__ y, const uint16_t *__restrict__ x,
                                                             const uint16_t *__restrict__ W, const uint16_t *__restrict__ bias, int M,
                                                             int N, int K) {
-    constexpr int PK = 1024, XROW = PK + 8;   // k per pass; staged row stride (+16 B against bank conflicts)
+    constexpr int PK = G16_PK, XROW = G16_XROW;
     __shared__ __align__(16) uint16_t xs[16 * XROW];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nl = lane & 15, g = lane >> 4;
@@ -137,25 +213,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
                     const uint4 au = *reinterpret_cast<const uint4 *>(xs + nl * XROW + b * 128 + 32 * g + 8 * j);
                     uint4 wv = w[b & 1][j];
                     if (TAIL && blk >= nblk) wv = make_uint4(0, 0, 0, 0);
-                    if constexpr (F16)
-                        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, au), __builtin_bit_cast(f16x8_t, wv), acc, 0, 0, 0);
-                    else
-                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, au), __builtin_bit_cast(vmx_bf16x8, wv), acc, 0, 0, 0);
+                    acc = gemm16_mfma<F16>(au, wv, acc);
                 }
                 weights(b & 1, blk + 2);
                 __builtin_amdgcn_sched_barrier(0);   // or the last two of a pass are requested behind it
             }
         }
-        // lane holds activation rows m = 4 g + r of output column (W row) tile * 16 + nl
-        const int col = tile * 16 + nl;
-        if (tile < tiles && col < N) {
-            const float bv = bias ? vmx_ld16<F16>(bias[col]) : 0.f;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = 4 * g + r;
-                if (m < M) y[(int64_t)m * N + col] = vmx_st16<F16>(acc[r] + bv);
-            }
-        }
+        if (tile < tiles) gemm16_store<F16>(y, bias, acc, tile, nl, g, M, N);
     }
 }
 
@@ -223,8 +287,10 @@ static int dense_gemv_launch_t(uint16_t *y, const uint16_t *x, const uint16_t *W
     if (mfma_min_m > 0 && M >= mfma_min_m && K % 128 == 0) {   // GEMM-shaped: matrix cores, activations staged in k-passes
         int g16 = ((N + 15) / 16 + 3) / 4;   // 4 waves x one 16-row tile of W per round
         if (g16 > 4096) g16 = 4096;   // one round of 16-row tiles for vocabularies up to 262144 (151936 rows at 16 activation rows: 286 -> 276 us)
-        if (K % 1024) hipLaunchKernelGGL((dense_gemm16_kernel<F16, true>), dim3(g16), dim3(256), 0, st, y, x, W, bias, M, N, K);
-        else hipLaunchKernelGGL((dense_gemm16_kernel<F16, false>), dim3(g16), dim3(256), 0, st, y, x, W, bias, M, N, K);
+        // a workgroup of its own for every compute unit at most, or several (both sides at the kernels)
+        if (g16 > vmx_num_cus()) hipLaunchKernelGGL((dense_gemm16_kernel<F16>), dim3(g16), dim3(256), 0, st, y, x, W, bias, M, N, K);
+        else if (K % 1024) hipLaunchKernelGGL((dense_gemm16_ahead_kernel<F16, true>), dim3(g16), dim3(256), 0, st, y, x, W, bias, M, N, K);
+        else hipLaunchKernelGGL((dense_gemm16_ahead_kernel<F16, false>), dim3(g16), dim3(256), 0, st, y, x, W, bias, M, N, K);
         VMX_CHECK_LAUNCH("dense_gemm16");
         return VMX_OK;
     }
