@@ -10,9 +10,8 @@ LIB = Path(__file__).resolve().parent.parent / "vllm-rust_amd" / "lib" / "libvmx
 LLVM = Path("/opt/rocm/llvm/bin")
 
 
-@pytest.fixture(scope="module")
-def attention_code(tmp_path_factory):
-    """The device code object that holds the decode-attention kernels."""
+def _code_with(kernel, to):
+    """The device code object that holds a kernel."""
     data = LIB.read_bytes()
     at = data.find(b"__CLANG_OFFLOAD_BUNDLE__")
     while at >= 0:
@@ -22,12 +21,17 @@ def attention_code(tmp_path_factory):
             name = data[p + 24:p + 24 + n]
             p += 24 + n
             code = data[at + off:at + off + size]
-            if name.endswith(b"gfx950") and b"split_decode_attn_kernel" in code:
-                f = tmp_path_factory.mktemp("code") / "attention.o"
+            if name.endswith(b"gfx950") and kernel.encode() in code:
+                f = to / "code.o"
                 f.write_bytes(code)
                 return f
         at = data.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 1)
-    pytest.fail("no decode-attention kernels in the library")
+    pytest.fail(f"no {kernel} in the library")
+
+
+@pytest.fixture(scope="module")
+def attention_code(tmp_path_factory):
+    return _code_with("split_decode_attn_kernel", tmp_path_factory.mktemp("code"))
 
 
 def _kernels(code, names):
@@ -85,3 +89,18 @@ def test_eight_heads_keep_their_values_in_registers(attention_code):
             sizes[name.group(1)] = int(size.group(1))
     assert len(sizes) >= 6
     assert not {n: b for n, b in sizes.items() if b}
+
+
+def test_normed_decode_products_leave_room_for_three_workgroups(tmp_path):
+    """Normed unquantised products of eight waves: LDS has room for three workgroups a compute unit, so wide products (many workgroups) are to use at most 80 registers, six waves a
+    SIMD, wherever rows need no more than two pieces a thread requested ahead; with up to four the two-block form has 93 and runs two workgroups."""
+    code = _code_with("dense_decode_kernel", tmp_path)
+    out = subprocess.run([LLVM / "llvm-readelf", "--notes", code], check=True, capture_output=True, text=True).stdout
+    used = {}
+    for entry in re.split(r"\n  - ", out):
+        name, n = re.search(r"\.name: +(\S*dense_decode_kernelILi(\d+)ELi16ELi[12]ELi1ELi[02]E(?:Li(\d)E)?\S*)", entry), re.search(r"\.vgpr_count: +(\d+)", entry)
+        if name:
+            used[name.group(1)] = (int(name.group(2)), name.group(3), int(n.group(1)))
+    small = {k: v for k, v in used.items() if v[1] != "4"}
+    assert len(small) >= 8
+    assert all(waves <= 8 and n <= 80 for waves, _, n in small.values()), small

@@ -56,7 +56,7 @@ constexpr int DD_STAGE = 16 * 1032;   // values that the norm and the merge stag
 // Their inputs come from the caches and are requested ahead of the weights of the first DEPTH blocks, because loads return in order.
 // What the first requests need comes as arguments of its own, which are in registers when a wave starts (members of a struct are not): a step of Qwen3-0.6B at
 // one row, 128 tokens, 821 -> 795 us, 0.2 us a launch.
-template <int NW, int CW, int DEPTH, int SRC, int DST>
+template <int NW, int CW, int DEPTH, int SRC, int DST, int HELD, int SUMS>
 __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W, const void *first, const void *second, const void *third, int M, int N, int K,
                                                                 int fourth, const DenseDecode rest) {
     DenseDecode p = rest;
@@ -65,29 +65,30 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
     else p.x = static_cast<const uint16_t *>(first), p.norm_w = static_cast<const uint16_t *>(second), p.ssq = static_cast<const float *>(third), p.tiles = fourth;
     constexpr int PARTS = 16 / CW, DEEP = 128 * PARTS;
     constexpr bool STAGED = SRC == DD_NORM || SRC == DD_MERGE, NORM = SRC == DD_NORM || SRC == DD_NORM_REG;
-    __shared__ float red[NW][64][4];
+    __shared__ float red[NW * SUMS][64][4];
     __shared__ __align__(16) uint16_t rows_lds[STAGED ? DD_STAGE : 8];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & (CW - 1), part = (lane & 15) / CW, g = lane >> 4, nt = blockIdx.x;
     const int nblk = (K + DEEP - 1) / DEEP, row = min(c, p.M - 1);
     const uint16_t *wrow = p.W + (int64_t)(DST == DD_GLU ? (c < CW / 2 ? 0 : p.N / 2) + nt * (CW / 2) + (c & (CW / 2 - 1)) : nt * CW + c) * K;
+    const uint16_t *idle = p.W + (int64_t)nt * (DST == DD_GLU ? CW / 2 : CW) * K;   // of the workgroup's own rows: a place for all of them is one channel of the L2
     const int k0 = 128 * part + 8 * g;
-    // Requests lie behind no condition (where one ends the compiler waits as if they had not been made, or, if it differs between lanes, for each before the next):
-    // what lies past K reads the last values again and is cleared before the product, a wave without a block reads one place (a compute unit is bound by its requests as well: one in
-    // every lane's own row cost down at 16 rows 8.9 -> 10.9 us), rows past M repeat the last
-    // one and are not stored.  Of several rows everything that has to be normed and its statistic come ahead of the weights.
-    // Qwen3-0.6B, a step of 1 / 2 / 4 / 9 / 16 rows: 723 / 774 / 944 / 1147 / 1407 -> 673 / 757 / 890 / 1116 / 1345 us (16 rows' gate|up 9.2 -> 8.0, q|k|v 6.8 -> 6.0).
+    // Requests lie behind no condition of a lane (the compiler waits for each before the next) and none that makes them more or fewer before a wait: what lies past K reads
+    // the last values again and is cleared before the product, rows past M repeat the last one and are not stored.  A wave without a first or a second block takes a way of
+    // its own; where a barrier stands between (staged rows) it reads one place instead, of the workgroup's own weights: the same for all workgroups is one channel of
+    // the L2, in which they queue, and one in every lane's own row cost down at 16 rows 8.9 -> 10.9 us.
+    // Of several rows what has to be normed and its statistic come ahead of the weights, HELD pieces a thread (dd_launch_norm).
     dd_u32x4 w[DEPTH][4], xr[DEPTH][4], nr[DEPTH][SRC == DD_NORM_REG ? 4 : 1];
     auto load_w = [&](int b, dd_u32x4 (&d)[4]) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) d[j] = __builtin_nontemporal_load(reinterpret_cast<const dd_u32x4 *>(b < nblk ? wrow + min(DEEP * b + k0 + 32 * j, K - 8) : p.W));
+        for (int j = 0; j < 4; j++) d[j] = __builtin_nontemporal_load(reinterpret_cast<const dd_u32x4 *>(!STAGED || b < nblk ? wrow + min(DEEP * b + k0 + 32 * j, K - 8) : idle));
     };
     auto load_rows = [&](int b, dd_u32x4 (&x)[4], dd_u32x4 (&n)[SRC == DD_NORM_REG ? 4 : 1]) {
         if constexpr (!STAGED) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int k = min(DEEP * b + k0 + 32 * j, K - 8);
-                x[j] = *reinterpret_cast<const dd_u32x4 *>(b < nblk ? p.x + (int64_t)row * K + k : p.x);
-                if constexpr (SRC == DD_NORM_REG) n[j] = *reinterpret_cast<const dd_u32x4 *>(b < nblk ? p.norm_w + k : p.norm_w);
+                x[j] = *reinterpret_cast<const dd_u32x4 *>(p.x + (int64_t)row * K + k);
+                if constexpr (SRC == DD_NORM_REG) n[j] = *reinterpret_cast<const dd_u32x4 *>(p.norm_w + k);
             }
         }
     };
@@ -129,8 +130,7 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
     const int row_bits = p.M <= 1 ? 0 : p.M <= 2 ? 1 : p.M <= 4 ? 2 : p.M <= 8 ? 3 : 4, rows = 1 << row_bits, quads = NORM ? p.tiles / 4 : 1;
     const float4 *tile = NORM ? reinterpret_cast<const float4 *>(p.ssq + (int64_t)min(lane & (rows - 1), p.M - 1) * p.tiles) : nullptr;
     float4 t0;
-    constexpr int HELD = 4;   // of several rows' chunks a thread requests ahead of the weights
-    dd_u32x4 xs[SRC == DD_NORM ? HELD : 1], ns[SRC == DD_NORM ? HELD : 1];
+    dd_u32x4 xs[HELD], ns[HELD];
     if constexpr (NORM) t0 = tile[min(lane >> row_bits, quads - 1)];
     float4 tq[HELD];
     if constexpr (SRC == DD_NORM) {
@@ -141,30 +141,31 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
             ns[u] = *reinterpret_cast<const dd_u32x4 *>(some ? p.norm_w + (at - row_of(at) * (K / 8)) * 8 : p.norm_w);
         };
         request(0);
-        if (p.M > 1) {   // six requests that one row has no use for cost it 0.4 us
+        if (HELD > 1 && p.M > 1) {   // always where HELD > 1 (dd_launch_norm); as a branch it keeps the compiler from 20 registers more
 #pragma unroll
             for (int u = 1; u < HELD; u++) tq[u] = tile[min((lane >> row_bits) + u * (64 >> row_bits), quads - 1)], request(u);
         }
     }
     if constexpr (SRC == DD_MERGE) load_parts(chunk0);
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++) load_rows(wave + d * NW, xr[d], nr[d]);
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++) load_w(wave + d * NW, w[d]);
     // DD_RESID: the thread's value of the stream, which the end waits for
     const int om = CW == 16 ? (tid >> 4) & 15 : (tid >> 2) & 3, on = tid & (CW - 1);
     const int64_t out_at = (int64_t)min(om, p.M - 1) * p.N + nt * CW + on;
     uint16_t hold = 0;
-    if constexpr (DST == DD_RESID) hold = p.h[out_at];
-    float inv = 0.f;
-    if constexpr (NORM) {
-        float sq = lane >> row_bits < quads ? (t0.x + t0.y) + (t0.z + t0.w) : 0.f;
-        const bool held = SRC == DD_NORM && p.M > 1;
-        if (held) {
+    auto request_hold = [&] {
+        if constexpr (DST == DD_RESID) hold = p.h[out_at];
+    };
+    if constexpr (STAGED) {
 #pragma unroll
-            for (int u = 1; u < HELD; u++) sq += (lane >> row_bits) + u * (64 >> row_bits) < quads ? (tq[u].x + tq[u].y) + (tq[u].z + tq[u].w) : 0.f;
-        }
-        for (int i = (lane >> row_bits) + (held ? HELD : 1) * (64 >> row_bits); i < quads; i += 64 >> row_bits) {
+        for (int d = 0; d < DEPTH; d++) load_w(wave + d * NW, w[d]);
+        request_hold();
+    }
+    float inv = 0.f;
+    auto statistic = [&] {
+        if constexpr (!NORM) return;
+        float sq = lane >> row_bits < quads ? (t0.x + t0.y) + (t0.z + t0.w) : 0.f;
+#pragma unroll
+        for (int u = 1; u < HELD; u++) sq += (lane >> row_bits) + u * (64 >> row_bits) < quads ? (tq[u].x + tq[u].y) + (tq[u].z + tq[u].w) : 0.f;
+        for (int i = (lane >> row_bits) + HELD * (64 >> row_bits); i < quads; i += 64 >> row_bits) {
             const float4 v = tile[i];
             sq += (v.x + v.y) + (v.z + v.w);
         }
@@ -175,7 +176,8 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
         sq += vmx_lane_xor<16>(sq);
         sq += vmx_lane_xor<32>(sq);
         inv = rsqrtf(sq / (float)K + p.eps);
-    }
+    };
+    if constexpr (STAGED) statistic();
     auto norm8 = [&](dd_u32x4 x, dd_u32x4 n, float by) {
         float f[8], gain[8];
         dd_unpack(x, f);
@@ -190,13 +192,10 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
             const float by = __shfl(inv, m);
             if (i < chunks) *reinterpret_cast<dd_u32x4 *>(&rows_lds[m * (K + 8) + (at - m * (K / 8)) * 8]) = norm8(x, n, by);
         };
-        if (64 * wave < chunks) stage(tid, xs[0], ns[0]);
-        if (p.M > 1) {
 #pragma unroll
-            for (int u = 1; u < HELD; u++)
-                if (64 * NW * u + 64 * wave < chunks) stage(tid + 64 * NW * u, xs[u], ns[u]);
-        }
-        for (int i = tid + 64 * NW * (p.M > 1 ? HELD : 1); i - lane < chunks; i += 64 * NW) {
+        for (int u = 0; u < HELD; u++)
+            if (64 * NW * u + 64 * wave < chunks) stage(tid + 64 * NW * u, xs[u], ns[u]);
+        for (int i = tid + 64 * NW * HELD; i - lane < chunks; i += 64 * NW) {
             const int at = min(i, chunks - 1), m = row_of(at);
             stage(i, *reinterpret_cast<const dd_u32x4 *>(p.x + (int64_t)at * 8), *reinterpret_cast<const dd_u32x4 *>(p.norm_w + (at - m * (K / 8)) * 8));
         }
@@ -209,8 +208,10 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
         }
     }
     if constexpr (STAGED) __syncthreads();
-    vmx_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    auto step = [&](int b, dd_u32x4 (&d)[4], dd_u32x4 (&x)[4], dd_u32x4 (&n)[SRC == DD_NORM_REG ? 4 : 1]) {
+    vmx_f32x4 acc[SUMS];
+#pragma unroll
+    for (int i = 0; i < SUMS; i++) acc[i] = vmx_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto step = [&](int b, dd_u32x4 (&d)[4], dd_u32x4 (&x)[4], dd_u32x4 (&n)[SRC == DD_NORM_REG ? 4 : 1], vmx_f32x4 &sum) {
         const bool past = DEEP * (b + 1) > K;   // the wave's
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -219,23 +220,39 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
             if constexpr (SRC == DD_NORM_REG) a = norm8(a, n[j], inv);
             else if constexpr (STAGED) a = *reinterpret_cast<const dd_u32x4 *>(&rows_lds[row * (K + 8) + min(k, K - 8)]);
             if (past && k >= K) a = v = dd_u32x4{0, 0, 0, 0};
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, a), __builtin_bit_cast(vmx_bf16x8, v), acc, 0, 0, 0);
-        }
-        if (DEPTH > 1 && b + DEPTH * NW < nblk) {
-            load_w(b + DEPTH * NW, d);
-            load_rows(b + DEPTH * NW, x, n);
+            sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, a), __builtin_bit_cast(vmx_bf16x8, v), sum, 0, 0, 0);
         }
     };
-    if constexpr (DEPTH == 1) {   // one block a wave
-        if (wave < nblk) step(wave, w[0], xr[0], nr[0]);
-    } else {
-        for (int b = wave; b < nblk; b += 2 * NW) {
-            step(b, w[0], xr[0], nr[0]);
-            if (b + NW < nblk) step(b + NW, w[1], xr[1], nr[1]);
+    if (DEPTH > 1 && wave + NW < nblk) {
+        constexpr int L = DEPTH - 1;
+        if constexpr (!STAGED) {
+            load_rows(wave, xr[0], nr[0]);
+            load_rows(wave + NW, xr[L], nr[L]);
+            load_w(wave, w[0]);
+            load_w(wave + NW, w[L]);
+            if constexpr (SRC == DD_ROWS && HELD > 1) __builtin_amdgcn_sched_barrier(0);
+            request_hold();
+            statistic();
         }
+        for (int b = wave; b < nblk; b += 2 * NW) {
+            step(b, w[0], xr[0], nr[0], acc[0]);
+            if (b + 2 * NW < nblk) load_w(b + 2 * NW, w[0]), load_rows(b + 2 * NW, xr[0], nr[0]);
+            if (b + NW < nblk) step(b + NW, w[L], xr[L], nr[L], acc[SUMS - 1]);
+            if (b + 3 * NW < nblk) load_w(b + 3 * NW, w[L]), load_rows(b + 3 * NW, xr[L], nr[L]);
+        }
+    } else {   // one block or none
+        if (!STAGED && wave < nblk) load_rows(wave, xr[0], nr[0]), load_w(wave, w[0]);
+        if constexpr (!STAGED) {
+            if constexpr (SRC == DD_ROWS && HELD > 1) __builtin_amdgcn_sched_barrier(0);
+            request_hold();
+            statistic();
+        }
+        if (wave < nblk) step(wave, w[0], xr[0], nr[0], acc[0]);
     }
 #pragma unroll
-    for (int r = 0; r < 4; r++) red[wave][lane][r] = acc[r];
+    for (int i = 0; i < SUMS; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[wave + NW * i][lane][r] = acc[i][r];
     __syncthreads();
     if (tid >= (CW == 4 ? 64 : 256)) return;
     // CW 16: thread -> row tid / 16, column tid % 16 (element (4 g + r, c) of a tile sits with lane 16 g + c); CW 4: thread -> part
@@ -244,7 +261,7 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
     const int from = CW == 16 ? (m >> 2) * 16 + n : (tid >> 4) * 20 + n, r = m & 3;
     float v = 0.f;
 #pragma unroll
-    for (int i = 0; i < NW; i++) v += red[i][from][r];
+    for (int i = 0; i < NW * SUMS; i++) v += red[i][from][r];
     if constexpr (CW == 4) {
         v += vmx_lane_xor<16>(v);
         v += vmx_lane_xor<32>(v);
@@ -275,19 +292,35 @@ __global__ __launch_bounds__(64 * NW) void dense_decode_kernel(const uint16_t *W
     }
 }
 
-template <int CW, int SRC, int DST>
+template <int CW, int SRC, int DST, int HELD = 1>
 int dd_launch(const DenseDecode &p, hipStream_t st) {
     const int nblk = (p.K + 128 * (16 / CW) - 1) / (128 * (16 / CW));
+    constexpr bool eight = SRC == DD_NORM || SRC == DD_NORM_REG;   // waves at most
     const dim3 grid((unsigned)(p.N / CW));
     const void *first = p.x, *second = p.norm_w, *third = p.ssq;
     int fourth = p.tiles;
     if (SRC == DD_MERGE) first = p.part, second = p.part_max, third = p.part_sum, fourth = p.P;
-    if (nblk <= 4) hipLaunchKernelGGL((dense_decode_kernel<4, CW, 1, SRC, DST>), grid, dim3(256), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
-    else if (nblk <= 8) hipLaunchKernelGGL((dense_decode_kernel<8, CW, 1, SRC, DST>), grid, dim3(512), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
-    else if (nblk <= 16 || SRC == DD_NORM_REG) hipLaunchKernelGGL((dense_decode_kernel<8, CW, 2, SRC, DST>), grid, dim3(512), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
-    else hipLaunchKernelGGL((dense_decode_kernel<SRC == DD_NORM_REG ? 8 : 16, CW, 2, SRC, DST>), grid, dim3(1024), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
+    if (nblk <= 4) hipLaunchKernelGGL((dense_decode_kernel<4, CW, 1, SRC, DST, HELD, 1>), grid, dim3(256), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
+    else if (nblk <= 8) hipLaunchKernelGGL((dense_decode_kernel<8, CW, 1, SRC, DST, HELD, 1>), grid, dim3(512), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
+    else if (nblk <= 16 || SRC == DD_NORM_REG) hipLaunchKernelGGL((dense_decode_kernel<8, CW, 2, SRC, DST, HELD, 1>), grid, dim3(512), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
+    else hipLaunchKernelGGL((dense_decode_kernel<eight ? 8 : 16, CW, 2, SRC, DST, HELD, SRC == DD_NORM ? 2 : 1>), grid, dim3(eight ? 512 : 1024), 0, st, p.W, first, second, third, p.M, p.N, p.K, fourth, p);
     VMX_CHECK_LAUNCH("dense_decode");
     return VMX_OK;
+}
+
+// The pieces of eight values that a thread of the normed forms requests ahead are registers of every wave: with room for four whatever the rows a compute unit held two
+// workgroups (one of 16 waves) where it has LDS for three, and wide products lost by it.  So one and two pieces have forms of their own (72 and 76 registers instead of 93), and
+// eight waves walk any K (16 waves of more than 64 registers are one workgroup; beyond 16 blocks a wave keeps the sums of 16 waves' blocks apart: the same bits).  Four pieces: more than two there are, or of many workgroups more than three (steps of
+// width 1536, 17920 gate|up columns, 6 / 8 / 10 rows, two or four pieces 604 633 681 / 614 635 669 us; 2048, 12288 columns, 8 rows 552 / 520).
+// Steps of 4 .. 12 such layers, 200 tokens, loads behind conditions / four pieces and 16 waves / now, us, 1 2 4 8 16 rows, width (gate|up columns):
+//    896 (9728): 320 332 379 468 530 / 312 337 374 474 514 / 279 307 354 441 499;    1024 (6144): 316 337 389 424 488 / 276 312 350 432 461 / 272 308 357 399 453
+//    1536 (17920): 443 480 552 638 830 / 464 492 577 637 789 / 436 470 546 636 778;  2048 (12288): 396 432 502 548 694 / 398 407 486 520 663 / 379 414 469 520 659
+//    2560 (19456): 424 447 498 613 718 / 455 511 559 568 687 / 411 435 486 567 676;  4096 (24576): 420 445 503 602 722 / 438 485 523 553 658 / 409 430 470 554 656
+template <int DST> int dd_launch_norm(const DenseDecode &p, hipStream_t st) {
+    if (p.M * (p.K + 8) > DD_STAGE) return dd_launch<16, DD_NORM_REG, DST>(p, st);
+    const int threads = p.K <= 512 ? 256 : 512, pieces = (p.M * (p.K / 8) + threads - 1) / threads;
+    if (p.M > 1 && pieces > (p.K > 1024 && p.N / 16 > 4 * vmx_num_cus() ? 3 : 2)) return dd_launch<16, DD_NORM, DST, 4>(p, st);
+    return pieces == 1 || p.M == 1 ? dd_launch<16, DD_NORM, DST, 1>(p, st) : dd_launch<16, DD_NORM, DST, 2>(p, st);
 }
 
 // Four columns a workgroup where sixteen would leave half of the compute units or more without one: each workgroup norms or merges all rows for
@@ -311,7 +344,8 @@ int vmx_dense_decode_tiles(int M, int N) { return N / (dd_narrow(M, N) ? 4 : 16)
 int vmx_dense_decode_f32(float *y, const uint16_t *x, const uint16_t *W, int M, int N, int K, hipStream_t st) {
     DenseDecode p{};
     p.W = W, p.x = x, p.y = y, p.M = M, p.N = N, p.K = K;
-    return dd_launch<16, DD_ROWS, DD_F32>(p, st);
+    // requests all made before the products (HELD > 1), or with the compiler's own order: 16 rows [4096, 1024] 4.2 / 4.4 us, [1024, 2304] 6.5 / 7.1; one 3.8 / 3.6, 5.6 / 5.4
+    return M > 8 ? dd_launch<16, DD_ROWS, DD_F32, 2>(p, st) : dd_launch<16, DD_ROWS, DD_F32>(p, st);
 }
 
 // y = rms_norm(h) W^T; ssq: what vmx_dense_decode_resid left for h
@@ -319,7 +353,7 @@ int vmx_dense_decode_norm_f32(float *y, const uint16_t *h, const uint16_t *norm_
                               int N, int K, hipStream_t st) {
     DenseDecode p{};
     p.W = W, p.x = h, p.norm_w = norm_w, p.eps = eps, p.ssq = ssq, p.tiles = tiles, p.y = y, p.M = M, p.N = N, p.K = K;
-    return M * (K + 8) <= DD_STAGE ? dd_launch<16, DD_NORM, DD_F32>(p, st) : dd_launch<16, DD_NORM_REG, DD_F32>(p, st);
+    return dd_launch_norm<DD_F32>(p, st);
 }
 
 // act [M][N / 2] = silu(gate) * up of rms_norm(h) W^T
@@ -327,7 +361,7 @@ int vmx_dense_decode_norm_glu(uint16_t *act, const uint16_t *h, const uint16_t *
                               int N, int K, hipStream_t st) {
     DenseDecode p{};
     p.W = W, p.x = h, p.norm_w = norm_w, p.eps = eps, p.ssq = ssq, p.tiles = tiles, p.act = act, p.M = M, p.N = N, p.K = K;
-    return M * (K + 8) <= DD_STAGE ? dd_launch<16, DD_NORM, DD_GLU>(p, st) : dd_launch<16, DD_NORM_REG, DD_GLU>(p, st);
+    return dd_launch_norm<DD_GLU>(p, st);
 }
 
 bool vmx_dense_decode_merge_ok(int M, int K, int head_dim, int parts) {
