@@ -401,11 +401,14 @@ __global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(co
 // wave order through LDS.
 // GluLinear: the sixteen columns are eight gate columns and the up columns that belong to them.
 // What the first requests need comes as arguments of its own (in registers when a wave starts; `plain`: no row list, no blocks, one product).  Requests lie behind no
-// condition, or the compiler waits for each before the next (dense_decode.hip): what lies past K reads the last values again and is cleared before the product, a
-// wave without a block reads one place, rows that do not exist read row 0 and are not stored.  f32 rows (A32) are rounded to bf16 as they are multiplied.
+// condition of a lane, or the compiler waits for each before the next (dense_decode.hip): what lies past K reads the last values again and is cleared before the product,
+// rows that do not exist read row 0 and are not stored.  A wave without a first or a second block takes a way of its own (as requests of one place, the same for every
+// workgroup, they made shallow products slower than behind conditions: below).  f32 rows (A32) are rounded to bf16 as they are multiplied.
+// HOLD: a block's requests are all made before its products, which the compiler else moves between them where a wave has one block: 16 rows of bf16, without / with,
+// [2048, 2048] 5.9 / 5.7 us, [3664, 2048] 9.3 / 8.4, [32000, 512] 12.8 / 11.2, [12288, 512] 6.2 / 5.6; of one row 3.2 / 3.3 [4096, 512], and f32 rows 3 % slower with.
 // 16 rows, us a launch before / now:  gate and up [12288, 2048] 16.5 / 15.9, [32000, 2048] 38.0 / 36.2, [11264, 2048] 16.9 / 15.6, [3664, 2048] 8.7 / 8.3, [2048, 6144] 13.1 /
 // 12.7, [2048, 2048] 6.5 / 5.8; a step of Larolorn's four layers with 1 / 4 / 16 rows 362 / 383 / 468 -> 354 / 371 / 453.
-template <int NW, int PARTS, int DEPTH, bool A32, class P = VmxLinear>
+template <int NW, int PARTS, int DEPTH, bool A32, bool HOLD, class P = VmxLinear>
 __global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const uint16_t *W, const void *A, int M, int N, int K, int lda, int w_sn, int plain, const P p) {
     constexpr bool GLU = std::is_same<P, GluLinear>::value;
     static_assert(!GLU || PARTS == 1, "eight gate and eight up columns a workgroup");
@@ -428,7 +431,7 @@ __global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const uint16_t *
     tg_u32x4 w[DEPTH][4], a[DEPTH][PARTS][4][AV];
     auto load_w = [&](int b, tg_u32x4 (&d)[4]) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) d[j] = *reinterpret_cast<const tg_u32x4 *>(b < nblk ? wrow + min(DEEP * b + 128 * part + 32 * j + 8 * fg, K - 8) : W);
+        for (int j = 0; j < 4; j++) d[j] = *reinterpret_cast<const tg_u32x4 *>(wrow + min(DEEP * b + 128 * part + 32 * j + 8 * fg, K - 8));
     };
     auto load_a = [&](int b, tg_u32x4 (&d)[PARTS][4][AV]) {
 #pragma unroll
@@ -437,7 +440,7 @@ __global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const uint16_t *
             for (int j = 0; j < 4; j++)
 #pragma unroll
                 for (int e = 0; e < AV; e++)
-                    d[q][j][e] = *reinterpret_cast<const tg_u32x4 *>(b < nblk ? arow + min(DEEP * b + 128 * q + 32 * j + 8 * fg, K - 8) * (A32 ? 4 : 2) + 16 * e : (const char *)A);
+                    d[q][j][e] = *reinterpret_cast<const tg_u32x4 *>(arow + min(DEEP * b + 128 * q + 32 * j + 8 * fg, K - 8) * (A32 ? 4 : 2) + 16 * e);
     };
     vmx_f32x4 acc[PARTS];
 #pragma unroll
@@ -461,23 +464,25 @@ __global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const uint16_t *
                 acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vmx_bf16x8, v), __builtin_bit_cast(vmx_bf16x8, x), acc[q], 0, 0, 0);
             }
         }
-        if (DEPTH > 1 && b + DEPTH * NW < nblk) {
-            load_w(b + DEPTH * NW, wv);
-            load_a(b + DEPTH * NW, av);
-        }
     };
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++) {
-        load_w(wave + d * NW, w[d]);
-        load_a(wave + d * NW, a[d]);
-    }
-    if constexpr (DEPTH == 1) {   // one block a wave
-        if (wave < nblk) step(wave, w[0], a[0]);
-    } else {
+    auto load = [&](int b, tg_u32x4 (&wv)[4], tg_u32x4 (&av)[PARTS][4][AV]) {
+        load_w(b, wv);
+        load_a(b, av);
+        if constexpr (HOLD) __builtin_amdgcn_sched_barrier(0);
+    };
+    if (DEPTH > 1 && wave + NW < nblk) {
+        constexpr int L = DEPTH - 1;
+        load(wave, w[0], a[0]);
+        load(wave + NW, w[L], a[L]);
         for (int b = wave; b < nblk; b += 2 * NW) {
             step(b, w[0], a[0]);
-            if (b + NW < nblk) step(b + NW, w[1], a[1]);
+            if (b + 2 * NW < nblk) load(b + 2 * NW, w[0], a[0]);
+            if (b + NW < nblk) step(b + NW, w[L], a[L]);
+            if (b + 3 * NW < nblk) load(b + 3 * NW, w[L], a[L]);
         }
+    } else if (wave < nblk) {   // one block, or none: no requests in their place
+        load(wave, w[0], a[0]);
+        step(wave, w[0], a[0]);
     }
     // the product of a column's own part
     vmx_f32x4 own = acc[0];
@@ -514,8 +519,12 @@ void launch_skinny_as(const P &p, hipStream_t st) {
     const dim3 grid((p.N + CW - 1) / CW, (p.M + 15) / 16, p.batch);
     const int64_t most = 0x7fffffff;
     const int plain = p.M <= 16 && p.batch == 1 && !p.row_ids && !p.block_expert && !p.total_rows && p.lda >= 0 && p.lda <= most && p.w_sn >= 0 && p.w_sn <= most;
-    if (p.a_f32) hipLaunchKernelGGL((linear_skinny_kernel<NW, PARTS, DEPTH, true, P>), grid, dim3(64 * NW), 0, st, p.W, p.A, p.M, p.N, p.K, (int)p.lda, (int)p.w_sn, plain, p);
-    else hipLaunchKernelGGL((linear_skinny_kernel<NW, PARTS, DEPTH, false, P>), grid, dim3(64 * NW), 0, st, p.W, p.A, p.M, p.N, p.K, (int)p.lda, (int)p.w_sn, plain, p);
+#define SKINNY(A32, HOLD) \
+    hipLaunchKernelGGL((linear_skinny_kernel<NW, PARTS, DEPTH, A32, HOLD, P>), grid, dim3(64 * NW), 0, st, p.W, p.A, p.M, p.N, p.K, (int)p.lda, (int)p.w_sn, plain, p)
+    if (p.a_f32) SKINNY(true, false);
+    else if (DEPTH == 1 && (PARTS == 2 || p.M > 8)) SKINNY(false, DEPTH == 1);
+    else SKINNY(false, DEPTH == 1 && PARTS == 2);
+#undef SKINNY
 }
 
 // What bounds these is the number of requests under way, so the split follows the number of 16-column groups (and K, never M: a row's
@@ -528,7 +537,7 @@ void launch_skinny_as(const P &p, hipStream_t st) {
 // Expert blocks bring row blocks of their own and keep four waves.
 void launch_skinny(const VmxLinear &p, hipStream_t st) {
     const int cols = (p.N + 15) / 16 * p.batch, cus = vmx_num_cus();
-    if (p.block_expert || cols >= 2 * cus) return launch_skinny_as<4, 1, 2>(p, st);
+    if (p.K > 512 && (p.block_expert || cols >= 2 * cus)) return launch_skinny_as<4, 1, 2>(p, st);
     if (cols >= cus || p.K <= 512) {
         const int nblk = (p.K + 127) / 128;
         return nblk <= 4 ? launch_skinny_as<4, 1, 1>(p, st) : nblk <= 8 ? launch_skinny_as<8, 1, 1>(p, st) : launch_skinny_as<8, 1, 2>(p, st);
@@ -540,7 +549,7 @@ void launch_skinny(const VmxLinear &p, hipStream_t st) {
 }
 void launch_skinny_glu(const GluLinear &p, hipStream_t st) {   // sixteen columns a workgroup
     const int nblk = (p.K + 127) / 128;
-    if (p.N / 16 >= 2 * vmx_num_cus()) return launch_skinny_as<4, 1, 2>(p, st);
+    if (nblk > 4 && p.N / 16 >= 2 * vmx_num_cus()) return launch_skinny_as<4, 1, 2>(p, st);
     return nblk <= 4 ? launch_skinny_as<4, 1, 1>(p, st) : nblk <= 8 ? launch_skinny_as<8, 1, 1>(p, st) : launch_skinny_as<8, 1, 2>(p, st);
 }
 
