@@ -45,3 +45,28 @@ def test_block_sizes(block_size, q_len, offset):
         torch.cuda.synchronize()
         outs.append(out)
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("hd,H,KVH,q_len,offset,window,kv_dtype", [(64, 128, 16, 352, 0, 296, 0), (64, 128, 16, 340, 169, 0, 1)])
+def test_more_workgroups_than_units(hd, H, KVH, q_len, offset, window, kv_dtype):
+    """352 workgroups and even chains: one group."""
+    one_group.test_prefill_attention_matches_float64(hd, H, KVH, q_len, offset, window, kv_dtype)
+
+
+# 256 compute units: up to that many workgroups whatever the chains, up to twice as many where the average chain is at most 0.7 of the longest and that is nine tiles or more
+@pytest.mark.parametrize("H,KVH,q_len,offset,window,groups", [
+    (8, 2, 321, 0, 0, 2), (16, 2, 2562, 0, 494, 1), (32, 8, 1627, 0, 406, 1), (32, 8, 1024, 0, 400, 2), (32, 8, 1025, 0, 400, 1), (32, 8, 1025, 0, 0, 2), (64, 16, 539, 0, 0, 1),
+    (64, 16, 576, 0, 0, 2), (64, 16, 600, 900, 0, 1), (32, 8, 1102, 423, 0, 2), (32, 8, 1500, 3000, 0, 1), (16, 8, 2100, 0, 1100, 1), (16, 8, 2100, 0, 2080, 2), (8, 2, 64, 1000, 0, 2)])
+def test_groups_chosen(H, KVH, q_len, offset, window, groups):
+    import torch
+    import vllm_rust_amd as vmx
+    from tests.helpers import launched_kernels
+    from vllm_rust_amd._lib import check, lib
+    vmx.init(0)
+    total = q_len + offset
+    q, k = torch.zeros(q_len, H, 128, dtype=torch.bfloat16, device="cuda"), torch.zeros((total + 15) // 16 * 16, KVH, 128, dtype=torch.bfloat16, device="cuda")
+    table, out = torch.arange((total + 15) // 16, dtype=torch.int32, device="cuda"), torch.empty_like(q)
+    (name,) = [n for n, *_ in launched_kernels(torch, lambda: check(lib.vmx_prefill_attention_bf16(
+        out.data_ptr(), q.data_ptr(), k.data_ptr(), k.data_ptr(), table.data_ptr(), q_len, offset, 128 ** -0.5, H, KVH, 128, 16, window, 0, None, None,
+        torch.cuda.current_stream().cuda_stream)))]
+    assert f"Li4ELi{groups}EE" in name, name

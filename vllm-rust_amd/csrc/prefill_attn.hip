@@ -343,14 +343,21 @@ int vmx_prefill_attention_tiled(uint16_t *out, const uint16_t *q, const void *k_
     static const int nw_env = vmx_tune("VMX_PREFILL_NW", 0);
     const int64_t wg8 = (int64_t)((q_len + 32 * (8 / hpw) - 1) / (32 * (8 / hpw))) * num_kv_heads * ((nq + hpw - 1) / hpw);
     const bool eight = nw_env ? nw_env == 8 : wg8 >= 2 * vmx_num_cus();
-    // Two groups of four waves share the keys of a workgroup while the workgroups are few (a unit holds one such workgroup, or two of one group) and the longest
+    // Two groups of four waves share the keys of a workgroup while the workgroups are few (a unit holds one such workgroup, or two of one group: below) and the longest
     // chain is six tiles or more; with a shorter one the merge costs what the halved chain gives.  us, one group / two, bf16, no history unless said, tokens
     // 200 / 256 / 333 / 512 / 1024 / 2048 / 4096: 32 heads over 8, 128 wide 9.6 11.0 12.8 17.1 29.1 58.1 169 / 10.4 11.4 12.9 16.5 26.8 55.3 178 (512 workgroups at 2048);
     // 8 over 8 10.2 11.1 13.1 17.1 28.5 51.6 98 / 9.6 10.9 11.8 15.4 24.4 41.7 78; 16 over 4, 64 wide 7.2 8.1 9.3 12.1 20.7 37.6 78 / 7.2 7.8 8.7 10.6 16.9 29.1 62;
     // 16 tokens behind 2000: 47.9 / 40.0; 64 heads over 8, 1024 tokens, window 256 (512 workgroups, chains of 5 tiles) 22.0 / 26.7.
     const int64_t wg4 = (int64_t)((q_len + 32 * (4 / hpw) - 1) / (32 * (4 / hpw))) * num_kv_heads * ((nq + hpw - 1) / hpw);
     const int64_t chain = std::min<int64_t>((int64_t)seqlen_offset + q_len, window > 0 ? (int64_t)window + 32 * (4 / hpw) : INT64_MAX);
-    const bool two = nw_env ? nw_env == 2 : wg4 <= 2 * vmx_num_cus() && chain > 5 * PA_KT;
+    // With more workgroups than units the second groups of some wait for others' places, which pays while chains are uneven (no history: from one tile to the longest) and long.
+    // Of 200 sizes with 257 .. 512 workgroups two groups took 0.71 .. 1.4 of one group's rate; by average / longest chain: up to 0.6 and nine tiles or more 0.96 .. 1.4, above
+    // 0.7 0.71 .. 1.14, even chains 0.87 .. 0.91.  16 heads over 2, 128 wide, 2562 tokens, window 494 (324 workgroups) 28.3 / 35.4 us (29.8 before there were two); 32 over 8,
+    // 1627 tokens, window 406 31.2 / 35.7 (33.9); 1558 tokens without a window 44.1 / 38.0 (55.9).
+    const int64_t average2 = chain >= (int64_t)seqlen_offset + q_len ? 2 * (int64_t)seqlen_offset + q_len   // twice the average over the tokens: min(place, chain)
+                             : seqlen_offset >= chain ? 2 * chain
+                                                      : (chain * chain - (int64_t)seqlen_offset * seqlen_offset + 2 * chain * ((int64_t)seqlen_offset + q_len - chain)) / q_len;
+    const bool two = nw_env ? nw_env == 2 : chain > 5 * PA_KT && (wg4 <= vmx_num_cus() || (wg4 <= 2 * vmx_num_cus() && chain >= 9 * PA_KT && 5 * average2 <= 7 * chain));
 #define PA_NW(HD, HPW, KVT) return eight ? launch_tiled<HD, HPW, KVT, 8, 1>(PA_ARGS) \
                                   : two ? launch_tiled<HD, HPW, KVT, 4, 2>(PA_ARGS) : launch_tiled<HD, HPW, KVT, 4, 1>(PA_ARGS)
 #define PA_KV(HD, HPW)                    \
