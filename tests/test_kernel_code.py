@@ -43,9 +43,9 @@ def _kernels(code, names):
             yield m.group(1), [line.split("//")[0].strip() for line in part.splitlines()[1:]]
 
 
-def _symbols(code):
+def _symbols(code, kernel="split_decode_attn_kernel"):
     out = subprocess.run([LLVM / "llvm-readelf", "-sW", code], check=True, capture_output=True, text=True).stdout
-    return [w for line in out.splitlines() if " FUNC " in line and "split_decode_attn_kernel" in line for w in line.split() if w.startswith("_Z")]
+    return [w for line in out.splitlines() if " FUNC " in line and kernel in line for w in line.split() if w.startswith("_Z")]
 
 
 def _registers(text):
@@ -104,3 +104,14 @@ def test_normed_decode_products_leave_room_for_three_workgroups(tmp_path):
     small = {k: v for k, v in used.items() if v[1] != "4"}
     assert len(small) >= 8
     assert all(waves <= 8 and n <= 80 for waves, _, n in small.values()), small
+
+
+def test_packed_products_without_norms_request_their_tables_in_a_short_loop(tmp_path):
+    """Decode tables of the packed IQ products reach LDS by up to 128 requests of a wave: without a norm prologue by the compiler's own instruction, no wait state or move before
+    each (a launch of few waves took up to 1.1 us longer with the untracked form, which is for the prologue)."""
+    code = _code_with("iq_pk_mmvq_kernel", tmp_path)
+    names = [n for n in _symbols(code, "iq_pk_mmvq_kernel") if re.search(r"iq_pk_mmvq_kernelILi\dELb0ELi0ELb[01]ELb0EE", n)]
+    assert len(names) >= 4
+    for name, lines in _kernels(code, names):
+        at = [i for i, line in enumerate(lines) if line.startswith("global_load_lds")]
+        assert at and not any(lines[i - 1].startswith("s_nop") for i in at), name
