@@ -110,8 +110,8 @@ def test_packed_products_without_norms_request_their_tables_in_a_short_loop(tmp_
     """Decode tables of the packed IQ products reach LDS by up to 128 requests of a wave: without a norm prologue by the compiler's own instruction, no wait state or move before
     each (a launch of few waves took up to 1.1 us longer with the untracked form, which is for the prologue)."""
     code = _code_with("iq_pk_mmvq_kernel", tmp_path)
-    names = [n for n in _symbols(code, "iq_pk_mmvq_kernel") if re.search(r"iq_pk_mmvq_kernelILi\dELb0ELi0ELb[01]ELb0EE", n)]
-    assert len(names) >= 4
+    names = [n for n in _symbols(code, "iq_pk_mmvq_kernel") if re.search(r"iq_pk_mmvq_kernelILi\dELb0ELi0ELb0ELb0EE", n)]
+    assert len(set(names)) == 3
     for name, lines in _kernels(code, names):
         at = [i for i, line in enumerate(lines) if line.startswith("global_load_lds")]
         assert at and not any(lines[i - 1].startswith("s_nop") for i in at), name
