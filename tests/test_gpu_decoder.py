@@ -308,6 +308,39 @@ def test_exl3_wide_heads_transform_in_attention(gpu, kv_dtype, bound, B):
     model.close()
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("lens,bound", [([290, 17], 300), ([850, 513, 64], 900)])
+def test_fp16_cache_of_wide_scores_matches_oracle(gpu, hd, lens, bound):
+    """A step over full fp16 caches whose scores spread by 4 standard deviations, so weights run from 1 to 2^-30 and their fp16 terms down to and below the smallest
+    normal number.  q and the cached rows are rounded by 2^-11: a score of ~ 4 moves by ~ 4 2^-11 times a few roundings (q's norm, rotation, storage), its weight by as
+    much of itself, under 1 % of the attention's output, which is about half of the stream."""
+    from tests.model_oracle import OracleQwen3
+    from vllm_rust_amd.qwen3 import QuantizedQwen3ForCausalLM, rope_cos_sin_cache
+    vmx, torch = gpu
+    width = (bound + 15) // 16
+    spec = _tiny_spec(head_dim=hd, act_dtype="f16", num_blocks=width * len(lens), max_seq_len=bound, max_position=1024)
+    model = QuantizedQwen3ForCausalLM(spec)
+    ck = model.load_synthetic_exl3(bits=4, codebook=0, seed=31, keep_host_copy=True)
+    ref = OracleQwen3(spec, ck, rope_cos_sin_cache(spec.head_dim, spec.max_position, spec.rope_theta, "f16"))
+    rng = np.random.default_rng(hd + bound)
+    for layer in range(spec.num_layers):
+        for which, (cache, by) in enumerate(((ref.k_cache[layer], 4.0), (ref.v_cache[layer], 1.0))):
+            cache[...] = (rng.standard_normal(cache.shape) * by).astype(np.float16).view(np.uint16)
+            model.debug_kv(layer, which, torch.from_numpy(cache.view(np.int16)).cuda(), True)
+    bt = rng.permutation(width * len(lens)).astype(np.int32).reshape(len(lens), width)
+    ids, pos = rng.integers(0, spec.vocab_size, len(lens)).astype(np.int32), np.array(lens, np.int32)
+    slots = (bt[np.arange(len(lens)), pos // 16] * 16 + pos % 16).astype(np.int32)
+    logits = torch.empty((len(lens), spec.vocab_size), dtype=torch.float16, device="cuda")
+    model.forward_decode_batch(*(torch.from_numpy(a).cuda() for a in (ids, pos, slots, bt, pos + 1)), max_seq_len=bound, logits=logits)
+    torch.cuda.synchronize()
+    exp = ref.decode(ids, pos, slots, bt, pos + 1)[0].view(np.float16).astype(np.float32)
+    got = logits.float().cpu().numpy()
+    assert np.isfinite(got).all()
+    for b in range(len(lens)):
+        assert np.linalg.norm(got[b] - exp[b]) <= 1e-2 * np.linalg.norm(exp[b]), (b, np.linalg.norm(got[b] - exp[b]) / np.linalg.norm(exp[b]))
+    model.close()
+
+
 def test_exl3_decoder_fp16_matches_oracle(gpu):
     """An EXL3 model run in fp16 end to end (vmx_qwen3_set_activation_dtype: fp16 embedding / norms / lm_head, fp16 activations,
     logits and cache) against the composed fp16 oracle; then the native prompt pass against the decode path on the same model."""

@@ -811,7 +811,8 @@ __device__ unsigned long long vmx_attn_stamp_buf[4096 * 8];
 // The scores are formed transposed, S^T = K Q^T: lane (dg, n) ends up with four tokens 4 dg + r of head n & 3, so the softmax of a tile is three
 // maxima in the lane and two across lanes, its sum stays in the lane until the end, and the probabilities lie as the second product takes them as its
 // left operand.  That product has 16 rows and only four heads, so the rows hold each probability in three bf16 terms of 8 bits (row 4 term + head:
-// together the 24 bits of the f32 number; fp16 caches: terms of 11 bits of 2^15 p) and the three sums are added at the end: no bit of p is lost.  (An infinite
+// together the 24 bits of the f32 number; fp16 caches: terms of 11 bits of 2^15 p) and the three sums are added at the end: no bit of p is lost (fp16: of a term what lies
+// below 2^-24, fp16's last bit, so less than 2^-39 of p each, where the largest p of a wave is 1).  (An infinite
 // value makes its number NaN, 0 inf in a term, where it was infinite: the projection behind makes NaN of either.)
 // V takes the way K takes (one address for both), goes through the wave's own rows in LDS and comes back transposed (ds_read_b64_tr_b16).
 // Against p broadcast lane by lane and a multiply-add per number (447 vector instructions a tile, a branch a token): see the kernel.
@@ -995,7 +996,8 @@ constexpr int split_wave_floats(int hd, int qpk) { return split_on_mfma(qpk) ? 8
 // for.  The tile of the new token is requested with the others; its own row, which this workgroup derives, is put in from LDS.
 // Before (loads behind branches, each waited for; 64-bit divisions; that tile behind the barrier; p broadcast lane by lane) / now, us a launch, 8 KV heads:
 // Qwen3-0.6B, one row of 128 tokens 7.5 / 5.4; Qwen3-8B of 300 8.9 / 6.8 (fp16 9.2 / 6.7); 256-wide FP8 heads 10.1 / 6.9; 16 rows of 1500 to 800 tokens 25.8 / 21.1
-// (75 MB of K and V; the tiles requested and not multiplied: 22.1 with the prologue as it was).  Steps: 770 / 718, 442 / 419, 747 / 725, 742 / 706, 713 / 674.
+// (75 MB of K and V: 3.6 TB/s, where a large copy reaches 4.65; the tiles requested and not multiplied: 22.1 with the prologue as it was).  Steps, each with this alone
+// changed: Qwen3-0.6B 795 / 737, AWQ 435 / 410, EXL3 702 / 676, Gemma 726 / 690, AWQ of 16 rows 693 / 655.
 template <int HD, int QPK, int FP8, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HD == 256 ? 2 : 4))) void split_decode_attn_kernel(
     const float *__restrict__ partial, const int32_t *__restrict__ seq_lens, const int32_t *__restrict__ block_tables, const int32_t *__restrict__ positions,
