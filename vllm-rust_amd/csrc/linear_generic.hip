@@ -406,8 +406,8 @@ __global__ __launch_bounds__(S::THREADS, S::PER_SIMD) void linear_tile_kernel(co
 // workgroup, they made shallow products slower than behind conditions: below).  f32 rows (A32) are rounded to bf16 as they are multiplied.
 // HOLD: a block's requests are all made before its products, which the compiler else moves between them where a wave has one block: 16 rows of bf16, without / with,
 // [2048, 2048] 5.9 / 5.7 us, [3664, 2048] 9.3 / 8.4, [32000, 512] 12.8 / 11.2, [12288, 512] 6.2 / 5.6; of one row 3.2 / 3.3 [4096, 512], and f32 rows 3 % slower with.
-// 16 rows, us a launch before / now:  gate and up [12288, 2048] 16.5 / 15.9, [32000, 2048] 38.0 / 36.2, [11264, 2048] 16.9 / 15.6, [3664, 2048] 8.7 / 8.3, [2048, 6144] 13.1 /
-// 12.7, [2048, 2048] 6.5 / 5.8; a step of Larolorn's four layers with 1 / 4 / 16 rows 362 / 383 / 468 -> 354 / 371 / 453.
+// 16 rows, us a launch, requests behind conditions / now:  gate and up [12288, 2048] 16.4 / 14.9, [32000, 2048] 36.9 / 34.3, [11264, 2048] 16.1 / 14.7, [3664, 2048] 9.2 / 8.4,
+// [2048, 6144] 13.5 / 11.8, [2048, 2048] 6.5 / 5.7; a step of Larolorn's four layers with 1 / 4 / 16 rows 362 / 383 / 468 -> 354 / 367 / 450.
 template <int NW, int PARTS, int DEPTH, bool A32, bool HOLD, class P = VmxLinear>
 __global__ __launch_bounds__(64 * NW) void linear_skinny_kernel(const uint16_t *W, const void *A, int M, int N, int K, int lda, int w_sn, int plain, const P p) {
     constexpr bool GLU = std::is_same<P, GluLinear>::value;
